@@ -154,6 +154,17 @@ def value_length(pkv: tuple) -> int:
     return n
 
 
+def _cover_on_device(idx_list, n: int) -> bool:
+    """The check of ``idx_cover_once`` as one launch over a bit per position (it waits for the answer)."""
+    dev, k = idx_list[0].device, len(idx_list)
+    scratch = torch.zeros(1 + (n + 31) // 32, dtype=torch.int32, device=dev)
+    with _lib.on_device(dev):
+        rc = _lib.load().hqekv_cover_once((C.c_void_p * k)(*[t.data_ptr() for t in idx_list]), (C.c_int64 * k)(*[t.numel() for t in idx_list]),
+                                          k, scratch.data_ptr(), scratch.numel() * 4, _lib.stream_ptr(dev))
+    _lib.check(rc, "cover_once")
+    return int(scratch[0]) == 0
+
+
 def idx_cover_once(idx_list, n: int) -> bool:
     """True when the class position arrays, taken together, hold every position in [0, n) exactly once -- what
     the softmax fused into the two GEMV launches relies on (a position nobody writes keeps whatever the score
@@ -182,6 +193,9 @@ def idx_cover_once(idx_list, n: int) -> bool:
     elif all(h is not None for h in hosts):
         c = np.concatenate(hosts)
         ok = bool(c.size == n and (c >= 0).all() and (c < n).all() and (np.bincount(c, minlength=n) == 1).all())
+    elif idx_list[0].is_cuda and len(idx_list) <= _lib.MAX_SEGS and n < 2 ** 38 and \
+            all(t.dtype == torch.int64 and t.is_contiguous() and t.device == idx_list[0].device for t in idx_list):
+        ok = _cover_on_device(idx_list, n)
     else:
         c = torch.cat([t.reshape(-1).to(torch.int64) for t in idx_list])
         inside = (c >= 0) & (c < n)

@@ -706,11 +706,14 @@ def reconstruct(past_key_value: tuple, quant_strategy: str, block_size: int = 32
     else:
         b = next(b for b in (8, 4, 2, 1) if v_side[b].data is not None)
         D = v_side[b].data.shape[3] * (32 // b)
-    K = torch.zeros(B, H, T, D, dtype=torch.float16, device=dev)
-    V = torch.zeros(B, H, T, D, dtype=torch.float16, device=dev)
     for b in CLASS_BITS:
         if b == 1 and (k_side[b].data is not None or v_side[b].data is not None):
             _check_low_bits(1, quant_strategy)
+    if dev.type == "cuda" and D % 32 == 0:
+        return _reconstruct_on_device(pkv, B, H, T, D, dev, quant_strategy != LOW_NORMAL)
+    K = torch.zeros(B, H, T, D, dtype=torch.float16, device=dev)
+    V = torch.zeros(B, H, T, D, dtype=torch.float16, device=dev)
+    for b in CLASS_BITS:
         if k_side[b].data is not None:
             K[:, :, k_side[b].idx, :] = _k_to_fp16(k_side[b], b, quant_strategy).transpose(2, 3)
         if v_side[b].data is not None:
@@ -720,3 +723,30 @@ def reconstruct(past_key_value: tuple, quant_strategy: str, block_size: int = 32
     if new_V is not None:
         V[:, :, T - new_V.shape[2]:, :] = new_V
     return K, V
+
+
+def _reconstruct_on_device(pkv: tuple, B: int, H: int, T: int, D: int, dev, low_uniform: bool):
+    """Both dense tensors from one launch (``hqekv_cache_reconstruct``).  Where the classes and the residual of a side do
+    not name every position exactly once -- evicted tokens counted in ``kv_seq_len``, an idle side, a cache from
+    elsewhere -- the side starts from zeros and its segments are written one after the other, a later one over an earlier
+    one as in the sequence of assignments this stands for."""
+    from . import _lib
+    from . import attention as A
+    keep: list = []
+    sides = ((A.key_segments(pkv, dev, T, keep, low_uniform)[0], A.K16, A.K_BASE, pkv[A.NEW_K]),
+             (A.value_segments(pkv, dev, T, keep, low_uniform)[0], A.V16, A.V_BASE, pkv[A.NEW_V]))
+    dense, calls = [], []
+    for items, base0, bases, new in sides:
+        idx = A._class_idx(pkv, base0, bases)
+        n = T - (new.shape[2] if new is not None else 0)
+        whole = n >= 0 and all(t is not None for t in idx) and A.idx_cover_once(idx, n)
+        dense.append((torch.empty if whole else torch.zeros)(B, H, T, D, dtype=torch.float16, device=dev))
+        calls.append([items] if whole else [[it] for it in items])
+    lib, st = _lib.load(), _lib.stream_ptr(dev)
+    ptrs = [t.data_ptr() for t in dense]
+    with _lib.on_device(dev):
+        for i in range(max(len(c) for c in calls)):
+            k, v = (c[i] if i < len(c) else [] for c in calls)
+            _lib.check(lib.hqekv_cache_reconstruct(_lib.make_segs(k), len(k), _lib.make_segs(v), len(v), *ptrs, B * H, D, T, st),
+                       "cache_reconstruct")
+    return dense[0], dense[1]

@@ -1,0 +1,290 @@
+// A hybrid cache back into dense fp16 K and V (B,Hkv,T,D) (KV_cache_reconstruct, quant/hybrid_quant.py:732-846, and
+// KV_cache_reconstruct_hqe, quant/hqe_2.py:967-1084): every class dequantised with the reference's two fp16 roundings
+// (quant/pack_unpack.py:331-332) and written to its tokens' positions, both sides in one launch.
+//
+// Bound: HBM -- the cache is read once and the dense tensors are written once, 16 bytes per lane.  A workgroup takes 128
+// tokens of one class of one (b, kv head).  V classes and token-major fp16 rows are 16 lanes (8 channels each) per token
+// as they lie.  K classes are channel-major, the result is token-major: a wave takes one 32-token group, a lane two
+// channels of it (its codes are one short run of each row; the four waves read neighbouring runs of the same lines), and
+// the tile is turned in LDS -- 68 words per token row, so the channel-pair writes walk all banks and the 16-byte reads
+// stay aligned.  34 KB of LDS: four workgroups per CU.
+// Measured at B=1, 16k tokens of the fp16 / 8 / 4 / 2-bit mix (73 MB): 258 us as dequantise launches, transposing copies
+// and index_put scatters; this launch 21 us (3.4 TB/s), 38 us with the host call around it.
+#include "common.h"
+#include "quant_math.h"
+
+#pragma clang fp contract(off)
+
+namespace hq {
+
+struct RcSeg {
+  const void *data;
+  const half_t *scale;
+  const half_t *zero;
+  const int64_t *idx;
+  half_t *out;          // the dense tensor of this segment's side
+  int64_t pos_base;
+  int64_t slab_tokens;  // token rows between two (b, kv head) slabs of a token-major segment
+  int32_t n_tokens;
+  int16_t bits;
+  int16_t kind;         // 0: channel-major K, 1: token-major; + 2: 1-bit normal-quantile coding
+};
+constexpr int RC_SEGS = 2 * HQEKV_MAX_SEGS;
+struct RcTable {
+  RcSeg seg[RC_SEGS];
+  int32_t begin[RC_SEGS];   // first tile (grid.y) of every segment; INT32_MAX past the last
+};
+
+constexpr int RC_THREADS = 256;
+constexpr int RC_TOK = 128;    // tokens per workgroup
+constexpr int RC_CH = 128;     // channels turned in LDS at a time
+constexpr int RC_ROW = 68;     // 32-bit words per token row in LDS
+
+// where token t of the segment goes; -1: outside the dense tensor (an index counts from the end when negative, as in
+// torch; one that names no row is dropped)
+__device__ __forceinline__ int64_t rc_position(const RcSeg &s, int64_t t, int64_t T) {
+  int64_t p = s.idx ? s.idx[t] : s.pos_base + t;
+  if (p < 0) p += T;
+  return p >= 0 && p < T ? p : -1;
+}
+
+// the value of a code pair: rnd16(rnd16(c * scale) + zero), or rnd16(rnd16(+-k * std) + mean)
+template <bool NORMAL>
+__device__ __forceinline__ half2_t rc_value(uint32_t c0, uint32_t c1, half2_t s2, half2_t z2) {
+  half2_t c;
+  if (NORMAL) {
+    c[0] = c0 ? (half_t)0.67431640625f : (half_t)-0.67431640625f;
+    c[1] = c1 ? (half_t)0.67431640625f : (half_t)-0.67431640625f;
+  } else {
+    c[0] = (half_t)(unsigned short)c0;
+    c[1] = (half_t)(unsigned short)c1;
+  }
+  const half2_t m = c * s2;
+  return m + z2;
+}
+
+// 8 adjacent channels of one token: BITS bytes of codes in the low bits of w0 (and w1)
+template <int BITS, bool NORMAL>
+__device__ __forceinline__ uint4 rc_piece(uint32_t w0, uint32_t w1, half_t s, half_t z) {
+  const half2_t s2 = {s, s}, z2 = {z, z};
+  uint32_t r[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const uint32_t w = BITS == 8 && j >= 2 ? w1 : w0;
+    const int k = BITS == 8 ? 2 * (j & 1) : 2 * j;
+    r[j] = h2_bits(rc_value<NORMAL>(code_at<BITS>(w, k), code_at<BITS>(w, k + 1), s2, z2));
+  }
+  return make_uint4(r[0], r[1], r[2], r[3]);
+}
+
+template <int BITS, bool NORMAL>
+__device__ __forceinline__ void rc_token_major(const RcSeg &s, int64_t bh, int t0, int D, int64_t T) {
+  const int P = D >> 3, items = RC_TOK * P;   // pieces of 8 channels
+  constexpr int U = 4;
+  for (int i0 = threadIdx.x; i0 < items; i0 += U * RC_THREADS) {
+    uint4 v[U];
+    half_t sc[U], zr[U];
+    int64_t pos[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {   // the requests of U pieces together
+      const int i = i0 + u * RC_THREADS;
+      const int t = t0 + i / P, cp = i % P;
+      const bool in = i < items && t < s.n_tokens;
+      const int64_t row = bh * s.slab_tokens + (in ? t : t0);
+      const char *src = (const char *)s.data + (row * D + cp * 8) * BITS / 8;
+      pos[u] = in ? rc_position(s, t, T) : -1;
+      if (BITS == 16) {
+        v[u] = *reinterpret_cast<const uint4 *>(src);
+      } else {
+        if (BITS == 8) {
+          v[u].x = reinterpret_cast<const uint32_t *>(src)[0];
+          v[u].y = reinterpret_cast<const uint32_t *>(src)[1];
+        } else if (BITS == 4) {
+          v[u].x = *reinterpret_cast<const uint32_t *>(src);
+        } else if (BITS == 2) {
+          v[u].x = *reinterpret_cast<const unsigned short *>(src);
+        } else {
+          v[u].x = *reinterpret_cast<const unsigned char *>(src);
+        }
+        const int64_t g = row * (D >> 5) + (cp >> 2);
+        sc[u] = s.scale[g];
+        zr[u] = s.zero[g];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int cp = (i0 + u * RC_THREADS) % P;
+      if constexpr (BITS != 16) v[u] = rc_piece<BITS, NORMAL>(v[u].x, v[u].y, sc[u], zr[u]);
+      if (pos[u] >= 0) *reinterpret_cast<uint4 *>(s.out + (bh * T + pos[u]) * D + cp * 8) = v[u];
+    }
+  }
+}
+
+template <int BITS, bool NORMAL>
+__device__ __forceinline__ void rc_channel_major(const RcSeg &s, int64_t bh, int t0, int D, int64_t T, uint32_t *tile) {
+  const int dp = threadIdx.x & 63, g = threadIdx.x >> 6;   // channel pair, 32-token group of the tile
+  const int n = s.n_tokens, tg = t0 + 32 * g;              // the group's first token
+  for (int c0 = 0; c0 < D; c0 += RC_CH) {
+    const int d = c0 + 2 * dp;
+    if (d < D && tg < n) {
+      uint32_t *col = tile + (32 * g) * RC_ROW + dp;
+      if constexpr (BITS == 16) {
+        const half_t *ra = (const half_t *)s.data + (bh * D + d) * (int64_t)n + tg, *rb = ra + n;
+        if ((n & 7) == 0) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            if (tg + 8 * q < n) {
+              const uint4 a = reinterpret_cast<const uint4 *>(ra)[q], b = reinterpret_cast<const uint4 *>(rb)[q];
+              const uint32_t av[4] = {a.x, a.y, a.z, a.w}, bv[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+              for (int j = 0; j < 4; ++j) {
+                col[(8 * q + 2 * j) * RC_ROW] = __builtin_amdgcn_perm(bv[j], av[j], 0x05040100u);
+                col[(8 * q + 2 * j + 1) * RC_ROW] = __builtin_amdgcn_perm(bv[j], av[j], 0x07060302u);
+              }
+            }
+          }
+        } else {
+          for (int i = 0; i < 32 && tg + i < n; ++i) col[i * RC_ROW] = h2_bits((half2_t){ra[i], rb[i]});
+        }
+      } else {   // (the class holds whole groups of 32 tokens)
+        constexpr int PF = 32 / BITS;
+        const int64_t ga = (bh * D + d) * (int64_t)(n >> 5) + (tg >> 5), gb = ga + (n >> 5);
+        const uint32_t *wa = (const uint32_t *)s.data + ga * BITS, *wb = (const uint32_t *)s.data + gb * BITS;
+        uint32_t a[BITS], b[BITS];
+#pragma unroll
+        for (int i = 0; i < BITS; ++i) {
+          a[i] = wa[i];
+          b[i] = wb[i];
+        }
+        const half2_t s2 = {s.scale[ga], s.scale[gb]}, z2 = {s.zero[ga], s.zero[gb]};
+#pragma unroll
+        for (int i = 0; i < 32; ++i)
+          col[i * RC_ROW] = h2_bits(rc_value<NORMAL>(code_at<BITS>(a[i / PF], i % PF), code_at<BITS>(b[i / PF], i % PF), s2, z2));
+      }
+    }
+    __syncthreads();
+    const int P = min(RC_CH, D - c0) >> 3;
+    for (int i = threadIdx.x; i < RC_TOK * P; i += RC_THREADS) {
+      const int tl = i / P, cp = i % P, t = t0 + tl;
+      if (t >= n) break;
+      const int64_t p = rc_position(s, t, T);
+      if (p >= 0) *reinterpret_cast<uint4 *>(s.out + (bh * T + p) * D + c0 + cp * 8) = *reinterpret_cast<const uint4 *>(tile + tl * RC_ROW + cp * 4);
+    }
+    if (c0 + RC_CH < D) __syncthreads();
+  }
+}
+
+__global__ __launch_bounds__(RC_THREADS, 4) void cache_reconstruct_kernel(RcTable tb, int D, int64_t T) {
+  __shared__ __align__(16) uint32_t tile[RC_TOK * RC_ROW];
+  int si = -1, first = 0;
+#pragma unroll
+  for (int k = 0; k < RC_SEGS; ++k) {
+    const bool in = (int)blockIdx.y >= tb.begin[k];
+    si += in ? 1 : 0;
+    first = in ? tb.begin[k] : first;
+  }
+  const RcSeg s = tb.seg[si];
+  const int64_t bh = blockIdx.x;
+  const int t0 = ((int)blockIdx.y - first) * RC_TOK;
+#define HQ_RC(B_, N_) \
+  if (s.kind & 1) rc_token_major<B_, N_>(s, bh, t0, D, T); else rc_channel_major<B_, N_>(s, bh, t0, D, T, tile)
+  switch (s.bits) {
+    case 16: HQ_RC(16, false); break;
+    case 8: HQ_RC(8, false); break;
+    case 4: HQ_RC(4, false); break;
+    case 2: HQ_RC(2, false); break;
+    default:
+      if (s.kind & 2) { HQ_RC(1, true); } else { HQ_RC(1, false); }
+  }
+#undef HQ_RC
+}
+
+// One bit per position: a position outside [0, n) or whose bit is set already raises status.  With as many indices as
+// positions, no complaint means every position is named once.
+struct CoverArgs {
+  const int64_t *idx[HQEKV_MAX_SEGS];
+  int64_t begin[HQEKV_MAX_SEGS];   // first of the back-to-back numbering; INT64_MAX past the last array
+};
+__global__ __launch_bounds__(256) void cover_once_kernel(CoverArgs a, int64_t n, uint32_t *status, uint32_t *bits) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  const int64_t *src = a.idx[0];
+  int64_t first = 0;
+#pragma unroll
+  for (int k = 1; k < HQEKV_MAX_SEGS; ++k) {
+    const bool in = i >= a.begin[k];
+    src = in ? a.idx[k] : src;
+    first = in ? a.begin[k] : first;
+  }
+  const int64_t p = src[i - first];
+  const uint32_t bit = 1u << (p & 31);
+  if (p < 0 || p >= n || (atomicOr(bits + (p >> 5), bit) & bit)) *status = 1u;
+}
+
+}  // namespace hq
+
+using namespace hq;
+
+extern "C" int hqekv_cover_once(const int64_t *const *idx, const int64_t *counts, int n_arrays, void *scratch, int64_t scratch_bytes,
+                                void *stream) {
+  if (n_arrays <= 0 || n_arrays > HQEKV_MAX_SEGS || !idx || !counts || !scratch) return fail(HQEKV_E_ARG, "cover_once: bad arrays");
+  CoverArgs a{};
+  int64_t n = 0;
+  for (int k = 0; k < HQEKV_MAX_SEGS; ++k) {
+    if (k < n_arrays && (counts[k] < 0 || (counts[k] > 0 && !idx[k]))) return fail(HQEKV_E_ARG, "cover_once: bad array %d", k);
+    a.idx[k] = k < n_arrays ? idx[k] : nullptr;
+    a.begin[k] = k < n_arrays ? n : 0x7fffffffffffffffLL;
+    if (k < n_arrays) n += counts[k];
+  }
+  if (n == 0) return HQEKV_OK;
+  if (n > (1LL << 38)) return fail(HQEKV_E_UNSUPPORTED, "cover_once: too many positions");
+  if ((uintptr_t)scratch & 3) return fail(HQEKV_E_ALIGN, "cover_once: scratch not 4-byte aligned");
+  if (scratch_bytes < 4 * (1 + (n + 31) / 32)) return fail(HQEKV_E_WORKSPACE, "cover_once: scratch too small");
+  hipLaunchKernelGGL(cover_once_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream, a, n,
+                     (uint32_t *)scratch, (uint32_t *)scratch + 1);
+  return check_launch("cover_once_kernel");
+}
+
+extern "C" int hqekv_cache_reconstruct(const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_segs, int n_v, void *K, void *V,
+                                       int64_t BH, int64_t D, int64_t T, void *stream) {
+  if (n_k < 0 || n_k > HQEKV_MAX_SEGS || n_v < 0 || n_v > HQEKV_MAX_SEGS || (n_k && (!k_segs || !K)) || (n_v && (!v_segs || !V)))
+    return fail(HQEKV_E_ARG, "cache_reconstruct: bad segment tables");
+  if (BH <= 0 || BH > 0x7fffffffLL || D <= 0 || D % 32 != 0 || D > 4096 || T < 0)
+    return fail(HQEKV_E_ARG, "cache_reconstruct: need B*H > 0 and head_dim a multiple of 32 up to 4096");
+  if (((uintptr_t)K | (uintptr_t)V) & 15) return fail(HQEKV_E_ALIGN, "cache_reconstruct: dense tensors must be 16-byte aligned");
+  RcTable tb{};
+  int m = 0;
+  int64_t tiles = 0;
+  for (int k = 0; k < n_k + n_v; ++k) {
+    const bool is_k = k < n_k;
+    const hqekv_seg &s = is_k ? k_segs[k] : v_segs[k - n_k];
+    if (s.n_tokens < 0 || s.n_tokens >= (1LL << 30)) return fail(HQEKV_E_ARG, "cache_reconstruct: segment %d: bad n_tokens", k);
+    if (s.n_tokens == 0) continue;
+    if (!(s.bits == 16 || s.bits == 8 || s.bits == 4 || s.bits == 2 || s.bits == 1))
+      return fail(HQEKV_E_ARG, "cache_reconstruct: segment %d bits=%d", k, s.bits);
+    if (!s.data || (s.bits != 16 && (!s.scale || !s.zero))) return fail(HQEKV_E_ARG, "cache_reconstruct: segment %d lacks data / scale / zero", k);
+    if ((uintptr_t)s.data & (s.bits == 16 ? 15 : 3)) return fail(HQEKV_E_ALIGN, "cache_reconstruct: segment %d data misaligned", k);
+    const bool tm = !is_k || (s.bits == 16 && s.layout == HQEKV_LAYOUT_TOKEN_MAJOR);
+    if (!tm && s.bits != 16 && s.n_tokens % 32) return fail(HQEKV_E_ARG, "cache_reconstruct: segment %d n_tokens not a multiple of 32", k);
+    if (s.slab_tokens != 0 && (s.slab_tokens < s.n_tokens || !tm))
+      return fail(HQEKV_E_ARG, "cache_reconstruct: segment %d: slab_tokens applies to token-major segments and must be >= n_tokens", k);
+    RcSeg &r = tb.seg[m];
+    r.data = s.data;
+    r.scale = (const half_t *)s.scale;
+    r.zero = (const half_t *)s.zero;
+    r.idx = s.idx;
+    r.out = (half_t *)(is_k ? K : V);
+    r.pos_base = s.pos_base;
+    r.slab_tokens = s.slab_tokens > 0 ? s.slab_tokens : s.n_tokens;
+    r.n_tokens = (int32_t)s.n_tokens;
+    r.bits = (int16_t)s.bits;
+    r.kind = (int16_t)((tm ? 1 : 0) | (s.bits == 1 && s.layout == HQEKV_LAYOUT_NORMAL1 ? 2 : 0));
+    tb.begin[m++] = (int32_t)tiles;
+    tiles += (s.n_tokens + RC_TOK - 1) / RC_TOK;
+    if (tiles > 65535) return fail(HQEKV_E_UNSUPPORTED, "cache_reconstruct: more than 65535 tiles of %d tokens", RC_TOK);
+  }
+  for (int k = m; k < RC_SEGS; ++k) tb.begin[k] = 0x7fffffff;
+  if (tiles == 0) return HQEKV_OK;
+  hipLaunchKernelGGL(cache_reconstruct_kernel, dim3((unsigned)BH, (unsigned)tiles), dim3(RC_THREADS), 0, (hipStream_t)stream, tb, (int)D, T);
+  return check_launch("cache_reconstruct_kernel");
+}

@@ -392,6 +392,21 @@ typedef struct hqekv_cache_class {
 int hqekv_cache_migrate(int is_k, const hqekv_cache_class *src, int n_src, const hqekv_cache_class *dst,
                         int n_dst, const int32_t *plan, int64_t BH, int64_t D, int32_t *status, void *stream);
 
+/* A hybrid cache back into dense fp16 K and V, (B,Hkv,T,D) each (BH = B * Hkv): every segment dequantised with the two
+ * fp16 roundings and written to its positions, one launch.  Replaces the dequantise / index_put sequence of
+ * KV_cache_reconstruct (quant/hybrid_quant.py:732-846) and KV_cache_reconstruct_hqe (quant/hqe_2.py:967-1084).  A position
+ * nobody names is not written; one named twice within a call holds either value; one outside [-T, T) is dropped.
+ */
+int hqekv_cache_reconstruct(const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_segs, int n_v, void *K, void *V,
+                            int64_t BH, int64_t D, int64_t T, void *stream);
+
+/* Do the index arrays (device; at most HQEKV_MAX_SEGS), taken together, name every position in [0, sum of counts) exactly
+ * once?  scratch: one int32 status and one bit per position, 4 * (1 + ceil(n / 32)) bytes the caller has zeroed; status is
+ * non-zero afterwards when a position is out of range or named twice.
+ */
+int hqekv_cover_once(const int64_t *const *idx, const int64_t *counts, int n_arrays, void *scratch, int64_t scratch_bytes,
+                     void *stream);
+
 /* The plan for hqekv_cache_migrate, worked out on the HOST (every pointer here is a host pointer; nothing is launched).
  * Replaces the class-by-class selection of one compression (quant/hqe_2.py:552-659 for K, :672-836 for V: torch.isin
  * masks per (source, target) pair) and the re-ranking of the positions after an eviction (:661-670) by their outcome.

@@ -1,0 +1,67 @@
+"""A hybrid cache back into dense K and V in one launch against the oracle's class-by-class restoration, bit for bit."""
+import pytest
+import torch
+
+from hqekv_amd import synth
+from oracle import hqe_oracle as O
+
+pytestmark = pytest.mark.gpu
+LOW_NORMAL = "high_uniform_group_low_normal_group"
+
+
+def _cache(dev, B, H, T, D, residual, fractions, strategy, seed=5):
+    from hqekv_amd import pack_unpack as PU
+
+    def quantize(x, group, bits):
+        if bits == 1 and strategy == LOW_NORMAL:
+            return PU.normal_group_quantize_pack_last_dim(x, group, 1)
+        return PU.uniform_group_quantize_pack_last_dim(x, group, bits)
+    _, K, V = synth.make_qkv(B, H, H, T + residual, D, seed, dev)
+    return synth.build_cache(K, V, synth.split_blocks(T, fractions, seed), residual, quantize)
+
+
+def _check(pkv, strategy):
+    from hqekv_amd.hqe_2 import KV_cache_reconstruct_hqe
+    got = KV_cache_reconstruct_hqe(pkv, strategy)
+    want = O.reconstruct_cache(synth.cache_to(pkv, "cpu"), strategy)
+    for g, w, side in zip(got, want, "KV"):
+        assert torch.equal(g.cpu().view(torch.int16), w.contiguous().view(torch.int16)), side
+
+
+@pytest.mark.parametrize("strategy", ["uniform_group", LOW_NORMAL])
+@pytest.mark.parametrize("B,H,T,D,residual,fractions", [
+    (1, 1, 32, 128, 0, (0, 0, 0, 1, 0, 0)),                      # one group of one class
+    (2, 3, 1056, 128, 17, (.1, .2, .2, .2, .2, .1)),             # every class, ragged tiles, a residual
+    (1, 2, 4096, 128, 63, (.05, .15, .3, .2, .1, .2)),
+    (1, 2, 416, 64, 1, (.2, .2, .2, .2, .1, .1)),                # other head sizes: half a channel tile, one and a half
+    (1, 2, 416, 192, 3, (.2, .2, .2, .2, .1, .1)),
+])
+def test_every_class(dev, B, H, T, D, residual, fractions, strategy):
+    _check(_cache(dev, B, H, T, D, residual, fractions, strategy), strategy)
+
+
+def test_positions_nobody_names_are_zero(dev):
+    """kv_seq_len beyond the kept tokens (it counts evicted ones), an absent side, a class of a ragged token count."""
+    pkv = _cache(dev, 1, 2, 512, 128, 5, (.2, .2, .2, .2, .2), "uniform_group")
+    _check(pkv[:41] + (pkv[41] + 100,), "uniform_group")
+    ragged = list(pkv)
+    ragged[0], ragged[1] = pkv[0][..., :45].contiguous(), pkv[1][:45].contiguous()
+    ragged[2], ragged[3] = pkv[2][:, :, :45].contiguous(), pkv[3][:45].contiguous()
+    _check(tuple(ragged), "uniform_group")
+    ragged[4:8] = [None] * 4
+    _check(tuple(ragged), "uniform_group")
+
+
+@pytest.mark.parametrize("n", [1, 31, 32, 257, 5000])
+def test_cover_check(dev, n):
+    from hqekv_amd.attention import idx_cover_once
+    p = torch.randperm(n, generator=torch.Generator().manual_seed(n))
+    cut = n // 3
+
+    def parts(x):
+        return [t for t in (x[:cut].to(dev), x[cut:].to(dev)) if t.numel()]
+    assert idx_cover_once(parts(p), n)
+    for bad in (-1, n, int(p[-1])):
+        q = p.clone()
+        q[0] = bad
+        assert idx_cover_once(parts(q), n) == (bad == int(p[0]))
