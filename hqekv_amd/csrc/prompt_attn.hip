@@ -24,13 +24,19 @@ typedef __attribute__((address_space(3))) h4raw_t lds_h4_t;
 constexpr int PA_D = 128;
 constexpr int PA_WAVES = 4;
 constexpr int PA_THREADS = 64 * PA_WAVES;
-constexpr int PA_BR = 32 * PA_WAVES;   // query rows per workgroup
-#ifndef HQ_PA_BC
-#define HQ_PA_BC 32
-#endif
-constexpr int PA_BC = HQ_PA_BC;        // keys per tile: 32 (164 registers, 32 KB of LDS: three workgroups per CU) or 64 (two)
-constexpr int PA_NS = PA_BC / 32;      // 32-key score tiles per key tile
-constexpr int PA_WGS = PA_BC == 64 ? 2 : 3;
+constexpr int PA_BC = 32;              // keys per score tile
+// How the four waves of a workgroup share its work.  KS = 1: 32 query rows each, 128 per workgroup, every wave walks all
+// key tiles (164 registers, 32 KB of LDS: three workgroups per CU).  KS = 2: the two waves of 32 query rows deal the key
+// tiles among themselves and merge their maxima, sums and outputs at the end: walks of half the length in twice as many
+// workgroups, for prompts whose 128-row workgroups would leave the chip waiting for the longest of them.  A step stages
+// two tiles, so LDS holds two workgroups per CU.
+template <int KS>
+struct PaShape {
+  static constexpr int ROWS = 128 / KS;            // query rows per workgroup
+  static constexpr int STEP = PA_BC * KS;          // keys staged per step
+  static constexpr int TILE = STEP * PA_D;         // fp16 elements of one staged K (or V) step
+  static constexpr int WGS = KS == 1 ? 3 : 2;
+};
 
 struct PromptArgs {
   const half_t *q, *k, *v;
@@ -40,9 +46,9 @@ struct PromptArgs {
   int64_t v_b, v_h, v_t;
   int64_t o_b, o_h, o_t;
   int32_t Hq, Hkv, T;
+  int32_t BH, by_xcd;      // B * Hq; by_xcd: B * Hkv is a multiple of 8
   float scale;
 };
-
 
 // A tile of keys goes from memory to LDS without passing through registers (`buffer_load_dwordx4 ... lds`: lane l's
 // 16 bytes land at M0 + 16 l, so one wave instruction fills four 256-byte rows).  K and V are both row-major in LDS,
@@ -73,44 +79,49 @@ struct PaSource {
   uint32_t k_lane, v_lane;   // this thread's byte offsets inside a tile (row tid / 16, swizzled piece)
   uint32_t k_row, v_row;     // bytes between two keys
 };
-// rows tid / 16 + 16 i of the tile; wave w's instruction i fills rows 16 i + 4 w .. + 3
+// rows tid / 16 + 16 i of the step; wave w's instruction i fills rows 16 i + 4 w .. + 3
+template <int KEYS>
 __device__ __forceinline__ void pa_tile_dma(const PaSource &src, int k0, const half_t *ks, const half_t *vs, int w) {
   const uint32_t kb = lds_offset_of(ks) + (uint32_t)w * 1024u, vb = lds_offset_of(vs) + (uint32_t)w * 1024u;
 #pragma unroll
-  for (int i = 0; i < PA_BC / 16; ++i) {
+  for (int i = 0; i < KEYS / 16; ++i) {
     dma_1k(kb + 4096u * i, src.k, src.k_lane, (uint32_t)(k0 + 16 * i) * src.k_row);
     dma_1k(vb + 4096u * i, src.v, src.v_lane, (uint32_t)(k0 + 16 * i) * src.v_row);
   }
 }
 
-// S^T of one key tile for the wave's 32 queries: PA_NS score tiles of 32 keys, 16 fp32 values per lane each
-__device__ __forceinline__ void pa_scores(const half_t *ks, const h8_t (&qreg)[8], int n, int h, f16_t (&sc)[PA_NS]) {
-#pragma unroll
-  for (int mt = 0; mt < PA_NS; ++mt) sc[mt] = (f16_t)(0.f);
+// S^T of one key tile for the wave's 32 queries: 16 fp32 values per lane
+__device__ __forceinline__ f16_t pa_scores(const half_t *ks, const h8_t (&qreg)[8], int n, int h) {
+  f16_t sc = (f16_t)(0.f);
 #pragma unroll
   for (int s = 0; s < 8; ++s) {
-    const int piece = ((2 * s + h) ^ (n & 15)) * 8;   // (rows n and 32 + n share the swizzle)
-#pragma unroll
-    for (int mt = 0; mt < PA_NS; ++mt) {
-      const h8_t kk = *reinterpret_cast<const h8_t *>(ks + (32 * mt + n) * PA_D + piece);
-      sc[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kk, qreg[s], sc[mt], 0, 0, 0);
-    }
+    const h8_t kk = *reinterpret_cast<const h8_t *>(ks + n * PA_D + ((2 * s + h) ^ (n & 15)) * 8);
+    sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(kk, qreg[s], sc, 0, 0, 0);
   }
+  return sc;
 }
-template <bool CAUSAL>
-__global__ __launch_bounds__(PA_THREADS, PA_WGS) void prompt_attn_kernel(PromptArgs a) {
-  __shared__ __align__(16) half_t ks_all[2][PA_BC * PA_D];
-  __shared__ __align__(16) half_t vs_all[2][PA_BC * PA_D];
+template <bool CAUSAL, int KS>
+__global__ __launch_bounds__(PA_THREADS, PaShape<KS>::WGS) void prompt_attn_kernel(PromptArgs a) {
+  using S = PaShape<KS>;
+  __shared__ __align__(16) half_t ks_all[2][S::TILE];
+  __shared__ __align__(16) half_t vs_all[2][S::TILE];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n = lane & 31, h = lane >> 5;
-  const int qb = (int)gridDim.x - 1 - (int)blockIdx.x;   // the longest rows first
-  const int q0 = qb * PA_BR;
-  const int b = (int)blockIdx.y / a.Hq, hq = (int)blockIdx.y % a.Hq, hkv = hq / (a.Hq / a.Hkv);
+  const int rg = w / KS, sp = w % KS;   // this wave's 32 rows of the workgroup, its share of the key tiles
+  // The grid is one-dimensional, longest rows first over ALL heads (a causal walk's length grows with its row: the short
+  // ones fill the gaps at the end).  Workgroup i runs on XCD i mod 8: where the KV heads divide evenly among the XCDs,
+  // the query heads of a KV head share one and meet in its L2.  With the rows of one head after the other (a head's row
+  // blocks dealt to all XCDs): T = 32768 9.35 -> 8.04 ms, 8192 0.73 -> 0.57 ms, 4099 196 -> 165 us (32 heads over 8).
+  const int nrep = a.Hq / a.Hkv;
+  const int qi = (int)blockIdx.x / a.BH, slot = (int)blockIdx.x % a.BH;
+  const int bh = a.by_xcd ? ((slot / 8 / nrep) * 8 + slot % 8) * nrep + slot / 8 % nrep : slot;
+  const int q0 = ((int)gridDim.x / a.BH - 1 - qi) * S::ROWS;
+  const int b = bh / a.Hq, hq = bh % a.Hq, hkv = hq / nrep;
   const int T = a.T;
   const half_t *qp = a.q + b * a.q_b + hq * a.q_h;
   const half_t *kp = a.k + b * a.k_b + hkv * a.k_h;
   const half_t *vp = a.v + b * a.v_b + hkv * a.v_h;
-  const int my_q = q0 + 32 * w + n;
+  const int my_q = q0 + 32 * rg + n;
   // the lane's query row: 8 steps of 16 channels, of which it supplies 8 (by lane half)
   h8_t qreg[8];
   {
@@ -123,21 +134,21 @@ __global__ __launch_bounds__(PA_THREADS, PA_WGS) void prompt_attn_kernel(PromptA
   for (int dt = 0; dt < 4; ++dt) o[dt] = (f16_t)(0.f);
   float m = -INFINITY, lsum = 0.f;
   const float sl2 = a.scale * 1.4426950408889634f;
-  const int kend = CAUSAL ? min(T, q0 + PA_BR) : T;
-  const int n_tiles = (kend + PA_BC - 1) / PA_BC;
+  const int kend = CAUSAL ? min(T, q0 + S::ROWS) : T;
+  const int n_steps = (kend + S::STEP - 1) / S::STEP;
   PaSource src;
   src.k = make_desc(kp, (uint32_t)((int64_t)T * a.k_t * 2));   // (below 4 GiB: checked by the host)
   src.v = make_desc(vp, (uint32_t)((int64_t)T * a.v_t * 2));
   src.k_row = (uint32_t)a.k_t * 2u;
   src.v_row = (uint32_t)a.v_t * 2u;
   {
-    const uint32_t row = threadIdx.x >> 4, slot = threadIdx.x & 15;
-    src.k_lane = row * src.k_row + ((slot ^ (row & 15)) * 16u);
-    src.v_lane = row * src.v_row + ((slot ^ (4 * (row & 3))) * 16u);
+    const uint32_t row = threadIdx.x >> 4, slot16 = threadIdx.x & 15;
+    src.k_lane = row * src.k_row + ((slot16 ^ (row & 15)) * 16u);
+    src.v_lane = row * src.v_row + ((slot16 ^ (4 * (row & 3))) * 16u);
   }
-  // Two tiles in LDS, one barrier per tile: iteration j waits for its own requests of tile j (made an iteration ago),
-  // passes the barrier -- now every wave's part of tile j is there and every wave has finished tile j - 1 -- requests
-  // tile j + 1 into the buffer that tile j - 1 was read from, and works on tile j.
+  // Two steps' tiles in LDS, one barrier per step: iteration j waits for its own requests of step j (made an iteration
+  // ago), passes the barrier -- now every wave's part of step j is there and every wave has finished step j - 1 --
+  // requests step j + 1 into the buffer that step j - 1 was read from, and works on its tile of step j.
   // where this lane points the transposing reads of V: lane r of a group of 16 names key row 4h + r / 4 of a step and
   // the 8 bytes of channels 32 dt + 16 (n / 16) + 4 (r % 4) ..; the row's pieces are swizzled by 4 (row % 4) = 4 (r / 4)
   int v_off[4];
@@ -152,36 +163,33 @@ __global__ __launch_bounds__(PA_THREADS, PA_WGS) void prompt_attn_kernel(PromptA
   // (rows past the end of the prompt are outside the buffer descriptors: whatever such a row holds in LDS -- zeros from
   // this fill or an older tile's finite values -- meets an exponential that is exactly zero)
 #pragma unroll
-  for (int i = 0; i < PA_BC / 8; ++i) *reinterpret_cast<uint4 *>(&vs_all[0][0] + (threadIdx.x + PA_THREADS * i) * 8) = make_uint4(0, 0, 0, 0);
+  for (int i = 0; i < 4 * KS; ++i) *reinterpret_cast<uint4 *>(&vs_all[0][0] + (threadIdx.x + PA_THREADS * i) * 8) = make_uint4(0, 0, 0, 0);
   __syncthreads();
-  pa_tile_dma(src, 0, ks_all[0], vs_all[0], w);   // (a tile past the last one is fetched and never used)
-  auto step = [&](int tile, const half_t *ks, const half_t *vs, half_t *ks_nxt, half_t *vs_nxt) {
-    const int k0 = tile * PA_BC;
-    wait_all_loads();   // this wave's part of tile j, requested an iteration ago
+  pa_tile_dma<S::STEP>(src, 0, ks_all[0], vs_all[0], w);   // (a step past the last one is fetched and never used)
+  auto step = [&](int j, const half_t *ks, const half_t *vs, half_t *ks_nxt, half_t *vs_nxt) {
+    const int k0 = j * S::STEP + sp * PA_BC;
+    wait_all_loads();   // this wave's part of step j, requested an iteration ago
     __syncthreads();
-    pa_tile_dma(src, k0 + PA_BC, ks_nxt, vs_nxt, w);   // in flight across the products
+    pa_tile_dma<S::STEP>(src, (j + 1) * S::STEP, ks_nxt, vs_nxt, w);   // in flight across the products
+    ks += sp * PA_BC * PA_D;
+    vs += sp * PA_BC * PA_D;
     // (a tile that lies after every query of this wave is worked through like any other: all its elements are masked,
     // the maximum stays and the exponentials are zeros; skipping it would cost a copy of the accumulators per tile)
-    f16_t s[PA_NS];
-    pa_scores(ks, qreg, n, h, s);
-    const bool edge = (k0 + PA_BC > T) || (CAUSAL && k0 + PA_BC - 1 > q0 + 32 * w);   // some element of the tile is masked
+    f16_t s = pa_scores(ks, qreg, n, h);
+    const bool edge = (k0 + PA_BC > T) || (CAUSAL && k0 + PA_BC - 1 > q0 + 32 * rg);   // some element of the tile is masked
     // the running maximum is kept in units of the scaled logit (base-2 exponent); a raw score enters as s * sl2
-    if (edge) {   // (uniform per wave; one branch around all 32 selects)
+    if (edge) {   // (uniform per wave; one branch around all 16 selects)
       const int last_key = (CAUSAL ? min(my_q, T - 1) : T - 1) - k0 - 4 * h;   // the last visible key, relative to element r's base
 #pragma unroll
-      for (int mt = 0; mt < PA_NS; ++mt)
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-          if (32 * mt + 8 * (r >> 2) + (r & 3) > last_key) s[mt][r] = -INFINITY;
+      for (int r = 0; r < 16; ++r)
+        if (8 * (r >> 2) + (r & 3) > last_key) s[r] = -INFINITY;
     }
     float raw = -INFINITY;
 #pragma unroll
-    for (int mt = 0; mt < PA_NS; ++mt)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) raw = fmaxf(raw, s[mt][r]);
+    for (int r = 0; r < 16; ++r) raw = fmaxf(raw, s[r]);
     float mx = fmaxf(m, raw * sl2);   // (sl2 > 0)
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    // (the first tile always holds key 0, which no query masks: mx is finite from then on)
+    // (KS = 1: the first tile always holds key 0, which no query masks: mx is finite from then on)
     // Per lane on purpose: a divergent branch keeps the accumulators where they are (inactive lanes must keep their
     // values, so the products are in place under the execution mask, skipped when no lane needs them); a wave-uniform
     // branch made the compiler copy all 64 accumulators per tile, and without a branch the 64 products are a quarter
@@ -193,19 +201,18 @@ __global__ __launch_bounds__(PA_THREADS, PA_WGS) void prompt_attn_kernel(PromptA
       for (int dt = 0; dt < 4; ++dt) o[dt] *= alpha;
       m = mx;
     }
+    const float base = KS > 1 && mx == -INFINITY ? 0.f : mx;   // nothing but masked keys so far: exponentials of -inf are zero
     float part = 0.f;
-    h8_t p[2 * PA_NS];
+    h8_t p[2];
 #pragma unroll
-    for (int mt = 0; mt < PA_NS; ++mt)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(s[mt][r], sl2, -mx));
-        part += e;
-        p[2 * mt + (r >> 3)][r & 7] = (half_t)e;
-      }
+    for (int r = 0; r < 16; ++r) {
+      const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], sl2, -base));
+      part += e;
+      p[r >> 3][r & 7] = (half_t)e;
+    }
     lsum += part;
 #pragma unroll
-    for (int t = 0; t < 2 * PA_NS; ++t)
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int dt = 0; dt < 4; ++dt) {
         // V^T operand through the transposing LDS read: a group of 16 lanes names four key rows x 32 bytes and each
@@ -219,14 +226,35 @@ __global__ __launch_bounds__(PA_THREADS, PA_WGS) void prompt_attn_kernel(PromptA
         o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av, p[t], o[dt], 0, 0, 0);
       }
   };
-  // two tiles per round, so that each half works on fixed buffers; an odd count runs one tile more, all of it masked
-  for (int tile = 0; tile < n_tiles; tile += 2) {
-    step(tile, ks_all[0], vs_all[0], ks_all[1], vs_all[1]);
-    step(tile + 1, ks_all[1], vs_all[1], ks_all[0], vs_all[0]);
+  // two steps per round, so that each half works on fixed buffers; an odd count runs one step more, all of it masked
+  for (int j = 0; j < n_steps; j += 2) {
+    step(j, ks_all[0], vs_all[0], ks_all[1], vs_all[1]);
+    step(j + 1, ks_all[1], vs_all[1], ks_all[0], vs_all[0]);
   }
-  wait_all_loads();   // the last request (a tile nobody reads) must have landed before this workgroup's LDS can go to another
+  wait_all_loads();   // the last request (a step nobody reads) must have landed before this workgroup's LDS can go to another
   lsum += __shfl_xor(lsum, 32, 64);
-  if (my_q < T) {
+  if constexpr (KS > 1) {
+    // The second wave of a row group leaves (maximum, sum, output) in LDS for the first.  A lane's 64 outputs go to words
+    // 64 apart, lanes adjacent: no bank conflicts.
+    float *pool_o = reinterpret_cast<float *>(&ks_all[0][0]) + rg * 64 * 64;
+    float2 *pool_ml = reinterpret_cast<float2 *>(&vs_all[0][0]) + rg * 64;
+    static_assert(KS == 2 && (4 / KS) * 64 * 64 * 4 <= (int)sizeof(ks_all), "one sender per row group");
+    __syncthreads();   // the tiles are no longer read
+    if (sp == 1) {
+      pool_ml[lane] = make_float2(m, lsum);
+#pragma unroll
+      for (int i = 0; i < 64; ++i) pool_o[i * 64 + lane] = o[i >> 4][i & 15];
+    }
+    __syncthreads();
+    if (sp == 0) {   // (its tiles start with key 0: m is finite; the other's may all have been masked)
+      const float2 ml = pool_ml[lane];
+      const float mx = fmaxf(m, ml.x), ca = __builtin_amdgcn_exp2f(m - mx), cb = __builtin_amdgcn_exp2f(ml.x - mx);
+      lsum = lsum * ca + ml.y * cb;
+#pragma unroll
+      for (int i = 0; i < 64; ++i) o[i >> 4][i & 15] = o[i >> 4][i & 15] * ca + pool_o[i * 64 + lane] * cb;
+    }
+  }
+  if (sp == 0 && my_q < T) {
     const float inv = 1.0f / lsum;
     half_t *orow = a.out + b * a.o_b + hq * a.o_h + (int64_t)my_q * a.o_t;
 #pragma unroll
@@ -254,14 +282,63 @@ struct LastRowsArgs {
   int64_t m_b, m_r;
   int32_t Hq, Hkv, T, R;
   float scale;
-  float2 *partial;      // (B * Hq, slices, 32) (maximum, sum) of a slice of the keys, or nullptr: one workgroup per head does it all
+  float2 *partial;      // (B * Hq, R, slices) (maximum, sum) of a slice of the keys, or nullptr: one workgroup per head does it all
   int32_t slices;
 };
 
-// PHASE 0: one workgroup per (b, query head) walks all keys twice.  With the keys cut into slices (grid.y) for short
-// prompts and small batches: PHASE 1 leaves each slice's (maximum, sum) per row in `partial`, PHASE 2 merges them and
-// writes the slice's probabilities.
-template <int PHASE>
+// One score tile's 16 values per lane, as the reference's fp16 chain leaves them: query column `my_q` (its mask row
+// `mrow`, or the causal rule) against keys 32 * tile + 8 (r / 4) + 4 h + r % 4; -inf where no key is visible.
+__device__ __forceinline__ void lr_logits(const LastRowsArgs &a, f16_t s, const half_t *mrow, int tile, int h, int my_q, half_t (&x)[16]) {
+  const half_t none = (half_t)-INFINITY;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const int key = 32 * tile + 8 * (r >> 2) + 4 * h + (r & 3);
+    half_t v = (half_t)((float)(half_t)s[r] * a.scale);
+    if (mrow) {
+      v = (half_t)((float)v + (float)mrow[min(key, a.T - 1)]);
+      v = (half_t)fmaxf((float)v, -65504.f);
+      x[r] = key < a.T ? v : none;
+    } else {
+      x[r] = (key < a.T && key <= my_q) ? v : none;
+    }
+  }
+}
+__device__ __forceinline__ void lr_load_keys(const half_t *kp, int64_t k_t, int T, int tile, int n, int h, h8_t (&k)[8]) {
+  const half_t *kr = kp + (int64_t)min(32 * tile + n, T - 1) * k_t + 8 * h;
+#pragma unroll
+  for (int st = 0; st < 8; ++st) k[st] = *reinterpret_cast<const h8_t *>(kr + 16 * st);
+}
+// running (maximum, sum) over one tile
+__device__ __forceinline__ void lr_tile_stats(const half_t (&x)[16], float &m, float &l) {
+  float mx = m;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) mx = fmaxf(mx, (float)x[r]);
+  if (mx == -INFINITY) return;   // nothing but masked keys so far
+  float part = 0.f;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) part += __expf((float)x[r] - mx);
+  l = l * __expf(m - mx) + part;
+  m = mx;
+}
+// over the two halves of every wave, then the four waves: afterwards every thread holds column n's pair
+__device__ __forceinline__ void lr_merge(float &m, float &l, int n, int h, int w, float (&sh_m)[PA_WAVES][32], float (&sh_l)[PA_WAVES][32]) {
+  const float mo = __shfl_xor(m, 32, 64), lo = __shfl_xor(l, 32, 64);
+  const float mx = fmaxf(m, mo);
+  l = (m == -INFINITY ? 0.f : l * __expf(m - mx)) + (mo == -INFINITY ? 0.f : lo * __expf(mo - mx));
+  if (h == 0) {
+    sh_m[w][n] = mx;
+    sh_l[w][n] = l;
+  }
+  __syncthreads();
+  m = -INFINITY;
+#pragma unroll
+  for (int k = 0; k < PA_WAVES; ++k) m = fmaxf(m, sh_m[k][n]);
+  l = 0.f;
+#pragma unroll
+  for (int k = 0; k < PA_WAVES; ++k) l += sh_m[k][n] == -INFINITY ? 0.f : sh_l[k][n] * __expf(sh_m[k][n] - m);
+}
+
+// Without room for the slices' statistics: one workgroup per (b, query head) walks all keys twice.
 __global__ __launch_bounds__(PA_THREADS, 2) void prompt_last_rows_kernel(LastRowsArgs a) {
   __shared__ float sh_m[PA_WAVES][32], sh_l[PA_WAVES][32];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -278,88 +355,141 @@ __global__ __launch_bounds__(PA_THREADS, 2) void prompt_last_rows_kernel(LastRow
     for (int s = 0; s < 8; ++s) qreg[s] = *reinterpret_cast<const h8_t *>(qr + 16 * s);
   }
   const half_t *mrow = a.mask ? a.mask + b * a.m_b + (int64_t)row * a.m_r : nullptr;
-  const int all_tiles = (T + 31) / 32;
-  const int per_slice = PHASE == 0 ? all_tiles : (all_tiles + a.slices - 1) / a.slices;
-  const int tile0 = PHASE == 0 ? 0 : (int)blockIdx.y * per_slice, n_tiles = min(all_tiles, tile0 + per_slice);
-  // the 16 scores of this lane for 32-key tile `tile`, as the reference's fp16 chain leaves them (in fp32)
-  auto tile_scores = [&](int tile, float (&x)[16]) {
-    const int key_row = min(32 * tile + n, T - 1);
-    const half_t *kr = kp + (int64_t)key_row * a.k_t + 8 * h;
+  const int n_tiles = (T + 31) / 32;
+  auto tile_logits = [&](int tile, half_t (&x)[16]) {
+    h8_t k[8];
+    lr_load_keys(kp, a.k_t, T, tile, n, h, k);
     f16_t s = (f16_t)(0.f);
 #pragma unroll
-    for (int st = 0; st < 8; ++st)
-      s = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const h8_t *>(kr + 16 * st), qreg[st], s, 0, 0, 0);
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int key = 32 * tile + 8 * (r >> 2) + 4 * h + (r & 3);
-      half_t v = (half_t)((float)(half_t)s[r] * a.scale);
-      if (mrow) {
-        v = (half_t)((float)v + (float)mrow[min(key, T - 1)]);
-        v = (half_t)fmaxf((float)v, -65504.f);
-        x[r] = key < T ? (float)v : -INFINITY;
-      } else {
-        x[r] = (key < T && key <= my_q) ? (float)v : -INFINITY;
-      }
-    }
+    for (int st = 0; st < 8; ++st) s = __builtin_amdgcn_mfma_f32_32x32x16_f16(k[st], qreg[st], s, 0, 0, 0);
+    lr_logits(a, s, mrow, tile, h, my_q, x);
   };
   float m = -INFINITY, l = 0.f;
-  if (PHASE != 2) {
-    for (int tile = tile0 + w; tile < n_tiles; tile += PA_WAVES) {
-      float x[16];
-      tile_scores(tile, x);
-      float mx = m;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) mx = fmaxf(mx, x[r]);
-      if (mx == -INFINITY) continue;   // nothing but masked keys so far
-      float part = 0.f;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) part += __expf(x[r] - mx);
-      l = l * __expf(m - mx) + part;
-      m = mx;
-    }
-    // the two halves of the wave, then the four waves
-    const float mo = __shfl_xor(m, 32, 64), lo = __shfl_xor(l, 32, 64);
-    const float mx = fmaxf(m, mo);
-    l = (m == -INFINITY ? 0.f : l * __expf(m - mx)) + (mo == -INFINITY ? 0.f : lo * __expf(mo - mx));
-    m = mx;
-    if (h == 0) {
-      sh_m[w][n] = m;
-      sh_l[w][n] = l;
-    }
-    __syncthreads();
-    float mx2 = -INFINITY;
-#pragma unroll
-    for (int k = 0; k < PA_WAVES; ++k) mx2 = fmaxf(mx2, sh_m[k][n]);
-    float tot = 0.f;
-#pragma unroll
-    for (int k = 0; k < PA_WAVES; ++k) tot += sh_m[k][n] == -INFINITY ? 0.f : sh_l[k][n] * __expf(sh_m[k][n] - mx2);
-    m = mx2;
-    l = tot;
-    if (PHASE == 1) {
-      if (threadIdx.x < 32) a.partial[((int64_t)blockIdx.x * a.slices + blockIdx.y) * 32 + n] = make_float2(m, l);
-      return;
-    }
-  } else {   // merge the slices' statistics, in slice order
-    const float2 *ps = a.partial + (int64_t)blockIdx.x * a.slices * 32 + n;
-    for (int sl = 0; sl < a.slices; ++sl) m = fmaxf(m, ps[sl * 32].x);
-    for (int sl = 0; sl < a.slices; ++sl) {
-      const float2 v = ps[sl * 32];
-      l += v.x == -INFINITY ? 0.f : v.y * __expf(v.x - m);
-    }
+  for (int tile = w; tile < n_tiles; tile += PA_WAVES) {
+    half_t x[16];
+    tile_logits(tile, x);
+    lr_tile_stats(x, m, l);
   }
+  lr_merge(m, l, n, h, w, sh_m, sh_l);
   const float inv = 1.0f / l;
   half_t *prow = a.probs + (((int64_t)b * a.Hq + hq) * R + row) * (int64_t)T;
-  for (int tile = tile0 + w; tile < n_tiles; tile += PA_WAVES) {
-    float x[16];
-    tile_scores(tile, x);
+  for (int tile = w; tile < n_tiles; tile += PA_WAVES) {
+    half_t x[16];
+    tile_logits(tile, x);
     if (n >= R) continue;
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       const int key = 32 * tile + 8 * g + 4 * h;
 #pragma unroll
       for (int j = 0; j < 4; ++j)
-        if (key + j < T) prow[key + j] = (half_t)(__expf(x[4 * g + j] - m) * inv);
+        if (key + j < T) prow[key + j] = (half_t)(__expf((float)x[4 * g + j] - m) * inv);
     }
+  }
+}
+
+// With that room, two launches.  Bound: HBM (K once, the rows' probabilities twice through the memory-side cache).
+// prompt_last_logits_kernel: the R rows of all query heads of a KV head lie side by side as columns of 32-column tiles
+// (4 heads x 20 rows: three tiles instead of four that are 3/8 empty); a workgroup takes one column tile and one slice of
+// the keys, leaves the logits where the probabilities will be -- four keys of a row per 8-byte store -- and the slice's
+// (maximum, sum) per row.  prompt_last_probs_kernel turns rows of logits into probabilities, 16 bytes per lane.  Walking
+// the keys a second time instead of the stored logits, with slices of 2048 keys and more: 38.8 us at T = 1003 (one slice),
+// 175 us at T = 32768 (32 heads over 8); now 9 us and 72 us.
+struct __attribute__((packed, aligned(2))) lr_quad_t { uint64_t v; };    // four fp16 at an element's alignment
+struct __attribute__((packed, aligned(2))) lr_oct_t { uint64_t v[2]; };  // eight
+__global__ __launch_bounds__(PA_THREADS, 3) void prompt_last_logits_kernel(LastRowsArgs a) {
+  __shared__ float sh_m[PA_WAVES][32], sh_l[PA_WAVES][32];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n = lane & 31, h = lane >> 5;
+  const int b = (int)blockIdx.x / a.Hkv, hkv = (int)blockIdx.x % a.Hkv;
+  const int T = a.T, R = a.R, nrep = a.Hq / a.Hkv;
+  const int col = 32 * (int)blockIdx.z + n;                    // (query head of the group, row)
+  const bool live = col < nrep * R;                            // lanes past the last column repeat it and store nothing
+  const int hq = hkv * nrep + (live ? col : nrep * R - 1) / R, row = (live ? col : nrep * R - 1) % R;
+  const half_t *kp = a.k + b * a.k_b + hkv * a.k_h;
+  const int my_q = T - R + row;
+  h8_t qreg[8];
+  {
+    const half_t *qr = a.q + b * a.q_b + hq * a.q_h + (int64_t)my_q * a.q_t + 8 * h;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) qreg[s] = *reinterpret_cast<const h8_t *>(qr + 16 * s);
+  }
+  const half_t *mrow = a.mask ? a.mask + b * a.m_b + (int64_t)row * a.m_r : nullptr;
+  const int all_tiles = (T + 31) / 32, per_slice = (all_tiles + a.slices - 1) / a.slices;
+  const int tile0 = (int)blockIdx.y * per_slice, n_tiles = min(all_tiles, tile0 + per_slice);
+  half_t *prow = a.probs + (((int64_t)b * a.Hq + hq) * R + row) * (int64_t)T;
+  float m = -INFINITY, l = 0.f;
+  h8_t k[8];
+  lr_load_keys(kp, a.k_t, T, min(tile0 + w, all_tiles - 1), n, h, k);
+#pragma unroll 1
+  for (int tile = tile0 + w; tile < n_tiles; tile += PA_WAVES) {
+    f16_t s = (f16_t)(0.f);
+    h8_t nxt[8];
+    lr_load_keys(kp, a.k_t, T, min(tile + PA_WAVES, all_tiles - 1), n, h, nxt);   // (past the last one: read, not used)
+#pragma unroll
+    for (int st = 0; st < 8; ++st) s = __builtin_amdgcn_mfma_f32_32x32x16_f16(k[st], qreg[st], s, 0, 0, 0);
+    half_t x[16];
+    lr_logits(a, s, mrow, tile, h, my_q, x);
+    lr_tile_stats(x, m, l);
+    if (live) {
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int key = 32 * tile + 8 * g + 4 * h;
+        if (key + 3 < T) {
+          lr_quad_t y;
+          __builtin_memcpy(&y, x + 4 * g, 8);
+          *reinterpret_cast<lr_quad_t *>(prow + key) = y;
+        } else {
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            if (key + j < T) prow[key + j] = x[4 * g + j];
+        }
+      }
+    }
+#pragma unroll
+    for (int st = 0; st < 8; ++st) k[st] = nxt[st];
+  }
+  lr_merge(m, l, n, h, w, sh_m, sh_l);
+  if (threadIdx.x < 32 && live) a.partial[((int64_t)b * a.Hq + hq) * R * a.slices + (int64_t)row * a.slices + blockIdx.y] = make_float2(m, l);
+}
+
+constexpr int LR_SPAN = 2048;   // probabilities of one row per workgroup: 256 lanes x 8
+__global__ __launch_bounds__(PA_THREADS) void prompt_last_probs_kernel(LastRowsArgs a) {
+  __shared__ float sh[2];
+  const int lane = threadIdx.x & 63;
+  half_t *prow = a.probs + (int64_t)blockIdx.y * a.T;
+  const int e0 = (int)blockIdx.x * LR_SPAN + (int)threadIdx.x * 8;
+  const bool whole = e0 + 8 <= a.T;
+  half_t x[8];
+  if (whole) {
+    const lr_oct_t v = *reinterpret_cast<const lr_oct_t *>(prow + e0);
+    __builtin_memcpy(x, &v, 16);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] = e0 + i < a.T ? prow[e0 + i] : (half_t)0;
+  }
+  if (threadIdx.x < 64) {   // the slices' statistics of this row
+    const float2 *ps = a.partial + (int64_t)blockIdx.y * a.slices;
+    const float2 v = lane < a.slices ? ps[lane] : make_float2(-INFINITY, 0.f);   // (at most 64 slices)
+    const float m = wave_max(v.x);
+    const float l = wave_sum(v.x == -INFINITY ? 0.f : v.y * __expf(v.x - m));
+    if (lane == 0) {
+      sh[0] = m;
+      sh[1] = 1.0f / l;
+    }
+  }
+  __syncthreads();
+  const float m = sh[0], inv = sh[1];
+  half_t y[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) y[i] = (half_t)(__expf((float)x[i] - m) * inv);
+  if (whole) {
+    lr_oct_t v;
+    __builtin_memcpy(&v, y, 16);
+    *reinterpret_cast<lr_oct_t *>(prow + e0) = v;
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (e0 + i < a.T) prow[e0 + i] = y[i];
   }
 }
 
@@ -370,6 +500,12 @@ using namespace hq;
 static bool rows_16_byte_aligned(const void *p, int64_t s0, int64_t s1, int64_t s2) {
   return ((uintptr_t)p & 15) == 0 && s0 % 8 == 0 && s1 % 8 == 0 && s2 % 8 == 0;
 }
+
+// Two waves per row group while the 128-row workgroups are fewer than two per CU (up to 480, B = 1 and 32 heads: T up to
+// 1900): T = 1003 29.3 -> 22.8 us, T = 1500 44.8 -> 36.7 us; at 512 it is even (T = 2048 61.0 against 57.3, B = 2 and
+// T = 1003 34.8 against 37.3), at 640 behind (65.5 against 70.5).  Four waves per row group never won (T = 500: 20.0
+// against 12.6 us).
+static int prompt_key_shares(int64_t T, int64_t BH) { return (T + 127) / 128 * BH > 480 ? 1 : 2; }
 
 extern "C" int hqekv_prompt_attn(const void *q, const int64_t *q_strides, const void *k, const int64_t *k_strides,
                                  const void *v, const int64_t *v_strides, void *out, const int64_t *out_strides, int64_t B,
@@ -393,19 +529,28 @@ extern "C" int hqekv_prompt_attn(const void *q, const int64_t *q_strides, const 
   a.v_b = v_strides[0]; a.v_h = v_strides[1]; a.v_t = v_strides[2];
   a.o_b = out_strides[0]; a.o_h = out_strides[1]; a.o_t = out_strides[2];
   a.Hq = (int32_t)Hq; a.Hkv = (int32_t)Hkv; a.T = (int32_t)T; a.scale = scale;
-  const dim3 grid((unsigned)((T + PA_BR - 1) / PA_BR), (unsigned)(B * Hq));
-  if (causal) hipLaunchKernelGGL(prompt_attn_kernel<true>, grid, dim3(PA_THREADS), 0, (hipStream_t)stream, a);
-  else hipLaunchKernelGGL(prompt_attn_kernel<false>, grid, dim3(PA_THREADS), 0, (hipStream_t)stream, a);
+  a.BH = (int32_t)(B * Hq); a.by_xcd = (B * Hkv) % 8 == 0;
+  const int ks = prompt_key_shares(T, B * Hq);
+  const int64_t rows = 128 / ks, wgs = (T + rows - 1) / rows * B * Hq;
+  if (wgs > 0x7fffffffLL) return fail(HQEKV_E_UNSUPPORTED, "prompt_attn: T * B * Hq too large");
+#define LAUNCH(C_, K_) hipLaunchKernelGGL((prompt_attn_kernel<C_, K_>), dim3((unsigned)wgs), dim3(PA_THREADS), 0, (hipStream_t)stream, a)
+#define LAUNCH_K(C_) \
+  if (ks == 1) LAUNCH(C_, 1); else LAUNCH(C_, 2)
+  if (causal) { LAUNCH_K(true); } else { LAUNCH_K(false); }
+#undef LAUNCH_K
+#undef LAUNCH
   return check_launch("prompt_attn");
 }
 
+// Slices of the keys: about 48 (b, query head) slices per column tile's 32 give the chip four to six workgroups per CU;
+// a slice keeps a tile for each of its four waves.  Up to 128 keys the one-launch kernel has nothing to gain from slices.
 static int last_rows_slices(int64_t B, int64_t Hq, int64_t T) {
-  // enough workgroups for the chip when there are few heads; a slice keeps at least 2048 keys
-  int64_t s = (512 + B * Hq - 1) / (B * Hq);
-  const int64_t most = (T + 2047) / 2048;
+  int64_t s = (1536 + B * Hq - 1) / (B * Hq);
+  const int64_t most = (T + 127) / 128;
   if (s > most) s = most;
   if (s > 64) s = 64;
-  return s < 1 ? 1 : (int)s;
+  if (s < 2) s = 2;
+  return T <= 128 || B * Hq * 32 > 65535 ? 1 : (int)s;
 }
 
 extern "C" int64_t hqekv_prompt_last_rows_workspace_bytes(int64_t B, int64_t Hq, int64_t T) {
@@ -438,13 +583,15 @@ extern "C" int hqekv_prompt_last_rows(const void *q, const int64_t *q_strides, c
     if ((uintptr_t)workspace & 7) return fail(HQEKV_E_ALIGN, "prompt_last_rows: workspace not 8-byte aligned");
     a.partial = (float2 *)workspace;
     a.slices = sl;
-    const dim3 grid((unsigned)(B * Hq), (unsigned)sl);
-    hipLaunchKernelGGL(prompt_last_rows_kernel<1>, grid, dim3(PA_THREADS), 0, (hipStream_t)stream, a);
-    hipLaunchKernelGGL(prompt_last_rows_kernel<2>, grid, dim3(PA_THREADS), 0, (hipStream_t)stream, a);
+    const int64_t nrep = Hq / Hkv;
+    hipLaunchKernelGGL(prompt_last_logits_kernel, dim3((unsigned)(B * Hkv), (unsigned)sl, (unsigned)((nrep * R + 31) / 32)), dim3(PA_THREADS), 0,
+                       (hipStream_t)stream, a);
+    hipLaunchKernelGGL(prompt_last_probs_kernel, dim3((unsigned)((T + LR_SPAN - 1) / LR_SPAN), (unsigned)(B * Hq * R)), dim3(PA_THREADS), 0,
+                       (hipStream_t)stream, a);
   } else {
     a.partial = nullptr;
     a.slices = 1;
-    hipLaunchKernelGGL(prompt_last_rows_kernel<0>, dim3((unsigned)(B * Hq)), dim3(PA_THREADS), 0, (hipStream_t)stream, a);
+    hipLaunchKernelGGL(prompt_last_rows_kernel, dim3((unsigned)(B * Hq)), dim3(PA_THREADS), 0, (hipStream_t)stream, a);
   }
   return check_launch("prompt_last_rows");
 }

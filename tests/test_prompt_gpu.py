@@ -185,3 +185,26 @@ def test_last_rows_in_key_slices_equal_the_single_workgroup_form(B, Hq, Hkv, T, 
     torch.testing.assert_close(a.float(), b.float(), rtol=2e-3, atol=2e-6)
     want = _reference_last_rows(q, k, scale, rows, _causal_mask(T, q.device))
     torch.testing.assert_close(a.float(), want.float(), rtol=2e-3, atol=2e-6)
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,T", [
+    (3, 35, 5, 513), (4, 48, 6, 257), (2, 64, 8, 385),                 # one wave per row group; heads over the XCDs or not
+    (1, 8, 8, 33), (1, 8, 8, 65), (1, 28, 4, 96), (8, 16, 2, 384), (1, 40, 8, 1537)])   # two; the last: 520 | 480 around the rule
+@pytest.mark.parametrize("causal", [True, False])
+def test_prompt_attention_on_either_side_of_the_row_group_rule(B, Hq, Hkv, T, causal):
+    from hqekv_amd.prompt_attention import prompt_attention
+    q, k, v = _qkv(B, Hq, Hkv, T, 4000 + T, spread=2.0)
+    out = prompt_attention(q, k, v, 0.09, causal=causal)
+    torch.testing.assert_close(out.float(), _dense(q, k, v, 0.09, causal), rtol=2e-3, atol=2e-3)
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,T,rows", [(1, 4, 1, 128, 20), (1, 4, 1, 129, 20), (2, 28, 4, 257, 20), (1, 40, 8, 2047, 20),
+                                             (1, 8, 8, 2056, 1), (1, 9, 1, 2049, 32), (1, 64, 1, 383, 32)])
+@pytest.mark.parametrize("with_mask", [True, False])
+def test_last_rows_column_tiles_and_slices(B, Hq, Hkv, T, rows, with_mask):
+    """Rows of several heads in one column tile, tiles past the last column, ragged slices, unaligned rows."""
+    from hqekv_amd.prompt_attention import prompt_last_rows
+    q, k, _ = _qkv(B, Hq, Hkv, T, 5000 + T)
+    mask = _causal_mask(T, q.device)
+    got = prompt_last_rows(q, k, 0.09, rows, attention_mask=mask if with_mask else None)
+    torch.testing.assert_close(got.float(), _reference_last_rows(q, k, 0.09, rows, mask).float(), rtol=2e-3, atol=2e-6)
