@@ -46,7 +46,7 @@ EXPORTS = (
     "hqekv_gemv_workspace_bytes", "hqekv_gemv_uniform_group", "hqekv_gemv_normal_group",
     "hqekv_qk_hybrid", "hqekv_scale_softmax", "hqekv_pv_workspace_bytes", "hqekv_pv_hybrid",
     "hqekv_decode_workspace_bytes", "hqekv_decode_attn", "hqekv_decode_attn_static", "hqekv_decode_step", "hqekv_ring_row",
-    "hqekv_importance_scores", "hqekv_weighted_block_scores", "hqekv_token_range",
+    "hqekv_importance_scores", "hqekv_weighted_block_scores", "hqekv_token_range", "hqekv_token_range_append", "hqekv_rank_blocks",
     "hqekv_prompt_attn", "hqekv_prompt_last_rows", "hqekv_prompt_last_rows_workspace_bytes",
     "hqekv_cache_migrate", "hqekv_cache_reconstruct", "hqekv_cover_once", "hqekv_plan_side",
 )
@@ -129,6 +129,8 @@ _PROTOS = {
     "hqekv_importance_scores": (C.c_int, [_vp, C.c_int32, _i64, _i64, _i64, _vp, _vp, _vp]),
     "hqekv_weighted_block_scores": (C.c_int, [_vp, _vp, _i64, _vp, _vp]),
     "hqekv_token_range": (C.c_int, [_vp, _i64, _i64, _i64, _i64, _i64, _vp, _vp]),
+    "hqekv_token_range_append": (C.c_int, [_vp, _i64, _i64, _i64, _i64, _i64, _vp, _i64, _vp, _vp]),
+    "hqekv_rank_blocks": (C.c_int, [_vp, _int, _i64, _vp, _vp]),
     "hqekv_prompt_attn": (C.c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, C.c_float, _int, _vp]),
     "hqekv_prompt_last_rows": (C.c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, C.c_float, _vp, _i64, _vp]),
     "hqekv_prompt_last_rows_workspace_bytes": (_i64, [_i64, _i64, _i64]),

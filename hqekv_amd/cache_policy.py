@@ -573,7 +573,7 @@ def _compress_gather(pkv: tuple, new_K, new_V, res_K, res_V, history: int, compr
     if isinstance(K_sorted_idx, RankedBlocks) and isinstance(V_sorted_idx, RankedBlocks) \
             and K_sorted_idx.scores.numel() == total_blocks == V_sorted_idx.scores.numel() \
             and K_sorted_idx.scores.device == V_sorted_idx.scores.device:
-        both = RankedBlocks.sort_together(K_sorted_idx, V_sorted_idx).to("cpu", torch.int64).numpy()
+        both = RankedBlocks.host_orders(K_sorted_idx, V_sorted_idx)
         k_order_h, v_order_h = both[0], both[1]
     k_ord = getattr(K_sorted_idx, "_hq_block_order", None) if k_order_h is None else None
     v_ord = getattr(V_sorted_idx, "_hq_block_order", None) if v_order_h is None else None

@@ -8,6 +8,8 @@
 //   * a sum over 32 CONTIGUOUS values is a balanced tree over adjacent pairs in fp32;
 //   * every intermediate tensor is fp16: each step rounds to nearest even; a division by 32 is a multiplication by
 //     its (exact) reciprocal; tensor / tensor is the correctly rounded fp32 quotient.
+#include <algorithm>
+
 #include "common.h"
 
 #pragma clang fp contract(off)
@@ -108,6 +110,115 @@ __global__ __launch_bounds__(IMP_THREADS) void token_range_kernel(const half_t *
   }
 }
 
+// The same for rows of whole 16-byte pieces: 16 lanes per (token, slab) row, 16 tokens per workgroup, so a token's rows
+// are a handful of independent 16-byte loads per lane and a reduction stays inside a row of 16 lanes (four DPP steps).
+// Bound by latency at 32 tokens (the later compressions: 8.0 us as one workgroup per token with 2-byte loads and trips
+// through the LDS crossbar; 4.9 us now) and by HBM at a whole prompt's.  Workgroups past the tokens copy the `n_prev` older
+// ranges that the new ones follow.
+constexpr int RANGE_TOK = 16;
+__global__ __launch_bounds__(IMP_THREADS) void token_range_rows_kernel(const half_t *__restrict__ v, int B, int H, int64_t T,
+                                                                      int D, int64_t slab_tokens, half_t *__restrict__ out,
+                                                                      const half_t *__restrict__ prev, int64_t n_prev,
+                                                                      int token_blocks) {
+  if ((int)blockIdx.x >= token_blocks) {
+    half_t *dst = out - n_prev;
+    for (int64_t i = ((int64_t)blockIdx.x - token_blocks) * IMP_THREADS + threadIdx.x; i < n_prev; i += ((int64_t)gridDim.x - token_blocks) * IMP_THREADS)
+      dst[i] = prev[i];
+    return;
+  }
+  __shared__ half_t r[RANGE_MAX_ROWS][RANGE_TOK];
+  const int cp = threadIdx.x & 15, tl = threadIdx.x >> 4;
+  const int64_t t = (int64_t)blockIdx.x * RANGE_TOK + tl, tc = t < T ? t : T - 1;
+  const int rows = B * H;
+  constexpr int U = 4;   // rows in flight per lane
+  for (int row0 = 0; row0 < rows; row0 += U) {
+    float mxs[U], mns[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      mxs[u] = -INFINITY;
+      mns[u] = INFINITY;
+    }
+    for (int d = cp * 8; d < D; d += 128) {
+      uint4 raw[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        raw[u] = *reinterpret_cast<const uint4 *>(v + ((int64_t)min(row0 + u, rows - 1) * slab_tokens + tc) * D + d);
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        half_t x[8];
+        __builtin_memcpy(x, &raw[u], 16);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          mxs[u] = fmaxf(mxs[u], (float)x[i]);
+          mns[u] = fminf(mns[u], (float)x[i]);
+        }
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      float mx = mxs[u], mn = mns[u];
+      mx = fmaxf(mx, dpp_f<0xB1>(mx));
+      mn = fminf(mn, dpp_f<0xB1>(mn));
+      mx = fmaxf(mx, dpp_f<0x4E>(mx));
+      mn = fminf(mn, dpp_f<0x4E>(mn));
+      mx = fmaxf(mx, dpp_f<0x141>(mx));
+      mn = fminf(mn, dpp_f<0x141>(mn));
+      mx = fmaxf(mx, dpp_f<0x140>(mx));
+      mn = fminf(mn, dpp_f<0x140>(mn));
+      if (cp == 0 && row0 + u < rows) r[row0 + u][tl] = (half_t)(mx - mn);
+    }
+  }
+  __syncthreads();
+  const int64_t to = (int64_t)blockIdx.x * RANGE_TOK + threadIdx.x;
+  if (threadIdx.x < RANGE_TOK && to < T) {
+    const float s = sum_rows_like_torch(H, [&](int h) {
+      if (B == 1) return (float)r[h][threadIdx.x];
+      return (float)(half_t)sum_rows_like_torch(B, [&](int b) { return (float)r[b * H + h][threadIdx.x]; });
+    });
+    out[to] = (half_t)s;
+  }
+}
+
+// Stable descending order of every row of scores, NaN first (what torch.sort(descending=True, stable=True) returns): a
+// block's place is the number of blocks that precede it.  A workgroup places 64 blocks; its 16 waves count over a
+// sixteenth of all keys each, read from LDS four at a time (every lane the same ones).  A key is the score's order-
+// preserving 16 bits above the complement of its index, so no two are equal.  Bound by latency: 2 x 1025 scores take
+// 5.8 us (written to host memory), a stack launch and a radix sort of both rows 15 us and their copy to the host 20 more.
+constexpr int RANK_THREADS = 1024, RANK_ITEMS = 64, RANK_MAX = 32768;
+__device__ __forceinline__ uint32_t rank_key(half_t x, int i) {
+  uint32_t u = (uint32_t)__builtin_bit_cast(unsigned short, x);
+  if ((u & 0x7fffu) == 0) u = 0;                     // -0 and +0 are equal
+  u = (u & 0x8000u) ? ~u & 0xffffu : u | 0x8000u;
+  if (x != x) u = 0xffffu;
+  return u << 16 | (0xffffu - (uint32_t)i);
+}
+struct RankRows {
+  const half_t *row[HQEKV_MAX_SEGS];
+};
+__global__ __launch_bounds__(RANK_THREADS) void rank_blocks_kernel(RankRows rows, int n, int32_t *__restrict__ order) {
+  extern __shared__ __align__(16) uint32_t keys[];   // n keys, padded with zeros (below every key) to a multiple of 64
+  __shared__ int counts[RANK_THREADS / 64][RANK_ITEMS];
+  const half_t *row = rows.row[blockIdx.y];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, padded = (n + 63) / 64 * 64;
+  for (int i = threadIdx.x; i < padded; i += RANK_THREADS) keys[i] = i < n ? rank_key(row[i], i) : 0u;
+  __syncthreads();
+  const int i = (int)blockIdx.x * RANK_ITEMS + lane;
+  const uint32_t mine = i < n ? keys[i] : 0xffffffffu;
+  int c = 0;
+  for (int j = 4 * w; j < padded; j += 4 * (RANK_THREADS / 64)) {
+    const uint4 k = *reinterpret_cast<const uint4 *>(keys + j);
+    c += (k.x > mine ? 1 : 0) + (k.y > mine ? 1 : 0) + (k.z > mine ? 1 : 0) + (k.w > mine ? 1 : 0);
+  }
+  counts[w][lane] = c;
+  __syncthreads();
+  if (w == 0 && i < n) {
+    int place = 0;
+#pragma unroll
+    for (int k = 0; k < RANK_THREADS / 64; ++k) place += counts[k][lane];
+    order[(int64_t)blockIdx.y * n + place] = i;
+  }
+}
+
 }  // namespace hq
 
 using namespace hq;
@@ -135,14 +246,46 @@ extern "C" int hqekv_weighted_block_scores(const void *x, const void *weights, i
   return check_launch("weighted_block_scores");
 }
 
-extern "C" int hqekv_token_range(const void *v, int64_t B, int64_t H, int64_t T, int64_t D, int64_t slab_tokens,
-                                 void *out, void *stream) {
+extern "C" int hqekv_token_range_append(const void *v, int64_t B, int64_t H, int64_t T, int64_t D, int64_t slab_tokens,
+                                        const void *prev, int64_t n_prev, void *out, void *stream) {
+  if (n_prev < 0 || (n_prev > 0 && !prev)) return fail(HQEKV_E_ARG, "token_range: bad older ranges");
   if (!v || !out) return fail(HQEKV_E_ARG, "token_range: null pointer");
   if (B <= 0 || H <= 0 || T <= 0 || D <= 0 || slab_tokens < T)
     return fail(HQEKV_E_ARG, "token_range: empty shape or slab_tokens < T");
   if (B * H > RANGE_MAX_ROWS) return fail(HQEKV_E_UNSUPPORTED, "token_range: B * H = %lld > %d", (long long)(B * H), RANGE_MAX_ROWS);
   if (T > 0x7fffffffLL || D > 0x7fffffffLL) return fail(HQEKV_E_UNSUPPORTED, "token_range: T or D too large");
+  if (D % 8 == 0 && ((uintptr_t)v & 15) == 0) {
+    const int token_blocks = (int)((T + RANGE_TOK - 1) / RANGE_TOK);
+    const int64_t copy_blocks = n_prev > 0 ? std::min<int64_t>((n_prev + 4 * IMP_THREADS - 1) / (4 * IMP_THREADS), 1024) : 0;
+    hipLaunchKernelGGL(token_range_rows_kernel, dim3((unsigned)(token_blocks + copy_blocks)), dim3(IMP_THREADS), 0, (hipStream_t)stream,
+                       (const half_t *)v, (int)B, (int)H, T, (int)D, slab_tokens, (half_t *)out + n_prev, (const half_t *)prev, n_prev, token_blocks);
+    return check_launch("token_range");
+  }
+  if (n_prev > 0) return fail(HQEKV_E_UNSUPPORTED, "token_range_append: rows of 16-byte aligned pieces only");
   hipLaunchKernelGGL(token_range_kernel, dim3((unsigned)T), dim3(IMP_THREADS), 0, (hipStream_t)stream, (const half_t *)v,
                      (int)B, (int)H, T, (int)D, slab_tokens, (half_t *)out);
   return check_launch("token_range");
+}
+
+extern "C" int hqekv_token_range(const void *v, int64_t B, int64_t H, int64_t T, int64_t D, int64_t slab_tokens,
+                                 void *out, void *stream) {
+  return hqekv_token_range_append(v, B, H, T, D, slab_tokens, nullptr, 0, out, stream);
+}
+
+extern "C" int hqekv_rank_blocks(const void *const *scores, int rows, int64_t n, int32_t *order, void *stream) {
+  if (!scores || !order || rows <= 0 || rows > HQEKV_MAX_SEGS || n <= 0) return fail(HQEKV_E_ARG, "rank_blocks: null pointer or bad shape");
+  if (n > RANK_MAX) return fail(HQEKV_E_UNSUPPORTED, "rank_blocks: more than %d scores per row", RANK_MAX);
+  RankRows rr{};
+  for (int r = 0; r < rows; ++r) {
+    if (!scores[r]) return fail(HQEKV_E_ARG, "rank_blocks: row %d is null", r);
+    rr.row[r] = (const half_t *)scores[r];
+  }
+  const size_t lds = (size_t)((n + 63) / 64 * 64) * sizeof(uint32_t);
+  if (lds > 48 * 1024) {   // beyond the default limit of a launch (128 KB of the CU's 160 at most)
+    const hipError_t e = hipFuncSetAttribute((const void *)rank_blocks_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, RANK_MAX * (int)sizeof(uint32_t));
+    if (e != hipSuccess) return fail((int)e, "rank_blocks: %s", hipGetErrorString(e));
+  }
+  hipLaunchKernelGGL(rank_blocks_kernel, dim3((unsigned)((n + RANK_ITEMS - 1) / RANK_ITEMS), (unsigned)rows), dim3(RANK_THREADS), lds,
+                     (hipStream_t)stream, rr, (int)n, order);
+  return check_launch("rank_blocks_kernel");
 }

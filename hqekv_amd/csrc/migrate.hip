@@ -56,10 +56,10 @@ __device__ __forceinline__ void plan_refused(const MigArgs &a) {
   if (a.status) atomicOr(a.status, 1);
 }
 
-// where one lane's group lives: fp16 values (with the element stride) or packed words + scale + zero
+// where one lane's group lives: 32 adjacent fp16 values or packed words + scale + zero (blocks of token-major keys, whose
+// groups are strided, are read by load_token_major_pair)
 struct GroupRef {
   half_t *f16;
-  int64_t stride;
   uint32_t *words;
   half_t *s, *z;
 };
@@ -71,13 +71,7 @@ __device__ __forceinline__ GroupRef group_ref(const MigClass &c, int64_t bh, int
   if (IS_K) {
     const int d = lane;  // channel
     if (c.bits == 16) {
-      if (c.layout == HQEKV_LAYOUT_TOKEN_MAJOR) {  // (B,H,T,D)
-        r.f16 = (half_t *)c.data + ((bh * c.slab_tokens + block * 32) * D + d);
-        r.stride = D;
-      } else {  // (B,H,D,T)
-        r.f16 = (half_t *)c.data + ((bh * D + d) * n + block * 32);
-        r.stride = 1;
-      }
+      r.f16 = (half_t *)c.data + ((bh * D + d) * n + block * 32);   // (B,H,D,T)
     } else {
       const int64_t g = (bh * D + d) * (n >> 5) + block;
       r.words = (uint32_t *)c.data + g * c.bits;  // 32 codes of b bits = b words
@@ -90,7 +84,6 @@ __device__ __forceinline__ GroupRef group_ref(const MigClass &c, int64_t bh, int
     if (c.bits == 16) {
       const int64_t t = bh * c.slab_tokens + block * 32 + k;
       r.f16 = (half_t *)c.data + (t * D + cg * 32);
-      r.stride = 1;
     } else {
       const int64_t g = (bh * n + block * 32 + k) * ng + cg;
       r.words = (uint32_t *)c.data + g * c.bits;
@@ -103,21 +96,14 @@ __device__ __forceinline__ GroupRef group_ref(const MigClass &c, int64_t bh, int
 
 // 32 fp16 values as 16 registers: xp[j] = (x[2j], x[2j+1])
 __device__ __forceinline__ void load_f16(const GroupRef &r, uint32_t (&xp)[16]) {
-  if (r.stride == 1) {
-    const uint4 *p = reinterpret_cast<const uint4 *>(r.f16);  // block starts are 64-byte aligned
+  const uint4 *p = reinterpret_cast<const uint4 *>(r.f16);  // block starts are 64-byte aligned
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const uint4 v = p[i];
-      xp[4 * i] = v.x;
-      xp[4 * i + 1] = v.y;
-      xp[4 * i + 2] = v.z;
-      xp[4 * i + 3] = v.w;
-    }
-  } else {
-    const unsigned short *p = reinterpret_cast<const unsigned short *>(r.f16);
-#pragma unroll
-    for (int j = 0; j < 16; ++j)
-      xp[j] = (uint32_t)p[(2 * j) * r.stride] | ((uint32_t)p[(2 * j + 1) * r.stride] << 16);
+  for (int i = 0; i < 4; ++i) {
+    const uint4 v = p[i];
+    xp[4 * i] = v.x;
+    xp[4 * i + 1] = v.y;
+    xp[4 * i + 2] = v.z;
+    xp[4 * i + 3] = v.w;
   }
 }
 __device__ __forceinline__ void store_f16(const GroupRef &r, const uint32_t (&xp)[16]) {
@@ -219,6 +205,50 @@ __device__ __forceinline__ void quant_group_normal1(const GroupRef &r, const uin
   *r.z = st.mean_h;
 }
 
+// a group's values into the destination's form
+__device__ __forceinline__ void quantize_to(const MigClass &dc, const GroupRef &dr, const uint32_t (&xp)[16]) {
+  switch (dc.bits) {
+    case 16: store_f16(dr, xp); break;
+    case 8: quant_group<8>(dr, xp); break;
+    case 4: quant_group<4>(dr, xp); break;
+    case 2: quant_group<2>(dr, xp); break;
+    default:
+      if (dc.layout == HQEKV_LAYOUT_NORMAL1) quant_group_normal1(dr, xp);
+      else quant_group<1>(dr, xp);
+  }
+}
+
+// the packed words, scale and zero of one group; a group's words start at a multiple of their own size, so they move as
+// vectors where the planes are 16-byte aligned (uniform; every plane this package allocates is)
+template <int BITS>
+__device__ __forceinline__ void copy_group(const GroupRef &sr, const GroupRef &dr) {
+  const half_t s = *sr.s, z = *sr.z;
+  uint32_t w[BITS];
+  constexpr int V = BITS < 4 ? BITS : 4;
+  typedef uint32_t vec_t __attribute__((ext_vector_type(V)));
+  const bool vec = (((uintptr_t)sr.words | (uintptr_t)dr.words) & (4 * V - 1)) == 0;
+  if (vec) {
+#pragma unroll
+    for (int i = 0; i < BITS; i += V) __builtin_memcpy(w + i, __builtin_assume_aligned(sr.words + i, 4 * V), 4 * V);
+  } else {
+#pragma unroll
+    for (int i = 0; i < BITS; ++i) w[i] = sr.words[i];
+  }
+  if (vec) {
+#pragma unroll
+    for (int i = 0; i < BITS; i += V) {
+      vec_t v;
+      __builtin_memcpy(&v, w + i, 4 * V);
+      *reinterpret_cast<vec_t *>(dr.words + i) = v;
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < BITS; ++i) dr.words[i] = w[i];
+  }
+  *dr.s = s;
+  *dr.z = z;
+}
+
 // One quantisation group: lane = channel (K) or (token, channel group) (V) of source block sb -> destination block db.
 template <bool IS_K>
 __device__ __forceinline__ void migrate_group(const MigClass &sc, const MigClass &dc, int64_t bh, int64_t sb, int64_t db,
@@ -226,9 +256,12 @@ __device__ __forceinline__ void migrate_group(const MigClass &sc, const MigClass
   const GroupRef sr = group_ref<IS_K>(sc, bh, sb, lane, D);
   const GroupRef dr = group_ref<IS_K>(dc, bh, db, lane, D);
   if (sc.bits != 16 && sc.bits == dc.bits) {  // a survivor of a quantised class keeps its bytes
-    for (int i = 0; i < sc.bits; ++i) dr.words[i] = sr.words[i];
-    *dr.s = *sr.s;
-    *dr.z = *sr.z;
+    switch (sc.bits) {
+      case 8: copy_group<8>(sr, dr); break;
+      case 4: copy_group<4>(sr, dr); break;
+      case 2: copy_group<2>(sr, dr); break;
+      default: copy_group<1>(sr, dr);
+    }
     return;
   }
   uint32_t xp[16];
@@ -242,15 +275,7 @@ __device__ __forceinline__ void migrate_group(const MigClass &sc, const MigClass
       if (sn) dequant_group<1, true>(sr, xp);
       else dequant_group<1, false>(sr, xp);
   }
-  switch (dc.bits) {
-    case 16: store_f16(dr, xp); break;
-    case 8: quant_group<8>(dr, xp); break;
-    case 4: quant_group<4>(dr, xp); break;
-    case 2: quant_group<2>(dr, xp); break;
-    default:
-      if (dc.layout == HQEKV_LAYOUT_NORMAL1) quant_group_normal1(dr, xp);
-      else quant_group<1>(dr, xp);
-  }
+  quantize_to(dc, dr, xp);
 }
 
 __device__ __forceinline__ int dst_class_of(const MigArgs &a, int u) {
@@ -260,8 +285,23 @@ __device__ __forceinline__ int dst_class_of(const MigArgs &a, int u) {
   return ci;
 }
 
-constexpr int MIG_THREADS = 128;
-constexpr int MIG_KB = 16;  // K side: destination blocks per workgroup
+constexpr int MIG_THREADS = 128;   // V side
+constexpr int MIG_KB = 16;         // K side: destination blocks per workgroup
+constexpr int MIG_KC = 32;         // ... and channels
+constexpr int MIG_KTHREADS = 256;
+
+// 32 tokens of channels d and d + 1 of a token-major block: two groups from 32 four-byte loads
+__device__ __forceinline__ void load_token_major_pair(const MigClass &c, int64_t bh, int64_t block, int d, int D, uint32_t (&xa)[16], uint32_t (&xb)[16]) {
+  const uint32_t *p = reinterpret_cast<const uint32_t *>((const half_t *)c.data + (bh * c.slab_tokens + block * 32) * D + d);
+  uint32_t w[32];
+#pragma unroll
+  for (int i = 0; i < 32; ++i) w[i] = p[(int64_t)i * (D >> 1)];
+#pragma unroll
+  for (int j = 0; j < 16; ++j) {
+    xa[j] = __builtin_amdgcn_perm(w[2 * j + 1], w[2 * j], 0x05040100u);
+    xb[j] = __builtin_amdgcn_perm(w[2 * j + 1], w[2 * j], 0x07060302u);
+  }
+}
 
 // V side: a workgroup per destination block; its 32 tokens x D/32 groups are one contiguous stretch of every plane.
 // K side: a group is 32 tokens of ONE channel row -- b words of the row -- and a block's groups lie a whole row
@@ -269,11 +309,13 @@ constexpr int MIG_KB = 16;  // K side: destination blocks per workgroup
 // blocks of a row: 16 b-word pieces side by side (64 bytes at 1 bit ... 512 at 8), and as long as the blocks come
 // from consecutive places of one source class (survivors of a class stay in order) the reads line up the same
 // way.  (A lane per channel, as on the V side, touched a separate cache line per lane: the K launch took four to
-// six times as long as the V launch for the same bytes.)  Blocks of new tokens arrive token-major, where the
-// channels of a token are what is contiguous: a workgroup that holds any of those walks its blocks one by one
-// with a lane per channel.
+// six times as long as the V launch for the same bytes.)  A workgroup covers 32 channels, so that a side of a thousand
+// blocks is some thousands of short workgroups; with all 128 channels in one workgroup of two waves, and its blocks of new
+// tokens (token-major: the channels of a token are what is contiguous) walked one after the other, the chip was nearly
+// idle: 50 us for 19 MB in and out at 32k tokens, 47 us for a 4k prompt of new tokens.  Those blocks now go side by side
+// as well, a lane holding two channels of one: 22 us and 13 us (V at 32k tokens 16.5 -> 13.4 us with vector copies).
 template <bool IS_K>
-__global__ __launch_bounds__(MIG_THREADS) void cache_migrate_kernel(MigArgs a, int D) {
+__global__ __launch_bounds__(IS_K ? MIG_KTHREADS : MIG_THREADS) void cache_migrate_kernel(MigArgs a, int D) {
   const int64_t bh = blockIdx.y;
   const int total = a.dst_begin[HQEKV_MAX_SEGS];
   if constexpr (!IS_K) {
@@ -289,19 +331,9 @@ __global__ __launch_bounds__(MIG_THREADS) void cache_migrate_kernel(MigArgs a, i
     for (int lane = threadIdx.x; lane < D; lane += MIG_THREADS)
       migrate_group<false>(a.src[code >> 24], dc, bh, code & 0xffffff, db, lane, D);
   } else {
-    const int u0 = blockIdx.x * MIG_KB;
-    const int u = u0 + (int)(threadIdx.x % MIG_KB);
-    const int uc = u < total ? u : u0;   // (u0 < total by the grid size)
-    const int ci = dst_class_of(a, uc);
-    const int64_t db = uc - a.dst_begin[ci];
-    const int32_t code = a.plan_src[uc];
-    const bool entry_ok = plan_entry_ok(a, code, a.plan_pos[uc], total);
-    const bool live = u < total && entry_ok;
-    if (u < total && !entry_ok && threadIdx.x < MIG_KB) plan_refused(a);
-    const int si = entry_ok ? (int)((uint32_t)code >> 24) : 0;
-    const bool token_major = entry_ok && a.src[si].bits == 16 && a.src[si].layout == HQEKV_LAYOUT_TOKEN_MAJOR;
-    if (bh == 0) {  // positions of the blocks' tokens
-      for (int e = threadIdx.x; e < MIG_KB * 32; e += MIG_THREADS) {
+    const int u0 = blockIdx.x * MIG_KB, d0 = blockIdx.z * MIG_KC;
+    if (bh == 0 && d0 == 0) {  // positions of the blocks' tokens
+      for (int e = threadIdx.x; e < MIG_KB * 32; e += MIG_KTHREADS) {
         const int ue = u0 + e / 32;
         if (ue < total && plan_entry_ok(a, a.plan_src[ue], a.plan_pos[ue], total)) {
           const int ce = dst_class_of(a, ue);
@@ -310,18 +342,46 @@ __global__ __launch_bounds__(MIG_THREADS) void cache_migrate_kernel(MigArgs a, i
         }
       }
     }
-    if (__syncthreads_or(live && token_major)) {
-      for (int j = 0; j < MIG_KB && u0 + j < total; ++j) {
-        const int cj = dst_class_of(a, u0 + j);
-        const int32_t code_j = a.plan_src[u0 + j];
-        if (!plan_entry_ok(a, code_j, a.plan_pos[u0 + j], total)) continue;   // uniform
-        for (int lane = threadIdx.x; lane < D; lane += MIG_THREADS)
-          migrate_group<true>(a.src[code_j >> 24], a.dst[cj], bh, code_j & 0xffffff, u0 + j - a.dst_begin[cj], lane, D);
+    // the block of thread `slot` (of the 16): its plan entry, its classes
+    auto block_of = [&](int slot, int &ci, int32_t &code, bool &token_major) -> bool {
+      const int u = u0 + slot;
+      if (u >= total) return false;
+      code = a.plan_src[u];
+      if (!plan_entry_ok(a, code, a.plan_pos[u], total)) {
+        plan_refused(a);
+        return false;
       }
-    } else if (live) {
-      const MigClass sc = a.src[si], dc = a.dst[ci];
-      for (int d = threadIdx.x / MIG_KB; d < D; d += MIG_THREADS / MIG_KB)
-        migrate_group<true>(sc, dc, bh, code & 0xffffff, db, d, D);
+      ci = dst_class_of(a, u);
+      const MigClass &sc = a.src[(uint32_t)code >> 24];
+      token_major = sc.bits == 16 && sc.layout == HQEKV_LAYOUT_TOKEN_MAJOR;
+      return true;
+    };
+    int ci = 0;
+    int32_t code = 0;
+    bool tm = false;
+    const int slot = threadIdx.x % MIG_KB;
+    const bool live = block_of(slot, ci, code, tm);
+    if (live && !tm) {
+      const MigClass sc = a.src[(uint32_t)code >> 24], dc = a.dst[ci];
+      for (int d = d0 + threadIdx.x / MIG_KB; d < d0 + MIG_KC; d += MIG_KTHREADS / MIG_KB)   // (D is a multiple of 32)
+        migrate_group<true>(sc, dc, bh, code & 0xffffff, u0 + slot - a.dst_begin[ci], d, D);
+    }
+    if (!__syncthreads_or(live && tm)) return;
+    // blocks of new tokens: 16 blocks x 16 channel pairs, eight neighbouring lanes on neighbouring pairs (32 bytes of a
+    // token row), the next eight on the next block
+    const int tslot = threadIdx.x / 8 % MIG_KB, pair = threadIdx.x % 8 + threadIdx.x / (8 * MIG_KB) * 8;
+    static_assert(MIG_KTHREADS == MIG_KB * MIG_KC / 2, "one channel pair of one block per thread");
+    if (!block_of(tslot, ci, code, tm) || !tm) return;
+    const MigClass sc = a.src[(uint32_t)code >> 24], dc = a.dst[ci];
+    uint32_t xp[2][16];
+    load_token_major_pair(sc, bh, code & 0xffffff, d0 + 2 * pair, D, xp[0], xp[1]);
+#pragma unroll 1
+    for (int e = 0; e < 2; ++e) {
+      const GroupRef dr = group_ref<true>(dc, bh, u0 + tslot - a.dst_begin[ci], d0 + 2 * pair + e, D);
+      uint32_t x[16];
+#pragma unroll
+      for (int j = 0; j < 16; ++j) x[j] = e ? xp[1][j] : xp[0][j];
+      quantize_to(dc, dr, x);
     }
   }
 }
@@ -381,12 +441,11 @@ extern "C" int hqekv_cache_migrate(int is_k, const hqekv_cache_class *src, int n
   a.status = status;
   a.plan_src = plan;
   a.plan_pos = plan + total;
-  const dim3 block(MIG_THREADS);
   if (is_k)
-    hipLaunchKernelGGL(cache_migrate_kernel<true>, dim3((unsigned)((total + MIG_KB - 1) / MIG_KB), (unsigned)BH), block, 0,
-                       (hipStream_t)stream, a, (int)D);
+    hipLaunchKernelGGL(cache_migrate_kernel<true>, dim3((unsigned)((total + MIG_KB - 1) / MIG_KB), (unsigned)BH, (unsigned)(D / MIG_KC)),
+                       dim3(MIG_KTHREADS), 0, (hipStream_t)stream, a, (int)D);
   else
-    hipLaunchKernelGGL(cache_migrate_kernel<false>, dim3((unsigned)total, (unsigned)BH), block, 0, (hipStream_t)stream, a,
+    hipLaunchKernelGGL(cache_migrate_kernel<false>, dim3((unsigned)total, (unsigned)BH), dim3(MIG_THREADS), 0, (hipStream_t)stream, a,
                        (int)D);
   return check_launch("cache_migrate_kernel");
 }

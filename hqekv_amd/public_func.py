@@ -53,6 +53,20 @@ def calculate_token_range(new_cache: Optional[torch.Tensor], token_range: Option
     """``calculate_new_token_range`` appended to the running per-token vector."""
     if new_cache is None:
         return None
+    old = token_range
+    if old is not None and new_cache.is_cuda and new_cache.dtype == torch.float16 == old.dtype and new_cache.dim() == 4 and new_cache.numel() \
+            and new_cache.shape[0] * new_cache.shape[1] <= 1024 and new_cache.shape[3] % 8 == 0 and new_cache.data_ptr() % 16 == 0 \
+            and old.dim() == 1 and old.is_contiguous() and old.device == new_cache.device:
+        slab = _token_major_slabs(new_cache)
+        if slab is not None:   # the older ranges are copied in front by the launch that makes the new ones
+            from . import _lib
+            B, H, T, D = new_cache.shape
+            out = torch.empty(old.numel() + T, dtype=torch.float16, device=old.device)
+            with _lib.on_device(old.device):
+                rc = _lib.load().hqekv_token_range_append(new_cache.data_ptr(), B, H, T, D, slab, old.data_ptr(), old.numel(),
+                                                          out.data_ptr(), _lib.stream_ptr(old.device))
+            _lib.check(rc, "token_range")
+            return out
     r = calculate_new_token_range(new_cache)
     return r if token_range is None else torch.cat((token_range, r), dim=-1)
 
@@ -96,6 +110,26 @@ class RankedBlocks:
             a._order, b._order = both[0], both[1]
             return both
         return torch.stack((a.order, b.order))
+
+    @staticmethod
+    def host_orders(a: "RankedBlocks", b: "RankedBlocks"):
+        """Both orders on the host, (2, blocks): ranked by one launch that writes them into page-locked memory, which
+        this call waits for; rankings it does not take (already sorted, another type, very many blocks) through
+        ``sort_together``."""
+        sa, sb = a.scores, b.scores
+        if a._order is None and b._order is None and sa.is_cuda and sa.dtype == torch.float16 == sb.dtype and sa.device == sb.device \
+                and sa.shape == sb.shape and sa.is_contiguous() and sb.is_contiguous() and 0 < sa.numel() <= 32768:
+            from . import _lib
+            import ctypes as C
+            n = sa.numel()
+            order = torch.empty(2, n, dtype=torch.int32, pin_memory=True)
+            with _lib.on_device(sa.device):
+                rc = _lib.load().hqekv_rank_blocks((C.c_void_p * 2)(sa.data_ptr(), sb.data_ptr()), 2, n, order.data_ptr(),
+                                                   _lib.stream_ptr(sa.device))
+                _lib.check(rc, "rank_blocks")
+                torch.cuda.current_stream(sa.device).synchronize()
+            return order.numpy()
+        return RankedBlocks.sort_together(a, b).to("cpu", torch.int64).numpy()
 
     @property
     def _hq_block_order(self):

@@ -332,6 +332,15 @@ int hqekv_importance_scores(const void *ring, int32_t rows, int64_t max_len, int
 int hqekv_weighted_block_scores(const void *x, const void *weights, int64_t total, void *scores_out, void *stream);
 int hqekv_token_range(const void *v, int64_t B, int64_t H, int64_t T, int64_t D, int64_t slab_tokens, void *out,
                       void *stream);
+/* The ranges of T new tokens behind a copy of the n_prev older ones: out (n_prev + T) = cat(prev, token_range(v)). With
+ * n_prev > 0: D a multiple of 8, v 16-byte aligned. */
+int hqekv_token_range_append(const void *v, int64_t B, int64_t H, int64_t T, int64_t D, int64_t slab_tokens, const void *prev,
+                             int64_t n_prev, void *out, void *stream);
+/* order (rows x n): the block numbers of every row of n <= 32768 fp16 scores (scores: host array of rows <=
+ * HQEKV_MAX_SEGS device pointers), highest score first, equal scores
+ * in ascending order, NaN before everything: torch.sort(scores, descending=True, stable=True)[1], the sort of
+ * get_block_token_idx (model/public_func.py:97).  order may be page-locked host memory. */
+int hqekv_rank_blocks(const void *const *scores, int rows, int64_t n, int32_t *order, void *stream);
 
 /* ------------------------------------------------------------------ the prompt side of the attention layer
  * Replaces, for head_dim 128 in fp16, what model/llama_hqe.py:141-188 does over a prompt: flash_attention_forward

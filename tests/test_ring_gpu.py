@@ -3,6 +3,8 @@ torch's own ``attn_weights.sum(0).sum(0)`` executed on the GPU, bit for bit -- t
 rankings (model/public_func.py:92-106, 243-257), so the kernels follow the order in which torch's reduction adds the
 rows.  Shapes: 32 heads, batch 1..8, rows from 256 tokens up, every residue of the length modulo 4, aligned and
 unaligned slots of the ring store."""
+import ctypes
+
 import pytest
 import torch
 
@@ -270,3 +272,31 @@ def test_step_extras_with_either_combine_route_and_dot_form(dev, B, Hq, Hkv, T):
             kbuf[:, :, 7] = 0
             vbuf[:, :, 7] = 0
             assert not bool(kbuf.any()) and not bool(vbuf.any()), where   # nothing else written
+
+
+@pytest.mark.parametrize("rows,n", [(1, 1), (2, 63), (2, 64), (2, 65), (2, 1025), (1, 4096), (2, 20000)])
+def test_rank_blocks_matches_the_stable_sort(dev, rows, n):
+    """Ties, both zeros, infinities and NaNs: the order of torch.sort(descending, stable)."""
+    from hqekv_amd import _lib
+    g = torch.Generator().manual_seed(n)
+    x = (torch.randint(-6, 7, (rows, n), generator=g) / 4).half()
+    x[:, torch.randperm(n, generator=g)[: n // 5]] = -0.0
+    x[:, torch.randperm(n, generator=g)[: n // 50]] = float("nan")
+    x[:, torch.randperm(n, generator=g)[: n // 50]] = float("-inf")
+    x[:, torch.randperm(n, generator=g)[: n // 50]] = float("inf")
+    x = x.to(dev)
+    order = torch.empty(rows, n, dtype=torch.int32).pin_memory()
+    ptrs = (ctypes.c_void_p * rows)(*[x[r].data_ptr() for r in range(rows)])
+    _lib.check(_lib.load().hqekv_rank_blocks(ptrs, rows, n, order.data_ptr(), _lib.stream_ptr(dev)), "rank_blocks")
+    torch.cuda.synchronize()
+    assert torch.equal(order.long(), torch.sort(x, dim=1, descending=True, stable=True)[1].cpu())
+
+
+@pytest.mark.parametrize("B,H,T,D,prev", [(1, 8, 32, 128, 1000), (2, 3, 17, 128, 1), (1, 1, 1, 64, 0), (4, 8, 33, 192, 70000), (1, 2, 5, 24, 9)])
+def test_token_range_behind_older_ranges(dev, B, H, T, D, prev):
+    from hqekv_amd.public_func import calculate_token_range
+    g = torch.Generator().manual_seed(T)
+    v, old = torch.randn(B, H, T, D, generator=g).half().to(dev), torch.rand(prev, generator=g).half().to(dev)
+    lo, hi = torch.aminmax(v, dim=-1)
+    want = torch.cat((old, (hi - lo).sum(0).sum(0)))
+    assert torch.equal(calculate_token_range(v, old if prev else None), want)
