@@ -164,6 +164,23 @@ def load() -> C.CDLL:
     return _lib
 
 
+_host = None
+
+
+def host():
+    """The native host module (``csrc/host.cpp``), bound to the kernels' library once; raises if it has not been built."""
+    global _host
+    if _host is None:
+        load()
+        try:
+            from . import _host as m
+        except ImportError as e:
+            raise RuntimeError(f"{_PKG / '_host.so'} is missing or does not load: build it with `python -m hqekv_amd.build` ({e})") from e
+        m.bind(str(_LIB_PATH))
+        _host = m
+    return _host
+
+
 def check(rc: int, what: str) -> None:
     """Turn a non-zero return code into the exception the reference's callers expect."""
     if rc == 0:

@@ -288,8 +288,7 @@ class SegmentMemo:
         self.Hkv = None
         self.dims = (None, None)
         self.partition = False                 # the classes' position arrays cover [0, kept) once per side
-        self._step = None                      # what step_call keeps between steps
-        self._spare = None                     # (attn_weights, attn_output) allocated ahead for the next step
+        self._native = None                    # the class entries as the native step takes them
 
     def lookup(self, pkv: tuple, dev, low_uniform: bool) -> bool:
         held = self.held
@@ -318,7 +317,7 @@ class SegmentMemo:
         self.held = tuple(pkv[:NEW_K])
         self.key = (dev, low_uniform)
         self.partition = classes_partition_positions(pkv)
-        self._step = None
+        self._native = None
 
     @staticmethod
     def _fill(s, t: torch.Tensor, end: int, layout: int, keep: list):
@@ -355,88 +354,17 @@ class SegmentMemo:
             self.ws = torch.empty(max(need + need // 8, 256) // 4, dtype=torch.float32, device=dev)
         return self.ws
 
-    SPARE_MAX_BYTES = 4 << 20   # largest attn_weights tensor that is allocated one step ahead
-
-    def step_call(self, q: torch.Tensor, pkv: tuple, Tall: int, k: torch.Tensor, v: torch.Tensor, res, n: int,
-                  ring_store: Optional[torch.Tensor], ring_row: int, low_uniform: bool, known: bool = False):
-        """One decode step of a layer as one C call (``hqekv_decode_step``) with as little host work as the call
-        allows: the class entries of the tables are the memo's, the residual is the first ``n`` token rows of the
-        capacity buffers ``res`` = (K, V), this step's ``k`` / ``v`` (B,Hkv,L,D, dense) are read as a segment of
-        their own and copied to row ``n`` of the buffers, and -- when ``ring_store`` (rows x max_length, fp16) is
-        given -- row ``ring_row`` of it receives the ring row.  ``known``: the caller vouches that ``pkv`` carries the
-        class tensors the tables were built from (it is the tuple the previous step returned).
-        -> (attn_weights, attn_output)."""
-        dev = q.device
+    def steps(self, pkv: tuple, dev, low_uniform: bool, known: bool):
+        """The native tables (``_host.StepTables``) of a cache whose classes cover every position once, else None.
+        ``known``: the caller vouches that ``pkv`` carries the class tensors the tables were built from (it is the tuple
+        the previous step returned)."""
         if not (known and self.held is not None) and not self.lookup(pkv, dev, low_uniform):
             self.build(pkv, dev, low_uniform)
-        B, Hq, _, D = q.shape
-        Hkv, L = k.shape[1], k.shape[2]
-        kbuf, vbuf = res
-        st = self._step
-        if st is None or st[0] is not kbuf:
-            # entries that stay the same from step to step: the residual's (bits, layout, data, slab), the tail's
-            # (bits, layout), and the appends' slab lengths
-            for arr, base, buf, layout in ((self.k_arr, self.n_k, kbuf, _lib.LAYOUT_TOKEN_MAJOR), (self.v_arr, self.n_v, vbuf, 0)):
-                for j in (0, 1):
-                    e = arr[base + j]
-                    e.bits, e.layout, e.scale, e.zero, e.idx, e.slab_tokens = 16, layout, None, None, None, 0
-            x = _lib.StepExtra()
-            x.k_dst_slab_tokens, x.v_dst_slab_tokens = kbuf.shape[2], vbuf.shape[2]
-            st = self._step = (kbuf, x, kbuf.data_ptr(), vbuf.data_ptr(), kbuf.shape[2])
-        _, x, kptr, vptr, cap = st
-        n_k, n_v = self.n_k, self.n_v
-        ka, va = self.k_arr, self.v_arr
-        if n:
-            e = ka[n_k]
-            e.n_tokens, e.pos_base, e.data, e.slab_tokens = n, Tall - L - n, kptr, cap
-            e = va[n_v]
-            e.n_tokens, e.pos_base, e.data, e.slab_tokens = n, Tall - L - n, vptr, cap
-            n_k += 1
-            n_v += 1
-        e = ka[n_k]
-        e.n_tokens, e.pos_base, e.data, e.slab_tokens = L, Tall - L, k.data_ptr(), 0
-        e = va[n_v]
-        e.n_tokens, e.pos_base, e.data, e.slab_tokens = L, Tall - L, v.data_ptr(), 0
-        n_k += 1
-        n_v += 1
-        # (positions nobody writes must read as zero when the classes do not cover every position)
-        spare, self._spare = self._spare, None
-        if spare is not None and self.partition and spare[0].shape == (B, Hq, 1, Tall) and spare[1].shape == (B, Hq, 1, D) \
-                and spare[0].device == dev:
-            weights, out = spare   # allocated while the previous step's kernels were running
-        else:
-            weights = (torch.empty if self.partition else torch.zeros)(B, Hq, 1, Tall, dtype=torch.float16, device=dev)
-            out = torch.empty(B, Hq, 1, D, dtype=torch.float16, device=dev)
-        if ring_store is not None:
-            x.ring_line = ring_store.data_ptr() + 2 * ring_row * ring_store.shape[1]
-            x.ring_order = 2 if (Tall % 4 == 0 and Tall >= 256 and weights.data_ptr() % 8 == 0) else 1
-        else:
-            x.ring_line = None
-        row_bytes = 2 * D
-        x.append_rows, x.new_k, x.new_v = L, k.data_ptr(), v.data_ptr()
-        x.k_dst, x.v_dst = kptr + n * row_bytes, vptr + n * row_bytes
-        flags = default_flags() if self.partition else 0
-        lib = _lib.load()
-        ws = self.ws
-        with _lib.on_device(dev):
-            for attempt in (0, 1):
-                if ws is None or attempt:
-                    need = lib.hqekv_decode_workspace_bytes(ka, n_k, va, n_v, B, Hq, Hkv, D)
-                    if need < 0:
-                        raise ValueError("invalid segment table")
-                    ws = self.workspace(2 * need, dev)   # room for the residual to grow without asking again
-                rc = lib.hqekv_decode_step(ka, n_k, va, n_v, q.data_ptr(), None, 0, weights.data_ptr(), out.data_ptr(),
-                                           B, Hq, Hkv, D, Tall, ws.data_ptr(), ws.numel() * 4, flags,
-                                           _lib.stream_ptr(dev), C.byref(x))
-                if rc != -3:   # HQEKV_E_WORKSPACE: the cache has outgrown the workspace kept from earlier steps
-                    break
-        _lib.check(rc, "decode_step")
-        # The next step's outputs, one position longer, allocated now: off that step's path to its first launch.  Only
-        # while they are small (every layer of a model holds its own): a long step does not notice the allocation.
-        if self.partition and B * Hq * (Tall + L) * 2 <= self.SPARE_MAX_BYTES:
-            self._spare = (torch.empty(B, Hq, 1, Tall + L, dtype=torch.float16, device=dev),
-                           torch.empty(B, Hq, 1, D, dtype=torch.float16, device=dev))
-        return weights, out
+        if not self.partition:
+            return None
+        if self._native is None:
+            self._native = _lib.host().StepTables(C.addressof(self.k_arr), self.n_k, C.addressof(self.v_arr), self.n_v)
+        return self._native
 
 
 def decode_attention(q: torch.Tensor, pkv: tuple, mask, Tall: int, zero_init: bool, flags: Optional[int] = None,

@@ -1,7 +1,8 @@
-"""Build libhqekv.so (hand-written HIP for gfx950) in-tree with hipcc.
+"""Build libhqekv.so (hand-written HIP for gfx950) and _host.so (the host side of the calls, C++ over torch) in-tree.
 
 ``python -m hqekv_amd.build`` compiles every source under ``hqekv_amd/csrc`` and links
-``hqekv_amd/libhqekv.so``.  hipcc cross-compiles for gfx950 without a GPU.
+``hqekv_amd/libhqekv.so`` with hipcc, which cross-compiles for gfx950 without a GPU, and ``hqekv_amd/_host.so`` with the
+host compiler.
 """
 from __future__ import annotations
 
@@ -9,6 +10,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -16,6 +18,7 @@ PKG = Path(__file__).resolve().parent
 ROOT = PKG.parent
 CSRC = PKG / "csrc"
 LIB = PKG / "libhqekv.so"
+HOST = PKG / "_host.so"
 SOURCES = ["capi.hip", "quant_pack.hip", "attn.hip", "decode_static.hip", "migrate.hip", "reconstruct.hip", "planner.hip", "importance.hip", "prompt_attn.hip"]
 
 HIPCC_FLAGS = [
@@ -42,6 +45,19 @@ def _run(cmd):
     return out
 
 
+def _build_host(objdir: Path) -> str:
+    """_host.so: torch's headers and libraries, no device code."""
+    import torch
+    base, rocm = Path(torch.__file__).resolve().parent, Path(_hipcc()).resolve().parents[1]
+    tmp = objdir / "_host.so.tmp"
+    log = _run([os.environ.get("CXX") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+                f"-I{ROOT / 'include'}", f"-I{base / 'include'}", f"-I{base / 'include/torch/csrc/api/include'}", f"-I{rocm / 'include'}",
+                "-I/opt/rocm/include", f"-I{sysconfig.get_paths()['include']}", str(CSRC / "host.cpp"), "-o", str(tmp), f"-L{base / 'lib'}",
+                "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-ltorch_hip", "-ldl"])
+    os.replace(tmp, HOST)
+    return log
+
+
 def build(verbose: bool = False) -> Path:
     hipcc = _hipcc()
     objdir = PKG / "build"
@@ -53,7 +69,9 @@ def build(verbose: bool = False) -> Path:
         return _run([hipcc, *HIPCC_FLAGS, "-c", str(CSRC / src), "-o", str(obj)])
 
     with ThreadPoolExecutor(max_workers=min(4, len(SOURCES))) as ex:
+        host = ex.submit(_build_host, objdir)
         logs = list(ex.map(compile_one, zip(SOURCES, objs)))
+        logs.append(host.result())
     tmp = LIB.with_suffix(".so.tmp")
     logs.append(_run([hipcc, "-shared", "-fPIC", "--offload-arch=gfx950", *map(str, objs), "-o", str(tmp)]))
     os.replace(tmp, LIB)

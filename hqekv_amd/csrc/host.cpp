@@ -1,0 +1,662 @@
+// The host side of the per-step and per-layer calls, as a CPython module over torch's C++ tensors.
+//
+// A decode step of a short or medium cache is three or four launches of a few microseconds each; reading the forty
+// fields of a cache tuple, filling the segment tables and building the views of the next tuple from Python took longer
+// than the launches ran (a plain call at 1k tokens: 46 us of Python around 7 us of launch calls and 16 us of device
+// time).  The functions here do that work on at::Tensor directly.  They take the plain case only -- contiguous device
+// tensors of the expected types -- and answer None for anything else, which the Python callers then handle in full.
+//
+// Kernels are reached through libhqekv's C ABI, bound by path (bind), so that whatever library the package loaded is
+// the one used here.
+#include <Python.h>
+#include <dlfcn.h>
+#include <math.h>
+#include <stdlib.h>
+#include <string.h>
+
+#include <initializer_list>
+
+#include <ATen/core/Tensor.h>
+#include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <ATen/ops/empty.h>
+#include <c10/core/DeviceGuard.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include "hqekv.h"
+
+namespace {
+
+using at::Tensor;
+
+// ------------------------------------------------------------------------------------------------ the C ABI
+#define HQ_SYMBOLS(X)             \
+  X(hqekv_last_error)             \
+  X(hqekv_decode_workspace_bytes) \
+  X(hqekv_decode_attn)            \
+  X(hqekv_decode_step)            \
+  X(hqekv_quant_pack_rows)        \
+  X(hqekv_quant_pack_k_tokenmajor)
+
+struct Api {
+#define X(n_) decltype(&::n_) n_ = nullptr;
+  HQ_SYMBOLS(X)
+#undef X
+} api;
+
+PyObject *s_cover = nullptr;   // interned attribute names
+
+// the exceptions of _lib.check
+PyObject *raise_rc(int64_t rc, const char *what) {
+  const char *msg = api.hqekv_last_error();
+  if (rc < 0) return PyErr_Format(PyExc_ValueError, "%s: %s (code %lld)", what, msg, (long long)rc);
+  return PyErr_Format(PyExc_RuntimeError, "%s: HIP error %lld: %s", what, (long long)rc, msg);
+}
+
+// ------------------------------------------------------------------------------------------------ tensors
+bool is_tensor(PyObject *o) { return THPVariable_Check(o); }
+const Tensor &ten(PyObject *o) { return THPVariable_Unpack(o); }
+
+bool plain_f16(const Tensor &t, int64_t dim, const at::Device &dev) {
+  return t.dim() == dim && t.scalar_type() == at::kHalf && t.device() == dev && t.is_contiguous();
+}
+bool plain_i32(const Tensor &t, int64_t dim, const at::Device &dev) {
+  return t.dim() == dim && t.scalar_type() == at::kInt && t.device() == dev && t.is_contiguous();
+}
+void *stream_of(const at::Device &dev) {
+  return (void *)c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(dev.index()).stream();
+}
+Tensor new_tensor(at::IntArrayRef shape, at::ScalarType type, const at::Device &dev) {
+  return at::empty(shape, at::TensorOptions().dtype(type).device(dev));
+}
+
+// ------------------------------------------------------------------------------------------------ the cache tuple
+// Field numbers of the 42-field tuple (hqekv_amd/attention.py): fp16 K 0/1, fp16 V 2/3, then per bit width code, idx,
+// scale, zero; 39/40 the fp16 residual.
+constexpr int BITS[4] = {8, 4, 2, 1};
+constexpr int K_BASE[4] = {4, 12, 20, 28}, V_BASE[4] = {8, 16, 24, 32};
+constexpr int NEW_K = 39, NEW_V = 40, TUPLE_LEN = 42;
+
+struct Side {
+  hqekv_seg seg[HQEKV_MAX_SEGS + 2];
+  PyObject *idx[HQEKV_MAX_SEGS];
+  int n = 0, n_idx = 0;
+  int64_t class_tokens = 0, tokens = 0, H = -1, D = -1;
+};
+
+bool same_heads(Side &s, int64_t H, int64_t D) {
+  if (s.H < 0) {
+    s.H = H;
+    s.D = D;
+  }
+  return s.H == H && s.D == D;
+}
+
+bool position_array(PyObject *o, int64_t n, const at::Device &dev, Side &s, hqekv_seg &e) {
+  if (!is_tensor(o)) return false;
+  const Tensor &t = ten(o);
+  if (t.scalar_type() != at::kLong || t.device() != dev || !t.is_contiguous() || t.numel() != n) return false;
+  e.idx = (const int64_t *)t.data_ptr();
+  s.idx[s.n_idx++] = o;
+  return true;
+}
+
+// One side of the tuple as a segment table, in launch order; false: something is not plain.  The residual's position
+// is filled in by the caller (Tall - its tokens).
+bool read_side(PyObject *pkv, bool is_k, bool low_uniform, int64_t B, const at::Device &dev, Side &s) {
+  memset(s.seg, 0, sizeof(s.seg));
+  PyObject *f16 = PyTuple_GET_ITEM(pkv, is_k ? 0 : 2);
+  if (f16 != Py_None) {
+    if (!is_tensor(f16)) return false;
+    const Tensor &t = ten(f16);
+    if (t.dim() != 4 || t.scalar_type() != at::kHalf || t.device() != dev || t.size(0) != B) return false;
+    hqekv_seg &e = s.seg[s.n++];
+    e.bits = 16;
+    const int64_t n = t.size(is_k ? 3 : 2), D = t.size(is_k ? 2 : 3), H = t.size(1);
+    if (!t.is_contiguous()) {
+      // fp16 keys may be the transposed view of token-major memory
+      if (!is_k || t.stride(2) != 1 || t.stride(3) != D || t.stride(1) != n * D || (B > 1 && t.stride(0) != H * n * D)) return false;
+      e.layout = HQEKV_LAYOUT_TOKEN_MAJOR;
+    }
+    e.n_tokens = n;
+    e.data = t.data_ptr();
+    if (!same_heads(s, H, D) || !position_array(PyTuple_GET_ITEM(pkv, is_k ? 1 : 3), n, dev, s, e)) return false;
+    s.class_tokens += n;
+  }
+  for (int c = 0; c < 4; ++c) {
+    const int base = is_k ? K_BASE[c] : V_BASE[c], bits = BITS[c];
+    PyObject *code = PyTuple_GET_ITEM(pkv, base);
+    if (code == Py_None) continue;
+    PyObject *sc = PyTuple_GET_ITEM(pkv, base + 2), *zr = PyTuple_GET_ITEM(pkv, base + 3);
+    if (!is_tensor(code) || !is_tensor(sc) || !is_tensor(zr)) return false;
+    const Tensor &tc = ten(code), &ts = ten(sc), &tz = ten(zr);
+    if (!plain_i32(tc, 4, dev) || !plain_f16(ts, 4, dev) || !plain_f16(tz, 4, dev) || tc.size(0) != B) return false;
+    hqekv_seg &e = s.seg[s.n++];
+    const int64_t per = 32 / bits;
+    const int64_t n = is_k ? tc.size(3) * per : tc.size(2), D = is_k ? tc.size(2) : tc.size(3) * per;
+    if (ts.numel() * 32 != tc.numel() * per || tz.numel() != ts.numel()) return false;
+    e.bits = bits;
+    e.layout = bits == 1 && !low_uniform ? HQEKV_LAYOUT_NORMAL1 : 0;
+    e.n_tokens = n;
+    e.data = tc.data_ptr();
+    e.scale = ts.data_ptr();
+    e.zero = tz.data_ptr();
+    if (!same_heads(s, tc.size(1), D) || !position_array(PyTuple_GET_ITEM(pkv, base + 1), n, dev, s, e)) return false;
+    s.class_tokens += n;
+  }
+  s.tokens = s.class_tokens;
+  PyObject *res = PyTuple_GET_ITEM(pkv, is_k ? NEW_K : NEW_V);
+  if (res != Py_None) {
+    if (!is_tensor(res)) return false;
+    const Tensor &t = ten(res);
+    if (t.dim() != 4 || t.scalar_type() != at::kHalf || t.device() != dev || t.size(0) != B) return false;
+    const int64_t H = t.size(1), n = t.size(2), D = t.size(3);
+    if (n > 0) {
+      hqekv_seg &e = s.seg[s.n++];
+      e.bits = 16;
+      e.layout = is_k ? HQEKV_LAYOUT_TOKEN_MAJOR : 0;
+      e.n_tokens = n;
+      e.data = t.data_ptr();
+      if (!t.is_contiguous()) {   // the head of a longer buffer
+        const int64_t sb = t.stride(0), sh = t.stride(1);
+        if (t.stride(3) != 1 || t.stride(2) != D || sh % D || sh < n * D || (B > 1 && sb != H * sh)) return false;
+        e.slab_tokens = sh / D;
+      }
+      if (!same_heads(s, H, D)) return false;
+      s.tokens += n;
+    }
+  }
+  return s.n <= HQEKV_MAX_SEGS;
+}
+
+// attention.idx_cover_once: the remembered verdict when it still holds for these very arrays, else the function itself
+// (which remembers).  -> 1, 0, or -1 with an exception set.
+int cover_once(PyObject *const *idx, int n_idx, int64_t n, PyObject *cover_fn) {
+  if (n_idx == 0) return n == 0;
+  PyObject *hit = PyObject_GetAttr(idx[0], s_cover);
+  if (!hit) {
+    if (!PyErr_ExceptionMatches(PyExc_AttributeError)) return -1;
+    PyErr_Clear();
+  } else {
+    int verdict = -1;
+    if (PyTuple_Check(hit) && PyTuple_GET_SIZE(hit) == 3) {
+      PyObject *key = PyTuple_GET_ITEM(hit, 0), *refs = PyTuple_GET_ITEM(hit, 2);
+      bool ok = PyTuple_Check(key) && PyTuple_GET_SIZE(key) == n_idx + 1 && PyList_Check(refs) && PyList_GET_SIZE(refs) == n_idx &&
+                PyLong_AsLongLong(PyTuple_GET_ITEM(key, n_idx)) == n;
+      for (int i = 0; ok && i < n_idx; ++i) {
+        const Tensor &t = ten(idx[i]);
+        PyObject *k = PyTuple_GET_ITEM(key, i);
+        ok = PyTuple_Check(k) && PyTuple_GET_SIZE(k) == 3 && !t.is_inference() &&
+             PyLong_AsUnsignedLongLongMask(PyTuple_GET_ITEM(k, 0)) == (unsigned long long)(uintptr_t)t.data_ptr() &&
+             PyLong_AsLongLong(PyTuple_GET_ITEM(k, 1)) == t.numel() && PyLong_AsLongLong(PyTuple_GET_ITEM(k, 2)) == (long long)t._version() &&
+             PyWeakref_Check(PyList_GET_ITEM(refs, i)) && PyWeakref_GET_OBJECT(PyList_GET_ITEM(refs, i)) == idx[i];
+      }
+      if (ok) verdict = PyTuple_GET_ITEM(hit, 1) == Py_True;
+    }
+    Py_DECREF(hit);
+    if (PyErr_Occurred()) return -1;
+    if (verdict >= 0) return verdict;
+  }
+  PyObject *list = PyList_New(n_idx);
+  if (!list) return -1;
+  for (int i = 0; i < n_idx; ++i) {
+    Py_INCREF(idx[i]);
+    PyList_SET_ITEM(list, i, idx[i]);
+  }
+  PyObject *r = PyObject_CallFunction(cover_fn, "NL", list, (long long)n);
+  if (!r) return -1;
+  const int v = PyObject_IsTrue(r);
+  Py_DECREF(r);
+  return v;
+}
+
+int default_flags() {
+  const char *v = getenv("HQEKV_UNFUSED");
+  return v && !strcmp(v, "1") ? 0 : HQEKV_FUSE_SOFTMAX;
+}
+
+// ------------------------------------------------------------------------------------------------ decode
+// decode(q, pkv, low_uniform, cover_fn) -> (attn_weights, attn_output), or None where the call is not plain
+PyObject *decode(PyObject *, PyObject *const *a, Py_ssize_t na) {
+  HANDLE_TH_ERRORS
+  if (na != 4) return PyErr_Format(PyExc_TypeError, "decode takes 4 arguments");
+  PyObject *pkv = a[1];
+  const int flags = default_flags();
+  if (!is_tensor(a[0]) || !PyTuple_Check(pkv) || PyTuple_GET_SIZE(pkv) != TUPLE_LEN || !flags) Py_RETURN_NONE;
+  const Tensor &q = ten(a[0]);
+  if (!q.is_cuda() || q.dim() != 4 || q.scalar_type() != at::kHalf || q.size(2) != 1 || !q.is_contiguous()) Py_RETURN_NONE;
+  const at::Device dev = q.device();
+  const int64_t B = q.size(0), Hq = q.size(1), D = q.size(3);
+  Side k, v;
+  const bool low_uniform = a[2] == Py_True;
+  if (!read_side(pkv, true, low_uniform, B, dev, k) || !read_side(pkv, false, low_uniform, B, dev, v)) Py_RETURN_NONE;
+  const int64_t Tall = v.tokens;
+  if (Tall == 0 || k.tokens != Tall || k.class_tokens != v.class_tokens || k.H != v.H || k.D != D || v.D != D) Py_RETURN_NONE;
+  for (const auto &side : {std::make_pair(k.idx, k.n_idx), std::make_pair(v.idx, v.n_idx)}) {
+    const int c = cover_once(side.first, side.second, v.class_tokens, a[3]);
+    if (c < 0) return nullptr;
+    if (!c) Py_RETURN_NONE;
+  }
+  for (Side *s : {&k, &v})
+    if (s->tokens > s->class_tokens) s->seg[s->n - 1].pos_base = s->class_tokens;
+  const c10::OptionalDeviceGuard guard(dev);
+  const int64_t need = api.hqekv_decode_workspace_bytes(k.seg, k.n, v.seg, v.n, B, Hq, k.H, D);
+  if (need < 0) return PyErr_Format(PyExc_ValueError, "invalid segment table");
+  Tensor weights = new_tensor({B, Hq, 1, Tall}, at::kHalf, dev), out = new_tensor({B, Hq, 1, D}, at::kHalf, dev);
+  Tensor ws = new_tensor({std::max<int64_t>(need, 256)}, at::kByte, dev);
+  const int rc = api.hqekv_decode_attn(k.seg, k.n, v.seg, v.n, q.data_ptr(), nullptr, 0, weights.data_ptr(), out.data_ptr(), B, Hq, k.H, D,
+                                       Tall, ws.data_ptr(), ws.numel(), flags, stream_of(dev));
+  if (rc) return raise_rc(rc, "decode_attention");
+  return Py_BuildValue("NN", THPVariable_Wrap(weights), THPVariable_Wrap(out));
+  END_HANDLE_TH_ERRORS
+}
+
+// ------------------------------------------------------------------------------------------------ a layer's steps
+// The class entries of a layer's segment tables between two compressions, with room for the residual and the step's own
+// token, and the workspace of its steps.
+struct StepTables {
+  PyObject_HEAD
+  hqekv_seg k[HQEKV_MAX_SEGS], v[HQEKV_MAX_SEGS];
+  int n_k, n_v;
+  Tensor ws;
+};
+
+PyObject *tables_new(PyTypeObject *type, PyObject *args, PyObject *) {
+  unsigned long long ka, va;
+  int nk, nv;
+  if (!PyArg_ParseTuple(args, "KiKi", &ka, &nk, &va, &nv)) return nullptr;
+  if (nk < 0 || nv < 0 || nk > HQEKV_MAX_SEGS - 2 || nv > HQEKV_MAX_SEGS - 2) return PyErr_Format(PyExc_ValueError, "too many segments");
+  StepTables *t = (StepTables *)type->tp_alloc(type, 0);
+  if (!t) return nullptr;
+  memset(t->k, 0, sizeof(t->k));
+  memset(t->v, 0, sizeof(t->v));
+  memcpy(t->k, (const void *)(uintptr_t)ka, nk * sizeof(hqekv_seg));
+  memcpy(t->v, (const void *)(uintptr_t)va, nv * sizeof(hqekv_seg));
+  t->n_k = nk;
+  t->n_v = nv;
+  new (&t->ws) Tensor();
+  return (PyObject *)t;
+}
+void tables_free(PyObject *o) {
+  ((StepTables *)o)->ws.~Tensor();
+  Py_TYPE(o)->tp_free(o);
+}
+
+void f16_rows(hqekv_seg &e, int layout, int64_t n, int64_t pos, const void *data, int64_t slab) {
+  e = hqekv_seg{};
+  e.bits = 16;
+  e.layout = layout;
+  e.n_tokens = n;
+  e.pos_base = pos;
+  e.data = data;
+  e.slab_tokens = slab;
+}
+
+// The attention call of a step, with the workspace kept from step to step (twice what is needed when it is made: room
+// for the residual to grow without asking again).
+int run_step(const hqekv_seg *k, int n_k, const hqekv_seg *v, int n_v, const Tensor &q, const Tensor &weights, const Tensor &out,
+             int64_t Hkv, int64_t Tall, Tensor &ws, const at::Device &dev, const hqekv_step_extra *x) {
+  const int64_t B = q.size(0), Hq = q.size(1), D = q.size(3);
+  for (int attempt = 0;; ++attempt) {
+    if (attempt || !ws.defined() || ws.device() != dev) {
+      const int64_t need = api.hqekv_decode_workspace_bytes(k, n_k, v, n_v, B, Hq, Hkv, D);
+      if (need < 0) return HQEKV_E_ARG;
+      ws = new_tensor({std::max<int64_t>(2 * need, 256)}, at::kByte, dev);
+    }
+    const int rc = api.hqekv_decode_step(k, n_k, v, n_v, q.data_ptr(), nullptr, 0, weights.data_ptr(), out.data_ptr(), B, Hq, Hkv, D, Tall,
+                                         ws.data_ptr(), ws.numel(), default_flags(), stream_of(dev), x);
+    if (rc != HQEKV_E_WORKSPACE || attempt) return rc;   // else the cache has outgrown the workspace of earlier steps
+  }
+}
+
+bool step_inputs(const Tensor &q, const Tensor &k, const Tensor &v, int64_t D) {
+  if (!q.is_cuda() || !plain_f16(q, 4, q.device()) || q.size(2) != 1 || q.size(3) != D) return false;
+  for (const Tensor *t : {&k, &v})
+    if (!plain_f16(*t, 4, q.device()) || t->size(0) != q.size(0) || t->size(2) != 1 || t->size(3) != D) return false;
+  return k.size(1) == v.size(1);
+}
+
+// StepTables.step(q, k, v, pkv, kbuf, vbuf, n, Tall, ring_store, ring_row, kv_seq_len): one decode step whose classes
+// cover every position once.  The residual is the first n token rows of the capacity buffers, k and v follow it as a
+// segment of their own and are copied to row n by the call's last launch; row `ring_row` of ring_store (None: no ring)
+// receives the ring row.  -> (attn_weights, attn_output, the next tuple), or None where the inputs are not plain.
+PyObject *tables_step(PyObject *self, PyObject *const *a, Py_ssize_t na) {
+  HANDLE_TH_ERRORS
+  if (na != 11) return PyErr_Format(PyExc_TypeError, "step takes 11 arguments");
+  StepTables *s = (StepTables *)self;
+  for (int i : {0, 1, 2, 4, 5})
+    if (!is_tensor(a[i])) Py_RETURN_NONE;
+  const Tensor &q = ten(a[0]), &k = ten(a[1]), &v = ten(a[2]), &kb = ten(a[4]), &vb = ten(a[5]);
+  PyObject *pkv = a[3];
+  const int64_t n = PyLong_AsLongLong(a[6]), Tall = PyLong_AsLongLong(a[7]), row = PyLong_AsLongLong(a[9]);
+  if (PyErr_Occurred()) return nullptr;
+  const int64_t D = kb.dim() == 4 ? kb.size(3) : 0;
+  if (!step_inputs(q, k, v, D) || !PyTuple_Check(pkv) || PyTuple_GET_SIZE(pkv) != TUPLE_LEN) Py_RETURN_NONE;
+  const at::Device dev = q.device();
+  for (const Tensor *b : {&kb, &vb})
+    if (!plain_f16(*b, 4, dev) || b->size(0) != q.size(0) || b->size(1) != k.size(1) || b->size(3) != D || n < 0 || n >= b->size(2)) Py_RETURN_NONE;
+  hqekv_step_extra x{};
+  if (a[8] != Py_None) {
+    if (!is_tensor(a[8])) Py_RETURN_NONE;
+    const Tensor &ring = ten(a[8]);
+    if (!plain_f16(ring, 2, dev) || row < 0 || row >= ring.size(0) || ring.size(1) < Tall) Py_RETURN_NONE;
+    x.ring_line = (char *)ring.data_ptr() + 2 * row * ring.size(1);
+  }
+  const int64_t cap_k = kb.size(2), cap_v = vb.size(2);
+  int n_k = s->n_k, n_v = s->n_v;
+  if (n) {
+    f16_rows(s->k[n_k++], HQEKV_LAYOUT_TOKEN_MAJOR, n, Tall - 1 - n, kb.data_ptr(), cap_k);
+    f16_rows(s->v[n_v++], 0, n, Tall - 1 - n, vb.data_ptr(), cap_v);
+  }
+  f16_rows(s->k[n_k++], HQEKV_LAYOUT_TOKEN_MAJOR, 1, Tall - 1, k.data_ptr(), 0);
+  f16_rows(s->v[n_v++], 0, 1, Tall - 1, v.data_ptr(), 0);
+  const c10::OptionalDeviceGuard guard(dev);
+  Tensor weights = new_tensor({q.size(0), q.size(1), 1, Tall}, at::kHalf, dev), out = new_tensor({q.size(0), q.size(1), 1, D}, at::kHalf, dev);
+  // (how torch's reduction deals the head rows to threads: attention.ring_order)
+  x.ring_order = Tall % 4 == 0 && Tall >= 256 && (uintptr_t)weights.data_ptr() % 8 == 0 ? 2 : 1;
+  x.append_rows = 1;
+  x.new_k = k.data_ptr();
+  x.new_v = v.data_ptr();
+  x.k_dst = (char *)kb.data_ptr() + 2 * D * n;
+  x.v_dst = (char *)vb.data_ptr() + 2 * D * n;
+  x.k_dst_slab_tokens = cap_k;
+  x.v_dst_slab_tokens = cap_v;
+  const int rc = run_step(s->k, n_k, s->v, n_v, q, weights, out, k.size(1), Tall, s->ws, dev, &x);
+  if (rc) return raise_rc(rc, "decode_step");
+  PyObject *next = PyTuple_New(TUPLE_LEN);
+  if (!next) return nullptr;
+  for (int i = 0; i < NEW_K; ++i) {
+    PyObject *o = PyTuple_GET_ITEM(pkv, i);
+    Py_INCREF(o);
+    PyTuple_SET_ITEM(next, i, o);
+  }
+  PyTuple_SET_ITEM(next, NEW_K, THPVariable_Wrap(kb.slice(2, 0, n + 1)));
+  PyTuple_SET_ITEM(next, NEW_V, THPVariable_Wrap(vb.slice(2, 0, n + 1)));
+  Py_INCREF(a[10]);
+  PyTuple_SET_ITEM(next, TUPLE_LEN - 1, a[10]);
+  return Py_BuildValue("NNN", THPVariable_Wrap(weights), THPVariable_Wrap(out), next);
+  END_HANDLE_TH_ERRORS
+}
+
+PyMethodDef tables_methods[] = {
+    {"step", (PyCFunction)(void (*)(void))tables_step, METH_FASTCALL, nullptr},
+    {nullptr, nullptr, 0, nullptr},
+};
+PyTypeObject tables_type = {PyVarObject_HEAD_INIT(nullptr, 0)};
+
+// What KiviAttentionLayer keeps between two decode steps: the K class, the fp16 K tail in a buffer of residual_length
+// rows, the V tail as a window [v0, v0 + nv) of a longer buffer, the V class in capacity buffers, and the tuple (views of
+// all this) it handed out last.
+struct KiviState {
+  PyObject_HEAD
+  Tensor kq, ks, kz, kt, vt, vcode, vscale, vzero, ws;
+  int64_t nk, v0, nv, n_vq;
+  PyObject *returned;   // the tuple handed out last
+};
+
+PyObject *kivi_new(PyTypeObject *type, PyObject *, PyObject *) {
+  KiviState *s = (KiviState *)type->tp_alloc(type, 0);
+  if (!s) return nullptr;
+  for (Tensor *t : {&s->kq, &s->ks, &s->kz, &s->kt, &s->vt, &s->vcode, &s->vscale, &s->vzero, &s->ws}) new (t) Tensor();
+  s->nk = s->v0 = s->nv = s->n_vq = 0;
+  Py_INCREF(Py_None);
+  s->returned = Py_None;
+  return (PyObject *)s;
+}
+void kivi_free(PyObject *o) {
+  KiviState *s = (KiviState *)o;
+  for (Tensor *t : {&s->kq, &s->ks, &s->kz, &s->kt, &s->vt, &s->vcode, &s->vscale, &s->vzero, &s->ws}) t->~Tensor();
+  Py_CLEAR(s->returned);
+  Py_TYPE(o)->tp_free(o);
+}
+
+template <Tensor KiviState::*F>
+PyObject *kivi_get(PyObject *o, void *) {
+  const Tensor &t = ((KiviState *)o)->*F;
+  if (!t.defined()) Py_RETURN_NONE;
+  return THPVariable_Wrap(t);
+}
+template <Tensor KiviState::*F>
+int kivi_set(PyObject *o, PyObject *v, void *) {
+  if (!v || (v != Py_None && !is_tensor(v))) {
+    PyErr_SetString(PyExc_TypeError, "a tensor or None");
+    return -1;
+  }
+  ((KiviState *)o)->*F = v == Py_None ? Tensor() : ten(v);
+  return 0;
+}
+template <int64_t KiviState::*F>
+PyObject *kivi_get_int(PyObject *o, void *) {
+  return PyLong_FromLongLong(((KiviState *)o)->*F);
+}
+template <int64_t KiviState::*F>
+int kivi_set_int(PyObject *o, PyObject *v, void *) {
+  const long long n = v ? PyLong_AsLongLong(v) : -1;
+  if (n < 0) {
+    if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "a count");
+    return -1;
+  }
+  ((KiviState *)o)->*F = n;
+  return 0;
+}
+PyObject *kivi_get_returned(PyObject *o, void *) {
+  PyObject *r = ((KiviState *)o)->returned;
+  Py_INCREF(r);
+  return r;
+}
+PyGetSetDef kivi_fields[] = {
+#define F(n_) {#n_, kivi_get<&KiviState::n_>, kivi_set<&KiviState::n_>, nullptr, nullptr}
+    F(kq), F(ks), F(kz), F(kt), F(vt), F(vcode), F(vscale), F(vzero),
+#undef F
+#define F(n_) {#n_, kivi_get_int<&KiviState::n_>, kivi_set_int<&KiviState::n_>, nullptr, nullptr}
+    F(nk), F(v0), F(nv), F(n_vq),
+#undef F
+    {"returned", kivi_get_returned, nullptr, nullptr, nullptr},
+    {nullptr, nullptr, nullptr, nullptr, nullptr},
+};
+
+// KiviState.step(q, k, v, T, k_bits, v_bits): the attention over (K class, K tail, this step's key) and (V class, V tail,
+// this step's value), the two rows appended behind their tails by the call's last launch, and -- when the tail is full
+// -- the quantiser launch that moves the oldest value row into the class buffers, which must have room for it.  Leaves a full K tail
+// (nk == its capacity) and a V window at the end of its buffer to the caller.  -> (attn_weights, attn_output) or None.
+PyObject *kivi_step(PyObject *self, PyObject *const *a, Py_ssize_t na) {
+  HANDLE_TH_ERRORS
+  if (na != 6) return PyErr_Format(PyExc_TypeError, "step takes 6 arguments");
+  KiviState *s = (KiviState *)self;
+  for (int i : {0, 1, 2})
+    if (!is_tensor(a[i])) Py_RETURN_NONE;
+  const Tensor &q = ten(a[0]), &k = ten(a[1]), &v = ten(a[2]);
+  const int64_t T = PyLong_AsLongLong(a[3]);
+  const int k_bits = (int)PyLong_AsLong(a[4]), v_bits = (int)PyLong_AsLong(a[5]);
+  if (PyErr_Occurred()) return nullptr;
+  if (!s->kt.defined() || !s->vt.defined() || !s->vcode.defined()) return PyErr_Format(PyExc_ValueError, "no buffers");
+  const int64_t D = s->kt.size(3), Hkv = s->kt.size(1), R = s->kt.size(2), cap_v = s->vt.size(2), row = 2 * D;
+  if (!step_inputs(q, k, v, D) || k.size(1) != Hkv) Py_RETURN_NONE;
+  const bool leaves = s->nv + 1 > R;   // a value row leaves the tail after this step
+  const int64_t n_kq = s->kq.defined() ? s->kq.size(3) * (32 / k_bits) : 0;
+  if (s->nk >= R || s->v0 + s->nv >= cap_v || s->n_vq + leaves > s->vcode.size(2) || n_kq + s->nk + 1 != T || s->n_vq + s->nv + 1 != T ||
+      s->kt.size(0) != q.size(0))
+    return PyErr_Format(PyExc_ValueError, "KiviAttentionLayer: the buffers do not hold the sequence before this step");
+  const at::Device dev = q.device();
+  hqekv_seg ks[3] = {}, vs[3] = {};
+  int n_k = 0, n_v = 0;
+  if (n_kq) {
+    hqekv_seg &e = ks[n_k++];
+    e.bits = k_bits;
+    e.n_tokens = n_kq;
+    e.data = s->kq.data_ptr();
+    e.scale = s->ks.data_ptr();
+    e.zero = s->kz.data_ptr();
+  }
+  if (s->nk) f16_rows(ks[n_k++], HQEKV_LAYOUT_TOKEN_MAJOR, s->nk, n_kq, s->kt.data_ptr(), R);
+  f16_rows(ks[n_k++], HQEKV_LAYOUT_TOKEN_MAJOR, 1, T - 1, k.data_ptr(), 0);
+  if (s->n_vq) {
+    hqekv_seg &e = vs[n_v++];
+    e.bits = v_bits;
+    e.n_tokens = s->n_vq;
+    e.data = s->vcode.data_ptr();
+    e.scale = s->vscale.data_ptr();
+    e.zero = s->vzero.data_ptr();
+    e.slab_tokens = s->vcode.size(2);
+  }
+  char *vt = (char *)s->vt.data_ptr();
+  if (s->nv) f16_rows(vs[n_v++], 0, s->nv, s->n_vq, vt + s->v0 * row, cap_v);
+  f16_rows(vs[n_v++], 0, 1, T - 1, v.data_ptr(), 0);
+  hqekv_step_extra x{};
+  x.append_rows = 1;
+  x.new_k = k.data_ptr();
+  x.new_v = v.data_ptr();
+  x.k_dst = (char *)s->kt.data_ptr() + s->nk * row;
+  x.v_dst = vt + (s->v0 + s->nv) * row;
+  x.k_dst_slab_tokens = R;
+  x.v_dst_slab_tokens = cap_v;
+  const c10::OptionalDeviceGuard guard(dev);
+  Tensor weights = new_tensor({q.size(0), q.size(1), 1, T}, at::kHalf, dev), out = new_tensor({q.size(0), q.size(1), 1, D}, at::kHalf, dev);
+  int rc = run_step(ks, n_k, vs, n_v, q, weights, out, Hkv, T, s->ws, dev, &x);
+  if (rc) return raise_rc(rc, "KiviAttentionLayer");
+  s->nk += 1;
+  s->nv += 1;
+  if (leaves) {
+    const int64_t words = s->vcode.size(3), groups = s->vscale.size(3), cap = s->vcode.size(2), n = s->n_vq;
+    rc = api.hqekv_quant_pack_rows(vt + s->v0 * row, cap_v * D, D, (char *)s->vcode.data_ptr() + n * words * 4, cap * words, words,
+                                   (char *)s->vscale.data_ptr() + n * groups * 2, (char *)s->vzero.data_ptr() + n * groups * 2, cap * groups,
+                                   groups, q.size(0) * Hkv, 1, D, v_bits, stream_of(dev));
+    if (rc) return raise_rc(rc, "uniform_group_quantize_pack_last_dim");
+    s->n_vq += 1;
+    s->v0 += 1;
+    s->nv -= 1;
+  }
+  return Py_BuildValue("NN", THPVariable_Wrap(weights), THPVariable_Wrap(out));
+  END_HANDLE_TH_ERRORS
+}
+
+// KiviState.fields(T): the 9-field tuple of views over the buffers, remembered as the one handed out last
+PyObject *kivi_tuple(PyObject *self, PyObject *T) {
+  HANDLE_TH_ERRORS
+  KiviState *s = (KiviState *)self;
+  auto put = [](PyObject *t, int i, const Tensor &x) {
+    if (x.defined()) {
+      PyTuple_SET_ITEM(t, i, THPVariable_Wrap(x));
+    } else {
+      Py_INCREF(Py_None);
+      PyTuple_SET_ITEM(t, i, Py_None);
+    }
+  };
+  auto head = [](const Tensor &x, int64_t n) { return n ? x.slice(2, 0, n) : Tensor(); };
+  PyObject *t = PyTuple_New(9);
+  if (!t) return nullptr;
+  put(t, 0, s->kq);
+  put(t, 1, head(s->kt, s->nk));
+  put(t, 2, s->ks);
+  put(t, 3, s->kz);
+  put(t, 4, head(s->vcode, s->n_vq));
+  put(t, 5, s->vt.slice(2, s->v0, s->v0 + s->nv));
+  put(t, 6, head(s->vscale, s->n_vq));
+  put(t, 7, head(s->vzero, s->n_vq));
+  Py_INCREF(T);
+  PyTuple_SET_ITEM(t, 8, T);
+  Py_INCREF(t);
+  Py_SETREF(s->returned, t);
+  return t;
+  END_HANDLE_TH_ERRORS
+}
+
+PyMethodDef kivi_methods[] = {
+    {"step", (PyCFunction)(void (*)(void))kivi_step, METH_FASTCALL, nullptr},
+    {"fields", kivi_tuple, METH_O, nullptr},
+    {nullptr, nullptr, 0, nullptr},
+};
+PyTypeObject kivi_type = {PyVarObject_HEAD_INIT(nullptr, 0)};
+
+// ------------------------------------------------------------------------------------------------ quantise and pack
+// quantize_into(data, bits, code, scale, mn) -> True, or None where a tensor is not plain (pack_unpack.quantize_pack_into)
+PyObject *quantize_into(PyObject *, PyObject *const *a, Py_ssize_t na) {
+  HANDLE_TH_ERRORS
+  if (na != 5) return PyErr_Format(PyExc_TypeError, "quantize_into takes 5 arguments");
+  for (int i : {0, 2, 3, 4})
+    if (!is_tensor(a[i])) Py_RETURN_NONE;
+  const Tensor &x = ten(a[0]), &code = ten(a[2]), &sc = ten(a[3]), &mn = ten(a[4]);
+  const int bits = (int)PyLong_AsLong(a[1]);
+  if (PyErr_Occurred()) return nullptr;
+  if (bits != 1 && bits != 2 && bits != 4 && bits != 8) Py_RETURN_NONE;
+  if (!x.is_cuda() || x.dim() != 4 || x.scalar_type() != at::kHalf || code.scalar_type() != at::kInt || sc.scalar_type() != at::kHalf ||
+      mn.scalar_type() != at::kHalf || !x.numel())
+    Py_RETURN_NONE;
+  const at::Device dev = x.device();
+  const int64_t B = x.size(0), H = x.size(1), R = x.size(2), L = x.size(3);
+  if (L % 32) Py_RETURN_NONE;
+  for (const Tensor *t : {&code, &sc, &mn}) {
+    if (t->dim() != 4 || t->device() != dev || t->size(0) != B || t->size(1) != H || t->size(2) != R || t->stride(3) != 1 ||
+        t->size(3) != (t == &code ? L * bits / 32 : L / 32) || t->stride(0) != H * t->stride(1))
+      Py_RETURN_NONE;
+  }
+  if (sc.stride(1) != mn.stride(1) || sc.stride(2) != mn.stride(2) || sc.stride(0) != mn.stride(0)) Py_RETURN_NONE;
+  // read in place: equally spaced (b, h) slabs of dense rows -- or, seen transposed, of dense token rows: the head of a
+  // longer tensor is not copied
+  const int64_t slab = x.stride(1);
+  if ((B > 1 && x.stride(0) != H * slab) || (H > 1 && slab < R * L)) Py_RETURN_NONE;
+  const bool token_major = x.stride(2) == 1 && x.stride(3) == R && R % 2 == 0 && R > 1 && slab % 2 == 0 && (uintptr_t)x.data_ptr() % 4 == 0;
+  const bool rows = x.stride(3) == 1 && x.stride(2) == L && slab % 8 == 0 && (uintptr_t)x.data_ptr() % 16 == 0;
+  if (!token_major && !rows) Py_RETURN_NONE;
+  const c10::OptionalDeviceGuard guard(dev);
+  const int rc = token_major ? api.hqekv_quant_pack_k_tokenmajor(x.data_ptr(), slab, R, code.data_ptr(), code.stride(1), code.stride(2),
+                                                                 sc.data_ptr(), mn.data_ptr(), sc.stride(1), sc.stride(2), B * H, L, R, bits,
+                                                                 stream_of(dev))
+                             : api.hqekv_quant_pack_rows(x.data_ptr(), slab, L, code.data_ptr(), code.stride(1), code.stride(2), sc.data_ptr(),
+                                                         mn.data_ptr(), sc.stride(1), sc.stride(2), B * H, R, L, bits, stream_of(dev));
+  if (rc) return raise_rc(rc, "uniform_group_quantize_pack_last_dim");
+  Py_RETURN_TRUE;
+  END_HANDLE_TH_ERRORS
+}
+
+// bind(path): take the kernels' entry points from this library
+PyObject *bind(PyObject *, PyObject *path) {
+  const char *p = PyUnicode_AsUTF8(path);
+  if (!p) return nullptr;
+  void *h = dlopen(p, RTLD_NOW | RTLD_LOCAL);
+  if (!h) return PyErr_Format(PyExc_RuntimeError, "%s", dlerror());
+#define X(n_)                                     \
+  api.n_ = (decltype(&::n_))dlsym(h, #n_);        \
+  if (!api.n_) return PyErr_Format(PyExc_RuntimeError, "%s lacks %s", p, #n_);
+  HQ_SYMBOLS(X)
+#undef X
+  Py_RETURN_NONE;
+}
+
+PyMethodDef module_methods[] = {
+    {"bind", bind, METH_O, nullptr},
+    {"decode", (PyCFunction)(void (*)(void))decode, METH_FASTCALL, nullptr},
+    {"quantize_into", (PyCFunction)(void (*)(void))quantize_into, METH_FASTCALL, nullptr},
+    {nullptr, nullptr, 0, nullptr},
+};
+PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, module_methods};
+
+bool add_type(PyObject *m, PyTypeObject &t, const char *qualified, const char *name, size_t size, newfunc make, destructor free_,
+              PyMethodDef *methods, PyGetSetDef *fields, unsigned long flags) {
+  t.tp_name = qualified;
+  t.tp_basicsize = (Py_ssize_t)size;
+  t.tp_flags = Py_TPFLAGS_DEFAULT | flags;
+  t.tp_new = make;
+  t.tp_dealloc = free_;
+  t.tp_methods = methods;
+  t.tp_getset = fields;
+  if (PyType_Ready(&t) < 0) return false;
+  Py_INCREF(&t);
+  return PyModule_AddObject(m, name, (PyObject *)&t) == 0;
+}
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__host(void) {
+  PyObject *m = PyModule_Create(&module_def);
+  if (!m) return nullptr;
+  s_cover = PyUnicode_InternFromString("_hq_cover");
+  if (!s_cover ||
+      !add_type(m, tables_type, "hqekv_amd._host.StepTables", "StepTables", sizeof(StepTables), tables_new, tables_free, tables_methods,
+                nullptr, 0) ||
+      !add_type(m, kivi_type, "hqekv_amd._host.KiviState", "KiviState", sizeof(KiviState), kivi_new, kivi_free, kivi_methods, kivi_fields, 0)) {
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
+}

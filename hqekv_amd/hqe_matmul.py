@@ -9,7 +9,8 @@ from typing import Tuple
 
 import torch
 
-from .attention import decode_attention, value_length
+from . import _lib
+from .attention import decode_attention, idx_cover_once, value_length
 
 
 def qkv_matmul_hqe_2(q: torch.Tensor, past_key_value: Tuple, attention_mask, head_dim: int,
@@ -24,11 +25,16 @@ def qkv_matmul_hqe_2(q: torch.Tensor, past_key_value: Tuple, attention_mask, hea
         raise ValueError('invalid quant_strategy')
     if block_size != 32 or group_size != 32:
         raise ValueError("block_size and group_size must be 32")
+    low_uniform = quant_strategy == "uniform_group"
+    if memo is None and tail is None and step is None:
+        done = _lib.host().decode(q, past_key_value, low_uniform, idx_cover_once)
+        if done is not None:   # (a cache that is not plain, or whose classes do not cover every position once, goes on below)
+            return done
     real_len = value_length(past_key_value) + (tail[1].shape[2] if tail is not None else 0)
     if real_len == 0:
         raise ValueError('invalid past_key_value')
     return decode_attention(q, past_key_value, None, real_len, zero_init=False,
-                            low_uniform=quant_strategy == "uniform_group", memo=memo, tail=tail, step=step)
+                            low_uniform=low_uniform, memo=memo, tail=tail, step=step)
 
 
 def qkv_matmul_hqe(q: torch.Tensor, past_key_value: Tuple, attention_mask, head_dim: int,

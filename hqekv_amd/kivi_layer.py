@@ -22,19 +22,7 @@ import torch
 from . import _lib
 from .attention import K_BASE, NEW_K, NEW_V, V_BASE, SegmentMemo, decode_attention, default_flags
 from .decode_layer import gqa_prompt_attention
-from .pack_unpack import uniform_group_quantize_pack_last_dim
-
-
-class _Buffers:
-    """What a ``KiviAttentionLayer`` keeps between decode steps: the K class tensors, the K tail in a buffer of
-    ``residual_length`` rows, the V tail as a window [v0, v0 + nv) of a longer buffer, the V class in capacity buffers,
-    and the tuple (views of all this) it handed out last."""
-    __slots__ = ("kq", "ks", "kz", "kt", "nk", "vt", "cap_vt", "v0", "nv", "vcode", "vscale", "vzero", "n_vq", "returned",
-                 "extra")
-
-    def __init__(self):
-        self.returned = None
-        self.extra = _lib.StepExtra()
+from .pack_unpack import quantize_pack_into, uniform_group_quantize_pack_last_dim
 
 
 class KiviAttentionLayer:
@@ -58,28 +46,39 @@ class KiviAttentionLayer:
         self._k_segs = (_lib.Seg * 3)()   # (quantised class, fp16 tail, this step's token) of each side, rewritten every step
         self._v_segs = (_lib.Seg * 3)()
         self._ws: Optional[torch.Tensor] = None
-        self._st = None                   # buffers behind the tuple this layer handed out last (see _Buffers)
+        self._st = None                   # buffers behind the tuple this layer handed out last (a _host.KiviState)
         self.in_place = True              # decode steps append in capacity buffers (False: upstream's cat / slice sequence)
 
     # ------------------------------------------------------------------ prompt
     def _prefill(self, q, k, v, attention_mask):
-        n_rep = q.shape[1] // k.shape[1]
+        """-> (output, the first eight fields of the tuple, None), or (output, None, the buffers that hold them) where the decode steps
+        will append in place: what such a step needs is quantised and copied straight into its capacity buffers."""
         T, R = k.shape[-2], self.residual_length
         out = gqa_prompt_attention(q, k, v, attention_mask, self.scaling)   # grouped heads: no repeat_kv copies
         tail = T % R
         k_quant = k if tail == 0 else (k[:, :, :T - tail, :] if T >= R else None)
-        k_full = None if tail == 0 else k[:, :, T - tail:, :].contiguous()
         kq = ks = kz = None
         if k_quant is not None:
             # (B,Hkv,D,T) view of token-major memory: the quantiser reads it in place
             kq, ks, kz = uniform_group_quantize_pack_last_dim(k_quant.transpose(2, 3), self.group_size, self.k_bits)
-        if T <= R:
+        n_vq = max(0, T - R)
+        if self._runs_in_place(q) and k.dtype == v.dtype == torch.float16:
+            st = self._buffers(k, n_vq)
+            st.kq, st.ks, st.kz = kq, ks, kz
+            if tail:
+                st.kt[:, :, :tail].copy_(k[:, :, T - tail:])
+            st.nk, st.nv, st.n_vq = tail, T - n_vq, n_vq
+            st.vt[:, :, :T - n_vq].copy_(v[:, :, n_vq:])
+            if n_vq:
+                quantize_pack_into(v[:, :, :n_vq], self.v_bits, *(x[:, :, :n_vq] for x in (st.vcode, st.vscale, st.vzero)))
+            return out, None, st
+        k_full = None if tail == 0 else k[:, :, T - tail:, :].contiguous()
+        if n_vq == 0:
             vq, v_full, vs, vz = None, v, None, None
         else:
-            v_full = v[:, :, T - R:, :].contiguous()
-            vq, vs, vz = uniform_group_quantize_pack_last_dim(v[:, :, :T - R, :].contiguous(), self.group_size,
-                                                              self.v_bits)
-        return out, (kq, k_full, ks, kz, vq, v_full, vs, vz)
+            v_full = v[:, :, n_vq:, :].contiguous()
+            vq, vs, vz = uniform_group_quantize_pack_last_dim(v[:, :, :n_vq, :], self.group_size, self.v_bits)
+        return out, (kq, k_full, ks, kz, vq, v_full, vs, vz), None
 
     # ------------------------------------------------------------------ decode attention
     def _attend(self, q, kq, ks, kz, k_full, vq, vs, vz, v_full, T: int):
@@ -131,42 +130,53 @@ class KiviAttentionLayer:
         return weights, out
 
     # ------------------------------------------------------------------ a decode step in place
-    def _adopt(self, pkv: tuple, like: torch.Tensor) -> "_Buffers":
+    def _runs_in_place(self, q: torch.Tensor) -> bool:
+        return self.in_place and q.is_cuda and q.dtype == torch.float16 and self.head_dim == q.shape[-1] == 128
+
+    def _buffers(self, like: torch.Tensor, n_vq: int):
+        """Empty capacity buffers for a sequence with ``n_vq`` value rows in the quantised class."""
+        B, H, _, D = like.shape
+        dev, R = like.device, self.residual_length
+        st = _lib.host().KiviState()
+        st.kt = torch.empty(B, H, R, D, dtype=torch.float16, device=dev)
+        st.vt = torch.empty(B, H, 2 * R + 32, D, dtype=torch.float16, device=dev)   # the tail's window slides one row per step
+        self._grow_v_class(st, B, H, D, dev, n_vq + 1)
+        return st
+
+    def _adopt(self, pkv: tuple, like: torch.Tensor):
         """Capacity buffers holding what ``pkv`` holds: the K tail, the V tail (a window that slides one row per step)
         and the V class (which grows one row per step).  The K class stays as it is: it changes every
         ``residual_length`` steps only."""
         kq, k_full, ks, kz, vq, v_full, vs, vz, _ = pkv
-        B, H, _, D = like.shape
-        dev, R = like.device, self.residual_length
-        st = _Buffers()
-        st.kq, st.ks, st.kz = kq, ks, kz
-        st.kt = torch.empty(B, H, R, D, dtype=torch.float16, device=dev)
+        n_vq = 0 if vq is None else vq.shape[2]
+        st = self._buffers(like, n_vq)
+        if kq is not None:
+            st.kq, st.ks, st.kz = kq.contiguous(), ks.contiguous(), kz.contiguous()
         st.nk = 0 if k_full is None else k_full.shape[2]
         if st.nk:
             st.kt[:, :, :st.nk].copy_(k_full)
-        st.cap_vt = 2 * R + 32
-        st.vt = torch.empty(B, H, st.cap_vt, D, dtype=torch.float16, device=dev)
-        st.v0, st.nv = 0, (0 if v_full is None else v_full.shape[2])
+        st.nv = 0 if v_full is None else v_full.shape[2]
         if st.nv:
             st.vt[:, :, :st.nv].copy_(v_full)
-        st.n_vq = 0 if vq is None else vq.shape[2]
-        st.vcode = st.vscale = st.vzero = None
-        self._grow_v_class(st, B, H, D, dev, st.n_vq + 1, (vq, vs, vz))
+        st.n_vq = n_vq
+        if n_vq:
+            for dst, src in ((st.vcode, vq), (st.vscale, vs), (st.vzero, vz)):
+                dst[:, :, :n_vq].copy_(src)
         return st
 
-    def _grow_v_class(self, st: "_Buffers", B: int, H: int, D: int, dev, need: int, old=None) -> None:
-        """Room for ``need`` rows in the V class buffers (doubling); ``old`` = (codes, scale, zero) to take over."""
-        if st.vcode is not None and need <= st.vcode.shape[2]:
+    def _grow_v_class(self, st, B: int, H: int, D: int, dev, need: int) -> None:
+        """Room for ``need`` rows in the V class buffers (doubling)."""
+        old = (st.vcode, st.vscale, st.vzero)
+        if old[0] is not None and need <= old[0].shape[2]:
             return
         cap = max(self.MIN_V_ROWS, 2 * need)
         code = torch.empty(B, H, cap, D * self.v_bits // 32, dtype=torch.int32, device=dev)
         scale = torch.empty(B, H, cap, D // 32, dtype=torch.float16, device=dev)
         zero = torch.empty_like(scale)
-        src = old if old is not None else (st.vcode, st.vscale, st.vzero)
-        if st.n_vq and src[0] is not None:
-            code[:, :, :st.n_vq].copy_(src[0][:, :, :st.n_vq])
-            scale[:, :, :st.n_vq].copy_(src[1][:, :, :st.n_vq])
-            zero[:, :, :st.n_vq].copy_(src[2][:, :, :st.n_vq])
+        n = st.n_vq
+        if n:
+            for dst, src in zip((code, scale, zero), old):
+                dst[:, :, :n].copy_(src[:, :, :n])
         st.vcode, st.vscale, st.vzero = code, scale, zero
 
     def _step_in_buffers(self, q, k, v, pkv: tuple, T: int):
@@ -174,90 +184,31 @@ class KiviAttentionLayer:
         step's key) and (V class, V tail, this step's value) with the two rows copied behind their tails in the
         call's last launch, one quantiser launch when the oldest value row leaves the tail (written straight into the
         class buffers), one concatenation every ``residual_length`` steps when a block of keys is quantised.  The
-        tuple handed back holds views of the buffers, with upstream's shapes and contents [117-266]."""
+        tuple handed back holds views of the buffers, with upstream's shapes and contents [117-266].  None: an input is
+        not what the native step takes."""
         q, k, v = (x if x.is_contiguous() else x.contiguous() for x in (q, k, v))
+        R = self.residual_length
         st = self._st
         if st is None or st.returned is not pkv:
             st = self._st = self._adopt(pkv, k)
-        B, Hq, _, D = q.shape
-        Hkv, R, dev = k.shape[1], self.residual_length, q.device
-        n_kq = 0 if st.kq is None else st.kq.shape[3] * (32 // self.k_bits)
-        row = 2 * D   # bytes per token row
-
-        def seg(e, bits, layout, n, pos, data, scale=None, zero=None, slab=0):
-            e.bits, e.layout, e.n_tokens, e.pos_base, e.slab_tokens = bits, layout, n, pos, slab
-            e.data, e.scale, e.zero, e.idx = data, scale, zero, None
-
-        ka, n_k = self._k_segs, 0
-        if n_kq:
-            seg(ka[n_k], self.k_bits, 0, n_kq, 0, st.kq.data_ptr(), st.ks.data_ptr(), st.kz.data_ptr())
-            n_k += 1
-        if st.nk:
-            seg(ka[n_k], 16, _lib.LAYOUT_TOKEN_MAJOR, st.nk, n_kq, st.kt.data_ptr(), slab=R)
-            n_k += 1
-        seg(ka[n_k], 16, _lib.LAYOUT_TOKEN_MAJOR, 1, T - 1, k.data_ptr())
-        n_k += 1
-        va, n_v = self._v_segs, 0
-        if st.n_vq:
-            seg(va[n_v], self.v_bits, 0, st.n_vq, 0, st.vcode.data_ptr(), st.vscale.data_ptr(), st.vzero.data_ptr(),
-                slab=st.vcode.shape[2])
-            n_v += 1
-        if st.nv:
-            seg(va[n_v], 16, 0, st.nv, st.n_vq, st.vt.data_ptr() + st.v0 * row, slab=st.cap_vt)
-            n_v += 1
-        seg(va[n_v], 16, 0, 1, T - 1, v.data_ptr())
-        n_v += 1
-        x = st.extra
-        x.ring_line, x.append_rows, x.new_k, x.new_v = None, 1, k.data_ptr(), v.data_ptr()
-        x.k_dst, x.v_dst = st.kt.data_ptr() + st.nk * row, st.vt.data_ptr() + (st.v0 + st.nv) * row
-        x.k_dst_slab_tokens, x.v_dst_slab_tokens = R, st.cap_vt
-        weights = torch.empty(B, Hq, 1, T, dtype=torch.float16, device=dev)
-        out = torch.empty(B, Hq, 1, D, dtype=torch.float16, device=dev)
-        lib = _lib.load()
-        import ctypes as C
-        with _lib.on_device(dev):
-            for attempt in (0, 1):
-                if self._ws is None or self._ws.device != dev or attempt:
-                    need = lib.hqekv_decode_workspace_bytes(ka, n_k, va, n_v, B, Hq, Hkv, D)
-                    if need < 0:
-                        raise ValueError("invalid segment table")
-                    self._ws = torch.empty(max(2 * need, 256) // 4, dtype=torch.float32, device=dev)
-                rc = lib.hqekv_decode_step(ka, n_k, va, n_v, q.data_ptr(), None, 0, weights.data_ptr(), out.data_ptr(),
-                                           B, Hq, Hkv, D, T, self._ws.data_ptr(), self._ws.numel() * 4, default_flags(),
-                                           _lib.stream_ptr(dev), C.byref(x))
-                if rc != -3:   # HQEKV_E_WORKSPACE: the cache has outgrown the workspace kept from earlier steps
-                    break
-            _lib.check(rc, "KiviAttentionLayer")
-            st.nk += 1
-            st.nv += 1
-            if st.nk == R:   # a full block of fp16 keys: quantise it per channel, straight from its rows [236-252]
-                c, s_, z = uniform_group_quantize_pack_last_dim(st.kt.transpose(2, 3), self.group_size, self.k_bits)
-                st.kq = c if st.kq is None else torch.cat((st.kq, c), dim=3)
-                st.ks = s_ if st.ks is None else torch.cat((st.ks, s_), dim=3)
-                st.kz = z if st.kz is None else torch.cat((st.kz, z), dim=3)
-                st.nk = 0
-            if st.nv > R:    # the oldest fp16 value row leaves the tail for the class [254-264]
-                self._grow_v_class(st, B, Hkv, D, dev, st.n_vq + 1)
-                code, scale, zero = st.vcode, st.vscale, st.vzero
-                n = st.n_vq
-                _lib.check(lib.hqekv_quant_pack_rows(
-                    st.vt.data_ptr() + st.v0 * row, st.cap_vt * D, D,
-                    code.data_ptr() + n * code.stride(2) * 4, code.stride(1), code.stride(2),
-                    scale.data_ptr() + n * scale.stride(2) * 2, zero.data_ptr() + n * zero.stride(2) * 2,
-                    scale.stride(1), scale.stride(2), B * Hkv, 1, D, self.v_bits, _lib.stream_ptr(dev)),
-                    "uniform_group_quantize_pack_last_dim")
-                st.n_vq += 1
-                st.v0 += 1
-                st.nv -= 1
-                if st.v0 + st.nv == st.cap_vt:   # the window has reached the end of its buffer: back to the start
-                    st.vt[:, :, :st.nv].copy_(st.vt[:, :, st.v0:st.v0 + st.nv].clone())
-                    st.v0 = 0
-        nq = st.n_vq
-        fields = (st.kq, st.kt[:, :, :st.nk] if st.nk else None, st.ks, st.kz,
-                  st.vcode[:, :, :nq] if nq else None, st.vt[:, :, st.v0:st.v0 + st.nv],
-                  st.vscale[:, :, :nq] if nq else None, st.vzero[:, :, :nq] if nq else None, T)
-        st.returned = fields
-        return out, weights, fields
+        if st.nv == R and st.n_vq == st.vcode.shape[2]:   # a value row is about to leave the tail [254-264]
+            self._grow_v_class(st, k.shape[0], k.shape[1], k.shape[3], k.device, st.n_vq + 1)
+        done = st.step(q, k, v, T, self.k_bits, self.v_bits)
+        if done is None:
+            self._st = None
+            return None
+        weights, out = done
+        if st.nk == R:   # a full block of fp16 keys: quantise it per channel, straight from its rows [236-252]
+            new = uniform_group_quantize_pack_last_dim(st.kt.transpose(2, 3), self.group_size, self.k_bits)
+            if st.kq is not None:
+                new = [torch.cat((old, x), dim=3) for old, x in zip((st.kq, st.ks, st.kz), new)]
+            st.kq, st.ks, st.kz = new
+            st.nk = 0
+        nv, v0 = st.nv, st.v0
+        if v0 + nv == st.vt.shape[2]:   # the window has reached the end of its buffer: back to the start
+            st.vt[:, :, :nv].copy_(st.vt[:, :, v0:v0 + nv].clone())
+            st.v0 = 0
+        return out, weights, st.fields(T)
 
     # ------------------------------------------------------------------ one call
     def forward(self, query_states: torch.Tensor, key_states: torch.Tensor, value_states: torch.Tensor,
@@ -268,13 +219,14 @@ class KiviAttentionLayer:
         L = key_states.shape[-2]
         kv_seq_len = L + (past_key_value[-1] if past_key_value is not None else 0)
         if past_key_value is None:
-            out, fields = self._prefill(query_states, key_states, value_states, attention_mask)
-            return out, None, fields + (kv_seq_len,)
+            out, fields, self._st = self._prefill(query_states, key_states, value_states, attention_mask)
+            return out, None, fields + (kv_seq_len,) if self._st is None else self._st.fields(kv_seq_len)
         if L != 1:
             raise ValueError("a decode step appends one token")
-        if (self.in_place and attention_mask is None and query_states.is_cuda and query_states.dtype == torch.float16
-                and self.head_dim == query_states.shape[-1] == 128):
-            return self._step_in_buffers(query_states, key_states, value_states, past_key_value, kv_seq_len)
+        if attention_mask is None and self._runs_in_place(query_states):
+            done = self._step_in_buffers(query_states, key_states, value_states, past_key_value, kv_seq_len)
+            if done is not None:
+                return done
         self._st = None
         kq, k_full, ks, kz, vq, v_full, vs, vz, _ = past_key_value
         R = self.residual_length

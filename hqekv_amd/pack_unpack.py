@@ -96,8 +96,12 @@ def quantize_pack_into(
     ``code`` (B, nh, R, L/pf) int32 and ``scale``/``mn`` (B, nh, R, L/32) fp16 may be windows of
     larger capacity-sized buffers (unit stride on the last axis); this is the append path.
     ``data`` may be contiguous or the ``.transpose(2, 3)`` view of a token-major tensor (how the
-    reference hands K to its quantiser, quant/hqe_2.py:32-35), which is read in place.
+    reference hands K to its quantiser, quant/hqe_2.py:32-35), or the first tokens of a longer such
+    tensor; all of these are read in place.
     """
+    if _lib.host().quantize_into(data, bit, code, scale, mn) is not None:
+        return
+    # what is left: invalid arguments, an empty input, an input that has to be made contiguous first
     pf = _check_bits(bit)
     _lib.require_gpu(data, "data")
     if data.dtype != torch.float16:
@@ -117,24 +121,8 @@ def quantize_pack_into(
             raise ValueError("outputs need a unit last stride and a flattenable (B, nh) prefix")
     if scale.stride() != mn.stride():
         raise ValueError("scale and mn must share strides")
-    lib = _lib.load()
-    st = _lib.stream_ptr(data.device)
-    with _lib.on_device(data.device):
-        tm = (data.stride(2) == 1 and data.stride(3) == R and data.stride(1) == R * L
-              and data.stride(0) == nh * R * L and R % 2 == 0 and R > 1)
-        if tm:
-            # token-major memory (B, nh, L, R): groups of 32 tokens per channel, read in place
-            _lib.check(lib.hqekv_quant_pack_k_tokenmajor(
-                data.data_ptr(), R * L, R, code.data_ptr(), code.stride(1), code.stride(2),
-                scale.data_ptr(), mn.data_ptr(), scale.stride(1), scale.stride(2),
-                B * nh, L, R, bit, st), "uniform_group_quantize_pack_last_dim")
-        else:
-            if not data.is_contiguous():
-                data = data.contiguous()
-            _lib.check(lib.hqekv_quant_pack_rows(
-                data.data_ptr(), R * L, L, code.data_ptr(), code.stride(1), code.stride(2),
-                scale.data_ptr(), mn.data_ptr(), scale.stride(1), scale.stride(2),
-                B * nh, R, L, bit, st), "uniform_group_quantize_pack_last_dim")
+    if _lib.host().quantize_into(data.contiguous(), bit, code, scale, mn) is None:
+        raise ValueError("the outputs must live on the input's device")
 
 
 def uniform_group_quantize_pack_last_dim(
