@@ -35,6 +35,7 @@ def qk_tiling(n: int) -> int:
 
 
 LAYOUT_TOKEN_MAJOR = 1   # fp16 K segment stored (B,Hkv,T,D)
+LAYOUT_RUNS = 4          # added to a layout: the index consists of whole runs of 32 consecutive positions
 LAYOUT_NORMAL1 = 2       # 1-bit segment in normal-quantile coding (scale = std, zero = mean)
 
 # every symbol include/hqekv.h declares
@@ -233,7 +234,7 @@ def make_segs(items) -> "C.Array[Seg]":
     arr = (Seg * max(1, len(items)))()
     for s, it in zip(arr, items):
         s.bits = it["bits"]
-        s.layout = LAYOUT_TOKEN_MAJOR if it.get("token_major") else int(it.get("layout", 0))
+        s.layout = int(it.get("layout", 0)) | (LAYOUT_TOKEN_MAJOR if it.get("token_major") else 0)
         s.n_tokens = it["n_tokens"]
         s.pos_base = int(it.get("pos_base", 0))
         s.data = ptr(it["data"])

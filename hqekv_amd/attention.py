@@ -154,15 +154,25 @@ def value_length(pkv: tuple) -> int:
     return n
 
 
-def _cover_on_device(idx_list, n: int) -> bool:
-    """The check of ``idx_cover_once`` as one launch over a bit per position (it waits for the answer)."""
+def _cover_on_device(idx_list, n: int):
+    """The checks of ``idx_cover_once`` as one launch over a bit per position (it waits for the answer).
+    -> (every position once, whole runs of 32 consecutive positions in every array)."""
     dev, k = idx_list[0].device, len(idx_list)
     scratch = torch.zeros(1 + (n + 31) // 32, dtype=torch.int32, device=dev)
     with _lib.on_device(dev):
         rc = _lib.load().hqekv_cover_once((C.c_void_p * k)(*[t.data_ptr() for t in idx_list]), (C.c_int64 * k)(*[t.numel() for t in idx_list]),
                                           k, scratch.data_ptr(), scratch.numel() * 4, _lib.stream_ptr(dev))
     _lib.check(rc, "cover_once")
-    return int(scratch[0]) == 0
+    status = int(scratch[0])
+    return not status & 1, not status & 2 and all(t.numel() % 32 == 0 for t in idx_list)
+
+
+def _whole_runs(a: np.ndarray) -> bool:
+    """Does ``a`` consist of whole runs of 32 consecutive positions?"""
+    if a.size % 32:
+        return False
+    r = a.reshape(-1, 32)
+    return bool((r == r[:, :1] + np.arange(32)).all())
 
 
 def idx_cover_once(idx_list, n: int) -> bool:
@@ -189,19 +199,31 @@ def idx_cover_once(idx_list, n: int) -> bool:
     if n % 32 == 0 and all(b is not None and b.shape[0] * 32 == t.numel() for b, t in zip(blocks, idx_list)):
         c = np.concatenate(blocks)   # whole aligned 32-token blocks: check the block numbers
         nb = n // 32
-        ok = bool(c.size == nb and (c >= 0).all() and (c < nb).all() and (np.bincount(c, minlength=nb) == 1).all())
+        ok, runs = bool(c.size == nb and (c >= 0).all() and (c < nb).all() and (np.bincount(c, minlength=nb) == 1).all()), True
     elif all(h is not None for h in hosts):
         c = np.concatenate(hosts)
         ok = bool(c.size == n and (c >= 0).all() and (c < n).all() and (np.bincount(c, minlength=n) == 1).all())
+        runs = all(_whole_runs(h) for h in hosts)
     elif idx_list[0].is_cuda and len(idx_list) <= _lib.MAX_SEGS and n < 2 ** 38 and \
             all(t.dtype == torch.int64 and t.is_contiguous() and t.device == idx_list[0].device for t in idx_list):
-        ok = _cover_on_device(idx_list, n)
+        ok, runs = _cover_on_device(idx_list, n)
     else:
         c = torch.cat([t.reshape(-1).to(torch.int64) for t in idx_list])
         inside = (c >= 0) & (c < n)
         ok = bool(inside.all() & (torch.bincount(c.clamp(0, n - 1), minlength=n) == 1).all())
-    idx_list[0]._hq_cover = (key, ok, [weakref.ref(t) for t in idx_list])
+        runs = all(_whole_runs(t.cpu().numpy().reshape(-1)) for t in idx_list)
+    idx_list[0]._hq_cover = (key, ok, [weakref.ref(t) for t in idx_list], ok and runs)
     return ok
+
+
+def mark_runs(items: List[dict]) -> None:
+    """Name the segments whose index arrays are known -- from ``idx_cover_once``, asked of exactly these arrays just now --
+    to consist of whole runs of 32 consecutive positions: the kernels then read one index per run."""
+    held = [it for it in items if it.get("idx") is not None]
+    hit = getattr(held[0]["idx"], "_hq_cover", None) if held else None
+    if hit is not None and hit[3] and len(hit[2]) == len(held) and all(r() is it["idx"] for r, it in zip(hit[2], held)):
+        for it in held:
+            it["layout"] = int(it.get("layout", 0)) | _lib.LAYOUT_RUNS
 
 
 def _class_idx(pkv: tuple, base0: int, bases) -> list:
@@ -305,6 +327,10 @@ class SegmentMemo:
         v_items, hv, dv = value_segments(pkv, dev, 0, self.keep, low_uniform, residual=False)
         if len(k_items) + 2 > _lib.MAX_SEGS or len(v_items) + 2 > _lib.MAX_SEGS:
             raise ValueError("too many segments")
+        self.partition = classes_partition_positions(pkv)
+        if self.partition:
+            mark_runs(k_items)
+            mark_runs(v_items)
         self.n_k, self.n_v = len(k_items), len(v_items)
         self.k_arr = (_lib.Seg * (self.n_k + 2))()   # two spare entries each: the residual and the step's new token
         self.v_arr = (_lib.Seg * (self.n_v + 2))()
@@ -316,7 +342,6 @@ class SegmentMemo:
         self.dims = (dk, dv)
         self.held = tuple(pkv[:NEW_K])
         self.key = (dev, low_uniform)
-        self.partition = classes_partition_positions(pkv)
         self._native = None
 
     @staticmethod
@@ -414,6 +439,9 @@ def decode_attention(q: torch.Tensor, pkv: tuple, mask, Tall: int, zero_init: bo
             v_items.append(dict(bits=16, n_tokens=n_tail, data=tv, idx=None, pos_base=Tall - n_tail))
             hk, dk, hv, dv = tk.shape[1], tk.shape[3], tv.shape[1], tv.shape[3]
         Hkv = hk if hk is not None else hv
+        if covered and use_flags & _lib.FUSE_SOFTMAX and mask is None:
+            mark_runs(k_items)
+            mark_runs(v_items)
         k_segs, v_segs, n_k, n_v = _lib.make_segs(k_items), _lib.make_segs(v_items), len(k_items), len(v_items)
     if Hkv is None:
         raise ValueError("invalid past_key_value")
@@ -480,6 +508,13 @@ class DecodePlan:
         self.Hkv = hk if hk is not None else hv
         if self.Hkv is None:
             raise ValueError("invalid past_key_value")
+        self.flags = default_flags() if flags is None else flags
+        if (self.flags & _lib.FUSE_SOFTMAX) and mask is None:
+            if classes_partition_positions(pkv):
+                mark_runs(k_items)
+                mark_runs(v_items)
+            else:
+                self.flags &= ~_lib.FUSE_SOFTMAX   # weights is zero-initialised below: uncovered positions stay 0
         self.B, self.Hq, self.D = B, Hq, D
         self.n_k, self.n_v = len(k_items), len(v_items)
         self.k_segs, self.v_segs = _lib.make_segs(k_items), _lib.make_segs(v_items)
@@ -488,9 +523,6 @@ class DecodePlan:
         self.mask_ptr, self.mask_stride = _mask_arg(mask, B, Hq, self.Tall, self.dev, self._keep)
         with _lib.on_device(self.dev):
             self.ws = decode_workspace(self.k_segs, self.n_k, self.v_segs, self.n_v, B, Hq, self.Hkv, D, self.dev)
-        self.flags = default_flags() if flags is None else flags
-        if (self.flags & _lib.FUSE_SOFTMAX) and mask is None and not classes_partition_positions(pkv):
-            self.flags &= ~_lib.FUSE_SOFTMAX   # weights is zero-initialised above: uncovered positions stay 0
         self._lib = _lib.load()
         self.inv_sqrt_d = 1.0 / (D ** 0.5)
 

@@ -19,7 +19,7 @@ ROOT = PKG.parent
 CSRC = PKG / "csrc"
 LIB = PKG / "libhqekv.so"
 HOST = PKG / "_host.so"
-SOURCES = ["capi.hip", "quant_pack.hip", "attn.hip", "decode_static.hip", "migrate.hip", "reconstruct.hip", "planner.hip", "importance.hip", "prompt_attn.hip"]
+SOURCES = ["capi.hip", "quant_pack.hip", "attn.hip", "decode_qk.hip", "decode_pv.hip", "decode_static.hip", "migrate.hip", "reconstruct.hip", "planner.hip", "importance.hip", "prompt_attn.hip"]
 
 HIPCC_FLAGS = [
     "-O3", "-std=c++17", "-fPIC", "--offload-arch=gfx950",

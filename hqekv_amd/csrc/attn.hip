@@ -22,338 +22,16 @@
 //            scale/zero and the gathered probabilities of a 512-token block are staged in LDS in
 //            pair-interleaved order; lanes are reduced by butterflies, waves through LDS, workgroups
 //            through fp32 partials summed in a fixed order.
-#include <stdlib.h>
+#include "attn_common.h"
+#include "decode_tiles.h"
 
-#include <type_traits>
-#include <utility>
-
-#include "common.h"
-
-#pragma clang fp contract(off)  // the two fp16 roundings of the dequantiser must stay separate
+#pragma clang fp contract(off)
 
 #ifndef HQ_DEFAULT_DOT_MFMA
 #define HQ_DEFAULT_DOT_MFMA true   // the form of the dot products for calls that name neither (see dot_on_matrix_cores)
 #endif
 
 namespace hq {
-
-struct SegDev {
-  const void *data;
-  const half_t *scale;
-  const half_t *zero;
-  const int64_t *idx;
-  int64_t pos_base;
-  int64_t n_tokens;
-  int32_t bits;
-  int32_t layout;      // HQEKV_LAYOUT_*: 1 = fp16 K stored token-major, 2 = 1-bit normal-quantile coding
-  int32_t unit_begin;  // first chunk of this segment in the p.V partial buffer
-  int32_t n_units;     // tiles (q.K^T) or chunks (p.V) of this segment
-  int64_t slab_tokens; // token rows between two (b, kv head) slabs of a token-major segment (>= n_tokens)
-};
-
-struct SegTable {
-  SegDev seg[HQEKV_MAX_SEGS];
-  int32_t nseg;
-  int32_t total_units;
-  int32_t max_units;   // the largest n_units of any segment
-  int32_t pad_;
-  int32_t begin[HQEKV_MAX_SEGS];  // first grid.y index of every segment (INT32_MAX past nseg): one scalar load finds a workgroup's segment
-};
-
-// grid.y enumerates the units of all segments back to back (no idle workgroups): unit u belongs to the last
-// segment whose first unit is <= u.  Branch-free on the eight begins, which arrive in one scalar load.
-__device__ __forceinline__ int seg_of_unit(const SegTable &tb, int u) {
-  int s = -1;
-#pragma unroll
-  for (int k = 0; k < HQEKV_MAX_SEGS; ++k) s += (u >= tb.begin[k]) ? 1 : 0;
-  return s;
-}
-// begin[s] without a second, dependent load from the argument segment
-__device__ __forceinline__ int begin_of_seg(const SegTable &tb, int s) {
-  int b = 0;
-#pragma unroll
-  for (int k = 0; k < HQEKV_MAX_SEGS; ++k) b += (k == s) ? tb.begin[k] : 0;
-  return b;
-}
-
-// Optional fusion of the softmax into the two GEMV launches (valid when no mask is added and the K
-// classes as well as the V classes each cover every position exactly once):
-//   q.K^T stores the scaled fp16 logit instead of the raw score and one (max, sum exp) pair per tile and
-//   head; p.V turns a logit into its probability while staging it and writes it back for the caller.
-// The split-K partials are summed by the LAST p.V workgroup of each (b, kv head) to finish, when there are few
-// enough of them; otherwise by a small launch of their own.  Nobody waits for anybody: a workgroup stores its
-// partial rows write-through (agent-scope relaxed stores go past the per-XCD L2), waits for the stores to be
-// acknowledged, and bumps one relaxed agent-scope counter; whoever reads the final count adds the rows up with
-// loads that bypass the L2 as well, in the fixed order of the separate launch.  No release / acquire fences are
-// involved: those write back and invalidate the whole L2 on this chip (the step went from 39 to 146 us with them).
-struct FuseArgs {
-  float2 *stats;       // (B*Hq, n_stat) pairs (m, l); nullptr = unfused
-  int32_t n_stat;      // tiles per row of stats = number of q.K^T tiles per (b, kv head)
-  float inv_sqrt_d;
-  // Folded combine (independent of the softmax fusion): one arrival counter per (b, kv head), zeroed by the q.K^T
-  // launch of the same call; nullptr = the split-K partials are summed by a launch of their own.
-  uint32_t *arrive;
-  half_t *out;         // (B*Hq, D) attention output, written by the last workgroup of each (b, kv head)
-  int32_t two_step;    // never fold the bias removal of a code into its multiply (HQEKV_TWO_STEP_DEQUANT)
-};
-// More than eight query heads per KV head are served in slices of at most eight, one launch each: the launch's NREP
-// heads are heads `off` .. `off` + NREP - 1 of the `group` query heads of their KV head (a launch that covers all
-// heads: group = NREP, off = 0).  Group and offset ride in the upper half of the kernels' head-count argument,
-// hq_slice = Hq | group << 16 | off << 24, and are used without a branch: as two members at the end of FuseArgs, or
-// behind a test for "no slices", the kernel's other scalar loads ended up behind a first, dependent one -- half a
-// microsecond in every workgroup -- and even one more plain argument moved the launches by a quarter.
-// -> first query head (inside its batch row) that a workgroup of KV head `hkv` works on
-__device__ __forceinline__ int first_head(int hq_slice, int hkv) { return hkv * ((hq_slice >> 16) & 0xff) + (int)((uint32_t)hq_slice >> 24); }
-__host__ __device__ constexpr int hq_with_slice(int Hq, int group, int off) { return Hq | group << 16 | off << 24; }
-
-// What the caller of a decode step does next to the attention (model/llama_hqe.py:131-133, 200), folded into the
-// step's last launch: the row of the importance ring -- the probabilities summed over the batch, rounded to fp16,
-// then summed over the heads and rounded again (model/public_func.py:243-257: attn_weights.sum(0).sum(0)) -- and
-// the copies that append the step's key and value rows to the fp16 residual.
-struct StepEpilogue {
-  const half_t *weights;   // (B, Hq, Tall) probabilities
-  half_t *ring_line;       // (Tall) or nullptr
-  int64_t Tall;
-  int32_t B, Hq;
-  int32_t ring_by;         // threads torch's reduction deals the head rows to for this shape: 1 or 2
-  int32_t app_rows;        // token rows to append per (b, kv head); 0 = none
-  int32_t app_row_elems;   // head_dim
-  int32_t app_bh;          // B * Hkv
-  const half_t *app_src[2];
-  half_t *app_dst[2];          // first destination row of slab 0
-  int64_t app_src_slab[2];     // elements between two (b, kv head) slabs
-  int64_t app_dst_slab[2];
-};
-
-// A workgroup learns its segment and its tile/chunk from its block id with two scalar loads at the top of
-// the kernel: the eight unit begins, then the segment's 64-byte entry (a scalar load that misses costs about
-// a microsecond; walking the table entry by entry would chain several of them).
-
-// Workgroups are handed to the 8 XCDs round-robin in launch order, and each XCD has its own L2.
-// Neighbouring tiles of one (b, kv head) slab share cache lines (a tile's row segment is shorter than a
-// line, its scale/zero rows are a quarter of one), so the (b, kv head) index is the FASTEST grid
-// dimension: with B*Hkv a multiple of 8, every tile of a slab runs on the same XCD, neighbours meet in
-// one L2, and the eight XCDs get equal work.  (Tile-fastest order fetched every line 2x on average.)
-
-// keep every load issued above this point ahead of the arithmetic below it (the scheduler would
-// otherwise sink loads next to their uses to save registers, serialising the memory latency)
-#define HQ_LOADS_ABOVE()                     \
-  do {                                       \
-    asm volatile("" ::: "memory");           \
-    __builtin_amdgcn_sched_barrier(0);       \
-  } while (0)
-
-__device__ __forceinline__ half2_t as_h2(uint32_t u) {
-  half2_t h;
-  __builtin_memcpy(&h, &u, 4);
-  return h;
-}
-__device__ __forceinline__ uint32_t as_u32(half2_t h) {
-  uint32_t u;
-  __builtin_memcpy(&u, &h, 4);
-  return u;
-}
-__device__ __forceinline__ half2_t pack_h2(half_t a, half_t b) {
-  half2_t h;
-  h[0] = a;
-  h[1] = b;
-  return h;
-}
-
-// [lo.byte_k, 0, hi.byte_k, 0]: byte k of two packed words side by side in the 16-bit halves
-template <int K>
-__device__ __forceinline__ uint32_t byte_pair(uint32_t lo, uint32_t hi) {
-  return __builtin_amdgcn_perm(hi, lo, 0x0c040c00u + (uint32_t)K * 0x00010001u);
-}
-// (lo.half_H, hi.half_H) of two registers holding fp16 pairs
-template <int H>
-__device__ __forceinline__ half2_t half_pair(uint32_t lo, uint32_t hi) {
-  return as_h2(__builtin_amdgcn_perm(hi, lo, H == 0 ? 0x05040100u : 0x07060302u));
-}
-
-// Field I (of 8/BITS) of the byte pair `u` as two exact fp16 integers.
-template <int BITS, int I>
-__device__ __forceinline__ half2_t field_pair(uint32_t u) {
-  constexpr int POS = I * BITS;                         // bit position inside the byte
-  constexpr uint32_t FMASK = ((1u << BITS) - 1u) << POS;
-  constexpr uint32_t MASK = FMASK | (FMASK << 16);
-  constexpr uint32_t EXPO = (uint32_t)(10 - POS + 15) << 10;  // fp16 bits of 2^(10-POS)
-  constexpr uint32_t MAGIC = EXPO | (EXPO << 16);
-  // (u & MASK) | MAGIC in one VALU op; the mask rides in a scalar register, the magic in a vector one
-  uint32_t r;
-  const uint32_t magic_v = MAGIC;
-  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(u), "s"(MASK), "v"(magic_v));
-  const half2_t biased = as_h2(r);                      // 2^(10-POS) + c, exact
-  const half2_t bias = as_h2(MAGIC);
-  return biased - bias;                                 // c, exact
-}
-
-// The same field still carrying its bias: 2^(10-POS) + c.
-template <int BITS, int I>
-__device__ __forceinline__ half2_t field_pair_biased(uint32_t u) {
-  constexpr int POS = I * BITS;
-  constexpr uint32_t FMASK = ((1u << BITS) - 1u) << POS;
-  constexpr uint32_t MASK = FMASK | (FMASK << 16);
-  constexpr uint32_t EXPO = (uint32_t)(10 - POS + 15) << 10;
-  constexpr uint32_t MAGIC = EXPO | (EXPO << 16);
-  uint32_t r;
-  const uint32_t magic_v = MAGIC;
-  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(u), "s"(MASK), "v"(magic_v));
-  return as_h2(r);
-}
-// -2^(10-POS) * s for field I: with it rnd16(c * s) is ONE fused multiply-add on the biased field,
-// (2^(10-POS) + c) * s - 2^(10-POS) * s = c * s before the single rounding -- exactly the product the reference
-// rounds -- provided 2^(10-POS) * s is itself an fp16 number, i.e. |s| < 64 at POS = 0 (scaling by a power of two
-// is exact short of overflow).  Callers take this route only after checking the scales of the whole tile.
-template <int BITS, int I>
-__device__ __forceinline__ half2_t bias_times_scale(half2_t s2) {
-  constexpr _Float16 NB = (_Float16)(-(float)(1 << (10 - I * BITS)));
-  return s2 * (half2_t){NB, NB};
-}
-
-// the reference dequantiser's two roundings (quant/pack_unpack.py:331-332) on a pair of codes
-__device__ __forceinline__ half2_t dequant_pair(half2_t c, half2_t s2, half2_t z2) {
-  const half2_t m = c * s2;
-  return m + z2;
-}
-
-// 1-bit normal-quantile coding (quant/pack_unpack.py:371-375): x = rnd16(rnd16(centre[c] * std) + mean)
-// with centre = -+k, k = fp16(0.6745).  rnd16(-+k * std) = -+a with a = rnd16(k * std), so with a2 formed
-// once per group the value is the single rounding of (2c - 1) * a + mean: two packed fused ops.
-#define HQ_NORMAL1_CENTER ((_Float16)0.67431640625f)  // fp16(norm.ppf(0.75))
-__device__ __forceinline__ half2_t normal1_spread(half2_t std2) {
-  return std2 * (half2_t){HQ_NORMAL1_CENTER, HQ_NORMAL1_CENTER};
-}
-__device__ __forceinline__ half2_t dequant_pair_normal1(half2_t c, half2_t a2, half2_t mean2) {
-  const half2_t t = __builtin_elementwise_fma(c, (half2_t){(_Float16)2, (_Float16)2}, (half2_t){(_Float16)-1, (_Float16)-1});
-  return __builtin_elementwise_fma(t, a2, mean2);
-}
-
-// Consume one byte pair: 8/BITS dequantised pairs, each dotted with NREP operand pairs.
-// NORMAL (1 bit only): s2 is the spread a2 = rnd16(k * std), z2 the mean.
-template <int BITS, int NREP, int PF, bool NORMAL = false, int NFIELD = 8 / BITS>
-__device__ __forceinline__ void consume_byte(uint32_t u, half2_t s2, half2_t z2, const half2_t (&a2)[NREP],
-                                             float (&acc)[NREP][PF], int tok0) {
-  constexpr int FPB = NFIELD;   // fields taken, from the low end of the byte
-#define HQ_FIELD(I_)                                                                     \
-  if constexpr (I_ < FPB) {                                                                      \
-    const half2_t c2_ = field_pair<BITS, (I_ < FPB ? I_ : 0)>(u);                        \
-    const half2_t x2 = NORMAL ? dequant_pair_normal1(c2_, s2, z2) : dequant_pair(c2_, s2, z2);  \
-    _Pragma("unroll") for (int h = 0; h < NREP; ++h)                                     \
-        acc[h][tok0 + I_] = __builtin_amdgcn_fdot2(x2, a2[h], acc[h][tok0 + I_], false); \
-  }
-  HQ_FIELD(0)
-  HQ_FIELD(1)
-  HQ_FIELD(2)
-  HQ_FIELD(3)
-  HQ_FIELD(4)
-  HQ_FIELD(5)
-  HQ_FIELD(6)
-  HQ_FIELD(7)
-#undef HQ_FIELD
-}
-
-// The same with the bias removal folded into the multiply (see bias_times_scale): nb[I] = -2^(10-POS_I) * s2.
-template <int BITS, int NREP, int PF, int NFIELD>
-__device__ __forceinline__ void consume_byte_fused_bias(uint32_t u, half2_t s2, half2_t z2, const half2_t (&nb)[8 / BITS],
-                                                        const half2_t (&a2)[NREP], float (&acc)[NREP][PF], int tok0) {
-#define HQ_FIELD(I_)                                                                      \
-  if constexpr (I_ < NFIELD) {                                                            \
-    const half2_t b2_ = field_pair_biased<BITS, (I_ < NFIELD ? I_ : 0)>(u);               \
-    const half2_t m2_ = __builtin_elementwise_fma(b2_, s2, nb[I_ < NFIELD ? I_ : 0]);     \
-    const half2_t x2 = m2_ + z2;                                                          \
-    _Pragma("unroll") for (int h = 0; h < NREP; ++h)                                      \
-        acc[h][tok0 + I_] = __builtin_amdgcn_fdot2(x2, a2[h], acc[h][tok0 + I_], false);  \
-  }
-  HQ_FIELD(0)
-  HQ_FIELD(1)
-  HQ_FIELD(2)
-  HQ_FIELD(3)
-  HQ_FIELD(4)
-  HQ_FIELD(5)
-  HQ_FIELD(6)
-  HQ_FIELD(7)
-#undef HQ_FIELD
-}
-
-template <int BITS, int NREP, int PF>
-__device__ __forceinline__ void consume_words(uint32_t w0, uint32_t w1, half2_t s2, half2_t z2,
-                                              const half2_t (&a2)[NREP], float (&acc)[NREP][PF]) {
-  constexpr int FPB = 8 / BITS;
-  consume_byte<BITS, NREP, PF>(byte_pair<0>(w0, w1), s2, z2, a2, acc, 0 * FPB);
-  consume_byte<BITS, NREP, PF>(byte_pair<1>(w0, w1), s2, z2, a2, acc, 1 * FPB);
-  consume_byte<BITS, NREP, PF>(byte_pair<2>(w0, w1), s2, z2, a2, acc, 2 * FPB);
-  consume_byte<BITS, NREP, PF>(byte_pair<3>(w0, w1), s2, z2, a2, acc, 3 * FPB);
-}
-
-// ------------------------------------------------------------------------------- matrix-core form of the dot products
-// With four query heads per KV head the inner product is a 4 x 4 x 4 matrix product per lane group: heads x
-// (four elements of the reduction axis) x (the four lanes' tokens or channels).  v_mfma_f32_4x4x4_16b_f16 runs sixteen
-// such blocks per wave, a block per four consecutive lanes: lane l supplies row l % 4 of its block's A (four fp16) and
-// column l % 4 of its block's B, and receives column l % 4 of D (four fp32).  A holds the query (or the probabilities)
-// of head l % 4, B the lane's own dequantised values -- bit for bit the ones the vector-ALU form feeds to its
-// dot products -- so D is (4 heads) x (this lane's token or channel): one instruction on the matrix pipe in place of
-// eight two-element dot products on the vector ALU.  Products are exact in fp32, accumulation is fp32; only the order
-// of the additions differs from the vector-ALU form.
-typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
-typedef float f4_t __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ f4_t mfma_4x4x4(half2_t a01, half2_t a23, half2_t b01, half2_t b23, f4_t c) {
-  const half4_t a = __builtin_shufflevector(a01, a23, 0, 1, 2, 3);
-  const half4_t b = __builtin_shufflevector(b01, b23, 0, 1, 2, 3);
-  return __builtin_amdgcn_mfma_f32_4x4x4f16(a, b, c, 0, 0, 0);
-}
-
-template <typename F, int... Is>
-__device__ __forceinline__ void static_for_impl(F &&f, std::integer_sequence<int, Is...>) {
-  (f(std::integral_constant<int, Is>{}), ...);
-}
-// f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>)
-template <int N, typename F>
-__device__ __forceinline__ void static_for(F &&f) {
-  static_for_impl(f, std::make_integer_sequence<int, N>{});
-}
-
-// field I of a byte pair, dequantised with the reference's two roundings
-template <int BITS, int I, bool NORMAL>
-__device__ __forceinline__ half2_t dequant_field(uint32_t u, half2_t s2, half2_t z2) {
-  const half2_t c2 = field_pair<BITS, I>(u);
-  return NORMAL ? dequant_pair_normal1(c2, s2, z2) : dequant_pair(c2, s2, z2);
-}
-// the same with the bias removal folded into the multiply: nb = bias_times_scale<BITS, I>(s2)
-template <int BITS, int I>
-__device__ __forceinline__ half2_t dequant_field_fused_bias(uint32_t u, half2_t s2, half2_t z2, half2_t nb) {
-  const half2_t m2 = __builtin_elementwise_fma(field_pair_biased<BITS, I>(u), s2, nb);
-  return m2 + z2;
-}
-
-// Matrix-core form of consume_byte: byte pair `ua` belongs to elements 0, 1 of the reduction axis (a row pair of K, a
-// token pair of V), `ub` to elements 2, 3; (a01, a23) is the A operand for those four elements.
-template <int BITS, bool NORMAL, int NFIELD, int N>
-__device__ __forceinline__ void consume_bytes_mfma(uint32_t ua, uint32_t ub, half2_t sa, half2_t za, half2_t sb, half2_t zb,
-                                                   half2_t a01, half2_t a23, f4_t (&acc)[N], int tok0) {
-  static_for<NFIELD>([&](auto I_) {
-    constexpr int I = decltype(I_)::value;
-    const half2_t xa = dequant_field<BITS, I, NORMAL>(ua, sa, za);
-    const half2_t xb = dequant_field<BITS, I, NORMAL>(ub, sb, zb);
-    acc[tok0 + I] = mfma_4x4x4(a01, a23, xa, xb, acc[tok0 + I]);
-  });
-}
-template <int BITS, int NFIELD, int N>
-__device__ __forceinline__ void consume_bytes_mfma_fused_bias(uint32_t ua, uint32_t ub, half2_t sa, half2_t za, half2_t sb,
-                                                              half2_t zb, const half2_t (&nba)[8 / BITS],
-                                                              const half2_t (&nbb)[8 / BITS], half2_t a01, half2_t a23,
-                                                              f4_t (&acc)[N], int tok0) {
-  static_for<NFIELD>([&](auto I_) {
-    constexpr int I = decltype(I_)::value;
-    const half2_t xa = dequant_field_fused_bias<BITS, I>(ua, sa, za, nba[I]);
-    const half2_t xb = dequant_field_fused_bias<BITS, I>(ub, sb, zb, nbb[I]);
-    acc[tok0 + I] = mfma_4x4x4(a01, a23, xa, xb, acc[tok0 + I]);
-  });
-}
-__device__ __forceinline__ uint32_t byte_pair_at(uint32_t lo, uint32_t hi, int k) {  // byte_pair<k>, k known after unrolling
-  return k == 0 ? byte_pair<0>(lo, hi) : k == 1 ? byte_pair<1>(lo, hi) : k == 2 ? byte_pair<2>(lo, hi) : byte_pair<3>(lo, hi);
-}
 
 // =============================================================================== q.K^T
 // A tile is worked on by W = 8 waves (small launches: shortest critical path per tile) or W = 4 waves
@@ -2213,10 +1891,11 @@ __global__ __launch_bounds__(CB_CH * CB_SLICES) void pv_combine_kernel(const flo
 
 // =============================================================================== host side
 
+// With a plan: the launches of decode_tiles.hip.  Else
 // `unit_tokens`: tokens per work unit -- the q.K^T tile of the chosen tiling (the token-major fp16 residual
 // always has 64-token tiles) or the p.V chunk.
 static int build_table(const hqekv_seg *segs, int nseg, bool is_k, int64_t D, int64_t unit_tokens,
-                       int64_t Tall, SegTable *tb, const char *who) {
+                       int64_t Tall, SegTable *tb, const char *who, const TilesPlan *plan = nullptr) {
   if (nseg < 0 || nseg > HQEKV_MAX_SEGS) return fail(HQEKV_E_ARG, "%s: nseg=%d out of range", who, nseg);
   if (nseg > 0 && !segs) return fail(HQEKV_E_ARG, "%s: null segment table", who);
   int64_t units = 0, max_units = 0;
@@ -2245,7 +1924,7 @@ static int build_table(const hqekv_seg *segs, int nseg, bool is_k, int64_t D, in
     if (s.n_tokens * D >= (1LL << 31))
       return fail(HQEKV_E_UNSUPPORTED, "%s: segment %d: n_tokens * D must stay below 2^31 per (b, head) slab", who, k);
     // (every V class is token-major; on the K side only the fp16 residual is)
-    const bool token_major = is_k ? (s.bits == 16 && s.layout == HQEKV_LAYOUT_TOKEN_MAJOR) : true;
+    const bool token_major = is_k ? (s.bits == 16 && (s.layout & 3) == HQEKV_LAYOUT_TOKEN_MAJOR) : true;
     if (s.slab_tokens != 0 && (s.slab_tokens < s.n_tokens || !token_major))
       return fail(HQEKV_E_ARG, "%s: segment %d: slab_tokens applies to token-major segments and must be >= n_tokens", who, k);
     SegDev &d = tb->seg[m++];
@@ -2256,12 +1935,13 @@ static int build_table(const hqekv_seg *segs, int nseg, bool is_k, int64_t D, in
     d.pos_base = s.pos_base;
     d.n_tokens = s.n_tokens;
     d.bits = s.bits;
-    d.layout = (is_k && s.bits == 16 && s.layout == HQEKV_LAYOUT_TOKEN_MAJOR) ? HQEKV_LAYOUT_TOKEN_MAJOR
-               : (s.bits == 1 && s.layout == HQEKV_LAYOUT_NORMAL1)              ? HQEKV_LAYOUT_NORMAL1
+    d.layout = (is_k && s.bits == 16 && (s.layout & 3) == HQEKV_LAYOUT_TOKEN_MAJOR) ? HQEKV_LAYOUT_TOKEN_MAJOR
+               : (s.bits == 1 && (s.layout & 3) == HQEKV_LAYOUT_NORMAL1)              ? HQEKV_LAYOUT_NORMAL1
                                                                                 : 0;
+    if ((s.layout & HQEKV_LAYOUT_RUNS) && s.idx && s.n_tokens % 32 == 0 && plan) d.layout |= HQEKV_LAYOUT_RUNS;
     d.slab_tokens = s.slab_tokens > 0 ? s.slab_tokens : s.n_tokens;
     d.unit_begin = (int32_t)units;
-    const int64_t per = (is_k && d.layout == HQEKV_LAYOUT_TOKEN_MAJOR) ? 64 : unit_tokens;
+    const int64_t per = plan ? tiles_unit_tokens(*plan, s) : token_major && is_k ? 64 : unit_tokens;
     const int64_t nu = (s.n_tokens + per - 1) / per;
     d.n_units = (int32_t)nu;
     if (nu > max_units) max_units = nu;
@@ -2272,8 +1952,8 @@ static int build_table(const hqekv_seg *segs, int nseg, bool is_k, int64_t D, in
   tb->nseg = m;
   tb->total_units = (int32_t)units;
   tb->max_units = (int32_t)max_units;
+  tb->per_unit = plan ? plan->per_unit : 0;
   for (int k = 0; k < HQEKV_MAX_SEGS; ++k) tb->begin[k] = k < m ? tb->seg[k].unit_begin : 0x7fffffff;
-  tb->pad_ = 0;
   (void)D;
   return HQEKV_OK;
 }
@@ -2300,7 +1980,7 @@ static int64_t qk_tile_of(int tiling) { return tiling == 4 ? qw_tile(4) : QK_TIL
 static bool qk_wave_tiling_fits(const hqekv_seg *segs, int nseg, int64_t D) {
   if (D != 128) return false;
   for (int k = 0; k < nseg; ++k)
-    if (segs[k].n_tokens > 0 && segs[k].bits == 16 && segs[k].layout != HQEKV_LAYOUT_TOKEN_MAJOR && segs[k].n_tokens % 8 != 0)
+    if (segs[k].n_tokens > 0 && segs[k].bits == 16 && (segs[k].layout & 3) != HQEKV_LAYOUT_TOKEN_MAJOR && segs[k].n_tokens % 8 != 0)
       return false;
   return true;
 }
@@ -2358,6 +2038,7 @@ static int launch_qk_heads(const SegTable &tb, const void *q, void *scores, int6
 static int launch_qk(const SegTable &tb, const void *q, void *scores, int64_t B, int64_t Hq, int64_t Hkv,
                      int64_t D, int64_t Tall, const FuseArgs &fz, hipStream_t st, int tiling, bool mf) {
   if (tb.total_units == 0) return HQEKV_OK;
+  if (tb.per_unit) return launch_qk_tiles(tb, q, scores, B, Hq, Hkv, Tall, fz, st);
   const int64_t nrep = Hq / Hkv;
   if (one_slice(nrep)) return launch_qk_heads(tb, q, scores, B, Hq, Hkv, D, Tall, fz, st, tiling, mf, (int)nrep, (int)(nrep << 16));
   const HeadSlices hs = head_slices(nrep);
@@ -2451,7 +2132,10 @@ static int launch_pv(const SegTable &tb, int64_t chunk, void *p, void *out, floa
                      int64_t Hq, int64_t Hkv, int64_t D, int64_t Tall, const FuseArgs &fz, hipStream_t st,
                      bool mf, int stages = 3, const StepEpilogue *ep = nullptr) {
   const int64_t n_bhq = B * Hq;
-  if (tb.total_units > 0 && (stages & 1)) {
+  if (tb.total_units > 0 && (stages & 1) && tb.per_unit) {
+    const int rc = launch_pv_tiles(tb, p, partial, B, Hq, Hkv, Tall, fz, st);
+    if (rc) return rc;
+  } else if (tb.total_units > 0 && (stages & 1)) {
     dim3 grid((unsigned)(B * Hkv), (unsigned)tb.total_units), block(PV_THREADS);
     const bool whole = one_slice(Hq / Hkv);
     HeadSlices hs = head_slices(Hq / Hkv);
@@ -2508,10 +2192,16 @@ extern "C" int hqekv_qk_hybrid(const hqekv_seg *segs, int nseg, const void *q, v
   if (rc) return rc;
   if (D > 1024) return fail(HQEKV_E_UNSUPPORTED, "qk_hybrid: D=%lld > 1024", (long long)D);
   if (!q || !scores || Tall <= 0) return fail(HQEKV_E_ARG, "qk_hybrid: null pointer or Tall <= 0");
+  SegTable tb{};
+  if (D == 128 && nseg >= 0 && nseg <= HQEKV_MAX_SEGS && segs && tiles_fit(segs, nseg, true, D, B, Hq, Hkv)) {
+    const TilesPlan plan = tiles_plan(segs, nseg, true, B * Hkv);
+    rc = build_table(segs, nseg, true, D, 0, Tall, &tb, "qk_hybrid", &plan);
+    if (rc) return rc;
+    return tb.total_units ? launch_qk_tiles(tb, q, scores, B, Hq, Hkv, Tall, FuseArgs{}, (hipStream_t)stream) : HQEKV_OK;
+  }
   int tiling = 0;
   rc = resolve_qk_tiling(0, segs, nseg, B * Hkv, D, "qk_hybrid", &tiling);
   if (rc) return rc;
-  SegTable tb{};
   rc = build_table(segs, nseg, true, D, qk_tile_of(tiling), Tall, &tb, "qk_hybrid");
   if (rc) return rc;
   return launch_qk(tb, q, scores, B, Hq, Hkv, D, Tall, FuseArgs{}, (hipStream_t)stream, tiling,
@@ -2539,14 +2229,27 @@ extern "C" int hqekv_scale_softmax(void *scores, const void *mask, int64_t mask_
   return check_launch("scale_softmax_kernel");
 }
 
+static bool pv_takes_tiles(const hqekv_seg *segs, int nseg, int64_t B, int64_t Hq, int64_t Hkv, int64_t D) {
+  return segs && tiles_fit(segs, nseg, false, D, B, Hq, Hkv);
+}
+// partial rows per (b, kv head) of a p.V launch
+static int64_t pv_units(const hqekv_seg *segs, int nseg, int64_t B, int64_t Hq, int64_t Hkv, int64_t D, bool tiles) {
+  int64_t units = 0;
+  if (tiles) {
+    units = tiles_plan(segs, nseg, false, B * Hkv).units;
+  } else {
+    const int64_t chunk = pv_chunk_tokens(seg_total_tokens(segs, nseg), B * Hkv);
+    for (int k = 0; k < nseg; ++k)
+      if (segs[k].n_tokens > 0) units += (segs[k].n_tokens + chunk - 1) / chunk;
+  }
+  (void)D;
+  return units > 0 ? units : 1;
+}
+
 extern "C" int64_t hqekv_pv_workspace_bytes(const hqekv_seg *segs, int nseg, int64_t B, int64_t Hq,
                                             int64_t Hkv, int64_t D) {
   if (nseg < 0 || nseg > HQEKV_MAX_SEGS || (nseg > 0 && !segs) || B <= 0 || Hq <= 0 || Hkv <= 0) return -1;
-  const int64_t chunk = pv_chunk_tokens(seg_total_tokens(segs, nseg), B * Hkv);
-  int64_t chunks = 0;
-  for (int k = 0; k < nseg; ++k)
-    if (segs[k].n_tokens > 0) chunks += (segs[k].n_tokens + chunk - 1) / chunk;
-  if (chunks == 0) chunks = 1;
+  const int64_t chunks = pv_units(segs, nseg, B, Hq, Hkv, D, pv_takes_tiles(segs, nseg, B, Hq, Hkv, D));
   return chunks * B * Hq * D * (int64_t)sizeof(float);
 }
 
@@ -2557,9 +2260,13 @@ extern "C" int hqekv_pv_hybrid(const hqekv_seg *segs, int nseg, const void *p, v
   if (rc) return rc;
   if (D != 128) return fail(HQEKV_E_UNSUPPORTED, "pv_hybrid: head_dim %lld (supported: 128)", (long long)D);
   if (!p || !out || Tall <= 0) return fail(HQEKV_E_ARG, "pv_hybrid: null pointer or Tall <= 0");
+  if (nseg < 0 || nseg > HQEKV_MAX_SEGS || (nseg > 0 && !segs)) return fail(HQEKV_E_ARG, "pv_hybrid: bad segment table");
+  const bool tiles = pv_takes_tiles(segs, nseg, B, Hq, Hkv, D);
   const int64_t chunk = pv_chunk_tokens(seg_total_tokens(segs, nseg), B * Hkv);
+  TilesPlan plan{};
+  if (tiles) plan = tiles_plan(segs, nseg, false, B * Hkv);
   SegTable tb{};
-  rc = build_table(segs, nseg, false, D, chunk, Tall, &tb, "pv_hybrid");
+  rc = build_table(segs, nseg, false, D, chunk, Tall, &tb, "pv_hybrid", tiles ? &plan : nullptr);
   if (rc) return rc;
   const int64_t need = (int64_t)(tb.total_units > 0 ? tb.total_units : 1) * B * Hq * D * (int64_t)sizeof(float);
   if (!workspace || workspace_bytes < need)
@@ -2567,7 +2274,7 @@ extern "C" int hqekv_pv_hybrid(const hqekv_seg *segs, int nseg, const void *p, v
                 (long long)need);
   if ((uintptr_t)workspace & 15) return fail(HQEKV_E_ALIGN, "pv_hybrid: workspace not 16-byte aligned");
   return launch_pv(tb, chunk, const_cast<void *>(p), out, (float *)workspace, B, Hq, Hkv, D, Tall, FuseArgs{},
-                   (hipStream_t)stream, dot_on_matrix_cores(0, Hq / Hkv));
+                   (hipStream_t)stream, dot_on_matrix_cores(0, Hq / Hkv), 3, nullptr);
 }
 
 static int64_t align_up(int64_t v, int64_t a) { return (v + a - 1) / a * a; }
@@ -2583,17 +2290,22 @@ static int decode_layout(const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_se
       (n_v > 0 && !v_segs) || B <= 0 || Hq <= 0 || Hkv <= 0 || D <= 0)
     return HQEKV_E_ARG;
   L->chunk = pv_chunk_tokens(seg_total_tokens(v_segs, n_v), B * Hkv);
-  int64_t chunks = 0;
-  for (int k = 0; k < n_v; ++k)
-    if (v_segs[k].n_tokens > 0) chunks += (v_segs[k].n_tokens + L->chunk - 1) / L->chunk;
-  if (chunks == 0) chunks = 1;
+  int64_t chunks = pv_units(v_segs, n_v, B, Hq, Hkv, D, false);
+  if (n_v > 0 && pv_takes_tiles(v_segs, n_v, B, Hq, Hkv, D)) {   // (a call may force either form)
+    const int64_t units = pv_units(v_segs, n_v, B, Hq, Hkv, D, true);
+    if (units > chunks) chunks = units;
+  }
   int64_t tiles = 0;
   for (int k = 0; k < n_k; ++k)
     if (k_segs[k].n_tokens > 0) {
       // room for the statistics of the smallest tile any tiling uses (the token-major residual: 64 tokens)
-      const int64_t per = (k_segs[k].bits == 16 && k_segs[k].layout == HQEKV_LAYOUT_TOKEN_MAJOR) ? 64 : qw_tile(4);   // 256
+      const int64_t per = (k_segs[k].bits == 16 && (k_segs[k].layout & 3) == HQEKV_LAYOUT_TOKEN_MAJOR) ? 64 : qw_tile(4);   // 256
       tiles += (k_segs[k].n_tokens + per - 1) / per;
     }
+  if (n_k > 0 && tiles_fit(k_segs, n_k, true, D, B, Hq, Hkv)) {
+    const int64_t pairs = tiles_plan(k_segs, n_k, true, B * Hkv).units;
+    if (pairs > tiles) tiles = pairs;
+  }
   if (tiles == 0) tiles = 1;
   L->n_stat = tiles;
   L->partial_bytes = align_up(chunks * B * Hq * D * (int64_t)sizeof(float), 256);
@@ -2705,10 +2417,18 @@ static int decode_impl(const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_segs
   int tiling = 0;
   rc = resolve_qk_tiling(qk_tiling_of(flags), k_segs, n_k, B * Hkv, D, "decode_attn", &tiling);
   if (rc) return rc;
+  // The launches of decode_tiles.hip take the call unless it names a form of the older ones.
+  const bool by_rule = !(flags & (HQEKV_QK_TILING(0xf) | HQEKV_DOT_MFMA | HQEKV_DOT_VALU | HQEKV_TWO_STEP_DEQUANT | HQEKV_FOLD_COMBINE |
+                                 HQEKV_SEPARATE_COMBINE));
+  const bool k_tiles = by_rule && n_k > 0 && tiles_fit(k_segs, n_k, true, D, B, Hq, Hkv);
+  const bool v_tiles = by_rule && n_v > 0 && tiles_fit(v_segs, n_v, false, D, B, Hq, Hkv);
+  TilesPlan k_plan{}, v_plan{};
+  if (k_tiles) k_plan = tiles_plan(k_segs, n_k, true, B * Hkv);
+  if (v_tiles) v_plan = tiles_plan(v_segs, n_v, false, B * Hkv);
   SegTable kt{}, vt{};
-  rc = build_table(k_segs, n_k, true, D, qk_tile_of(tiling), Tall, &kt, "decode_attn(K)");
+  rc = build_table(k_segs, n_k, true, D, qk_tile_of(tiling), Tall, &kt, "decode_attn(K)", k_tiles ? &k_plan : nullptr);
   if (rc) return rc;
-  rc = build_table(v_segs, n_v, false, D, L.chunk, Tall, &vt, "decode_attn(V)");
+  rc = build_table(v_segs, n_v, false, D, L.chunk, Tall, &vt, "decode_attn(V)", v_tiles ? &v_plan : nullptr);
   if (rc) return rc;
   hipStream_t st = (hipStream_t)stream;
   char *ws = (char *)workspace;
@@ -2730,7 +2450,7 @@ static int decode_impl(const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_segs
   const bool fold_pays = seg_total_tokens(v_segs, n_v) * B * Hkv >= CB_FOLD_MIN_TOKEN_ROWS;
   const bool fold_forced = (flags & HQEKV_FOLD_COMBINE) != 0;
   // (more than eight heads per KV head run as several p.V launches against the one counter: they keep the combine launch)
-  if (kt.total_units > 0 && vt.total_units > 0 && vt.total_units <= CB_FOLD_MAX && !(flags & HQEKV_SEPARATE_COMBINE) &&
+  if (kt.total_units > 0 && vt.total_units > 0 && !v_tiles && !k_tiles && vt.total_units <= CB_FOLD_MAX && !(flags & HQEKV_SEPARATE_COMBINE) &&
       (fold_pays || fold_forced) && one_slice(Hq / Hkv)) {
     fz.arrive = (uint32_t *)(ws + L.arrive_off);
     fz.out = (half_t *)attn_out;
@@ -2769,10 +2489,9 @@ static int decode_impl(const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_segs
 static bool gemv_is_pv_shape(int64_t K, int64_t N) { return N == 128 && (K > N || K % 32 != 0); }
 
 extern "C" int64_t hqekv_gemv_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t K, int64_t N, int bits) {
-  (void)bits;
   if (!gemv_is_pv_shape(K, N)) return 0;
   hqekv_seg s{};
-  s.bits = 2;
+  s.bits = bits;
   s.n_tokens = K;
   return hqekv_pv_workspace_bytes(&s, 1, B, Hq, Hkv, N);
 }

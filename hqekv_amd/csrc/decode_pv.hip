@@ -1,0 +1,354 @@
+// p.V of a decode step on matrix instructions (see decode_tiles.h).
+#include "decode_tiles.h"
+
+#pragma clang fp contract(off)
+
+namespace hq {
+
+// A workgroup takes `per_unit` consecutive blocks of one class: 256 tokens of codes (128 of the 8-bit and fp16
+// classes, whose rows are long), 64 (32) per wave.  Lane l owns channels 8 (l % 16) ... + 7 of eight consecutive tokens 8 (l / 16) ... of a step of
+// 32, so a step is eight products, one per channel.  Scale and zero rows of the block and its probabilities are staged in
+// LDS by the whole workgroup, which gathers the heads' logits at the block's positions, turns them into probabilities,
+// writes those back for the caller and parks them.  Several blocks: two buffers, so one barrier per block.
+constexpr int PT_WAVES = 4;
+
+template <int BITS>
+struct PtGeom {
+  static constexpr int STEPS = BITS >= 8 ? 1 : 2;             // per wave and block
+  static constexpr int BLOCK = PT_WAVES * 32 * STEPS;
+  static constexpr int ROWB = 128 * BITS / 8;                  // bytes per token row
+  static constexpr int WPL = BITS == 16 ? 4 : BITS == 8 ? 2 : 1;
+};
+constexpr int PT_BLOCK = 256;
+constexpr int PT_PSTRIDE = PT_BLOCK + 8;   // halves between two heads' probabilities
+
+template <int HP, bool LOOP>
+struct PtLds {
+  static constexpr int BUFS = LOOP ? 2 : 1;
+  uint2 sz[BUFS][PT_BLOCK / 2][4];         // token pair x channel group: (s, s'), (z, z')
+  half_t p[BUFS][HP][PT_PSTRIDE];
+};
+
+// What a thread holds of a block's logits on their way to LDS.  Positions in runs of 32 and an even token count: a pair
+// of neighbouring tokens for every other head (thread t: pair t % 128, heads t / 128, t / 128 + 2, ...), one 4-byte access
+// each.  Else: token t for every head.
+template <int HP>
+struct PtValues {
+  uint32_t pos;
+  uint32_t x[HP];
+};
+
+template <int BITS, int HP, bool EXACT, bool NORMAL, bool LOOP, bool FUSED, bool PAIRED, typename StatsLoad, typename StatsMerge>
+__device__ __forceinline__ void pt_class_job(const SegDev &sg, int blk0, int blk1, int bh, int wave, int lane, half_t *rows, int64_t Tall,
+                                             int nrep_arg, PtLds<HP, LOOP> &lds, const float *ml, f4_t (&acc)[8], StatsLoad &&load_stats,
+                                             StatsMerge &&merge_stats) {
+  using G = PtGeom<BITS>;
+  constexpr bool QUANT = BITS != 16;
+  constexpr int STEPS = G::STEPS, BLOCK = G::BLOCK, ROWB = G::ROWB, WPL = G::WPL;
+  const int nrep = EXACT ? HP : nrep_arg;
+  const int n = lane & 15, r = lane >> 4, tid = threadIdx.x;
+  const uint32_t n_tok = (uint32_t)sg.n_tokens;
+  const char *codes = (const char *)sg.data + (int64_t)bh * sg.slab_tokens * ROWB;
+  const half_t *sc = QUANT ? sg.scale + (int64_t)bh * sg.slab_tokens * 4 : nullptr;
+  const half_t *zr = QUANT ? sg.zero + (int64_t)bh * sg.slab_tokens * 4 : nullptr;
+  const Positions position(sg);
+
+  uint32_t cur[STEPS][8][WPL];
+  auto load_codes = [&](int blk, uint32_t (&w)[STEPS][8][WPL]) {
+    const uint32_t ch = (uint32_t)n * BITS, last = (n_tok - 1) * ROWB + ch;   // tokens past the end repeat the last row, and count with probability zero
+    const uint32_t off0 = ((uint32_t)blk * BLOCK + (uint32_t)wave * 32u * STEPS + 8u * r) * ROWB + ch;
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const uint32_t off = min(off0 + (uint32_t)(32 * s + i) * ROWB, last);
+        if constexpr (BITS == 2) {
+          w[s][i][0] = gload<uint16_t>(codes, off);
+        } else if constexpr (BITS == 1) {
+          w[s][i][0] = gload<uint8_t>(codes, off);
+        } else {
+          load_words<WPL, Words4<WPL>>(codes, off, w[s][i]);
+        }
+      }
+  };
+  PtValues<HP> f;
+  // thread t in the paired form: pair pt, heads ph, ph + 2, ...
+  constexpr int PAIRS = BLOCK / 2, HSTEP = PT_WAVES * 64 / PAIRS, PHEADS = HP / HSTEP > 0 ? HP / HSTEP : 1;
+  static_assert(HP % HSTEP == 0, "heads are dealt evenly");
+  const int pt = tid % PAIRS, ph = tid / PAIRS;
+  auto fetch_position = [&](int blk) {
+    f.pos = position.fetch(min((uint32_t)blk * BLOCK + (PAIRED ? 2u * pt : (uint32_t)tid), n_tok - 1));
+  };
+  auto fetch_values = [&](int blk) {
+    const uint32_t t = min((uint32_t)blk * BLOCK + (PAIRED ? 2u * pt : (uint32_t)tid), n_tok - 1);
+    f.pos = 2u * position.of(t, f.pos);   // byte offset in a row
+    if constexpr (PAIRED) {
+      // (past the end: the class's last pair once more.  min() above gives its second token: one step back)
+      f.pos -= t == n_tok - 1 ? 2u : 0u;
+#pragma unroll
+      for (int k = 0; k < PHEADS; ++k) {
+        const int h = ph + k * HSTEP;
+        uint32_t one[1];
+        load_words<1, Words2<1>>(rows + (int64_t)(EXACT ? h : min(h, nrep - 1)) * Tall, f.pos, one);
+        f.x[k] = one[0];
+      }
+    } else {
+#pragma unroll
+      for (int h = 0; h < HP; ++h)
+        if (h < nrep) f.x[h] = gload<uint16_t>(rows + (int64_t)h * Tall, f.pos);
+    }
+  };
+  uint32_t sa[2], sb[2], za[2], zb[2];
+  auto fetch_scales = [&](int blk) {
+    if (QUANT && tid < BLOCK / 2) {
+      const uint32_t a = min((uint32_t)blk * BLOCK + 2u * tid, n_tok - 1), b = min(a + 1, n_tok - 1);
+      load_words<2, Words4<2>>(sc, a * 8u, sa);
+      load_words<2, Words4<2>>(sc, b * 8u, sb);
+      load_words<2, Words4<2>>(zr, a * 8u, za);
+      load_words<2, Words4<2>>(zr, b * 8u, zb);
+    }
+  };
+  // fused: the row holds scaled logits: p = rnd16(exp(x - M) / L), written back for the caller.  Every position belongs to
+  // exactly one token of exactly one V class, so nobody else touches it.
+  auto probability = [&](half_t x, int h) { return FUSED ? (half_t)(__expf((float)x - ml[2 * h]) * ml[2 * h + 1]) : x; };
+  auto commit = [&](int blk, int buf) {
+    if constexpr (PAIRED) {
+      const bool valid = (uint32_t)blk * BLOCK + 2u * pt < n_tok;
+#pragma unroll
+      for (int k = 0; k < PHEADS; ++k) {
+        const int h = ph + k * HSTEP;
+        if (EXACT || h < nrep) {
+          const half2_t x = as_h2(f.x[k]);
+          const uint32_t p = as_u32(pack_h2(probability(x[0], h), probability(x[1], h)));
+          if (FUSED && valid) {
+            Words2<1> w;
+            w.v[0] = p;
+            gstore(rows + (int64_t)h * Tall, f.pos, w);
+          }
+          *reinterpret_cast<uint32_t *>(&lds.p[buf][h][2 * pt]) = valid ? p : 0u;
+        }
+      }
+    } else if (tid < BLOCK) {
+      const bool valid = (uint32_t)blk * BLOCK + tid < n_tok;
+#pragma unroll
+      for (int h = 0; h < HP; ++h)
+        if (h < nrep) {
+          const half_t p = probability(__builtin_bit_cast(half_t, (uint16_t)f.x[h]), h);
+          if (FUSED && valid) gstore(rows + (int64_t)h * Tall, f.pos, p);
+          lds.p[buf][h][tid] = valid ? p : (half_t)0;
+        }
+    }
+    if (QUANT && tid < BLOCK / 2) {
+      uint32_t v[8];
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        v[2 * g] = (g & 1) ? as_u32(half_pair<1>(sa[g >> 1], sb[g >> 1])) : as_u32(half_pair<0>(sa[g >> 1], sb[g >> 1]));
+        v[2 * g + 1] = (g & 1) ? as_u32(half_pair<1>(za[g >> 1], zb[g >> 1])) : as_u32(half_pair<0>(za[g >> 1], zb[g >> 1]));
+      }
+      uint4 *dst = reinterpret_cast<uint4 *>(lds.sz[buf][tid]);
+      dst[0] = make_uint4(v[0], v[1], v[2], v[3]);
+      dst[1] = make_uint4(v[4], v[5], v[6], v[7]);
+    }
+  };
+
+  // The longest chain of dependent loads is position -> logit: it goes first, with the statistics beside it (code words
+  // asked for ahead of the logits would queue in front of them).
+  fetch_position(blk0);
+  load_stats();
+  fetch_values(blk0);
+  HQ_LOADS_ABOVE();
+  fetch_scales(blk0);
+  load_codes(blk0, cur);
+  HQ_LOADS_ABOVE();
+  merge_stats();
+  commit(blk0, 0);
+  if (LOOP && blk0 + 1 < blk1) fetch_position(blk0 + 1);
+  __syncthreads();
+#pragma unroll 1
+  for (int blk = blk0; blk < (LOOP ? blk1 : blk0 + 1); ++blk) {
+    const int buf = LOOP ? (blk - blk0) & 1 : 0;
+    const bool more = LOOP && blk + 1 < blk1;
+    uint32_t nxt[STEPS][8][WPL];
+    if (more) {
+      fetch_values(blk + 1);
+      load_codes(blk + 1, nxt);
+      fetch_scales(blk + 1);
+    }
+    HQ_LOADS_ABOVE();
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s) {
+      const int t = (wave * STEPS + s) * 32 + 8 * r;   // this lane's first token of the step, inside the block
+      const u32x4 a = *reinterpret_cast<const u32x4 *>(&lds.p[buf][min(n, nrep - 1)][t]);
+      half2_t s2[4], z2[4];
+      if constexpr (QUANT) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const uint2 e = lds.sz[buf][t / 2 + i][n >> 2];
+          s2[i] = as_h2(e.x);
+          z2[i] = as_h2(e.y);
+          if (NORMAL) s2[i] = normal1_spread(s2[i]);
+        }
+        constexpr int B = BITS == 16 ? 8 : BITS;   // (named for the discarded instantiation)
+        static_for<B>([&](auto K_) {   // byte K of a lane's channels
+          constexpr int K = decltype(K_)::value;
+          uint32_t u[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) u[i] = byte_pair<K % 4>(cur[s][2 * i][K / 4 % WPL], cur[s][2 * i + 1][K / 4 % WPL]);
+          static_for<8 / B>([&](auto F_) {
+            constexpr int F = decltype(F_)::value, C = K * (8 / B) + F;
+            u32x4 b;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) b[i] = as_u32(dequant_field<B, F, NORMAL>(u[i], s2[i], z2[i]));
+            acc[C] = mfma16(a, b, acc[C]);
+          });
+        });
+      } else {
+        static_for<8>([&](auto C_) {
+          constexpr int C = decltype(C_)::value;
+          u32x4 b;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) b[i] = as_u32(half_pair<C & 1>(cur[s][2 * i][C / 2 % WPL], cur[s][2 * i + 1][C / 2 % WPL]));
+          acc[C] = mfma16(a, b, acc[C]);
+        });
+      }
+    }
+    if (more) {
+      commit(blk + 1, buf ^ 1);
+      if (blk + 2 < blk1) fetch_position(blk + 2);
+#pragma unroll
+      for (int s = 0; s < STEPS; ++s)
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+#pragma unroll
+          for (int k = 0; k < WPL; ++k) cur[s][i][k] = nxt[s][i][k];
+      __syncthreads();
+    }
+  }
+}
+
+template <int HP, bool EXACT, bool LOOP, bool FUSED>
+__global__ __launch_bounds__(PT_WAVES * 64, HP <= 8 ? (LOOP ? 4 : 6) : 2) void pv_tiles_kernel(SegTable tb, half_t *__restrict__ p, float *__restrict__ partial,
+                                                                   TilesArgs ta, int64_t Tall, int64_t n_bhq, FuseArgs fz) {
+  __shared__ __align__(16) PtLds<HP, LOOP> lds;
+  __shared__ __align__(16) float red[PT_WAVES][HP][128];
+  __shared__ float ml[2 * HP];   // (max, 1 / sum exp) of each head's row
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int bh = blockIdx.x, u = blockIdx.y;
+  const SegDev sg = tb.seg[tiles_segment(tb, u)];
+  const int b = tiles_batch_row(ta, bh), hkv = bh - b * ta.Hkv;
+  const int Hq = ta.hq_slice & 0xffff, head0 = first_head(ta.hq_slice, hkv), nrep = EXACT ? HP : ta.nrep;
+  half_t *rows = p + ((int64_t)b * Hq + head0) * Tall;
+  f4_t acc[8];
+#pragma unroll
+  for (int c = 0; c < 8; ++c) acc[c] = (f4_t){0.f, 0.f, 0.f, 0.f};
+  // wave w merges the per-tile pairs of heads w, w + 4, ...; up to 256 tiles of the first are read once, ahead of the rest
+  // (past the last tile: the last one again, left out of the sum)
+  float2 sv[4];
+  auto read_stats = [&](const float2 *sp) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (k == 0 || fz.n_stat > 64 * k) {
+        uint32_t w[2];
+        load_words<2, Words4<2>>(sp, 8u * (uint32_t)min(lane + 64 * k, fz.n_stat - 1), w);
+        sv[k] = make_float2(__builtin_bit_cast(float, w[0]), __builtin_bit_cast(float, w[1]));
+      }
+  };
+  const float2 *srow = fz.stats + ((int64_t)b * Hq + head0 + min(wave, nrep - 1)) * fz.n_stat;
+  auto load_stats = [&]() {
+    if (FUSED) read_stats(srow);
+  };
+  auto merge_stats = [&]() {
+    if (!FUSED) return;
+    for (int h = wave; h < nrep; h += PT_WAVES) {
+      const float2 *sp = srow + (int64_t)(h - wave) * fz.n_stat;
+      if (h != wave) read_stats(sp);
+      float m = sv[0].x;
+#pragma unroll
+      for (int k = 1; k < 4; ++k)
+        if (fz.n_stat > 64 * k) m = fmaxf(m, sv[k].x);
+      for (int e = lane + 256; e < fz.n_stat; e += 64) m = fmaxf(m, sp[e].x);
+      m = wave_max(m);
+      float l = 0.f;
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (k == 0 || fz.n_stat > 64 * k) l += lane + 64 * k < fz.n_stat ? sv[k].y * __expf(sv[k].x - m) : 0.f;
+      for (int e = lane + 256; e < fz.n_stat; e += 64) {
+        const float2 w = sp[e];
+        l += w.y * __expf(w.x - m);
+      }
+      l = wave_sum(l);
+      if (lane == 0) {
+        ml[2 * h] = m;
+        ml[2 * h + 1] = 1.0f / l;
+      }
+    }
+    __syncthreads();
+  };
+  const int unit = u - sg.unit_begin, per = tb.per_unit, b0 = unit * per;
+  const bool paired = qt_runs(sg) && sg.n_tokens % 2 == 0;
+#define HQ_JOB_P(B_, NORMAL_, PAIRED_)                                                                                                   \
+  pt_class_job<B_, HP, EXACT, NORMAL_, LOOP, FUSED, PAIRED_>(sg, b0, min(b0 + per, (int)((sg.n_tokens + PtGeom<B_>::BLOCK - 1) / PtGeom<B_>::BLOCK)), \
+                                                             bh, wave, lane, rows, Tall, nrep, lds, ml, acc, load_stats, merge_stats)
+#define HQ_JOB(B_, NORMAL_)                  \
+  do {                                       \
+    if (paired) HQ_JOB_P(B_, NORMAL_, true); \
+    else HQ_JOB_P(B_, NORMAL_, false);       \
+  } while (0)
+  switch (sg.bits) {
+    case 1:
+      if ((sg.layout & 3) == HQEKV_LAYOUT_NORMAL1) HQ_JOB(1, true);
+      else HQ_JOB(1, false);
+      break;
+    case 2: HQ_JOB(2, false); break;
+    case 4: HQ_JOB(4, false); break;
+    case 8: HQ_JOB(8, false); break;
+    default: HQ_JOB(16, false);
+  }
+#undef HQ_JOB
+#undef HQ_JOB_P
+  // lane l holds heads 4 (l / 16) ... + 3 of channels 8 (l % 16) ... + 7
+  const int n = lane & 15, r = lane >> 4;
+  if (4 * r < HP) {
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {
+      float4 *dst = reinterpret_cast<float4 *>(&red[wave][4 * r + h][8 * n]);
+      dst[0] = make_float4(acc[0][h], acc[1][h], acc[2][h], acc[3][h]);
+      dst[1] = make_float4(acc[4][h], acc[5][h], acc[6][h], acc[7][h]);
+    }
+  }
+  __syncthreads();
+  float *dst = partial + ((int64_t)u * n_bhq + (int64_t)b * Hq + head0) * 128;
+#pragma unroll
+  for (int k = threadIdx.x; k < (EXACT ? HP : nrep) * 64; k += PT_WAVES * 64) {
+    const int h = k >> 6, c = 2 * (k & 63);
+    float2 v[PT_WAVES];
+#pragma unroll
+    for (int w = 0; w < PT_WAVES; ++w) v[w] = *reinterpret_cast<const float2 *>(&red[w][h][c]);
+    *reinterpret_cast<float2 *>(dst + h * 128 + c) = make_float2(((v[0].x + v[1].x) + v[2].x) + v[3].x, ((v[0].y + v[1].y) + v[2].y) + v[3].y);
+  }
+}
+
+// =============================================================================== host side
+int64_t pv_block_tokens(int bits) { return bits >= 8 ? PtGeom<8>::BLOCK : PT_BLOCK; }
+
+int launch_pv_tiles(const SegTable &tb, void *p, float *partial, int64_t B, int64_t Hq, int64_t Hkv, int64_t Tall, const FuseArgs &fz,
+                    hipStream_t st) {
+  const TilesArgs ta = tiles_args(B, Hq, Hkv);
+  const int nrep = ta.nrep;
+  const dim3 grid((unsigned)(B * Hkv), (unsigned)tb.total_units), block(PT_WAVES * 64);
+#define LAUNCH(HP_, EXACT_, LOOP_, FUSED_) \
+  hipLaunchKernelGGL((pv_tiles_kernel<HP_, EXACT_, LOOP_, FUSED_>), grid, block, 0, st, tb, (half_t *)p, partial, ta, Tall, B * Hq, fz)
+  const bool loop = tb.per_unit > 1;
+#define LAUNCH_H(HP_)                                                                 \
+  if (!fz.stats) LAUNCH(HP_, false, true, false);                                     \
+  else if (HP_ <= 8 && nrep == HP_ && loop) LAUNCH(HP_, (HP_ <= 8), true, true);     \
+  else if (HP_ <= 8 && nrep == HP_) LAUNCH(HP_, (HP_ <= 8), false, true);            \
+  else if (loop) LAUNCH(HP_, false, true, true);                                      \
+  else LAUNCH(HP_, false, false, true)
+  if (nrep <= 4) { LAUNCH_H(4); } else if (nrep <= 8) { LAUNCH_H(8); } else { LAUNCH_H(16); }
+#undef LAUNCH_H
+#undef LAUNCH
+  return check_launch("pv_tiles_kernel");
+}
+
+}  // namespace hq

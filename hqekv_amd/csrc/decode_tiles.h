@@ -1,0 +1,126 @@
+// Decode launches (decode_qk.hip: q.K^T, decode_pv.hip: p.V) on 16x16x32 matrix instructions, head_dim 128, up to 16 query
+// heads per KV head.
+//
+// One instruction multiplies 16 rows of heads with 16 columns.  Lane l of the wave supplies eight consecutive elements
+// of the reduction axis, 8 (l / 16) ..., of row l % 16 of A and of column l % 16 of B, and receives rows 4 (l / 16) ... + 3
+// of column l % 16 of D.  So a lane dequantises eight codes along the reduction axis -- eight channels of a K token, eight
+// tokens of a V channel -- straight into a B operand, packed in pairs exactly as the dequantiser works, and the sums over
+// head_dim or tokens stay on the matrix pipe up to the four-fold split over a workgroup's waves.
+//
+// With fewer than 16 heads the spare rows of A are put to use in q.K^T: A is laid out HP heads (4, 8 or 16) to a "band"
+// of rows, and the operand for token i of a packed word has only band i / (tokens per band) filled.  Products of different
+// bands then share one accumulator, every lane ends up with the scores of its own tokens, and four heads need a quarter
+// of the accumulators (and leave all 64 lanes busy in the softmax statistics instead of 16).
+#pragma once
+
+#include "attn_common.h"
+
+#pragma clang fp contract(off)
+
+namespace hq {
+
+typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ f4_t mfma16(u32x4 a, u32x4 b, f4_t c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, a), __builtin_bit_cast(half8_t, b), c, 0, 0, 0);
+}
+
+#if defined(__HIP_DEVICE_COMPILE__)
+#define HQ_GLOBAL __attribute__((address_space(1)))   // pointers out of the segment table carry no address space of their own
+#else
+#define HQ_GLOBAL
+#endif
+
+// loads of N words at the alignment of an element (the target reads unaligned)
+template <int N>
+struct __attribute__((packed, aligned(2))) Words2 { uint32_t v[N]; };
+template <int N>
+struct __attribute__((packed, aligned(4))) Words4 { uint32_t v[N]; };
+
+template <int N, typename W>
+__device__ __forceinline__ void load_words(const void *base, uint32_t off, uint32_t (&out)[N]) {
+  typedef const HQ_GLOBAL W *src_t;
+  const W w = *(src_t)(uintptr_t)((const char *)base + off);
+#pragma unroll
+  for (int i = 0; i < N; ++i) out[i] = w.v[i];
+}
+template <typename T>
+__device__ __forceinline__ T gload(const void *base, uint32_t off) {
+  return *(const HQ_GLOBAL T *)(uintptr_t)((const char *)base + off);
+}
+template <typename T>
+__device__ __forceinline__ void gstore(void *base, uint32_t off, T v) {
+  *(HQ_GLOBAL T *)(uintptr_t)((char *)base + off) = v;
+}
+
+// keep LDS traffic of one wave in program order (the hardware does; this holds the compiler to it)
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// =============================================================================== what both launches take apart
+// A workgroup's segment, its (b, kv head) taken apart, its first query head: scalar arithmetic only, since everything the
+// workgroup does waits for it (the compiler's own choice went through vector registers for the comparisons and through a
+// float reciprocal for the division).
+struct TilesArgs {
+  int32_t hq_slice, nrep;
+  int32_t Hkv;
+  uint32_t div_hkv;   // ceil(2^32 / Hkv): bh / Hkv is the high word of the product as long as bh Hkv < 2^32
+  int32_t n_bh;
+};
+__device__ __forceinline__ int tiles_segment(const SegTable &tb, int u) {
+  int s = -1;
+#pragma unroll
+  for (int k = 0; k < HQEKV_MAX_SEGS; ++k) s -= (tb.begin[k] - u - 1) >> 31;   // (an unused entry's begin is INT32_MAX)
+  return s;
+}
+__device__ __forceinline__ int tiles_batch_row(const TilesArgs &a, int bh) { return a.Hkv == 1 ? bh : (int)__umulhi((uint32_t)bh, a.div_hkv); }
+
+// Position of token t, below 2^31 (it indexes a row of Tall scores): the low word of its index is enough, read at the first
+// token of its run of 32 where positions come in runs (HQEKV_LAYOUT_RUNS).  In two parts without a branch between them, so
+// that the load is not waited for where it is issued: a segment without an index reads a word it ignores.
+struct Positions {
+  const void *src;      // the index, or anything readable
+  uint32_t keep, scale, run, base;
+  __device__ __forceinline__ explicit Positions(const SegDev &sg) {
+    const bool has = sg.idx != nullptr;
+    src = has ? (const void *)sg.idx : sg.data;
+    keep = __builtin_amdgcn_readfirstlane(has ? ~0u : 0u);   // (or the compiler makes two code paths of it)
+    scale = keep & 8u;
+    run = ((sg.layout & HQEKV_LAYOUT_RUNS) ? 31u : 0u) | ~keep;   // bits of t that are added to what was read
+    base = (uint32_t)sg.pos_base & ~keep;
+  }
+  __device__ __forceinline__ uint32_t fetch(uint32_t t) const { return gload<uint32_t>(src, scale * (t & ~run)); }
+  __device__ __forceinline__ uint32_t of(uint32_t t, uint32_t fetched) const { return (fetched & keep) + (t & run) + base; }
+  __device__ __forceinline__ uint32_t operator()(uint32_t t) const { return of(t, fetch(t)); }
+};
+__device__ __forceinline__ bool qt_runs(const SegDev &sg) { return (sg.layout & HQEKV_LAYOUT_RUNS) || !sg.idx; }
+
+// =============================================================================== host side
+constexpr int64_t PT_RESIDENT = 6 * 256, PT_RESIDENT_LOOP = 4 * 256;   // p.V workgroups the chip holds
+
+// How a launch is cut up.
+struct TilesPlan {
+  bool is_k;
+  int per_unit;       // p.V: blocks per workgroup
+  int64_t units;      // workgroups per (b, kv head); q.K^T leaves one softmax pair per query head in each
+};
+// head_dim 128, at most 16 query heads per KV head, channel-major fp16 K classes of whole 8-token columns
+bool tiles_fit(const hqekv_seg *segs, int nseg, bool is_k, int64_t D, int64_t B, int64_t Hq, int64_t Hkv);
+TilesPlan tiles_plan(const hqekv_seg *segs, int nseg, bool is_k, int64_t BHkv);
+int64_t tiles_unit_tokens(const TilesPlan &p, const hqekv_seg &s);
+
+inline TilesArgs tiles_args(int64_t B, int64_t Hq, int64_t Hkv) {
+  const int nrep = (int)(Hq / Hkv);
+  return TilesArgs{hq_with_slice((int)Hq, nrep, 0), nrep, (int32_t)Hkv, (uint32_t)(((1ULL << 32) + Hkv - 1) / Hkv), (int32_t)(B * Hkv)};
+}
+
+int64_t pv_block_tokens(int bits);   // tokens of a p.V block
+int launch_qk_tiles(const SegTable &tb, const void *q, void *scores, int64_t B, int64_t Hq, int64_t Hkv, int64_t Tall, const FuseArgs &fz,
+                    hipStream_t st);
+int launch_pv_tiles(const SegTable &tb, void *p, float *partial, int64_t B, int64_t Hq, int64_t Hkv, int64_t Tall, const FuseArgs &fz,
+                    hipStream_t st);
+
+}  // namespace hq

@@ -170,16 +170,16 @@ bool read_side(PyObject *pkv, bool is_k, bool low_uniform, int64_t B, const at::
 }
 
 // attention.idx_cover_once: the remembered verdict when it still holds for these very arrays, else the function itself
-// (which remembers).  -> 1, 0, or -1 with an exception set.
-int cover_once(PyObject *const *idx, int n_idx, int64_t n, PyObject *cover_fn) {
-  if (n_idx == 0) return n == 0;
+// (which remembers).  -> 3 (covered, in whole runs of 32 positions), 1 (covered), 0, or -1 with an exception set.
+int cover_once(PyObject *const *idx, int n_idx, int64_t n, PyObject *cover_fn, bool again = true) {
+  if (n_idx == 0) return n == 0 ? 1 : 0;
   PyObject *hit = PyObject_GetAttr(idx[0], s_cover);
   if (!hit) {
     if (!PyErr_ExceptionMatches(PyExc_AttributeError)) return -1;
     PyErr_Clear();
   } else {
     int verdict = -1;
-    if (PyTuple_Check(hit) && PyTuple_GET_SIZE(hit) == 3) {
+    if (PyTuple_Check(hit) && PyTuple_GET_SIZE(hit) == 4) {
       PyObject *key = PyTuple_GET_ITEM(hit, 0), *refs = PyTuple_GET_ITEM(hit, 2);
       bool ok = PyTuple_Check(key) && PyTuple_GET_SIZE(key) == n_idx + 1 && PyList_Check(refs) && PyList_GET_SIZE(refs) == n_idx &&
                 PyLong_AsLongLong(PyTuple_GET_ITEM(key, n_idx)) == n;
@@ -191,7 +191,7 @@ int cover_once(PyObject *const *idx, int n_idx, int64_t n, PyObject *cover_fn) {
              PyLong_AsLongLong(PyTuple_GET_ITEM(k, 1)) == t.numel() && PyLong_AsLongLong(PyTuple_GET_ITEM(k, 2)) == (long long)t._version() &&
              PyWeakref_Check(PyList_GET_ITEM(refs, i)) && PyWeakref_GET_OBJECT(PyList_GET_ITEM(refs, i)) == idx[i];
       }
-      if (ok) verdict = PyTuple_GET_ITEM(hit, 1) == Py_True;
+      if (ok) verdict = PyTuple_GET_ITEM(hit, 1) != Py_True ? 0 : PyTuple_GET_ITEM(hit, 3) == Py_True ? 3 : 1;
     }
     Py_DECREF(hit);
     if (PyErr_Occurred()) return -1;
@@ -207,7 +207,7 @@ int cover_once(PyObject *const *idx, int n_idx, int64_t n, PyObject *cover_fn) {
   if (!r) return -1;
   const int v = PyObject_IsTrue(r);
   Py_DECREF(r);
-  return v;
+  return v > 0 && again ? cover_once(idx, n_idx, n, cover_fn, false) : v;   // (once more for what it remembered)
 }
 
 int default_flags() {
@@ -232,10 +232,12 @@ PyObject *decode(PyObject *, PyObject *const *a, Py_ssize_t na) {
   if (!read_side(pkv, true, low_uniform, B, dev, k) || !read_side(pkv, false, low_uniform, B, dev, v)) Py_RETURN_NONE;
   const int64_t Tall = v.tokens;
   if (Tall == 0 || k.tokens != Tall || k.class_tokens != v.class_tokens || k.H != v.H || k.D != D || v.D != D) Py_RETURN_NONE;
-  for (const auto &side : {std::make_pair(k.idx, k.n_idx), std::make_pair(v.idx, v.n_idx)}) {
-    const int c = cover_once(side.first, side.second, v.class_tokens, a[3]);
+  for (Side *s : {&k, &v}) {
+    const int c = cover_once(s->idx, s->n_idx, v.class_tokens, a[3]);
     if (c < 0) return nullptr;
     if (!c) Py_RETURN_NONE;
+    for (int i = 0; c == 3 && i < s->n; ++i)
+      if (s->seg[i].idx) s->seg[i].layout |= HQEKV_LAYOUT_RUNS;
   }
   for (Side *s : {&k, &v})
     if (s->tokens > s->class_tokens) s->seg[s->n - 1].pos_base = s->class_tokens;

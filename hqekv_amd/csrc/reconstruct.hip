@@ -216,9 +216,11 @@ __global__ __launch_bounds__(256) void cover_once_kernel(CoverArgs a, int64_t n,
     src = in ? a.idx[k] : src;
     first = in ? a.begin[k] : first;
   }
-  const int64_t p = src[i - first];
+  const int64_t at = i - first, p = src[at];
   const uint32_t bit = 1u << (p & 31);
-  if (p < 0 || p >= n || (atomicOr(bits + (p >> 5), bit) & bit)) *status = 1u;
+  uint32_t bad = p < 0 || p >= n || (atomicOr(bits + (p >> 5), bit) & bit) ? 1u : 0u;
+  if (p != src[at & ~31LL] + (at & 31)) bad |= 2u;
+  if (bad) atomicOr(status, bad);
 }
 
 }  // namespace hq
@@ -264,7 +266,7 @@ extern "C" int hqekv_cache_reconstruct(const hqekv_seg *k_segs, int n_k, const h
       return fail(HQEKV_E_ARG, "cache_reconstruct: segment %d bits=%d", k, s.bits);
     if (!s.data || (s.bits != 16 && (!s.scale || !s.zero))) return fail(HQEKV_E_ARG, "cache_reconstruct: segment %d lacks data / scale / zero", k);
     if ((uintptr_t)s.data & (s.bits == 16 ? 15 : 3)) return fail(HQEKV_E_ALIGN, "cache_reconstruct: segment %d data misaligned", k);
-    const bool tm = !is_k || (s.bits == 16 && s.layout == HQEKV_LAYOUT_TOKEN_MAJOR);
+    const bool tm = !is_k || (s.bits == 16 && (s.layout & 3) == HQEKV_LAYOUT_TOKEN_MAJOR);
     if (!tm && s.bits != 16 && s.n_tokens % 32) return fail(HQEKV_E_ARG, "cache_reconstruct: segment %d n_tokens not a multiple of 32", k);
     if (s.slab_tokens != 0 && (s.slab_tokens < s.n_tokens || !tm))
       return fail(HQEKV_E_ARG, "cache_reconstruct: segment %d: slab_tokens applies to token-major segments and must be >= n_tokens", k);
@@ -278,7 +280,7 @@ extern "C" int hqekv_cache_reconstruct(const hqekv_seg *k_segs, int n_k, const h
     r.slab_tokens = s.slab_tokens > 0 ? s.slab_tokens : s.n_tokens;
     r.n_tokens = (int32_t)s.n_tokens;
     r.bits = (int16_t)s.bits;
-    r.kind = (int16_t)((tm ? 1 : 0) | (s.bits == 1 && s.layout == HQEKV_LAYOUT_NORMAL1 ? 2 : 0));
+    r.kind = (int16_t)((tm ? 1 : 0) | (s.bits == 1 && (s.layout & 3) == HQEKV_LAYOUT_NORMAL1 ? 2 : 0));
     tb.begin[m++] = (int32_t)tiles;
     tiles += (s.n_tokens + RC_TOK - 1) / RC_TOK;
     if (tiles > 65535) return fail(HQEKV_E_UNSUPPORTED, "cache_reconstruct: more than 65535 tiles of %d tokens", RC_TOK);

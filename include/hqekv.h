@@ -174,6 +174,10 @@ int hqekv_gemv_normal_group(const void *fA, const void *code, const void *stdv, 
                                    /* x = rnd16(rnd16(+-0.6745 * std) + mean), the 1-bit class of the   */
                                    /* 'high_uniform_group_low_normal_group' strategy                    */
                                    /* (quant/pack_unpack.py:356-376, quant/hqe_matmul.py:371-374)       */
+#define HQEKV_LAYOUT_RUNS 4        /* may be added to the value above: idx consists of whole runs of 32 consecutive     */
+                                   /* positions (idx[32 i + j] == idx[32 i] + j, n_tokens % 32 == 0), as the cache        */
+                                   /* policy's classes do; the decode launches then read one index per run.  Trusted:     */
+                                   /* hqekv_cover_once finds it out                                                       */
 typedef struct hqekv_seg {
   int32_t bits;          /* 16, 8, 4, 2 or 1                                           */
   int32_t layout;        /* HQEKV_LAYOUT_*: 0 = as listed at the top of this file       */
@@ -410,8 +414,9 @@ int hqekv_cache_reconstruct(const hqekv_seg *k_segs, int n_k, const hqekv_seg *v
                             int64_t BH, int64_t D, int64_t T, void *stream);
 
 /* Do the index arrays (device; at most HQEKV_MAX_SEGS), taken together, name every position in [0, sum of counts) exactly
- * once?  scratch: one int32 status and one bit per position, 4 * (1 + ceil(n / 32)) bytes the caller has zeroed; status is
- * non-zero afterwards when a position is out of range or named twice.
+ * once?  scratch: one int32 status and one bit per position, 4 * (1 + ceil(n / 32)) bytes the caller has zeroed; bit 0 of
+ * status is set afterwards when a position is out of range or named twice, bit 1 when some array does not consist of whole
+ * runs of 32 consecutive positions (HQEKV_LAYOUT_RUNS).
  */
 int hqekv_cover_once(const int64_t *const *idx, const int64_t *counts, int n_arrays, void *scratch, int64_t scratch_bytes,
                      void *stream);

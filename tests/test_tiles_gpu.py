@@ -1,0 +1,63 @@
+"""The matrix-core launches of a decode step (csrc/decode_qk.hip, decode_pv.hip) at the edges of their tiles, against the
+CPU oracle: classes of a few blocks up to one more than a tile, every count of query heads per KV head they pad (1 to 16),
+positions in runs and shuffled, residuals of odd and even length, and a launch of several blocks per workgroup."""
+import pytest
+import torch
+
+from hqekv_amd import synth
+from oracle import hqe_oracle as O
+
+pytestmark = pytest.mark.gpu
+RTOL, ATOL = 1e-3, 2e-3
+
+
+def _quant(low_normal):
+    def f(x, g, bits):
+        if bits == 1 and low_normal:
+            return O.normal_group_quantize_pack_last_dim(x, 32, 1)
+        return O.uniform_group_quantize_pack_last_dim(x, 32, bits)
+    return f
+
+
+@pytest.mark.parametrize("blocks", [(1, 1, 1, 1, 1), (4, 7, 8, 9, 8), (5, 9, 16, 17, 1), (0, 4, 0, 33, 7)],
+                         ids=lambda b: "-".join(map(str, b)))
+@pytest.mark.parametrize("n_rep,B,residual,low_normal,fused", [
+    (1, 2, 0, False, True), (3, 1, 1, False, True), (4, 1, 64, True, True), (4, 3, 65, False, False),
+    (5, 2, 16, False, True), (8, 1, 31, True, True), (12, 1, 2, False, True), (16, 1, 0, False, False)])
+@pytest.mark.parametrize("shuffled", [False, True], ids=["runs", "shuffled"])
+def test_tile_edges(dev, blocks, n_rep, B, residual, low_normal, fused, shuffled):
+    from hqekv_amd.attention import decode_attention
+    Hkv, D, n = 2, 128, 32 * sum(blocks)
+    q, K, V = synth.make_qkv(B, n_rep * Hkv, Hkv, n + residual, D, 77)
+    order = torch.randperm(n // 32, generator=torch.Generator().manual_seed(n))
+    classes, at = {}, 0
+    for bits, c in zip((16, 8, 4, 2, 1), blocks):
+        classes[bits] = (order[at:at + c].sort()[0][:, None] * 32 + torch.arange(32)).reshape(-1)
+        at += c
+    override = None
+    if shuffled:
+        perm, override, at = torch.randperm(n, generator=torch.Generator().manual_seed(n + 1)), {}, 0
+        for bits, tok in classes.items():
+            override[bits] = perm[at:at + tok.numel()]
+            at += tok.numel()
+    cache = synth.build_cache(K, V, classes, residual, _quant(low_normal), override)
+    strategy = "high_uniform_group_low_normal_group" if low_normal else "uniform_group"
+    w_ref, o_ref = O.qkv_matmul(q, cache, None, D, strategy, use_mask=False, round_per_class=False)
+    w, o = decode_attention(q.to(dev), synth.cache_to(cache, dev), None, n + residual, zero_init=False, flags=1 if fused else 0,
+                            low_uniform=not low_normal)
+    torch.testing.assert_close(w.float().cpu(), w_ref.float(), rtol=RTOL, atol=ATOL)
+    torch.testing.assert_close(o.float().cpu(), o_ref.float(), rtol=RTOL, atol=ATOL)
+
+
+@pytest.mark.parametrize("n_rep", [4, 5])
+def test_several_blocks_per_workgroup(dev, n_rep):
+    """More blocks of V than workgroups fit on the chip: the looping form, with every class and a ragged last round."""
+    from hqekv_amd.attention import decode_attention
+    B, Hkv, D, residual = 20, 8, 128, 13
+    q, K, V = synth.make_qkv(B, n_rep * Hkv, Hkv, 3200 + residual, D, 5)
+    classes = synth.split_blocks(3200, (0.1, 0.2, 0.3, 0.3, 0.1), 5)
+    cache = synth.build_cache(K, V, classes, residual, O.uniform_group_quantize_pack_last_dim)
+    w_ref, o_ref = O.qkv_matmul(q, cache, None, D, use_mask=False, round_per_class=False)
+    w, o = decode_attention(q.to(dev), synth.cache_to(cache, dev), None, int(cache[41]), zero_init=False, flags=1)
+    torch.testing.assert_close(w.float().cpu(), w_ref.float(), rtol=RTOL, atol=ATOL)
+    torch.testing.assert_close(o.float().cpu(), o_ref.float(), rtol=RTOL, atol=ATOL)
