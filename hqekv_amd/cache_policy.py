@@ -25,6 +25,7 @@ are not made of whole aligned blocks (token-level V selections): the reference's
 """
 from __future__ import annotations
 
+import functools
 import os
 import threading
 from typing import Dict, List, Optional
@@ -179,6 +180,7 @@ def _none_if_empty(x: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
 
 
 LOW_NORMAL = "high_uniform_group_low_normal_group"
+_new_array = functools.partial(np.empty, dtype=np.int64)
 
 
 def _quantize(x: torch.Tensor, bits: int, strategy: str):
@@ -643,6 +645,19 @@ def compress(past_key_value: tuple, compress_length: int, history_length, K_sort
         raise ValueError("compress_length and history_length must be multiples of 32")
     if K_bit_num.numel() != n_targets or V_bit_num.numel() != n_targets:
         raise ValueError(f"K_bit_num / V_bit_num must hold {n_targets} entries")
+    engine = engine or os.environ.get("HQEKV_POLICY_ENGINE", "auto")
+    if engine not in ("auto", "gather", "steps"):
+        raise ValueError("engine must be 'auto', 'gather' or 'steps'")
+    if engine != "steps" and isinstance(K_sorted_idx, RankedBlocks) and K_sorted_idx._order is None and K_sorted_idx.block_size == BLOCK \
+            and new_V.is_cuda and quant_strategy in ("uniform_group", LOW_NORMAL):
+        # a ranking that lives on the device and classes whose blocks the host knows: the same gathers, prepared in C++
+        from . import _lib
+        done = _lib.host().compress(pkv, history, compress_length, K_sorted_idx.scores, token_importance, bool(times_range),
+                                    V_token_range, K_bit_num, V_bit_num, quant_strategy == LOW_NORMAL, _new_array)
+        if done is not None:
+            if done[1] is not None and last_weights is not None:
+                last_weights.eviction(done[1])
+            return done[0]
     whole = new_K.shape[2] == compress_length and new_V.shape[2] == compress_length   # nothing stays behind
     res_K = None if whole else _none_if_empty(new_K[:, :, compress_length:, :].clone())
     res_V = None if whole else _none_if_empty(new_V[:, :, compress_length:, :].clone())
@@ -655,9 +670,6 @@ def compress(past_key_value: tuple, compress_length: int, history_length, K_sort
     V_sorted_idx = rank_blocks_weighted(block_num, token_importance, V_norm if times_range else None)
 
     dev = new_V.device
-    engine = engine or os.environ.get("HQEKV_POLICY_ENGINE", "auto")
-    if engine not in ("auto", "gather", "steps"):
-        raise ValueError("engine must be 'auto', 'gather' or 'steps'")
     if engine != "steps":
         done = _compress_gather(pkv, new_K, new_V, res_K, res_V, history, compress_length, K_sorted_idx, K_bit_num,
                                 V_bit_num, V_norm, V_sorted_idx, last_weights, quant_strategy, n_targets)
@@ -693,6 +705,12 @@ def reconstruct(past_key_value: tuple, quant_strategy: str, block_size: int = 32
     if quant_strategy not in _STRATEGIES:
         raise ValueError('invalid quant_strategy')
     pkv = past_key_value
+    if quant_strategy in ("uniform_group", LOW_NORMAL) and any(torch.is_tensor(x) and x.is_cuda for x in (pkv[2], pkv[8], pkv[16], pkv[24], pkv[32], pkv[40])):
+        from . import _lib
+        from . import attention as A
+        done = _lib.host().reconstruct(pkv, quant_strategy != LOW_NORMAL, A.idx_cover_once)
+        if done is not None:
+            return done
     k_side, v_side = _read_side(pkv, K_SLOT), _read_side(pkv, V_SLOT)
     new_K, new_V, T = pkv[39], pkv[40], int(pkv[41])
     some = next((x for x in (v_side[16].data, v_side[8].data, v_side[4].data, v_side[2].data, v_side[1].data, new_V) if x is not None), None)

@@ -14,11 +14,15 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <chrono>
 #include <initializer_list>
+#include <vector>
 
 #include <ATen/core/Tensor.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <ATen/ops/empty.h>
+#include <ATen/ops/index_select.h>
+#include <hip/hip_runtime_api.h>
 #include <c10/core/DeviceGuard.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -36,7 +40,18 @@ using at::Tensor;
   X(hqekv_decode_attn)            \
   X(hqekv_decode_step)            \
   X(hqekv_quant_pack_rows)        \
-  X(hqekv_quant_pack_k_tokenmajor)
+  X(hqekv_quant_pack_k_tokenmajor)  \
+  X(hqekv_prompt_attn)              \
+  X(hqekv_prompt_last_rows)         \
+  X(hqekv_prompt_last_rows_workspace_bytes) \
+  X(hqekv_cache_reconstruct)        \
+  X(hqekv_importance_scores)        \
+  X(hqekv_weighted_block_scores)    \
+  X(hqekv_token_range)              \
+  X(hqekv_token_range_append)       \
+  X(hqekv_rank_blocks)              \
+  X(hqekv_plan_side)                \
+  X(hqekv_cache_migrate)
 
 struct Api {
 #define X(n_) decltype(&::n_) n_ = nullptr;
@@ -44,7 +59,7 @@ struct Api {
 #undef X
 } api;
 
-PyObject *s_cover = nullptr;   // interned attribute names
+PyObject *s_cover, *s_blocks, *s_host_version;   // interned attribute names
 
 // the exceptions of _lib.check
 PyObject *raise_rc(int64_t rc, const char *what) {
@@ -611,6 +626,459 @@ PyObject *quantize_into(PyObject *, PyObject *const *a, Py_ssize_t na) {
   END_HANDLE_TH_ERRORS
 }
 
+// ------------------------------------------------------------------------------------------------ prompt
+bool prompt_rows(const Tensor &t, const at::Device &dev, int64_t (&st)[3]) {
+  if (t.dim() != 4 || t.scalar_type() != at::kHalf || t.device() != dev || t.size(3) != 128 || t.stride(3) != 1 || (uintptr_t)t.data_ptr() % 16) return false;
+  for (int i = 0; i < 3; ++i) {
+    st[i] = t.stride(i);
+    if (st[i] % 8) return false;
+  }
+  return true;
+}
+
+// prompt_attention(q, k, v, scaling, causal) -> (B, Hq, T, 128), or None where rows would have to be copied first
+PyObject *prompt_attention(PyObject *, PyObject *const *a, Py_ssize_t na) {
+  HANDLE_TH_ERRORS
+  if (na != 5) return PyErr_Format(PyExc_TypeError, "prompt_attention takes 5 arguments");
+  for (int i : {0, 1, 2})
+    if (!is_tensor(a[i])) Py_RETURN_NONE;
+  const Tensor &q = ten(a[0]), &k = ten(a[1]), &v = ten(a[2]);
+  const double scaling = PyFloat_AsDouble(a[3]);
+  if (PyErr_Occurred()) return nullptr;
+  if (!q.is_cuda()) Py_RETURN_NONE;
+  const at::Device dev = q.device();
+  int64_t sq[3], sk[3], sv[3];
+  if (!prompt_rows(q, dev, sq) || !prompt_rows(k, dev, sk) || !prompt_rows(v, dev, sv)) Py_RETURN_NONE;
+  const int64_t B = q.size(0), Hq = q.size(1), T = q.size(2), Hkv = k.size(1);
+  if (k.size(0) != B || v.size(0) != B || v.size(1) != Hkv || k.size(2) != T || v.size(2) != T) Py_RETURN_NONE;
+  const c10::OptionalDeviceGuard guard(dev);
+  Tensor out = new_tensor({B, Hq, T, 128}, at::kHalf, dev);
+  const int64_t so[3] = {Hq * T * 128, T * 128, 128};
+  const int rc = api.hqekv_prompt_attn(q.data_ptr(), sq, k.data_ptr(), sk, v.data_ptr(), sv, out.data_ptr(), so, B, Hq, Hkv, T, 128, (float)scaling,
+                                       a[4] == Py_True ? 1 : 0, stream_of(dev));
+  if (rc) return raise_rc(rc, "prompt_attn");
+  return THPVariable_Wrap(out);
+  END_HANDLE_TH_ERRORS
+}
+
+// prompt_last_rows(q, k, scaling, rows) -> (B, Hq, rows, T), the causal rule; None as above
+PyObject *prompt_last_rows(PyObject *, PyObject *const *a, Py_ssize_t na) {
+  HANDLE_TH_ERRORS
+  if (na != 4) return PyErr_Format(PyExc_TypeError, "prompt_last_rows takes 4 arguments");
+  if (!is_tensor(a[0]) || !is_tensor(a[1])) Py_RETURN_NONE;
+  const Tensor &q = ten(a[0]), &k = ten(a[1]);
+  const double scaling = PyFloat_AsDouble(a[2]);
+  const int64_t rows = PyLong_AsLongLong(a[3]);
+  if (PyErr_Occurred()) return nullptr;
+  if (!q.is_cuda()) Py_RETURN_NONE;
+  const at::Device dev = q.device();
+  int64_t sq[3], sk[3];
+  if (!prompt_rows(q, dev, sq) || !prompt_rows(k, dev, sk)) Py_RETURN_NONE;
+  const int64_t B = q.size(0), Hq = q.size(1), T = q.size(2), Hkv = k.size(1);
+  if (k.size(0) != B || k.size(2) != T || rows <= 0 || rows > T || rows > 32) Py_RETURN_NONE;
+  const c10::OptionalDeviceGuard guard(dev);
+  Tensor probs = new_tensor({B, Hq, rows, T}, at::kHalf, dev), ws;
+  const int64_t need = api.hqekv_prompt_last_rows_workspace_bytes(B, Hq, T);
+  if (need > 0) ws = new_tensor({need}, at::kByte, dev);
+  const int rc = api.hqekv_prompt_last_rows(q.data_ptr(), sq, k.data_ptr(), sk, nullptr, nullptr, probs.data_ptr(), B, Hq, Hkv, T, 128, rows,
+                                            (float)scaling, need > 0 ? ws.data_ptr() : nullptr, need > 0 ? need : 0, stream_of(dev));
+  if (rc) return raise_rc(rc, "prompt_last_rows");
+  return THPVariable_Wrap(probs);
+  END_HANDLE_TH_ERRORS
+}
+
+// ------------------------------------------------------------------------------------------------ cache maintenance
+// reconstruct(pkv, low_uniform, cover_fn) -> (K, V) dense, or None where the classes and the residual of a side do not
+// name every position exactly once, or a field is not plain
+PyObject *reconstruct(PyObject *, PyObject *const *a, Py_ssize_t na) {
+  HANDLE_TH_ERRORS
+  if (na != 3) return PyErr_Format(PyExc_TypeError, "reconstruct takes 3 arguments");
+  PyObject *pkv = a[0];
+  if (!PyTuple_Check(pkv) || PyTuple_GET_SIZE(pkv) != TUPLE_LEN || !PyLong_Check(PyTuple_GET_ITEM(pkv, TUPLE_LEN - 1))) Py_RETURN_NONE;
+  const int64_t T = PyLong_AsLongLong(PyTuple_GET_ITEM(pkv, TUPLE_LEN - 1));
+  const Tensor *some = nullptr;
+  for (int i : {2, 8, 16, 24, 32, NEW_V})
+    if (!some && is_tensor(PyTuple_GET_ITEM(pkv, i))) some = &ten(PyTuple_GET_ITEM(pkv, i));
+  if (!some || !some->is_cuda() || some->dim() != 4) Py_RETURN_NONE;
+  const at::Device dev = some->device();
+  const int64_t B = some->size(0);
+  Side k, v;
+  const bool low_uniform = a[1] == Py_True;
+  if (!read_side(pkv, true, low_uniform, B, dev, k) || !read_side(pkv, false, low_uniform, B, dev, v)) Py_RETURN_NONE;
+  if (k.tokens != T || v.tokens != T || k.H != v.H || k.D != v.D || k.D % 32) Py_RETURN_NONE;
+  for (Side *s : {&k, &v}) {
+    const int c = cover_once(s->idx, s->n_idx, s->class_tokens, a[2], false);
+    if (c < 0) return nullptr;
+    if (!c) Py_RETURN_NONE;
+    if (s->tokens > s->class_tokens) s->seg[s->n - 1].pos_base = s->class_tokens;
+  }
+  const c10::OptionalDeviceGuard guard(dev);
+  Tensor K = new_tensor({B, k.H, T, k.D}, at::kHalf, dev), V = new_tensor({B, k.H, T, k.D}, at::kHalf, dev);
+  const int rc = api.hqekv_cache_reconstruct(k.seg, k.n, v.seg, v.n, K.data_ptr(), V.data_ptr(), B * k.H, k.D, T, stream_of(dev));
+  if (rc) return raise_rc(rc, "cache_reconstruct");
+  return Py_BuildValue("NN", THPVariable_Wrap(K), THPVariable_Wrap(V));
+  END_HANDLE_TH_ERRORS
+}
+
+// importance(ring, n, total) -> (importance / 32 (total,), block scores (total / 32,)), or None
+PyObject *importance(PyObject *, PyObject *const *a, Py_ssize_t na) {
+  HANDLE_TH_ERRORS
+  if (na != 3) return PyErr_Format(PyExc_TypeError, "importance takes 3 arguments");
+  if (!is_tensor(a[0])) Py_RETURN_NONE;
+  const Tensor &w = ten(a[0]);
+  const int64_t n = PyLong_AsLongLong(a[1]), total = PyLong_AsLongLong(a[2]);
+  if (PyErr_Occurred()) return nullptr;
+  if (!w.is_cuda() || !plain_f16(w, 2, w.device()) || total <= 0 || total > n || total % 32) Py_RETURN_NONE;
+  const at::Device dev = w.device();
+  const c10::OptionalDeviceGuard guard(dev);
+  Tensor imp = new_tensor({total}, at::kHalf, dev), scores = new_tensor({total / 32}, at::kHalf, dev);
+  const int rc = api.hqekv_importance_scores(w.data_ptr(), (int32_t)w.size(0), w.size(1), n, total, imp.data_ptr(), scores.data_ptr(), stream_of(dev));
+  if (rc) return raise_rc(rc, "importance_scores");
+  return Py_BuildValue("NN", THPVariable_Wrap(imp), THPVariable_Wrap(scores));
+  END_HANDLE_TH_ERRORS
+}
+
+// Block numbers of a position array that carries them (see cache_policy._host_blocks), written to `out` as int32.
+bool known_blocks(PyObject *idx, std::vector<int32_t> &out) {
+  const Tensor &t = ten(idx);
+  PyObject *ver = PyObject_GetAttr(idx, s_host_version), *blocks = ver ? PyObject_GetAttr(idx, s_blocks) : nullptr;
+  bool ok = false;
+  if (ver && blocks && PyLong_Check(ver) && !t.is_inference() && PyLong_AsLongLong(ver) == (long long)t._version()) {
+    Py_buffer b;
+    if (PyObject_GetBuffer(blocks, &b, PyBUF_C_CONTIGUOUS | PyBUF_FORMAT) == 0) {
+      if (b.itemsize == 8 && b.ndim == 1 && b.format && (b.format[0] == 'l' || b.format[0] == 'q') && b.len / 8 * 32 == t.numel()) {
+        const int64_t *p = (const int64_t *)b.buf;
+        out.assign(p, p + b.len / 8);
+        ok = true;
+      }
+      PyBuffer_Release(&b);
+    }
+  }
+  Py_XDECREF(ver);
+  Py_XDECREF(blocks);
+  if (PyErr_Occurred()) PyErr_Clear();
+  return ok;
+}
+
+// One side's classes as sources of a migration, with their block numbers.
+struct OldSide {
+  hqekv_cache_class src[6] = {};
+  std::vector<int32_t> blocks[5];
+  int64_t n_blocks = 0;
+};
+constexpr int CLASS_BITS[5] = {16, 8, 4, 2, 1}, K_SLOT[5] = {0, 4, 12, 20, 28}, V_SLOT[5] = {2, 8, 16, 24, 32};
+
+bool old_side(PyObject *pkv, bool is_k, bool low_normal, int64_t B, int64_t H, int64_t D, const at::Device &dev, OldSide &o) {
+  for (int c = 0; c < 5; ++c) {
+    const int slot = is_k ? K_SLOT[c] : V_SLOT[c], bits = CLASS_BITS[c];
+    PyObject *data = PyTuple_GET_ITEM(pkv, slot), *idx = PyTuple_GET_ITEM(pkv, slot + 1);
+    if (data == Py_None) continue;
+    if (!is_tensor(data) || !is_tensor(idx)) return false;
+    const Tensor &t = ten(data);
+    hqekv_cache_class &e = o.src[c];
+    if (bits == 16 ? !plain_f16(t, 4, dev) : !plain_i32(t, 4, dev)) return false;
+    e.bits = bits;
+    e.n_tokens = is_k ? t.size(3) * (bits == 16 ? 1 : 32 / bits) : t.size(2);
+    if (t.size(0) != B || t.size(1) != H || (is_k ? t.size(2) : t.size(3) * (bits == 16 ? 1 : 32 / bits)) != D || ten(idx).numel() != e.n_tokens)
+      return false;
+    e.data = t.data_ptr();
+    if (bits != 16) {
+      PyObject *sc = PyTuple_GET_ITEM(pkv, slot + 2), *zr = PyTuple_GET_ITEM(pkv, slot + 3);
+      if (!is_tensor(sc) || !is_tensor(zr) || !plain_f16(ten(sc), 4, dev) || !plain_f16(ten(zr), 4, dev)) return false;
+      e.scale = ten(sc).data_ptr();
+      e.zero = ten(zr).data_ptr();
+      if (bits == 1 && low_normal) e.layout = HQEKV_LAYOUT_NORMAL1;
+    }
+    if (!known_blocks(idx, o.blocks[c])) return false;
+    o.n_blocks += (int64_t)o.blocks[c].size();
+  }
+  return true;
+}
+
+// A tensor over a part of another's storage, without the dispatcher's way of making a view (two dozen of them per
+// compression).
+Tensor part_of(const Tensor &base, at::IntArrayRef shape, int64_t offset) {
+  Tensor t = at::detail::make_tensor<c10::TensorImpl>(c10::Storage(base.storage()), base.key_set(), base.dtype());
+  t.unsafeGetTensorImpl()->set_sizes_contiguous(shape);
+  t.unsafeGetTensorImpl()->set_storage_offset(offset);
+  return t;
+}
+
+int64_t up(int64_t n, int64_t a) { return (n + a - 1) / a * a; }
+
+// The new classes of one side: three allocations, views of them, the launch that fills them, the fields of the tuple.
+// counts: blocks per class; positions: numpy int64 array of every new block's number, class after class (kept with the
+// tensors for the next compression).
+bool new_side(PyObject *tuple, bool is_k, bool low_normal, OldSide &o, const int32_t *counts, const int32_t *plan_dev, PyObject *positions, int64_t B,
+              int64_t H, int64_t D, const at::Device &dev) {
+  int64_t n16 = 0, n32 = 0, n64 = 0;
+  struct {
+    int64_t n, o_data, o_scale, o_zero, o_idx;
+  } at_[5];
+  for (int c = 0; c < 5; ++c) {
+    const int bits = CLASS_BITS[c];
+    const int64_t n = (int64_t)counts[c] * 32;
+    auto &p = at_[c];
+    p.n = n;
+    if (!n) continue;
+    if (bits == 16) {
+      p.o_data = n16;
+      n16 += up(B * H * D * n, 128);
+    } else {
+      const int64_t groups = up(B * H * n * D / 32, 128);
+      p.o_scale = n16;
+      p.o_zero = n16 + groups;
+      n16 += 2 * groups;
+      p.o_data = n32;
+      n32 += up(B * H * D * n * bits / 32, 64);
+    }
+    p.o_idx = n64;
+    n64 += n;
+  }
+  if (!n64) return true;
+  const Tensor b16 = new_tensor({std::max<int64_t>(n16, 1)}, at::kHalf, dev), b32 = new_tensor({std::max<int64_t>(n32, 1)}, at::kInt, dev),
+               b64 = new_tensor({n64}, at::kLong, dev);
+  hqekv_cache_class dst[5] = {};
+  int n_dst = 0;
+  int64_t blk = 0;
+  auto put = [&](int i, const Tensor &t) {
+    PyObject *v = THPVariable_Wrap(t);
+    PyObject *old = PyTuple_GET_ITEM(tuple, i);
+    PyTuple_SET_ITEM(tuple, i, v);
+    Py_XDECREF(old);
+    return v;
+  };
+  for (int c = 0; c < 5; ++c) {
+    const auto &p = at_[c];
+    if (!p.n) continue;
+    const int bits = CLASS_BITS[c], slot = is_k ? K_SLOT[c] : V_SLOT[c];
+    hqekv_cache_class &e = dst[n_dst++];
+    e.bits = bits;
+    e.n_tokens = p.n;
+    const Tensor idx = part_of(b64, {p.n}, p.o_idx);
+    e.idx = (int64_t *)idx.data_ptr();
+    Tensor data;
+    if (bits == 16) {
+      data = is_k ? part_of(b16, {B, H, D, p.n}, p.o_data) : part_of(b16, {B, H, p.n, D}, p.o_data);
+    } else {
+      data = is_k ? part_of(b32, {B, H, D, p.n * bits / 32}, p.o_data) : part_of(b32, {B, H, p.n, D * bits / 32}, p.o_data);
+      const int64_t shape[4] = {B, H, is_k ? D : p.n, (is_k ? p.n : D) / 32};
+      const Tensor sc = part_of(b16, shape, p.o_scale), zr = part_of(b16, shape, p.o_zero);
+      e.scale = sc.data_ptr();
+      e.zero = zr.data_ptr();
+      if (bits == 1 && low_normal) e.layout = HQEKV_LAYOUT_NORMAL1;
+      put(slot + 2, sc);
+      put(slot + 3, zr);
+    }
+    e.data = data.data_ptr();
+    put(slot, data);
+    PyObject *idx_py = put(slot + 1, idx);
+    // the kernel writes the positions behind torch's back: what rides along describes exactly what it writes
+    PyObject *mine = PySequence_GetSlice(positions, blk, blk + counts[c]), *ver = PyLong_FromLongLong((long long)idx._version());
+    const bool ok = mine && ver && PyObject_SetAttr(idx_py, s_blocks, mine) == 0 && PyObject_SetAttr(idx_py, s_host_version, ver) == 0;
+    Py_XDECREF(mine);
+    Py_XDECREF(ver);
+    if (!ok) return false;
+    blk += counts[c];
+  }
+  const int rc = api.hqekv_cache_migrate(is_k ? 1 : 0, o.src, 6, dst, n_dst, plan_dev, B * H, D, nullptr, stream_of(dev));
+  if (rc) {
+    raise_rc(rc, "cache_migrate");
+    return false;
+  }
+  return true;
+}
+
+bool new_tokens(const Tensor &t, bool is_k, int64_t B, int64_t H, int64_t n, int64_t D, const at::Device &dev, hqekv_cache_class &e) {
+  if (t.dim() != 4 || t.scalar_type() != at::kHalf || t.device() != dev || t.size(0) != B || t.size(1) != H || t.size(2) < n || t.size(3) != D ||
+      t.stride(3) != 1 || t.stride(2) != D || ((H > 1 || B > 1) && (t.stride(1) % D || t.stride(1) < n * D)) || (B > 1 && t.stride(0) != H * t.stride(1)))
+    return false;
+  e.bits = 16;
+  e.n_tokens = n;
+  e.data = t.data_ptr();
+  e.slab_tokens = H > 1 || B > 1 ? t.stride(1) / D : n;
+  e.layout = is_k ? HQEKV_LAYOUT_TOKEN_MAJOR : 0;
+  return true;
+}
+
+// Both block rankings, written by one launch into page-locked memory.  Every entry is stored exactly once, so the ranking
+// is there as soon as no entry holds its initial value: that is watched for a while (a stream synchronisation wakes up
+// some ten microseconds later), then the stream is waited for.
+bool host_orders(const void *const (&scores)[2], int64_t n, const Tensor &order, const at::Device &dev) {
+  volatile int32_t *p = (volatile int32_t *)order.data_ptr();
+  for (int64_t i = 0; i < 2 * n; ++i) p[i] = -1;
+  const int rc = api.hqekv_rank_blocks(scores, 2, n, (int32_t *)order.data_ptr(), stream_of(dev));
+  if (rc) {
+    raise_rc(rc, "rank_blocks");
+    return false;
+  }
+  hipError_t err = hipSuccess;
+  Py_BEGIN_ALLOW_THREADS;
+  const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(2);
+  int64_t i = 0;
+  while (i < 2 * n) {
+    if (p[i] >= 0) {
+      ++i;
+    } else if (std::chrono::steady_clock::now() > until) {
+      err = hipStreamSynchronize((hipStream_t)stream_of(dev));
+      break;
+    }
+  }
+  Py_END_ALLOW_THREADS;
+  if (err != hipSuccess) PyErr_Format(PyExc_RuntimeError, "rank_blocks: HIP error %d", (int)err);
+  return err == hipSuccess;
+}
+
+bool six_counts(PyObject *o, int64_t (&out)[6], int &n) {
+  if (!is_tensor(o)) return false;
+  const Tensor &t = ten(o);
+  if (!t.device().is_cpu() || t.dim() != 1 || !t.is_contiguous() || (t.numel() != 5 && t.numel() != 6)) return false;
+  n = (int)t.numel();
+  if (t.scalar_type() == at::kInt)
+    for (int i = 0; i < n; ++i) out[i] = t.data_ptr<int32_t>()[i];
+  else if (t.scalar_type() == at::kLong)
+    for (int i = 0; i < n; ++i) out[i] = t.data_ptr<int64_t>()[i];
+  else return false;
+  return true;
+}
+
+// compress(pkv, history, length, k_scores, importance, times_range, V_range or None, K_counts, V_counts, low_normal,
+// new_array): cache_policy.compress for a cache, rankings and counts made of whole blocks.  new_array(n): an int64 numpy
+// array.  -> (the new tuple, kept positions (device) or None when nothing was evicted), or None where that does not hold
+// -- found out before anything is launched except the two score kernels.
+PyObject *compress(PyObject *, PyObject *const *a, Py_ssize_t na) {
+  HANDLE_TH_ERRORS
+  if (na != 11) return PyErr_Format(PyExc_TypeError, "compress takes 11 arguments");
+  PyObject *pkv = a[0];
+  const int64_t history = PyLong_AsLongLong(a[1]), length = PyLong_AsLongLong(a[2]);
+  if (PyErr_Occurred()) return nullptr;
+  const bool times_range = a[5] == Py_True, low_normal = a[9] == Py_True;
+  if (!PyTuple_Check(pkv) || PyTuple_GET_SIZE(pkv) != TUPLE_LEN || !is_tensor(a[3]) || !is_tensor(a[4])) Py_RETURN_NONE;
+  PyObject *nk = PyTuple_GET_ITEM(pkv, NEW_K), *nv = PyTuple_GET_ITEM(pkv, NEW_V), *prev = PyTuple_GET_ITEM(pkv, 38);
+  if (!is_tensor(nk) || !is_tensor(nv)) Py_RETURN_NONE;
+  const Tensor &newK = ten(nk), &newV = ten(nv), &scores_k = ten(a[3]), &imp = ten(a[4]);
+  if (!newV.is_cuda() || newV.dim() != 4) Py_RETURN_NONE;
+  const at::Device dev = newV.device();
+  const int64_t B = newV.size(0), H = newV.size(1), D = newV.size(3), total = history + length, nb = total / 32;
+  if (total <= 0 || total % 32 || history % 32 || length <= 0 || nb > 32768 || D % 32 || B * H > 1024) Py_RETURN_NONE;
+  if (!plain_f16(imp, 1, dev) || imp.numel() != total || !plain_f16(scores_k, 1, dev) || scores_k.numel() != nb) Py_RETURN_NONE;
+  OldSide ks, vs;
+  int64_t kc[6] = {}, vc[6] = {};
+  int n_k = 0, n_v = 0;
+  if (!six_counts(a[7], kc, n_k) || !six_counts(a[8], vc, n_v) || !new_tokens(newK, true, B, H, length, D, dev, ks.src[5]) ||
+      !new_tokens(newV, false, B, H, length, D, dev, vs.src[5]) || !old_side(pkv, true, low_normal, B, H, D, dev, ks) ||
+      !old_side(pkv, false, low_normal, B, H, D, dev, vs) || ks.n_blocks != history / 32 || vs.n_blocks != history / 32)
+    Py_RETURN_NONE;
+  if ((uintptr_t)newV.data_ptr() % 16) Py_RETURN_NONE;
+  for (const int64_t *c : {kc, vc}) {   // what the planner will ask for
+    int64_t sum = 0;
+    for (int i = 0; i < 6; ++i) {
+      if (c[i] < 0 || c[i] % 32) Py_RETURN_NONE;
+      sum += c[i];
+    }
+    if (sum != total) Py_RETURN_NONE;
+  }
+  const c10::OptionalDeviceGuard guard(dev);
+  void *stream = stream_of(dev);
+  // ---- token ranges of V: the older ones and the new tokens'
+  Tensor range;
+  int rc = 0;
+  if (a[6] != Py_None) {
+    if (!is_tensor(a[6])) Py_RETURN_NONE;
+    range = ten(a[6]);
+    if (!plain_f16(range, 1, dev) || range.numel() != total) Py_RETURN_NONE;
+  } else if (prev == Py_None) {
+    if (history) Py_RETURN_NONE;
+    range = new_tensor({length}, at::kHalf, dev);
+    rc = api.hqekv_token_range(newV.data_ptr(), B, H, length, D, vs.src[5].slab_tokens, range.data_ptr(), stream);
+  } else {
+    if (!is_tensor(prev) || !plain_f16(ten(prev), 1, dev) || ten(prev).numel() != history) Py_RETURN_NONE;
+    range = new_tensor({total}, at::kHalf, dev);
+    rc = api.hqekv_token_range_append(newV.data_ptr(), B, H, length, D, vs.src[5].slab_tokens, ten(prev).data_ptr(), history, range.data_ptr(), stream);
+  }
+  if (rc) return raise_rc(rc, "token_range");
+  // ---- both rankings
+  const Tensor scores_v = new_tensor({nb}, at::kHalf, dev);
+  rc = api.hqekv_weighted_block_scores(imp.data_ptr(), times_range ? range.data_ptr() : nullptr, total, scores_v.data_ptr(), stream);
+  if (rc) return raise_rc(rc, "weighted_block_scores");
+  const Tensor order = at::empty({2 * nb}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+  const void *const sc[2] = {scores_k.data_ptr(), scores_v.data_ptr()};
+  if (!host_orders(sc, nb, order, dev)) return nullptr;
+  // ---- the plans of both sides, one transfer for them and for the positions that survive on the V side
+  std::vector<int64_t> order64(nb);
+  std::vector<int32_t> alive(nb);
+  Tensor up_h = at::empty({2 * nb + total}, at::TensorOptions().dtype(at::kLong).pinned_memory(true));
+  int32_t *words = (int32_t *)up_h.data_ptr(), counts[2][5];
+  int32_t n_alive[2] = {0, 0};
+  for (int side = 0; side < 2; ++side) {
+    OldSide &o = side ? vs : ks;
+    const int32_t *old[5];
+    int32_t cnt[5];
+    for (int c = 0; c < 5; ++c) {
+      old[c] = o.blocks[c].data();
+      cnt[c] = (int32_t)o.blocks[c].size();
+    }
+    for (int64_t i = 0; i < nb; ++i) order64[i] = ((const int32_t *)order.data_ptr())[side * nb + i];
+    rc = api.hqekv_plan_side(old, cnt, (int32_t)(history / 32), (int32_t)(length / 32), order64.data(), side ? vc : kc, side ? n_v : n_k, counts[side],
+                             words + side * 2 * nb, alive.data(), &n_alive[side]);
+    if (rc) Py_RETURN_NONE;   // not a whole-block selection after all
+  }
+  const bool evicted = n_alive[1] < nb;
+  int64_t n_up = 2 * nb;
+  if (evicted) {
+    int64_t *keep = (int64_t *)up_h.data_ptr() + n_up;
+    for (int32_t i = 0; i < n_alive[1]; ++i)
+      for (int j = 0; j < 32; ++j) *keep++ = (int64_t)alive[i] * 32 + j;
+    n_up += (int64_t)n_alive[1] * 32;
+  }
+  const Tensor up_d = new_tensor({n_up}, at::kLong, dev);
+  up_d.copy_(part_of(up_h, {n_up}, 0), /*non_blocking=*/true);
+  // ---- the new tuple
+  PyObject *out = PyTuple_New(TUPLE_LEN);
+  if (!out) return nullptr;
+  for (int i = 0; i < TUPLE_LEN; ++i) {
+    PyObject *x = (i < 36 || i == NEW_K || i == NEW_V) ? Py_None : PyTuple_GET_ITEM(pkv, i);
+    Py_INCREF(x);
+    PyTuple_SET_ITEM(out, i, x);
+  }
+  for (int side = 0; side < 2; ++side) {
+    PyObject *pos = PyObject_CallFunction(a[10], "L", (long long)n_alive[side]);
+    Py_buffer b;
+    if (!pos || PyObject_GetBuffer(pos, &b, PyBUF_WRITABLE | PyBUF_C_CONTIGUOUS) != 0) {
+      Py_XDECREF(pos);
+      Py_DECREF(out);
+      return nullptr;
+    }
+    const int32_t *w = words + side * 2 * nb;
+    const bool room = b.len == 8 * (Py_ssize_t)n_alive[side];
+    for (int32_t i = 0; room && i < n_alive[side]; ++i) ((int64_t *)b.buf)[i] = w[n_alive[side] + i];
+    PyBuffer_Release(&b);
+    const bool ok = room && new_side(out, side == 0, low_normal, side ? vs : ks, counts[side], (const int32_t *)up_d.data_ptr() + side * 2 * nb, pos, B, H, D, dev);
+    Py_DECREF(pos);
+    if (!ok) {
+      if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "new_array");
+      Py_DECREF(out);
+      return nullptr;
+    }
+  }
+  auto put = [&](int i, PyObject *v) {
+    PyObject *old = PyTuple_GET_ITEM(out, i);
+    PyTuple_SET_ITEM(out, i, v);
+    Py_XDECREF(old);
+  };
+  Tensor keep;
+  if (evicted) {
+    keep = part_of(up_d, {n_up - 2 * nb}, 2 * nb);
+    range = at::index_select(range, 0, keep);
+  }
+  put(38, THPVariable_Wrap(range));
+  if (newK.size(2) > length) put(NEW_K, THPVariable_Wrap(newK.slice(2, length).clone(at::MemoryFormat::Contiguous)));
+  if (newV.size(2) > length) put(NEW_V, THPVariable_Wrap(newV.slice(2, length).clone(at::MemoryFormat::Contiguous)));
+  if (evicted) return Py_BuildValue("NN", out, THPVariable_Wrap(keep));
+  return Py_BuildValue("NO", out, Py_None);
+  END_HANDLE_TH_ERRORS
+}
+
 // bind(path): take the kernels' entry points from this library
 PyObject *bind(PyObject *, PyObject *path) {
   const char *p = PyUnicode_AsUTF8(path);
@@ -628,6 +1096,11 @@ PyObject *bind(PyObject *, PyObject *path) {
 PyMethodDef module_methods[] = {
     {"bind", bind, METH_O, nullptr},
     {"decode", (PyCFunction)(void (*)(void))decode, METH_FASTCALL, nullptr},
+    {"prompt_attention", (PyCFunction)(void (*)(void))prompt_attention, METH_FASTCALL, nullptr},
+    {"prompt_last_rows", (PyCFunction)(void (*)(void))prompt_last_rows, METH_FASTCALL, nullptr},
+    {"reconstruct", (PyCFunction)(void (*)(void))reconstruct, METH_FASTCALL, nullptr},
+    {"importance", (PyCFunction)(void (*)(void))importance, METH_FASTCALL, nullptr},
+    {"compress", (PyCFunction)(void (*)(void))compress, METH_FASTCALL, nullptr},
     {"quantize_into", (PyCFunction)(void (*)(void))quantize_into, METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr},
 };
@@ -653,7 +1126,9 @@ PyMODINIT_FUNC PyInit__host(void) {
   PyObject *m = PyModule_Create(&module_def);
   if (!m) return nullptr;
   s_cover = PyUnicode_InternFromString("_hq_cover");
-  if (!s_cover ||
+  s_blocks = PyUnicode_InternFromString("_hq_blocks");
+  s_host_version = PyUnicode_InternFromString("_hq_host_version");
+  if (!s_cover || !s_blocks || !s_host_version ||
       !add_type(m, tables_type, "hqekv_amd._host.StepTables", "StepTables", sizeof(StepTables), tables_new, tables_free, tables_methods,
                 nullptr, 0) ||
       !add_type(m, kivi_type, "hqekv_amd._host.KiviState", "KiviState", sizeof(KiviState), kivi_new, kivi_free, kivi_methods, kivi_fields, 0)) {

@@ -36,6 +36,9 @@ def prompt_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scaling:
     """softmax(q k^T * scaling [causal]) v -> (B, Hq, T, 128) fp16, contiguous."""
     if not supported(q, k, v):
         raise NotImplementedError("prompt_attention: fp16 CUDA tensors of head_dim 128 only")
+    out = _lib.host().prompt_attention(q, k, v, scaling, bool(causal))
+    if out is not None:
+        return out
     B, Hq, T, D = q.shape
     Hkv = k.shape[1]
     q, k, v = _rows(q), _rows(k), _rows(v)
@@ -55,6 +58,10 @@ def prompt_last_rows(q: torch.Tensor, k: torch.Tensor, scaling: float, rows: int
     ``sliced``: let the library cut the keys into slices over more workgroups (two launches) when there are few heads."""
     if not supported(q, k):
         raise NotImplementedError("prompt_last_rows: fp16 CUDA tensors of head_dim 128 only")
+    if attention_mask is None and sliced:
+        probs = _lib.host().prompt_last_rows(q, k, scaling, rows)
+        if probs is not None:
+            return probs
     B, Hq, T, D = q.shape
     Hkv = k.shape[1]
     if not 0 < rows <= min(MAX_LAST_ROWS, T):

@@ -245,13 +245,8 @@ class last_attn_weights:
         n, w = self.kv_seq_len, self.weights
         if w.is_cuda and w.dtype == torch.float16 and w.is_contiguous() and 0 < total <= n and total % 32 == 0:
             from . import _lib
-            imp = torch.empty(total, dtype=torch.float16, device=w.device)
-            scores = torch.empty(total // 32, dtype=torch.float16, device=w.device)
-            with _lib.on_device(w.device):
-                rc = _lib.load().hqekv_importance_scores(w.data_ptr(), w.shape[0], w.shape[1], n, total, imp.data_ptr(),
-                                                         scores.data_ptr(), _lib.stream_ptr(w.device))
-            _lib.check(rc, "importance_scores")
-            return imp, RankedBlocks(scores, 32)
+            done = _lib.host().importance(w, n, total)
+            return done[0], RankedBlocks(done[1], 32)
         imp = self.calculate_token_importance()[:total].clone()
         return imp, rank_blocks(32, total // 32, imp)
 

@@ -310,3 +310,34 @@ def test_cache_migrate_random_plans(dev, is_k, low_normal, D):
             else:
                 assert torch.equal(oi[sl], wi[sl]), f"{b}-bit class: block {k} of a plan with refused entries"
         u += wi.numel() // 32
+
+
+@pytest.mark.parametrize("times_range", [True, False])
+@pytest.mark.parametrize("strategy", ["uniform_group", "high_uniform_group_low_normal_group"])
+def test_native_compression_equals_step_engine(dev, strategy, times_range, monkeypatch):
+    """Rankings still on the device (``RankedBlocks``) and classes whose blocks the host knows take the compression
+    prepared in C++ -- demotions, evictions from both sides and the ring, a residual left over -- bit for bit what the
+    step-by-step engine does with the same rankings spelt out."""
+    from hqekv_amd import _lib, cache_policy
+    from hqekv_amd.public_func import last_attn_weights, rank_blocks
+    native, taken = _lib.host().compress, []
+    monkeypatch.setattr(_lib.host(), "compress", lambda *a: taken.append(native(*a)) or taken[-1])
+
+    def runner(engine):
+        lw = last_attn_weights(20)
+        lw.set_max_length(512)
+        lw.weights = torch.rand(20, 512, generator=torch.Generator().manual_seed(2)).half().to(dev)
+
+        def f(pkv, cl, hist, ks, kb, vb, imp):
+            imp = imp.half()
+            ranked = rank_blocks(32, (hist + cl) // 32, imp)
+            return cache_policy.compress(pkv, cl, hist, ranked if engine is None else ranked.tokens(), kb, vb, imp, strategy,
+                                         last_weights=lw, times_range=times_range, n_targets=6, engine=engine)
+        return PC.run(f, to_dev=lambda x: x.to(dev))[0], lw.weights.cpu()
+
+    (fast, ring), (slow, ring_slow) = runner(None), runner("steps")
+    assert len(taken) == len(PC.STEPS) and all(t is not None for t in taken)
+    for step, (a, b) in enumerate(zip(fast, slow)):
+        for slot in range(42):
+            _same(a[slot], b[slot].cpu() if torch.is_tensor(b[slot]) else b[slot], f"step {step} slot {slot}")
+    assert torch.equal(ring, ring_slow)
