@@ -47,9 +47,9 @@ EXPORTS = (
     "hqekv_gemv_workspace_bytes", "hqekv_gemv_uniform_group", "hqekv_gemv_normal_group",
     "hqekv_qk_hybrid", "hqekv_scale_softmax", "hqekv_pv_workspace_bytes", "hqekv_pv_hybrid",
     "hqekv_decode_workspace_bytes", "hqekv_decode_attn", "hqekv_decode_attn_static", "hqekv_decode_step", "hqekv_ring_row",
-    "hqekv_importance_scores", "hqekv_weighted_block_scores", "hqekv_token_range", "hqekv_token_range_append", "hqekv_rank_blocks",
+    "hqekv_importance_scores", "hqekv_weighted_block_scores", "hqekv_token_range", "hqekv_token_range_append", "hqekv_range_block_scores", "hqekv_rank_blocks",
     "hqekv_prompt_attn", "hqekv_prompt_last_rows", "hqekv_prompt_last_rows_workspace_bytes",
-    "hqekv_cache_migrate", "hqekv_cache_reconstruct", "hqekv_cover_once", "hqekv_plan_side",
+    "hqekv_cache_migrate", "hqekv_cache_migrate_both", "hqekv_fetch_words", "hqekv_cache_reconstruct", "hqekv_cover_once", "hqekv_plan_side",
 )
 
 
@@ -131,6 +131,7 @@ _PROTOS = {
     "hqekv_weighted_block_scores": (C.c_int, [_vp, _vp, _i64, _vp, _vp]),
     "hqekv_token_range": (C.c_int, [_vp, _i64, _i64, _i64, _i64, _i64, _vp, _vp]),
     "hqekv_token_range_append": (C.c_int, [_vp, _i64, _i64, _i64, _i64, _i64, _vp, _i64, _vp, _vp]),
+    "hqekv_range_block_scores": (C.c_int, [_vp, _i64, _i64, _i64, _i64, _i64, _vp, _i64, _vp, _int, _vp, _vp, _vp]),
     "hqekv_rank_blocks": (C.c_int, [_vp, _int, _i64, _vp, _vp]),
     "hqekv_prompt_attn": (C.c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, C.c_float, _int, _vp]),
     "hqekv_prompt_last_rows": (C.c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, C.c_float, _vp, _i64, _vp]),
@@ -140,6 +141,8 @@ _PROTOS = {
     "hqekv_decode_attn_static": (C.c_int, [_SEGP, _int, _SEGP, _int, _vp, _vp, _i64, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _int, _vp]),
     "hqekv_plan_side": (C.c_int, [C.POINTER(_vp), _vp, C.c_int32, C.c_int32, _vp, _vp, C.c_int32, _vp, _vp, _vp, _vp]),
     "hqekv_cache_migrate": (C.c_int, [_int, _CCP, _int, _CCP, _int, _vp, _i64, _i64, _vp, _vp]),
+    "hqekv_cache_migrate_both": (C.c_int, [_CCP, _int, _CCP, _int, _vp, _CCP, _int, _CCP, _int, _vp, _i64, _i64, _vp, _vp]),
+    "hqekv_fetch_words": (C.c_int, [_vp, _vp, _i64, _vp]),
 }
 STATIC_SCRATCH_BYTES = 8 << 20   # HQEKV_STATIC_SCRATCH_BYTES
 

@@ -28,13 +28,14 @@ from __future__ import annotations
 import functools
 import os
 import threading
+import weakref
 from typing import Dict, List, Optional
 
 import numpy as np
 import torch
 
 from . import pack_unpack as PU
-from .public_func import RankedBlocks, calculate_token_range, get_block_token_idx, rank_blocks_weighted
+from .public_func import RankedBlocks, calculate_token_range, get_block_token_idx, last_attn_weights, rank_blocks_weighted
 
 BLOCK = 32
 CLASS_BITS = (16, 8, 4, 2, 1)
@@ -629,8 +630,10 @@ def compress(past_key_value: tuple, compress_length: int, history_length, K_sort
              K_bit_num: torch.Tensor, V_bit_num: torch.Tensor, token_importance: torch.Tensor,
              quant_strategy: str, *, last_weights=None, block_size: int = 32, group_size: int = 32,
              times_range: bool = True, n_targets: int = 6, V_token_range: Optional[torch.Tensor] = None,
-             engine: Optional[str] = None) -> tuple:
-    """``engine``: None / "auto" = the one-launch-per-side gather when the selection is made of whole aligned blocks,
+             engine: Optional[str] = None, residual_buffers: Optional[tuple] = None) -> tuple:
+    """``residual_buffers``: a (K, V) pair of (B, H, capacity, D) tensors the residual may be put into; its fields in the
+    result are then their heads.
+    ``engine``: None / "auto" = the one-launch-per-side gather when the selection is made of whole aligned blocks,
     else the step-by-step engine; "steps" forces the latter, "gather" raises when it does not apply (tests)."""
     if quant_strategy not in _STRATEGIES:
         raise ValueError('invalid quant_strategy')
@@ -652,8 +655,10 @@ def compress(past_key_value: tuple, compress_length: int, history_length, K_sort
             and new_V.is_cuda and quant_strategy in ("uniform_group", LOW_NORMAL):
         # a ranking that lives on the device and classes whose blocks the host knows: the same gathers, prepared in C++
         from . import _lib
+        ring = last_weights.weights if type(last_weights) is last_attn_weights else None
         done = _lib.host().compress(pkv, history, compress_length, K_sorted_idx.scores, token_importance, bool(times_range),
-                                    V_token_range, K_bit_num, V_bit_num, quant_strategy == LOW_NORMAL, _new_array)
+                                    V_token_range, K_bit_num, V_bit_num, quant_strategy == LOW_NORMAL,
+                                    ring, residual_buffers, _new_array, weakref.ref)
         if done is not None:
             if done[1] is not None and last_weights is not None:
                 last_weights.eviction(done[1])

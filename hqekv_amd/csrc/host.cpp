@@ -21,7 +21,7 @@
 #include <ATen/core/Tensor.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <ATen/ops/empty.h>
-#include <ATen/ops/index_select.h>
+#include <ATen/core/CachingHostAllocator.h>
 #include <hip/hip_runtime_api.h>
 #include <c10/core/DeviceGuard.h>
 #include <torch/csrc/Exceptions.h>
@@ -47,11 +47,11 @@ using at::Tensor;
   X(hqekv_cache_reconstruct)        \
   X(hqekv_importance_scores)        \
   X(hqekv_weighted_block_scores)    \
-  X(hqekv_token_range)              \
-  X(hqekv_token_range_append)       \
+  X(hqekv_range_block_scores)       \
   X(hqekv_rank_blocks)              \
   X(hqekv_plan_side)                \
-  X(hqekv_cache_migrate)
+  X(hqekv_fetch_words)              \
+  X(hqekv_cache_migrate_both)
 
 struct Api {
 #define X(n_) decltype(&::n_) n_ = nullptr;
@@ -90,7 +90,7 @@ Tensor new_tensor(at::IntArrayRef shape, at::ScalarType type, const at::Device &
 // scale, zero; 39/40 the fp16 residual.
 constexpr int BITS[4] = {8, 4, 2, 1};
 constexpr int K_BASE[4] = {4, 12, 20, 28}, V_BASE[4] = {8, 16, 24, 32};
-constexpr int NEW_K = 39, NEW_V = 40, TUPLE_LEN = 42;
+constexpr int RANGES = 38, NEW_K = 39, NEW_V = 40, TUPLE_LEN = 42;
 
 struct Side {
   hqekv_seg seg[HQEKV_MAX_SEGS + 2];
@@ -806,11 +806,14 @@ Tensor part_of(const Tensor &base, at::IntArrayRef shape, int64_t offset) {
 
 int64_t up(int64_t n, int64_t a) { return (n + a - 1) / a * a; }
 
-// The new classes of one side: three allocations, views of them, the launch that fills them, the fields of the tuple.
-// counts: blocks per class; positions: numpy int64 array of every new block's number, class after class (kept with the
-// tensors for the next compression).
-bool new_side(PyObject *tuple, bool is_k, bool low_normal, OldSide &o, const int32_t *counts, const int32_t *plan_dev, PyObject *positions, int64_t B,
-              int64_t H, int64_t D, const at::Device &dev) {
+// The new classes of one side: three allocations, tensors over parts of them.
+struct NewSide {
+  hqekv_cache_class dst[5] = {};
+  Tensor data[5], scale[5], zero[5], idx[5];
+  int n_dst = 0;
+};
+
+void new_side(bool is_k, bool low_normal, const int32_t *counts, int64_t B, int64_t H, int64_t D, const at::Device &dev, NewSide &o) {
   int64_t n16 = 0, n32 = 0, n64 = 0;
   struct {
     int64_t n, o_data, o_scale, o_zero, o_idx;
@@ -835,58 +838,84 @@ bool new_side(PyObject *tuple, bool is_k, bool low_normal, OldSide &o, const int
     p.o_idx = n64;
     n64 += n;
   }
-  if (!n64) return true;
+  if (!n64) return;
   const Tensor b16 = new_tensor({std::max<int64_t>(n16, 1)}, at::kHalf, dev), b32 = new_tensor({std::max<int64_t>(n32, 1)}, at::kInt, dev),
                b64 = new_tensor({n64}, at::kLong, dev);
-  hqekv_cache_class dst[5] = {};
-  int n_dst = 0;
-  int64_t blk = 0;
-  auto put = [&](int i, const Tensor &t) {
-    PyObject *v = THPVariable_Wrap(t);
-    PyObject *old = PyTuple_GET_ITEM(tuple, i);
-    PyTuple_SET_ITEM(tuple, i, v);
-    Py_XDECREF(old);
-    return v;
-  };
   for (int c = 0; c < 5; ++c) {
     const auto &p = at_[c];
     if (!p.n) continue;
-    const int bits = CLASS_BITS[c], slot = is_k ? K_SLOT[c] : V_SLOT[c];
-    hqekv_cache_class &e = dst[n_dst++];
+    const int bits = CLASS_BITS[c];
+    hqekv_cache_class &e = o.dst[o.n_dst++];
     e.bits = bits;
     e.n_tokens = p.n;
-    const Tensor idx = part_of(b64, {p.n}, p.o_idx);
-    e.idx = (int64_t *)idx.data_ptr();
-    Tensor data;
+    o.idx[c] = part_of(b64, {p.n}, p.o_idx);
+    e.idx = (int64_t *)o.idx[c].data_ptr();
     if (bits == 16) {
-      data = is_k ? part_of(b16, {B, H, D, p.n}, p.o_data) : part_of(b16, {B, H, p.n, D}, p.o_data);
+      o.data[c] = is_k ? part_of(b16, {B, H, D, p.n}, p.o_data) : part_of(b16, {B, H, p.n, D}, p.o_data);
     } else {
-      data = is_k ? part_of(b32, {B, H, D, p.n * bits / 32}, p.o_data) : part_of(b32, {B, H, p.n, D * bits / 32}, p.o_data);
+      o.data[c] = is_k ? part_of(b32, {B, H, D, p.n * bits / 32}, p.o_data) : part_of(b32, {B, H, p.n, D * bits / 32}, p.o_data);
       const int64_t shape[4] = {B, H, is_k ? D : p.n, (is_k ? p.n : D) / 32};
-      const Tensor sc = part_of(b16, shape, p.o_scale), zr = part_of(b16, shape, p.o_zero);
-      e.scale = sc.data_ptr();
-      e.zero = zr.data_ptr();
+      o.scale[c] = part_of(b16, shape, p.o_scale);
+      o.zero[c] = part_of(b16, shape, p.o_zero);
+      e.scale = o.scale[c].data_ptr();
+      e.zero = o.zero[c].data_ptr();
       if (bits == 1 && low_normal) e.layout = HQEKV_LAYOUT_NORMAL1;
-      put(slot + 2, sc);
-      put(slot + 3, zr);
     }
-    e.data = data.data_ptr();
-    put(slot, data);
-    PyObject *idx_py = put(slot + 1, idx);
-    // the kernel writes the positions behind torch's back: what rides along describes exactly what it writes
-    PyObject *mine = PySequence_GetSlice(positions, blk, blk + counts[c]), *ver = PyLong_FromLongLong((long long)idx._version());
-    const bool ok = mine && ver && PyObject_SetAttr(idx_py, s_blocks, mine) == 0 && PyObject_SetAttr(idx_py, s_host_version, ver) == 0;
+    e.data = o.data[c].data_ptr();
+  }
+}
+
+void put_item(PyObject *tuple, int i, PyObject *v) {
+  PyObject *old = PyTuple_GET_ITEM(tuple, i);
+  PyTuple_SET_ITEM(tuple, i, v);
+  Py_XDECREF(old);
+}
+
+// The fields of one side into the new tuple.  The kernel writes the positions behind torch's back, and what rides on
+// the arrays says exactly what it writes: the block numbers (positions: numpy int64, class after class), for the next
+// compression, and -- the classes together are a permutation of the n_blocks surviving blocks -- the verdict of
+// attention.idx_cover_once about these arrays: every position once, in whole runs of 32.
+bool put_side(PyObject *tuple, bool is_k, const NewSide &o, const int32_t *counts, int64_t n_blocks, PyObject *positions, PyObject *weak_ref) {
+  PyObject *idx[5];
+  int n_idx = 0;
+  int64_t blk = 0;
+  for (int c = 0; c < 5; ++c) {
+    if (!counts[c]) continue;
+    const int slot = is_k ? K_SLOT[c] : V_SLOT[c];
+    put_item(tuple, slot, THPVariable_Wrap(o.data[c]));
+    if (CLASS_BITS[c] != 16) {
+      put_item(tuple, slot + 2, THPVariable_Wrap(o.scale[c]));
+      put_item(tuple, slot + 3, THPVariable_Wrap(o.zero[c]));
+    }
+    PyObject *i = idx[n_idx++] = THPVariable_Wrap(o.idx[c]);
+    put_item(tuple, slot + 1, i);
+    PyObject *mine = PySequence_GetSlice(positions, blk, blk + counts[c]), *ver = PyLong_FromLongLong((long long)o.idx[c]._version());
+    const bool ok = mine && ver && PyObject_SetAttr(i, s_blocks, mine) == 0 && PyObject_SetAttr(i, s_host_version, ver) == 0;
     Py_XDECREF(mine);
     Py_XDECREF(ver);
     if (!ok) return false;
     blk += counts[c];
   }
-  const int rc = api.hqekv_cache_migrate(is_k ? 1 : 0, o.src, 6, dst, n_dst, plan_dev, B * H, D, nullptr, stream_of(dev));
-  if (rc) {
-    raise_rc(rc, "cache_migrate");
-    return false;
+  if (!n_idx) return true;
+  PyObject *key = PyTuple_New(n_idx + 1), *refs = PyList_New(n_idx);
+  bool ok = key && refs;
+  for (int i = 0; ok && i < n_idx; ++i) {
+    const Tensor &t = ten(idx[i]);
+    PyObject *k = Py_BuildValue("KLL", (unsigned long long)(uintptr_t)t.data_ptr(), (long long)t.numel(), (long long)t._version());
+    PyObject *r = PyObject_CallFunctionObjArgs(weak_ref, idx[i], nullptr);
+    ok = k && r;
+    PyTuple_SET_ITEM(key, i, k);
+    PyList_SET_ITEM(refs, i, r);
   }
-  return true;
+  if (ok) {
+    PyTuple_SET_ITEM(key, n_idx, PyLong_FromLongLong((long long)n_blocks * 32));
+    PyObject *cover = Py_BuildValue("(OOOO)", key, Py_True, refs, Py_True);
+    ok = cover && PyObject_SetAttr(idx[0], s_cover, cover) == 0;
+    Py_XDECREF(cover);
+  }
+  Py_XDECREF(key);
+  Py_XDECREF(refs);
+  return ok;
 }
 
 bool new_tokens(const Tensor &t, bool is_k, int64_t B, int64_t H, int64_t n, int64_t D, const at::Device &dev, hqekv_cache_class &e) {
@@ -943,18 +972,20 @@ bool six_counts(PyObject *o, int64_t (&out)[6], int &n) {
 }
 
 // compress(pkv, history, length, k_scores, importance, times_range, V_range or None, K_counts, V_counts, low_normal,
-// new_array): cache_policy.compress for a cache, rankings and counts made of whole blocks.  new_array(n): an int64 numpy
-// array.  -> (the new tuple, kept positions (device) or None when nothing was evicted), or None where that does not hold
-// -- found out before anything is launched except the two score kernels.
+// ring or None, (K buffer, V buffer) or None, new_array, weak_ref): cache_policy.compress for a cache, rankings and counts
+// made of whole blocks.  ring: the importance ring, whose evicted columns are taken out; buffers (B, H, capacity, D): where
+// the residual goes, its fields are their heads then.  new_array(n): an int64 numpy array; weak_ref: weakref.ref.
+// -> (the new tuple, positions kept where tokens were evicted and no ring was given, else None), or None where that does not
+// hold -- found out before anything is launched except the score and rank kernels.
 PyObject *compress(PyObject *, PyObject *const *a, Py_ssize_t na) {
   HANDLE_TH_ERRORS
-  if (na != 11) return PyErr_Format(PyExc_TypeError, "compress takes 11 arguments");
+  if (na != 14) return PyErr_Format(PyExc_TypeError, "compress takes 14 arguments");
   PyObject *pkv = a[0];
   const int64_t history = PyLong_AsLongLong(a[1]), length = PyLong_AsLongLong(a[2]);
   if (PyErr_Occurred()) return nullptr;
   const bool times_range = a[5] == Py_True, low_normal = a[9] == Py_True;
   if (!PyTuple_Check(pkv) || PyTuple_GET_SIZE(pkv) != TUPLE_LEN || !is_tensor(a[3]) || !is_tensor(a[4])) Py_RETURN_NONE;
-  PyObject *nk = PyTuple_GET_ITEM(pkv, NEW_K), *nv = PyTuple_GET_ITEM(pkv, NEW_V), *prev = PyTuple_GET_ITEM(pkv, 38);
+  PyObject *nk = PyTuple_GET_ITEM(pkv, NEW_K), *nv = PyTuple_GET_ITEM(pkv, NEW_V), *prev = PyTuple_GET_ITEM(pkv, RANGES);
   if (!is_tensor(nk) || !is_tensor(nv)) Py_RETURN_NONE;
   const Tensor &newK = ten(nk), &newV = ten(nv), &scores_k = ten(a[3]), &imp = ten(a[4]);
   if (!newV.is_cuda() || newV.dim() != 4) Py_RETURN_NONE;
@@ -969,7 +1000,7 @@ PyObject *compress(PyObject *, PyObject *const *a, Py_ssize_t na) {
       !new_tokens(newV, false, B, H, length, D, dev, vs.src[5]) || !old_side(pkv, true, low_normal, B, H, D, dev, ks) ||
       !old_side(pkv, false, low_normal, B, H, D, dev, vs) || ks.n_blocks != history / 32 || vs.n_blocks != history / 32)
     Py_RETURN_NONE;
-  if ((uintptr_t)newV.data_ptr() % 16) Py_RETURN_NONE;
+  if (((uintptr_t)newV.data_ptr() | (uintptr_t)newK.data_ptr()) % 16) Py_RETURN_NONE;
   for (const int64_t *c : {kc, vc}) {   // what the planner will ask for
     int64_t sum = 0;
     for (int i = 0; i < 6; ++i) {
@@ -978,38 +1009,56 @@ PyObject *compress(PyObject *, PyObject *const *a, Py_ssize_t na) {
     }
     if (sum != total) Py_RETURN_NONE;
   }
+  hqekv_migrate_extra x{};
+  Tensor ring;
+  if (a[10] != Py_None) {
+    if (!is_tensor(a[10])) Py_RETURN_NONE;
+    ring = ten(a[10]);
+    if (!plain_f16(ring, 2, dev) || ring.size(1) < total || ring.size(0) > 65535) Py_RETURN_NONE;
+  }
+  const int64_t rk = newK.size(2) - length, rv = newV.size(2) - length;
+  if (rk != rv) Py_RETURN_NONE;
+  Tensor resK, resV;
+  if (rk) {
+    if (a[11] != Py_None) {
+      if (!PyTuple_Check(a[11]) || PyTuple_GET_SIZE(a[11]) != 2 || !is_tensor(PyTuple_GET_ITEM(a[11], 0)) || !is_tensor(PyTuple_GET_ITEM(a[11], 1))) Py_RETURN_NONE;
+      resK = ten(PyTuple_GET_ITEM(a[11], 0));
+      resV = ten(PyTuple_GET_ITEM(a[11], 1));
+      for (const Tensor *t : {&resK, &resV})
+        if (!plain_f16(*t, 4, dev) || t->size(0) != B || t->size(1) != H || t->size(2) < rk || t->size(3) != D) Py_RETURN_NONE;
+    } else {
+      resK = new_tensor({B, H, rk, D}, at::kHalf, dev);
+      resV = new_tensor({B, H, rv, D}, at::kHalf, dev);
+    }
+  }
   const c10::OptionalDeviceGuard guard(dev);
   void *stream = stream_of(dev);
-  // ---- token ranges of V: the older ones and the new tokens'
+  // ---- token ranges of V -- the older ones and the new tokens' -- and the scores of the V side's blocks
   Tensor range;
+  const Tensor scores_v = new_tensor({nb}, at::kHalf, dev);
   int rc = 0;
   if (a[6] != Py_None) {
     if (!is_tensor(a[6])) Py_RETURN_NONE;
     range = ten(a[6]);
     if (!plain_f16(range, 1, dev) || range.numel() != total) Py_RETURN_NONE;
-  } else if (prev == Py_None) {
-    if (history) Py_RETURN_NONE;
-    range = new_tensor({length}, at::kHalf, dev);
-    rc = api.hqekv_token_range(newV.data_ptr(), B, H, length, D, vs.src[5].slab_tokens, range.data_ptr(), stream);
+    rc = api.hqekv_weighted_block_scores(imp.data_ptr(), times_range ? range.data_ptr() : nullptr, total, scores_v.data_ptr(), stream);
   } else {
-    if (!is_tensor(prev) || !plain_f16(ten(prev), 1, dev) || ten(prev).numel() != history) Py_RETURN_NONE;
+    if (prev == Py_None ? history != 0 : (!is_tensor(prev) || !plain_f16(ten(prev), 1, dev) || ten(prev).numel() != history)) Py_RETURN_NONE;
     range = new_tensor({total}, at::kHalf, dev);
-    rc = api.hqekv_token_range_append(newV.data_ptr(), B, H, length, D, vs.src[5].slab_tokens, ten(prev).data_ptr(), history, range.data_ptr(), stream);
+    rc = api.hqekv_range_block_scores(newV.data_ptr(), B, H, length, D, vs.src[5].slab_tokens, history ? ten(prev).data_ptr() : nullptr, history,
+                                      imp.data_ptr(), times_range ? 1 : 0, range.data_ptr(), scores_v.data_ptr(), stream);
   }
-  if (rc) return raise_rc(rc, "token_range");
+  if (rc) return raise_rc(rc, "range_block_scores");
   // ---- both rankings
-  const Tensor scores_v = new_tensor({nb}, at::kHalf, dev);
-  rc = api.hqekv_weighted_block_scores(imp.data_ptr(), times_range ? range.data_ptr() : nullptr, total, scores_v.data_ptr(), stream);
-  if (rc) return raise_rc(rc, "weighted_block_scores");
-  const Tensor order = at::empty({2 * nb}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+  const Tensor host = at::empty({2 * nb + 5 * nb + 4}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
   const void *const sc[2] = {scores_k.data_ptr(), scores_v.data_ptr()};
-  if (!host_orders(sc, nb, order, dev)) return nullptr;
-  // ---- the plans of both sides, one transfer for them and for the positions that survive on the V side
+  const Tensor up_d = new_tensor({5 * nb}, at::kInt, dev);   // (made while the ranking runs)
+  if (!host_orders(sc, nb, host, dev)) return nullptr;
+  // ---- the plans of both sides and the V side's surviving blocks, one transfer for all
+  const int32_t *order = (const int32_t *)host.data_ptr();
+  int32_t *words = (int32_t *)host.data_ptr() + up(2 * nb, 4), counts[2][5], n_alive[2] = {0, 0};
   std::vector<int64_t> order64(nb);
-  std::vector<int32_t> alive(nb);
-  Tensor up_h = at::empty({2 * nb + total}, at::TensorOptions().dtype(at::kLong).pinned_memory(true));
-  int32_t *words = (int32_t *)up_h.data_ptr(), counts[2][5];
-  int32_t n_alive[2] = {0, 0};
+  std::vector<int32_t> alive_k(nb);
   for (int side = 0; side < 2; ++side) {
     OldSide &o = side ? vs : ks;
     const int32_t *old[5];
@@ -1018,31 +1067,58 @@ PyObject *compress(PyObject *, PyObject *const *a, Py_ssize_t na) {
       old[c] = o.blocks[c].data();
       cnt[c] = (int32_t)o.blocks[c].size();
     }
-    for (int64_t i = 0; i < nb; ++i) order64[i] = ((const int32_t *)order.data_ptr())[side * nb + i];
+    for (int64_t i = 0; i < nb; ++i) order64[i] = order[side * nb + i];
     rc = api.hqekv_plan_side(old, cnt, (int32_t)(history / 32), (int32_t)(length / 32), order64.data(), side ? vc : kc, side ? n_v : n_k, counts[side],
-                             words + side * 2 * nb, alive.data(), &n_alive[side]);
+                             words + side * 2 * nb, side ? words + 4 * nb : alive_k.data(), &n_alive[side]);
     if (rc) Py_RETURN_NONE;   // not a whole-block selection after all
   }
   const bool evicted = n_alive[1] < nb;
-  int64_t n_up = 2 * nb;
+  rc = api.hqekv_fetch_words(words, up_d.data_ptr(), evicted ? 4 * nb + n_alive[1] : 4 * nb, stream);
+  if (rc) return raise_rc(rc, "fetch_words");
+  at::getHostAllocator(at::kCUDA)->record_event(host.data_ptr(), host.storage().data_ptr().get_context(),
+                                                c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(dev.index()).unwrap());
+  // ---- the launch that moves everything
+  NewSide k_new, v_new;
+  new_side(true, low_normal, counts[0], B, H, D, dev, k_new);
+  new_side(false, low_normal, counts[1], B, H, D, dev, v_new);
+  const int32_t *plan = (const int32_t *)up_d.data_ptr();
+  Tensor kept_range = range;
   if (evicted) {
-    int64_t *keep = (int64_t *)up_h.data_ptr() + n_up;
-    for (int32_t i = 0; i < n_alive[1]; ++i)
-      for (int j = 0; j < 32; ++j) *keep++ = (int64_t)alive[i] * 32 + j;
-    n_up += (int64_t)n_alive[1] * 32;
+    const int32_t *alive = words + 4 * nb;
+    x.alive = plan + 4 * nb;
+    x.n_alive = n_alive[1];
+    while (x.first_moved < x.n_alive && alive[x.first_moved] == x.first_moved) ++x.first_moved;
+    if (ring.defined()) {
+      x.ring = ring.data_ptr();
+      x.ring_rows = (int32_t)ring.size(0);
+      x.ring_stride = ring.size(1);
+    }
+    kept_range = new_tensor({32 * (int64_t)n_alive[1]}, at::kHalf, dev);
+    x.range_in = range.data_ptr();
+    x.range_out = kept_range.data_ptr();
   }
-  const Tensor up_d = new_tensor({n_up}, at::kLong, dev);
-  up_d.copy_(part_of(up_h, {n_up}, 0), /*non_blocking=*/true);
-  // ---- the new tuple
+  if (rk) {
+    const Tensor *src[2] = {&newK, &newV}, *dst[2] = {&resK, &resV};
+    x.res_rows = (int32_t)rk;
+    for (int side = 0; side < 2; ++side) {
+      x.res_src[side] = (const char *)src[side]->data_ptr() + 2 * D * length;
+      x.res_src_slab[side] = (side ? vs : ks).src[5].slab_tokens;
+      x.res_dst[side] = dst[side]->data_ptr();
+      x.res_dst_slab[side] = dst[side]->size(2);
+    }
+  }
+  rc = api.hqekv_cache_migrate_both(ks.src, 6, k_new.dst, k_new.n_dst, plan, vs.src, 6, v_new.dst, v_new.n_dst, plan + 2 * nb, B * H, D, &x, stream);
+  if (rc) return raise_rc(rc, "cache_migrate");
+  // ---- the new tuple, while it runs
   PyObject *out = PyTuple_New(TUPLE_LEN);
   if (!out) return nullptr;
   for (int i = 0; i < TUPLE_LEN; ++i) {
-    PyObject *x = (i < 36 || i == NEW_K || i == NEW_V) ? Py_None : PyTuple_GET_ITEM(pkv, i);
-    Py_INCREF(x);
-    PyTuple_SET_ITEM(out, i, x);
+    PyObject *o = (i < 36 || i == RANGES || i == NEW_K || i == NEW_V) ? Py_None : PyTuple_GET_ITEM(pkv, i);
+    Py_INCREF(o);
+    PyTuple_SET_ITEM(out, i, o);
   }
   for (int side = 0; side < 2; ++side) {
-    PyObject *pos = PyObject_CallFunction(a[10], "L", (long long)n_alive[side]);
+    PyObject *pos = PyObject_CallFunction(a[12], "L", (long long)n_alive[side]);
     Py_buffer b;
     if (!pos || PyObject_GetBuffer(pos, &b, PyBUF_WRITABLE | PyBUF_C_CONTIGUOUS) != 0) {
       Py_XDECREF(pos);
@@ -1053,7 +1129,7 @@ PyObject *compress(PyObject *, PyObject *const *a, Py_ssize_t na) {
     const bool room = b.len == 8 * (Py_ssize_t)n_alive[side];
     for (int32_t i = 0; room && i < n_alive[side]; ++i) ((int64_t *)b.buf)[i] = w[n_alive[side] + i];
     PyBuffer_Release(&b);
-    const bool ok = room && new_side(out, side == 0, low_normal, side ? vs : ks, counts[side], (const int32_t *)up_d.data_ptr() + side * 2 * nb, pos, B, H, D, dev);
+    const bool ok = room && put_side(out, side == 0, side ? v_new : k_new, counts[side], n_alive[side], pos, a[13]);
     Py_DECREF(pos);
     if (!ok) {
       if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "new_array");
@@ -1061,21 +1137,17 @@ PyObject *compress(PyObject *, PyObject *const *a, Py_ssize_t na) {
       return nullptr;
     }
   }
-  auto put = [&](int i, PyObject *v) {
-    PyObject *old = PyTuple_GET_ITEM(out, i);
-    PyTuple_SET_ITEM(out, i, v);
-    Py_XDECREF(old);
-  };
-  Tensor keep;
-  if (evicted) {
-    keep = part_of(up_d, {n_up - 2 * nb}, 2 * nb);
-    range = at::index_select(range, 0, keep);
+  put_item(out, RANGES, THPVariable_Wrap(kept_range));
+  if (rk) {
+    put_item(out, NEW_K, THPVariable_Wrap(resK.size(2) > rk ? resK.slice(2, 0, rk) : resK));
+    put_item(out, NEW_V, THPVariable_Wrap(resV.size(2) > rk ? resV.slice(2, 0, rk) : resV));
   }
-  put(38, THPVariable_Wrap(range));
-  if (newK.size(2) > length) put(NEW_K, THPVariable_Wrap(newK.slice(2, length).clone(at::MemoryFormat::Contiguous)));
-  if (newV.size(2) > length) put(NEW_V, THPVariable_Wrap(newV.slice(2, length).clone(at::MemoryFormat::Contiguous)));
-  if (evicted) return Py_BuildValue("NN", out, THPVariable_Wrap(keep));
-  return Py_BuildValue("NO", out, Py_None);
+  if (!evicted || ring.defined()) return Py_BuildValue("NO", out, Py_None);
+  Tensor keep = at::empty({32 * (int64_t)n_alive[1]}, at::TensorOptions().dtype(at::kLong));
+  int64_t *p = (int64_t *)keep.data_ptr();
+  for (int32_t i = 0; i < n_alive[1]; ++i)
+    for (int j = 0; j < 32; ++j) *p++ = (int64_t)words[4 * nb + i] * 32 + j;
+  return Py_BuildValue("NN", out, THPVariable_Wrap(keep.to(dev)));
   END_HANDLE_TH_ERRORS
 }
 

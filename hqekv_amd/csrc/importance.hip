@@ -110,23 +110,35 @@ __global__ __launch_bounds__(IMP_THREADS) void token_range_kernel(const half_t *
   }
 }
 
-// The same for rows of whole 16-byte pieces: 16 lanes per (token, slab) row, 16 tokens per workgroup, so a token's rows
+__device__ __forceinline__ void block_score(half_t x, half_t w, bool weighted, half_t *score) {
+  const half_t t = weighted ? (half_t)((float)x * (float)w) : x;
+  const float v = tree_sum_32((float)(half_t)((float)t * 0.03125f));
+  if ((threadIdx.x & 31) == 0) *score = (half_t)v;
+}
+
+// The same for rows of whole 16-byte pieces: 16 lanes per (token, slab) row, 32 tokens per workgroup, so a token's rows
 // are a handful of independent 16-byte loads per lane and a reduction stays inside a row of 16 lanes (four DPP steps).
 // Bound by latency at 32 tokens (the later compressions: 8.0 us as one workgroup per token with 2-byte loads and trips
 // through the LDS crossbar; 4.9 us now) and by HBM at a whole prompt's.  Workgroups past the tokens copy the `n_prev` older
-// ranges that the new ones follow.
-constexpr int RANGE_TOK = 16;
-__global__ __launch_bounds__(IMP_THREADS) void token_range_rows_kernel(const half_t *__restrict__ v, int B, int H, int64_t T,
-                                                                      int D, int64_t slab_tokens, half_t *__restrict__ out,
-                                                                      const half_t *__restrict__ prev, int64_t n_prev,
-                                                                      int token_blocks) {
+// ranges that the new ones follow.  With `x`, the scores of the blocks go with them (T and n_prev are multiples of 32 then):
+// one launch for two of 4.0 and 2.3 us.
+constexpr int RANGE_TOK = 32, RANGE_THREADS = 16 * RANGE_TOK;
+__global__ __launch_bounds__(RANGE_THREADS) void token_range_rows_kernel(const half_t *__restrict__ v, int B, int H, int64_t T,
+                                                                        int D, int64_t slab_tokens, half_t *__restrict__ out,
+                                                                        const half_t *__restrict__ prev, int64_t n_prev,
+                                                                        int token_blocks, const half_t *__restrict__ x, int weighted,
+                                                                        half_t *__restrict__ scores) {
   if ((int)blockIdx.x >= token_blocks) {
     half_t *dst = out - n_prev;
-    for (int64_t i = ((int64_t)blockIdx.x - token_blocks) * IMP_THREADS + threadIdx.x; i < n_prev; i += ((int64_t)gridDim.x - token_blocks) * IMP_THREADS)
-      dst[i] = prev[i];
+    for (int64_t i = ((int64_t)blockIdx.x - token_blocks) * RANGE_THREADS + threadIdx.x; i < n_prev; i += ((int64_t)gridDim.x - token_blocks) * RANGE_THREADS) {
+      const half_t r = prev[i];
+      dst[i] = r;
+      if (x) block_score(x[i], r, weighted, scores + (i >> 5));   // (whole groups of 32 lanes come this far)
+    }
     return;
   }
-  __shared__ half_t r[RANGE_MAX_ROWS][RANGE_TOK];
+  extern __shared__ half_t range_rows[];   // B * H rows of RANGE_TOK
+  half_t (*r)[RANGE_TOK] = reinterpret_cast<half_t (*)[RANGE_TOK]>(range_rows);
   const int cp = threadIdx.x & 15, tl = threadIdx.x >> 4;
   const int64_t t = (int64_t)blockIdx.x * RANGE_TOK + tl, tc = t < T ? t : T - 1;
   const int rows = B * H;
@@ -176,6 +188,7 @@ __global__ __launch_bounds__(IMP_THREADS) void token_range_rows_kernel(const hal
       return (float)(half_t)sum_rows_like_torch(B, [&](int b) { return (float)r[b * H + h][threadIdx.x]; });
     });
     out[to] = (half_t)s;
+    if (x) block_score(x[n_prev + to], (half_t)s, weighted, scores + ((n_prev + to) >> 5));
   }
 }
 
@@ -246,8 +259,8 @@ extern "C" int hqekv_weighted_block_scores(const void *x, const void *weights, i
   return check_launch("weighted_block_scores");
 }
 
-extern "C" int hqekv_token_range_append(const void *v, int64_t B, int64_t H, int64_t T, int64_t D, int64_t slab_tokens,
-                                        const void *prev, int64_t n_prev, void *out, void *stream) {
+static int range_launch(const void *v, int64_t B, int64_t H, int64_t T, int64_t D, int64_t slab_tokens, const void *prev, int64_t n_prev,
+                        void *out, const void *x, int weighted, void *scores, void *stream) {
   if (n_prev < 0 || (n_prev > 0 && !prev)) return fail(HQEKV_E_ARG, "token_range: bad older ranges");
   if (!v || !out) return fail(HQEKV_E_ARG, "token_range: null pointer");
   if (B <= 0 || H <= 0 || T <= 0 || D <= 0 || slab_tokens < T)
@@ -256,15 +269,28 @@ extern "C" int hqekv_token_range_append(const void *v, int64_t B, int64_t H, int
   if (T > 0x7fffffffLL || D > 0x7fffffffLL) return fail(HQEKV_E_UNSUPPORTED, "token_range: T or D too large");
   if (D % 8 == 0 && ((uintptr_t)v & 15) == 0) {
     const int token_blocks = (int)((T + RANGE_TOK - 1) / RANGE_TOK);
-    const int64_t copy_blocks = n_prev > 0 ? std::min<int64_t>((n_prev + 4 * IMP_THREADS - 1) / (4 * IMP_THREADS), 1024) : 0;
-    hipLaunchKernelGGL(token_range_rows_kernel, dim3((unsigned)(token_blocks + copy_blocks)), dim3(IMP_THREADS), 0, (hipStream_t)stream,
-                       (const half_t *)v, (int)B, (int)H, T, (int)D, slab_tokens, (half_t *)out + n_prev, (const half_t *)prev, n_prev, token_blocks);
+    const int64_t copy_blocks = std::min<int64_t>((n_prev + RANGE_THREADS - 1) / RANGE_THREADS, 1024);
+    hipLaunchKernelGGL(token_range_rows_kernel, dim3((unsigned)(token_blocks + copy_blocks)), dim3(RANGE_THREADS),
+                       (size_t)(B * H * RANGE_TOK) * sizeof(half_t), (hipStream_t)stream, (const half_t *)v, (int)B, (int)H, T, (int)D, slab_tokens,
+                       (half_t *)out + n_prev, (const half_t *)prev, n_prev, token_blocks, (const half_t *)x, weighted, (half_t *)scores);
     return check_launch("token_range");
   }
-  if (n_prev > 0) return fail(HQEKV_E_UNSUPPORTED, "token_range_append: rows of 16-byte aligned pieces only");
+  if (n_prev > 0 || x) return fail(HQEKV_E_UNSUPPORTED, "token_range_append: rows of 16-byte aligned pieces only");
   hipLaunchKernelGGL(token_range_kernel, dim3((unsigned)T), dim3(IMP_THREADS), 0, (hipStream_t)stream, (const half_t *)v,
                      (int)B, (int)H, T, (int)D, slab_tokens, (half_t *)out);
   return check_launch("token_range");
+}
+
+extern "C" int hqekv_token_range_append(const void *v, int64_t B, int64_t H, int64_t T, int64_t D, int64_t slab_tokens,
+                                        const void *prev, int64_t n_prev, void *out, void *stream) {
+  return range_launch(v, B, H, T, D, slab_tokens, prev, n_prev, out, nullptr, 0, nullptr, stream);
+}
+
+extern "C" int hqekv_range_block_scores(const void *v, int64_t B, int64_t H, int64_t T, int64_t D, int64_t slab_tokens, const void *prev,
+                                        int64_t n_prev, const void *x, int weighted, void *range_out, void *scores_out, void *stream) {
+  if (!x || !scores_out) return fail(HQEKV_E_ARG, "range_block_scores: null pointer");
+  if (T % 32 || n_prev % 32) return fail(HQEKV_E_ARG, "range_block_scores: whole blocks of 32 tokens only");
+  return range_launch(v, B, H, T, D, slab_tokens, prev, n_prev, range_out, x, weighted, scores_out, stream);
 }
 
 extern "C" int hqekv_token_range(const void *v, int64_t B, int64_t H, int64_t T, int64_t D, int64_t slab_tokens,

@@ -1,4 +1,4 @@
-// Cache maintenance on the device: one launch rebuilds every precision class of one side (K or V) of a layer's
+// Cache maintenance on the device: one launch rebuilds every precision class of both sides (K and V) of a layer's
 // cache from the old classes and the new fp16 tokens, following a block-level plan the host worked out.
 //
 // What the reference does per compression (quant/hqe_2.py:552-836) is a sequence of boolean-mask gathers,
@@ -14,6 +14,8 @@
 //   fp16 -> fp16          copy (new K arrives token-major and is stored channel-major)
 // Evicted blocks are simply in nobody's plan.  The arithmetic is the one of the stand-alone kernels (quant_math.h),
 // so the bytes equal those of the step-by-step path.
+#include <stddef.h>
+
 #include "common.h"
 #include "quant_math.h"
 
@@ -30,27 +32,36 @@ struct MigClass {
   int64_t slab_tokens;  // tokens between (b, h) slabs of a token-major fp16 source (>= n_tokens)
   int32_t bits;
   int32_t layout;
+  int32_t begin;        // destination: its first plan entry
+  int32_t pad;
 };
 
-struct MigArgs {
+struct MigSide {
   MigClass src[HQEKV_MAX_SEGS];
   MigClass dst[HQEKV_MAX_SEGS];
   int32_t dst_begin[HQEKV_MAX_SEGS + 1];  // first plan entry of every destination class; [n_dst] = total
   int32_t n_dst;
   int32_t n_src;
+  int32_t wgs;              // workgroups that serve the side
   const int32_t *plan_src;  // (source slot << 24) | source block, per destination block
   const int32_t *plan_pos;  // new position of the block's first token / 32
-  int32_t *status;          // optional: set to non-zero when a plan entry is refused
+};
+
+struct MigArgs {
+  MigSide side[2];   // K, V
+  hqekv_migrate_extra x;
+  int32_t *status;   // optional: set to non-zero when a plan entry is refused
+  int32_t BH, D;
 };
 
 // The plan lives in device memory and is read by the kernel only, so the kernel is what checks it: an entry must name
 // a populated source class, a block inside it and a position inside the new sequence.  An entry that does not is
 // skipped (its destination block keeps whatever the buffer held) and flagged; nothing is read or written out of range.
-__device__ __forceinline__ bool plan_entry_ok(const MigArgs &a, int32_t code, int32_t pos, int total) {
+__device__ __forceinline__ bool plan_entry_ok(const MigClass *src, int n_src, int32_t code, int32_t pos, int total) {
   const uint32_t slot = (uint32_t)code >> 24, blk = (uint32_t)code & 0xffffffu;
-  if (slot >= (uint32_t)a.n_src) return false;
-  const int64_t n = a.src[slot].n_tokens;
-  return n > 0 && a.src[slot].data != nullptr && (int64_t)blk < (n >> 5) && pos >= 0 && pos < total;
+  if (slot >= (uint32_t)n_src) return false;
+  const int64_t n = src[slot].n_tokens;
+  return n > 0 && src[slot].data != nullptr && (int64_t)blk < (n >> 5) && pos >= 0 && pos < total;
 }
 __device__ __forceinline__ void plan_refused(const MigArgs &a) {
   if (a.status) atomicOr(a.status, 1);
@@ -218,172 +229,297 @@ __device__ __forceinline__ void quantize_to(const MigClass &dc, const GroupRef &
   }
 }
 
-// the packed words, scale and zero of one group; a group's words start at a multiple of their own size, so they move as
-// vectors where the planes are 16-byte aligned (uniform; every plane this package allocates is)
-template <int BITS>
-__device__ __forceinline__ void copy_group(const GroupRef &sr, const GroupRef &dr) {
-  const half_t s = *sr.s, z = *sr.z;
-  uint32_t w[BITS];
+// The packed words, scale and zero of N groups, all requested before the first is stored; a group's words start at a
+// multiple of their own size, so they move as vectors where the planes are 16-byte aligned (every plane this package
+// allocates is).
+template <int BITS, int N>
+__device__ __forceinline__ void copy_groups(const GroupRef (&sr)[N], const GroupRef (&dr)[N]) {
   constexpr int V = BITS < 4 ? BITS : 4;
   typedef uint32_t vec_t __attribute__((ext_vector_type(V)));
-  const bool vec = (((uintptr_t)sr.words | (uintptr_t)dr.words) & (4 * V - 1)) == 0;
-  if (vec) {
+  half_t s[N], z[N];
 #pragma unroll
-    for (int i = 0; i < BITS; i += V) __builtin_memcpy(w + i, __builtin_assume_aligned(sr.words + i, 4 * V), 4 * V);
-  } else {
-#pragma unroll
-    for (int i = 0; i < BITS; ++i) w[i] = sr.words[i];
+  for (int g = 0; g < N; ++g) {
+    s[g] = *sr[g].s;
+    z[g] = *sr[g].z;
   }
-  if (vec) {
+  if ((((uintptr_t)sr[0].words | (uintptr_t)dr[0].words) & (4 * V - 1)) == 0) {   // (the same for all groups of a class)
+    vec_t w[N][BITS / V];
 #pragma unroll
-    for (int i = 0; i < BITS; i += V) {
-      vec_t v;
-      __builtin_memcpy(&v, w + i, 4 * V);
-      *reinterpret_cast<vec_t *>(dr.words + i) = v;
-    }
+    for (int g = 0; g < N; ++g)
+#pragma unroll
+      for (int i = 0; i < BITS / V; ++i) w[g][i] = reinterpret_cast<const vec_t *>(sr[g].words)[i];
+#pragma unroll
+    for (int g = 0; g < N; ++g)
+#pragma unroll
+      for (int i = 0; i < BITS / V; ++i) reinterpret_cast<vec_t *>(dr[g].words)[i] = w[g][i];
   } else {
+    uint32_t w[N][BITS];
 #pragma unroll
-    for (int i = 0; i < BITS; ++i) dr.words[i] = w[i];
+    for (int g = 0; g < N; ++g)
+#pragma unroll
+      for (int i = 0; i < BITS; ++i) w[g][i] = sr[g].words[i];
+#pragma unroll
+    for (int g = 0; g < N; ++g)
+#pragma unroll
+      for (int i = 0; i < BITS; ++i) dr[g].words[i] = w[g][i];
   }
-  *dr.s = s;
-  *dr.z = z;
+#pragma unroll
+  for (int g = 0; g < N; ++g) {
+    *dr[g].s = s[g];
+    *dr[g].z = z[g];
+  }
 }
 
-// One quantisation group: lane = channel (K) or (token, channel group) (V) of source block sb -> destination block db.
-template <bool IS_K>
-__device__ __forceinline__ void migrate_group(const MigClass &sc, const MigClass &dc, int64_t bh, int64_t sb, int64_t db,
-                                              int lane, int D) {
-  const GroupRef sr = group_ref<IS_K>(sc, bh, sb, lane, D);
-  const GroupRef dr = group_ref<IS_K>(dc, bh, db, lane, D);
-  if (sc.bits != 16 && sc.bits == dc.bits) {  // a survivor of a quantised class keeps its bytes
-    switch (sc.bits) {
-      case 8: copy_group<8>(sr, dr); break;
-      case 4: copy_group<4>(sr, dr); break;
-      case 2: copy_group<2>(sr, dr); break;
-      default: copy_group<1>(sr, dr);
+// a survivor of a quantised class keeps its bytes
+template <int N>
+__device__ __forceinline__ void copy_groups_of(int bits, const GroupRef (&sr)[N], const GroupRef (&dr)[N]) {
+  switch (bits) {
+    case 8: copy_groups<8>(sr, dr); break;
+    case 4: copy_groups<4>(sr, dr); break;
+    case 2: copy_groups<2>(sr, dr); break;
+    default: copy_groups<1>(sr, dr);
+  }
+}
+
+// N quantisation groups: lane, lane + step, ... = channel (K) or (token, channel group) (V) of source block sb ->
+// destination block db.
+template <bool IS_K, int N>
+__device__ __forceinline__ void migrate_groups(const MigClass &sc, const MigClass &dc, int64_t bh, int64_t sb, int64_t db,
+                                               int lane, int step, int D) {
+  if (sc.bits != 16 && sc.bits == dc.bits) {
+    GroupRef sr[N], dr[N];
+#pragma unroll
+    for (int g = 0; g < N; ++g) {
+      sr[g] = group_ref<IS_K>(sc, bh, sb, lane + g * step, D);
+      dr[g] = group_ref<IS_K>(dc, bh, db, lane + g * step, D);
     }
+    copy_groups_of(sc.bits, sr, dr);
     return;
   }
-  uint32_t xp[16];
   const bool sn = sc.layout == HQEKV_LAYOUT_NORMAL1;
-  switch (sc.bits) {
-    case 16: load_f16(sr, xp); break;
-    case 8: dequant_group<8, false>(sr, xp); break;
-    case 4: dequant_group<4, false>(sr, xp); break;
-    case 2: dequant_group<2, false>(sr, xp); break;
-    default:
-      if (sn) dequant_group<1, true>(sr, xp);
-      else dequant_group<1, false>(sr, xp);
+#pragma unroll 1
+  for (int g = 0; g < N; ++g) {
+    const GroupRef s = group_ref<IS_K>(sc, bh, sb, lane + g * step, D), d = group_ref<IS_K>(dc, bh, db, lane + g * step, D);
+    uint32_t xp[16];
+    switch (sc.bits) {
+      case 16: load_f16(s, xp); break;
+      case 8: dequant_group<8, false>(s, xp); break;
+      case 4: dequant_group<4, false>(s, xp); break;
+      case 2: dequant_group<2, false>(s, xp); break;
+      default:
+        if (sn) dequant_group<1, true>(s, xp);
+        else dequant_group<1, false>(s, xp);
+    }
+    quantize_to(dc, d, xp);
   }
-  quantize_to(dc, dr, xp);
 }
 
-__device__ __forceinline__ int dst_class_of(const MigArgs &a, int u) {
+__device__ __forceinline__ int dst_class_of(const MigSide &a, int u) {
   int ci = 0;
 #pragma unroll
   for (int k = 1; k < HQEKV_MAX_SEGS; ++k) ci += (k < a.n_dst && u >= a.dst_begin[k]) ? 1 : 0;
   return ci;
 }
 
-constexpr int MIG_THREADS = 128;   // V side
+constexpr int MIG_THREADS = 256;
 constexpr int MIG_KB = 16;         // K side: destination blocks per workgroup
 constexpr int MIG_KC = 32;         // ... and channels
-constexpr int MIG_KTHREADS = 256;
+constexpr int MIG_VB = 4;          // V side: destination blocks per workgroup
+constexpr int MIG_XC = 16;         // columns of a ring row a thread moves at a time
+static_assert(MIG_KC == 2 * (MIG_THREADS / MIG_KB), "a lane of the K side holds two channels of a block");
 
-// 32 tokens of channels d and d + 1 of a token-major block: two groups from 32 four-byte loads
-__device__ __forceinline__ void load_token_major_pair(const MigClass &c, int64_t bh, int64_t block, int d, int D, uint32_t (&xa)[16], uint32_t (&xb)[16]) {
-  const uint32_t *p = reinterpret_cast<const uint32_t *>((const half_t *)c.data + (bh * c.slab_tokens + block * 32) * D + d);
-  uint32_t w[32];
-#pragma unroll
-  for (int i = 0; i < 32; ++i) w[i] = p[(int64_t)i * (D >> 1)];
-#pragma unroll
-  for (int j = 0; j < 16; ++j) {
-    xa[j] = __builtin_amdgcn_perm(w[2 * j + 1], w[2 * j], 0x05040100u);
-    xb[j] = __builtin_amdgcn_perm(w[2 * j + 1], w[2 * j], 0x07060302u);
-  }
+// The side's class tables in LDS: a lane's classes follow from its plan entry, and tables in the argument block would be
+// a second trip to memory behind that of the entry.
+struct MigTables {
+  MigClass src[HQEKV_MAX_SEGS], dst[HQEKV_MAX_SEGS];
+};
+__device__ __forceinline__ void fetch_tables(const MigSide &a, MigTables &t) {
+  static_assert(offsetof(MigSide, src) == 0 && offsetof(MigSide, dst) == sizeof(MigClass) * HQEKV_MAX_SEGS && sizeof(MigTables) % 4 == 0 &&
+                    sizeof(MigTables) / 4 <= MIG_THREADS, "one word per thread");
+  if (threadIdx.x < sizeof(MigTables) / 4) reinterpret_cast<uint32_t *>(&t)[threadIdx.x] = reinterpret_cast<const uint32_t *>(&a)[threadIdx.x];
 }
 
-// V side: a workgroup per destination block; its 32 tokens x D/32 groups are one contiguous stretch of every plane.
-// K side: a group is 32 tokens of ONE channel row -- b words of the row -- and a block's groups lie a whole row
+// K side.  A group is 32 tokens of ONE channel row -- b words of the row -- and a block's groups lie a whole row
 // apart, so a workgroup takes 16 consecutive destination blocks and lets neighbouring lanes take neighbouring
 // blocks of a row: 16 b-word pieces side by side (64 bytes at 1 bit ... 512 at 8), and as long as the blocks come
 // from consecutive places of one source class (survivors of a class stay in order) the reads line up the same
-// way.  (A lane per channel, as on the V side, touched a separate cache line per lane: the K launch took four to
-// six times as long as the V launch for the same bytes.)  A workgroup covers 32 channels, so that a side of a thousand
-// blocks is some thousands of short workgroups; with all 128 channels in one workgroup of two waves, and its blocks of new
-// tokens (token-major: the channels of a token are what is contiguous) walked one after the other, the chip was nearly
-// idle: 50 us for 19 MB in and out at 32k tokens, 47 us for a 4k prompt of new tokens.  Those blocks now go side by side
-// as well, a lane holding two channels of one: 22 us and 13 us (V at 32k tokens 16.5 -> 13.4 us with vector copies).
-template <bool IS_K>
-__global__ __launch_bounds__(IS_K ? MIG_KTHREADS : MIG_THREADS) void cache_migrate_kernel(MigArgs a, int D) {
-  const int64_t bh = blockIdx.y;
-  const int total = a.dst_begin[HQEKV_MAX_SEGS];
-  if constexpr (!IS_K) {
-    const int u = blockIdx.x;
-    const MigClass dc = a.dst[dst_class_of(a, u)];
-    const int64_t db = u - a.dst_begin[dst_class_of(a, u)];
-    const int32_t code = a.plan_src[u];
-    if (!plan_entry_ok(a, code, a.plan_pos[u], total)) {   // uniform: the whole workgroup serves this entry
-      if (threadIdx.x == 0) plan_refused(a);
-      return;
-    }
-    if (bh == 0 && threadIdx.x < 32 && dc.idx) dc.idx[db * 32 + threadIdx.x] = (int64_t)a.plan_pos[u] * 32 + threadIdx.x;
-    for (int lane = threadIdx.x; lane < D; lane += MIG_THREADS)
-      migrate_group<false>(a.src[code >> 24], dc, bh, code & 0xffffff, db, lane, D);
-  } else {
-    const int u0 = blockIdx.x * MIG_KB, d0 = blockIdx.z * MIG_KC;
-    if (bh == 0 && d0 == 0) {  // positions of the blocks' tokens
-      for (int e = threadIdx.x; e < MIG_KB * 32; e += MIG_KTHREADS) {
-        const int ue = u0 + e / 32;
-        if (ue < total && plan_entry_ok(a, a.plan_src[ue], a.plan_pos[ue], total)) {
-          const int ce = dst_class_of(a, ue);
-          int64_t *idx = a.dst[ce].idx;
-          if (idx) idx[(int64_t)(ue - a.dst_begin[ce]) * 32 + e % 32] = (int64_t)a.plan_pos[ue] * 32 + e % 32;
-        }
-      }
-    }
-    // the block of thread `slot` (of the 16): its plan entry, its classes
-    auto block_of = [&](int slot, int &ci, int32_t &code, bool &token_major) -> bool {
-      const int u = u0 + slot;
-      if (u >= total) return false;
-      code = a.plan_src[u];
-      if (!plan_entry_ok(a, code, a.plan_pos[u], total)) {
-        plan_refused(a);
-        return false;
-      }
-      ci = dst_class_of(a, u);
-      const MigClass &sc = a.src[(uint32_t)code >> 24];
-      token_major = sc.bits == 16 && sc.layout == HQEKV_LAYOUT_TOKEN_MAJOR;
-      return true;
-    };
-    int ci = 0;
-    int32_t code = 0;
-    bool tm = false;
-    const int slot = threadIdx.x % MIG_KB;
-    const bool live = block_of(slot, ci, code, tm);
-    if (live && !tm) {
-      const MigClass sc = a.src[(uint32_t)code >> 24], dc = a.dst[ci];
-      for (int d = d0 + threadIdx.x / MIG_KB; d < d0 + MIG_KC; d += MIG_KTHREADS / MIG_KB)   // (D is a multiple of 32)
-        migrate_group<true>(sc, dc, bh, code & 0xffffff, u0 + slot - a.dst_begin[ci], d, D);
-    }
-    if (!__syncthreads_or(live && tm)) return;
-    // blocks of new tokens: 16 blocks x 16 channel pairs, eight neighbouring lanes on neighbouring pairs (32 bytes of a
-    // token row), the next eight on the next block
-    const int tslot = threadIdx.x / 8 % MIG_KB, pair = threadIdx.x % 8 + threadIdx.x / (8 * MIG_KB) * 8;
-    static_assert(MIG_KTHREADS == MIG_KB * MIG_KC / 2, "one channel pair of one block per thread");
-    if (!block_of(tslot, ci, code, tm) || !tm) return;
-    const MigClass sc = a.src[(uint32_t)code >> 24], dc = a.dst[ci];
-    uint32_t xp[2][16];
-    load_token_major_pair(sc, bh, code & 0xffffff, d0 + 2 * pair, D, xp[0], xp[1]);
-#pragma unroll 1
-    for (int e = 0; e < 2; ++e) {
-      const GroupRef dr = group_ref<true>(dc, bh, u0 + tslot - a.dst_begin[ci], d0 + 2 * pair + e, D);
-      uint32_t x[16];
-#pragma unroll
-      for (int j = 0; j < 16; ++j) x[j] = e ? xp[1][j] : xp[0][j];
-      quantize_to(dc, dr, x);
-    }
+// way.  (A lane per channel, as on the V side, touched a separate cache line per lane: the K side took four to
+// six times as long as the V side for the same bytes.)  A workgroup covers 32 channels, so that a side of a thousand
+// blocks is some thousands of short workgroups.  Blocks of new tokens (token-major: the channels of a token are what is
+// contiguous) go side by side as well, a lane holding two channels of one.
+__device__ __forceinline__ void migrate_keys(const MigArgs &a, int wg, const MigTables &tab) {
+  const MigSide &s = a.side[0];
+  const int total = s.dst_begin[HQEKV_MAX_SEGS], D = a.D, groups = (total + MIG_KB - 1) / MIG_KB;
+  const int u0 = wg % groups * MIG_KB, d0 = wg / groups / a.BH * MIG_KC;
+  const int64_t bh = wg / groups % a.BH;
+  // thread -> block of the 16: `slot` for the class to class part, `tslot` for blocks of new tokens
+  const int slot = threadIdx.x % MIG_KB, tslot = threadIdx.x / 8 % MIG_KB;
+  const int u = u0 + slot, tu = u0 + tslot;
+  const int uc = min(u, total - 1), tuc = min(tu, total - 1);
+  const int32_t code = s.plan_src[uc], pos = s.plan_pos[uc], tcode = s.plan_src[tuc], tpos = s.plan_pos[tuc];
+  __syncthreads();   // the tables
+  auto token_major = [&](int32_t c) {
+    const MigClass &sc = tab.src[(uint32_t)c >> 24];
+    return sc.bits == 16 && sc.layout == HQEKV_LAYOUT_TOKEN_MAJOR;
+  };
+  const bool ok = u < total && plan_entry_ok(tab.src, s.n_src, code, pos, total);
+  if (u < total && !ok) plan_refused(a);
+  const int ci = dst_class_of(s, uc);
+  if (bh == 0 && d0 == 0 && ok && tab.dst[ci].idx) {   // positions of the blocks' tokens
+    int64_t *idx = tab.dst[ci].idx + (int64_t)(u - tab.dst[ci].begin) * 32;
+    for (int e = threadIdx.x / MIG_KB; e < 32; e += MIG_THREADS / MIG_KB) idx[e] = (int64_t)pos * 32 + e;
   }
+  const bool tm = ok && token_major(code);
+  if (ok && !tm)
+    migrate_groups<true, 2>(tab.src[(uint32_t)code >> 24], tab.dst[ci], bh, code & 0xffffff, u - tab.dst[ci].begin, d0 + threadIdx.x / MIG_KB,
+                            MIG_THREADS / MIG_KB, D);
+  if (!__syncthreads_or(tm)) return;
+  // blocks of new tokens: 16 blocks x 16 channel pairs, eight neighbouring lanes on neighbouring pairs (32 bytes of a
+  // token row), the next eight on the next block
+  const int pair = threadIdx.x % 8 + threadIdx.x / (8 * MIG_KB) * 8;
+  static_assert(MIG_THREADS == MIG_KB * MIG_KC / 2, "one channel pair of one block per thread");
+  if (tu >= total || !plan_entry_ok(tab.src, s.n_src, tcode, tpos, total) || !token_major(tcode)) return;
+  const int tci = dst_class_of(s, tu);
+  const MigClass &sc = tab.src[(uint32_t)tcode >> 24], &dc = tab.dst[tci];
+  // 32 tokens of channels d and d + 1: two groups from 32 four-byte loads
+  const uint32_t *p = reinterpret_cast<const uint32_t *>((const half_t *)sc.data + (bh * sc.slab_tokens + (tcode & 0xffffff) * 32LL) * D + d0 + 2 * pair);
+  uint32_t w[32];
+#pragma unroll
+  for (int i = 0; i < 32; ++i) w[i] = p[i * (D >> 1)];
+#pragma unroll 1
+  for (int e = 0; e < 2; ++e) {
+    const GroupRef dr = group_ref<true>(dc, bh, tu - dc.begin, d0 + 2 * pair + e, D);
+    const uint32_t halves = e ? 0x07060302u : 0x05040100u;   // which channel of every word
+    uint32_t x[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) x[j] = __builtin_amdgcn_perm(w[2 * j + 1], w[2 * j], halves);
+    quantize_to(dc, dr, x);
+  }
+}
+
+// V side: half a workgroup per two destination blocks; a block's 32 tokens x D/32 groups are one contiguous stretch of every
+// plane.  The two blocks are in flight together where both only move within one class.
+__device__ __forceinline__ void migrate_values(const MigArgs &a, int wg, const MigTables &tab) {
+  const MigSide &s = a.side[1];
+  const int total = s.dst_begin[HQEKV_MAX_SEGS], D = a.D, groups = (total + MIG_VB - 1) / MIG_VB;
+  const int64_t bh = wg / groups;
+  constexpr int LANES = 2 * MIG_THREADS / MIG_VB;
+  const int u0 = wg % groups * MIG_VB + threadIdx.x / LANES * 2, l0 = threadIdx.x % LANES;
+  int32_t code[2], pos[2];
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const int uc = min(u0 + k, total - 1);
+    code[k] = s.plan_src[uc];
+    pos[k] = s.plan_pos[uc];
+  }
+  __syncthreads();   // the tables
+  bool ok[2];
+  int ci[2];
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {   // uniform: the whole half serves these entries
+    ok[k] = u0 + k < total && plan_entry_ok(tab.src, s.n_src, code[k], pos[k], total);
+    if (u0 + k < total && !ok[k] && l0 == 0) plan_refused(a);
+    ci[k] = dst_class_of(s, min(u0 + k, total - 1));
+    int64_t *idx = tab.dst[ci[k]].idx;
+    if (ok[k] && bh == 0 && l0 < 32 && idx) idx[(int64_t)(u0 + k - tab.dst[ci[k]].begin) * 32 + l0] = (int64_t)pos[k] * 32 + l0;
+  }
+  const int bits = tab.dst[ci[0]].bits;
+  if (ok[0] && ok[1] && ci[0] == ci[1] && bits != 16 && tab.src[(uint32_t)code[0] >> 24].bits == bits && tab.src[(uint32_t)code[1] >> 24].bits == bits) {
+    for (int lane = l0; lane < D; lane += LANES) {
+      GroupRef sr[2], dr[2];
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        sr[k] = group_ref<false>(tab.src[(uint32_t)code[k] >> 24], bh, code[k] & 0xffffff, lane, D);
+        dr[k] = group_ref<false>(tab.dst[ci[k]], bh, u0 + k - tab.dst[ci[k]].begin, lane, D);
+      }
+      copy_groups_of(bits, sr, dr);
+    }
+    return;
+  }
+#pragma unroll 1
+  for (int k = 0; k < 2; ++k) {
+    const int32_t c = k ? code[1] : code[0];
+    const MigClass &dc = tab.dst[k ? ci[1] : ci[0]];
+    if (!(k ? ok[1] : ok[0])) continue;
+    for (int lane = l0; lane < D; lane += LANES)
+      migrate_groups<false, 1>(tab.src[(uint32_t)c >> 24], dc, bh, c & 0xffffff, u0 + k - dc.begin, lane, 0, D);
+  }
+}
+
+struct __attribute__((packed, aligned(2))) ring_quad_t { uint64_t v; };   // four fp16 columns at an element's alignment
+
+// What rides along: workgroup by workgroup the rows of the importance ring without the evicted columns, the token ranges
+// without them, and the residual rows that stay behind.
+__device__ __forceinline__ void migrate_extras(const MigArgs &a, int wg) {
+  const hqekv_migrate_extra &x = a.x;
+  if (wg < x.ring_rows) {
+    // In place, ascending: a column moves to the left or stays, so a pass overwrites nothing a later pass reads, and
+    // within a pass every thread holds its columns before the first is stored.
+    half_t *row = (half_t *)x.ring + (int64_t)wg * x.ring_stride;
+    const int n = x.n_alive * 32;
+    for (int c0 = x.first_moved * 32; c0 < n; c0 += MIG_THREADS * MIG_XC) {
+      const int c = c0 + threadIdx.x * MIG_XC;
+      ring_quad_t v[MIG_XC / 4];
+      if (c < n) {
+        const ring_quad_t *from = reinterpret_cast<const ring_quad_t *>(row + (int64_t)x.alive[c >> 5] * 32 + (c & 31));
+#pragma unroll
+        for (int i = 0; i < MIG_XC / 4; ++i) v[i] = from[i];
+      }
+      __syncthreads();
+      if (c < n) {
+        ring_quad_t *to = reinterpret_cast<ring_quad_t *>(row + c);
+#pragma unroll
+        for (int i = 0; i < MIG_XC / 4; ++i) to[i] = v[i];
+      }
+      __syncthreads();
+    }
+    return;
+  }
+  wg -= x.ring_rows;
+  const int range_wgs = x.range_out ? (x.n_alive * 32 + MIG_THREADS - 1) / MIG_THREADS : 0;
+  if (wg < range_wgs) {
+    const int c = wg * MIG_THREADS + threadIdx.x;
+    if (c < x.n_alive * 32) ((half_t *)x.range_out)[c] = ((const half_t *)x.range_in)[(int64_t)x.alive[c >> 5] * 32 + (c & 31)];
+    return;
+  }
+  wg -= range_wgs;
+  // 16-byte pieces of the residual rows of both sides
+  const int64_t per_slab = (int64_t)x.res_rows * a.D / 8, i = (int64_t)wg * MIG_THREADS + threadIdx.x;
+  if (i >= 2 * a.BH * per_slab) return;
+  const int side = i >= a.BH * per_slab ? 1 : 0;
+  const int64_t j = i - side * a.BH * per_slab, bh = j / per_slab, k = j % per_slab;
+  const uint4 *src = reinterpret_cast<const uint4 *>((const half_t *)x.res_src[side] + bh * x.res_src_slab[side] * a.D) + k;
+  reinterpret_cast<uint4 *>((half_t *)x.res_dst[side] + bh * x.res_dst_slab[side] * a.D)[k] = *src;
+}
+
+// Both sides of a layer in one launch, the K workgroups (the longer ones) first.  Bound by latency -- plan entry, group,
+// store, each a trip to memory -- at 35 MB in and 35 out at 32k tokens: 22 + 12 us as two launches, with the class tables in
+// the argument block and one group in flight per lane; 28 us as one launch of three waves per SIMD, 25 of four, 22.7 with
+// two V blocks in flight (a copy of those bytes takes 14).  4 waves per SIMD are what the 1-bit normal statistics leave.
+__global__ __launch_bounds__(MIG_THREADS, 4) void cache_migrate_kernel(MigArgs a) {
+  __shared__ MigTables tab;
+  int wg = blockIdx.x;
+  if (wg < a.side[0].wgs) {
+    fetch_tables(a.side[0], tab);
+    migrate_keys(a, wg, tab);
+    return;
+  }
+  wg -= a.side[0].wgs;
+  if (wg < a.side[1].wgs) {
+    fetch_tables(a.side[1], tab);
+    migrate_values(a, wg, tab);
+    return;
+  }
+  migrate_extras(a, wg - a.side[1].wgs);
+}
+
+// Words from page-locked memory: a launch of a few workgroups arrives sooner than a copy through the DMA engines, whose
+// completion another queue has to be told of.
+__global__ __launch_bounds__(256) void fetch_words_kernel(const uint32_t *__restrict__ src, uint32_t *__restrict__ dst, int n) {
+  const int i = (blockIdx.x * 256 + threadIdx.x) * 4;
+  if (i + 4 <= n) *reinterpret_cast<uint4 *>(dst + i) = *reinterpret_cast<const uint4 *>(src + i);
+  else
+    for (int k = i; k < n; ++k) dst[k] = src[k];
 }
 
 static int check_class(const hqekv_cache_class &c, bool is_src, int k, int64_t D) {
@@ -400,17 +536,11 @@ static int check_class(const hqekv_cache_class &c, bool is_src, int k, int64_t D
   return HQEKV_OK;
 }
 
-}  // namespace hq
-
-using namespace hq;
-
-extern "C" int hqekv_cache_migrate(int is_k, const hqekv_cache_class *src, int n_src, const hqekv_cache_class *dst,
-                                   int n_dst, const int32_t *plan, int64_t BH, int64_t D, int32_t *status, void *stream) {
+// One side's tables, checked.
+static int fill_side(bool is_k, const hqekv_cache_class *src, int n_src, const hqekv_cache_class *dst, int n_dst, const int32_t *plan,
+                     int64_t BH, int64_t D, MigSide *a) {
   if (n_src < 0 || n_src > HQEKV_MAX_SEGS || n_dst < 0 || n_dst > HQEKV_MAX_SEGS || (n_src && !src) || (n_dst && !dst))
     return fail(HQEKV_E_ARG, "cache_migrate: bad class tables");
-  if (BH <= 0 || BH > 65535 || D <= 0 || D % 32 != 0 || D > 1024)
-    return fail(HQEKV_E_ARG, "cache_migrate: need 0 < B*H <= 65535 and head_dim a multiple of 32 up to 1024");
-  MigArgs a{};
   int64_t total = 0;
   for (int k = 0; k < n_src; ++k) {
     const int rc = check_class(src[k], true, k, D);
@@ -419,7 +549,7 @@ extern "C" int hqekv_cache_migrate(int is_k, const hqekv_cache_class *src, int n
     const int64_t slab = src[k].slab_tokens > 0 ? src[k].slab_tokens : src[k].n_tokens;
     if (slab < src[k].n_tokens || (slab != src[k].n_tokens && !(src[k].bits == 16 && (!is_k || src[k].layout == HQEKV_LAYOUT_TOKEN_MAJOR))))
       return fail(HQEKV_E_ARG, "cache_migrate: source %d: slab_tokens applies to token-major fp16 sources and must be >= n_tokens", k);
-    a.src[k] = MigClass{src[k].data, (half_t *)src[k].scale, (half_t *)src[k].zero, nullptr, src[k].n_tokens, slab, src[k].bits, src[k].layout};
+    a->src[k] = MigClass{src[k].data, (half_t *)src[k].scale, (half_t *)src[k].zero, nullptr, src[k].n_tokens, slab, src[k].bits, src[k].layout, 0, 0};
   }
   for (int k = 0; k < n_dst; ++k) {
     const int rc = check_class(dst[k], false, k, D);
@@ -428,24 +558,80 @@ extern "C" int hqekv_cache_migrate(int is_k, const hqekv_cache_class *src, int n
       return fail(HQEKV_E_UNSUPPORTED, "cache_migrate: the fp16 K class is stored channel-major");
     if (dst[k].slab_tokens != 0 && dst[k].slab_tokens != dst[k].n_tokens)
       return fail(HQEKV_E_ARG, "cache_migrate: destination %d must be stored densely", k);
-    a.dst[k] = MigClass{dst[k].data, (half_t *)dst[k].scale, (half_t *)dst[k].zero, dst[k].idx, dst[k].n_tokens, dst[k].n_tokens, dst[k].bits, dst[k].layout};
-    a.dst_begin[k] = (int32_t)total;
+    a->dst[k] = MigClass{dst[k].data, (half_t *)dst[k].scale, (half_t *)dst[k].zero, dst[k].idx, dst[k].n_tokens, dst[k].n_tokens, dst[k].bits, dst[k].layout, (int32_t)total, 0};
+    a->dst_begin[k] = (int32_t)total;
     total += dst[k].n_tokens / 32;
   }
-  for (int k = n_dst; k <= HQEKV_MAX_SEGS; ++k) a.dst_begin[k] = (int32_t)total;
+  for (int k = n_dst; k <= HQEKV_MAX_SEGS; ++k) a->dst_begin[k] = (int32_t)total;
   if (total == 0) return HQEKV_OK;
   if (total >= (1 << 24)) return fail(HQEKV_E_UNSUPPORTED, "cache_migrate: %lld blocks (limit 2^24)", (long long)total);
   if (!plan) return fail(HQEKV_E_ARG, "cache_migrate: null plan");
-  a.n_dst = n_dst;
-  a.n_src = n_src;
-  a.status = status;
-  a.plan_src = plan;
-  a.plan_pos = plan + total;
-  if (is_k)
-    hipLaunchKernelGGL(cache_migrate_kernel<true>, dim3((unsigned)((total + MIG_KB - 1) / MIG_KB), (unsigned)BH, (unsigned)(D / MIG_KC)),
-                       dim3(MIG_KTHREADS), 0, (hipStream_t)stream, a, (int)D);
-  else
-    hipLaunchKernelGGL(cache_migrate_kernel<false>, dim3((unsigned)total, (unsigned)BH), dim3(MIG_THREADS), 0, (hipStream_t)stream, a,
-                       (int)D);
+  a->n_dst = n_dst;
+  a->n_src = n_src;
+  a->plan_src = plan;
+  a->plan_pos = plan + total;
+  const int64_t wgs = is_k ? (total + MIG_KB - 1) / MIG_KB * BH * (D / MIG_KC) : (total + MIG_VB - 1) / MIG_VB * BH;
+  if (wgs > 0x3fffffff) return fail(HQEKV_E_UNSUPPORTED, "cache_migrate: too many blocks and heads for one launch");
+  a->wgs = (int32_t)wgs;
+  return HQEKV_OK;
+}
+
+static int launch_migrate(MigArgs &a, int64_t BH, int64_t D, hipStream_t stream) {
+  a.BH = (int32_t)BH;
+  a.D = (int32_t)D;
+  const hqekv_migrate_extra &x = a.x;
+  const int64_t extra = x.ring_rows + (x.range_out ? ((int64_t)x.n_alive * 32 + MIG_THREADS - 1) / MIG_THREADS : 0) +
+                        (2 * BH * x.res_rows * D / 8 + MIG_THREADS - 1) / MIG_THREADS;
+  const int64_t wgs = a.side[0].wgs + a.side[1].wgs + extra;
+  if (wgs == 0) return HQEKV_OK;
+  if (wgs > 0x7fffffff) return fail(HQEKV_E_UNSUPPORTED, "cache_migrate: too many blocks and heads for one launch");
+  hipLaunchKernelGGL(cache_migrate_kernel, dim3((unsigned)wgs), dim3(MIG_THREADS), 0, stream, a);
   return check_launch("cache_migrate_kernel");
+}
+
+}  // namespace hq
+
+using namespace hq;
+
+extern "C" int hqekv_cache_migrate(int is_k, const hqekv_cache_class *src, int n_src, const hqekv_cache_class *dst,
+                                   int n_dst, const int32_t *plan, int64_t BH, int64_t D, int32_t *status, void *stream) {
+  if (BH <= 0 || BH > 65535 || D <= 0 || D % 32 != 0 || D > 1024)
+    return fail(HQEKV_E_ARG, "cache_migrate: need 0 < B*H <= 65535 and head_dim a multiple of 32 up to 1024");
+  MigArgs a{};
+  a.status = status;
+  const int rc = fill_side(is_k != 0, src, n_src, dst, n_dst, plan, BH, D, &a.side[is_k ? 0 : 1]);
+  return rc ? rc : launch_migrate(a, BH, D, (hipStream_t)stream);
+}
+
+extern "C" int hqekv_cache_migrate_both(const hqekv_cache_class *k_src, int n_k_src, const hqekv_cache_class *k_dst, int n_k_dst,
+                                        const int32_t *k_plan, const hqekv_cache_class *v_src, int n_v_src,
+                                        const hqekv_cache_class *v_dst, int n_v_dst, const int32_t *v_plan, int64_t BH, int64_t D,
+                                        const hqekv_migrate_extra *extra, void *stream) {
+  if (BH <= 0 || BH > 65535 || D <= 0 || D % 32 != 0 || D > 1024)
+    return fail(HQEKV_E_ARG, "cache_migrate: need 0 < B*H <= 65535 and head_dim a multiple of 32 up to 1024");
+  MigArgs a{};
+  int rc = fill_side(true, k_src, n_k_src, k_dst, n_k_dst, k_plan, BH, D, &a.side[0]);
+  if (!rc) rc = fill_side(false, v_src, n_v_src, v_dst, n_v_dst, v_plan, BH, D, &a.side[1]);
+  if (rc) return rc;
+  if (extra) {
+    const hqekv_migrate_extra &x = *extra;
+    const bool columns = x.ring_rows > 0 || x.range_out;
+    if (x.ring_rows < 0 || x.res_rows < 0 || x.res_rows > 0x7fffff || x.n_alive < 0 || x.n_alive >= (1 << 24) || x.first_moved < 0 ||
+        (columns && !x.alive) || (x.ring_rows > 0 && !x.ring) || (x.range_out && !x.range_in))
+      return fail(HQEKV_E_ARG, "cache_migrate: bad eviction or residual arguments");
+    for (int k = 0; k < 2 && x.res_rows; ++k)
+      if (!x.res_src[k] || !x.res_dst[k] || (((uintptr_t)x.res_src[k] | (uintptr_t)x.res_dst[k]) & 15) || x.res_src_slab[k] < 0 || x.res_dst_slab[k] < x.res_rows)
+        return fail(HQEKV_E_ARG, "cache_migrate: the residual rows must be 16-byte aligned and fit their destination");
+    a.x = x;
+  }
+  return launch_migrate(a, BH, D, (hipStream_t)stream);
+}
+
+extern "C" int hqekv_fetch_words(const void *host_src, void *dst, int64_t n, void *stream) {
+  if (n < 0 || n > 0x7fffff00LL || (n && (!host_src || !dst))) return fail(HQEKV_E_ARG, "fetch_words: null pointer or bad count");
+  if (((uintptr_t)host_src | (uintptr_t)dst) & 15) return fail(HQEKV_E_ALIGN, "fetch_words: 16-byte aligned buffers only");
+  if (n == 0) return HQEKV_OK;
+  hipLaunchKernelGGL(fetch_words_kernel, dim3((unsigned)((n + 1023) / 1024)), dim3(256), 0, (hipStream_t)stream, (const uint32_t *)host_src,
+                     (uint32_t *)dst, (int)n);
+  return check_launch("fetch_words_kernel");
 }

@@ -60,25 +60,36 @@ extern "C" int hqekv_plan_side(const int32_t *const *old_blocks, const int32_t *
   // ---- lay the new classes out: destination class, then origin (stays / new / down from fp16, 8, 4, 2), then source order
   int32_t *plan_src = plan_out;
   std::vector<int32_t> plan_pos((size_t)total);
+  auto each = [&](auto &&f) {   // every block: (source, its place there, its number, destination), sources in order
+    for (int src = 0; src <= NEW; ++src) {
+      const int32_t n_src = src == NEW ? n_new_blocks : old_counts[src];
+      for (int32_t j = 0; j < n_src; ++j) {
+        const int32_t b = src == NEW ? hist_blocks + j : old_blocks[src][j];
+        const int8_t to = label[(size_t)b];
+        f(src, j, b, src == NEW || to > src ? (int)to : src);
+      }
+    }
+  };
+  // (an evicted block's destination is beyond every class; the last row counts those)
+  int32_t at[NCLS + 1][NCLS + 2] = {};
+  const auto rank_in = [](int src, int dest) { return src == dest ? 0 : src == NEW ? 1 : 2 + src; };
+  each([&](int src, int32_t, int32_t, int dest) { ++at[dest][rank_in(src, dest)]; });
   int64_t u = 0;
   for (int d = 0; d < NCLS; ++d) {
     const int64_t begin = u;
-    auto take = [&](int src, int32_t n_src, auto &&block_of) {   // blocks of source `src` whose destination is d
-      for (int32_t j = 0; j < n_src; ++j) {
-        const int32_t b = block_of(j);
-        const int own = src == NEW ? -1 : src;
-        const int dest = std::max(own, (int)label[(size_t)b]);
-        if (dest != d) continue;
-        plan_src[u] = (int32_t)(((uint32_t)src << 24) | (uint32_t)j);
-        plan_pos[(size_t)u] = b;   // old position for now
-        ++u;
-      }
-    };
-    take(d, old_counts[d], [&](int32_t j) { return old_blocks[d][j]; });                    // stays
-    take(NEW, n_new_blocks, [&](int32_t j) { return hist_blocks + j; });                     // new tokens
-    for (int c = 0; c < d; ++c) take(c, old_counts[c], [&](int32_t j) { return old_blocks[c][j]; });   // comes down
+    for (int32_t &n : at[d]) {
+      const int32_t k = n;
+      n = (int32_t)u;
+      u += k;
+    }
     counts_out[d] = (int32_t)(u - begin);
   }
+  each([&](int src, int32_t j, int32_t b, int dest) {
+    if (dest == EVICT) return;
+    const int32_t k = at[dest][rank_in(src, dest)]++;
+    plan_src[k] = (int32_t)(((uint32_t)src << 24) | (uint32_t)j);
+    plan_pos[(size_t)k] = b;   // old position for now
+  });
   // ---- survivors in position order (a block ranked "evicted" is dropped whatever class it is in); a block's new
   // number is its rank among them
   int32_t n_alive = 0;

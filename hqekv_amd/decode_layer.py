@@ -23,9 +23,8 @@ from typing import Optional, Tuple
 import numpy as np
 import torch
 
-from . import prompt_attention
+from . import cache_policy, prompt_attention
 from .attention import SegmentMemo, value_length
-from .hqe_2 import KV_cache_hqe_2
 from .hqe_matmul import qkv_matmul_hqe_2
 from .public_func import last_attn_weights
 
@@ -179,6 +178,11 @@ class HqeAttentionLayer:
         return attn_weights, attn_output
 
     # ------------------------------------------------------------------ residual storage
+    @staticmethod
+    def _residual_rows(n: int) -> int:
+        """Capacity of the residual buffers for n tokens: whole blocks and one to spare."""
+        return max(2 * BLOCK, (n + BLOCK - 1) // BLOCK * BLOCK + BLOCK)
+
     def _residual_in_buffers(self, pkv: tuple, key_states: torch.Tensor) -> tuple:
         """The tuple with its fp16 residual held as the head of this layer's capacity-sized buffers (B,Hkv,cap,D), so
         that a decode step appends a row in place instead of re-allocating ``cat(residual, k)`` [131-133].  A residual
@@ -195,7 +199,7 @@ class HqeAttentionLayer:
         if fits and (n == 0 or (res_K.data_ptr() == buf[0].data_ptr() and res_V.data_ptr() == buf[1].data_ptr()
                                 and res_K.stride() == buf[0].stride() and res_V.stride() == buf[1].stride())):
             return pkv
-        cap = max(2 * BLOCK, (n + L + BLOCK - 1) // BLOCK * BLOCK + BLOCK)
+        cap = self._residual_rows(n + L)
         kb = torch.empty(B, H, cap, D, dtype=key_states.dtype, device=key_states.device)
         vb = torch.empty_like(kb)
         if n:
@@ -288,9 +292,16 @@ class HqeAttentionLayer:
         # the importance of every token and the ranking of the blocks; like the reference's ranking helper, which
         # divides its argument by the block length in place, this leaves the policy the divided values [226-231]
         importance, K_token_idx = self.last_weights.ranked_importance(total_length)
-        past_key_value = KV_cache_hqe_2(past_key_value, compress_length, self.history_reserve_length,
-                                        K_token_idx, K_bit_num, V_bit_num, importance,
-                                        self.quant_strategy, self.last_weights, BLOCK, BLOCK, self.times_range)
+        buffers = None
+        left = past_key_value[-3].shape[2] - compress_length
+        if left:   # what stays behind goes where the next step appends to it
+            B, H, _, D = key_states.shape
+            buffers = tuple(key_states.new_empty(B, H, self._residual_rows(left + 1), D) for _ in range(2))
+        past_key_value = cache_policy.compress(past_key_value, compress_length, self.history_reserve_length, K_token_idx, K_bit_num,
+                                               V_bit_num, importance, self.quant_strategy, last_weights=self.last_weights,
+                                               times_range=self.times_range, n_targets=6, residual_buffers=buffers)
+        if buffers is not None:
+            self._res = buffers
         self.history_reserve_length += compress_length - int(K_bit_num[-1])
         self.current_length -= compress_length
         if not shared:

@@ -340,6 +340,10 @@ int hqekv_token_range(const void *v, int64_t B, int64_t H, int64_t T, int64_t D,
  * n_prev > 0: D a multiple of 8, v 16-byte aligned. */
 int hqekv_token_range_append(const void *v, int64_t B, int64_t H, int64_t T, int64_t D, int64_t slab_tokens, const void *prev,
                              int64_t n_prev, void *out, void *stream);
+/* The same, and with the ranges the block scores of x weighted with them (hqekv_weighted_block_scores; weighted 0: of x
+ * alone): one launch.  x (n_prev + T) values, T and n_prev multiples of 32; D a multiple of 8, v 16-byte aligned. */
+int hqekv_range_block_scores(const void *v, int64_t B, int64_t H, int64_t T, int64_t D, int64_t slab_tokens, const void *prev,
+                             int64_t n_prev, const void *x, int weighted, void *range_out, void *scores_out, void *stream);
 /* order (rows x n): the block numbers of every row of n <= 32768 fp16 scores (scores: host array of rows <=
  * HQEKV_MAX_SEGS device pointers), highest score first, equal scores
  * in ascending order, NaN before everything: torch.sort(scores, descending=True, stable=True)[1], the sort of
@@ -404,6 +408,34 @@ typedef struct hqekv_cache_class {
 } hqekv_cache_class;
 int hqekv_cache_migrate(int is_k, const hqekv_cache_class *src, int n_src, const hqekv_cache_class *dst,
                         int n_dst, const int32_t *plan, int64_t BH, int64_t D, int32_t *status, void *stream);
+
+/* Both sides in one launch, and with it what else a compression moves (extra, NULL: nothing):
+ *   ring ...       fp16, ring_rows rows ring_stride columns apart: its first 32 * n_alive columns become the columns of the
+ *                  surviving blocks, in place (last_attn_weights.eviction, model/public_func.py:223-230); alive (device): their
+ *                  old block numbers, ascending; first_moved: the first i with alive[i] != i
+ *   range_in/_out  the same for a vector, out of place (NULL: none)
+ *   res_...        the res_rows token rows of either side that stay behind (K, V; slabs res_src_slab and res_dst_slab tokens
+ *                  apart) are copied to res_dst
+ */
+typedef struct {
+  void *ring;
+  int64_t ring_stride;
+  const void *range_in;
+  void *range_out;
+  const int32_t *alive;
+  int32_t ring_rows, n_alive, first_moved, res_rows;
+  const void *res_src[2];
+  void *res_dst[2];
+  int64_t res_src_slab[2], res_dst_slab[2];
+} hqekv_migrate_extra;
+int hqekv_cache_migrate_both(const hqekv_cache_class *k_src, int n_k_src, const hqekv_cache_class *k_dst, int n_k_dst,
+                             const int32_t *k_plan, const hqekv_cache_class *v_src, int n_v_src,
+                             const hqekv_cache_class *v_dst, int n_v_dst, const int32_t *v_plan, int64_t BH, int64_t D,
+                             const hqekv_migrate_extra *extra, void *stream);
+/* n 32-bit words from page-locked host memory into device memory, both 16-byte aligned, as a kernel on the stream: for
+ * the few kilobytes of a plan this is there sooner than a copy.  host_src must stay as it is until the stream has got
+ * that far. */
+int hqekv_fetch_words(const void *host_src, void *dst, int64_t n, void *stream);
 
 /* A hybrid cache back into dense fp16 K and V, (B,Hkv,T,D) each (BH = B * Hkv): every segment dequantised with the two
  * fp16 roundings and written to its positions, one launch.  Replaces the dequantise / index_put sequence of

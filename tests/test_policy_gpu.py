@@ -341,3 +341,34 @@ def test_native_compression_equals_step_engine(dev, strategy, times_range, monke
         for slot in range(42):
             _same(a[slot], b[slot].cpu() if torch.is_tensor(b[slot]) else b[slot], f"step {step} slot {slot}")
     assert torch.equal(ring, ring_slow)
+
+
+@pytest.mark.parametrize("blocks,first,max_len", [(1, 0, 33), (33, 1, 1100), (300, 5, 9601), (520, 300, 16640)])
+def test_eviction_that_rides_on_the_migration(dev, blocks, first, max_len):
+    """Ring columns in place (rows of odd length, more columns than one pass holds), a vector out of place, residual
+    rows of two lengths of slab -- ``hqekv_cache_migrate_both`` with nothing to migrate."""
+    import ctypes as C
+    from hqekv_amd import _lib
+
+    class Extra(C.Structure):
+        _fields_ = [("ring", C.c_void_p), ("ring_stride", C.c_int64), ("range_in", C.c_void_p), ("range_out", C.c_void_p), ("alive", C.c_void_p),
+                    ("ring_rows", C.c_int32), ("n_alive", C.c_int32), ("first_moved", C.c_int32), ("res_rows", C.c_int32),
+                    ("res_src", C.c_void_p * 2), ("res_dst", C.c_void_p * 2), ("res_src_slab", C.c_int64 * 2), ("res_dst_slab", C.c_int64 * 2)]
+    g = torch.Generator().manual_seed(blocks)
+    ring = torch.rand(3, max_len, generator=g).half()
+    vec = torch.rand(max_len, generator=g).half()
+    keep = torch.cat((torch.arange(first), first + torch.randperm(blocks - first, generator=g)[:max(1, (blocks - first) // 2)].sort()[0]))
+    moved = next((i for i, b in enumerate(keep.tolist()) if b != i), len(keep))
+    cols = (keep[:, None] * 32 + torch.arange(32)).reshape(-1)
+    want = ring.clone()
+    want[:, :cols.numel()] = ring[:, cols]
+    k, v = torch.rand(2, 3, 50, 128, generator=g).half().to(dev), torch.rand(2, 3, 9, 128, generator=g).half().to(dev)
+    kd, vd = torch.zeros(2, 3, 64, 128, dtype=torch.float16, device=dev), torch.zeros(2, 3, 7, 128, dtype=torch.float16, device=dev)
+    ring_d, vec_d, alive = ring.to(dev), vec.to(dev), keep.to(torch.int32).to(dev)
+    out = torch.empty(cols.numel(), dtype=torch.float16, device=dev)
+    x = Extra(ring_d.data_ptr(), max_len, vec_d.data_ptr(), out.data_ptr(), alive.data_ptr(), 3, len(keep), moved, 7,
+              (C.c_void_p * 2)(k.data_ptr() + 2 * 128 * 43, v.data_ptr() + 2 * 128 * 2), (C.c_void_p * 2)(kd.data_ptr(), vd.data_ptr()),
+              (C.c_int64 * 2)(50, 9), (C.c_int64 * 2)(64, 7))
+    _lib.check(_lib.load().hqekv_cache_migrate_both(None, 0, None, 0, None, None, 0, None, 0, None, 6, 128, C.byref(x), _lib.stream_ptr(dev)), "migrate")
+    assert torch.equal(ring_d.cpu(), want) and torch.equal(out.cpu(), vec[cols])
+    assert torch.equal(kd[:, :, :7], k[:, :, 43:]) and not kd[:, :, 7:].any() and torch.equal(vd, v[:, :, 2:])
