@@ -61,3 +61,29 @@ def test_several_blocks_per_workgroup(dev, n_rep):
     w, o = decode_attention(q.to(dev), synth.cache_to(cache, dev), None, int(cache[41]), zero_init=False, flags=1)
     torch.testing.assert_close(w.float().cpu(), w_ref.float(), rtol=RTOL, atol=ATOL)
     torch.testing.assert_close(o.float().cpu(), o_ref.float(), rtol=RTOL, atol=ATOL)
+
+
+@pytest.mark.parametrize("n_rep,low_normal,shuffled,B", [(4, False, False, 512), (5, True, False, 512), (4, True, True, 512), (3, False, False, 300), (12, False, False, 512)])
+def test_several_tiles_per_workgroup_of_scores(dev, n_rep, low_normal, shuffled, B):
+    """A launch long enough for q.K^T to take four tiles per workgroup -- classes that end inside a wave's tile, inside a
+    workgroup's four, exactly at their end -- against the same rows in a batch of two, which takes one tile each."""
+    from hqekv_amd.attention import decode_attention
+    from hqekv_amd.pack_unpack import normal_group_quantize_pack_last_dim, uniform_group_quantize_pack_last_dim
+    blocks, residual, Hkv, D = (5, 9, 33, 31, 33), 65, 2, 128
+    n = 32 * sum(blocks)
+
+    def quantize(x, g, bits):
+        return normal_group_quantize_pack_last_dim(x, 32, 1) if bits == 1 and low_normal else uniform_group_quantize_pack_last_dim(x, 32, bits)
+    q, K, V = synth.make_qkv(2, n_rep * Hkv, Hkv, n + residual, D, 78, dev)
+    order = torch.randperm(n if shuffled else n // 32, generator=torch.Generator().manual_seed(n))
+    tokens = order if shuffled else (order[:, None] * 32 + torch.arange(32)).reshape(-1)
+    classes, at = {}, 0
+    for bits, c in zip((16, 8, 4, 2, 1), blocks):
+        classes[bits] = tokens[at:at + 32 * c].sort()[0]
+        at += 32 * c
+    pkv = synth.build_cache(K, V, classes, residual, quantize)
+    big = tuple(x.repeat(B // 2, 1, 1, 1) if torch.is_tensor(x) and x.dim() == 4 else x for x in pkv)
+    small = decode_attention(q, pkv, None, n + residual, True, low_uniform=not low_normal)
+    got = decode_attention(q.repeat(B // 2, 1, 1, 1), big, None, n + residual, True, low_uniform=not low_normal)
+    for g, w in zip(got, small):
+        torch.testing.assert_close(g.float(), w.repeat(B // 2, 1, 1, 1).float(), rtol=2e-3, atol=1e-3)
