@@ -80,6 +80,13 @@ class StepExtra(C.Structure):
         ("v_dst", C.c_void_p),
         ("k_dst_slab_tokens", C.c_int64),
         ("v_dst_slab_tokens", C.c_int64),
+        ("leave_bits", C.c_int32),
+        ("leave_src", C.c_void_p),
+        ("leave_slab_tokens", C.c_int64),
+        ("leave_code", C.c_void_p),
+        ("leave_scale", C.c_void_p),
+        ("leave_zero", C.c_void_p),
+        ("leave_dst_slab_tokens", C.c_int64),
     ]
 
 

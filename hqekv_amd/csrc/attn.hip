@@ -24,6 +24,7 @@
 //            through fp32 partials summed in a fixed order.
 #include "attn_common.h"
 #include "decode_tiles.h"
+#include "quant_math.h"
 
 #pragma clang fp contract(off)
 
@@ -1840,6 +1841,20 @@ __device__ __forceinline__ void step_epilogue_block(const StepEpilogue &e, int64
       *dst = *src;
     }
   }
+  if (e.leave_bits) {   // four lanes per group of 32 (a KIVI layer's step: a launch of 2.6 us of its own before)
+    const int64_t n = (int64_t)e.app_bh * e.leave_groups * 4;
+    for (int64_t i = blk * blockDim.x + threadIdx.x; i < n; i += nblk * blockDim.x) {
+      const int64_t bh = (i >> 2) / e.leave_groups, g = (i >> 2) % e.leave_groups, at = bh * e.leave_rows * e.leave_groups + g;
+      const half_t *src = e.leave_src + bh * e.leave_slab + 32 * g;
+      const uint32_t sub = (uint32_t)i & 3u;
+      switch (e.leave_bits) {
+        case 8: quant_group_of_4<8>(src, sub, e.leave_code + at * 8, e.leave_scale + at, e.leave_zero + at); break;
+        case 4: quant_group_of_4<4>(src, sub, e.leave_code + at * 4, e.leave_scale + at, e.leave_zero + at); break;
+        case 2: quant_group_of_4<2>(src, sub, e.leave_code + at * 2, e.leave_scale + at, e.leave_zero + at); break;
+        default: quant_group_of_4<1>(src, sub, e.leave_code + at, e.leave_scale + at, e.leave_zero + at);
+      }
+    }
+  }
 }
 
 // fixed-order sum over chunks: deterministic replacement for the reference's half atomics
@@ -2166,7 +2181,7 @@ static int launch_pv(const SegTable &tb, int64_t chunk, void *p, void *out, floa
     }
   }
   const bool combine = (stages & 2) && !fz.arrive;   // folded: the last p.V workgroups have written the output
-  const bool epilogue = ep && (ep->ring_line || ep->app_rows > 0) && stages == 3;
+  const bool epilogue = ep && (ep->ring_line || ep->app_rows > 0 || ep->leave_bits) && stages == 3;
   if (!combine && !epilogue) return HQEKV_OK;
   // The epilogue rides in the combine launch as extra workgroups (grid.z); one workgroup per RING_SPAN columns of
   // the ring row.  Without a combine (folded into p.V) the launch holds the epilogue alone.
@@ -2347,7 +2362,6 @@ static int fill_epilogue(const hqekv_step_extra *x, const void *attn_weights, in
       return fail(HQEKV_E_ALIGN, "decode_step: appended rows and their destinations must be 16-byte aligned");
     e->app_rows = x->append_rows;
     e->app_row_elems = (int32_t)D;
-    e->app_bh = (int32_t)(B * Hkv);
     e->app_src[0] = (const half_t *)x->new_k;
     e->app_src[1] = (const half_t *)x->new_v;
     e->app_dst[0] = (half_t *)x->k_dst;
@@ -2355,6 +2369,22 @@ static int fill_epilogue(const hqekv_step_extra *x, const void *attn_weights, in
     e->app_src_slab[0] = e->app_src_slab[1] = (int64_t)x->append_rows * D;
     e->app_dst_slab[0] = x->k_dst_slab_tokens * D;
     e->app_dst_slab[1] = x->v_dst_slab_tokens * D;
+  }
+  e->app_bh = (int32_t)(B * Hkv);
+  if (x->leave_bits) {
+    if (x->leave_bits != 8 && x->leave_bits != 4 && x->leave_bits != 2 && x->leave_bits != 1) return fail(HQEKV_E_ARG, "decode_step: leave_bits=%d", x->leave_bits);
+    if (!x->leave_src || !x->leave_code || !x->leave_scale || !x->leave_zero || x->leave_slab_tokens < 1 || x->leave_dst_slab_tokens < 1 || D % 32)
+      return fail(HQEKV_E_ARG, "decode_step: a row to quantise without source or destination");
+    if (((uintptr_t)x->leave_src & 15) || ((uintptr_t)x->leave_code & 3) || (x->leave_slab_tokens * D) % 8)
+      return fail(HQEKV_E_ALIGN, "decode_step: the row to quantise must be 16-byte aligned");
+    e->leave_bits = x->leave_bits;
+    e->leave_groups = (int32_t)(D / 32);
+    e->leave_src = (const half_t *)x->leave_src;
+    e->leave_slab = x->leave_slab_tokens * D;
+    e->leave_code = (uint32_t *)x->leave_code;
+    e->leave_scale = (half_t *)x->leave_scale;
+    e->leave_zero = (half_t *)x->leave_zero;
+    e->leave_rows = x->leave_dst_slab_tokens;
   }
   return HQEKV_OK;
 }

@@ -100,6 +100,12 @@ struct StepEpilogue {
   half_t *app_dst[2];          // first destination row of slab 0
   int64_t app_src_slab[2];     // elements between two (b, kv head) slabs
   int64_t app_dst_slab[2];
+  // a row per (b, kv head) that is quantised on the way (hqekv_step_extra.leave_*); slabs in elements of each array
+  int32_t leave_bits, leave_groups;   // groups of 32 per row
+  const half_t *leave_src;
+  uint32_t *leave_code;
+  half_t *leave_scale, *leave_zero;
+  int64_t leave_slab, leave_rows;     // elements / destination token rows between two slabs
 };
 
 // A workgroup learns its segment and its tile/chunk from its block id with two scalar loads at the top of

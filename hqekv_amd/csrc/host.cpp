@@ -85,6 +85,19 @@ Tensor new_tensor(at::IntArrayRef shape, at::ScalarType type, const at::Device &
   return at::empty(shape, at::TensorOptions().dtype(type).device(dev));
 }
 
+// Token rows [from, from + n) of a (B, H, capacity, X) buffer: x.slice(2, from, from + n) at a third of its price (a step
+// makes up to seven).  The version counter is the buffer's, as a view's is.
+Tensor rows_of(const Tensor &x, int64_t from, int64_t n) {
+  if (x.requires_grad()) return x.slice(2, from, from + n);
+  c10::TensorImpl *base = x.unsafeGetTensorImpl();
+  Tensor t = at::detail::make_tensor<c10::TensorImpl>(c10::TensorImpl::VIEW, c10::Storage(x.storage()), x.key_set(), x.dtype());
+  c10::TensorImpl *impl = t.unsafeGetTensorImpl();
+  const int64_t shape[4] = {x.size(0), x.size(1), n, x.size(3)};
+  impl->set_sizes_and_strides(shape, x.strides(), x.storage_offset() + from * x.stride(2));
+  if (!x.is_inference()) impl->set_version_counter(base->version_counter());
+  return t;
+}
+
 // ------------------------------------------------------------------------------------------------ the cache tuple
 // Field numbers of the 42-field tuple (hqekv_amd/attention.py): fp16 K 0/1, fp16 V 2/3, then per bit width code, idx,
 // scale, zero; 39/40 the fp16 residual.
@@ -387,8 +400,8 @@ PyObject *tables_step(PyObject *self, PyObject *const *a, Py_ssize_t na) {
     Py_INCREF(o);
     PyTuple_SET_ITEM(next, i, o);
   }
-  PyTuple_SET_ITEM(next, NEW_K, THPVariable_Wrap(kb.slice(2, 0, n + 1)));
-  PyTuple_SET_ITEM(next, NEW_V, THPVariable_Wrap(vb.slice(2, 0, n + 1)));
+  PyTuple_SET_ITEM(next, NEW_K, THPVariable_Wrap(rows_of(kb, 0, n + 1)));
+  PyTuple_SET_ITEM(next, NEW_V, THPVariable_Wrap(rows_of(vb, 0, n + 1)));
   Py_INCREF(a[10]);
   PyTuple_SET_ITEM(next, TUPLE_LEN - 1, a[10]);
   return Py_BuildValue("NNN", THPVariable_Wrap(weights), THPVariable_Wrap(out), next);
@@ -473,8 +486,8 @@ PyGetSetDef kivi_fields[] = {
 };
 
 // KiviState.step(q, k, v, T, k_bits, v_bits): the attention over (K class, K tail, this step's key) and (V class, V tail,
-// this step's value), the two rows appended behind their tails by the call's last launch, and -- when the tail is full
-// -- the quantiser launch that moves the oldest value row into the class buffers, which must have room for it.  Leaves a full K tail
+// this step's value); the call's last launch appends the two rows behind their tails and -- when the tail is full --
+// quantises the oldest value row into the class buffers, which must have room for it.  Leaves a full K tail
 // (nk == its capacity) and a V window at the end of its buffer to the caller.  -> (attn_weights, attn_output) or None.
 PyObject *kivi_step(PyObject *self, PyObject *const *a, Py_ssize_t na) {
   HANDLE_TH_ERRORS
@@ -527,6 +540,16 @@ PyObject *kivi_step(PyObject *self, PyObject *const *a, Py_ssize_t na) {
   x.v_dst = vt + (s->v0 + s->nv) * row;
   x.k_dst_slab_tokens = R;
   x.v_dst_slab_tokens = cap_v;
+  if (leaves) {   // (R > nk >= 0, so the tail has a row: not the one this step appends)
+    const int64_t n = s->n_vq, groups = s->vscale.size(3);
+    x.leave_bits = v_bits;
+    x.leave_src = vt + s->v0 * row;
+    x.leave_slab_tokens = cap_v;
+    x.leave_code = (char *)s->vcode.data_ptr() + n * s->vcode.size(3) * 4;
+    x.leave_scale = (char *)s->vscale.data_ptr() + n * groups * 2;
+    x.leave_zero = (char *)s->vzero.data_ptr() + n * groups * 2;
+    x.leave_dst_slab_tokens = s->vcode.size(2);
+  }
   const c10::OptionalDeviceGuard guard(dev);
   Tensor weights = new_tensor({q.size(0), q.size(1), 1, T}, at::kHalf, dev), out = new_tensor({q.size(0), q.size(1), 1, D}, at::kHalf, dev);
   int rc = run_step(ks, n_k, vs, n_v, q, weights, out, Hkv, T, s->ws, dev, &x);
@@ -534,11 +557,6 @@ PyObject *kivi_step(PyObject *self, PyObject *const *a, Py_ssize_t na) {
   s->nk += 1;
   s->nv += 1;
   if (leaves) {
-    const int64_t words = s->vcode.size(3), groups = s->vscale.size(3), cap = s->vcode.size(2), n = s->n_vq;
-    rc = api.hqekv_quant_pack_rows(vt + s->v0 * row, cap_v * D, D, (char *)s->vcode.data_ptr() + n * words * 4, cap * words, words,
-                                   (char *)s->vscale.data_ptr() + n * groups * 2, (char *)s->vzero.data_ptr() + n * groups * 2, cap * groups,
-                                   groups, q.size(0) * Hkv, 1, D, v_bits, stream_of(dev));
-    if (rc) return raise_rc(rc, "uniform_group_quantize_pack_last_dim");
     s->n_vq += 1;
     s->v0 += 1;
     s->nv -= 1;
@@ -559,7 +577,7 @@ PyObject *kivi_tuple(PyObject *self, PyObject *T) {
       PyTuple_SET_ITEM(t, i, Py_None);
     }
   };
-  auto head = [](const Tensor &x, int64_t n) { return n ? x.slice(2, 0, n) : Tensor(); };
+  auto head = [](const Tensor &x, int64_t n) { return n ? rows_of(x, 0, n) : Tensor(); };
   PyObject *t = PyTuple_New(9);
   if (!t) return nullptr;
   put(t, 0, s->kq);
@@ -567,7 +585,7 @@ PyObject *kivi_tuple(PyObject *self, PyObject *T) {
   put(t, 2, s->ks);
   put(t, 3, s->kz);
   put(t, 4, head(s->vcode, s->n_vq));
-  put(t, 5, s->vt.slice(2, s->v0, s->v0 + s->nv));
+  put(t, 5, rows_of(s->vt, s->v0, s->nv));
   put(t, 6, head(s->vscale, s->n_vq));
   put(t, 7, head(s->vzero, s->n_vq));
   Py_INCREF(T);
@@ -1139,8 +1157,8 @@ PyObject *compress(PyObject *, PyObject *const *a, Py_ssize_t na) {
   }
   put_item(out, RANGES, THPVariable_Wrap(kept_range));
   if (rk) {
-    put_item(out, NEW_K, THPVariable_Wrap(resK.size(2) > rk ? resK.slice(2, 0, rk) : resK));
-    put_item(out, NEW_V, THPVariable_Wrap(resV.size(2) > rk ? resV.slice(2, 0, rk) : resV));
+    put_item(out, NEW_K, THPVariable_Wrap(resK.size(2) > rk ? rows_of(resK, 0, rk) : resK));
+    put_item(out, NEW_V, THPVariable_Wrap(resV.size(2) > rk ? rows_of(resV, 0, rk) : resV));
   }
   if (!evicted || ring.defined()) return Py_BuildValue("NO", out, Py_None);
   Tensor keep = at::empty({32 * (int64_t)n_alive[1]}, at::TensorOptions().dtype(at::kLong));

@@ -81,6 +81,92 @@ __device__ __forceinline__ uint32_t first_zero_bits(const half_t (&x)[N]) {
   return r;
 }
 
+// One group of 32 contiguous values (16-byte aligned) by four neighbouring lanes, `sub` = 0 .. 3: codes, scale and zero are
+// stored by them.
+template <int BITS>
+__device__ __forceinline__ void quant_group_of_4(const half_t *x, uint32_t sub, uint32_t *crow, half_t *scale, half_t *zero) {
+  constexpr float INV_QMAX = 1.0f / (float)((1 << BITS) - 1);
+  const uint4 raw = *reinterpret_cast<const uint4 *>(x + sub * 8u);
+  const half2_t p[4] = {bits_h2(raw.x), bits_h2(raw.y), bits_h2(raw.z), bits_h2(raw.w)};
+
+  half2_t lo2 = __builtin_elementwise_min(__builtin_elementwise_min(p[0], p[1]), __builtin_elementwise_min(p[2], p[3]));
+  half2_t hi2 = __builtin_elementwise_max(__builtin_elementwise_max(p[0], p[1]), __builtin_elementwise_max(p[2], p[3]));
+  // (min, -max) in one register: one packed min per butterfly step serves both
+  half2_t mm = {(half_t)__builtin_fminf((float)lo2[0], (float)lo2[1]), (half_t)(-__builtin_fmaxf((float)hi2[0], (float)hi2[1]))};
+  mm = __builtin_elementwise_min(mm, bits_h2(quad_xor_u<1>(h2_bits(mm))));
+  mm = __builtin_elementwise_min(mm, bits_h2(quad_xor_u<2>(h2_bits(mm))));
+  half_t mn_h = mm[0];
+  float mn = (float)mn_h, mx = -(float)mm[1];
+  // A zero extreme takes the sign of the group's first zero (torch's tie rule, see first_zero_bits).  The wave
+  // branches around this as a whole (a scalar branch on the ballot): groups with a zero extreme are rare, and a
+  // predicated copy of the block in every lane's path cost the kernel 5-10 %.
+  const bool zero_extreme = __builtin_fminf(__builtin_fabsf(mn), __builtin_fabsf(mx)) == 0.0f;   // mn == 0 or mx == 0
+  if (__builtin_amdgcn_ballot_w64(zero_extreme) != 0 && zero_extreme) {
+    // (the condition is the same for the four lanes of a group: they hold its minimum and maximum)
+    const half_t mine[8] = {p[0][0], p[0][1], p[1][0], p[1][1], p[2][0], p[2][1], p[3][0], p[3][1]};
+    const uint32_t own = first_zero_bits(mine);
+    const uint32_t x1 = quad_xor_u<1>(own), x2 = quad_xor_u<2>(own), x3 = quad_xor_u<1>(x2);  // lanes sub^1, sub^2, sub^3
+    uint32_t by_lane[4];
+#pragma unroll
+    for (int l = 0; l < 4; ++l) by_lane[l] = (sub == (uint32_t)l) ? own : (sub == (uint32_t)(l ^ 1)) ? x1 : (sub == (uint32_t)(l ^ 2)) ? x2 : x3;
+    uint32_t first = 1u;
+#pragma unroll
+    for (int l = 3; l >= 0; --l)
+      if (by_lane[l] != 1u) first = by_lane[l];
+    const half_t z = __builtin_bit_cast(half_t, (unsigned short)first);   // (a zero extreme implies a zero element)
+    if (mn == 0.0f) {
+      mn_h = z;
+      mn = (float)z;
+    }
+    if (mx == 0.0f) mx = (float)z;
+  }
+
+  const half_t d = (half_t)(mx - mn);
+  const half_t sc = (half_t)((float)d * INV_QMAX);
+  const float rcp = group_recip((float)sc);
+
+  const half2_t mn2 = {mn_h, mn_h};
+  float u[8];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const half2_t c = p[i] - mn2;
+    u[2 * i] = (float)c[0];
+    u[2 * i + 1] = (float)c[1];
+  }
+
+  if (BITS == 8) {
+    uint32_t z[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      z[0] = code_pair_biased<8>(u[4 * h + 0], rcp, u[4 * h + 2], rcp);
+      z[1] = code_pair_biased<8>(u[4 * h + 1], rcp, u[4 * h + 3], rcp);
+      crow[sub * 2 + h] = horner_pack<8, 2>(z);
+    }
+  } else {
+    uint32_t z[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) z[i] = code_pair_biased<BITS>(u[i], rcp, u[i + 4], rcp);
+    if (BITS == 4) {
+      crow[sub] = horner_pack<4, 4>(z);
+    } else if (BITS == 1) {
+      const uint32_t w = horner_pack<1, 4>(z);             // codes 0-3 in bits 0-3, codes 4-7 in bits 16-19
+      const uint32_t b8 = (w & 0xfu) | ((w >> 12) & 0xf0u);  // this lane's 8 codes
+      const uint32_t b16 = b8 | (quad_xor_u<1>(b8) << 8);        // even lanes: two lanes' codes in order
+      const uint32_t other = quad_xor_u<2>(b16);
+      if (sub == 0) crow[0] = b16 | (other << 16);
+    } else {
+      const uint32_t w = horner_pack<2, 4>(z);             // codes 0-3 in byte 0, codes 4-7 in byte 2
+      const uint32_t h = __builtin_amdgcn_perm(0u, w, 0x0c0c0200u);   // 16 bits: this lane's 8 codes
+      const uint32_t other = quad_xor_u<1>(h);
+      if ((sub & 1) == 0) crow[sub >> 1] = h | (other << 16);
+    }
+  }
+  if (sub == 0) {
+    *scale = sc;
+    *zero = mn_h;
+  }
+}
+
 struct Normal1Stats {
   half_t mean_h, std_h;
   float thr;  // std * 2^-25

@@ -307,6 +307,15 @@ typedef struct hqekv_step_extra {
   void *k_dst, *v_dst;         /* where slab 0's first appended row goes (16-byte aligned)                 */
   int64_t k_dst_slab_tokens;   /* token rows between two (b, kv head) slabs of the destination buffers     */
   int64_t v_dst_slab_tokens;
+  /* One token row per (b, kv head) quantised on the way, as hqekv_quant_pack_rows does (8, 4, 2 or 1 bit; 0 = none): the
+   * value row that leaves the fp16 tail of a KIVI layer.  Neither a row this call appends nor one its segments read as
+   * codes; leave_src, slabs leave_slab_tokens token rows apart, is 16-byte aligned; codes, scale and zero of slab 0 at
+   * leave_code / _scale / _zero, slabs leave_dst_slab_tokens token rows apart.                                        */
+  int32_t leave_bits;
+  const void *leave_src;
+  int64_t leave_slab_tokens;
+  void *leave_code, *leave_scale, *leave_zero;
+  int64_t leave_dst_slab_tokens;
 } hqekv_step_extra;
 int hqekv_decode_step(const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_segs, int n_v,
                       const void *q, const void *mask, int64_t mask_row_stride,
