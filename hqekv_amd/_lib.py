@@ -47,7 +47,7 @@ EXPORTS = (
     "hqekv_gemv_workspace_bytes", "hqekv_gemv_uniform_group", "hqekv_gemv_normal_group",
     "hqekv_qk_hybrid", "hqekv_scale_softmax", "hqekv_pv_workspace_bytes", "hqekv_pv_hybrid",
     "hqekv_decode_workspace_bytes", "hqekv_decode_attn", "hqekv_decode_attn_static", "hqekv_decode_step", "hqekv_ring_row",
-    "hqekv_importance_scores", "hqekv_weighted_block_scores", "hqekv_token_range", "hqekv_token_range_append", "hqekv_range_block_scores", "hqekv_rank_blocks",
+    "hqekv_ring_rows", "hqekv_importance_scores", "hqekv_weighted_block_scores", "hqekv_token_range", "hqekv_token_range_append", "hqekv_range_block_scores", "hqekv_rank_blocks",
     "hqekv_prompt_attn", "hqekv_prompt_last_rows", "hqekv_prompt_last_rows_workspace_bytes",
     "hqekv_cache_migrate", "hqekv_cache_migrate_both", "hqekv_fetch_words", "hqekv_cache_reconstruct", "hqekv_cover_once", "hqekv_plan_side",
 )
@@ -134,6 +134,7 @@ _PROTOS = {
     "hqekv_decode_attn": (C.c_int, [_SEGP, _int, _SEGP, _int, _vp, _vp, _i64, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _vp, _i64, _int, _vp]),
     "hqekv_decode_step": (C.c_int, [_SEGP, _int, _SEGP, _int, _vp, _vp, _i64, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _vp, _i64, _int, _vp, C.POINTER(StepExtra)]),
     "hqekv_ring_row": (C.c_int, [_vp, _i64, _i64, _i64, _vp, _int, _vp]),
+    "hqekv_ring_rows": (C.c_int, [_vp, _i64, _i64, _i64, _i64, _vp, _i64, _i64, _int, _int, _vp]),
     "hqekv_importance_scores": (C.c_int, [_vp, C.c_int32, _i64, _i64, _i64, _vp, _vp, _vp]),
     "hqekv_weighted_block_scores": (C.c_int, [_vp, _vp, _i64, _vp, _vp]),
     "hqekv_token_range": (C.c_int, [_vp, _i64, _i64, _i64, _i64, _i64, _vp, _vp]),

@@ -1711,7 +1711,11 @@ __device__ __forceinline__ float torch_row_sum_n(Load &&load) {
 }
 
 constexpr int RING_V = 4;                 // adjacent columns of the ring row a lane loads at a time (8 bytes)
-constexpr int RING_SPAN = 64 * RING_V;    // columns a workgroup covers per pass
+// Columns a workgroup of 1024 threads covers per pass: 256 with the heads dealt to 16 waves, eight loads per lane -- or 64
+// with a head row per 16 lanes, all heads of a batch row in flight at once and four times as many workgroups: the form for
+// rows that fit one such pass or two (3.3k columns in a step's last launch: 5.4 -> 4.2 us).
+constexpr int RING_SPAN = 64 * RING_V, RING_SPAN_SHORT = 16 * RING_V;
+constexpr int RING_BLOCKS = 512;          // workgroups of a launch of its own: two per CU
 constexpr int RING_LDS_HEADS = 64;        // most heads whose batch sums a pass parks in LDS
 
 // The probabilities as a pointer into global memory: the pointer arrives inside a by-value struct, where the
@@ -1732,10 +1736,10 @@ struct RingShape {
 // time: the loads of HU heads are issued before the first sum is formed (the additions keep torch_row_sum's order)
 // `shift` > 0 marks the row's last, ragged quad: its loads start `shift` columns early, so that they end with the
 // row, and the wanted columns are moved down afterwards.
-template <int NB>
+template <int NB, int SPAN>
 __device__ __forceinline__ void ring_heads_to_lds(const RingShape r, ring_src_t col, int shift, int g, int waves,
                                                   half_t *tile_lane) {
-  constexpr int HU = 8 / NB;   // heads in flight per thread: about eight loads
+  constexpr int HU = SPAN == RING_SPAN ? 8 / NB : 1;   // heads in flight per thread: about eight loads, or one per batch row
   const int64_t hs = r.Tall, bs = (int64_t)r.Hq * r.Tall;
   for (int h0 = g; h0 < r.Hq; h0 += waves * HU) {
     uint64_t raw[HU][NB];   // a quad is loaded, shifted and stored as one 64-bit word
@@ -1759,7 +1763,7 @@ __device__ __forceinline__ void ring_heads_to_lds(const RingShape r, ring_src_t 
           v |= (uint64_t)__builtin_bit_cast(uint16_t, s) << (16 * i);
         }
       }
-      if (h < r.Hq) *reinterpret_cast<uint64_t *>(tile_lane + h * RING_SPAN) = v;   // 8-byte aligned: lane * RING_V halves
+      if (h < r.Hq) *reinterpret_cast<uint64_t *>(tile_lane + h * SPAN) = v;   // 8-byte aligned: lane * RING_V halves
     }
   }
 }
@@ -1776,48 +1780,51 @@ __device__ __noinline__ float ring_column_alone(const RingShape r, int64_t t) {
   return r.by == 2 ? torch_row_sum<2>(r.Hq, head) : torch_row_sum<1>(r.Hq, head);
 }
 
-// Columns [c0, c1) of the ring row, RING_SPAN per pass (c0 a multiple of RING_SPAN).  The loads are spread over the
-// whole workgroup -- lane l of every wave looks at columns 4 l .. 4 l + 3 of the pass, wave g at heads g, g + waves,
+// Columns [c0, c1) of the ring row, SPAN per pass (c0 a multiple of SPAN).  The loads are spread over the whole workgroup
+// -- lane l of every group of SPAN / 4 threads looks at columns 4 l .. 4 l + 3 of the pass, group g at heads g, g + groups,
 // ... -- so every load is independent of the others and 8 bytes wide; the head values (fp16 by construction) meet
-// in LDS, where the first RING_SPAN threads add them up in torch's order, one column each.  Every thread of the
-// workgroup must call this with the same arguments; blockDim.x is a multiple of 64 and at least RING_SPAN.
+// in LDS, where the first SPAN threads add them up in torch's order, one column each.  Every thread of the
+// workgroup must call this with the same arguments; blockDim.x is a multiple of 64 and at least SPAN.
+template <int SPAN>
 __device__ __forceinline__ void ring_row_columns(const StepEpilogue &e, int64_t c0, int64_t c1, half_t *tile) {
   const RingShape r{(ring_src_t)(uintptr_t)e.weights, e.Tall, e.B, e.Hq, e.ring_by};
   half_t *const line = e.ring_line;
-  const int lane = threadIdx.x & 63, g = threadIdx.x >> 6, waves = blockDim.x >> 6;
+  constexpr int QUADS = SPAN / RING_V;
+  const int lane = threadIdx.x % QUADS, g = threadIdx.x / QUADS, groups = blockDim.x / QUADS;
   const bool lds = r.Hq <= RING_LDS_HEADS && r.B <= 8;
-  for (int64_t t0 = c0; t0 < c1; t0 += RING_SPAN) {
-    const int64_t t = t0 + threadIdx.x;   // the column this thread sums in the end (threads below RING_SPAN)
+  for (int64_t t0 = c0; t0 < c1; t0 += SPAN) {
+    const int64_t t = t0 + threadIdx.x;   // the column this thread sums in the end (threads below SPAN)
     if (lds) {
       const int64_t c = t0 + lane * RING_V;
       // the row's last quad may stick out by `shift` columns (the passes of all workgroups but the last end on a
-      // multiple of RING_SPAN): it is loaded from `shift` columns earlier, which needs a row of RING_V columns at least
+      // multiple of SPAN): it is loaded from `shift` columns earlier, which needs a row of RING_V columns at least
       const int shift = (int)max((int64_t)0, c + RING_V - c1);
       const bool mine = shift < RING_V && c - shift >= 0;
       ring_src_t col = r.w + (mine ? c - shift : 0);
       half_t *tile_lane = tile + lane * RING_V;
       switch (mine ? r.B : 0) {
-        case 1: ring_heads_to_lds<1>(r, col, shift, g, waves, tile_lane); break;
-        case 2: ring_heads_to_lds<2>(r, col, shift, g, waves, tile_lane); break;
-        case 3: ring_heads_to_lds<3>(r, col, shift, g, waves, tile_lane); break;
-        case 4: ring_heads_to_lds<4>(r, col, shift, g, waves, tile_lane); break;
-        case 5: ring_heads_to_lds<5>(r, col, shift, g, waves, tile_lane); break;
-        case 6: ring_heads_to_lds<6>(r, col, shift, g, waves, tile_lane); break;
-        case 7: ring_heads_to_lds<7>(r, col, shift, g, waves, tile_lane); break;
-        case 8: ring_heads_to_lds<8>(r, col, shift, g, waves, tile_lane); break;
+        case 1: ring_heads_to_lds<1, SPAN>(r, col, shift, g, groups, tile_lane); break;
+        case 2: ring_heads_to_lds<2, SPAN>(r, col, shift, g, groups, tile_lane); break;
+        case 3: ring_heads_to_lds<3, SPAN>(r, col, shift, g, groups, tile_lane); break;
+        case 4: ring_heads_to_lds<4, SPAN>(r, col, shift, g, groups, tile_lane); break;
+        case 5: ring_heads_to_lds<5, SPAN>(r, col, shift, g, groups, tile_lane); break;
+        case 6: ring_heads_to_lds<6, SPAN>(r, col, shift, g, groups, tile_lane); break;
+        case 7: ring_heads_to_lds<7, SPAN>(r, col, shift, g, groups, tile_lane); break;
+        case 8: ring_heads_to_lds<8, SPAN>(r, col, shift, g, groups, tile_lane); break;
         default: break;
       }
       __syncthreads();
     }
-    if (threadIdx.x < RING_SPAN && t < c1) {
+    if (threadIdx.x < SPAN && t < c1) {
       float sum;
       if (lds && c1 >= RING_V) {
-        auto head = [&](int h) -> float { return (float)tile[h * RING_SPAN + threadIdx.x]; };
+        auto head = [&](int h) -> float { return (float)tile[h * SPAN + threadIdx.x]; };
         sum = r.by == 2 ? torch_row_sum<2>(r.Hq, head) : torch_row_sum<1>(r.Hq, head);
       } else {   // outside what the LDS tile covers: the thread walks its column alone
         sum = ring_column_alone(r, t);
       }
-      line[t] = (half_t)sum;
+      // (several rows at once: the columns are (row, token) pairs)
+      line[e.ring_tokens ? t / e.ring_tokens * e.ring_stride + t % e.ring_tokens : t] = (half_t)sum;
     }
     if (lds) __syncthreads();
   }
@@ -1826,8 +1833,19 @@ __device__ __forceinline__ void ring_row_columns(const StepEpilogue &e, int64_t 
 // block `blk` of `nblk` of the epilogue: a share of the ring row's columns, and of the appended rows
 __device__ __forceinline__ void step_epilogue_block(const StepEpilogue &e, int64_t blk, int64_t nblk, half_t *sh) {
   if (e.ring_line) {
-    const int64_t per = ((e.Tall + nblk - 1) / nblk + RING_SPAN - 1) / RING_SPAN * RING_SPAN;
-    ring_row_columns(e, min(e.Tall, blk * per), min(e.Tall, (blk + 1) * per), sh);
+    if (e.Tall <= 2 * RING_SPAN_SHORT * nblk) {
+      const int64_t per = ((e.Tall + nblk - 1) / nblk + RING_SPAN_SHORT - 1) / RING_SPAN_SHORT * RING_SPAN_SHORT;
+      ring_row_columns<RING_SPAN_SHORT>(e, min(e.Tall, blk * per), min(e.Tall, (blk + 1) * per), sh);
+    } else {
+      const int64_t per = ((e.Tall + nblk - 1) / nblk + RING_SPAN - 1) / RING_SPAN * RING_SPAN;
+      ring_row_columns<RING_SPAN>(e, min(e.Tall, blk * per), min(e.Tall, (blk + 1) * per), sh);
+    }
+  }
+  if (e.ring_fill_rows) {   // a new store: zeros wherever these rows do not reach
+    const uint32_t stride = (uint32_t)e.ring_stride, n = (uint32_t)e.ring_fill_rows * stride;
+    const uint32_t rows = (uint32_t)(e.Tall / e.ring_tokens), tokens = (uint32_t)e.ring_tokens;
+    for (uint32_t i = (uint32_t)blk * blockDim.x + threadIdx.x; i < n; i += (uint32_t)nblk * blockDim.x)
+      if (i / stride >= rows || i % stride >= tokens) e.ring_line[i] = (half_t)0;
   }
   if (e.app_rows > 0) {   // 16-byte pieces of the appended rows, dealt over the blocks
     const int64_t row16 = e.app_row_elems / 8;   // pieces per row (head_dim is a multiple of 32)
@@ -2399,11 +2417,31 @@ extern "C" int hqekv_ring_row(const void *attn_weights, int64_t B, int64_t Hq, i
   StepEpilogue e;
   const int rc = fill_epilogue(&x, attn_weights, B, Hq, 1, 32, Tall, &e);
   if (rc) return rc;
-  const int64_t blocks = (Tall + RING_SPAN - 1) / RING_SPAN;
-  if (blocks > 0x7fffffffLL) return fail(HQEKV_E_UNSUPPORTED, "ring_row: Tall too large");
-  hipLaunchKernelGGL(pv_combine_kernel, dim3((unsigned)blocks, 1, 1), dim3(CB_CH * CB_SLICES), 0, (hipStream_t)stream,
+  const int64_t blocks = (Tall + RING_SPAN_SHORT - 1) / RING_SPAN_SHORT;
+  hipLaunchKernelGGL(pv_combine_kernel, dim3((unsigned)std::min<int64_t>(blocks, RING_BLOCKS)), dim3(CB_CH * CB_SLICES), 0, (hipStream_t)stream,
                      (const float *)nullptr, (half_t *)nullptr, 0, (int64_t)0, 0, e, 0);
   return check_launch("ring_row");
+}
+
+extern "C" int hqekv_ring_rows(const void *attn_weights, int64_t B, int64_t Hq, int64_t rows, int64_t T, void *ring, int64_t ring_rows,
+                               int64_t ring_stride, int order, int fresh, void *stream) {
+  if (!attn_weights || !ring || B <= 0 || Hq <= 0 || rows <= 0 || T <= 0 || B > 0x7fffffffLL || Hq > 0x7fffffffLL || rows > ring_rows ||
+      T > ring_stride || (order != 1 && order != 2))
+    return fail(HQEKV_E_ARG, "ring_rows: null pointer, empty shape, or a store too small");
+  if (ring_rows * ring_stride >= (1LL << 31)) return fail(HQEKV_E_UNSUPPORTED, "ring_rows: store too large");
+  hqekv_step_extra x{};
+  x.ring_line = ring;
+  x.ring_order = order;
+  StepEpilogue e;
+  const int rc = fill_epilogue(&x, attn_weights, B, Hq, 1, 32, rows * T, &e);
+  if (rc) return rc;
+  e.ring_tokens = T;
+  e.ring_stride = ring_stride;
+  e.ring_fill_rows = fresh ? (int32_t)ring_rows : 0;
+  const int64_t blocks = (rows * T + RING_SPAN_SHORT - 1) / RING_SPAN_SHORT;
+  hipLaunchKernelGGL(pv_combine_kernel, dim3((unsigned)std::min<int64_t>(blocks, RING_BLOCKS)), dim3(CB_CH * CB_SLICES), 0, (hipStream_t)stream,
+                     (const float *)nullptr, (half_t *)nullptr, 0, (int64_t)0, 0, e, 0);
+  return check_launch("ring_rows");
 }
 
 static int decode_impl(const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_segs, int n_v,

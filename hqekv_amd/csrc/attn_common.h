@@ -93,6 +93,9 @@ struct StepEpilogue {
   int64_t Tall;
   int32_t B, Hq;
   int32_t ring_by;         // threads torch's reduction deals the head rows to for this shape: 1 or 2
+  int64_t ring_tokens;     // several rows at once (Tall = rows * ring_tokens, ring_stride columns apart in the store); 0 = one
+  int64_t ring_stride;
+  int32_t ring_fill_rows;  // rows of the store to zero where nothing else is written
   int32_t app_rows;        // token rows to append per (b, kv head); 0 = none
   int32_t app_row_elems;   // head_dim
   int32_t app_bh;          // B * Hkv

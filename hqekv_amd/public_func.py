@@ -269,12 +269,40 @@ class last_attn_weights:
         self.kv_seq_len = T
         self.next_line = (self.next_line + 1) % self.last_length
 
+    def _prompt_rows(self, attn_weights: torch.Tensor) -> bool:
+        """The rows of a prompt into the store, zeros behind them when the store is made here, in one launch
+        (``hqekv_ring_rows``) in place of a fill, two reductions and a copy; False where the order in which torch adds is
+        not pinned."""
+        from . import _lib
+        from .attention import ring_order, ring_row_on_device_applies
+        B, H, L, T = attn_weights.shape
+        w = self.weights
+        if not (attn_weights.is_contiguous() and ring_row_on_device_applies(attn_weights.view(B, H, 1, L * T))):
+            return False
+        if w is not None and not (w.dtype == torch.float16 and w.is_contiguous() and w.device == attn_weights.device):
+            return False
+        if T > (self.max_length if w is None else w.shape[1]):
+            return False
+        fresh = w is None
+        if fresh:
+            w = attn_weights.new_empty(self.last_length, self.max_length)
+        with _lib.on_device(w.device):
+            rc = _lib.load().hqekv_ring_rows(attn_weights.data_ptr(), B, H, L, T, w.data_ptr(), w.shape[0], w.shape[1],
+                                             ring_order(L * T, attn_weights), 1 if fresh else 0, _lib.stream_ptr(w.device))
+        _lib.check(rc, "ring_rows")
+        self.weights = w
+        return True
+
     def update(self, attn_weights: torch.Tensor) -> None:
         """attn_weights (B, H, L, T): a prompt (L > 1) stores its last rows, a decode step (L == 1) one ring row.
         The sums run over the batch first and over the heads second, each rounded to the store's dtype."""
+        L, T = attn_weights.shape[2], attn_weights.shape[3]
+        if L > 1 and L <= self.last_length and attn_weights.is_cuda and self._prompt_rows(attn_weights):
+            self.kv_seq_len = T
+            self.next_line = (self.next_line + L) % self.last_length
+            return
         if self.weights is None:
             self.weights = attn_weights.new_zeros(self.last_length, self.max_length)
-        L, T = attn_weights.shape[2], attn_weights.shape[3]
         if L > 1:
             rows = min(L, self.last_length)
             self.weights[:rows, :T] = attn_weights[:, :, L - rows:, :].sum(0).sum(0)

@@ -326,6 +326,10 @@ int hqekv_decode_step(const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_segs,
  * ring_order above).  Replaces last_attn_weights.update for one decode row (model/public_func.py:250-254). */
 int hqekv_ring_row(const void *attn_weights, int64_t B, int64_t Hq, int64_t Tall, void *line, int order,
                    void *stream);
+/* The rows of a prompt: attn_weights (B, Hq, rows, T), the row sums written to the first `rows` rows of the store
+ * (ring_rows x ring_stride); `order`: ring_order for a row of rows * T columns.  fresh: the rest of the store is zeroed. */
+int hqekv_ring_rows(const void *attn_weights, int64_t B, int64_t Hq, int64_t rows, int64_t T, void *ring, int64_t ring_rows,
+                    int64_t ring_stride, int order, int fresh, void *stream);
 
 /* What the cache policy ranks blocks by (model/public_func.py:217-221 calculate_token_importance, :85-106
  * get_block_importance / get_block_token_idx with its in-place divide, quant/hqe_2.py:510-518 the V ranking's

@@ -300,3 +300,26 @@ def test_token_range_behind_older_ranges(dev, B, H, T, D, prev):
     lo, hi = torch.aminmax(v, dim=-1)
     want = torch.cat((old, (hi - lo).sum(0).sum(0)))
     assert torch.equal(calculate_token_range(v, old if prev else None), want)
+
+
+@pytest.mark.parametrize("B", [1, 2, 3, 4, 5, 8])
+@pytest.mark.parametrize("kind", ["order_sensitive", "probabilities"])
+def test_prompt_rows_equal_torch_sums_on_device(dev, B, kind):
+    """A prompt's rows enter the store in one launch: torch's own reductions over the (B, 32, rows, T) tensor, bit for
+    bit, short and long rows; the rest of a new store is zero, of an old one untouched."""
+    from hqekv_amd.public_func import last_attn_weights
+    g = torch.Generator().manual_seed(300 * B + len(kind))
+    for rows, T in ((20, 20), (7, 41), (20, 63), (20, 1027), (19, 4099), (20, 8192), (20, 20000 if B == 1 else 9001)):
+        w = (_order_sensitive if kind == "order_sensitive" else _probabilities)(B, 32, rows * T, g).to(dev).view(B, 32, rows, T)
+        expect = w.sum(0).sum(0)
+        for extra, old in ((0, False), (25, False), (11, True)):
+            ring = last_attn_weights()
+            ring.set_max_length(T + extra)
+            if old:
+                ring.weights = torch.full((20, T + extra), -5.0, dtype=torch.float16, device=dev)
+            assert ring._prompt_rows(w) if not old else True
+            ring.update(w)
+            want = torch.full((20, T + extra), -5.0 if old else 0.0, dtype=torch.float16, device=dev)
+            want[:rows, :T] = expect
+            assert torch.equal(ring.weights.view(torch.int16), want.view(torch.int16)), (B, rows, T, extra, old)
+            assert ring.kv_seq_len == T and ring.next_line == rows % 20
