@@ -2485,7 +2485,7 @@ static int decode_impl(const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_segs
   int tiling = 0;
   rc = resolve_qk_tiling(qk_tiling_of(flags), k_segs, n_k, B * Hkv, D, "decode_attn", &tiling);
   if (rc) return rc;
-  // The launches of decode_tiles.hip take the call unless it names a form of the older ones.
+  // The launches of decode_qk.hip and decode_pv.hip take the call unless it names a form of the older ones.
   const bool by_rule = !(flags & (HQEKV_QK_TILING(0xf) | HQEKV_DOT_MFMA | HQEKV_DOT_VALU | HQEKV_TWO_STEP_DEQUANT | HQEKV_FOLD_COMBINE |
                                  HQEKV_SEPARATE_COMBINE));
   const bool k_tiles = by_rule && n_k > 0 && tiles_fit(k_segs, n_k, true, D, B, Hq, Hkv);
