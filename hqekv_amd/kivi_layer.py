@@ -138,10 +138,17 @@ class KiviAttentionLayer:
         B, H, _, D = like.shape
         dev, R = like.device, self.residual_length
         st = _lib.host().KiviState()
-        st.kt = torch.empty(B, H, R, D, dtype=torch.float16, device=dev)
-        st.vt = torch.empty(B, H, 2 * R + 32, D, dtype=torch.float16, device=dev)   # the tail's window slides one row per step
+        st.kt = self._tail_buffer(like, R)
+        st.vt = self._tail_buffer(like, 2 * R + 32)   # the tail's window slides one row per step
         self._grow_v_class(st, B, H, D, dev, n_vq + 1)
         return st
+
+    @staticmethod
+    def _tail_buffer(like: torch.Tensor, rows: int) -> torch.Tensor:
+        """Rows for a tail.  A row is written once: views of it are in tuples that the caller may keep, so a buffer that is
+        used up is replaced by another."""
+        B, H, _, D = like.shape
+        return torch.empty(B, H, rows, D, dtype=torch.float16, device=like.device)
 
     def _adopt(self, pkv: tuple, like: torch.Tensor):
         """Capacity buffers holding what ``pkv`` holds: the K tail, the V tail (a window that slides one row per step)
@@ -181,11 +188,11 @@ class KiviAttentionLayer:
 
     def _step_in_buffers(self, q, k, v, pkv: tuple, T: int):
         """One decode step with everything appended in place: ONE call for the attention over (K class, K tail, this
-        step's key) and (V class, V tail, this step's value) with the two rows copied behind their tails in the
-        call's last launch, one quantiser launch when the oldest value row leaves the tail (written straight into the
-        class buffers), one concatenation every ``residual_length`` steps when a block of keys is quantised.  The
-        tuple handed back holds views of the buffers, with upstream's shapes and contents [117-266].  None: an input is
-        not what the native step takes."""
+        step's key) and (V class, V tail, this step's value), whose last launch also copies the two rows behind their
+        tails and quantises the oldest value row when it leaves the tail (straight into the class buffers); one
+        concatenation every ``residual_length`` steps when a block of keys is quantised.  The tuple handed back holds
+        views of the buffers, with upstream's shapes and contents [117-266]; later steps write only rows that no tuple
+        shows.  None: an input is not what the native step takes."""
         q, k, v = (x if x.is_contiguous() else x.contiguous() for x in (q, k, v))
         R = self.residual_length
         st = self._st
@@ -203,11 +210,12 @@ class KiviAttentionLayer:
             if st.kq is not None:
                 new = [torch.cat((old, x), dim=3) for old, x in zip((st.kq, st.ks, st.kz), new)]
             st.kq, st.ks, st.kz = new
-            st.nk = 0
+            st.kt, st.nk = self._tail_buffer(k, R), 0
         nv, v0 = st.nv, st.v0
-        if v0 + nv == st.vt.shape[2]:   # the window has reached the end of its buffer: back to the start
-            st.vt[:, :, :nv].copy_(st.vt[:, :, v0:v0 + nv].clone())
-            st.v0 = 0
+        if v0 + nv == st.vt.shape[2]:   # the window has reached the end of its buffer: on to the start of another
+            vt = self._tail_buffer(k, st.vt.shape[2])
+            vt[:, :, :nv].copy_(st.vt[:, :, v0:v0 + nv])
+            st.vt, st.v0 = vt, 0
         return out, weights, st.fields(T)
 
     # ------------------------------------------------------------------ one call

@@ -132,3 +132,32 @@ def test_kivi_layer_argument_errors(dev):
         KiviAttentionLayer(D, k_bits=3)
     with pytest.raises(ValueError):
         KiviAttentionLayer(D, group_size=64)
+
+
+def test_kivi_tuples_keep_their_contents(dev):
+    """What a call handed out is not written again by later steps -- past a full K tail, the end of the V window's buffer and
+    a V class that outgrows its own -- so one prompt can be continued several times."""
+    from hqekv_amd.kivi_layer import KiviAttentionLayer
+    B, Hq, Hkv, T0, steps, R = 1, 8, 2, 45, 80, 32
+    layer = KiviAttentionLayer(D, 2, 2, 32, R)
+    data = [tuple(x.to(dev) for x in _qkv(B, Hq, Hkv, T0 if s == 0 else 1, 700 + s)) for s in range(steps + 1)]
+
+    def copy(pkv):
+        return tuple(x.clone() if torch.is_tensor(x) else x for x in pkv)
+
+    def run(pkv, n):
+        outs, tuples = [], [(pkv, copy(pkv))]
+        for s in range(1, n + 1):
+            out, w, pkv = layer(*data[s], None, pkv)
+            outs.append((out, w))
+            tuples.append((pkv, copy(pkv)))
+        return outs, tuples
+    prompt = layer(*data[0])[2]
+    first, tuples = run(prompt, steps)
+    again, more = run(prompt, steps)
+    late, most = run(tuples[30][0], 5)        # and one from the middle
+    for (a, wa), (b, wb) in zip(first, again):
+        assert torch.equal(a, b) and torch.equal(wa, wb)
+    assert len(late) == 5
+    for i, (kept, want) in enumerate(tuples + more + most):
+        _same_tuple(kept, tuple(x.cpu() if torch.is_tensor(x) else x for x in want), f"tuple {i}")
