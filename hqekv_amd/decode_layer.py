@@ -149,6 +149,7 @@ class HqeAttentionLayer:
         self.last_weights = last_attn_weights(last_length=last_length)
         self._memo = SegmentMemo()   # segment tables of the classes, rebuilt after each compression
         self._res = None             # (K buffer, V buffer): the fp16 residual in capacity-sized storage
+        self._res_rows = 0           # its first rows, which tuples handed out show: never written again
         self.fused_step = True       # ring row and residual appends inside the attention call (False: separate launches)
         self._own_tuple = False      # the tuple handed in carries the class tensors this layer built its tables from
         self._returned = None        # (the tuple the last plain decode step returned, tokens in its residual)
@@ -186,8 +187,9 @@ class HqeAttentionLayer:
     def _residual_in_buffers(self, pkv: tuple, key_states: torch.Tensor) -> tuple:
         """The tuple with its fp16 residual held as the head of this layer's capacity-sized buffers (B,Hkv,cap,D), so
         that a decode step appends a row in place instead of re-allocating ``cat(residual, k)`` [131-133].  A residual
-        that is not there yet -- after the prompt, after a compression, or a tuple from elsewhere -- is copied in
-        once; the fields of the tuple are views of the same shape and content as the reference's tensors."""
+        that is not there yet -- after the prompt, a tuple from elsewhere -- or whose next row is already another tuple's
+        is copied into new buffers; the fields of the tuple are views of the same shape and content as the reference's
+        tensors."""
         res_K, res_V = pkv[-3], pkv[-2]
         B, H, L, D = key_states.shape
         n = res_K.shape[2] if res_K is not None else 0
@@ -195,7 +197,8 @@ class HqeAttentionLayer:
         held = self._memo.held
         self._own_tuple = held is not None and all(a is b for a, b in zip(held, pkv))
         fits = (buf is not None and buf[0].shape[0] == B and buf[0].shape[1] == H and buf[0].shape[3] == D
-                and buf[0].device == key_states.device and buf[0].dtype == key_states.dtype and n + L <= buf[0].shape[2])
+                and buf[0].device == key_states.device and buf[0].dtype == key_states.dtype
+                and n == self._res_rows and n + L <= buf[0].shape[2])
         if fits and (n == 0 or (res_K.data_ptr() == buf[0].data_ptr() and res_V.data_ptr() == buf[1].data_ptr()
                                 and res_K.stride() == buf[0].stride() and res_V.stride() == buf[1].stride())):
             return pkv
@@ -205,7 +208,7 @@ class HqeAttentionLayer:
         if n:
             kb[:, :, :n].copy_(res_K)
             vb[:, :, :n].copy_(res_V)
-        self._res = (kb, vb)
+        self._res, self._res_rows = (kb, vb), n
         if n == 0:
             return pkv
         return pkv[:-3] + (kb[:, :, :n], vb[:, :, :n], pkv[-1])
@@ -270,6 +273,7 @@ class HqeAttentionLayer:
                 self._res[1][:, :, n:n + L].copy_(value_states)
                 new_K, new_V = self._res[0][:, :, :n + L], self._res[1][:, :, :n + L]
                 past_key_value = past_key_value[:-3] + (new_K, new_V, kv_seq_len)
+            self._res_rows = n + L
         else:
             attn_weights, attn_output = self._prefill(query_states, key_states, value_states, attention_mask)
             past_key_value = (None,) * 39 + (key_states, value_states, kv_seq_len)
@@ -300,8 +304,7 @@ class HqeAttentionLayer:
         past_key_value = cache_policy.compress(past_key_value, compress_length, self.history_reserve_length, K_token_idx, K_bit_num,
                                                V_bit_num, importance, self.quant_strategy, last_weights=self.last_weights,
                                                times_range=self.times_range, n_targets=6, residual_buffers=buffers)
-        if buffers is not None:
-            self._res = buffers
+        self._res, self._res_rows = buffers, left   # (nothing left: the next step starts new ones)
         self.history_reserve_length += compress_length - int(K_bit_num[-1])
         self.current_length -= compress_length
         if not shared:

@@ -99,3 +99,23 @@ def test_layer_in_lockstep_with_oracle(dev, B, Hq, Hkv, T0, steps, strategy, bit
     kept = sum(pkv_g[s].shape[2] for s in (2, 8, 16, 24, 32) if pkv_g[s] is not None)
     assert kept == layer.history_reserve_length
     assert int(pkv_g[41]) == T0 + steps
+
+
+@pytest.mark.parametrize("fused", [True, False], ids=["one-call", "separate"])
+def test_layer_tuples_keep_their_contents(dev, fused):
+    """What a call handed out is not written again by later steps, compressions that leave a residual behind and ones that
+    leave nothing among them; a tuple continued a second time does not touch what its first continuation returned."""
+    from hqekv_amd.decode_layer import HqeAttentionLayer
+    B, Hq, Hkv, D, T0, steps = 1, 8, 2, 128, 300, 72
+    layer = HqeAttentionLayer(D, 0.2, 0.3, 0.5)
+    layer.set_max_length(T0 + steps)
+    layer.fused_step = fused
+    data = [tuple(x.to(dev) for x in _qkv(B, Hq, Hkv, T0 if s == 0 else 1, D, 800 + s)) for s in range(steps + 1)]
+
+    pkv, tuples = None, []
+    for s in range(steps + 1):
+        pkv = layer(*data[s], None, pkv)[2]
+        tuples.append((pkv, tuple(x.to("cpu", copy=True) if torch.is_tensor(x) else x for x in pkv)))
+    layer(*data[1], None, tuples[-2][0])
+    for i, (kept, want) in enumerate(tuples):
+        _same_tuple(kept, want, f"tuple {i}")
