@@ -292,7 +292,7 @@ __device__ __forceinline__ void qk_f16_tm_tile(const SegDev &sg, int tile, int b
   float m_run[NREP], l_run[NREP];  // running softmax statistics of this wave's tokens (fused mode)
 #pragma unroll
   for (int h = 0; h < NREP; ++h) {
-    m_run[h] = -INFINITY;
+    m_run[h] = SM_FLOOR;
     l_run[h] = 0.f;
   }
   if (D == 128) {
@@ -326,7 +326,7 @@ __device__ __forceinline__ void qk_f16_tm_tile(const SegDev &sg, int tile, int b
           const float x = valid ? (float)rr : -INFINITY;
           const float mn = fmaxf(m_run[h], wave_max(x));
           const float e = (valid && lg == 0) ? __expf(x - mn) : 0.f;
-          const float keep = (m_run[h] == mn) ? 1.f : __expf(m_run[h] - mn);  // also covers -inf == -inf
+          const float keep = (m_run[h] == mn) ? 1.f : __expf(m_run[h] - mn);
           l_run[h] = l_run[h] * keep + wave_sum(e);
           m_run[h] = mn;
         }
@@ -371,7 +371,7 @@ __device__ __forceinline__ void qk_f16_tm_tile(const SegDev &sg, int tile, int b
     __syncthreads();
     if (threadIdx.x < NREP) {
       const int h = threadIdx.x;
-      float m = -INFINITY, l = 0.f;
+      float m = SM_FLOOR, l = 0.f;
       for (int w = 0; w < QK_WAVES; ++w) m = fmaxf(m, red[(w * NREP + h) * 2]);
       for (int w = 0; w < QK_WAVES; ++w) {
         const float lw = red[(w * NREP + h) * 2 + 1];
@@ -513,7 +513,7 @@ __global__ __launch_bounds__(QK_WAVES * 64, NREP <= 4 ? 16 / QK_WAVES : 1) void 
           for (int i = 0; i < VPT; ++i) a[i] += part[i];
         }
         half_t v[VPT];
-        float m_lane = -INFINITY;
+        float m_lane = SM_FLOOR;
 #pragma unroll
         for (int i = 0; i < VPT; ++i) {
           v[i] = (half_t)a[i];
@@ -548,7 +548,7 @@ __global__ __launch_bounds__(QK_WAVES * 64, NREP <= 4 ? 16 / QK_WAVES : 1) void 
         __syncthreads();
         if (threadIdx.x < NREP) {
           const int h = threadIdx.x;
-          float m = -INFINITY, l = 0.f;
+          float m = SM_FLOOR, l = 0.f;
 #pragma unroll
           for (int w = 0; w < WPH; ++w) m = fmaxf(m, wave_ml[h][w].x);
 #pragma unroll
@@ -1045,7 +1045,7 @@ __global__ __launch_bounds__(64, NREP <= 4 ? (TPL == 8 ? 4 : 6) : 2) void qk_wav
 #pragma unroll
   for (int h = 0; h < NREP; ++h) {
     half_t v[TPL];
-    float m_lane = -INFINITY;
+    float m_lane = SM_FLOOR;
 #pragma unroll
     for (int i = 0; i < TPL; ++i) {
       v[i] = (half_t)acc[h][i];
@@ -1055,7 +1055,7 @@ __global__ __launch_bounds__(64, NREP <= 4 ? (TPL == 8 ? 4 : 6) : 2) void qk_wav
       }
     }
     if (fz.stats) {  // (max, sum exp) of the tile
-      if (!valid) m_lane = -INFINITY;
+      if (!valid) m_lane = SM_FLOOR;
       const float m = wave_max(m_lane);
       float l_lane = 0.f;
 #pragma unroll

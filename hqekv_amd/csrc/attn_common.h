@@ -53,6 +53,11 @@ __device__ __forceinline__ int begin_of_seg(const SegTable &tb, int s) {
   return b;
 }
 
+// A running maximum starts at SM_FLOOR, below every finite fp16 logit but finite: a logit of -inf (a score beyond fp16's
+// range) then adds exp(-inf) = 0 wherever it meets other logits or none, where exp(-inf - -inf) would be NaN.  A row of
+// nothing but -inf still sums to zero and becomes NaN, as in torch.
+constexpr float SM_FLOOR = -3.0e38f;
+
 // Optional fusion of the softmax into the two GEMV launches (valid when no mask is added and the K
 // classes as well as the V classes each cover every position exactly once):
 //   q.K^T stores the scaled fp16 logit instead of the raw score and one (max, sum exp) pair per tile and

@@ -51,14 +51,14 @@ __device__ __forceinline__ void qt_finish_tile(QtLds<HP> &lds, const f4_t (&acc)
     for (int t = 0; t < TPV; ++t) lds.part(wave, h)[(t / P) * 64 * P + lane * P + t % P] = acc[t][h];
   __syncthreads();
   half_t x[TPV];
-  float m = -INFINITY;
+  float m = SM_FLOOR;
 #pragma unroll
   for (int t = 0; t < TPV; ++t) {
     const int at = (t / P) * 64 * P + lane * P + t % P;
     x[t] = (half_t)(((lds.part(0, wave)[at] + lds.part(1, wave)[at]) + lds.part(2, wave)[at]) + lds.part(3, wave)[at]);
     if (FUSED) {   // the fp16 steps of the reference epilogue: round the score, scale, round again
       x[t] = (half_t)((float)x[t] * inv_sqrt_d);
-      m = fmaxf(m, t < n_valid ? (float)x[t] : -INFINITY);
+      m = fmaxf(m, t < n_valid ? (float)x[t] : SM_FLOOR);
     }
   }
   if (TPV > 1 && run && n_valid >= TPV) {
@@ -235,7 +235,7 @@ __global__ __launch_bounds__(QT_WAVES * 64, HP == 4 ? 5 : HP == 8 ? 4 : 2) void 
   const int head = (4 * r) % HP + wave;   // the head this lane finishes
   const bool has_head = head < nrep;
   half_t *row = scores + ((int64_t)b * Hq + head0 + min(head, nrep - 1)) * Tall;
-  float m = -INFINITY, l = 0.f;
+  float m = SM_FLOOR, l = 0.f;
 #define HQ_TILE(B_, NORMAL_) qt_class_tile<B_, HP, FUSED, NORMAL_>(sg, tile, bh, ta.n_bh, wave, lane, qv, lds, row, has_head, fz.inv_sqrt_d, m, l)
   switch (sg.bits) {
     case 1:
@@ -259,7 +259,7 @@ __global__ __launch_bounds__(QT_WAVES * 64, HP == 4 ? 5 : HP == 8 ? 4 : 2) void 
   mm = fmaxf(mm, dpp_f<0x140>(mm));
   if (HP <= 4) mm = fmaxf(mm, xor_f(mm, 16));
   if (HP <= 8) mm = fmaxf(mm, xor_f(mm, 32));
-  l = m == mm ? l : l * __expf(m - mm);   // (a lane that saw no token: l = 0, m = -inf)
+  l = m == mm ? l : l * __expf(m - mm);   // (a lane that saw no token: l = 0, m the floor)
   l += dpp_f<0xB1>(l);
   l += dpp_f<0x4E>(l);
   l += dpp_f<0x141>(l);
@@ -292,13 +292,13 @@ __device__ __forceinline__ void ql_finish(const f4_t (&acc)[TPV], int r, Pos &&p
     const int nv = head < nrep ? n_valid : 0;
     half_t *row = rows + (int64_t)min(head, nrep - 1) * Tall;
     half_t x[TPV];
-    float mm = -INFINITY;
+    float mm = SM_FLOOR;
 #pragma unroll
     for (int t = 0; t < TPV; ++t) {
       x[t] = (half_t)acc[t][h];
       if (FUSED) {   // the fp16 steps of the reference epilogue: round the score, scale, round again
         x[t] = (half_t)((float)x[t] * inv_sqrt_d);
-        mm = fmaxf(mm, t < nv ? (float)x[t] : -INFINITY);
+        mm = fmaxf(mm, t < nv ? (float)x[t] : SM_FLOOR);
       }
     }
     if (TPV > 1 && run && nv >= TPV) {
@@ -497,7 +497,7 @@ __global__ __launch_bounds__(QT_WAVES * 64, HP == 4 ? 4 : 2) void qk_long_kernel
   float m[4], l[4];
 #pragma unroll
   for (int h = 0; h < 4; ++h) {
-    m[h] = -INFINITY;
+    m[h] = SM_FLOOR;
     l[h] = 0.f;
   }
 #define HQ_TILE(B_, NORMAL_) ql_class<B_, HP, FUSED, NORMAL_>(sg, unit, bh, ta.n_bh, wave, lane, qrow, sz, rows, Tall, nrep, fz.inv_sqrt_d, m, l)
@@ -524,7 +524,7 @@ __global__ __launch_bounds__(QT_WAVES * 64, HP == 4 ? 4 : 2) void qk_long_kernel
     mm = fmaxf(mm, dpp_f<0x140>(mm));
     if (HP <= 4) mm = fmaxf(mm, xor_f(mm, 16));
     if (HP <= 8) mm = fmaxf(mm, xor_f(mm, 32));
-    ll = m[h] == mm ? ll : ll * __expf(m[h] - mm);   // (a lane that saw no token: l = 0, m = -inf)
+    ll = m[h] == mm ? ll : ll * __expf(m[h] - mm);   // (a lane that saw no token: l = 0, m the floor)
     ll += dpp_f<0xB1>(ll);
     ll += dpp_f<0x4E>(ll);
     ll += dpp_f<0x141>(ll);
@@ -537,7 +537,7 @@ __global__ __launch_bounds__(QT_WAVES * 64, HP == 4 ? 4 : 2) void qk_long_kernel
   const int head = threadIdx.x;
   if (head < nrep) {
     float2 v[QT_WAVES];
-    float mm = -INFINITY, ll = 0.f;
+    float mm = SM_FLOOR, ll = 0.f;
 #pragma unroll
     for (int w = 0; w < QT_WAVES; ++w) {
       v[w] = st[w][head];

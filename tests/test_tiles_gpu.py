@@ -87,3 +87,30 @@ def test_several_tiles_per_workgroup_of_scores(dev, n_rep, low_normal, shuffled,
     got = decode_attention(q.repeat(B // 2, 1, 1, 1), big, None, n + residual, True, low_uniform=not low_normal)
     for g, w in zip(got, small):
         torch.testing.assert_close(g.float(), w.repeat(B // 2, 1, 1, 1).float(), rtol=2e-3, atol=1e-3)
+
+
+@pytest.mark.parametrize("n_rep", [1, 4, 5, 12])
+@pytest.mark.parametrize("B,tiling", [(1, 0), (400, 0), (1, 1), (1, 3)], ids=["one-tile", "four-tiles", "8waves", "wave512"])
+def test_a_score_of_minus_infinity_has_probability_zero(dev, n_rep, B, tiling):
+    """A finite key whose score leaves fp16's range on the negative side, alone in its lane, its tile or its class."""
+    from hqekv_amd import _lib
+    from hqekv_amd.attention import decode_attention
+    Hkv, D, blocks, residual = 2, 128, (4, 8, 8, 8, 8), 65
+    n = 32 * sum(blocks)
+    q, K, V = synth.make_qkv(1, Hkv, Hkv, n + residual, D, 43)
+    far = [0, 1, 2, 3, 40, *range(n, n + 8), n + 64]   # (the residual's last token is alone in its tile)
+    K[:, :, far] = (-30000.0 * q.sign()).half()   # scores of -30000 |q|_1: three million
+    far += list(range(32 * 4, 32 * 12))           # and a whole class: tiles without a finite score
+    K[:, :, 32 * 4:32 * 12] = (-30000.0 * q.sign()).half()
+    classes, at = {}, 0
+    for bits, c in zip((16, 8, 4, 2, 1), blocks):
+        classes[bits] = torch.arange(32 * at, 32 * (at + c))
+        at += c
+    q = q.repeat_interleave(n_rep, 1)
+    pkv = synth.build_cache(K, V, classes, residual, O.uniform_group_quantize_pack_last_dim)
+    w_ref, o_ref = O.qkv_matmul(q, pkv, None, D, use_mask=False, round_per_class=False)
+    big = tuple(x.repeat(B, 1, 1, 1) if torch.is_tensor(x) and x.dim() == 4 else x for x in synth.cache_to(pkv, dev))
+    w, o = decode_attention(q.to(dev).repeat(B, 1, 1, 1), big, None, n + residual, zero_init=False, flags=1 | _lib.qk_tiling(tiling))
+    assert not w[..., far].any()
+    torch.testing.assert_close(w[-1:].float().cpu(), w_ref.float(), rtol=RTOL, atol=ATOL)
+    torch.testing.assert_close(o[-1:].float().cpu(), o_ref.float(), rtol=RTOL, atol=ATOL)
