@@ -38,12 +38,40 @@ struct QtLds {
   __device__ __forceinline__ float *part(int wave, int head) { return reinterpret_cast<float *>(bytes[wave]) + head * HP * 64; }
 };
 
+// One score element by element.  Tokens of different bands share an accumulator, with zeros in the others' rows of A: a key
+// that is not finite (or overflows in its group's scale) makes 0 x inf = NaN of up to three other tokens' sums.  A tile
+// with a NaN among its sums -- never, in a cache of numbers -- takes those scores again here, each token to itself.  The
+// test is one addition per score; a select per lane after products without bands would cost four times the accumulators.
+template <int BITS, bool NORMAL, bool ROWS>
+__device__ __forceinline__ float qk_alone(const SegDev &sg, int bh, uint32_t token, const half_t *q) {
+  const uint32_t n_tok = (uint32_t)sg.n_tokens;
+  float sum = 0.f;
+#pragma unroll 1
+  for (int c = 0; c < 128; ++c) {
+    half_t x;
+    const int64_t row = (int64_t)bh * 128 + c;
+    if constexpr (ROWS) {
+      x = gload<half_t>((const half_t *)sg.data + (int64_t)bh * sg.slab_tokens * 128, token * 256u + 2u * c);
+    } else if constexpr (BITS == 16) {
+      x = gload<half_t>((const half_t *)sg.data + row * n_tok, token * 2u);
+    } else {
+      const uint8_t byte = gload<uint8_t>((const char *)sg.data + row * (n_tok * BITS / 8), token * BITS / 8);
+      const half_t code = (half_t)(unsigned short)((byte >> (token * BITS & 7)) & ((1 << BITS) - 1));
+      const int64_t g = row * (n_tok / 32) + token / 32;
+      const half2_t c2 = {code, code}, s2 = {sg.scale[g], sg.scale[g]}, z2 = {sg.zero[g], sg.zero[g]};
+      x = (NORMAL ? dequant_pair_normal1(c2, normal1_spread(s2), z2) : dequant_pair(c2, s2, z2))[0];
+    }
+    sum += (float)x * (float)gload<half_t>(q, 2u * c);
+  }
+  return sum;
+}
+
 // The end of a tile: the partial sums of this wave's head are added up in order, rounded, scaled, stored, and turned into
 // the lane's (max, sum exp).  `pos(t)`: position of the lane's token t, the first `n_valid` of which exist; `run`: they
-// are consecutive.
-template <int HP, bool FUSED, int TPV, typename Pos>
+// are consecutive; `alone(t)`: its score once more.
+template <int HP, bool FUSED, int TPV, typename Pos, typename Alone>
 __device__ __forceinline__ void qt_finish_tile(QtLds<HP> &lds, const f4_t (&acc)[TPV], int wave, int lane, Pos &&pos, int n_valid, bool run,
-                                               half_t *row, float inv_sqrt_d, float &m_lane, float &l_lane) {
+                                               half_t *row, float inv_sqrt_d, float &m_lane, float &l_lane, Alone &&alone) {
   constexpr int P = TPV < 4 ? TPV : 4;   // tokens side by side
 #pragma unroll
   for (int h = 0; h < 4; ++h)
@@ -51,11 +79,27 @@ __device__ __forceinline__ void qt_finish_tile(QtLds<HP> &lds, const f4_t (&acc)
     for (int t = 0; t < TPV; ++t) lds.part(wave, h)[(t / P) * 64 * P + lane * P + t % P] = acc[t][h];
   __syncthreads();
   half_t x[TPV];
-  float m = SM_FLOOR;
+  float m = SM_FLOOR, sum[TPV], all = 0.f;
 #pragma unroll
   for (int t = 0; t < TPV; ++t) {
     const int at = (t / P) * 64 * P + lane * P + t % P;
-    x[t] = (half_t)(((lds.part(0, wave)[at] + lds.part(1, wave)[at]) + lds.part(2, wave)[at]) + lds.part(3, wave)[at]);
+    sum[t] = ((lds.part(0, wave)[at] + lds.part(1, wave)[at]) + lds.part(2, wave)[at]) + lds.part(3, wave)[at];
+    all += sum[t];
+  }
+  if (HP < 16 && __builtin_expect(__builtin_amdgcn_ballot_w64(all != all && n_valid > 0) != 0, 0)) {
+#pragma unroll 1
+    for (int t = 0; t < n_valid; ++t) {
+      bool bad = false;
+#pragma unroll
+      for (int k = 0; k < TPV; ++k) bad = bad || (k == t && sum[k] != sum[k]);
+      const float again = bad ? alone(t) : 0.f;
+#pragma unroll
+      for (int k = 0; k < TPV; ++k) sum[k] = k == t && bad ? again : sum[k];
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < TPV; ++t) {
+    x[t] = (half_t)sum[t];
     if (FUSED) {   // the fp16 steps of the reference epilogue: round the score, scale, round again
       x[t] = (half_t)((float)x[t] * inv_sqrt_d);
       m = fmaxf(m, t < n_valid ? (float)x[t] : SM_FLOOR);
@@ -81,9 +125,9 @@ __device__ __forceinline__ void qt_finish_tile(QtLds<HP> &lds, const f4_t (&acc)
   }
 }
 
-template <int BITS, int HP, bool FUSED, bool NORMAL>
+template <int BITS, int HP, bool FUSED, bool NORMAL, typename QueryRow>
 __device__ __forceinline__ void qt_class_tile(const SegDev &sg, int tile, int bh, int n_bh, int wave, int lane, u32x4 q, QtLds<HP> &lds,
-                                              half_t *row, bool has_head, float inv_sqrt_d, float &m, float &l) {
+                                              half_t *row, bool has_head, float inv_sqrt_d, float &m, float &l, QueryRow &&qrow) {
   using G = QtGeom<BITS>;
   constexpr bool QUANT = BITS != 16;
   constexpr int BANDS = 16 / HP, TPV = G::TOK / BANDS > 0 ? G::TOK / BANDS : 1;   // tokens a lane ends up with = accumulators
@@ -177,16 +221,16 @@ __device__ __forceinline__ void qt_class_tile(const SegDev &sg, int tile, int bh
     }
   });
   qt_finish_tile<HP, FUSED, TPV>(lds, acc, wave, lane, [&](int t) { return runs ? position.of(tok0c, index0) + t : position(tok0 + t); }, n_valid,
-                                 runs, row, inv_sqrt_d, m, l);
+                                 runs, row, inv_sqrt_d, m, l, [&](int t) { return qk_alone<BITS, NORMAL, false>(sg, bh, tok0 + t, qrow()); });
 }
 
 // fp16 K rows stored token by token (the residual, a step's own key): four blocks of 16 tokens; lane l reads 16 bytes of
 // token l % 16 of every block -- already a B operand.
 constexpr int QT_TM_TILE = 64;
 
-template <int HP, bool FUSED>
+template <int HP, bool FUSED, typename QueryRow>
 __device__ __forceinline__ void qt_rows_tile(const SegDev &sg, int tile, int bh, int wave, int lane, u32x4 q, QtLds<HP> &lds, half_t *row,
-                                             bool has_head, float inv_sqrt_d, float &m, float &l) {
+                                             bool has_head, float inv_sqrt_d, float &m, float &l, QueryRow &&qrow) {
   constexpr int BANDS = 16 / HP, TPV = 4 / BANDS;
   const int n = lane & 15, r = lane >> 4;
   const uint32_t n_tok = (uint32_t)sg.n_tokens;
@@ -211,11 +255,12 @@ __device__ __forceinline__ void qt_rows_tile(const SegDev &sg, int tile, int bh,
     for (int i = 0; i < 4; ++i) a[i] = BANDS == 1 || n / HP == K / TPV ? q[i] : 0u;
     acc[K % TPV] = mfma16(a, x[K], acc[K % TPV]);
   });
-  qt_finish_tile<HP, FUSED, TPV>(lds, acc, wave, lane, [&](int t) { return position(token(t)); }, n_valid, false, row, inv_sqrt_d, m, l);
+  qt_finish_tile<HP, FUSED, TPV>(lds, acc, wave, lane, [&](int t) { return position(token(t)); }, n_valid, false, row, inv_sqrt_d, m, l,
+                                 [&](int t) { return qk_alone<16, false, true>(sg, bh, token(t), qrow()); });
 }
 
 template <int HP, bool FUSED>
-__global__ __launch_bounds__(QT_WAVES * 64, HP == 4 ? 5 : HP == 8 ? 4 : 2) void qk_tiles_kernel(SegTable tb, const half_t *__restrict__ q,
+__global__ __launch_bounds__(QT_WAVES * 64, HP == 16 ? 2 : HP == 4 || FUSED ? 5 : 4) void qk_tiles_kernel(SegTable tb, const half_t *__restrict__ q,
                                                                     half_t *__restrict__ scores, TilesArgs ta, int64_t Tall, FuseArgs fz) {
   __shared__ __align__(16) QtLds<HP> lds;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -235,8 +280,9 @@ __global__ __launch_bounds__(QT_WAVES * 64, HP == 4 ? 5 : HP == 8 ? 4 : 2) void 
   const int head = (4 * r) % HP + wave;   // the head this lane finishes
   const bool has_head = head < nrep;
   half_t *row = scores + ((int64_t)b * Hq + head0 + min(head, nrep - 1)) * Tall;
+  auto qrow = [&]() { return q + ((int64_t)b * Hq + head0 + min((4 * (lane >> 4)) % HP + wave, nrep - 1)) * 128; };
   float m = SM_FLOOR, l = 0.f;
-#define HQ_TILE(B_, NORMAL_) qt_class_tile<B_, HP, FUSED, NORMAL_>(sg, tile, bh, ta.n_bh, wave, lane, qv, lds, row, has_head, fz.inv_sqrt_d, m, l)
+#define HQ_TILE(B_, NORMAL_) qt_class_tile<B_, HP, FUSED, NORMAL_>(sg, tile, bh, ta.n_bh, wave, lane, qv, lds, row, has_head, fz.inv_sqrt_d, m, l, qrow)
   switch (sg.bits) {
     case 1:
       if ((sg.layout & 3) == HQEKV_LAYOUT_NORMAL1) HQ_TILE(1, true);
@@ -246,7 +292,7 @@ __global__ __launch_bounds__(QT_WAVES * 64, HP == 4 ? 5 : HP == 8 ? 4 : 2) void 
     case 4: HQ_TILE(4, false); break;
     case 8: HQ_TILE(8, false); break;
     default:
-      if ((sg.layout & 3) == HQEKV_LAYOUT_TOKEN_MAJOR) qt_rows_tile<HP, FUSED>(sg, tile, bh, wave, lane, qv, lds, row, has_head, fz.inv_sqrt_d, m, l);
+      if ((sg.layout & 3) == HQEKV_LAYOUT_TOKEN_MAJOR) qt_rows_tile<HP, FUSED>(sg, tile, bh, wave, lane, qv, lds, row, has_head, fz.inv_sqrt_d, m, l, qrow);
       else HQ_TILE(16, false);
   }
 #undef HQ_TILE
@@ -283,9 +329,26 @@ constexpr int64_t QT_LONG = 8192;                // one-tile workgroups of a lau
 constexpr int QL_NG = QL_TILES * QT_NG;          // 32-token groups
 constexpr int QL_NGP = QL_NG + 2;                // LDS row of a channel pair: the four lane groups of a read meet different banks
 
-template <int BITS, int HP, bool FUSED, int TPV, typename Pos>
-__device__ __forceinline__ void ql_finish(const f4_t (&acc)[TPV], int r, Pos &&pos, int n_valid, bool run, half_t *rows, int64_t Tall, int nrep,
-                                          float inv_sqrt_d, float (&m)[4], float (&l)[4]) {
+template <int BITS, int HP, bool FUSED, int TPV, typename Pos, typename Alone>
+__device__ __forceinline__ void ql_finish(f4_t (&acc)[TPV], int r, Pos &&pos, int n_valid, bool run, half_t *rows, int64_t Tall, int nrep,
+                                          float inv_sqrt_d, float (&m)[4], float (&l)[4], Alone &&alone) {
+  if constexpr (HP < 16) {   // a NaN among the sums: see qk_alone
+    f4_t all = acc[0];
+#pragma unroll
+    for (int t = 1; t < TPV; ++t) all += acc[t];
+    const float any = (all[0] + all[1]) + (all[2] + all[3]);
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(any != any && n_valid > 0) != 0, 0)) {
+#pragma unroll 1
+      for (int e = 0; e < 4 * n_valid; ++e) {
+        bool bad = false;
+#pragma unroll
+        for (int k = 0; k < 4 * TPV; ++k) bad = bad || (k == e && acc[k / 4][k % 4] != acc[k / 4][k % 4]);
+        const float again = bad ? alone(min((4 * r) % HP + e % 4, nrep - 1), e / 4) : 0.f;
+#pragma unroll
+        for (int k = 0; k < 4 * TPV; ++k) acc[k / 4][k % 4] = k == e && bad ? again : acc[k / 4][k % 4];
+      }
+    }
+  }
 #pragma unroll
   for (int h = 0; h < 4; ++h) {
     const int head = (4 * r) % HP + h;
@@ -324,7 +387,7 @@ __device__ __forceinline__ void ql_finish(const f4_t (&acc)[TPV], int r, Pos &&p
 
 template <int BITS, int HP, bool FUSED, bool NORMAL>
 __device__ __forceinline__ void ql_class(const SegDev &sg, int unit, int bh, int n_bh, int wave, int lane, const half_t *qrow, uint2 *sz, half_t *rows,
-                                         int64_t Tall, int nrep, float inv_sqrt_d, float (&m)[4], float (&l)[4]) {
+                                         int64_t Tall, int nrep, float inv_sqrt_d, float (&m)[4], float (&l)[4], const half_t *q0) {
   using G = QtGeom<BITS>;
   constexpr bool QUANT = BITS != 16;
   constexpr int BANDS = 16 / HP, TPV = G::TOK / BANDS > 0 ? G::TOK / BANDS : 1;
@@ -442,13 +505,13 @@ __device__ __forceinline__ void ql_class(const SegDev &sg, int unit, int bh, int
     if constexpr (C + NB < 4) load_codes(C + NB, cur[C % NB]);
   });
   ql_finish<BITS, HP, FUSED, TPV>(acc, r, [&](int t) { return runs ? position.of(tok0c, index0) + t : position(tok0 + t); }, n_valid, runs, rows, Tall,
-                                  nrep, inv_sqrt_d, m, l);
+                                  nrep, inv_sqrt_d, m, l, [&](int head, int t) { return qk_alone<BITS, NORMAL, false>(sg, bh, tok0 + t, q0 + head * 128); });
 }
 
 // fp16 K rows stored token by token: a wave takes the 64 tokens of one tile, 32 channels at a time
 template <int HP, bool FUSED>
 __device__ __forceinline__ void ql_rows(const SegDev &sg, int unit, int bh, int wave, int lane, const half_t *qrow, half_t *rows, int64_t Tall, int nrep,
-                                        float inv_sqrt_d, float (&m)[4], float (&l)[4]) {
+                                        float inv_sqrt_d, float (&m)[4], float (&l)[4], const half_t *q0) {
   constexpr int BANDS = 16 / HP, TPV = 4 / BANDS;
   const int n = lane & 15, r = lane >> 4;
   const uint32_t n_tok = (uint32_t)sg.n_tokens, t0 = ((uint32_t)unit * QL_TILES + wave) * QT_TM_TILE;
@@ -478,7 +541,8 @@ __device__ __forceinline__ void ql_rows(const SegDev &sg, int unit, int bh, int 
   int n_valid = 0;
 #pragma unroll
   for (int t = 0; t < TPV; ++t) n_valid += token(t) < n_tok ? 1 : 0;
-  ql_finish<16, HP, FUSED, TPV>(acc, r, [&](int t) { return position(token(t)); }, n_valid, false, rows, Tall, nrep, inv_sqrt_d, m, l);
+  ql_finish<16, HP, FUSED, TPV>(acc, r, [&](int t) { return position(token(t)); }, n_valid, false, rows, Tall, nrep, inv_sqrt_d, m, l,
+                           [&](int head, int t) { return qk_alone<16, false, true>(sg, bh, token(t), q0 + head * 128); });
 }
 
 template <int HP, bool FUSED>
@@ -492,7 +556,7 @@ __global__ __launch_bounds__(QT_WAVES * 64, HP == 4 ? 4 : 2) void qk_long_kernel
   const int b = tiles_batch_row(ta, bh), hkv = bh - b * ta.Hkv;
   const int Hq = ta.hq_slice & 0xffff, head0 = first_head(ta.hq_slice, hkv), nrep = ta.nrep;
   const int n = lane & 15, r = lane >> 4, unit = u - sg.unit_begin;
-  const half_t *qrow = q + ((int64_t)b * Hq + head0 + min(n % HP, nrep - 1)) * 128;
+  const half_t *q0 = q + ((int64_t)b * Hq + head0) * 128, *qrow = q0 + min(n % HP, nrep - 1) * 128;
   half_t *rows = scores + ((int64_t)b * Hq + head0) * Tall;
   float m[4], l[4];
 #pragma unroll
@@ -500,7 +564,7 @@ __global__ __launch_bounds__(QT_WAVES * 64, HP == 4 ? 4 : 2) void qk_long_kernel
     m[h] = SM_FLOOR;
     l[h] = 0.f;
   }
-#define HQ_TILE(B_, NORMAL_) ql_class<B_, HP, FUSED, NORMAL_>(sg, unit, bh, ta.n_bh, wave, lane, qrow, sz, rows, Tall, nrep, fz.inv_sqrt_d, m, l)
+#define HQ_TILE(B_, NORMAL_) ql_class<B_, HP, FUSED, NORMAL_>(sg, unit, bh, ta.n_bh, wave, lane, qrow, sz, rows, Tall, nrep, fz.inv_sqrt_d, m, l, q0)
   switch (sg.bits) {
     case 1:
       if ((sg.layout & 3) == HQEKV_LAYOUT_NORMAL1) HQ_TILE(1, true);
@@ -510,7 +574,7 @@ __global__ __launch_bounds__(QT_WAVES * 64, HP == 4 ? 4 : 2) void qk_long_kernel
     case 4: HQ_TILE(4, false); break;
     case 8: HQ_TILE(8, false); break;
     default:
-      if ((sg.layout & 3) == HQEKV_LAYOUT_TOKEN_MAJOR) ql_rows<HP, FUSED>(sg, unit, bh, wave, lane, qrow, rows, Tall, nrep, fz.inv_sqrt_d, m, l);
+      if ((sg.layout & 3) == HQEKV_LAYOUT_TOKEN_MAJOR) ql_rows<HP, FUSED>(sg, unit, bh, wave, lane, qrow, rows, Tall, nrep, fz.inv_sqrt_d, m, l, q0);
       else HQ_TILE(16, false);
   }
 #undef HQ_TILE

@@ -10,7 +10,8 @@
 // With fewer than 16 heads the spare rows of A are put to use in q.K^T: A is laid out HP heads (4, 8 or 16) to a "band"
 // of rows, and the operand for token i of a packed word has only band i / (tokens per band) filled.  Products of different
 // bands then share one accumulator, every lane ends up with the scores of its own tokens, and four heads need a quarter
-// of the accumulators (and leave all 64 lanes busy in the softmax statistics instead of 16).
+// of the accumulators (and leave all 64 lanes busy in the softmax statistics instead of 16).  A key that is not a number
+// or not finite reaches the other bands' tokens through the zeros: such scores are taken again (qk_alone, decode_qk.hip).
 #pragma once
 
 #include "attn_common.h"

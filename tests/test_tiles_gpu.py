@@ -114,3 +114,59 @@ def test_a_score_of_minus_infinity_has_probability_zero(dev, n_rep, B, tiling):
     assert not w[..., far].any()
     torch.testing.assert_close(w[-1:].float().cpu(), w_ref.float(), rtol=RTOL, atol=ATOL)
     torch.testing.assert_close(o[-1:].float().cpu(), o_ref.float(), rtol=RTOL, atol=ATOL)
+
+
+def _bad_cache(n_rep, value):
+    """Every class and a residual, some keys of each not finite: an element of the fp16 rows, the scale of a quantised group."""
+    Hkv, D, blocks, residual = 2, 128, (5, 9, 9, 9, 9), 33
+    n = 32 * sum(blocks)
+    q, K, V = synth.make_qkv(1, n_rep * Hkv, Hkv, n + residual, D, 41)
+    classes, at = {}, 0
+    for bits, c in zip((16, 8, 4, 2, 1), blocks):
+        classes[bits] = torch.arange(32 * at, 32 * (at + c))
+        at += c
+    pkv = synth.build_cache(K, V, classes, residual, O.uniform_group_quantize_pack_last_dim)
+    for h, d, t in ((0, 3, 0), (0, 70, 37), (1, 127, 159)):
+        pkv[0][0, h, d, t] = value                      # fp16 class (B, H, D, T)
+    for h, t, d in ((0, 3, 9), (1, 0, 64), (1, 32, 5)):   # (32: the last one, which the unused rows of its tile repeat)
+        pkv[39][0, h, t, d] = value                     # residual (B, H, T, D)
+    for base in (4, 12, 20, 28):
+        pkv[base + 2][0, 0, 17, 0] = value              # a group's scale
+        pkv[base + 2][0, 1, 99, 8] = value
+    return q, pkv
+
+
+@pytest.mark.parametrize("n_rep", [1, 4, 5, 12])
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+@pytest.mark.parametrize("B", [1, 400], ids=["one-tile", "four-tiles"])
+def test_a_key_that_is_not_finite_stays_with_its_token(dev, n_rep, value, B):
+    """Raw scores: infinities and NaN exactly where the definition has them, every other token's score as it is."""
+    from hqekv_amd.attention import DecodePlan
+    q, pkv = _bad_cache(n_rep, value)
+    K = O.reconstruct_cache(pkv, "uniform_group")[0]
+    want = (q.view(1, 2, n_rep, 1, 128).double() * K[:, :, None].double()).sum(-1).view(1, 2 * n_rep, 1, -1)
+    big = tuple(x.repeat(B, 1, 1, 1) if torch.is_tensor(x) and x.dim() == 4 else x for x in synth.cache_to(pkv, dev))
+    plan = DecodePlan(q.to(dev).repeat(B, 1, 1, 1), big)
+    plan.run_qk(q.to(dev).repeat(B, 1, 1, 1))
+    got = plan.weights.cpu()
+    assert torch.equal(got.view(torch.int16), got[:1].expand_as(got).contiguous().view(torch.int16))
+    # scores are a few hundred at the most, rounded to fp16 once; fp32 sums of 128 products move them by a place
+    torch.testing.assert_close(got[:1].double(), want.half().double(), rtol=2e-3, atol=2e-3, equal_nan=True)
+
+
+@pytest.mark.parametrize("n_rep", [4, 5])
+def test_a_masked_slot_that_holds_no_number(dev, n_rep):
+    """Slots whose keys are NaN, masked out: the probabilities of all others are what they are without them."""
+    from hqekv_amd.attention import decode_attention
+    q, pkv = _bad_cache(n_rep, float("nan"))
+    pkv = [x.clone() if torch.is_tensor(x) else x for x in pkv]
+    bad = torch.isnan(O.reconstruct_cache(tuple(pkv), "uniform_group")[0]).any(-1).any(0).any(0)
+    mask = torch.zeros(1, 1, 1, int(pkv[41]), dtype=torch.float16)
+    mask[..., bad] = torch.finfo(torch.float16).min
+    w, o = decode_attention(q.to(dev), synth.cache_to(tuple(pkv), dev), mask.to(dev), int(pkv[41]), zero_init=False)
+    for i, x in enumerate(pkv[:41]):
+        if torch.is_tensor(x) and x.dtype == torch.float16:
+            x[torch.isnan(x)] = 0
+    w_ref, o_ref = O.qkv_matmul(q, tuple(pkv), mask, 128, round_per_class=False)
+    torch.testing.assert_close(w.float().cpu(), w_ref.float(), rtol=RTOL, atol=ATOL)
+    torch.testing.assert_close(o.float().cpu(), o_ref.float(), rtol=RTOL, atol=ATOL)
