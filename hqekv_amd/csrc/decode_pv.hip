@@ -145,6 +145,13 @@ __device__ __forceinline__ void pt_class_job(const SegDev &sg, int blk0, int blk
         v[2 * g] = (g & 1) ? as_u32(half_pair<1>(sa[g >> 1], sb[g >> 1])) : as_u32(half_pair<0>(sa[g >> 1], sb[g >> 1]));
         v[2 * g + 1] = (g & 1) ? as_u32(half_pair<1>(za[g >> 1], zb[g >> 1])) : as_u32(half_pair<0>(za[g >> 1], zb[g >> 1]));
       }
+      // Tokens past the end hold the last row's codes and probability zero; with scale and zero point zero too they are
+      // zeros, where an infinity in the last row would be 0 x inf.
+      if ((uint32_t)(blk + 1) * BLOCK > n_tok) {
+        const uint32_t left = n_tok - min((uint32_t)blk * BLOCK + 2u * tid, n_tok), mask = (left > 0 ? 0xffffu : 0u) | (left > 1 ? 0xffff0000u : 0u);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] &= mask;
+      }
       uint4 *dst = reinterpret_cast<uint4 *>(lds.sz[buf][tid]);
       dst[0] = make_uint4(v[0], v[1], v[2], v[3]);
       dst[1] = make_uint4(v[4], v[5], v[6], v[7]);
@@ -175,6 +182,15 @@ __device__ __forceinline__ void pt_class_job(const SegDev &sg, int blk0, int blk
       fetch_scales(blk + 1);
     }
     HQ_LOADS_ABOVE();
+    if (!QUANT && (uint32_t)(blk + 1) * BLOCK > n_tok) {   // (rows past the end: zeros, as commit() makes of codes)
+#pragma unroll
+      for (int s = 0; s < STEPS; ++s)
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+#pragma unroll
+          for (int k = 0; k < WPL; ++k)
+            cur[s][i][k] = (uint32_t)blk * BLOCK + (uint32_t)((wave * STEPS + s) * 32 + 8 * r + i) < n_tok ? cur[s][i][k] : 0u;
+    }
 #pragma unroll
     for (int s = 0; s < STEPS; ++s) {
       const int t = (wave * STEPS + s) * 32 + 8 * r;   // this lane's first token of the step, inside the block

@@ -170,3 +170,40 @@ def test_a_masked_slot_that_holds_no_number(dev, n_rep):
     w_ref, o_ref = O.qkv_matmul(q, tuple(pkv), mask, 128, round_per_class=False)
     torch.testing.assert_close(w.float().cpu(), w_ref.float(), rtol=RTOL, atol=ATOL)
     torch.testing.assert_close(o.float().cpu(), o_ref.float(), rtol=RTOL, atol=ATOL)
+
+
+@pytest.mark.parametrize("n_rep,residual", [(4, 33), (5, 2), (12, 1)])
+@pytest.mark.parametrize("fused", [True, False], ids=["fused", "general"])
+def test_a_value_row_that_is_not_finite(dev, n_rep, residual, fused):
+    """The last row of every V class holds an infinity (which the unused rows of its block repeat): the outputs are the
+    infinities of the definition, not NaN."""
+    from hqekv_amd.attention import decode_attention
+    Hkv, D, sizes = 2, 128, (45, 33, 31, 70, 5)
+    n = sum(sizes)
+    g = torch.Generator().manual_seed(3)
+    q, K, V = synth.make_qkv(1, n_rep * Hkv, Hkv, n + residual, D, 44)
+    q = q * 0.05                                  # (every probability above fp16's smallest)
+    pkv = [None] * 42
+    pkv[0], pkv[1] = K[:, :, :n].transpose(2, 3).contiguous(), torch.arange(n)   # K: one fp16 class
+    perm, at = torch.randperm(n, generator=g), 0
+    for bits, slot, c in zip((16, 8, 4, 2, 1), (2, 8, 16, 24, 32), sizes):
+        pos = perm[at:at + c]
+        rows = V[:, :, pos].contiguous()
+        if bits == 16:
+            rows[:, :, -1, 7] = float("inf")
+            pkv[2], pkv[3] = rows, pos
+        else:
+            code, scale, zero = O.uniform_group_quantize_pack_last_dim(rows, 32, bits)
+            zero[:, :, -1, 2] = float("inf")
+            pkv[slot], pkv[slot + 1], pkv[slot + 2], pkv[slot + 3] = code, pos, scale, zero
+        at += c
+    pkv[39], pkv[40] = K[:, :, n:].contiguous(), V[:, :, n:].contiguous()
+    pkv[40][:, :, -1, 20] = float("inf")
+    pkv[41] = n + residual
+    pkv = tuple(pkv)
+    w, o = decode_attention(q.to(dev), synth.cache_to(pkv, dev), None, n + residual, zero_init=False, flags=1 if fused else 0)
+    assert float(w.min()) > 0
+    dense = O.reconstruct_cache(pkv, "uniform_group")[1].double()
+    want = torch.matmul(w.cpu().double().view(1, Hkv, n_rep, -1), dense).view(1, n_rep * Hkv, 1, D)
+    assert torch.isinf(want).any()
+    torch.testing.assert_close(o.cpu().double(), want.half().double(), rtol=RTOL, atol=ATOL, equal_nan=True)
