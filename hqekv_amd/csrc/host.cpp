@@ -627,11 +627,11 @@ PyObject *quantize_into(PyObject *, PyObject *const *a, Py_ssize_t na) {
   }
   if (sc.stride(1) != mn.stride(1) || sc.stride(2) != mn.stride(2) || sc.stride(0) != mn.stride(0)) Py_RETURN_NONE;
   // read in place: equally spaced (b, h) slabs of dense rows -- or, seen transposed, of dense token rows: the head of a
-  // longer tensor is not copied
-  const int64_t slab = x.stride(1);
-  if ((B > 1 && x.stride(0) != H * slab) || (H > 1 && slab < R * L)) Py_RETURN_NONE;
+  // longer tensor is not copied (the stride of a dimension of one element says nothing: it is not looked at)
+  const int64_t slab = H > 1 ? x.stride(1) : B > 1 ? x.stride(0) : R * L;
+  if ((B > 1 && H > 1 && x.stride(0) != H * slab) || slab < R * L) Py_RETURN_NONE;
   const bool token_major = x.stride(2) == 1 && x.stride(3) == R && R % 2 == 0 && R > 1 && slab % 2 == 0 && (uintptr_t)x.data_ptr() % 4 == 0;
-  const bool rows = x.stride(3) == 1 && x.stride(2) == L && slab % 8 == 0 && (uintptr_t)x.data_ptr() % 16 == 0;
+  const bool rows = x.stride(3) == 1 && (R == 1 || x.stride(2) == L) && slab % 8 == 0 && (uintptr_t)x.data_ptr() % 16 == 0;
   if (!token_major && !rows) Py_RETURN_NONE;
   const c10::OptionalDeviceGuard guard(dev);
   const int rc = token_major ? api.hqekv_quant_pack_k_tokenmajor(x.data_ptr(), slab, R, code.data_ptr(), code.stride(1), code.stride(2),

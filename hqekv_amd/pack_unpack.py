@@ -121,8 +121,13 @@ def quantize_pack_into(
             raise ValueError("outputs need a unit last stride and a flattenable (B, nh) prefix")
     if scale.stride() != mn.stride():
         raise ValueError("scale and mn must share strides")
-    if _lib.host().quantize_into(data.contiguous(), bit, code, scale, mn) is None:
+    if any(t.device != data.device for t in (code, scale, mn)):
         raise ValueError("the outputs must live on the input's device")
+    data = data.contiguous()
+    with _lib.on_device(data.device):
+        _lib.check(_lib.load().hqekv_quant_pack_rows(
+            data.data_ptr(), R * L, L, code.data_ptr(), code.stride(1), code.stride(2), scale.data_ptr(), mn.data_ptr(),
+            scale.stride(1), scale.stride(2), B * nh, R, L, bit, _lib.stream_ptr(data.device)), "uniform_group_quantize_pack_last_dim")
 
 
 def uniform_group_quantize_pack_last_dim(

@@ -363,3 +363,31 @@ def test_dequant_keeps_the_sign_of_zero_products(dev):
     assert torch.equal(torch.isnan(out), nan)
     assert torch.equal(out[~nan].view(torch.int16), ref[~nan].view(torch.int16))
     assert bool((out[0, 0, 0, 32 + 16:64].view(torch.int16) == -32768).all())   # std +0, mean -0, code 0  ->  -0
+
+
+@pytest.mark.parametrize("B,H,R", [(2, 1, 64), (1, 1, 64), (3, 1, 1), (1, 4, 1), (1, 3, 64)])
+@pytest.mark.parametrize("transposed", [False, True], ids=["V", "K"])
+def test_quant_takes_projection_views(dev, B, H, R, transposed):
+    """(B, T, H, 128) seen per head -- contiguous for torch with strides of its own where a dimension has one element --
+    and the head of a longer tensor, as V rows and as the transposed view of K."""
+    from hqekv_amd.pack_unpack import uniform_group_quantize_pack_last_dim
+    x = _data((B, R, H, 128), 31)
+    for src in (x.to(dev).transpose(1, 2), torch.cat((x, x), 1).to(dev).transpose(1, 2)[:, :, :R]):
+        view = src.transpose(2, 3) if transposed else src
+        if view.shape[3] % 32:
+            continue
+        want = O.uniform_group_quantize_pack_last_dim(x.transpose(1, 2).transpose(2, 3).contiguous() if transposed else x.transpose(1, 2).contiguous(), 32, 4)
+        for g, w in zip(uniform_group_quantize_pack_last_dim(view, 32, 4), want):
+            assert torch.equal(g.cpu(), w)
+
+
+def test_quant_names_the_alignment_of_its_input(dev):
+    from hqekv_amd.pack_unpack import uniform_group_quantize_pack_last_dim
+    x = torch.zeros(2 * 32 * 128 + 8, dtype=torch.float16, device=dev)[1:2 * 32 * 128 + 1].view(1, 2, 32, 128)
+    with pytest.raises(ValueError, match="align"):
+        uniform_group_quantize_pack_last_dim(x, 32, 4)
+    code = torch.empty(1, 2, 32, 16, dtype=torch.int32)
+    scale = torch.empty(1, 2, 32, 4, dtype=torch.float16)
+    with pytest.raises((ValueError, RuntimeError)):
+        from hqekv_amd.pack_unpack import quantize_pack_into
+        quantize_pack_into(torch.zeros(1, 2, 32, 128, dtype=torch.float16, device=dev), 4, code, scale, scale.clone())
