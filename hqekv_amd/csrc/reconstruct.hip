@@ -10,6 +10,8 @@
 // stay aligned.  34 KB of LDS: four workgroups per CU.
 // Measured at B=1, 16k tokens of the fp16 / 8 / 4 / 2-bit mix (73 MB): 258 us as dequantise launches, transposing copies
 // and index_put scatters; this launch 21 us (3.4 TB/s), 38 us with the host call around it.
+#include <algorithm>
+
 #include "common.h"
 #include "quant_math.h"
 
@@ -32,13 +34,14 @@ struct RcSeg {
 constexpr int RC_SEGS = 2 * HQEKV_MAX_SEGS;
 struct RcTable {
   RcSeg seg[RC_SEGS];
-  int32_t begin[RC_SEGS];   // first tile (grid.y) of every segment; INT32_MAX past the last
+  int32_t begin[RC_SEGS];   // first tile of every segment, counted from grid.y = 0 of the launch; INT32_MAX past the last
 };
 
 constexpr int RC_THREADS = 256;
 constexpr int RC_TOK = 128;    // tokens per workgroup
 constexpr int RC_CH = 128;     // channels turned in LDS at a time
 constexpr int RC_ROW = 68;     // 32-bit words per token row in LDS
+constexpr int64_t RC_GRID_Y = 65535;
 
 // where token t of the segment goes; -1: outside the dense tensor (an index counts from the end when negative, as in
 // torch; one that names no row is dropped)
@@ -283,10 +286,16 @@ extern "C" int hqekv_cache_reconstruct(const hqekv_seg *k_segs, int n_k, const h
     r.kind = (int16_t)((tm ? 1 : 0) | (s.bits == 1 && (s.layout & 3) == HQEKV_LAYOUT_NORMAL1 ? 2 : 0));
     tb.begin[m++] = (int32_t)tiles;
     tiles += (s.n_tokens + RC_TOK - 1) / RC_TOK;
-    if (tiles > 65535) return fail(HQEKV_E_UNSUPPORTED, "cache_reconstruct: more than 65535 tiles of %d tokens", RC_TOK);
   }
   for (int k = m; k < RC_SEGS; ++k) tb.begin[k] = 0x7fffffff;
-  if (tiles == 0) return HQEKV_OK;
-  hipLaunchKernelGGL(cache_reconstruct_kernel, dim3((unsigned)BH, (unsigned)tiles), dim3(RC_THREADS), 0, (hipStream_t)stream, tb, (int)D, T);
-  return check_launch("cache_reconstruct_kernel");
+  // More tiles than grid.y holds (4.2 million tokens on both sides together): another launch, whose begins are counted from
+  // its first tile.  (At most 16 segments of 2^30 tokens: fewer than 2^28 tiles.)
+  for (int64_t first = 0; first < tiles; first += RC_GRID_Y) {
+    hipLaunchKernelGGL(cache_reconstruct_kernel, dim3((unsigned)BH, (unsigned)std::min(tiles - first, RC_GRID_Y)), dim3(RC_THREADS), 0,
+                       (hipStream_t)stream, tb, (int)D, T);
+    const int rc = check_launch("cache_reconstruct_kernel");
+    if (rc) return rc;
+    for (int k = 0; k < m; ++k) tb.begin[k] -= (int32_t)RC_GRID_Y;
+  }
+  return HQEKV_OK;
 }

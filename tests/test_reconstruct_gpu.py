@@ -65,3 +65,23 @@ def test_cover_check(dev, n):
         q = p.clone()
         q[0] = bad
         assert idx_cover_once(parts(q), n) == (bad == int(p[0]))
+
+
+def test_more_tiles_than_a_grid_dimension_holds(dev):
+    """4.2 million tokens per side: 66000 tiles of 128 for both."""
+    from hqekv_amd import pack_unpack as PU
+    from hqekv_amd.hqe_2 import KV_cache_reconstruct_hqe
+    T, D = 32 * 132000, 32
+    g = torch.Generator(device=dev).manual_seed(3)
+    kc = torch.randint(-2 ** 31, 2 ** 31 - 1, (1, 1, D, T // 16), generator=g, device=dev, dtype=torch.int32)
+    vc = torch.randint(-2 ** 31, 2 ** 31 - 1, (1, 1, T, D // 16), generator=g, device=dev, dtype=torch.int32)
+    ks, kz = (torch.randn(1, 1, D, T // 32, generator=g, device=dev).half() for _ in range(2))
+    vs, vz = (torch.randn(1, 1, T, 1, generator=g, device=dev).half() for _ in range(2))
+    idx = torch.arange(T, device=dev)
+    pkv = [None] * 42
+    pkv[20:24] = kc, idx, ks, kz
+    pkv[24:28] = vc, idx.clone(), vs, vz
+    pkv[41] = T
+    K, V = KV_cache_reconstruct_hqe(tuple(pkv), "uniform_group")
+    assert torch.equal(V, PU.uniform_group_dequantize_unpack_last_dim(vc, vs, vz, 32, 2))
+    assert torch.equal(K, PU.uniform_group_dequantize_unpack_last_dim(kc, ks, kz, 32, 2).transpose(2, 3))
