@@ -732,7 +732,7 @@ def reconstruct(past_key_value: tuple, quant_strategy: str, block_size: int = 32
     for b in CLASS_BITS:
         if b == 1 and (k_side[b].data is not None or v_side[b].data is not None):
             _check_low_bits(1, quant_strategy)
-    if dev.type == "cuda" and D % 32 == 0:
+    if dev.type == "cuda" and D % 32 == 0 and D <= 4096:
         return _reconstruct_on_device(pkv, B, H, T, D, dev, quant_strategy != LOW_NORMAL)
     K = torch.zeros(B, H, T, D, dtype=torch.float16, device=dev)
     V = torch.zeros(B, H, T, D, dtype=torch.float16, device=dev)
@@ -760,6 +760,9 @@ def _reconstruct_on_device(pkv: tuple, B: int, H: int, T: int, D: int, dev, low_
              (A.value_segments(pkv, dev, T, keep, low_uniform)[0], A.V16, A.V_BASE, pkv[A.NEW_V]))
     dense, calls = [], []
     for items, base0, bases, new in sides:
+        for it in items:   # the kernel reads fp16 rows in 16-byte pieces
+            if it["bits"] == 16 and it["data"].data_ptr() % 16:
+                it["data"], it["slab_tokens"] = it["data"].clone(), 0   # (dense, a transposed view stays one)
         idx = A._class_idx(pkv, base0, bases)
         n = T - (new.shape[2] if new is not None else 0)
         whole = n >= 0 and all(t is not None for t in idx) and A.idx_cover_once(idx, n)

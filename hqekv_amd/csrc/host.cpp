@@ -723,8 +723,10 @@ PyObject *reconstruct(PyObject *, PyObject *const *a, Py_ssize_t na) {
   Side k, v;
   const bool low_uniform = a[1] == Py_True;
   if (!read_side(pkv, true, low_uniform, B, dev, k) || !read_side(pkv, false, low_uniform, B, dev, v)) Py_RETURN_NONE;
-  if (k.tokens != T || v.tokens != T || k.H != v.H || k.D != v.D || k.D % 32) Py_RETURN_NONE;
+  if (k.tokens != T || v.tokens != T || k.H != v.H || k.D != v.D || k.D % 32 || k.D > 4096) Py_RETURN_NONE;
   for (Side *s : {&k, &v}) {
+    for (int i = 0; i < s->n; ++i)
+      if (s->seg[i].bits == 16 && (uintptr_t)s->seg[i].data % 16) Py_RETURN_NONE;
     const int c = cover_once(s->idx, s->n_idx, s->class_tokens, a[2], false);
     if (c < 0) return nullptr;
     if (!c) Py_RETURN_NONE;

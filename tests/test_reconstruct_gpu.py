@@ -85,3 +85,21 @@ def test_more_tiles_than_a_grid_dimension_holds(dev):
     K, V = KV_cache_reconstruct_hqe(tuple(pkv), "uniform_group")
     assert torch.equal(V, PU.uniform_group_dequantize_unpack_last_dim(vc, vs, vz, 32, 2))
     assert torch.equal(K, PU.uniform_group_dequantize_unpack_last_dim(kc, ks, kz, 32, 2).transpose(2, 3))
+
+
+@pytest.mark.parametrize("slots", [(0,), ("transposed", 0), (2,), (39, 40), ("window", 39, 40)])
+def test_fp16_planes_at_any_element(dev, slots):
+    """Planes that start at an odd element: dense, K as the transposed view of token-major rows, heads of longer buffers."""
+    pkv = list(_cache(dev, 1, 2, 512, 128, 5, (.2, .2, .2, .2, .2), "uniform_group"))
+    for s in slots[isinstance(slots[0], str):]:
+        x = pkv[s].transpose(2, 3) if slots[0] == "transposed" else pkv[s]
+        rows = x.shape[2] + (3 if slots[0] == "window" else 0)
+        room = torch.empty(x.numel() // x.shape[2] * rows + 1, dtype=torch.float16, device=dev)[1:]
+        room = room.view(*x.shape[:2], rows, x.shape[3])[:, :, :x.shape[2]].copy_(x)
+        pkv[s] = room.transpose(2, 3) if slots[0] == "transposed" else room
+        assert pkv[s].data_ptr() % 16 == 2
+    _check(tuple(pkv), "uniform_group")
+
+
+def test_head_size_beyond_the_kernel(dev):
+    _check(_cache(dev, 1, 1, 64, 4128, 3, (.5, 0, 0, .5, 0), "uniform_group"), "uniform_group")
