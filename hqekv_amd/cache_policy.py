@@ -765,7 +765,13 @@ def _reconstruct_on_device(pkv: tuple, B: int, H: int, T: int, D: int, dev, low_
                 it["data"], it["slab_tokens"] = it["data"].clone(), 0   # (dense, a transposed view stays one)
         idx = A._class_idx(pkv, base0, bases)
         n = T - (new.shape[2] if new is not None else 0)
-        whole = n >= 0 and all(t is not None for t in idx) and A.idx_cover_once(idx, n)
+        if n < 0:
+            raise ValueError("invalid past_key_value: a residual longer than kv_seq_len")
+        whole = all(t is not None for t in idx) and A.idx_cover_once(idx, n)
+        if not whole:   # (asked on the way that waits for the device anyway)
+            out = [((t < -T) | (t >= T)).any() for t in (it["idx"] for it in items) if t is not None]
+            if out and bool(torch.stack(out).any()):
+                raise IndexError(f"a position outside the cache of {T} tokens")
         dense.append((torch.empty if whole else torch.zeros)(B, H, T, D, dtype=torch.float16, device=dev))
         calls.append([items] if whole else [[it] for it in items])
     lib, st = _lib.load(), _lib.stream_ptr(dev)

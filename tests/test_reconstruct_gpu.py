@@ -103,3 +103,20 @@ def test_fp16_planes_at_any_element(dev, slots):
 
 def test_head_size_beyond_the_kernel(dev):
     _check(_cache(dev, 1, 1, 64, 4128, 3, (.5, 0, 0, .5, 0), "uniform_group"), "uniform_group")
+
+
+def test_positions_outside_the_cache(dev):
+    """One that counts from the end is taken, as an index into a tensor is; one that names no row is an error."""
+    from hqekv_amd.hqe_2 import KV_cache_reconstruct_hqe
+    pkv = list(_cache(dev, 1, 2, 512, 128, 5, (.2, .2, .2, .2, .2), "uniform_group"))
+    T = pkv[41]
+    pkv[1] = pkv[1] - T
+    _check(tuple(pkv), "uniform_group")
+    for slot, bad in ((3, T), (13, -T - 1), (25, 2 ** 40)):
+        wrong = list(pkv)
+        wrong[slot] = pkv[slot].clone()
+        wrong[slot][-1] = bad
+        with pytest.raises(IndexError):
+            KV_cache_reconstruct_hqe(tuple(wrong), "uniform_group")
+    with pytest.raises(ValueError):
+        KV_cache_reconstruct_hqe(tuple(pkv[:41]) + (3,), "uniform_group")   # fewer positions than the residual has rows
