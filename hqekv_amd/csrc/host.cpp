@@ -68,6 +68,19 @@ PyObject *raise_rc(int64_t rc, const char *what) {
   return PyErr_Format(PyExc_RuntimeError, "%s: HIP error %lld: %s", what, (long long)rc, msg);
 }
 
+// Other Python threads run while the kernels' library is entered (a launch waits in there when the device's queue is full)
+// and while memory is asked for.  `f` touches nothing of Python's, and no field of an object that a second thread may call
+// into: those are read before it, into copies that keep tensors alive, and written after it.
+struct WithoutGil {
+  PyThreadState *state = PyEval_SaveThread();
+  ~WithoutGil() { PyEval_RestoreThread(state); }
+};
+template <typename F>
+auto without_gil(F &&f) {
+  const WithoutGil others;
+  return f();
+}
+
 // ------------------------------------------------------------------------------------------------ tensors
 bool is_tensor(PyObject *o) { return THPVariable_Check(o); }
 const Tensor &ten(PyObject *o) { return THPVariable_Unpack(o); }
@@ -272,10 +285,14 @@ PyObject *decode(PyObject *, PyObject *const *a, Py_ssize_t na) {
   const c10::OptionalDeviceGuard guard(dev);
   const int64_t need = api.hqekv_decode_workspace_bytes(k.seg, k.n, v.seg, v.n, B, Hq, k.H, D);
   if (need < 0) return PyErr_Format(PyExc_ValueError, "invalid segment table");
-  Tensor weights = new_tensor({B, Hq, 1, Tall}, at::kHalf, dev), out = new_tensor({B, Hq, 1, D}, at::kHalf, dev);
-  Tensor ws = new_tensor({std::max<int64_t>(need, 256)}, at::kByte, dev);
-  const int rc = api.hqekv_decode_attn(k.seg, k.n, v.seg, v.n, q.data_ptr(), nullptr, 0, weights.data_ptr(), out.data_ptr(), B, Hq, k.H, D,
-                                       Tall, ws.data_ptr(), ws.numel(), flags, stream_of(dev));
+  Tensor weights, out;
+  const int rc = without_gil([&] {
+    weights = new_tensor({B, Hq, 1, Tall}, at::kHalf, dev);
+    out = new_tensor({B, Hq, 1, D}, at::kHalf, dev);
+    const Tensor ws = new_tensor({std::max<int64_t>(need, 256)}, at::kByte, dev);
+    return api.hqekv_decode_attn(k.seg, k.n, v.seg, v.n, q.data_ptr(), nullptr, 0, weights.data_ptr(), out.data_ptr(), B, Hq, k.H, D, Tall,
+                                 ws.data_ptr(), ws.numel(), flags, stream_of(dev));
+  });
   if (rc) return raise_rc(rc, "decode_attention");
   return Py_BuildValue("NN", THPVariable_Wrap(weights), THPVariable_Wrap(out));
   END_HANDLE_TH_ERRORS
@@ -323,20 +340,28 @@ void f16_rows(hqekv_seg &e, int layout, int64_t n, int64_t pos, const void *data
 }
 
 // The attention call of a step, with the workspace kept from step to step (twice what is needed when it is made: room
-// for the residual to grow without asking again).
+// for the residual to grow without asking again).  The tables are the caller's own copies.
 int run_step(const hqekv_seg *k, int n_k, const hqekv_seg *v, int n_v, const Tensor &q, const Tensor &weights, const Tensor &out,
-             int64_t Hkv, int64_t Tall, Tensor &ws, const at::Device &dev, const hqekv_step_extra *x) {
+             int64_t Hkv, int64_t Tall, Tensor &kept, const at::Device &dev, const hqekv_step_extra *x) {
   const int64_t B = q.size(0), Hq = q.size(1), D = q.size(3);
-  for (int attempt = 0;; ++attempt) {
-    if (attempt || !ws.defined() || ws.device() != dev) {
-      const int64_t need = api.hqekv_decode_workspace_bytes(k, n_k, v, n_v, B, Hq, Hkv, D);
-      if (need < 0) return HQEKV_E_ARG;
-      ws = new_tensor({std::max<int64_t>(2 * need, 256)}, at::kByte, dev);
+  const int flags = default_flags();
+  Tensor ws = kept;
+  const int rc = without_gil([&] {
+    auto call = [&]() -> int {
+      return api.hqekv_decode_step(k, n_k, v, n_v, q.data_ptr(), nullptr, 0, weights.data_ptr(), out.data_ptr(), B, Hq, Hkv, D, Tall,
+                                   ws.data_ptr(), ws.numel(), flags, stream_of(dev), x);
+    };
+    if (ws.defined() && ws.device() == dev) {
+      const int rc = call();
+      if (rc != HQEKV_E_WORKSPACE) return rc;   // else the cache has outgrown the workspace of earlier steps
     }
-    const int rc = api.hqekv_decode_step(k, n_k, v, n_v, q.data_ptr(), nullptr, 0, weights.data_ptr(), out.data_ptr(), B, Hq, Hkv, D, Tall,
-                                         ws.data_ptr(), ws.numel(), default_flags(), stream_of(dev), x);
-    if (rc != HQEKV_E_WORKSPACE || attempt) return rc;   // else the cache has outgrown the workspace of earlier steps
-  }
+    const int64_t need = api.hqekv_decode_workspace_bytes(k, n_k, v, n_v, B, Hq, Hkv, D);
+    if (need < 0) return (int)HQEKV_E_ARG;
+    ws = new_tensor({std::max<int64_t>(2 * need, 256)}, at::kByte, dev);
+    return call();
+  });
+  kept = ws;
+  return rc;
 }
 
 bool step_inputs(const Tensor &q, const Tensor &k, const Tensor &v, int64_t D) {
@@ -374,12 +399,15 @@ PyObject *tables_step(PyObject *self, PyObject *const *a, Py_ssize_t na) {
   }
   const int64_t cap_k = kb.size(2), cap_v = vb.size(2);
   int n_k = s->n_k, n_v = s->n_v;
+  hqekv_seg ks[HQEKV_MAX_SEGS], vs[HQEKV_MAX_SEGS];
+  memcpy(ks, s->k, n_k * sizeof(hqekv_seg));
+  memcpy(vs, s->v, n_v * sizeof(hqekv_seg));
   if (n) {
-    f16_rows(s->k[n_k++], HQEKV_LAYOUT_TOKEN_MAJOR, n, Tall - 1 - n, kb.data_ptr(), cap_k);
-    f16_rows(s->v[n_v++], 0, n, Tall - 1 - n, vb.data_ptr(), cap_v);
+    f16_rows(ks[n_k++], HQEKV_LAYOUT_TOKEN_MAJOR, n, Tall - 1 - n, kb.data_ptr(), cap_k);
+    f16_rows(vs[n_v++], 0, n, Tall - 1 - n, vb.data_ptr(), cap_v);
   }
-  f16_rows(s->k[n_k++], HQEKV_LAYOUT_TOKEN_MAJOR, 1, Tall - 1, k.data_ptr(), 0);
-  f16_rows(s->v[n_v++], 0, 1, Tall - 1, v.data_ptr(), 0);
+  f16_rows(ks[n_k++], HQEKV_LAYOUT_TOKEN_MAJOR, 1, Tall - 1, k.data_ptr(), 0);
+  f16_rows(vs[n_v++], 0, 1, Tall - 1, v.data_ptr(), 0);
   const c10::OptionalDeviceGuard guard(dev);
   Tensor weights = new_tensor({q.size(0), q.size(1), 1, Tall}, at::kHalf, dev), out = new_tensor({q.size(0), q.size(1), 1, D}, at::kHalf, dev);
   // (how torch's reduction deals the head rows to threads: attention.ring_order)
@@ -391,7 +419,7 @@ PyObject *tables_step(PyObject *self, PyObject *const *a, Py_ssize_t na) {
   x.v_dst = (char *)vb.data_ptr() + 2 * D * n;
   x.k_dst_slab_tokens = cap_k;
   x.v_dst_slab_tokens = cap_v;
-  const int rc = run_step(s->k, n_k, s->v, n_v, q, weights, out, k.size(1), Tall, s->ws, dev, &x);
+  const int rc = run_step(ks, n_k, vs, n_v, q, weights, out, k.size(1), Tall, s->ws, dev, &x);
   if (rc) return raise_rc(rc, "decode_step");
   PyObject *next = PyTuple_New(TUPLE_LEN);
   if (!next) return nullptr;
@@ -508,6 +536,7 @@ PyObject *kivi_step(PyObject *self, PyObject *const *a, Py_ssize_t na) {
       s->kt.size(0) != q.size(0))
     return PyErr_Format(PyExc_ValueError, "KiviAttentionLayer: the buffers do not hold the sequence before this step");
   const at::Device dev = q.device();
+  const Tensor held[] = {s->kq, s->ks, s->kz, s->kt, s->vt, s->vcode, s->vscale, s->vzero};
   hqekv_seg ks[3] = {}, vs[3] = {};
   int n_k = 0, n_v = 0;
   if (n_kq) {
@@ -634,11 +663,12 @@ PyObject *quantize_into(PyObject *, PyObject *const *a, Py_ssize_t na) {
   const bool rows = x.stride(3) == 1 && (R == 1 || x.stride(2) == L) && slab % 8 == 0 && (uintptr_t)x.data_ptr() % 16 == 0;
   if (!token_major && !rows) Py_RETURN_NONE;
   const c10::OptionalDeviceGuard guard(dev);
-  const int rc = token_major ? api.hqekv_quant_pack_k_tokenmajor(x.data_ptr(), slab, R, code.data_ptr(), code.stride(1), code.stride(2),
-                                                                 sc.data_ptr(), mn.data_ptr(), sc.stride(1), sc.stride(2), B * H, L, R, bits,
-                                                                 stream_of(dev))
-                             : api.hqekv_quant_pack_rows(x.data_ptr(), slab, L, code.data_ptr(), code.stride(1), code.stride(2), sc.data_ptr(),
-                                                         mn.data_ptr(), sc.stride(1), sc.stride(2), B * H, R, L, bits, stream_of(dev));
+  const int rc = without_gil([&] {
+    return token_major ? api.hqekv_quant_pack_k_tokenmajor(x.data_ptr(), slab, R, code.data_ptr(), code.stride(1), code.stride(2), sc.data_ptr(),
+                                                           mn.data_ptr(), sc.stride(1), sc.stride(2), B * H, L, R, bits, stream_of(dev))
+                       : api.hqekv_quant_pack_rows(x.data_ptr(), slab, L, code.data_ptr(), code.stride(1), code.stride(2), sc.data_ptr(),
+                                                   mn.data_ptr(), sc.stride(1), sc.stride(2), B * H, R, L, bits, stream_of(dev));
+  });
   if (rc) return raise_rc(rc, "uniform_group_quantize_pack_last_dim");
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS
@@ -672,8 +702,11 @@ PyObject *prompt_attention(PyObject *, PyObject *const *a, Py_ssize_t na) {
   const c10::OptionalDeviceGuard guard(dev);
   Tensor out = new_tensor({B, Hq, T, 128}, at::kHalf, dev);
   const int64_t so[3] = {Hq * T * 128, T * 128, 128};
-  const int rc = api.hqekv_prompt_attn(q.data_ptr(), sq, k.data_ptr(), sk, v.data_ptr(), sv, out.data_ptr(), so, B, Hq, Hkv, T, 128, (float)scaling,
-                                       a[4] == Py_True ? 1 : 0, stream_of(dev));
+  const int causal = a[4] == Py_True ? 1 : 0;
+  const int rc = without_gil([&] {
+    return api.hqekv_prompt_attn(q.data_ptr(), sq, k.data_ptr(), sk, v.data_ptr(), sv, out.data_ptr(), so, B, Hq, Hkv, T, 128, (float)scaling, causal,
+                                 stream_of(dev));
+  });
   if (rc) return raise_rc(rc, "prompt_attn");
   return THPVariable_Wrap(out);
   END_HANDLE_TH_ERRORS
@@ -698,8 +731,10 @@ PyObject *prompt_last_rows(PyObject *, PyObject *const *a, Py_ssize_t na) {
   Tensor probs = new_tensor({B, Hq, rows, T}, at::kHalf, dev), ws;
   const int64_t need = api.hqekv_prompt_last_rows_workspace_bytes(B, Hq, T);
   if (need > 0) ws = new_tensor({need}, at::kByte, dev);
-  const int rc = api.hqekv_prompt_last_rows(q.data_ptr(), sq, k.data_ptr(), sk, nullptr, nullptr, probs.data_ptr(), B, Hq, Hkv, T, 128, rows,
-                                            (float)scaling, need > 0 ? ws.data_ptr() : nullptr, need > 0 ? need : 0, stream_of(dev));
+  const int rc = without_gil([&] {
+    return api.hqekv_prompt_last_rows(q.data_ptr(), sq, k.data_ptr(), sk, nullptr, nullptr, probs.data_ptr(), B, Hq, Hkv, T, 128, rows, (float)scaling,
+                                      need > 0 ? ws.data_ptr() : nullptr, need > 0 ? need : 0, stream_of(dev));
+  });
   if (rc) return raise_rc(rc, "prompt_last_rows");
   return THPVariable_Wrap(probs);
   END_HANDLE_TH_ERRORS
@@ -734,7 +769,8 @@ PyObject *reconstruct(PyObject *, PyObject *const *a, Py_ssize_t na) {
   }
   const c10::OptionalDeviceGuard guard(dev);
   Tensor K = new_tensor({B, k.H, T, k.D}, at::kHalf, dev), V = new_tensor({B, k.H, T, k.D}, at::kHalf, dev);
-  const int rc = api.hqekv_cache_reconstruct(k.seg, k.n, v.seg, v.n, K.data_ptr(), V.data_ptr(), B * k.H, k.D, T, stream_of(dev));
+  const int rc = without_gil(
+      [&] { return api.hqekv_cache_reconstruct(k.seg, k.n, v.seg, v.n, K.data_ptr(), V.data_ptr(), B * k.H, k.D, T, stream_of(dev)); });
   if (rc) return raise_rc(rc, "cache_reconstruct");
   return Py_BuildValue("NN", THPVariable_Wrap(K), THPVariable_Wrap(V));
   END_HANDLE_TH_ERRORS
@@ -752,7 +788,9 @@ PyObject *importance(PyObject *, PyObject *const *a, Py_ssize_t na) {
   const at::Device dev = w.device();
   const c10::OptionalDeviceGuard guard(dev);
   Tensor imp = new_tensor({total}, at::kHalf, dev), scores = new_tensor({total / 32}, at::kHalf, dev);
-  const int rc = api.hqekv_importance_scores(w.data_ptr(), (int32_t)w.size(0), w.size(1), n, total, imp.data_ptr(), scores.data_ptr(), stream_of(dev));
+  const int rc = without_gil([&] {
+    return api.hqekv_importance_scores(w.data_ptr(), (int32_t)w.size(0), w.size(1), n, total, imp.data_ptr(), scores.data_ptr(), stream_of(dev));
+  });
   if (rc) return raise_rc(rc, "importance_scores");
   return Py_BuildValue("NN", THPVariable_Wrap(imp), THPVariable_Wrap(scores));
   END_HANDLE_TH_ERRORS
@@ -956,24 +994,26 @@ bool new_tokens(const Tensor &t, bool is_k, int64_t B, int64_t H, int64_t n, int
 bool host_orders(const void *const (&scores)[2], int64_t n, const Tensor &order, const at::Device &dev) {
   volatile int32_t *p = (volatile int32_t *)order.data_ptr();
   for (int64_t i = 0; i < 2 * n; ++i) p[i] = -1;
-  const int rc = api.hqekv_rank_blocks(scores, 2, n, (int32_t *)order.data_ptr(), stream_of(dev));
+  hipError_t err = hipSuccess;
+  const int rc = without_gil([&]() -> int {
+    const int rc = api.hqekv_rank_blocks(scores, 2, n, (int32_t *)order.data_ptr(), stream_of(dev));
+    if (rc) return rc;
+    const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(2);
+    int64_t i = 0;
+    while (i < 2 * n) {
+      if (p[i] >= 0) {
+        ++i;
+      } else if (std::chrono::steady_clock::now() > until) {
+        err = hipStreamSynchronize((hipStream_t)stream_of(dev));
+        break;
+      }
+    }
+    return HQEKV_OK;
+  });
   if (rc) {
     raise_rc(rc, "rank_blocks");
     return false;
   }
-  hipError_t err = hipSuccess;
-  Py_BEGIN_ALLOW_THREADS;
-  const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(2);
-  int64_t i = 0;
-  while (i < 2 * n) {
-    if (p[i] >= 0) {
-      ++i;
-    } else if (std::chrono::steady_clock::now() > until) {
-      err = hipStreamSynchronize((hipStream_t)stream_of(dev));
-      break;
-    }
-  }
-  Py_END_ALLOW_THREADS;
   if (err != hipSuccess) PyErr_Format(PyExc_RuntimeError, "rank_blocks: HIP error %d", (int)err);
   return err == hipSuccess;
 }
@@ -1061,12 +1101,16 @@ PyObject *compress(PyObject *, PyObject *const *a, Py_ssize_t na) {
     if (!is_tensor(a[6])) Py_RETURN_NONE;
     range = ten(a[6]);
     if (!plain_f16(range, 1, dev) || range.numel() != total) Py_RETURN_NONE;
-    rc = api.hqekv_weighted_block_scores(imp.data_ptr(), times_range ? range.data_ptr() : nullptr, total, scores_v.data_ptr(), stream);
+    rc = without_gil(
+        [&] { return api.hqekv_weighted_block_scores(imp.data_ptr(), times_range ? range.data_ptr() : nullptr, total, scores_v.data_ptr(), stream); });
   } else {
     if (prev == Py_None ? history != 0 : (!is_tensor(prev) || !plain_f16(ten(prev), 1, dev) || ten(prev).numel() != history)) Py_RETURN_NONE;
     range = new_tensor({total}, at::kHalf, dev);
-    rc = api.hqekv_range_block_scores(newV.data_ptr(), B, H, length, D, vs.src[5].slab_tokens, history ? ten(prev).data_ptr() : nullptr, history,
-                                      imp.data_ptr(), times_range ? 1 : 0, range.data_ptr(), scores_v.data_ptr(), stream);
+    const void *older = history ? ten(prev).data_ptr() : nullptr;
+    rc = without_gil([&] {
+      return api.hqekv_range_block_scores(newV.data_ptr(), B, H, length, D, vs.src[5].slab_tokens, older, history, imp.data_ptr(), times_range ? 1 : 0,
+                                          range.data_ptr(), scores_v.data_ptr(), stream);
+    });
   }
   if (rc) return raise_rc(rc, "range_block_scores");
   // ---- both rankings
@@ -1076,7 +1120,7 @@ PyObject *compress(PyObject *, PyObject *const *a, Py_ssize_t na) {
   if (!host_orders(sc, nb, host, dev)) return nullptr;
   // ---- the plans of both sides and the V side's surviving blocks, one transfer for all
   const int32_t *order = (const int32_t *)host.data_ptr();
-  int32_t *words = (int32_t *)host.data_ptr() + up(2 * nb, 4), counts[2][5], n_alive[2] = {0, 0};
+  int32_t *words = (int32_t *)host.data_ptr() + up(2 * nb, 4), counts[2][5] = {}, n_alive[2] = {0, 0};
   std::vector<int64_t> order64(nb);
   std::vector<int32_t> alive_k(nb);
   for (int side = 0; side < 2; ++side) {
@@ -1088,12 +1132,14 @@ PyObject *compress(PyObject *, PyObject *const *a, Py_ssize_t na) {
       cnt[c] = (int32_t)o.blocks[c].size();
     }
     for (int64_t i = 0; i < nb; ++i) order64[i] = order[side * nb + i];
-    rc = api.hqekv_plan_side(old, cnt, (int32_t)(history / 32), (int32_t)(length / 32), order64.data(), side ? vc : kc, side ? n_v : n_k, counts[side],
-                             words + side * 2 * nb, side ? words + 4 * nb : alive_k.data(), &n_alive[side]);
+    rc = without_gil([&] {
+      return api.hqekv_plan_side(old, cnt, (int32_t)(history / 32), (int32_t)(length / 32), order64.data(), side ? vc : kc, side ? n_v : n_k, counts[side],
+                                 words + side * 2 * nb, side ? words + 4 * nb : alive_k.data(), &n_alive[side]);
+    });
     if (rc) Py_RETURN_NONE;   // not a whole-block selection after all
   }
   const bool evicted = n_alive[1] < nb;
-  rc = api.hqekv_fetch_words(words, up_d.data_ptr(), evicted ? 4 * nb + n_alive[1] : 4 * nb, stream);
+  rc = without_gil([&] { return api.hqekv_fetch_words(words, up_d.data_ptr(), evicted ? 4 * nb + n_alive[1] : 4 * nb, stream); });
   if (rc) return raise_rc(rc, "fetch_words");
   at::getHostAllocator(at::kCUDA)->record_event(host.data_ptr(), host.storage().data_ptr().get_context(),
                                                 c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(dev.index()).unwrap());
@@ -1127,7 +1173,9 @@ PyObject *compress(PyObject *, PyObject *const *a, Py_ssize_t na) {
       x.res_dst_slab[side] = dst[side]->size(2);
     }
   }
-  rc = api.hqekv_cache_migrate_both(ks.src, 6, k_new.dst, k_new.n_dst, plan, vs.src, 6, v_new.dst, v_new.n_dst, plan + 2 * nb, B * H, D, &x, stream);
+  rc = without_gil([&] {
+    return api.hqekv_cache_migrate_both(ks.src, 6, k_new.dst, k_new.n_dst, plan, vs.src, 6, v_new.dst, v_new.n_dst, plan + 2 * nb, B * H, D, &x, stream);
+  });
   if (rc) return raise_rc(rc, "cache_migrate");
   // ---- the new tuple, while it runs
   PyObject *out = PyTuple_New(TUPLE_LEN);
