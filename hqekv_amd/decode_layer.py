@@ -238,41 +238,45 @@ class HqeAttentionLayer:
             # tokens the classes hold = the history this layer has kept; a tuple from elsewhere is counted
             Tall = (self.history_reserve_length if self._own_tuple else value_length(past_key_value) - n) + n + L
             lw = self.last_weights
-            done = None
-            if self.fused_step and attention_mask is None and L == 1 and query_states.is_cuda \
-                    and self.quant_strategy in ("uniform_group", "high_uniform_group_low_normal_group"):
+            done, on_device = None, False
+            one_call = (self.fused_step and attention_mask is None and L == 1 and query_states.is_cuda
+                        and query_states.dtype == key_states.dtype == value_states.dtype == torch.float16
+                        and self.quant_strategy in ("uniform_group", "high_uniform_group_low_normal_group"))
+            if one_call:
                 # One call: attention, the ring row (in torch's own summation order) and the two residual appends
                 # [131-133, 200]; the kernels read this step's key and value where they are, as a segment behind the
                 # residual, and copy them into the residual buffers in the call's last launch.
+                # Slices of a fused projection's output arrive with a batch stride of their own: one small copy each
+                # buys the one-call step.
+                query_states, key_states, value_states = (x if x.is_contiguous() else x.contiguous()
+                                                          for x in (query_states, key_states, value_states))
+                # shapes for which the ring row's summation order is pinned against torch's on the device
+                on_device = (Tall >= 256 and query_states.shape[1] == 32 and query_states.shape[0] <= 8
+                             and (lw.weights is None or lw.weights.dtype == torch.float16) and lw.max_length >= Tall)
+                line = lw.decode_row(query_states, Tall) if on_device else None   # (creates the store)
                 tables = self._memo.steps(past_key_value, query_states.device, self.quant_strategy == "uniform_group", known)
                 if tables is not None:
-                    # slices of a fused projection's output arrive with a batch stride of their own: one small copy each
-                    # buys the one-call step
-                    query_states, key_states, value_states = (x if x.is_contiguous() else x.contiguous()
-                                                              for x in (query_states, key_states, value_states))
-                    # shapes for which the ring row's summation order is pinned against torch's on the device
-                    on_device = (Tall >= 256 and query_states.shape[1] == 32 and query_states.shape[0] <= 8
-                                 and (lw.weights is None or lw.weights.dtype == torch.float16) and lw.max_length >= Tall)
-                    if on_device and lw.weights is None:
-                        lw.decode_row(query_states, Tall)   # creates the store
                     done = tables.step(query_states, key_states, value_states, past_key_value, *self._res, n, Tall,
                                        lw.weights if on_device else None, lw.next_line, kv_seq_len)
             if done is not None:
                 attn_weights, attn_output, past_key_value = done
-                if on_device:
-                    lw.advance(Tall)
-                else:
-                    lw.update(attn_weights)
                 self._returned = (past_key_value, n + L)
-            else:   # the plain sequence of the reference: the attention, the ring row, two copies
+            else:
+                # Classes that do not cover every position once, as one call through the general path; else the plain
+                # sequence of the reference: the attention, the ring row, two copies.
+                step = dict(ring_line=line, append=(*self._res, n)) if one_call else None
                 attn_weights, attn_output = qkv_matmul_hqe_2(query_states, past_key_value, attention_mask,
                                                              self.head_dim, self.quant_strategy, memo=self._memo,
-                                                             tail=(key_states, value_states))
-                lw.update(attn_weights)
-                self._res[0][:, :, n:n + L].copy_(key_states)
-                self._res[1][:, :, n:n + L].copy_(value_states)
+                                                             tail=(key_states, value_states), step=step)
+                if step is None:
+                    self._res[0][:, :, n:n + L].copy_(key_states)
+                    self._res[1][:, :, n:n + L].copy_(value_states)
                 new_K, new_V = self._res[0][:, :, :n + L], self._res[1][:, :, :n + L]
                 past_key_value = past_key_value[:-3] + (new_K, new_V, kv_seq_len)
+            if on_device:
+                lw.advance(Tall)
+            else:
+                lw.update(attn_weights)
             self._res_rows = n + L
         else:
             attn_weights, attn_output = self._prefill(query_states, key_states, value_states, attention_mask)

@@ -119,3 +119,36 @@ def test_layer_tuples_keep_their_contents(dev, fused):
     layer(*data[1], None, tuples[-2][0])
     for i, (kept, want) in enumerate(tuples):
         _same_tuple(kept, want, f"tuple {i}")
+
+
+def test_a_step_over_classes_that_leave_positions_out_is_one_call_too(dev, monkeypatch):
+    """Two tokens of a K class at one position, another position in none: ring row and appends ride in the attention call as
+    they do over a whole cover, with the bits of the separate launches."""
+    from hqekv_amd import _lib
+    from hqekv_amd.decode_layer import HqeAttentionLayer
+    B, Hq, Hkv, D, T0, steps = 2, 32, 8, 128, 350, 9
+    data = [tuple(x.to(dev) for x in _qkv(B, Hq, Hkv, T0 if s == 0 else 1, D, 900 + s)) for s in range(steps + 1)]
+    results, calls = [], []
+    entry = _lib.load().hqekv_decode_step
+
+    def counted(*a):
+        calls.append(a)
+        return entry(*a)
+    monkeypatch.setattr(_lib.load(), "hqekv_decode_step", counted)
+    for fused in (True, False):
+        layer = HqeAttentionLayer(D, 0.2, 0.3, 0.5)
+        layer.set_max_length(T0 + steps)
+        layer.fused_step = fused
+        pkv = list(layer(*data[0])[2])
+        pkv[13] = pkv[13].clone()                    # positions of the 4-bit K class
+        pkv[13][0] = pkv[13][1]
+        pkv, outs = tuple(pkv), []
+        for s in range(1, steps + 1):
+            out, w, pkv, _ = layer(*data[s], None, pkv)
+            outs += [out, w]
+        results.append((outs, layer.last_weights.weights, pkv))
+        assert len(calls) == steps                   # the first layer's, none of the second's
+    for a, b in zip(results[0][0], results[1][0]):
+        assert torch.equal(a, b)
+    assert torch.equal(results[0][1], results[1][1])
+    _same_tuple(results[0][2], tuple(x.cpu() if torch.is_tensor(x) else x for x in results[1][2]), "tuple")
