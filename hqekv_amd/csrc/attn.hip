@@ -2227,7 +2227,7 @@ extern "C" int hqekv_qk_hybrid(const hqekv_seg *segs, int nseg, const void *q, v
   if (!q || !scores || Tall <= 0) return fail(HQEKV_E_ARG, "qk_hybrid: null pointer or Tall <= 0");
   SegTable tb{};
   if (D == 128 && nseg >= 0 && nseg <= HQEKV_MAX_SEGS && segs && tiles_fit(segs, nseg, true, D, B, Hq, Hkv)) {
-    const TilesPlan plan = tiles_plan(segs, nseg, true, B * Hkv);
+    const TilesPlan plan = tiles_plan(segs, nseg, true, B * Hkv, Hq / Hkv);
     rc = build_table(segs, nseg, true, D, 0, Tall, &tb, "qk_hybrid", &plan);
     if (rc) return rc;
     return tb.total_units ? launch_qk_tiles(tb, q, scores, B, Hq, Hkv, Tall, FuseArgs{}, (hipStream_t)stream) : HQEKV_OK;
@@ -2269,7 +2269,7 @@ static bool pv_takes_tiles(const hqekv_seg *segs, int nseg, int64_t B, int64_t H
 static int64_t pv_units(const hqekv_seg *segs, int nseg, int64_t B, int64_t Hq, int64_t Hkv, int64_t D, bool tiles) {
   int64_t units = 0;
   if (tiles) {
-    units = tiles_plan(segs, nseg, false, B * Hkv).units;
+    units = tiles_plan(segs, nseg, false, B * Hkv, Hq / Hkv).units;
   } else {
     const int64_t chunk = pv_chunk_tokens(seg_total_tokens(segs, nseg), B * Hkv);
     for (int k = 0; k < nseg; ++k)
@@ -2297,7 +2297,7 @@ extern "C" int hqekv_pv_hybrid(const hqekv_seg *segs, int nseg, const void *p, v
   const bool tiles = pv_takes_tiles(segs, nseg, B, Hq, Hkv, D);
   const int64_t chunk = pv_chunk_tokens(seg_total_tokens(segs, nseg), B * Hkv);
   TilesPlan plan{};
-  if (tiles) plan = tiles_plan(segs, nseg, false, B * Hkv);
+  if (tiles) plan = tiles_plan(segs, nseg, false, B * Hkv, Hq / Hkv);
   SegTable tb{};
   rc = build_table(segs, nseg, false, D, chunk, Tall, &tb, "pv_hybrid", tiles ? &plan : nullptr);
   if (rc) return rc;
@@ -2336,7 +2336,7 @@ static int decode_layout(const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_se
       tiles += (k_segs[k].n_tokens + per - 1) / per;
     }
   if (n_k > 0 && tiles_fit(k_segs, n_k, true, D, B, Hq, Hkv)) {
-    const int64_t pairs = tiles_plan(k_segs, n_k, true, B * Hkv).units;
+    const int64_t pairs = tiles_plan(k_segs, n_k, true, B * Hkv, Hq / Hkv).units;
     if (pairs > tiles) tiles = pairs;
   }
   if (tiles == 0) tiles = 1;
@@ -2491,8 +2491,8 @@ static int decode_impl(const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_segs
   const bool k_tiles = by_rule && n_k > 0 && tiles_fit(k_segs, n_k, true, D, B, Hq, Hkv);
   const bool v_tiles = by_rule && n_v > 0 && tiles_fit(v_segs, n_v, false, D, B, Hq, Hkv);
   TilesPlan k_plan{}, v_plan{};
-  if (k_tiles) k_plan = tiles_plan(k_segs, n_k, true, B * Hkv);
-  if (v_tiles) v_plan = tiles_plan(v_segs, n_v, false, B * Hkv);
+  if (k_tiles) k_plan = tiles_plan(k_segs, n_k, true, B * Hkv, Hq / Hkv);
+  if (v_tiles) v_plan = tiles_plan(v_segs, n_v, false, B * Hkv, Hq / Hkv);
   SegTable kt{}, vt{};
   rc = build_table(k_segs, n_k, true, D, qk_tile_of(tiling), Tall, &kt, "decode_attn(K)", k_tiles ? &k_plan : nullptr);
   if (rc) return rc;

@@ -630,7 +630,7 @@ bool tiles_fit(const hqekv_seg *segs, int nseg, bool is_k, int64_t D, int64_t B,
   return true;
 }
 
-TilesPlan tiles_plan(const hqekv_seg *segs, int nseg, bool is_k, int64_t BHkv) {
+TilesPlan tiles_plan(const hqekv_seg *segs, int nseg, bool is_k, int64_t BHkv, int64_t nrep) {
   TilesPlan p{};
   p.is_k = is_k;
   p.per_unit = 1;
@@ -648,9 +648,10 @@ TilesPlan tiles_plan(const hqekv_seg *segs, int nseg, bool is_k, int64_t BHkv) {
     if (p.units * BHkv > QT_LONG) p.per_unit = QL_TILES;
     p.units = count();
   } else {
-    // One block per workgroup while all of them are resident at once (six per CU); else as many as make one resident
-    // round of the looping kernel (four per CU): a second, nearly empty round would cost a workgroup's whole life.
-    if (p.units * BHkv > PT_RESIDENT) p.per_unit = (int)((p.units * BHkv + PT_RESIDENT_LOOP - 1) / PT_RESIDENT_LOOP);
+    // One block per workgroup while all of them are resident at once; else as many as make one resident round of the
+    // looping kernel: a second, nearly empty round would cost a workgroup's whole life.
+    const int64_t all = p.units * BHkv, loop = pt_loop_units(nrep, all);
+    if (all > pt_resident(nrep)) p.per_unit = (int)((all + loop - 1) / loop);
     p.units = count();
   }
   return p;

@@ -100,7 +100,13 @@ struct Positions {
 __device__ __forceinline__ bool qt_runs(const SegDev &sg) { return (sg.layout & HQEKV_LAYOUT_RUNS) || !sg.idx; }
 
 // =============================================================================== host side
-constexpr int64_t PT_RESIDENT = 6 * 256, PT_RESIDENT_LOOP = 4 * 256;   // p.V workgroups the chip holds
+// p.V workgroups the chip holds at once, of the single-block form, and the workgroups a looping launch is made of: one
+// resident round.  Up to eight heads per KV head: six and four per CU (80 and 128 registers).  Above: three and two (45 and
+// 58 KB of LDS) -- two rounds of those for launches of more than 4096 blocks, whose last round weighs less than the runs of
+// a workgroup that meets the end of its class.  p.V at 16 heads, 512 / 1024 workgroups: 1800 blocks (B=1, 64k tokens) 27.4 /
+// 33.2 us, 3700 (4 x 32k) 42.0 / 46.9, 5500 (8 x 24k) 64.8 / 65.1, 7400 (8 x 32k) 84.3 / 81.8, 14700 (8 x 64k) 155.8 / 152.2.
+constexpr int64_t pt_resident(int64_t nrep) { return (nrep <= 8 ? 6 : 3) * 256; }
+constexpr int64_t pt_loop_units(int64_t nrep, int64_t blocks) { return (nrep <= 8 || blocks > 4096 ? 4 : 2) * 256; }
 
 // How a launch is cut up.
 struct TilesPlan {
@@ -108,9 +114,14 @@ struct TilesPlan {
   int per_unit;       // p.V: blocks per workgroup
   int64_t units;      // workgroups per (b, kv head); q.K^T leaves one softmax pair per query head in each
 };
-// head_dim 128, at most 16 query heads per KV head, channel-major fp16 K classes of whole 8-token columns
+// head_dim 128, at most 16 query heads per KV head (the rows of A), channel-major fp16 K classes of whole 8-token columns.
+// Every ratio up to there is faster here than in the forms of attn.hip, also where rows are spare.  A step at 1k, 32k and
+// 8 x 64k tokens of the fp16 / 8 / 4 / 2-bit mix, us, here against there: 1 head 10.7 / 14.4, 21.9 / 25.1, 158 / 178; 2 heads
+// 10.8 / 15.5, 22.8 / 26.8, 167 / 187; 4 heads 10.8 / 17.3, 23.3 / 29.3, 178 / 205; 5 heads 11.9 / 20.9, 25.2 / 38.8, 201 /
+// 260; 8 heads 12.0 / 23.3, 26.7 / 51.9, 221 / 322; 9 heads 14.1 / 35.7, 31.8 / 70.4, 242 / 489; 16 heads 15.4 / 45.8, 35.8 /
+// 98.2, 295 / 644.  (One head: p.V alone is a tie, q.K^T is what gains.)
 bool tiles_fit(const hqekv_seg *segs, int nseg, bool is_k, int64_t D, int64_t B, int64_t Hq, int64_t Hkv);
-TilesPlan tiles_plan(const hqekv_seg *segs, int nseg, bool is_k, int64_t BHkv);
+TilesPlan tiles_plan(const hqekv_seg *segs, int nseg, bool is_k, int64_t BHkv, int64_t nrep);
 int64_t tiles_unit_tokens(const TilesPlan &p, const hqekv_seg &s);
 
 inline TilesArgs tiles_args(int64_t B, int64_t Hq, int64_t Hkv) {

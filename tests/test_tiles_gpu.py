@@ -49,7 +49,7 @@ def test_tile_edges(dev, blocks, n_rep, B, residual, low_normal, fused, shuffled
     torch.testing.assert_close(o.float().cpu(), o_ref.float(), rtol=RTOL, atol=ATOL)
 
 
-@pytest.mark.parametrize("n_rep", [4, 5])
+@pytest.mark.parametrize("n_rep", [4, 5, 12])
 def test_several_blocks_per_workgroup(dev, n_rep):
     """More blocks of V than workgroups fit on the chip: the looping form, with every class and a ragged last round."""
     from hqekv_amd.attention import decode_attention
