@@ -175,12 +175,13 @@ def _whole_runs(a: np.ndarray) -> bool:
     return bool((r == r[:, :1] + np.arange(32)).all())
 
 
-def idx_cover_once(idx_list, n: int) -> bool:
+def idx_cover_once(idx_list, n: int, may_wait: bool = True) -> bool:
     """True when the class position arrays, taken together, hold every position in [0, n) exactly once -- what
     the softmax fused into the two GEMV launches relies on (a position nobody writes keeps whatever the score
     buffer held, one written twice is counted twice).  Arrays that carry a host copy (the cache policy's) are
     checked there; others on the device, which waits for it once: the verdict is remembered per set of tensors
-    until one of them is written to."""
+    until one of them is written to.  Without ``may_wait`` -- the stream is being captured -- a set that has to be looked at
+    on the device counts as not covering."""
     idx_list = [t for t in idx_list if t is not None]
     if sum(int(t.numel()) for t in idx_list) != n:
         return False
@@ -204,6 +205,8 @@ def idx_cover_once(idx_list, n: int) -> bool:
         c = np.concatenate(hosts)
         ok = bool(c.size == n and (c >= 0).all() and (c < n).all() and (np.bincount(c, minlength=n) == 1).all())
         runs = all(_whole_runs(h) for h in hosts)
+    elif not may_wait:
+        return False
     elif idx_list[0].is_cuda and len(idx_list) <= _lib.MAX_SEGS and n < 2 ** 38 and \
             all(t.dtype == torch.int64 and t.is_contiguous() and t.device == idx_list[0].device for t in idx_list):
         ok, runs = _cover_on_device(idx_list, n)

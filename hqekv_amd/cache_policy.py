@@ -712,8 +712,7 @@ def reconstruct(past_key_value: tuple, quant_strategy: str, block_size: int = 32
     pkv = past_key_value
     if quant_strategy in ("uniform_group", LOW_NORMAL) and any(torch.is_tensor(x) and x.is_cuda for x in (pkv[2], pkv[8], pkv[16], pkv[24], pkv[32], pkv[40])):
         from . import _lib
-        from . import attention as A
-        done = _lib.host().reconstruct(pkv, quant_strategy != LOW_NORMAL, A.idx_cover_once)
+        done = _lib.host().reconstruct(pkv, quant_strategy != LOW_NORMAL, _cover_for_reconstruction)
         if done is not None:
             return done
     k_side, v_side = _read_side(pkv, K_SLOT), _read_side(pkv, V_SLOT)
@@ -732,7 +731,7 @@ def reconstruct(past_key_value: tuple, quant_strategy: str, block_size: int = 32
     for b in CLASS_BITS:
         if b == 1 and (k_side[b].data is not None or v_side[b].data is not None):
             _check_low_bits(1, quant_strategy)
-    if dev.type == "cuda" and D % 32 == 0 and D <= 4096:
+    if dev.type == "cuda" and D % 32 == 0 and D <= 4096 and not torch.cuda.is_current_stream_capturing():
         return _reconstruct_on_device(pkv, B, H, T, D, dev, quant_strategy != LOW_NORMAL)
     K = torch.zeros(B, H, T, D, dtype=torch.float16, device=dev)
     V = torch.zeros(B, H, T, D, dtype=torch.float16, device=dev)
@@ -746,6 +745,13 @@ def reconstruct(past_key_value: tuple, quant_strategy: str, block_size: int = 32
     if new_V is not None:
         V[:, :, T - new_V.shape[2]:, :] = new_V
     return K, V
+
+
+def _cover_for_reconstruction(idx_list, n: int) -> bool:
+    """A reconstruction may be captured into a graph, where nothing can be waited for: then a set of positions whose verdict
+    is not known goes class by class."""
+    from . import attention as A
+    return A.idx_cover_once(idx_list, n, may_wait=not torch.cuda.is_current_stream_capturing())
 
 
 def _reconstruct_on_device(pkv: tuple, B: int, H: int, T: int, D: int, dev, low_uniform: bool):

@@ -120,3 +120,32 @@ def test_positions_outside_the_cache(dev):
             KV_cache_reconstruct_hqe(tuple(wrong), "uniform_group")
     with pytest.raises(ValueError):
         KV_cache_reconstruct_hqe(tuple(pkv[:41]) + (3,), "uniform_group")   # fewer positions than the residual has rows
+
+
+@pytest.mark.parametrize("seen", [False, True])
+def test_reconstruction_captured_into_a_graph(dev, seen):
+    """Positions never looked at before (class by class) or known to cover the cache (one launch): every replay gives what
+    the eager call gives, on the cache's contents of the time."""
+    from hqekv_amd.hqe_2 import KV_cache_reconstruct_hqe
+    pkv = _cache(dev, 1, 2, 512, 128, 5, (.2, .2, .2, .2, .2), "uniform_group")
+    if seen:
+        KV_cache_reconstruct_hqe(pkv, "uniform_group")
+    warm = _cache(dev, 1, 2, 512, 128, 5, (.2, .2, .2, .2, .2), "uniform_group")
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        KV_cache_reconstruct_hqe(warm, "uniform_group")
+        stream.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            got = KV_cache_reconstruct_hqe(pkv, "uniform_group")
+    torch.cuda.synchronize()
+    want = O.reconstruct_cache(synth.cache_to(pkv, "cpu"), "uniform_group")
+    for turn in range(4):
+        for g in got:
+            g.fill_(turn)
+        graph.replay()
+        torch.cuda.synchronize()
+        for g, w in zip(got, want):
+            assert torch.equal(g.cpu().view(torch.int16), w.contiguous().view(torch.int16)), turn
+        pkv[2].neg_()
+        want = O.reconstruct_cache(synth.cache_to(pkv, "cpu"), "uniform_group")
