@@ -152,7 +152,7 @@ _PROTOS = {
     "hqekv_cache_migrate_both": (C.c_int, [_CCP, _int, _CCP, _int, _vp, _CCP, _int, _CCP, _int, _vp, _i64, _i64, _vp, _vp]),
     "hqekv_fetch_words": (C.c_int, [_vp, _vp, _i64, _vp]),
 }
-STATIC_SCRATCH_BYTES = 8 << 20   # HQEKV_STATIC_SCRATCH_BYTES
+STATIC_SCRATCH_BYTES = 10 << 20   # HQEKV_STATIC_SCRATCH_BYTES
 
 
 def lib_path() -> Path:

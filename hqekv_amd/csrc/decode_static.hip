@@ -8,6 +8,8 @@
 
 #include "common.h"
 
+// 10 MiB: what fitted into 8 when the split-K partials were one row per chunk of the older p.V form fits (the decode launches
+// write up to 1.16 times as many rows at 8 to 16 query heads per KV head and many slabs; tests/test_capi_symbols.py).
 // The kernels receive the array through the same workspace argument the caller-workspace entry point passes.
 static __device__ __align__(256) unsigned char scratch[HQEKV_STATIC_SCRATCH_BYTES];
 

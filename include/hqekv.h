@@ -498,7 +498,7 @@ int hqekv_plan_side(const int32_t *const *old_blocks, const int32_t *old_counts,
  * HQEKV_E_WORKSPACE (use hqekv_decode_attn then).  All calls on one GPU share the buffer: calls that overlap in
  * time on one GPU (two streams, two threads) race; calls ordered on one stream are fine.
  */
-#define HQEKV_STATIC_SCRATCH_BYTES (8u << 20)
+#define HQEKV_STATIC_SCRATCH_BYTES (10u << 20)
 int hqekv_decode_attn_static(const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_segs, int n_v,
                              const void *q, const void *mask, int64_t mask_row_stride,
                              void *attn_weights, void *attn_out, int64_t B, int64_t Hq, int64_t Hkv,

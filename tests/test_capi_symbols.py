@@ -76,6 +76,41 @@ def test_argument_validation_without_a_gpu():
         _lib.check(700, "x")
 
 
+def test_static_scratch_holds_what_the_chunked_form_needed():
+    """Calls whose partials took up to 8 MiB as chunks of the older p.V form fit into the fixed buffer in the form that
+    the calls take now, which may have more rows of partials."""
+    import random
+    from hqekv_amd import _lib, synth
+    lib, rng, near = _lib.load(), random.Random(1), 0
+
+    def up(v):
+        return (v + 255) // 256 * 256
+    # the widest cases first, then shapes at random
+    cases = [(32, 8, 8, 8416, 0, 63), (32, 8, 10, 4576, 0, 17), (16, 8, 14, 14624, 2, 0), (3, 32, 13, 1632, 2, 17), (8, 4, 15, 21888, 3, 63)]
+    while len(cases) < 20000:
+        cases.append((rng.choice((1, 1, 2, 3, 4, 8, 16, 32)), rng.choice((1, 2, 4, 8, 16, 32)), rng.randint(1, 16),
+                      32 * int(2 ** rng.uniform(3, 13)), rng.randrange(4), rng.choice((0, 17, 63))))
+    for B, Hkv, rep, T, mix, residual in cases:
+        mix = ((.05, .15, .3, .3, .2), (0, 0, 0, 1, 0), (.1, 0, .2, .5, .2), (.02, .03, .25, .5, .2))[mix]
+        counts = [int(round(T // 32 * f)) * 32 for f in mix[:4]]
+        items = [dict(bits=b, n_tokens=n, data=None) for b, n in zip(synth.CLASS_ORDER, counts) if n]
+        items += [dict(bits=16, n_tokens=residual, data=None, token_major=1)] if residual else []
+        if not items:
+            continue
+        tokens = sum(i["n_tokens"] for i in items)
+        per = -(-(2048 if tokens * B * Hkv >= 2 << 20 else 1024) // (B * Hkv))
+        chunk = min(4096, max(64, (-(-tokens // per) + 63) // 64 * 64))
+        chunks = sum(-(-i["n_tokens"] // chunk) for i in items)
+        tiles = sum(-(-i["n_tokens"] // (64 if i.get("token_major") else 256)) for i in items)
+        before = up(chunks * B * Hkv * rep * 512) + up(B * Hkv * rep * tiles * 8) + up(B * Hkv * 4)
+        if before <= 8 << 20:
+            segs = _lib.make_segs(items)
+            need = lib.hqekv_decode_workspace_bytes(segs, len(items), segs, len(items), B, rep * Hkv, Hkv, 128)
+            near += need > 8 << 20
+            assert 0 < need <= _lib.STATIC_SCRATCH_BYTES, (B, Hkv, rep, T, mix, residual)
+    assert near >= 5   # the sample reaches the shapes this is about
+
+
 def test_reference_import_names_resolve():
     """`from pack_unpack import ...`, `from quant.hqe_matmul import ...`, `from model.public_func import ...`"""
     import importlib
