@@ -152,3 +152,34 @@ def test_a_step_over_classes_that_leave_positions_out_is_one_call_too(dev, monke
         assert torch.equal(a, b)
     assert torch.equal(results[0][1], results[1][1])
     _same_tuple(results[0][2], tuple(x.cpu() if torch.is_tensor(x) else x for x in results[1][2]), "tuple")
+
+
+@pytest.mark.parametrize("Hkv", [2, 1])
+@pytest.mark.parametrize("kind", ["hqe", "kivi"])
+def test_layers_take_projection_views(dev, kind, Hkv):
+    """What a model hands over -- slices of one projection's (B, T, heads, D) output, seen per head -- gives the tuples and
+    outputs of dense tensors, through prompt, compressions and steps."""
+    from hqekv_amd.decode_layer import HqeAttentionLayer
+    from hqekv_amd.kivi_layer import KiviAttentionLayer
+    B, Hq, D, T0, steps = 2, 4 * Hkv, 128, 203, 40
+
+    def run(views):
+        if kind == "hqe":
+            layer = HqeAttentionLayer(D, 0.2, 0.3, 0.5)
+            layer.set_max_length(T0 + steps)
+        else:
+            layer = KiviAttentionLayer(D, 2, 2, 32, 32)
+        pkv, outs = None, []
+        for s in range(steps + 1):
+            y = torch.cat(_qkv(B, Hq, Hkv, T0 if s == 0 else 1, D, 600 + s), 1).to(dev)
+            if views:
+                y = y.transpose(1, 2).contiguous().transpose(1, 2)
+            parts = y[:, :Hq], y[:, Hq:Hq + Hkv], y[:, Hq + Hkv:]
+            out, w, pkv = layer(*(parts if views else (x.contiguous() for x in parts)), None, pkv)[:3]
+            outs += [out] + ([w] if w is not None else [])
+        return outs, pkv
+    (a, pa), (b, pb) = run(False), run(True)
+    for x, y in zip(a, b):
+        assert torch.equal(x, y)
+    for i, (x, y) in enumerate(zip(pa, pb)):
+        assert (x is None) == (y is None) and (not torch.is_tensor(x) or torch.equal(x, y)), i
