@@ -762,20 +762,20 @@ def _reconstruct_on_device(pkv: tuple, B: int, H: int, T: int, D: int, dev, low_
     from . import _lib
     from . import attention as A
     keep: list = []
-    sides = ((A.key_segments(pkv, dev, T, keep, low_uniform)[0], A.K16, A.K_BASE, pkv[A.NEW_K]),
-             (A.value_segments(pkv, dev, T, keep, low_uniform)[0], A.V16, A.V_BASE, pkv[A.NEW_V]))
+    sides = ((A.key_segments(pkv, dev, T, keep, low_uniform)[0], pkv[A.NEW_K]), (A.value_segments(pkv, dev, T, keep, low_uniform)[0], pkv[A.NEW_V]))
     dense, calls = [], []
-    for items, base0, bases, new in sides:
+    for items, new in sides:
         for it in items:   # the kernel reads fp16 rows in 16-byte pieces
             if it["bits"] == 16 and it["data"].data_ptr() % 16:
                 it["data"], it["slab_tokens"] = it["data"].clone(), 0   # (dense, a transposed view stays one)
-        idx = A._class_idx(pkv, base0, bases)
+        classes = items[:-1] if new is not None and new.shape[2] > 0 else items
+        idx = [it["idx"] for it in classes]   # (as 64-bit words on the device, whatever the tuple holds)
         n = T - (new.shape[2] if new is not None else 0)
         if n < 0:
             raise ValueError("invalid past_key_value: a residual longer than kv_seq_len")
         whole = all(t is not None for t in idx) and A.idx_cover_once(idx, n)
         if not whole:   # (asked on the way that waits for the device anyway)
-            out = [((t < -T) | (t >= T)).any() for t in (it["idx"] for it in items) if t is not None]
+            out = [((t < -T) | (t >= T)).any() for t in idx if t is not None]
             if out and bool(torch.stack(out).any()):
                 raise IndexError(f"a position outside the cache of {T} tokens")
         dense.append((torch.empty if whole else torch.zeros)(B, H, T, D, dtype=torch.float16, device=dev))

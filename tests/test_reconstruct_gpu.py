@@ -149,3 +149,12 @@ def test_reconstruction_captured_into_a_graph(dev, seen):
             assert torch.equal(g.cpu().view(torch.int16), w.contiguous().view(torch.int16)), turn
         pkv[2].neg_()
         want = O.reconstruct_cache(synth.cache_to(pkv, "cpu"), "uniform_group")
+
+
+def test_positions_as_any_integers_anywhere(dev):
+    """Positions as 32-bit numbers, on the host, as every other element of a longer array: what indexing a tensor takes."""
+    pkv = list(_cache(dev, 1, 2, 512, 128, 5, (.2, .2, .2, .2, .2), "uniform_group"))
+    pkv[1], pkv[5], pkv[9] = pkv[1].cpu(), pkv[5].to(torch.int32), pkv[9].repeat_interleave(2)[::2]
+    _check(tuple(pkv), "uniform_group")
+    pkv[1] = pkv[1] - pkv[41]                    # counted from the end, as well
+    _check(tuple(pkv), "uniform_group")
