@@ -1,6 +1,10 @@
 // Decode attention over the hybrid fp16 / 8 / 4 / 2-bit cache: fused dequantize-GEMV for q.K^T,
 // scale+mask+clamp+softmax, fused dequantize-GEMV for p.V with a deterministic split-K combine.
 //
+// The entry points, the softmax, the combine and the step's epilogue are for every call.  The two GEMVs in this file are the
+// forms that a call's flags name, and serve more than 16 query heads per KV head, q.K^T at other head sizes and over fp16
+// classes that do not hold whole eights of tokens; everything else runs in decode_qk.hip and decode_pv.hip.
+//
 // Arithmetic.  The reference defines a correct result as "dequantise with the library's own
 // unpack, then matmul" (quant/cuda_hq_test.py:82,242), and its dequantiser rounds twice in fp16
 // (quant/pack_unpack.py:331-332).  The kernels reproduce exactly those values in registers:
@@ -10,7 +14,7 @@
 // Codes become fp16 integers without a shift or an int->float convert: a byte permute lines up the
 // same byte of two rows in the two 16-bit halves of a register, one AND-OR drops a code field into
 // the mantissa of 2^(10-pos) (giving 2^(10-pos) + c exactly) and one packed subtract removes the bias.
-// With four query heads per KV head the products of those values with the query (or the probabilities) run as
+// With four query heads per KV head the products of those values with the query (or the probabilities) can run as
 // 4x4x4 fp16 matrix instructions (same dequantised bits, exact products, fp32 accumulation; HQEKV_DOT_VALU keeps them
 // on the vector ALU).  No packed-fp32 instructions are used.
 //
@@ -1924,7 +1928,7 @@ __global__ __launch_bounds__(CB_CH * CB_SLICES) void pv_combine_kernel(const flo
 
 // =============================================================================== host side
 
-// With a plan: the launches of decode_tiles.hip.  Else
+// With a plan: the launches of decode_qk.hip and decode_pv.hip.  Else
 // `unit_tokens`: tokens per work unit -- the q.K^T tile of the chosen tiling (the token-major fp16 residual
 // always has 64-token tiles) or the p.V chunk.
 static int build_table(const hqekv_seg *segs, int nseg, bool is_k, int64_t D, int64_t unit_tokens,
@@ -2201,8 +2205,9 @@ static int launch_pv(const SegTable &tb, int64_t chunk, void *p, void *out, floa
   const bool combine = (stages & 2) && !fz.arrive;   // folded: the last p.V workgroups have written the output
   const bool epilogue = ep && (ep->ring_line || ep->app_rows > 0 || ep->leave_bits) && stages == 3;
   if (!combine && !epilogue) return HQEKV_OK;
-  // The epilogue rides in the combine launch as extra workgroups (grid.z); one workgroup per RING_SPAN columns of
-  // the ring row.  Without a combine (folded into p.V) the launch holds the epilogue alone.
+  // The epilogue rides in the combine launch as extra workgroups: as many layers of grid.z (B * Hq * D / 32 workgroups each)
+  // as make one workgroup per RING_SPAN columns of the ring row at the least.  Without a combine (folded into p.V) the
+  // launch holds the epilogue alone.
   const dim3 base((unsigned)n_bhq, (unsigned)((D + CB_CH - 1) / CB_CH));
   unsigned z = combine ? 1u : 0u;
   if (epilogue) {

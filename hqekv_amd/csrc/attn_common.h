@@ -33,7 +33,7 @@ struct SegTable {
   int32_t nseg;
   int32_t total_units;
   int32_t max_units;   // the largest n_units of any segment
-  int32_t per_unit;    // tiles or blocks per unit (decode_tiles.hip)
+  int32_t per_unit;    // tiles or blocks per unit of the matrix-core launches (decode_tiles.h); 0 = the older forms
   int32_t begin[HQEKV_MAX_SEGS];  // first grid.y index of every segment (INT32_MAX past nseg): one scalar load finds a workgroup's segment
 };
 

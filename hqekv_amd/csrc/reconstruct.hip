@@ -9,7 +9,8 @@
 // the tile is turned in LDS -- 68 words per token row, so the channel-pair writes walk all banks and the 16-byte reads
 // stay aligned.  34 KB of LDS: four workgroups per CU.
 // Measured at B=1, 16k tokens of the fp16 / 8 / 4 / 2-bit mix (73 MB): 258 us as dequantise launches, transposing copies
-// and index_put scatters; this launch 21 us (3.4 TB/s), 38 us with the host call around it.
+// and index_put scatters; this launch 21 us (3.4 TB/s), 20 us a call among others.  Positions that are looked at for the
+// first time cost two position checks and a wait for each on top (see cover_once_kernel).
 #include <algorithm>
 
 #include "common.h"

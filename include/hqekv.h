@@ -238,16 +238,20 @@ int hqekv_pv_hybrid(const hqekv_seg *segs, int nseg, const void *p, void *out, i
  * HQEKV_ONLY_QK / HQEKV_ONLY_PV / HQEKV_ONLY_COMBINE run one part of the call (q.K^T [+ softmax] / the p.V
  * kernel / the combine) so that each can be timed on its own; the later parts expect the earlier ones to
  * have run on the same buffers.
- * HQEKV_QK_TILING(n): which q.K^T tiling the call uses, n = 0 (default) chooses by launch size; any other
- * value forces one of the tilings listed below, whatever the size -- results agree to the stated tolerance
- * (the summation order over head_dim differs), so tests and measurements can name a tiling per call.
+ * A call that names none of the forms below (flags = 0 or HQEKV_FUSE_SOFTMAX) with up to 16 query heads per KV head
+ * runs on 16x16x32 matrix instructions (decode_qk.hip, decode_pv.hip); the q.K^T side of a call whose fp16 class does
+ * not hold whole eights of tokens, and any larger ratio, runs on the forms that the flags name, chosen by launch size.
+ * HQEKV_QK_TILING(n): n = 0 is the rule above; any other value forces one of the tilings listed below, whatever the
+ * size, and the older p.V with it -- results agree to the stated tolerance (the summation order differs), so tests and
+ * measurements can name a tiling per call.
  */
 #define HQEKV_FUSE_SOFTMAX 1
-#define HQEKV_SEPARATE_COMBINE 2 /* always sum the split-K partials with a launch of their own                       */
-#define HQEKV_FOLD_COMBINE 4     /* let the last p.V workgroup of each (b, kv head) sum them whenever there are at
-                                    most 64 chunks; by default that is done only for long launches (>= 2^21 V token
-                                    rows), where it saves more than it costs.  Both ways add in the same order and
-                                    give the same bits                                                            */
+#define HQEKV_SEPARATE_COMBINE 2 /* older p.V, its split-K partials always summed by a launch of their own (as those of the
+                                    matrix-core launches are)                                                     */
+#define HQEKV_FOLD_COMBINE 4     /* older p.V, whose last workgroup of each (b, kv head) sums them whenever there are at
+                                    most 64 chunks; a call that names another older form does so for long launches
+                                    (>= 2^21 V token rows) only, where it saves more than it costs.  Both ways add in
+                                    the same order and give the same bits                                         */
 #define HQEKV_TWO_STEP_DEQUANT 8  /* The kernels read a code c out of a packed word as the fp16 number bias + c.  The
                                     one-wave q.K^T tilings turn a tile whose scales are all below 32 in magnitude into
                                     c * s with one fused multiply-add, (bias + c) * s - bias * s (bias * s is exact
@@ -263,14 +267,16 @@ int hqekv_pv_hybrid(const hqekv_seg *segs, int nseg, const void *p, void *out, i
 #define HQEKV_ONLY_QK 0x100
 #define HQEKV_ONLY_PV 0x200
 #define HQEKV_ONLY_COMBINE 0x400
-/* Form of the inner products of both GEMV launches.  With four query heads per KV head (Hq/Hkv == 4) the products of
+/* Form of the inner products of the older GEMV launches.  With four query heads per KV head (Hq/Hkv == 4) the products of
  * the dequantised values with the query (or with the probabilities) can run on the matrix cores: one 4x4x4 fp16 matrix
  * instruction per four elements of the reduction axis and lane, in place of eight two-element dot products on the
  * vector ALU.  The dequantised values are the same bits either way, products are exact and accumulation is fp32 in
- * both; only the order of the additions differs.  Neither flag: the library's default for the shape.
- * Head ratios (Hq up to 65535): the kernels exist for 1 to 8 query heads per KV head; a larger ratio, up to 64, is served in slices of
- * at most eight heads (12 = 8 + 4, 13 = 8 + 5, ...), one launch per slice and GEMV (each reads the cache again), a
- * slice of four in the form the flags name.  HQEKV_DOT_MFMA with a ratio of 1-3 or 5-8 returns HQEKV_E_UNSUPPORTED. */
+ * both; only the order of the additions differs.  Neither flag, but another older form: 4x4x4 for four heads, else the
+ * vector ALU.
+ * Head ratios (Hq up to 65535): the older kernels exist for 1 to 8 query heads per KV head; there a larger ratio, up to 64,
+ * is served in slices of at most eight heads (12 = 8 + 4, 13 = 8 + 5, ...), one launch per slice and GEMV (each reads the
+ * cache again), a slice of four in the form the flags name.  HQEKV_DOT_MFMA with a ratio of 1-3 or 5-8 returns
+ * HQEKV_E_UNSUPPORTED. */
 #define HQEKV_DOT_MFMA 0x800
 #define HQEKV_DOT_VALU 0x1000
 /* Run the q.K^T launch alone and leave the RAW fp16 scores in attn_weights (no scaling, no softmax), with the tiling
