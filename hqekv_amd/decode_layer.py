@@ -253,7 +253,8 @@ class HqeAttentionLayer:
                 # shapes for which the ring row's summation order is pinned against torch's on the device
                 on_device = (Tall >= 256 and query_states.shape[1] == 32 and query_states.shape[0] <= 8
                              and (lw.weights is None or lw.weights.dtype == torch.float16) and lw.max_length >= Tall)
-                line = lw.decode_row(query_states, Tall) if on_device else None   # (creates the store)
+                if on_device and lw.weights is None:
+                    lw.decode_row(query_states, Tall)   # creates the store
                 tables = self._memo.steps(past_key_value, query_states.device, self.quant_strategy == "uniform_group", known)
                 if tables is not None:
                     done = tables.step(query_states, key_states, value_states, past_key_value, *self._res, n, Tall,
@@ -264,7 +265,9 @@ class HqeAttentionLayer:
             else:
                 # Classes that do not cover every position once, as one call through the general path; else the plain
                 # sequence of the reference: the attention, the ring row, two copies.
-                step = dict(ring_line=line, append=(*self._res, n)) if one_call else None
+                step = None
+                if one_call:
+                    step = dict(ring_line=lw.decode_row(query_states, Tall) if on_device else None, append=(*self._res, n))
                 attn_weights, attn_output = qkv_matmul_hqe_2(query_states, past_key_value, attention_mask,
                                                              self.head_dim, self.quant_strategy, memo=self._memo,
                                                              tail=(key_states, value_states), step=step)
