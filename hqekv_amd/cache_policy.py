@@ -16,8 +16,9 @@ survivors (quant/hqe_2.py:661-670).
 Two engines produce the same bytes.  ``gather`` (the default wherever it applies): everything the reference
 moves is a whole block of 32 tokens and every block ends in exactly one place, so the host works out, per
 block, where each class's blocks come from (``hqekv_plan_side``, the library's host-side planner: one C call
-per side over a few thousand entries), and ONE kernel launch per side
-(``hqekv_cache_migrate``) rebuilds all classes from the old ones and the new tokens -- survivors copied, demoted
+per side over a few thousand entries), and ONE kernel launch (``hqekv_cache_migrate_both``, from ``_host.compress``;
+``hqekv_cache_migrate``, one per side, for what that does not take: new tokens that are not dense rows, rankings
+already spelt out) rebuilds all classes from the old ones and the new tokens -- survivors copied, demoted
 blocks dequantised and re-quantised, new blocks quantised, evicted blocks left out, positions re-ranked; the
 device is waited for once, to fetch the two block rankings.  ``steps``: the general engine for selections that
 are not made of whole aligned blocks (token-level V selections): the reference's sequence of moves with
