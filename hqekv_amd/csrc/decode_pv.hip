@@ -146,7 +146,8 @@ __device__ __forceinline__ void pt_class_job(const SegDev &sg, int blk0, int blk
         v[2 * g + 1] = (g & 1) ? as_u32(half_pair<1>(za[g >> 1], zb[g >> 1])) : as_u32(half_pair<0>(za[g >> 1], zb[g >> 1]));
       }
       // Tokens past the end hold the last row's codes and probability zero; with scale and zero point zero too they are
-      // zeros, where an infinity in the last row would be 0 x inf.
+      // zeros, where an infinity in the last row would be 0 x inf.  Only in a block that ends short: masks in every block cost
+      // a step at 32k tokens 0.2 us (19.6 -> 19.8), these 0.1, and nothing at 8 x 64k (masks everywhere: 152.4 -> 152.9).
       if ((uint32_t)(blk + 1) * BLOCK > n_tok) {
         const uint32_t left = n_tok - min((uint32_t)blk * BLOCK + 2u * tid, n_tok), mask = (left > 0 ? 0xffffu : 0u) | (left > 1 ? 0xffff0000u : 0u);
 #pragma unroll
