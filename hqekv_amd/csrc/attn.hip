@@ -1926,6 +1926,46 @@ __global__ __launch_bounds__(CB_CH * CB_SLICES) void pv_combine_kernel(const flo
   }
 }
 
+// The same sum after pv_tiles_kernel, where nothing rides along: 256 threads, 16 bytes of a chunk per lane, LANES x 4
+// channels of a row per workgroup.  Bound by latency: pv_combine_kernel's workgroups of 16 waves, four to a row, fill the
+// chip at 128 rows and come in two, four, eight rounds beyond, whatever the number of chunks.  A decode step with it / with
+// this, device time, us: B = 1 x 1k tokens 10.9 / 10.8, 4 x 2k 14.7 / 13.3, 8 x 2k 19.3 / 15.9, 16 x 2k 28.0 / 20.7, 16 x 8k
+// 60.3 / 53.6, 8 x 64k 159.0 / 154.6.
+// The additions are that kernel's, in its order: 32 strided slices of the chunks, neighbouring slices, the 16 pairs.
+constexpr int RS_THREADS = 256, RS_FLIGHT = 8;
+template <int LANES>
+__global__ __launch_bounds__(RS_THREADS) void pv_rows_sum_kernel(const float *__restrict__ partial, half_t *__restrict__ out, int n_chunks, uint32_t n_bhq) {
+  constexpr int GROUPS = RS_THREADS / LANES, OWN = CB_SLICES / GROUPS, ROW = 128 / 4;   // a group of lanes has slices g, g + GROUPS, ...
+  static_assert(RS_FLIGHT % OWN == 0, "a request's slice is known at compile time");
+  __shared__ f4_t sh[CB_SLICES][LANES];
+  const int lane = threadIdx.x % LANES, g = threadIdx.x / LANES;
+  const uint32_t at = blockIdx.x * ROW + blockIdx.y * LANES, stride = n_bhq * ROW;
+  const f4_t *src = reinterpret_cast<const f4_t *>(partial) + at + lane;
+  f4_t v[OWN];
+#pragma unroll
+  for (int k = 0; k < OWN; ++k) v[k] = (f4_t){0.f, 0.f, 0.f, 0.f};
+  for (int c0 = g; c0 < n_chunks; c0 += GROUPS * RS_FLIGHT) {
+    f4_t t[RS_FLIGHT];
+#pragma unroll
+    for (int k = 0; k < RS_FLIGHT; ++k) {
+      t[k] = (f4_t){0.f, 0.f, 0.f, 0.f};
+      if (c0 + k * GROUPS < n_chunks) t[k] = src[(uint64_t)(c0 + k * GROUPS) * stride];
+    }
+#pragma unroll
+    for (int k = 0; k < RS_FLIGHT; ++k) v[k % OWN] += t[k];
+  }
+#pragma unroll
+  for (int k = 0; k < OWN; ++k) sh[g + k * GROUPS][lane] = v[k];
+  __syncthreads();
+  if (threadIdx.x < 4 * LANES) {   // a channel each
+    const float *col = reinterpret_cast<const float *>(&sh[0][0]) + threadIdx.x;
+    float t = col[0] + col[4 * LANES];
+#pragma unroll
+    for (int k = 2; k < CB_SLICES; k += 2) t += col[4 * LANES * k] + col[4 * LANES * (k + 1)];
+    out[(uint64_t)at * 4 + threadIdx.x] = (half_t)t;
+  }
+}
+
 // =============================================================================== host side
 
 // With a plan: the launches of decode_qk.hip and decode_pv.hip.  Else
@@ -2205,6 +2245,18 @@ static int launch_pv(const SegTable &tb, int64_t chunk, void *p, void *out, floa
   const bool combine = (stages & 2) && !fz.arrive;   // folded: the last p.V workgroups have written the output
   const bool epilogue = ep && (ep->ring_line || ep->app_rows > 0 || ep->leave_bits) && stages == 3;
   if (!combine && !epilogue) return HQEKV_OK;
+  if (tb.per_unit && !epilogue) {
+    // A workgroup per row, two where rows are few and long (device time of a step, one / two / the 16-wave form, us: 32 rows
+    // of 33 chunks 13.1 / 13.3 / 13.5, of 52 16.2 / 15.8 / 16.0, of 103 21.6 / 21.0 / 21.0; 120 rows of 56 27.0 / - / 28.2).
+    const bool one = n_bhq >= 96 || tb.total_units <= 40;
+#define LAUNCH(LANES_)                                                                                                                        \
+  hipLaunchKernelGGL((pv_rows_sum_kernel<LANES_>), dim3((unsigned)n_bhq, 32 / LANES_), dim3(RS_THREADS), 0, st, partial, (half_t *)out, \
+                     (int)tb.total_units, (uint32_t)n_bhq)
+    if (one) LAUNCH(32);
+    else LAUNCH(16);
+#undef LAUNCH
+    return check_launch("pv_rows_sum_kernel");
+  }
   // The epilogue rides in the combine launch as extra workgroups: as many layers of grid.z (B * Hq * D / 32 workgroups each)
   // as make one workgroup per RING_SPAN columns of the ring row at the least.  Without a combine (folded into p.V) the
   // launch holds the epilogue alone.
