@@ -2246,14 +2246,14 @@ static int launch_pv(const SegTable &tb, int64_t chunk, void *p, void *out, floa
   const bool epilogue = ep && (ep->ring_line || ep->app_rows > 0 || ep->leave_bits) && stages == 3;
   if (!combine && !epilogue) return HQEKV_OK;
   if (tb.per_unit && !epilogue) {
-    // A workgroup per row, two where rows are few and long (device time of a step, one / two / the 16-wave form, us: 32 rows
-    // of 33 chunks 13.1 / 13.3 / 13.5, of 52 16.2 / 15.8 / 16.0, of 103 21.6 / 21.0 / 21.0; 120 rows of 56 27.0 / - / 28.2).
+    // A workgroup per row, four where rows are few and long (device time of a step, one / four / the 16-wave form, us: 32 rows
+    // of 33 chunks 13.1 / 13.5 / 13.5, of 52 16.4 / 15.7 / 15.9, of 103 21.8 / 20.7 / 20.9; 120 rows of 56 27.0 / - / 28.2).
     const bool one = n_bhq >= 96 || tb.total_units <= 40;
 #define LAUNCH(LANES_)                                                                                                                        \
   hipLaunchKernelGGL((pv_rows_sum_kernel<LANES_>), dim3((unsigned)n_bhq, 32 / LANES_), dim3(RS_THREADS), 0, st, partial, (half_t *)out, \
                      (int)tb.total_units, (uint32_t)n_bhq)
     if (one) LAUNCH(32);
-    else LAUNCH(16);
+    else LAUNCH(8);
 #undef LAUNCH
     return check_launch("pv_rows_sum_kernel");
   }

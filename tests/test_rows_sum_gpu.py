@@ -9,7 +9,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("B,Hq,Hkv", [(1, 4, 1), (3, 32, 8), (1, 15, 3), (2, 32, 2)])
-@pytest.mark.parametrize("chunks", [1, 2, 7, 8, 9, 31, 32, 33, 40, 41, 64, 65, 103])
+@pytest.mark.parametrize("chunks", [1, 2, 7, 8, 9, 31, 32, 33, 40, 41, 64, 65, 103, 257])
 def test_exact_sums(dev, B, Hq, Hkv, chunks):
     """Probabilities of 2^-6 and zero, values of small integers: every partial sum is a multiple of 2^-6 below 2^13."""
     from hqekv_amd import _lib
