@@ -1,5 +1,6 @@
 // p.V of a decode step on matrix instructions (see decode_tiles.h).
 #include "decode_tiles.h"
+#include "step_epilogue.h"
 
 #pragma clang fp contract(off)
 
@@ -29,6 +30,59 @@ struct PtLds {
   half_t p[BUFS][HP][PT_PSTRIDE];
 };
 
+// (max, 1 / sum exp) of a row from its tiles' pairs, by sixteen lanes; up to 64 of them are read at once (past the last one:
+// the last one again, left out of the sum)
+__device__ __forceinline__ void row16_read(const float2 *sp, int n_stat, int lane, float2 (&sv)[4]) {
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    if (k == 0 || n_stat > 16 * k) {
+      uint32_t w[2];
+      load_words<2, Words4<2>>(sp, 8u * (uint32_t)min(lane + 16 * k, n_stat - 1), w);
+      sv[k] = make_float2(__builtin_bit_cast(float, w[0]), __builtin_bit_cast(float, w[1]));
+    }
+}
+__device__ __forceinline__ float row16_max(float v) {
+  v = fmaxf(v, dpp_f<0xB1>(v));
+  v = fmaxf(v, dpp_f<0x4E>(v));
+  v = fmaxf(v, dpp_f<0x141>(v));
+  return fmaxf(v, dpp_f<0x140>(v));
+}
+__device__ __forceinline__ float row16_sum(float v) {
+  v += dpp_f<0xB1>(v);
+  v += dpp_f<0x4E>(v);
+  v += dpp_f<0x141>(v);
+  return v + dpp_f<0x140>(v);
+}
+__device__ __forceinline__ float2 row16_merge(const float2 *sp, int n_stat, int lane, const float2 (&sv)[4]) {
+  float m = sv[0].x;
+#pragma unroll
+  for (int k = 1; k < 4; ++k)
+    if (n_stat > 16 * k) m = fmaxf(m, sv[k].x);
+  for (int e = lane + 64; e < n_stat; e += 16) m = fmaxf(m, sp[e].x);
+  m = row16_max(m);
+  float l = 0.f;
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    if (k == 0 || n_stat > 16 * k) l += lane + 16 * k < n_stat ? sv[k].y * __expf(sv[k].x - m) : 0.f;
+  for (int e = lane + 64; e < n_stat; e += 16) {
+    const float2 w = sp[e];
+    l += w.y * __expf(w.x - m);
+  }
+  return make_float2(m, 1.0f / row16_sum(l));
+}
+// TWICE: the product is rounded to fp32 before it is rounded to fp16, always.  Left to the compiler some places get a mixed
+// multiply-add that rounds once: one in some ten thousand probabilities is another fp16 number then, and the ring row would
+// not be the sum of the probabilities that the caller sees.
+template <bool TWICE>
+__device__ __forceinline__ half_t pt_probability(half_t x, float m, float inv_l) {
+  float p = __expf((float)x - m) * inv_l;
+  if (TWICE) asm("" : "+v"(p));
+  return (half_t)p;
+}
+
+constexpr int PT_LAST_ROWS = 16;    // partial rows whose loads are in flight together
+constexpr int PT_RING_ROWS = 256;   // (b, head) rows of a step whose ring row rides in the p.V launch
+
 // What a thread holds of a block's logits on their way to LDS.  Positions in runs of 32 and an even token count: a pair
 // of neighbouring tokens for every other head (thread t: pair t % 128, heads t / 128, t / 128 + 2, ...), one 4-byte access
 // each.  Else: token t for every head.
@@ -38,8 +92,8 @@ struct PtValues {
   uint32_t x[HP];
 };
 
-template <int BITS, int HP, bool EXACT, bool NORMAL, bool LOOP, bool FUSED, bool PAIRED, typename StatsLoad, typename StatsMerge>
-__device__ __forceinline__ void pt_class_job(const SegDev &sg, int blk0, int blk1, int bh, int wave, int lane, half_t *rows, int64_t Tall,
+template <int BITS, int HP, bool EXACT, bool NORMAL, bool LOOP, bool FUSED, bool LAST, bool PAIRED, typename StatsLoad, typename StatsMerge>
+__device__ __forceinline__ void pt_class_job(const SegDev &sg, int blk0, int blk1, int bh, int wave, int lane, const half_t *rows, half_t *prows, int64_t Tall,
                                              int nrep_arg, PtLds<HP, LOOP> &lds, const float *ml, f4_t (&acc)[8], StatsLoad &&load_stats,
                                              StatsMerge &&merge_stats) {
   using G = PtGeom<BITS>;
@@ -110,7 +164,7 @@ __device__ __forceinline__ void pt_class_job(const SegDev &sg, int blk0, int blk
   };
   // fused: the row holds scaled logits: p = rnd16(exp(x - M) / L), written back for the caller.  Every position belongs to
   // exactly one token of exactly one V class, so nobody else touches it.
-  auto probability = [&](half_t x, int h) { return FUSED ? (half_t)(__expf((float)x - ml[2 * h]) * ml[2 * h + 1]) : x; };
+  auto probability = [&](half_t x, int h) { return FUSED ? pt_probability<LAST>(x, ml[2 * h], ml[2 * h + 1]) : x; };
   auto commit = [&](int blk, int buf) {
     if constexpr (PAIRED) {
       const bool valid = (uint32_t)blk * BLOCK + 2u * pt < n_tok;
@@ -123,7 +177,7 @@ __device__ __forceinline__ void pt_class_job(const SegDev &sg, int blk0, int blk
           if (FUSED && valid) {
             Words2<1> w;
             w.v[0] = p;
-            gstore(rows + (int64_t)h * Tall, f.pos, w);
+            gstore(prows + (int64_t)h * Tall, f.pos, w);
           }
           *reinterpret_cast<uint32_t *>(&lds.p[buf][h][2 * pt]) = valid ? p : 0u;
         }
@@ -134,7 +188,7 @@ __device__ __forceinline__ void pt_class_job(const SegDev &sg, int blk0, int blk
       for (int h = 0; h < HP; ++h)
         if (h < nrep) {
           const half_t p = probability(__builtin_bit_cast(half_t, (uint16_t)f.x[h]), h);
-          if (FUSED && valid) gstore(rows + (int64_t)h * Tall, f.pos, p);
+          if (FUSED && valid) gstore(prows + (int64_t)h * Tall, f.pos, p);
           lds.p[buf][h][tid] = valid ? p : (half_t)0;
         }
     }
@@ -243,9 +297,15 @@ __device__ __forceinline__ void pt_class_job(const SegDev &sg, int blk0, int blk
   }
 }
 
-template <int HP, bool EXACT, bool LOOP, bool FUSED>
-__global__ __launch_bounds__(PT_WAVES * 64, HP <= 8 ? (LOOP ? 4 : 6) : 2) void pv_tiles_kernel(SegTable tb, half_t *__restrict__ p, float *__restrict__ partial,
-                                                                   TilesArgs ta, int64_t Tall, int64_t n_bhq, FuseArgs fz) {
+struct PtEpilogue {
+  half_t ring[RING_LDS_HEADS * RING_SPAN_SHORT];
+  float2 ml[PT_RING_ROWS];   // (max, 1 / sum exp) of every (b, head) row
+};
+
+// `logits` is `p` unless LAST: then the logits lie in the workspace.
+template <int HP, bool EXACT, bool LOOP, bool FUSED, bool LAST>
+__device__ __forceinline__ void pv_tiles_body(const SegTable &tb, const half_t *logits, half_t *p, float *partial, const TilesArgs &ta, int64_t Tall,
+                                              int64_t n_bhq, const FuseArgs &fz) {
   __shared__ __align__(16) PtLds<HP, LOOP> lds;
   __shared__ __align__(16) float red[PT_WAVES][HP][128];
   __shared__ float ml[2 * HP];   // (max, 1 / sum exp) of each head's row
@@ -254,12 +314,14 @@ __global__ __launch_bounds__(PT_WAVES * 64, HP <= 8 ? (LOOP ? 4 : 6) : 2) void p
   const SegDev sg = tb.seg[tiles_segment(tb, u)];
   const int b = tiles_batch_row(ta, bh), hkv = bh - b * ta.Hkv;
   const int Hq = ta.hq_slice & 0xffff, head0 = first_head(ta.hq_slice, hkv), nrep = EXACT ? HP : ta.nrep;
-  half_t *rows = p + ((int64_t)b * Hq + head0) * Tall;
+  const half_t *rows = logits + ((int64_t)b * Hq + head0) * Tall;
+  half_t *prows = p + ((int64_t)b * Hq + head0) * Tall;
   f4_t acc[8];
 #pragma unroll
   for (int c = 0; c < 8; ++c) acc[c] = (f4_t){0.f, 0.f, 0.f, 0.f};
   // wave w merges the per-tile pairs of heads w, w + 4, ...; up to 256 tiles of the first are read once, ahead of the rest
-  // (past the last tile: the last one again, left out of the sum)
+  // (past the last tile: the last one again, left out of the sum).  LAST: sixteen lanes a head, as the ring row's workgroups
+  // do it for every row of the step, hence with the same bits.
   float2 sv[4];
   auto read_stats = [&](const float2 *sp) {
 #pragma unroll
@@ -270,12 +332,25 @@ __global__ __launch_bounds__(PT_WAVES * 64, HP <= 8 ? (LOOP ? 4 : 6) : 2) void p
         sv[k] = make_float2(__builtin_bit_cast(float, w[0]), __builtin_bit_cast(float, w[1]));
       }
   };
-  const float2 *srow = fz.stats + ((int64_t)b * Hq + head0 + min(wave, nrep - 1)) * fz.n_stat;
+  const int first = LAST ? (int)threadIdx.x >> 4 : wave;
+  const float2 *srow = fz.stats + ((int64_t)b * Hq + head0 + min(first, nrep - 1)) * fz.n_stat;
   auto load_stats = [&]() {
-    if (FUSED) read_stats(srow);
+    if constexpr (LAST) row16_read(srow, fz.n_stat, lane & 15, sv);
+    else if (FUSED) read_stats(srow);
   };
   auto merge_stats = [&]() {
     if (!FUSED) return;
+    if constexpr (LAST) {
+      if (wave * 4 < nrep) {
+        const float2 v = row16_merge(srow, fz.n_stat, lane & 15, sv);
+        if ((lane & 15) == 0 && first < nrep) {
+          ml[2 * first] = v.x;
+          ml[2 * first + 1] = v.y;
+        }
+      }
+      __syncthreads();
+      return;
+    }
     for (int h = wave; h < nrep; h += PT_WAVES) {
       const float2 *sp = srow + (int64_t)(h - wave) * fz.n_stat;
       if (h != wave) read_stats(sp);
@@ -304,8 +379,8 @@ __global__ __launch_bounds__(PT_WAVES * 64, HP <= 8 ? (LOOP ? 4 : 6) : 2) void p
   const int unit = u - sg.unit_begin, per = tb.per_unit, b0 = unit * per;
   const bool paired = qt_runs(sg) && sg.n_tokens % 2 == 0;
 #define HQ_JOB_P(B_, NORMAL_, PAIRED_)                                                                                                   \
-  pt_class_job<B_, HP, EXACT, NORMAL_, LOOP, FUSED, PAIRED_>(sg, b0, min(b0 + per, (int)((sg.n_tokens + PtGeom<B_>::BLOCK - 1) / PtGeom<B_>::BLOCK)), \
-                                                             bh, wave, lane, rows, Tall, nrep, lds, ml, acc, load_stats, merge_stats)
+  pt_class_job<B_, HP, EXACT, NORMAL_, LOOP, FUSED, LAST, PAIRED_>(sg, b0, min(b0 + per, (int)((sg.n_tokens + PtGeom<B_>::BLOCK - 1) / PtGeom<B_>::BLOCK)), \
+                                                             bh, wave, lane, rows, prows, Tall, nrep, lds, ml, acc, load_stats, merge_stats)
 #define HQ_JOB(B_, NORMAL_)                  \
   do {                                       \
     if (paired) HQ_JOB_P(B_, NORMAL_, true); \
@@ -341,8 +416,92 @@ __global__ __launch_bounds__(PT_WAVES * 64, HP <= 8 ? (LOOP ? 4 : 6) : 2) void p
     float2 v[PT_WAVES];
 #pragma unroll
     for (int w = 0; w < PT_WAVES; ++w) v[w] = *reinterpret_cast<const float2 *>(&red[w][h][c]);
-    *reinterpret_cast<float2 *>(dst + h * 128 + c) = make_float2(((v[0].x + v[1].x) + v[2].x) + v[3].x, ((v[0].y + v[1].y) + v[2].y) + v[3].y);
+    const float2 sum = make_float2(((v[0].x + v[1].x) + v[2].x) + v[3].x, ((v[0].y + v[1].y) + v[2].y) + v[3].y);
+    if constexpr (LAST) {
+      __hip_atomic_store(reinterpret_cast<uint64_t *>(dst + h * 128 + c), __builtin_bit_cast(uint64_t, sum), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    } else {
+      *reinterpret_cast<float2 *>(dst + h * 128 + c) = sum;
+    }
   }
+  if constexpr (LAST) {
+    // The rows are in memory when their stores are acknowledged; whoever counts the last of this (b, kv head)'s workgroups
+    // adds them up, in order.  (Agent-scope accesses go past the L2, which the XCDs do not share; see FuseArgs.)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    __shared__ int last;
+    if (threadIdx.x == 0) last = __hip_atomic_fetch_add(&fz.arrive[bh], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == (uint32_t)tb.total_units;
+    __syncthreads();
+    if (!last) return;
+    // 16 bytes of a row per lane; HP = 4: the even and the odd rows by one half of the workgroup each.
+    constexpr int LANES = HP * 32, GROUPS = PT_WAVES * 64 / LANES;
+    static_assert(GROUPS >= 1, "a row in one go");
+    const int at = threadIdx.x % LANES, g = threadIdx.x / LANES;
+    const bool mine = EXACT || at < nrep * 32;
+    const uint32_t row_b = (uint32_t)n_bhq * 512u;   // (the rows of a short launch span a few MB)
+    const rsrc_t rows_of = make_rsrc(partial + ((int64_t)b * Hq + head0) * 128, (uint32_t)(tb.total_units - 1) * row_b + (uint32_t)nrep * 512u);
+    f4_t v = (f4_t){0.f, 0.f, 0.f, 0.f};
+    if (mine) {
+      for (int c0 = 0; c0 < tb.total_units; c0 += GROUPS * PT_LAST_ROWS) {
+        f4_t t[PT_LAST_ROWS];
+        static_for<PT_LAST_ROWS>([&](auto I_) {   // (past the last row: zeros, without a trip to memory)
+          constexpr int I = decltype(I_)::value;
+          t[I] = __builtin_bit_cast(f4_t, __builtin_amdgcn_raw_buffer_load_b128(rows_of, 16 * at + (c0 + GROUPS * I + g) * (int)row_b, 0, 16));   // sc1
+        });
+        static_for<PT_LAST_ROWS>([&](auto I_) { v += t[decltype(I_)::value]; });
+      }
+    }
+    if constexpr (GROUPS > 1) {
+      float *half = &red[0][0][0];
+      if (g == 1 && mine) *reinterpret_cast<f4_t *>(half + 4 * at) = v;
+      __syncthreads();
+      if (g == 0 && mine) v += *reinterpret_cast<const f4_t *>(half + 4 * at);
+    }
+    if (g == 0 && mine) {
+      uint2 w = make_uint2(as_u32(pack_h2((half_t)v[0], (half_t)v[1])), as_u32(pack_h2((half_t)v[2], (half_t)v[3])));
+      *reinterpret_cast<uint2 *>(fz.out + ((int64_t)b * Hq + head0) * 128 + 4 * at) = w;
+    }
+  }
+}
+
+template <int HP, bool EXACT, bool LOOP, bool FUSED>
+__global__ __launch_bounds__(PT_WAVES * 64, HP <= 8 ? (LOOP ? 4 : 6) : 2) void pv_tiles_kernel(SegTable tb, half_t *__restrict__ p, float *__restrict__ partial,
+                                                                   TilesArgs ta, int64_t Tall, int64_t n_bhq, FuseArgs fz) {
+  pv_tiles_body<HP, EXACT, LOOP, FUSED, false>(tb, p, p, partial, ta, Tall, n_bhq, fz);
+}
+
+template <int HP, bool EXACT>
+__global__ __launch_bounds__(PT_WAVES * 64, 4) void pv_last_kernel(SegTable tb, const half_t *__restrict__ logits, half_t *__restrict__ p,
+                                                                   float *__restrict__ partial, TilesArgs ta, int64_t Tall, int64_t n_bhq, FuseArgs fz,
+                                                                   StepEpilogue ep) {
+  if ((int)blockIdx.y < tb.total_units) {
+    pv_tiles_body<HP, EXACT, false, true, true>(tb, logits, p, partial, ta, Tall, n_bhq, fz);
+    return;
+  }
+  __shared__ __align__(16) PtEpilogue sh;
+  if (ep.ring_line) {
+    const int lane = threadIdx.x & 15, rows = ep.B * ep.Hq;
+    for (int row = threadIdx.x >> 4; row < rows; row += 2 * PT_WAVES * 4) {   // two rows at a time
+      float2 sv[2][4];
+#pragma unroll
+      for (int k = 0; k < 2; ++k) row16_read(fz.stats + (int64_t)min(row + k * PT_WAVES * 4, rows - 1) * fz.n_stat, fz.n_stat, lane, sv[k]);
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const int at = min(row + k * PT_WAVES * 4, rows - 1);
+        const float2 v = row16_merge(fz.stats + (int64_t)at * fz.n_stat, fz.n_stat, lane, sv[k]);
+        if (lane == 0) sh.ml[at] = v;
+      }
+    }
+    __syncthreads();
+  }
+  step_epilogue_block<false>(ep, (int64_t)(blockIdx.y - tb.total_units) * gridDim.x + blockIdx.x, (int64_t)(gridDim.y - tb.total_units) * gridDim.x,
+                             sh.ring, [&](int row, uint64_t quad) {
+    const float2 ml = sh.ml[row];
+    uint64_t v = 0;
+#pragma unroll
+    for (int i = 0; i < RING_V; ++i)
+      v |= (uint64_t)__builtin_bit_cast(uint16_t, pt_probability<true>(__builtin_bit_cast(half_t, (uint16_t)(quad >> (16 * i))), ml.x, ml.y)) << (16 * i);
+    return v;
+  });
 }
 
 // =============================================================================== host side
@@ -366,6 +525,41 @@ int launch_pv_tiles(const SegTable &tb, void *p, float *partial, int64_t B, int6
 #undef LAUNCH_H
 #undef LAUNCH
   return check_launch("pv_tiles_kernel");
+}
+
+// One p.V launch that also adds its partial rows up and carries the step's epilogue, in place of two launches.  What it adds
+// to every workgroup's end (stores acknowledged by memory, a counter, 2 KB per partial row into one CU) equals a launch's
+// start at about 20 rows; the host saves 2.5 us at any size.  A step of the fp16 / 8 / 4 / 2-bit mix, B = 1, device time in
+// us, three launches / two: 1k tokens 11.1 / 10.3, 2k 11.0 / 10.4, 4k (18 rows) 12.1 / 11.6, 5k 12.2 / 12.1, 6k (25 rows)
+// 12.6 / 13.0, 8k 13.3 / 14.5; 4 x 2k 13.6 / 12.7, 4 x 4k 15.9 / 15.5, 16 x 2k 21.4 / 20.5, 8 x 4k 20.8 / 20.9; five heads per
+// KV head, 4 x 2k 14.7 / 13.0.  With and without an epilogue alike, so that a step and the separate calls give the same bits.
+constexpr int64_t PT_LAST_UNITS = 20;
+bool decode_in_two(const hqekv_seg *v_segs, int n_v, int64_t D, int64_t B, int64_t Hq, int64_t Hkv) {
+  if (n_v <= 0 || !tiles_fit(v_segs, n_v, false, D, B, Hq, Hkv) || Hq / Hkv > 8) return false;
+  const TilesPlan p = tiles_plan(v_segs, n_v, false, B * Hkv, Hq / Hkv);
+  return p.per_unit == 1 && p.units <= PT_LAST_UNITS;
+}
+bool pv_last_takes(const StepEpilogue &ep, int64_t Tall) {
+  return !ep.ring_line || (ep.B <= 8 && ep.Hq <= RING_LDS_HEADS && (int64_t)ep.B * ep.Hq <= PT_RING_ROWS && Tall >= RING_V);   // what the ring's LDS tile covers
+}
+
+int launch_pv_last(const SegTable &tb, const void *logits, void *probs, float *partial, int64_t B, int64_t Hq, int64_t Hkv, int64_t Tall,
+                   const FuseArgs &fz, const StepEpilogue &ep, hipStream_t st) {
+  const TilesArgs ta = tiles_args(B, Hq, Hkv);
+  const int nrep = ta.nrep;
+  int64_t more = 0;   // workgroups for the epilogue
+  if (ep.ring_line) more = (Tall + RING_SPAN_SHORT - 1) / RING_SPAN_SHORT;
+  else if (ep.app_rows > 0 || ep.leave_bits) more = 1;
+  const dim3 grid((unsigned)(B * Hkv), (unsigned)(tb.total_units + (more + B * Hkv - 1) / (B * Hkv)));
+#define LAUNCH(HP_, EXACT_)                                                                                                                     \
+  hipLaunchKernelGGL((pv_last_kernel<HP_, EXACT_>), grid, dim3(PT_WAVES * 64), 0, st, tb, (const half_t *)logits, (half_t *)probs, partial, ta, \
+                     Tall, B *Hq, fz, ep)
+  if (nrep == 4) LAUNCH(4, true);
+  else if (nrep < 4) LAUNCH(4, false);
+  else if (nrep == 8) LAUNCH(8, true);
+  else LAUNCH(8, false);
+#undef LAUNCH
+  return check_launch("pv_last_kernel");
 }
 
 }  // namespace hq

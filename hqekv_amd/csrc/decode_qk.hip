@@ -260,7 +260,9 @@ __device__ __forceinline__ void qt_rows_tile(const SegDev &sg, int tile, int bh,
                                  [&](int t) { return qk_alone<16, false, true>(sg, bh, token(t), qrow()); });
 }
 
-template <int HP, bool FUSED>
+// COUNT: the p.V launch of the same call counts arrivals, from zero (a form of its own: a test for it costs every launch a
+// scalar load in its prologue, 0.3 us of a step at 32k tokens).
+template <int HP, bool FUSED, bool COUNT>
 __global__ __launch_bounds__(QT_WAVES * 64, HP == 16 ? 2 : HP == 4 || FUSED ? 5 : 4) void qk_tiles_kernel(SegTable tb, const half_t *__restrict__ q,
                                                                     half_t *__restrict__ scores, TilesArgs ta, int64_t Tall, FuseArgs fz) {
   __shared__ __align__(16) QtLds<HP> lds;
@@ -277,6 +279,7 @@ __global__ __launch_bounds__(QT_WAVES * 64, HP == 16 ? 2 : HP == 4 || FUSED ? 5 
     load_words<4, Words2<4>>(q + ((int64_t)b * Hq + head0) * 128, (uint32_t)min(n % HP, nrep - 1) * 256u + 64u * wave + 16u * r, w);
     qv = (u32x4){w[0], w[1], w[2], w[3]};
   }
+  if (COUNT && u == 0 && threadIdx.x == 0) fz.arrive[bh] = 0u;
   const int tile = u - sg.unit_begin;
   const int head = (4 * r) % HP + wave;   // the head this lane finishes
   const bool has_head = head < nrep;
@@ -664,13 +667,13 @@ int launch_qk_tiles(const SegTable &tb, const void *q, void *scores, int64_t B, 
   const TilesArgs ta = tiles_args(B, Hq, Hkv);
   const int nrep = ta.nrep;
   const dim3 grid((unsigned)(B * Hkv), (unsigned)tb.total_units);
-#define LAUNCH(KERNEL_, HP_, FUSED_) \
-  hipLaunchKernelGGL((KERNEL_<HP_, FUSED_>), grid, dim3(QT_WAVES * 64), 0, st, tb, (const half_t *)q, (half_t *)scores, ta, Tall, fz)
-#define LAUNCH_H(HP_)                                                 \
-  if (tb.per_unit > 1 && fz.stats) LAUNCH(qk_long_kernel, HP_, true); \
-  else if (tb.per_unit > 1) LAUNCH(qk_long_kernel, HP_, false);       \
-  else if (fz.stats) LAUNCH(qk_tiles_kernel, HP_, true);              \
-  else LAUNCH(qk_tiles_kernel, HP_, false)
+#define LAUNCH(...) hipLaunchKernelGGL((__VA_ARGS__), grid, dim3(QT_WAVES * 64), 0, st, tb, (const half_t *)q, (half_t *)scores, ta, Tall, fz)
+#define LAUNCH_H(HP_)                                                             \
+  if (tb.per_unit > 1 && fz.stats) LAUNCH(qk_long_kernel<HP_, true>);             \
+  else if (tb.per_unit > 1) LAUNCH(qk_long_kernel<HP_, false>);                   \
+  else if (fz.stats && fz.arrive) LAUNCH(qk_tiles_kernel<HP_, true, (HP_ <= 8)>); \
+  else if (fz.stats) LAUNCH(qk_tiles_kernel<HP_, true, false>);                   \
+  else LAUNCH(qk_tiles_kernel<HP_, false, false>)
   if (nrep <= 4) { LAUNCH_H(4); } else if (nrep <= 8) { LAUNCH_H(8); } else { LAUNCH_H(16); }
 #undef LAUNCH_H
 #undef LAUNCH

@@ -134,5 +134,10 @@ int launch_qk_tiles(const SegTable &tb, const void *q, void *scores, int64_t B, 
                     hipStream_t st);
 int launch_pv_tiles(const SegTable &tb, void *p, float *partial, int64_t B, int64_t Hq, int64_t Hkv, int64_t Tall, const FuseArgs &fz,
                     hipStream_t st);
+// Short steps: p.V, the sum of its partial rows and the step's epilogue in one launch (decode_pv.hip).
+bool decode_in_two(const hqekv_seg *v_segs, int n_v, int64_t D, int64_t B, int64_t Hq, int64_t Hkv);
+bool pv_last_takes(const StepEpilogue &ep, int64_t Tall);
+int launch_pv_last(const SegTable &tb, const void *logits, void *probs, float *partial, int64_t B, int64_t Hq, int64_t Hkv, int64_t Tall,
+                   const FuseArgs &fz, const StepEpilogue &ep, hipStream_t st);
 
 }  // namespace hq
