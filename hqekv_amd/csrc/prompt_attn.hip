@@ -25,17 +25,20 @@ constexpr int PA_D = 128;
 constexpr int PA_WAVES = 4;
 constexpr int PA_THREADS = 64 * PA_WAVES;
 constexpr int PA_BC = 32;              // keys per score tile
-// How the four waves of a workgroup share its work.  KS = 1: 32 query rows each, 128 per workgroup, every wave walks all
-// key tiles (164 registers, 32 KB of LDS: three workgroups per CU).  KS = 2: the two waves of 32 query rows deal the key
-// tiles among themselves and merge their maxima, sums and outputs at the end: walks of half the length in twice as many
-// workgroups, for prompts whose 128-row workgroups would leave the chip waiting for the longest of them.  A step stages
-// two tiles, so LDS holds two workgroups per CU.
-template <int KS>
+// How the four waves of a workgroup share its work, and how many keys a wave takes at a time.
+// <1, 1>: 32 query rows each, 128 per workgroup, every wave walks all key tiles (164 registers, 32 KB of LDS: three
+// workgroups per CU).  For long prompts, which are bound by the chip's power: no order of the same instructions is faster.
+// <1, 2>: the same with 64 keys per step, two workgroups per CU.  A short prompt waits for its longest walk: a lone wave needs
+// 0.77 us for 32 keys and 1.2 us for 64 (one barrier, one maximum across the lane halves, one test of the rescale; the second
+// tile's products run beside the first one's exponentials).
+// <2, 1>: the two waves of 32 query rows deal the key tiles among themselves and merge their maxima, sums and outputs at the
+// end: walks of half the length in twice as many workgroups.  A step stages two tiles, so LDS holds two workgroups per CU.
+template <int KS_, int NB_>
 struct PaShape {
+  static constexpr int KS = KS_, NB = NB_, WGS = KS_ * NB_ == 1 ? 3 : 2;
   static constexpr int ROWS = 128 / KS;            // query rows per workgroup
-  static constexpr int STEP = PA_BC * KS;          // keys staged per step
+  static constexpr int STEP = PA_BC * NB * KS;     // keys staged per step
   static constexpr int TILE = STEP * PA_D;         // fp16 elements of one staged K (or V) step
-  static constexpr int WGS = KS == 1 ? 3 : 2;
 };
 
 struct PromptArgs {
@@ -100,9 +103,9 @@ __device__ __forceinline__ f16_t pa_scores(const half_t *ks, const h8_t (&qreg)[
   }
   return sc;
 }
-template <bool CAUSAL, int KS>
-__global__ __launch_bounds__(PA_THREADS, PaShape<KS>::WGS) void prompt_attn_kernel(PromptArgs a) {
-  using S = PaShape<KS>;
+template <bool CAUSAL, typename S>
+__global__ __launch_bounds__(PA_THREADS, S::WGS) void prompt_attn_kernel(PromptArgs a) {
+  constexpr int KS = S::KS, NB = S::NB;
   __shared__ __align__(16) half_t ks_all[2][S::TILE];
   __shared__ __align__(16) half_t vs_all[2][S::TILE];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -113,7 +116,14 @@ __global__ __launch_bounds__(PA_THREADS, PaShape<KS>::WGS) void prompt_attn_kern
   // the query heads of a KV head share one and meet in its L2.  With the rows of one head after the other (a head's row
   // blocks dealt to all XCDs): T = 32768 9.35 -> 8.04 ms, 8192 0.73 -> 0.57 ms, 4099 196 -> 165 us (32 heads over 8).
   const int nrep = a.Hq / a.Hkv;
-  const int qi = (int)blockIdx.x / a.BH, slot = (int)blockIdx.x % a.BH;
+  // Two workgroups per CU: the second 256 come in the opposite order (eight by eight, so that a KV head stays on its XCD), and a
+  // CU that began with a long walk is given a short one: T = 2048 54.4 -> 53.2 us, 3500 130 -> 124, 4099 171.6 -> 165.9.
+  int item = (int)blockIdx.x;
+  if (S::WGS == 2 && item >> 8 == 1) {
+    const int m = min((int)gridDim.x - 256, 256), g = a.by_xcd ? 8 : 1, p = item - 256;
+    item = 256 + m - g - p / g * g + p % g;
+  }
+  const int qi = item / a.BH, slot = item % a.BH;
   const int bh = a.by_xcd ? ((slot / 8 / nrep) * 8 + slot % 8) * nrep + slot / 8 % nrep : slot;
   const int q0 = ((int)gridDim.x / a.BH - 1 - qi) * S::ROWS;
   const int b = bh / a.Hq, hq = bh % a.Hq, hkv = hq / nrep;
@@ -163,30 +173,36 @@ __global__ __launch_bounds__(PA_THREADS, PaShape<KS>::WGS) void prompt_attn_kern
   // (rows past the end of the prompt are outside the buffer descriptors: whatever such a row holds in LDS -- zeros from
   // this fill or an older tile's finite values -- meets an exponential that is exactly zero)
 #pragma unroll
-  for (int i = 0; i < 4 * KS; ++i) *reinterpret_cast<uint4 *>(&vs_all[0][0] + (threadIdx.x + PA_THREADS * i) * 8) = make_uint4(0, 0, 0, 0);
+  for (int i = 0; i < 4 * KS * NB; ++i) *reinterpret_cast<uint4 *>(&vs_all[0][0] + (threadIdx.x + PA_THREADS * i) * 8) = make_uint4(0, 0, 0, 0);
   __syncthreads();
   pa_tile_dma<S::STEP>(src, 0, ks_all[0], vs_all[0], w);   // (a step past the last one is fetched and never used)
   auto step = [&](int j, const half_t *ks, const half_t *vs, half_t *ks_nxt, half_t *vs_nxt) {
-    const int k0 = j * S::STEP + sp * PA_BC;
+    const int k0 = j * S::STEP + sp * PA_BC * NB;
     wait_all_loads();   // this wave's part of step j, requested an iteration ago
     __syncthreads();
     pa_tile_dma<S::STEP>(src, (j + 1) * S::STEP, ks_nxt, vs_nxt, w);   // in flight across the products
-    ks += sp * PA_BC * PA_D;
-    vs += sp * PA_BC * PA_D;
+    ks += sp * PA_BC * NB * PA_D;
+    vs += sp * PA_BC * NB * PA_D;
     // (a tile that lies after every query of this wave is worked through like any other: all its elements are masked,
     // the maximum stays and the exponentials are zeros; skipping it would cost a copy of the accumulators per tile)
-    f16_t s = pa_scores(ks, qreg, n, h);
-    const bool edge = (k0 + PA_BC > T) || (CAUSAL && k0 + PA_BC - 1 > q0 + 32 * rg);   // some element of the tile is masked
+    f16_t s[NB];
+#pragma unroll
+    for (int i = 0; i < NB; ++i) s[i] = pa_scores(ks + i * PA_BC * PA_D, qreg, n, h);
+    const bool edge = (k0 + PA_BC * NB > T) || (CAUSAL && k0 + PA_BC * NB - 1 > q0 + 32 * rg);   // some element of the tile is masked
     // the running maximum is kept in units of the scaled logit (base-2 exponent); a raw score enters as s * sl2
-    if (edge) {   // (uniform per wave; one branch around all 16 selects)
+    if (edge) {   // (uniform per wave; one branch around all selects)
       const int last_key = (CAUSAL ? min(my_q, T - 1) : T - 1) - k0 - 4 * h;   // the last visible key, relative to element r's base
 #pragma unroll
-      for (int r = 0; r < 16; ++r)
-        if (8 * (r >> 2) + (r & 3) > last_key) s[r] = -INFINITY;
+      for (int i = 0; i < NB; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (32 * i + 8 * (r >> 2) + (r & 3) > last_key) s[i][r] = -INFINITY;
     }
     float raw = -INFINITY;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) raw = fmaxf(raw, s[r]);
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) raw = fmaxf(raw, s[i][r]);
     float mx = fmaxf(m, raw * sl2);   // (sl2 > 0)
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
     // (KS = 1: the first tile always holds key 0, which no query masks: mx is finite from then on)
@@ -203,28 +219,31 @@ __global__ __launch_bounds__(PA_THREADS, PaShape<KS>::WGS) void prompt_attn_kern
     }
     const float base = KS > 1 && mx == -INFINITY ? 0.f : mx;   // nothing but masked keys so far: exponentials of -inf are zero
     float part = 0.f;
-    h8_t p[2];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], sl2, -base));
-      part += e;
-      p[r >> 3][r & 7] = (half_t)e;
+    for (int i = 0; i < NB; ++i) {
+      h8_t p[2];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i][r], sl2, -base));
+        part += e;
+        p[r >> 3][r & 7] = (half_t)e;
+      }
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) {
+          // V^T operand through the transposing LDS read: a group of 16 lanes names four key rows x 32 bytes and each
+          // lane receives four consecutive keys of one channel; two reads (keys 4h + j, 8 + 4h + j) make the operand
+          const half_t *src_lo = vs + v_off[dt] + (32 * i + 16 * t) * PA_D;
+          const h4raw_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4f16((lds_h4_t *)(src_lo));
+          const h4raw_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4f16((lds_h4_t *)(src_lo + 8 * PA_D));
+          h8_t av;
+          __builtin_memcpy(&av, &lo, 8);
+          __builtin_memcpy(reinterpret_cast<char *>(&av) + 8, &hi, 8);
+          o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av, p[t], o[dt], 0, 0, 0);
+        }
     }
     lsum += part;
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int dt = 0; dt < 4; ++dt) {
-        // V^T operand through the transposing LDS read: a group of 16 lanes names four key rows x 32 bytes and each
-        // lane receives four consecutive keys of one channel; two reads (keys 4h + j, 8 + 4h + j) make the operand
-        const half_t *src_lo = vs + v_off[dt] + 16 * t * PA_D;
-        const h4raw_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4f16((lds_h4_t *)(src_lo));
-        const h4raw_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4f16((lds_h4_t *)(src_lo + 8 * PA_D));
-        h8_t av;
-        __builtin_memcpy(&av, &lo, 8);
-        __builtin_memcpy(reinterpret_cast<char *>(&av) + 8, &hi, 8);
-        o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av, p[t], o[dt], 0, 0, 0);
-      }
   };
   // two steps per round, so that each half works on fixed buffers; an odd count runs one step more, all of it masked
   for (int j = 0; j < n_steps; j += 2) {
@@ -501,11 +520,15 @@ static bool rows_16_byte_aligned(const void *p, int64_t s0, int64_t s1, int64_t 
   return ((uintptr_t)p & 15) == 0 && s0 % 8 == 0 && s1 % 8 == 0 && s2 % 8 == 0;
 }
 
-// Two waves per row group while the 128-row workgroups are fewer than two per CU (up to 480, B = 1 and 32 heads: T up to
-// 1900): T = 1003 29.3 -> 22.8 us, T = 1500 44.8 -> 36.7 us; at 512 it is even (T = 2048 61.0 against 57.3, B = 2 and
-// T = 1003 34.8 against 37.3), at 640 behind (65.5 against 70.5).  Four waves per row group never won (T = 500: 20.0
-// against 12.6 us).
-static int prompt_key_shares(int64_t T, int64_t BH) { return (T + 127) / 128 * BH > 480 ? 1 : 2; }
+// Which form, by the number of 128-row workgroups.  Up to 400 (B = 1 and 32 heads: T up to 1600) two waves per row group: 256
+// (T = 1003) 22.3 us against 25.3 of <1, 2> and 31.5 of <1, 1>, 384 (1500) 37.2 / 37.7 / 44.1; at 480 (1800) 49.3 / 46.4 /
+// 52.6.  Up to 1500 64 keys per step: 512 (2048) 53.2 against 60.5 of <1, 1>, 672 (28 heads over 4, 3000) 84.5 / 93.1, 1056
+// (4099) 165.9 / 171, 1376 (5500) 274 / 288; beyond it is behind: 2048 (8192) 580 / 573, 4128 (16384) 2218 / 2163.
+// Four waves per row group never won (T = 500: 20.0 against 12.6 us).
+static int prompt_form(int64_t T, int64_t BH) {
+  const int64_t wgs = (T + 127) / 128 * BH;
+  return wgs <= 400 ? 2 : wgs <= 1500 ? 1 : 0;
+}
 
 extern "C" int hqekv_prompt_attn(const void *q, const int64_t *q_strides, const void *k, const int64_t *k_strides,
                                  const void *v, const int64_t *v_strides, void *out, const int64_t *out_strides, int64_t B,
@@ -530,12 +553,15 @@ extern "C" int hqekv_prompt_attn(const void *q, const int64_t *q_strides, const 
   a.o_b = out_strides[0]; a.o_h = out_strides[1]; a.o_t = out_strides[2];
   a.Hq = (int32_t)Hq; a.Hkv = (int32_t)Hkv; a.T = (int32_t)T; a.scale = scale;
   a.BH = (int32_t)(B * Hq); a.by_xcd = (B * Hkv) % 8 == 0;
-  const int ks = prompt_key_shares(T, B * Hq);
-  const int64_t rows = 128 / ks, wgs = (T + rows - 1) / rows * B * Hq;
+  const int form = prompt_form(T, B * Hq);
+  const int64_t rows = form == 2 ? 64 : 128, wgs = (T + rows - 1) / rows * B * Hq;
   if (wgs > 0x7fffffffLL) return fail(HQEKV_E_UNSUPPORTED, "prompt_attn: T * B * Hq too large");
-#define LAUNCH(C_, K_) hipLaunchKernelGGL((prompt_attn_kernel<C_, K_>), dim3((unsigned)wgs), dim3(PA_THREADS), 0, (hipStream_t)stream, a)
-#define LAUNCH_K(C_) \
-  if (ks == 1) LAUNCH(C_, 1); else LAUNCH(C_, 2)
+#define LAUNCH(C_, KS_, NB_)                                                                                                                     \
+  hipLaunchKernelGGL((prompt_attn_kernel<C_, PaShape<KS_, NB_>>), dim3((unsigned)wgs), dim3(PA_THREADS), 0, (hipStream_t)stream, a)
+#define LAUNCH_K(C_)                    \
+  if (form == 2) LAUNCH(C_, 2, 1);      \
+  else if (form == 1) LAUNCH(C_, 1, 2); \
+  else LAUNCH(C_, 1, 1)
   if (causal) { LAUNCH_K(true); } else { LAUNCH_K(false); }
 #undef LAUNCH_K
 #undef LAUNCH
