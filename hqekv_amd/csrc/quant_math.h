@@ -81,12 +81,13 @@ __device__ __forceinline__ uint32_t first_zero_bits(const half_t (&x)[N]) {
   return r;
 }
 
-// One group of 32 contiguous values (16-byte aligned) by four neighbouring lanes, `sub` = 0 .. 3: codes, scale and zero are
-// stored by them.
+// One group of 32 contiguous values by four neighbouring lanes, `sub` = 0 .. 3, of which each holds eight: they store the codes.
+struct QuantScale {
+  half_t scale, zero;   // the same in all four lanes
+};
 template <int BITS>
-__device__ __forceinline__ void quant_group_of_4(const half_t *x, uint32_t sub, uint32_t *crow, half_t *scale, half_t *zero) {
+__device__ __forceinline__ QuantScale quant_group_of_4(uint4 raw, uint32_t sub, uint32_t *crow) {
   constexpr float INV_QMAX = 1.0f / (float)((1 << BITS) - 1);
-  const uint4 raw = *reinterpret_cast<const uint4 *>(x + sub * 8u);
   const half2_t p[4] = {bits_h2(raw.x), bits_h2(raw.y), bits_h2(raw.z), bits_h2(raw.w)};
 
   half2_t lo2 = __builtin_elementwise_min(__builtin_elementwise_min(p[0], p[1]), __builtin_elementwise_min(p[2], p[3]));
@@ -161,9 +162,15 @@ __device__ __forceinline__ void quant_group_of_4(const half_t *x, uint32_t sub, 
       if ((sub & 1) == 0) crow[sub >> 1] = h | (other << 16);
     }
   }
+  return {sc, mn_h};
+}
+// the same from memory (16-byte aligned), scale and zero stored, too
+template <int BITS>
+__device__ __forceinline__ void quant_group_of_4(const half_t *x, uint32_t sub, uint32_t *crow, half_t *scale, half_t *zero) {
+  const QuantScale q = quant_group_of_4<BITS>(*reinterpret_cast<const uint4 *>(x + sub * 8u), sub, crow);
   if (sub == 0) {
-    *scale = sc;
-    *zero = mn_h;
+    *scale = q.scale;
+    *zero = q.zero;
   }
 }
 

@@ -20,29 +20,51 @@ namespace hq {
 
 // ---------------------------------------------------------------- rows: groups along a contiguous axis
 // 4 lanes per 32-element group, 8 contiguous fp16 (one 128-bit load) per lane.  grid.x enumerates
-// (outer slab, block of 64 groups); a slab's groups are numbered row-major over (row, group in row).
-template <int BITS>
+// (outer slab, block of 64 U groups); a slab's groups are numbered row-major over (row, group in row).  A wave takes 16 U
+// consecutive groups, its loads all in flight, and U = 4 stores their scales and zeros as 128 bytes each.  Bound by memory.
+template <int BITS, int U>
 __global__ __launch_bounds__(256) void quant_rows_kernel(
     const half_t *__restrict__ x, int64_t xo, int64_t xr, uint32_t *__restrict__ code, int64_t co,
     int64_t cr, half_t *__restrict__ scale, half_t *__restrict__ zero, int64_t so, int64_t sr,
     uint32_t groups_per_row, int gpr_shift, uint32_t groups_per_slab, uint32_t blocks_per_slab) {
   const uint32_t o = blockIdx.x / blocks_per_slab;
   const uint32_t blk = blockIdx.x - o * blocks_per_slab;
-  const uint32_t gin = blk * 64u + (threadIdx.x >> 2);
+  const uint32_t first = blk * (64u * U) + (threadIdx.x >> 6) * (16u * U) + ((threadIdx.x & 63u) >> 2);   // then every 16th
   const uint32_t sub = threadIdx.x & 3;
-  if (gin >= groups_per_slab) return;  // the four lanes of a group leave together
-  uint32_t r, g;
-  if (gpr_shift >= 0) {
-    r = gin >> gpr_shift;
-    g = gin & (groups_per_row - 1u);
-  } else {
-    r = gin / groups_per_row;
-    g = gin - r * groups_per_row;
+  if (first >= groups_per_slab) return;  // the four lanes of a group leave together
+  auto place = [&](uint32_t gin, uint32_t &r, uint32_t &g) {
+    if (gpr_shift >= 0) {
+      r = gin >> gpr_shift;
+      g = gin & (groups_per_row - 1u);
+    } else {
+      r = gin / groups_per_row;
+      g = gin - r * groups_per_row;
+    }
+  };
+  uint32_t r[U], g[U];
+  uint4 raw[U];
+#pragma unroll
+  for (int k = 0; k < U; ++k) {   // (past the last group: the lanes' first once more, not stored)
+    place(first + 16u * k < groups_per_slab ? first + 16u * k : first, r[k], g[k]);
+    raw[k] = *reinterpret_cast<const uint4 *>(x + (int64_t)o * xo + (int64_t)r[k] * xr + g[k] * 32u + sub * 8u);
   }
-
-  const int64_t at = (int64_t)o * so + (int64_t)r * sr + g;
-  quant_group_of_4<BITS>(x + (int64_t)o * xo + (int64_t)r * xr + g * 32u, sub, code + (int64_t)o * co + (int64_t)r * cr + g * BITS, scale + at,
-                         zero + at);
+  QuantScale mine = {};
+  uint32_t mr = r[0], mg = g[0];
+#pragma unroll
+  for (int k = 0; k < U; ++k) {
+    if (k && first + 16u * k >= groups_per_slab) break;
+    const QuantScale q = quant_group_of_4<BITS>(raw[k], sub, code + (int64_t)o * co + (int64_t)r[k] * cr + g[k] * BITS);
+    if (U == 1 || sub == k % U) {   // lane `sub` stores its quad's group `sub`
+      mine = q;
+      mr = r[k];
+      mg = g[k];
+    }
+  }
+  if (U == 1 ? sub == 0 : sub < U && first + 16u * sub < groups_per_slab) {
+    const int64_t at = (int64_t)o * so + (int64_t)mr * sr + mg;
+    scale[at] = mine.scale;
+    zero[at] = mine.zero;
+  }
 }
 
 // ---------------------------------------------------------------- K handed over token-major
@@ -53,11 +75,19 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(
 // of 8 groups (64 to 256 bytes of codes) instead of one group at a time.
 constexpr int QK_GROUPS_PER_BLOCK = 8;
 
+// Block i of the launch runs on XCD i mod 8: each XCD takes a contiguous range of (slab, block of groups).  A block writes 16
+// bytes of a channel's scales and 64 (2 bit) of its codes; with its neighbours on other XCDs every line went to memory in
+// pieces.  K of 8 x 8k tokens at 2 bit 8.9 -> 8.0 us, 8 x 16k 13.1 -> 11.4, 32 x 8k 26.4 -> 22.1.
+__device__ __forceinline__ uint32_t by_xcd(uint32_t i, uint32_t n) {
+  const uint32_t per = n / 8u;
+  return i < 8u * per ? (i & 7u) * per + (i >> 3) : i;
+}
+
 template <int BITS>
 __global__ __launch_bounds__(512) void quant_k_tokenmajor_kernel(
     const half_t *__restrict__ x, int64_t xo, int64_t xt, uint32_t *__restrict__ code, int64_t co,
     int64_t cr, half_t *__restrict__ scale, half_t *__restrict__ zero, int64_t so, int64_t sr,
-    uint32_t D, uint32_t n_groups) {
+    uint32_t D, uint32_t n_groups, uint32_t blocks_per_slab) {
   constexpr int PF = 32 / BITS;
   constexpr int WPG = 32 / PF;  // words per group
   constexpr int HALF = PF / 2;
@@ -65,9 +95,10 @@ __global__ __launch_bounds__(512) void quant_k_tokenmajor_kernel(
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t cp = lane & 7u, tg = lane >> 3;
-  const uint32_t G0 = blockIdx.x * QK_GROUPS_PER_BLOCK;
+  const uint32_t id = by_xcd(blockIdx.x, gridDim.x), slab = id / blocks_per_slab;
+  const uint32_t G0 = (id - slab * blocks_per_slab) * QK_GROUPS_PER_BLOCK;
   const uint32_t G = G0 + tg;
-  const int64_t o = blockIdx.y;
+  const int64_t o = slab;
   const uint32_t row_b = (uint32_t)xt * 2u;  // bytes between token rows
   const uint32_t groups_here = min((uint32_t)QK_GROUPS_PER_BLOCK, n_groups - G0);
   const rsrc_t rx = make_rsrc(x + o * xo + (int64_t)G0 * 32 * xt, (groups_here * 32u - 1u) * row_b + D * 2u);
@@ -130,6 +161,120 @@ __global__ __launch_bounds__(512) void quant_k_tokenmajor_kernel(
         zero[o * so + (int64_t)(c + ch) * sr + G] = lo2[ch];
       }
     }
+  }
+}
+
+// The same with a wave per token group and a lane per channel pair: whole token rows are read (256 bytes per instruction where
+// the form above has eight pieces of 32), and the block's codes and scales meet in LDS to be written in the same runs, 16
+// bytes per lane.  For long calls, bound by memory (K of 32 x 64k tokens at 4 bit 175 -> 139 us, 5.1 TB/s), and for blocks of up to
+// four groups, which leave that form's lanes idle; between them the way through LDS costs more than it gives.
+template <int BITS>
+__global__ __launch_bounds__(512) void quant_k_groups_kernel(
+    const half_t *__restrict__ x, int64_t xo, int64_t xt, uint32_t *__restrict__ code, int64_t co,
+    int64_t cr, half_t *__restrict__ scale, half_t *__restrict__ zero, int64_t so, int64_t sr,
+    uint32_t D, uint32_t n_groups, uint32_t blocks_per_slab) {
+  constexpr int PF = 32 / BITS;
+  constexpr int WPG = 32 / PF;  // words per group
+  constexpr int HALF = PF / 2;
+  constexpr int NG = QK_GROUPS_PER_BLOCK, CS = NG * WPG + 1;
+  constexpr float INV_QMAX = 1.0f / (float)((1 << BITS) - 1);
+  __shared__ uint32_t cw[128 * CS];
+  __shared__ half_t sz[2][128][NG + 2];
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t tg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t id = by_xcd(blockIdx.x, gridDim.x), slab = id / blocks_per_slab;
+  const uint32_t G0 = (id - slab * blocks_per_slab) * NG;
+  const uint32_t groups_here = min((uint32_t)NG, n_groups - G0);
+  const int64_t o = slab;
+  const uint32_t row_b = (uint32_t)xt * 2u;  // bytes between token rows
+  const rsrc_t rx = make_rsrc(x + o * xo + (int64_t)G0 * 32 * xt, (groups_here * 32u - 1u) * row_b + D * 2u);
+
+  for (uint32_t c0 = 0; c0 < D; c0 += 128u) {
+    const uint32_t c = c0 + lane * 2u;
+    if (tg < groups_here) {
+      const uint32_t voff = tg * 32u * row_b + min(c, D - 2u) * 2u;   // idle lanes repeat the last channels
+      half2_t t[32];
+#pragma unroll
+      for (int k = 0; k < 32; ++k) t[k] = bits_h2(buf_u32(rx, voff, (uint32_t)k * row_b));
+      half2_t lo2 = t[0], hi2 = t[0];
+#pragma unroll
+      for (int k = 1; k < 32; ++k) {
+        lo2 = __builtin_elementwise_min(lo2, t[k]);
+        hi2 = __builtin_elementwise_max(hi2, t[k]);
+      }
+      const bool zero_extreme = (float)lo2[0] == 0.0f || (float)hi2[0] == 0.0f || (float)lo2[1] == 0.0f || (float)hi2[1] == 0.0f;
+      if (__builtin_amdgcn_ballot_w64(zero_extreme) != 0)   // rare: the wave branches around it as a whole
+#pragma unroll
+        for (int ch = 0; ch < 2; ++ch) {
+          if ((float)lo2[ch] == 0.0f || (float)hi2[ch] == 0.0f) {  // a zero extreme takes the sign of the group's first zero
+            half_t col[32];
+#pragma unroll
+            for (int k = 0; k < 32; ++k) col[k] = t[k][ch];
+            const half_t z = __builtin_bit_cast(half_t, (unsigned short)first_zero_bits(col));
+            if ((float)lo2[ch] == 0.0f) lo2[ch] = z;
+            if ((float)hi2[ch] == 0.0f) hi2[ch] = z;
+          }
+        }
+      half_t sc[2];
+      float rcp[2];
+#pragma unroll
+      for (int ch = 0; ch < 2; ++ch) {
+        const half_t d = (half_t)((float)hi2[ch] - (float)lo2[ch]);
+        sc[ch] = (half_t)((float)d * INV_QMAX);
+        rcp[ch] = group_recip((float)sc[ch]);
+      }
+      float u[2][32];
+#pragma unroll
+      for (int k = 0; k < 32; ++k) {
+        const half2_t cpair = t[k] - lo2;
+        u[0][k] = (float)cpair[0];
+        u[1][k] = (float)cpair[1];
+      }
+#pragma unroll
+      for (int ch = 0; ch < 2; ++ch) {
+        uint32_t *crow = cw + (2 * lane + ch) * CS + tg * WPG;
+#pragma unroll
+        for (int wj = 0; wj < WPG; ++wj) {
+          uint32_t z[HALF];
+#pragma unroll
+          for (int i = 0; i < HALF; ++i)
+            z[i] = code_pair_biased<BITS>(u[ch][wj * PF + i], rcp[ch], u[ch][wj * PF + i + HALF], rcp[ch]);
+          crow[wj] = horner_pack<BITS, HALF>(z);
+        }
+        sz[0][2 * lane + ch][tg] = sc[ch];
+        sz[1][2 * lane + ch][tg] = lo2[ch];
+      }
+    }
+    __syncthreads();
+    // a channel row's words of the block's groups, NQ at a time
+    constexpr int WORDS = NG * WPG, NQ = WORDS < 4 ? WORDS : 4, PER_ROW = WORDS / NQ;
+    const uint32_t here = groups_here * WPG;
+    for (uint32_t i = threadIdx.x; i < 128u * PER_ROW; i += 512u) {
+      const uint32_t ch = i / PER_ROW, w0 = i % PER_ROW * NQ;
+      if (c0 + ch < D && w0 < here) {
+        uint32_t *dst = code + o * co + (int64_t)(c0 + ch) * cr + (int64_t)G0 * WPG + w0;
+        struct __attribute__((packed, aligned(4))) Run { uint32_t v[NQ]; } run;
+#pragma unroll
+        for (int k = 0; k < NQ; ++k) run.v[k] = cw[ch * CS + w0 + k];
+        if (w0 + NQ <= here) *reinterpret_cast<Run *>(dst) = run;
+        else
+          for (int k = 0; k < NQ; ++k)
+            if (w0 + k < here) dst[k] = run.v[k];
+      }
+    }
+    if (threadIdx.x < 256u) {
+      const uint32_t ch = threadIdx.x & 127u, p = threadIdx.x >> 7;
+      if (c0 + ch < D) {
+        half_t *dst = (p ? zero : scale) + o * so + (int64_t)(c0 + ch) * sr + G0;
+        struct __attribute__((packed, aligned(2))) Run { half_t v[NG]; } run;
+#pragma unroll
+        for (int k = 0; k < NG; ++k) run.v[k] = sz[p][ch][k];
+        if (groups_here == NG) *reinterpret_cast<Run *>(dst) = run;
+        else
+          for (uint32_t k = 0; k < groups_here; ++k) dst[k] = sz[p][ch][k];
+      }
+    }
+    __syncthreads();
   }
 }
 
@@ -198,13 +343,14 @@ __global__ __launch_bounds__(256) void normal1_rows_kernel(
 __global__ __launch_bounds__(512) void normal1_k_tokenmajor_kernel(
     const half_t *__restrict__ x, int64_t xo, int64_t xt, uint32_t *__restrict__ code, int64_t co,
     int64_t cr, half_t *__restrict__ stdv, half_t *__restrict__ meanv, int64_t so, int64_t sr,
-    uint32_t D, uint32_t n_groups) {
+    uint32_t D, uint32_t n_groups, uint32_t blocks_per_slab) {
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t cp = lane & 7u, tg = lane >> 3;
-  const uint32_t G0 = blockIdx.x * QK_GROUPS_PER_BLOCK;
+  const uint32_t id = by_xcd(blockIdx.x, gridDim.x), slab = id / blocks_per_slab;
+  const uint32_t G0 = (id - slab * blocks_per_slab) * QK_GROUPS_PER_BLOCK;
   const uint32_t G = G0 + tg;
-  const int64_t o = blockIdx.y;
+  const int64_t o = slab;
   const uint32_t row_b = (uint32_t)xt * 2u;
   const uint32_t groups_here = min((uint32_t)QK_GROUPS_PER_BLOCK, n_groups - G0);
   const rsrc_t rx = make_rsrc(x + o * xo + (int64_t)G0 * 32 * xt, (groups_here * 32u - 1u) * row_b + D * 2u);
@@ -366,18 +512,24 @@ extern "C" int hqekv_quant_pack_rows(const void *x, int64_t xo, int64_t xr, void
   if (((uintptr_t)x & 15) || (xo % 8) || (xr % 8))
     return fail(HQEKV_E_ALIGN, "quant_pack_rows: x rows must be 16-byte aligned");
   const int64_t gpr = L / 32, gps = n_rows * gpr;
-  const int64_t bps = (gps + 63) / 64;
+  // Four groups per quad of lanes where that leaves two workgroups per CU: V of 8 x 16k tokens at 4 bit 11.6 -> 11.2 us, 32 x
+  // 64k 136 -> 126; at 8 x 8k 8.0 either way, below it is behind (8 x 2k 4.6 -> 4.9).
+  const int u = n_groups >= 524288 ? 4 : 1;
+  const int64_t bps = (gps + 64 * u - 1) / (64 * u);
   if (gps > 0x7fffffffLL || bps * n_outer > 0x7fffffffLL)
     return fail(HQEKV_E_ARG, "quant_pack_rows: too many groups");
   int shift = -1;
   if ((gpr & (gpr - 1)) == 0) for (shift = 0; (1LL << shift) < gpr; ++shift) {}
   hipStream_t st = (hipStream_t)stream;
   dim3 grid((unsigned)(bps * n_outer)), block(256);
-#define LAUNCH(B_)                                                                              \
-  hipLaunchKernelGGL(quant_rows_kernel<B_>, grid, block, 0, st, (const half_t *)x, xo, xr,     \
+#define LAUNCH(B_, U_)                                                                          \
+  hipLaunchKernelGGL((quant_rows_kernel<B_, U_>), grid, block, 0, st, (const half_t *)x, xo, xr, \
                      (uint32_t *)code, co, cr, (half_t *)scale, (half_t *)zero, so, sr,         \
                      (uint32_t)gpr, shift, (uint32_t)gps, (uint32_t)bps)
-  if (bits == 1) LAUNCH(1); else if (bits == 2) LAUNCH(2); else if (bits == 4) LAUNCH(4); else LAUNCH(8);
+#define LAUNCH_U(B_) \
+  if (u == 4) LAUNCH(B_, 4); else LAUNCH(B_, 1)
+  if (bits == 1) { LAUNCH_U(1); } else if (bits == 2) { LAUNCH_U(2); } else if (bits == 4) { LAUNCH_U(4); } else { LAUNCH_U(8); }
+#undef LAUNCH_U
 #undef LAUNCH
   return check_launch("quant_rows_kernel");
 }
@@ -400,13 +552,21 @@ extern "C" int hqekv_quant_pack_k_tokenmajor(const void *x, int64_t xo, int64_t 
     return fail(HQEKV_E_ARG, "quant_pack_k_tokenmajor: need D <= xt <= 2^22 (xt=%lld D=%lld)", (long long)xt, (long long)D);
   const int64_t n_groups = T / 32;
   hipStream_t st = (hipStream_t)stream;
-  dim3 grid((unsigned)((n_groups + QK_GROUPS_PER_BLOCK - 1) / QK_GROUPS_PER_BLOCK), (unsigned)n_outer), block(512);
-#define LAUNCH(B_)                                                                                  \
-  hipLaunchKernelGGL(quant_k_tokenmajor_kernel<B_>, grid, block, 0, st, (const half_t *)x, xo, xt, \
-                     (uint32_t *)code, co, cr, (half_t *)scale, (half_t *)zero, so, sr,             \
-                     (uint32_t)D, (uint32_t)n_groups)
-  if (bits == 1) LAUNCH(1); else if (bits == 2) LAUNCH(2); else if (bits == 4) LAUNCH(4); else LAUNCH(8);
+  const int64_t bps = (n_groups + QK_GROUPS_PER_BLOCK - 1) / QK_GROUPS_PER_BLOCK;
+  dim3 grid((unsigned)(bps * n_outer)), block(512);
+  // Which of the two, us here / there: 8 x 32 tokens 6.5 / 4.8, 8 x 128 5.3 / 5.1, 8 x 256 at 2 bit 5.5 / 5.9, 8 x 4k 6.2 / 7.1, 8 x
+  // 8k at 2, 4 and 8 bit 8.0 / 8.5, 8.3 / 8.3, 9.3 / 9.1, 8 x 16k 11.4 / 11.6, 11.9 / 11.6, 13.7 / 12.7, 32 x 64k 158 / 131 and
+  // 175 / 139 at 2 and 4 bit.
+  const bool staged = n_groups <= 4 || bps * n_outer * (bits < 2 ? 2 : bits) >= 2048;
+#define LAUNCH_K(KERNEL_)                                                                                                          \
+  hipLaunchKernelGGL(KERNEL_, grid, block, 0, st, (const half_t *)x, xo, xt, (uint32_t *)code, co, cr, (half_t *)scale, (half_t *)zero, \
+                     so, sr, (uint32_t)D, (uint32_t)n_groups, (uint32_t)bps)
+#define LAUNCH(B_)                                       \
+  if (staged) LAUNCH_K(quant_k_groups_kernel<B_>);       \
+  else LAUNCH_K(quant_k_tokenmajor_kernel<B_>)
+  if (bits == 1) { LAUNCH(1); } else if (bits == 2) { LAUNCH(2); } else if (bits == 4) { LAUNCH(4); } else { LAUNCH(8); }
 #undef LAUNCH
+#undef LAUNCH_K
   return check_launch("quant_k_tokenmajor_kernel");
 }
 
@@ -447,9 +607,10 @@ extern "C" int hqekv_normal1_quant_pack_k_tokenmajor(const void *x, int64_t xo, 
   if (xt < D || xt > (1LL << 22) || D > (1LL << 22) || T / 32 > 0x7fffffffLL)
     return fail(HQEKV_E_ARG, "normal1_quant_pack_k_tokenmajor: need D <= xt <= 2^22 (xt=%lld D=%lld)", (long long)xt, (long long)D);
   const int64_t n_groups = T / 32;
-  dim3 grid((unsigned)((n_groups + QK_GROUPS_PER_BLOCK - 1) / QK_GROUPS_PER_BLOCK), (unsigned)n_outer);
+  const int64_t bps = (n_groups + QK_GROUPS_PER_BLOCK - 1) / QK_GROUPS_PER_BLOCK;
+  dim3 grid((unsigned)(bps * n_outer));
   hipLaunchKernelGGL(normal1_k_tokenmajor_kernel, grid, dim3(512), 0, (hipStream_t)stream, (const half_t *)x, xo, xt,
-                     (uint32_t *)code, co, cr, (half_t *)stdv, (half_t *)meanv, so, sr, (uint32_t)D, (uint32_t)n_groups);
+                     (uint32_t *)code, co, cr, (half_t *)stdv, (half_t *)meanv, so, sr, (uint32_t)D, (uint32_t)n_groups, (uint32_t)bps);
   return check_launch("normal1_k_tokenmajor_kernel");
 }
 
