@@ -74,6 +74,13 @@ __device__ __forceinline__ float wave_sum(float v) { HQ_WAVE_REDUCE(hq_add) }
 __device__ __forceinline__ float wave_max(float v) { HQ_WAVE_REDUCE(fmaxf) }
 #undef HQ_WAVE_REDUCE
 
+// Workgroup i of n runs on XCD i mod 8 (of a range that starts anywhere: some rotation of it): work items dealt so that each
+// XCD, and its L2, takes a contiguous eighth of them.
+__device__ __forceinline__ uint32_t by_xcd(uint32_t i, uint32_t n) {
+  const uint32_t per = n / 8u;
+  return i < 8u * per ? (i & 7u) * per + (i >> 3) : i;
+}
+
 // Buffer addressing: a 128-bit descriptor per (b, head) slab in scalar registers, a per-lane byte offset
 // that never changes, and the row offset in a scalar register -- no vector ALU work per load, and reads
 // past the end of the slab return zero instead of faulting.

@@ -495,13 +495,14 @@ __device__ __forceinline__ void migrate_extras(const MigArgs &a, int wg) {
 // Both sides of a layer in one launch, the K workgroups (the longer ones) first.  Bound by latency -- plan entry, group,
 // store, each a trip to memory -- at 35 MB in and 35 out at 32k tokens: 22 + 12 us as two launches, with the class tables in
 // the argument block and one group in flight per lane; 28 us as one launch of three waves per SIMD, 25 of four, 22.7 with
-// two V blocks in flight (a copy of those bytes takes 14).  4 waves per SIMD are what the 1-bit normal statistics leave.
+// two V blocks in flight, 19.3 with neighbouring K workgroups on one XCD (32 bytes of a channel's scales each: lines met in
+// memory instead of in one L2; a copy of those bytes takes 14).  4 waves per SIMD are what the 1-bit normal statistics leave.
 __global__ __launch_bounds__(MIG_THREADS, 4) void cache_migrate_kernel(MigArgs a) {
   __shared__ MigTables tab;
   int wg = blockIdx.x;
   if (wg < a.side[0].wgs) {
     fetch_tables(a.side[0], tab);
-    migrate_keys(a, wg, tab);
+    migrate_keys(a, (int)by_xcd((uint32_t)wg, (uint32_t)a.side[0].wgs), tab);
     return;
   }
   wg -= a.side[0].wgs;

@@ -75,13 +75,9 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(
 // of 8 groups (64 to 256 bytes of codes) instead of one group at a time.
 constexpr int QK_GROUPS_PER_BLOCK = 8;
 
-// Block i of the launch runs on XCD i mod 8: each XCD takes a contiguous range of (slab, block of groups).  A block writes 16
+// Each XCD takes a contiguous range of (slab, block of groups), by_xcd(): a block writes 16
 // bytes of a channel's scales and 64 (2 bit) of its codes; with its neighbours on other XCDs every line went to memory in
 // pieces.  K of 8 x 8k tokens at 2 bit 8.9 -> 8.0 us, 8 x 16k 13.1 -> 11.4, 32 x 8k 26.4 -> 22.1.
-__device__ __forceinline__ uint32_t by_xcd(uint32_t i, uint32_t n) {
-  const uint32_t per = n / 8u;
-  return i < 8u * per ? (i & 7u) * per + (i >> 3) : i;
-}
 
 template <int BITS>
 __global__ __launch_bounds__(512) void quant_k_tokenmajor_kernel(
