@@ -6,12 +6,14 @@
 // tokens of one class of one (b, kv head).  V classes and token-major fp16 rows are 16 lanes (8 channels each) per token
 // as they lie.  K classes are channel-major, the result is token-major: a wave takes one 32-token group, a lane two
 // channels of it (its codes are one short run of each row; the four waves read neighbouring runs of the same lines), and
-// the tile is turned in LDS -- 68 words per token row, so the channel-pair writes walk all banks and the 16-byte reads
-// stay aligned.  34 KB of LDS: four workgroups per CU.
-// Measured at B=1, 16k tokens of the fp16 / 8 / 4 / 2-bit mix (73 MB): 258 us as dequantise launches, transposing copies
-// and index_put scatters; this launch 21 us (3.4 TB/s), 20 us a call among others.  Positions that are looked at for the
-// first time cost two position checks and a wait for each on top (see cover_once_kernel).
+// turns it in a corner of LDS of its own, sixteen tokens at a time -- 68 words per token row, so the channel-pair writes
+// walk all banks and the 16-byte reads stay aligned.  17 KB of LDS and 67 registers: seven workgroups per CU, no barrier.
+// Measured at B=1 of the fp16 / 8 / 4 / 2-bit mix, us a launch: 16k tokens (73 MB) 258 as dequantise launches, transposing copies
+// and index_put scatters, 28.9 with the whole 128-token tile in LDS (four workgroups per CU, and 80 bytes of scratch memory
+// per lane for what is a uint4 in an array), now 26.6; 512 tokens 7.0 -> 6.1, 64k 103 -> 88, 2 x 64k 197 -> 158.  Positions
+// that are looked at for the first time cost two position checks and a wait for each on top (see cover_once_kernel).
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 #include "quant_math.h"
@@ -32,6 +34,7 @@ struct RcSeg {
   int16_t bits;
   int16_t kind;         // 0: channel-major K, 1: token-major; + 2: 1-bit normal-quantile coding
 };
+typedef uint32_t rc_words_t __attribute__((ext_vector_type(4)));   // (uint4 in an array went through scratch memory)
 constexpr int RC_SEGS = 2 * HQEKV_MAX_SEGS;
 struct RcTable {
   RcSeg seg[RC_SEGS];
@@ -42,7 +45,14 @@ constexpr int RC_THREADS = 256;
 constexpr int RC_TOK = 128;    // tokens per workgroup
 constexpr int RC_CH = 128;     // channels turned in LDS at a time
 constexpr int RC_ROW = 68;     // 32-bit words per token row in LDS
+constexpr int RC_HALF = 16;    // tokens a wave turns at a time
 constexpr int64_t RC_GRID_Y = 65535;
+
+// keep LDS traffic of one wave in program order (the hardware does; this holds the compiler to it)
+__device__ __forceinline__ void rc_wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
 
 // where token t of the segment goes; -1: outside the dense tensor (an index counts from the end when negative, as in
 // torch; one that names no row is dropped)
@@ -69,7 +79,7 @@ __device__ __forceinline__ half2_t rc_value(uint32_t c0, uint32_t c1, half2_t s2
 
 // 8 adjacent channels of one token: BITS bytes of codes in the low bits of w0 (and w1)
 template <int BITS, bool NORMAL>
-__device__ __forceinline__ uint4 rc_piece(uint32_t w0, uint32_t w1, half_t s, half_t z) {
+__device__ __forceinline__ rc_words_t rc_piece(uint32_t w0, uint32_t w1, half_t s, half_t z) {
   const half2_t s2 = {s, s}, z2 = {z, z};
   uint32_t r[4];
 #pragma unroll
@@ -78,15 +88,17 @@ __device__ __forceinline__ uint4 rc_piece(uint32_t w0, uint32_t w1, half_t s, ha
     const int k = BITS == 8 ? 2 * (j & 1) : 2 * j;
     r[j] = h2_bits(rc_value<NORMAL>(code_at<BITS>(w, k), code_at<BITS>(w, k + 1), s2, z2));
   }
-  return make_uint4(r[0], r[1], r[2], r[3]);
+  return (rc_words_t){r[0], r[1], r[2], r[3]};
 }
 
-template <int BITS, bool NORMAL>
-__device__ __forceinline__ void rc_token_major(const RcSeg &s, int64_t bh, int t0, int D, int64_t T) {
+// `dim`: head_dim where it is known (128: the pieces of a row are counted by shifts)
+template <int BITS, bool NORMAL, typename Dim>
+__device__ __forceinline__ void rc_token_major_of(const RcSeg &s, int64_t bh, int t0, Dim dim, int64_t T) {
+  const int D = dim;
   const int P = D >> 3, items = RC_TOK * P;   // pieces of 8 channels
   constexpr int U = 4;
   for (int i0 = threadIdx.x; i0 < items; i0 += U * RC_THREADS) {
-    uint4 v[U];
+    rc_words_t v[U];
     half_t sc[U], zr[U];
     int64_t pos[U];
 #pragma unroll
@@ -98,7 +110,7 @@ __device__ __forceinline__ void rc_token_major(const RcSeg &s, int64_t bh, int t
       const char *src = (const char *)s.data + (row * D + cp * 8) * BITS / 8;
       pos[u] = in ? rc_position(s, t, T) : -1;
       if (BITS == 16) {
-        v[u] = *reinterpret_cast<const uint4 *>(src);
+        v[u] = *reinterpret_cast<const rc_words_t *>(src);
       } else {
         if (BITS == 8) {
           v[u].x = reinterpret_cast<const uint32_t *>(src)[0];
@@ -119,67 +131,104 @@ __device__ __forceinline__ void rc_token_major(const RcSeg &s, int64_t bh, int t
     for (int u = 0; u < U; ++u) {
       const int cp = (i0 + u * RC_THREADS) % P;
       if constexpr (BITS != 16) v[u] = rc_piece<BITS, NORMAL>(v[u].x, v[u].y, sc[u], zr[u]);
-      if (pos[u] >= 0) *reinterpret_cast<uint4 *>(s.out + (bh * T + pos[u]) * D + cp * 8) = v[u];
+      if (pos[u] >= 0) *reinterpret_cast<rc_words_t *>(s.out + (bh * T + pos[u]) * D + cp * 8) = v[u];
     }
   }
 }
+template <int BITS, bool NORMAL>
+__device__ __forceinline__ void rc_token_major(const RcSeg &s, int64_t bh, int t0, int D, int64_t T) {
+  if (D == 128) rc_token_major_of<BITS, NORMAL>(s, bh, t0, std::integral_constant<int, 128>{}, T);
+  else rc_token_major_of<BITS, NORMAL>(s, bh, t0, D, T);
+}
 
 template <int BITS, bool NORMAL>
-__device__ __forceinline__ void rc_channel_major(const RcSeg &s, int64_t bh, int t0, int D, int64_t T, uint32_t *tile) {
-  const int dp = threadIdx.x & 63, g = threadIdx.x >> 6;   // channel pair, 32-token group of the tile
+__device__ __forceinline__ void rc_channel_major(const RcSeg &s, int64_t bh, int t0, int D, int64_t T, uint32_t *tiles) {
+  const int dp = threadIdx.x & 63, g = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // channel pair, 32-token group
   const int n = s.n_tokens, tg = t0 + 32 * g;              // the group's first token
+  if (tg >= n) return;                                      // (whole waves; nothing below is shared between them)
+  uint32_t *tile = tiles + g * (RC_HALF * RC_ROW);
+  // where the lane's 16-byte pieces go: a piece of token dp / P + ... of each half.  Asked for ahead of the codes.
+  const int P = min(RC_CH, D) >> 3;                         // pieces of a token row
+  int64_t pos[2][RC_HALF / 4];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int j = 0; j < RC_HALF / 4; ++j) {
+      const int k = RC_HALF * h + 4 * j + (dp >> 4);        // (for rows of 128 channels; others ask again below)
+      pos[h][j] = tg + k < n ? rc_position(s, tg + k, T) : -1;
+    }
   for (int c0 = 0; c0 < D; c0 += RC_CH) {
-    const int d = c0 + 2 * dp;
-    if (d < D && tg < n) {
-      uint32_t *col = tile + (32 * g) * RC_ROW + dp;
+    const int d = min(c0 + 2 * dp, D - 2);                  // (past the last channel: that one again, not stored)
+    uint32_t a[BITS], b[BITS];   // the group's words of both channels
+    half2_t s2 = {}, z2 = {};
+    {
       if constexpr (BITS == 16) {
         const half_t *ra = (const half_t *)s.data + (bh * D + d) * (int64_t)n + tg, *rb = ra + n;
         if ((n & 7) == 0) {
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
-            if (tg + 8 * q < n) {
-              const uint4 a = reinterpret_cast<const uint4 *>(ra)[q], b = reinterpret_cast<const uint4 *>(rb)[q];
-              const uint32_t av[4] = {a.x, a.y, a.z, a.w}, bv[4] = {b.x, b.y, b.z, b.w};
-#pragma unroll
-              for (int j = 0; j < 4; ++j) {
-                col[(8 * q + 2 * j) * RC_ROW] = __builtin_amdgcn_perm(bv[j], av[j], 0x05040100u);
-                col[(8 * q + 2 * j + 1) * RC_ROW] = __builtin_amdgcn_perm(bv[j], av[j], 0x07060302u);
-              }
-            }
+            const int at = tg + 8 * q < n ? q : 0;          // (past the class's end: the first eight again, not stored)
+            const uint4 x = reinterpret_cast<const uint4 *>(ra)[at], y = reinterpret_cast<const uint4 *>(rb)[at];
+            a[4 * q] = x.x; a[4 * q + 1] = x.y; a[4 * q + 2] = x.z; a[4 * q + 3] = x.w;
+            b[4 * q] = y.x; b[4 * q + 1] = y.y; b[4 * q + 2] = y.z; b[4 * q + 3] = y.w;
           }
         } else {
-          for (int i = 0; i < 32 && tg + i < n; ++i) col[i * RC_ROW] = h2_bits((half2_t){ra[i], rb[i]});
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            const int k0 = min(2 * i, n - 1 - tg), k1 = min(2 * i + 1, n - 1 - tg);
+            a[i] = h2_bits((half2_t){ra[k0], ra[k1]});
+            b[i] = h2_bits((half2_t){rb[k0], rb[k1]});
+          }
         }
       } else {   // (the class holds whole groups of 32 tokens)
-        constexpr int PF = 32 / BITS;
         const int64_t ga = (bh * D + d) * (int64_t)(n >> 5) + (tg >> 5), gb = ga + (n >> 5);
         const uint32_t *wa = (const uint32_t *)s.data + ga * BITS, *wb = (const uint32_t *)s.data + gb * BITS;
-        uint32_t a[BITS], b[BITS];
 #pragma unroll
         for (int i = 0; i < BITS; ++i) {
           a[i] = wa[i];
           b[i] = wb[i];
         }
-        const half2_t s2 = {s.scale[ga], s.scale[gb]}, z2 = {s.zero[ga], s.zero[gb]};
-#pragma unroll
-        for (int i = 0; i < 32; ++i)
-          col[i * RC_ROW] = h2_bits(rc_value<NORMAL>(code_at<BITS>(a[i / PF], i % PF), code_at<BITS>(b[i / PF], i % PF), s2, z2));
+        s2 = (half2_t){s.scale[ga], s.scale[gb]};
+        z2 = (half2_t){s.zero[ga], s.zero[gb]};
       }
     }
-    __syncthreads();
-    const int P = min(RC_CH, D - c0) >> 3;
-    for (int i = threadIdx.x; i < RC_TOK * P; i += RC_THREADS) {
-      const int tl = i / P, cp = i % P, t = t0 + tl;
-      if (t >= n) break;
-      const int64_t p = rc_position(s, t, T);
-      if (p >= 0) *reinterpret_cast<uint4 *>(s.out + (bh * T + p) * D + c0 + cp * 8) = *reinterpret_cast<const uint4 *>(tile + tl * RC_ROW + cp * 4);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      {
+        uint32_t *col = tile + dp;
+#pragma unroll
+        for (int i = 0; i < RC_HALF; ++i) {
+          const int k = RC_HALF * h + i;
+          if constexpr (BITS == 16) {
+            col[i * RC_ROW] = __builtin_amdgcn_perm(b[k / 2], a[k / 2], k & 1 ? 0x07060302u : 0x05040100u);
+          } else {
+            constexpr int PF = 32 / BITS;
+            col[i * RC_ROW] = h2_bits(rc_value<NORMAL>(code_at<BITS>(a[k / PF], k % PF), code_at<BITS>(b[k / PF], k % PF), s2, z2));
+          }
+        }
+      }
+      rc_wave_fence();
+      if (P == 16 && c0 + RC_CH <= D) {
+#pragma unroll
+        for (int j = 0; j < RC_HALF / 4; ++j)
+          if (pos[h][j] >= 0)
+            *reinterpret_cast<uint4 *>(s.out + (bh * T + pos[h][j]) * D + c0 + (dp & 15) * 8) =
+                *reinterpret_cast<const uint4 *>(tile + (4 * j + (dp >> 4)) * RC_ROW + (dp & 15) * 4);
+      } else {   // other head sizes, and the last channels of one that is no multiple of 128
+        const int pieces = min(RC_CH, D - c0) >> 3;
+        for (int i = dp; i < RC_HALF * pieces; i += 64) {
+          const int k = i / pieces, cp = i % pieces, t = tg + RC_HALF * h + k;
+          const int64_t p = t < n ? rc_position(s, t, T) : -1;
+          if (p >= 0) *reinterpret_cast<uint4 *>(s.out + (bh * T + p) * D + c0 + cp * 8) = *reinterpret_cast<const uint4 *>(tile + k * RC_ROW + cp * 4);
+        }
+      }
+      rc_wave_fence();
     }
-    if (c0 + RC_CH < D) __syncthreads();
   }
 }
 
-__global__ __launch_bounds__(RC_THREADS, 4) void cache_reconstruct_kernel(RcTable tb, int D, int64_t T) {
-  __shared__ __align__(16) uint32_t tile[RC_TOK * RC_ROW];
+__global__ __launch_bounds__(RC_THREADS, 7) void cache_reconstruct_kernel(RcTable tb, int D, int64_t T) {
+  __shared__ __align__(16) uint32_t tile[RC_THREADS / 64 * RC_HALF * RC_ROW];
   int si = -1, first = 0;
 #pragma unroll
   for (int k = 0; k < RC_SEGS; ++k) {
