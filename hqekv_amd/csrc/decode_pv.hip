@@ -464,7 +464,7 @@ __device__ __forceinline__ void pv_tiles_body(const SegTable &tb, const half_t *
 }
 
 template <int HP, bool EXACT, bool LOOP, bool FUSED>
-__global__ __launch_bounds__(PT_WAVES * 64, HP <= 8 ? (LOOP ? 4 : 6) : 2) void pv_tiles_kernel(SegTable tb, half_t *__restrict__ p, float *__restrict__ partial,
+__global__ __launch_bounds__(PT_WAVES * 64, HP <= 8 ? (LOOP ? (HP == 8 ? 3 : 4) : 6) : 2) void pv_tiles_kernel(SegTable tb, half_t *__restrict__ p, float *__restrict__ partial,
                                                                    TilesArgs ta, int64_t Tall, int64_t n_bhq, FuseArgs fz) {
   pv_tiles_body<HP, EXACT, LOOP, FUSED, false>(tb, p, p, partial, ta, Tall, n_bhq, fz);
 }

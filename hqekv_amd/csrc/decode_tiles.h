@@ -101,12 +101,18 @@ __device__ __forceinline__ bool qt_runs(const SegDev &sg) { return (sg.layout & 
 
 // =============================================================================== host side
 // p.V workgroups the chip holds at once, of the single-block form, and the workgroups a looping launch is made of: one
-// resident round.  Up to eight heads per KV head: six and four per CU (80 and 128 registers).  Above: three and two (45 and
-// 58 KB of LDS) -- two rounds of those for launches of more than 4096 blocks, whose last round weighs less than the runs of
-// a workgroup that meets the end of its class.  p.V at 16 heads, 512 / 1024 workgroups: 1800 blocks (B=1, 64k tokens) 27.4 /
-// 33.2 us, 3700 (4 x 32k) 42.0 / 46.9, 5500 (8 x 24k) 64.8 / 65.1, 7400 (8 x 32k) 84.3 / 81.8, 14700 (8 x 64k) 155.8 / 152.2.
+// resident round.  Single block: six per CU up to eight heads per KV head (80 registers), three above (45 KB of LDS).
+// Looping: four per CU up to four heads (128 registers), three up to eight -- the 33 KB of LDS would let four in, but at
+// their 128 registers 43 are spilled, inside the loop; at three per CU it takes 150 and spills none.  A step of the fp16 / 8 /
+// 4 / 2-bit mix, four / three per CU, us: 5 heads x 8 KV heads at 48k tokens 32.0 / 30.9, at 64k 38.2 / 35.8, at 8 x 32k 107.8 /
+// 100.1; 8 heads, 8 x 32k 116.3 / 109.5; 7 heads x 4, 4 x 64k 59.8 / 55.7; two per CU 31.1, 37.4, 112.6, 120.8, 58.3.  (Up to
+// four heads three per CU is a tie, and single blocks for fewer than six per CU lose up to 2 %.)  Above eight heads two
+// per CU (58 KB of LDS) -- two rounds of those for launches of more than 4096 blocks, whose last round weighs less than the
+// runs of a workgroup that meets the end of its class.  p.V at 16 heads, 512 / 1024 workgroups: 1800 blocks (B=1, 64k tokens)
+// 27.4 / 33.2 us, 3700 (4 x 32k) 42.0 / 46.9, 5500 (8 x 24k) 64.8 / 65.1, 7400 (8 x 32k) 84.3 / 81.8, 14700 (8 x 64k) 155.8 /
+// 152.2.
 constexpr int64_t pt_resident(int64_t nrep) { return (nrep <= 8 ? 6 : 3) * 256; }
-constexpr int64_t pt_loop_units(int64_t nrep, int64_t blocks) { return (nrep <= 8 || blocks > 4096 ? 4 : 2) * 256; }
+constexpr int64_t pt_loop_units(int64_t nrep, int64_t blocks) { return (nrep <= 4 ? 4 : nrep <= 8 ? 3 : blocks > 4096 ? 4 : 2) * 256; }
 
 // How a launch is cut up.
 struct TilesPlan {
