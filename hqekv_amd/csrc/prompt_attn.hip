@@ -33,8 +33,9 @@ constexpr int PA_BC = 32;              // keys per score tile
 // tile's products run beside the first one's exponentials).
 // <2, 1>: the two waves of 32 query rows deal the key tiles among themselves and merge their maxima, sums and outputs at the
 // end: walks of half the length in twice as many workgroups.  A step stages two tiles, so LDS holds two workgroups per CU.
-template <int KS_, int NB_>
+template <int KS_, int NB_, bool REVERSED_>
 struct PaShape {
+  static constexpr bool REVERSED = REVERSED_;   // the second 256 workgroups come in the opposite order
   static constexpr int KS = KS_, NB = NB_, WGS = KS_ * NB_ == 1 ? 3 : 2;
   static constexpr int ROWS = 128 / KS;            // query rows per workgroup
   static constexpr int STEP = PA_BC * NB * KS;     // keys staged per step
@@ -119,7 +120,7 @@ __global__ __launch_bounds__(PA_THREADS, S::WGS) void prompt_attn_kernel(PromptA
   // Two workgroups per CU: the second 256 come in the opposite order (eight by eight, so that a KV head stays on its XCD), and a
   // CU that began with a long walk is given a short one: T = 2048 54.4 -> 53.2 us, 3500 130 -> 124, 4099 171.6 -> 165.9.
   int item = (int)blockIdx.x;
-  if (S::WGS == 2 && item >> 8 == 1) {
+  if (S::REVERSED && item >> 8 == 1) {
     const int m = min((int)gridDim.x - 256, 256), g = a.by_xcd ? 8 : 1, p = item - 256;
     item = 256 + m - g - p / g * g + p % g;
   }
@@ -556,12 +557,15 @@ extern "C" int hqekv_prompt_attn(const void *q, const int64_t *q_strides, const 
   const int form = prompt_form(T, B * Hq);
   const int64_t rows = form == 2 ? 64 : 128, wgs = (T + rows - 1) / rows * B * Hq;
   if (wgs > 0x7fffffffLL) return fail(HQEKV_E_UNSUPPORTED, "prompt_attn: T * B * Hq too large");
-#define LAUNCH(C_, KS_, NB_)                                                                                                                     \
-  hipLaunchKernelGGL((prompt_attn_kernel<C_, PaShape<KS_, NB_>>), dim3((unsigned)wgs), dim3(PA_THREADS), 0, (hipStream_t)stream, a)
+  // Walks of half the length gain from the opposite order only when a third round follows: 728 workgroups (T = 777, B = 2, 28
+  // heads) 26.4 -> 25.5 us, 768 (1500) 36.7 -> 36.3; 320 (478, 40 heads) 13.6 / 14.0, 608 (1200) 27.3 / 27.6.
+#define LAUNCH(C_, KS_, NB_, REV_)                                                                                                                \
+  hipLaunchKernelGGL((prompt_attn_kernel<C_, PaShape<KS_, NB_, REV_>>), dim3((unsigned)wgs), dim3(PA_THREADS), 0, (hipStream_t)stream, a)
 #define LAUNCH_K(C_)                    \
-  if (form == 2) LAUNCH(C_, 2, 1);      \
-  else if (form == 1) LAUNCH(C_, 1, 2); \
-  else LAUNCH(C_, 1, 1)
+  if (form == 2 && wgs > 640) LAUNCH(C_, 2, 1, true); \
+  else if (form == 2) LAUNCH(C_, 2, 1, false);        \
+  else if (form == 1) LAUNCH(C_, 1, 2, true);         \
+  else LAUNCH(C_, 1, 1, false)
   if (causal) { LAUNCH_K(true); } else { LAUNCH_K(false); }
 #undef LAUNCH_K
 #undef LAUNCH

@@ -11,6 +11,7 @@ pytestmark = pytest.mark.gpu
     (1, 100, 100, 450), (1, 101, 101, 450),              # 400 and 404 workgroups of 128 rows
     (2, 64, 8, 385), (4, 32, 8, 511),                    # 512: by eights
     (1, 70, 10, 1024), (1, 96, 24, 700),                 # 560, 576
+    (1, 64, 8, 640), (1, 64, 8, 641),                    # 640 and 704 of 64 rows
     (3, 125, 25, 512), (4, 94, 47, 449)])                # 1500 and 1504
 def test_on_both_sides_of_the_lines(dev, B, Hq, Hkv, T, causal):
     """Tolerance: probabilities are rounded to fp16 (2^-11) before the second product and the output once more."""
