@@ -313,7 +313,8 @@ class SegmentMemo:
         self.Hkv = None
         self.dims = (None, None)
         self.partition = False                 # the classes' position arrays cover [0, kept) once per side
-        self._native = None                    # the class entries as the native step takes them
+        self._native = None                    # the class entries as the native step takes them (k_arr is None where
+                                               # they were built there: ``build`` makes the rest when it is asked for)
 
     def lookup(self, pkv: tuple, dev, low_uniform: bool) -> bool:
         held = self.held
@@ -382,11 +383,17 @@ class SegmentMemo:
             self.ws = torch.empty(max(need + need // 8, 256) // 4, dtype=torch.float32, device=dev)
         return self.ws
 
-    def steps(self, pkv: tuple, dev, low_uniform: bool, known: bool):
+    def steps(self, pkv: tuple, q: torch.Tensor, low_uniform: bool, known: bool):
         """The native tables (``_host.StepTables``) of a cache whose classes cover every position once, else None.
         ``known``: the caller vouches that ``pkv`` carries the class tensors the tables were built from (it is the tuple
         the previous step returned)."""
+        dev = q.device
         if not (known and self.held is not None) and not self.lookup(pkv, dev, low_uniform):
+            native = _lib.host().step_tables(q, pkv, low_uniform, idx_cover_once)
+            if native is not None:
+                self.held, self.key, self._native, self.partition = tuple(pkv[:NEW_K]), (dev, low_uniform), native, True
+                self.keep, self.need, self.k_arr, self.v_arr = [], {}, None, None
+                return native
             self.build(pkv, dev, low_uniform)
         if not self.partition:
             return None
@@ -422,7 +429,7 @@ def decode_attention(q: torch.Tensor, pkv: tuple, mask, Tall: int, zero_init: bo
     keep: list = []
     use_flags = default_flags() if flags is None else flags
     if memo is not None:
-        if not memo.lookup(pkv, dev, low_uniform):
+        if not memo.lookup(pkv, dev, low_uniform) or memo.k_arr is None:
             memo.build(pkv, dev, low_uniform)
         k_segs, n_k, v_segs, n_v, Hkv, (dk, dv), res_tail = memo.tables(pkv, Tall, keep, tail)
         covered = memo.partition

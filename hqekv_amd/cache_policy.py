@@ -631,8 +631,10 @@ def compress(past_key_value: tuple, compress_length: int, history_length, K_sort
              K_bit_num: torch.Tensor, V_bit_num: torch.Tensor, token_importance: torch.Tensor,
              quant_strategy: str, *, last_weights=None, block_size: int = 32, group_size: int = 32,
              times_range: bool = True, n_targets: int = 6, V_token_range: Optional[torch.Tensor] = None,
-             engine: Optional[str] = None, residual_buffers: Optional[tuple] = None) -> tuple:
-    """``residual_buffers``: a (K, V) pair of (B, H, capacity, D) tensors the residual may be put into; its fields in the
+             engine: Optional[str] = None, residual_buffers: Optional[tuple] = None, meanwhile=None) -> tuple:
+    """``meanwhile``: a callable that queues work which neither needs the compression nor is needed by it; called exactly
+    once, as soon as the rankings the host will wait for are queued, so that the device is busy while the host plans.
+    ``residual_buffers``: a (K, V) pair of (B, H, capacity, D) tensors the residual may be put into; its fields in the
     result are then their heads.
     ``engine``: None / "auto" = the one-launch-per-side gather when the selection is made of whole aligned blocks,
     else the step-by-step engine; "steps" forces the latter, "gather" raises when it does not apply (tests)."""
@@ -640,6 +642,12 @@ def compress(past_key_value: tuple, compress_length: int, history_length, K_sort
         raise ValueError('invalid quant_strategy')
     if block_size != BLOCK or group_size != BLOCK:
         raise ValueError("block_size and group_size must be 32")
+    called = []
+
+    def once():
+        if meanwhile is not None and not called:
+            called.append(True)
+            meanwhile()
     pkv = past_key_value
     new_K, new_V = pkv[39], pkv[40]
     if new_K is None or new_V is None:
@@ -659,11 +667,12 @@ def compress(past_key_value: tuple, compress_length: int, history_length, K_sort
         ring = last_weights.weights if type(last_weights) is last_attn_weights else None
         done = _lib.host().compress(pkv, history, compress_length, K_sorted_idx.scores, token_importance, bool(times_range),
                                     V_token_range, K_bit_num, V_bit_num, quant_strategy == LOW_NORMAL,
-                                    ring, residual_buffers, _new_array, weakref.ref)
+                                    ring, residual_buffers, _new_array, weakref.ref, None if meanwhile is None else once)
         if done is not None:
             if done[1] is not None and last_weights is not None:
                 last_weights.eviction(done[1])
             return done[0]
+    once()
     whole = new_K.shape[2] == compress_length and new_V.shape[2] == compress_length   # nothing stays behind
     res_K = None if whole else _none_if_empty(new_K[:, :, compress_length:, :].clone())
     res_V = None if whole else _none_if_empty(new_V[:, :, compress_length:, :].clone())

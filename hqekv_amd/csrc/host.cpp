@@ -324,6 +324,42 @@ PyObject *tables_new(PyTypeObject *type, PyObject *args, PyObject *) {
   new (&t->ws) Tensor();
   return (PyObject *)t;
 }
+// step_tables(q, pkv, low_uniform, cover_fn) -> StepTables over the tuple's classes -- they have to cover every position
+// once --, or None where the tuple is not plain.  The caller keeps the class tensors.  (Built from Python's segment lists
+// they cost the first step after a compression 45 us: a prompt of 1024 tokens and 24 steps 515 -> 437 us.)
+PyTypeObject *tables_type_ptr();
+PyObject *step_tables(PyObject *, PyObject *const *a, Py_ssize_t na) {
+  HANDLE_TH_ERRORS
+  if (na != 4) return PyErr_Format(PyExc_TypeError, "step_tables takes 4 arguments");
+  PyObject *pkv = a[1];
+  if (!is_tensor(a[0]) || !PyTuple_Check(pkv) || PyTuple_GET_SIZE(pkv) != TUPLE_LEN) Py_RETURN_NONE;
+  const Tensor &q = ten(a[0]);
+  if (!q.is_cuda() || q.dim() != 4) Py_RETURN_NONE;
+  const at::Device dev = q.device();
+  const int64_t B = q.size(0);
+  const bool low_uniform = a[2] == Py_True;
+  Side k, v;
+  if (!read_side(pkv, true, low_uniform, B, dev, k) || !read_side(pkv, false, low_uniform, B, dev, v)) Py_RETURN_NONE;
+  if (!v.class_tokens || k.class_tokens != v.class_tokens || k.H != v.H || k.D != v.D || k.n_idx > HQEKV_MAX_SEGS - 2 || v.n_idx > HQEKV_MAX_SEGS - 2)
+    Py_RETURN_NONE;
+  for (Side *s : {&k, &v}) {
+    const int c = cover_once(s->idx, s->n_idx, v.class_tokens, a[3]);
+    if (c < 0) return nullptr;
+    if (!c) Py_RETURN_NONE;
+    for (int i = 0; c == 3 && i < s->n_idx; ++i) s->seg[i].layout |= HQEKV_LAYOUT_RUNS;
+  }
+  StepTables *t = (StepTables *)tables_type_ptr()->tp_alloc(tables_type_ptr(), 0);
+  if (!t) return nullptr;
+  memset(t->k, 0, sizeof(t->k));
+  memset(t->v, 0, sizeof(t->v));
+  memcpy(t->k, k.seg, k.n_idx * sizeof(hqekv_seg));   // (the classes come first, one position array each)
+  memcpy(t->v, v.seg, v.n_idx * sizeof(hqekv_seg));
+  t->n_k = k.n_idx;
+  t->n_v = v.n_idx;
+  new (&t->ws) Tensor();
+  return (PyObject *)t;
+  END_HANDLE_TH_ERRORS
+}
 void tables_free(PyObject *o) {
   ((StepTables *)o)->ws.~Tensor();
   Py_TYPE(o)->tp_free(o);
@@ -441,6 +477,7 @@ PyMethodDef tables_methods[] = {
     {nullptr, nullptr, 0, nullptr},
 };
 PyTypeObject tables_type = {PyVarObject_HEAD_INIT(nullptr, 0)};
+PyTypeObject *tables_type_ptr() { return &tables_type; }
 
 // What KiviAttentionLayer keeps between two decode steps: the K class, the fp16 K tail in a buffer of residual_length
 // rows, the V tail as a window [v0, v0 + nv) of a longer buffer, the V class in capacity buffers, and the tuple (views of
@@ -990,14 +1027,22 @@ bool new_tokens(const Tensor &t, bool is_k, int64_t B, int64_t H, int64_t n, int
 
 // Both block rankings, written by one launch into page-locked memory.  Every entry is stored exactly once, so the ranking
 // is there as soon as no entry holds its initial value: that is watched for a while (a stream synchronisation wakes up
-// some ten microseconds later), then the stream is waited for.
-bool host_orders(const void *const (&scores)[2], int64_t n, const Tensor &order, const at::Device &dev) {
+// some ten microseconds later), then the stream is waited for.  meanwhile: None, or what the caller has to queue that does
+// not need the ranking -- the kernels run it while the host reads the ranking and plans; called once, behind the launch.  (The
+// memory may not be let go before the kernel has written it: what the call raises is raised after the wait.)
+bool host_orders(const void *const (&scores)[2], int64_t n, const Tensor &order, const at::Device &dev, PyObject *meanwhile) {
   volatile int32_t *p = (volatile int32_t *)order.data_ptr();
   for (int64_t i = 0; i < 2 * n; ++i) p[i] = -1;
   hipError_t err = hipSuccess;
-  const int rc = without_gil([&]() -> int {
-    const int rc = api.hqekv_rank_blocks(scores, 2, n, (int32_t *)order.data_ptr(), stream_of(dev));
-    if (rc) return rc;
+  const int rc = without_gil([&] { return api.hqekv_rank_blocks(scores, 2, n, (int32_t *)order.data_ptr(), stream_of(dev)); });
+  if (rc) {
+    raise_rc(rc, "rank_blocks");
+    return false;
+  }
+  PyObject *did = meanwhile == Py_None ? nullptr : PyObject_CallNoArgs(meanwhile);
+  const bool raised = meanwhile != Py_None && !did;
+  Py_XDECREF(did);
+  without_gil([&]() -> int {
     const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(2);
     int64_t i = 0;
     while (i < 2 * n) {
@@ -1010,10 +1055,7 @@ bool host_orders(const void *const (&scores)[2], int64_t n, const Tensor &order,
     }
     return HQEKV_OK;
   });
-  if (rc) {
-    raise_rc(rc, "rank_blocks");
-    return false;
-  }
+  if (raised) return false;
   if (err != hipSuccess) PyErr_Format(PyExc_RuntimeError, "rank_blocks: HIP error %d", (int)err);
   return err == hipSuccess;
 }
@@ -1032,14 +1074,15 @@ bool six_counts(PyObject *o, int64_t (&out)[6], int &n) {
 }
 
 // compress(pkv, history, length, k_scores, importance, times_range, V_range or None, K_counts, V_counts, low_normal,
-// ring or None, (K buffer, V buffer) or None, new_array, weak_ref): cache_policy.compress for a cache, rankings and counts
-// made of whole blocks.  ring: the importance ring, whose evicted columns are taken out; buffers (B, H, capacity, D): where
-// the residual goes, its fields are their heads then.  new_array(n): an int64 numpy array; weak_ref: weakref.ref.
+// ring or None, (K buffer, V buffer) or None, new_array, weak_ref[, meanwhile or None]): cache_policy.compress for a cache,
+// rankings and counts made of whole blocks.  ring: the importance ring, whose evicted columns are taken out; buffers (B, H,
+// capacity, D): where the residual goes, its fields are their heads then.  new_array(n): an int64 numpy array; weak_ref:
+// weakref.ref; meanwhile(): see host_orders -- not called where None is returned before the ranking is launched.
 // -> (the new tuple, positions kept where tokens were evicted and no ring was given, else None), or None where that does not
 // hold -- found out before anything is launched except the score and rank kernels.
 PyObject *compress(PyObject *, PyObject *const *a, Py_ssize_t na) {
   HANDLE_TH_ERRORS
-  if (na != 14) return PyErr_Format(PyExc_TypeError, "compress takes 14 arguments");
+  if (na != 14 && na != 15) return PyErr_Format(PyExc_TypeError, "compress takes 14 or 15 arguments");
   PyObject *pkv = a[0];
   const int64_t history = PyLong_AsLongLong(a[1]), length = PyLong_AsLongLong(a[2]);
   if (PyErr_Occurred()) return nullptr;
@@ -1117,7 +1160,7 @@ PyObject *compress(PyObject *, PyObject *const *a, Py_ssize_t na) {
   const Tensor host = at::empty({2 * nb + 5 * nb + 4}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
   const void *const sc[2] = {scores_k.data_ptr(), scores_v.data_ptr()};
   const Tensor up_d = new_tensor({5 * nb}, at::kInt, dev);   // (made while the ranking runs)
-  if (!host_orders(sc, nb, host, dev)) return nullptr;
+  if (!host_orders(sc, nb, host, dev, na > 14 ? a[14] : Py_None)) return nullptr;
   // ---- the plans of both sides and the V side's surviving blocks, one transfer for all
   const int32_t *order = (const int32_t *)host.data_ptr();
   int32_t *words = (int32_t *)host.data_ptr() + up(2 * nb, 4), counts[2][5] = {}, n_alive[2] = {0, 0};
@@ -1236,6 +1279,7 @@ PyObject *bind(PyObject *, PyObject *path) {
 PyMethodDef module_methods[] = {
     {"bind", bind, METH_O, nullptr},
     {"decode", (PyCFunction)(void (*)(void))decode, METH_FASTCALL, nullptr},
+    {"step_tables", (PyCFunction)(void (*)(void))step_tables, METH_FASTCALL, nullptr},
     {"prompt_attention", (PyCFunction)(void (*)(void))prompt_attention, METH_FASTCALL, nullptr},
     {"prompt_last_rows", (PyCFunction)(void (*)(void))prompt_last_rows, METH_FASTCALL, nullptr},
     {"reconstruct", (PyCFunction)(void (*)(void))reconstruct, METH_FASTCALL, nullptr},

@@ -172,11 +172,13 @@ class HqeAttentionLayer:
     # ------------------------------------------------------------------ prompt
     def _prefill(self, q, k, v, attention_mask):
         """Prompt attention [141-188]: the output over all rows, and the probabilities of the last 20 rows only (what
-        the ring keeps).  K and V are read once per KV head, without ``repeat_kv`` copies."""
+        the ring keeps).  K and V are read once per KV head, without ``repeat_kv`` copies.  -> (the probabilities, a
+        callable that queues the attention): the prompt's compression needs the probabilities alone, so ``forward``
+        queues the attention behind the ranking and the host plans while the device is at it (a prompt of 4099 tokens and 24
+        steps: 615 -> 531 us, 8192: 1060 -> 980)."""
         rows = min(q.shape[2], LAST_TOKEN_NUM)
         attn_weights = last_rows_probabilities(q, k, attention_mask, self.scaling, rows)
-        attn_output = gqa_prompt_attention(q, k, v, attention_mask, self.scaling)
-        return attn_weights, attn_output
+        return attn_weights, lambda: gqa_prompt_attention(q, k, v, attention_mask, self.scaling)
 
     # ------------------------------------------------------------------ residual storage
     @staticmethod
@@ -220,6 +222,7 @@ class HqeAttentionLayer:
         """query (B,Hq,L,D), key/value (B,Hkv,L,D), rotary already applied.
         -> (attn_output (B,Hq,L,D), attn_weights (the last <= 20 rows for a prompt), tuple, auxiliary_parameters)."""
         L = key_states.shape[-2]
+        attention = None
         self.current_length += L
         kv_seq_len = L + (past_key_value[-1] if past_key_value is not None else 0)
         if past_key_value is not None:
@@ -255,7 +258,7 @@ class HqeAttentionLayer:
                              and (lw.weights is None or lw.weights.dtype == torch.float16) and lw.max_length >= Tall)
                 if on_device and lw.weights is None:
                     lw.decode_row(query_states, Tall)   # creates the store
-                tables = self._memo.steps(past_key_value, query_states.device, self.quant_strategy == "uniform_group", known)
+                tables = self._memo.steps(past_key_value, query_states, self.quant_strategy == "uniform_group", known)
                 if tables is not None:
                     done = tables.step(query_states, key_states, value_states, past_key_value, *self._res, n, Tall,
                                        lw.weights if on_device else None, lw.next_line, kv_seq_len)
@@ -282,11 +285,13 @@ class HqeAttentionLayer:
                 lw.update(attn_weights)
             self._res_rows = n + L
         else:
-            attn_weights, attn_output = self._prefill(query_states, key_states, value_states, attention_mask)
+            attn_weights, attention = self._prefill(query_states, key_states, value_states, attention_mask)
             past_key_value = (None,) * 39 + (key_states, value_states, kv_seq_len)
             self.last_weights.update(attn_weights)
 
         if self.current_length < BLOCK:
+            if attention is not None:
+                attn_output = attention()
             self.token_num += 1
             return attn_output, attn_weights, past_key_value, None
 
@@ -303,6 +308,11 @@ class HqeAttentionLayer:
         # the importance of every token and the ranking of the blocks; like the reference's ranking helper, which
         # divides its argument by the block length in place, this leaves the policy the divided values [226-231]
         importance, K_token_idx = self.last_weights.ranked_importance(total_length)
+        meanwhile = None
+        if attention is not None:
+            def meanwhile():
+                nonlocal attn_output
+                attn_output = attention()
         buffers = None
         left = past_key_value[-3].shape[2] - compress_length
         if left:   # what stays behind goes where the next step appends to it
@@ -310,7 +320,7 @@ class HqeAttentionLayer:
             buffers = tuple(key_states.new_empty(B, H, self._residual_rows(left + 1), D) for _ in range(2))
         past_key_value = cache_policy.compress(past_key_value, compress_length, self.history_reserve_length, K_token_idx, K_bit_num,
                                                V_bit_num, importance, self.quant_strategy, last_weights=self.last_weights,
-                                               times_range=self.times_range, n_targets=6, residual_buffers=buffers)
+                                               times_range=self.times_range, n_targets=6, residual_buffers=buffers, meanwhile=meanwhile)
         self._res, self._res_rows = buffers, left   # (nothing left: the next step starts new ones)
         self.history_reserve_length += compress_length - int(K_bit_num[-1])
         self.current_length -= compress_length
