@@ -306,6 +306,9 @@ struct LastRowsArgs {
   int32_t slices;
 };
 
+struct __attribute__((packed, aligned(2))) lr_quad_t { uint64_t v; };    // four fp16 at an element's alignment
+struct __attribute__((packed, aligned(2))) lr_oct_t { uint64_t v[2]; };  // eight
+
 // One score tile's 16 values per lane, as the reference's fp16 chain leaves them: query column `my_q` (its mask row
 // `mrow`, or the causal rule) against keys 32 * tile + 8 (r / 4) + 4 h + r % 4; -inf where no key is visible.
 __device__ __forceinline__ void lr_logits(const LastRowsArgs &a, f16_t s, const half_t *mrow, int tile, int h, int my_q, half_t (&x)[16]) {
@@ -340,8 +343,9 @@ __device__ __forceinline__ void lr_tile_stats(const half_t (&x)[16], float &m, f
   l = l * __expf(m - mx) + part;
   m = mx;
 }
-// over the two halves of every wave, then the four waves: afterwards every thread holds column n's pair
-__device__ __forceinline__ void lr_merge(float &m, float &l, int n, int h, int w, float (&sh_m)[PA_WAVES][32], float (&sh_l)[PA_WAVES][32]) {
+// over the two halves of every wave, then the waves: afterwards every thread holds column n's pair
+template <int WAVES>
+__device__ __forceinline__ void lr_merge(float &m, float &l, int n, int h, int w, float (&sh_m)[WAVES][32], float (&sh_l)[WAVES][32]) {
   const float mo = __shfl_xor(m, 32, 64), lo = __shfl_xor(l, 32, 64);
   const float mx = fmaxf(m, mo);
   l = (m == -INFINITY ? 0.f : l * __expf(m - mx)) + (mo == -INFINITY ? 0.f : lo * __expf(mo - mx));
@@ -352,10 +356,10 @@ __device__ __forceinline__ void lr_merge(float &m, float &l, int n, int h, int w
   __syncthreads();
   m = -INFINITY;
 #pragma unroll
-  for (int k = 0; k < PA_WAVES; ++k) m = fmaxf(m, sh_m[k][n]);
+  for (int k = 0; k < WAVES; ++k) m = fmaxf(m, sh_m[k][n]);
   l = 0.f;
 #pragma unroll
-  for (int k = 0; k < PA_WAVES; ++k) l += sh_m[k][n] == -INFINITY ? 0.f : sh_l[k][n] * __expf(sh_m[k][n] - m);
+  for (int k = 0; k < WAVES; ++k) l += sh_m[k][n] == -INFINITY ? 0.f : sh_l[k][n] * __expf(sh_m[k][n] - m);
 }
 
 // Without room for the slices' statistics: one workgroup per (b, query head) walks all keys twice.
@@ -407,15 +411,83 @@ __global__ __launch_bounds__(PA_THREADS, 2) void prompt_last_rows_kernel(LastRow
   }
 }
 
-// With that room, two launches.  Bound: HBM (K once, the rows' probabilities twice through the memory-side cache).
+// Short prompts in one launch: the R rows of a KV head's query heads as columns of 32-column tiles, a workgroup per column
+// tile, one of its waves per 32 keys; the logits stay in registers until the row's statistics are there.  Bound: one chain --
+// K rows -> LDS -> products -> statistics across the waves -> stores -- and, with sixteen waves on a CU, their vector
+// instructions (a second tile per wave costs 6 us: 1003 keys 14.6 us against 10.1 in two launches).  K and the query rows are
+// fetched whole rows at a time and turned in LDS: as fragments straight from memory, 32 lines per load, a CU's address unit
+// alone took 4 us per sixteen tiles.
+__device__ __forceinline__ int ls_piece(int row, int piece) { return row * PA_D + ((piece ^ (row & 15)) << 3); }   // 16-byte pieces, in halves
+template <int WAVES>
+__global__ __launch_bounds__(WAVES * 64, 1) void prompt_last_short_kernel(LastRowsArgs a) {
+  __shared__ __align__(16) half_t sh_k[WAVES][32 * PA_D];
+  __shared__ __align__(16) half_t sh_q[32 * PA_D];
+  __shared__ float sh_m[WAVES][32], sh_l[WAVES][32];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n = lane & 31, h = lane >> 5, r4 = lane >> 4, piece = lane & 15;   // (a load takes four rows)
+  const int b = (int)blockIdx.x / a.Hkv, hkv = (int)blockIdx.x % a.Hkv;
+  const int T = a.T, R = a.R, nrep = a.Hq / a.Hkv;
+  half_t *ks = sh_k[w];
+  {
+    const half_t *kp = a.k + b * a.k_b + hkv * a.k_h + 8 * piece;
+    const half_t *qp = a.q + b * a.q_b + hkv * nrep * a.q_h + 8 * piece;
+    h8_t k[8], q[8 / WAVES + 1];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) k[j] = *reinterpret_cast<const h8_t *>(kp + (int64_t)min(32 * w + 4 * j + r4, T - 1) * a.k_t);
+#pragma unroll
+    for (int j = 0; 4 * WAVES * j < 32; ++j) {
+      const int c = min(32 * (int)blockIdx.y + ((4 * (WAVES * j + w) + r4) & 31), nrep * R - 1);   // (columns past the last one repeat it)
+      q[j] = *reinterpret_cast<const h8_t *>(qp + (c / R) * a.q_h + (int64_t)(T - R + c % R) * a.q_t);
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) *reinterpret_cast<h8_t *>(ks + ls_piece(4 * j + r4, piece)) = k[j];
+#pragma unroll
+    for (int j = 0; 4 * WAVES * j < 32; ++j)
+      if (4 * (WAVES * j + w) < 32) *reinterpret_cast<h8_t *>(sh_q + ls_piece(4 * (WAVES * j + w) + r4, piece)) = q[j];
+  }
+  const int col = 32 * (int)blockIdx.y + n;                    // (query head of the group, row)
+  const bool live = col < nrep * R;                            // lanes past the last column store nothing
+  const int hq = hkv * nrep + (live ? col : nrep * R - 1) / R, row = (live ? col : nrep * R - 1) % R;
+  const half_t *mrow = a.mask ? a.mask + b * a.m_b + (int64_t)row * a.m_r : nullptr;
+  __syncthreads();
+  f16_t s = (f16_t)(0.f);
+#pragma unroll
+  for (int st = 0; st < 8; ++st)
+    s = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const h8_t *>(ks + ls_piece(n, 2 * st + h)),
+                                               *reinterpret_cast<const h8_t *>(sh_q + ls_piece(n, 2 * st + h)), s, 0, 0, 0);
+  half_t x[16];
+  float m = -INFINITY, l = 0.f;
+  lr_logits(a, s, mrow, w, h, T - R + row, x);   // (a tile past the last one: no key is visible)
+  lr_tile_stats(x, m, l);
+  lr_merge(m, l, n, h, w, sh_m, sh_l);
+  if (!live) return;
+  const float inv = 1.0f / l;
+  half_t *prow = a.probs + (((int64_t)b * a.Hq + hq) * R + row) * (int64_t)T;
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    const int key = 32 * w + 8 * g + 4 * h;
+    half_t p[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) p[j] = (half_t)(__expf((float)x[4 * g + j] - m) * inv);
+    if (key + 3 < T) {
+      lr_quad_t y;
+      __builtin_memcpy(&y, p, 8);
+      *reinterpret_cast<lr_quad_t *>(prow + key) = y;
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (key + j < T) prow[key + j] = p[j];
+    }
+  }
+}
+
+// With room for the slices' statistics, two launches.  Bound: HBM (K once, the rows' probabilities twice through the memory-side cache).
 // prompt_last_logits_kernel: the R rows of all query heads of a KV head lie side by side as columns of 32-column tiles
 // (4 heads x 20 rows: three tiles instead of four that are 3/8 empty); a workgroup takes one column tile and one slice of
 // the keys, leaves the logits where the probabilities will be -- four keys of a row per 8-byte store -- and the slice's
 // (maximum, sum) per row.  prompt_last_probs_kernel turns rows of logits into probabilities, 16 bytes per lane.  Walking
 // the keys a second time instead of the stored logits, with slices of 2048 keys and more: 38.8 us at T = 1003 (one slice),
 // 175 us at T = 32768 (32 heads over 8); now 9 us and 72 us.
-struct __attribute__((packed, aligned(2))) lr_quad_t { uint64_t v; };    // four fp16 at an element's alignment
-struct __attribute__((packed, aligned(2))) lr_oct_t { uint64_t v[2]; };  // eight
 __global__ __launch_bounds__(PA_THREADS, 3) void prompt_last_logits_kernel(LastRowsArgs a) {
   __shared__ float sh_m[PA_WAVES][32], sh_l[PA_WAVES][32];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -572,15 +644,19 @@ extern "C" int hqekv_prompt_attn(const void *q, const int64_t *q_strides, const 
   return check_launch("prompt_attn");
 }
 
-// Slices of the keys: about 48 (b, query head) slices per column tile's 32 give the chip four to six workgroups per CU;
-// a slice keeps a tile for each of its four waves.  Up to 128 keys the one-launch kernel has nothing to gain from slices.
+// Up to 512 keys one launch, a wave per 32 keys.  One launch against two, us (32 heads over 8, 20 rows, host included): 128 keys
+// 6.2 / 7.1 (one workgroup of four waves per head then), 256 7.1 / 9.3, 512 8.2 / 9.4; B = 4 500 8.0 / 14.2, B = 64 64 / 126;
+// 1003 keys at two tiles per wave 14.6 / 10.1, B = 4 15.3 / 17.6.
+constexpr int64_t LS_KEYS = 512;
+// Beyond, slices of the keys: about 48 (b, query head) slices per column tile's 32 give the chip four to six workgroups per CU;
+// a slice keeps a tile for each of its four waves.
 static int last_rows_slices(int64_t B, int64_t Hq, int64_t T) {
   int64_t s = (1536 + B * Hq - 1) / (B * Hq);
   const int64_t most = (T + 127) / 128;
   if (s > most) s = most;
   if (s > 64) s = 64;
   if (s < 2) s = 2;
-  return T <= 128 || B * Hq * 32 > 65535 ? 1 : (int)s;
+  return T <= LS_KEYS || B * Hq * 32 > 65535 ? 1 : (int)s;
 }
 
 extern "C" int64_t hqekv_prompt_last_rows_workspace_bytes(int64_t B, int64_t Hq, int64_t T) {
@@ -606,6 +682,19 @@ extern "C" int hqekv_prompt_last_rows(const void *q, const int64_t *q_strides, c
   a.k_b = k_strides[0]; a.k_h = k_strides[1]; a.k_t = k_strides[2];
   a.m_b = mask ? mask_strides[0] : 0; a.m_r = mask ? mask_strides[1] : 0;
   a.Hq = (int32_t)Hq; a.Hkv = (int32_t)Hkv; a.T = (int32_t)T; a.R = (int32_t)R; a.scale = scale;
+  const int64_t columns = (Hq / Hkv * R + 31) / 32;
+  if (T <= LS_KEYS && B * Hkv <= 0x7fffffffLL && columns <= 65535) {
+    const dim3 grid((unsigned)(B * Hkv), (unsigned)columns);
+    a.partial = nullptr;
+    a.slices = 1;
+#define LAUNCH(W_) hipLaunchKernelGGL(prompt_last_short_kernel<W_>, grid, dim3(W_ * 64), 0, (hipStream_t)stream, a)
+    if (T <= 64) LAUNCH(2);
+    else if (T <= 128) LAUNCH(4);
+    else if (T <= 256) LAUNCH(8);
+    else LAUNCH(16);
+#undef LAUNCH
+    return check_launch("prompt_last_rows");
+  }
   // the keys in slices when the caller brought room for the slices' statistics; else one workgroup per head
   const int sl = last_rows_slices(B, Hq, T);
   const int64_t need = hqekv_prompt_last_rows_workspace_bytes(B, Hq, T);

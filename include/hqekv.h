@@ -384,6 +384,7 @@ int hqekv_rank_blocks(const void *const *scores, int rows, int64_t n, int32_t *o
  *                           and row strides (key stride 1), or NULL for the causal rule (row r sees keys <= T - R + r).
  *                           workspace (hqekv_prompt_last_rows_workspace_bytes, may be 0): room for per-slice statistics,
  *                           with which few heads are spread over the chip in two launches; NULL: one workgroup per head.
+ *                           Up to 512 keys one launch either way.
  */
 int hqekv_prompt_attn(const void *q, const int64_t *q_strides, const void *k, const int64_t *k_strides, const void *v,
                       const int64_t *v_strides, void *out, const int64_t *out_strides, int64_t B, int64_t Hq, int64_t Hkv,
