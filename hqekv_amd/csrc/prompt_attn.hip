@@ -219,9 +219,9 @@ __global__ __launch_bounds__(PA_THREADS, S::WGS) void prompt_attn_kernel(PromptA
       m = mx;
     }
     const float base = KS > 1 && mx == -INFINITY ? 0.f : mx;   // nothing but masked keys so far: exponentials of -inf are zero
-    float part = 0.f;
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
+      float part = 0.f;
       h8_t p[2];
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
@@ -229,6 +229,7 @@ __global__ __launch_bounds__(PA_THREADS, S::WGS) void prompt_attn_kernel(PromptA
         part += e;
         p[r >> 3][r & 7] = (half_t)e;
       }
+      lsum += part;
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -244,7 +245,6 @@ __global__ __launch_bounds__(PA_THREADS, S::WGS) void prompt_attn_kernel(PromptA
           o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av, p[t], o[dt], 0, 0, 0);
         }
     }
-    lsum += part;
   };
   // two steps per round, so that each half works on fixed buffers; an odd count runs one step more, all of it masked
   for (int j = 0; j < n_steps; j += 2) {
