@@ -417,6 +417,11 @@ __global__ __launch_bounds__(PA_THREADS, 2) void prompt_last_rows_kernel(LastRow
 // instructions (a second tile per wave costs 6 us: 1003 keys 14.6 us against 10.1 in two launches).  K and the query rows are
 // fetched whole rows at a time and turned in LDS: as fragments straight from memory, 32 lines per load, a CU's address unit
 // alone took 4 us per sixteen tiles.
+// (a wave's own LDS traffic in order, without a barrier)
+__device__ __forceinline__ void lr_wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
 __device__ __forceinline__ int ls_piece(int row, int piece) { return row * PA_D + ((piece ^ (row & 15)) << 3); }   // 16-byte pieces, in halves
 template <int WAVES>
 __global__ __launch_bounds__(WAVES * 64, 1) void prompt_last_short_kernel(LastRowsArgs a) {
@@ -487,38 +492,59 @@ __global__ __launch_bounds__(WAVES * 64, 1) void prompt_last_short_kernel(LastRo
 // the keys, leaves the logits where the probabilities will be -- four keys of a row per 8-byte store -- and the slice's
 // (maximum, sum) per row.  prompt_last_probs_kernel turns rows of logits into probabilities, 16 bytes per lane.  Walking
 // the keys a second time instead of the stored logits, with slices of 2048 keys and more: 38.8 us at T = 1003 (one slice),
-// 175 us at T = 32768 (32 heads over 8); now 9 us and 72 us.
+// 175 us at T = 32768 (32 heads over 8); now 9 us and 53 us.  K and the query rows are fetched whole rows at a time and turned in
+// LDS, in a wave's own corner: as fragments straight from memory, 32 lines per load, T = 4099 19.0 us against 15.4, B = 2 29.0 /
+// 22.3, 8192 27.9 / 21.0, 32768 65.9 / 52.6.
 __global__ __launch_bounds__(PA_THREADS, 3) void prompt_last_logits_kernel(LastRowsArgs a) {
+  __shared__ __align__(16) half_t sh_k[PA_WAVES][32 * PA_D];
+  __shared__ __align__(16) half_t sh_q[32 * PA_D];
   __shared__ float sh_m[PA_WAVES][32], sh_l[PA_WAVES][32];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int n = lane & 31, h = lane >> 5;
+  const int n = lane & 31, h = lane >> 5, r4 = lane >> 4, piece = lane & 15;   // (a load takes four rows)
   const int b = (int)blockIdx.x / a.Hkv, hkv = (int)blockIdx.x % a.Hkv;
   const int T = a.T, R = a.R, nrep = a.Hq / a.Hkv;
-  const int col = 32 * (int)blockIdx.z + n;                    // (query head of the group, row)
-  const bool live = col < nrep * R;                            // lanes past the last column repeat it and store nothing
-  const int hq = hkv * nrep + (live ? col : nrep * R - 1) / R, row = (live ? col : nrep * R - 1) % R;
-  const half_t *kp = a.k + b * a.k_b + hkv * a.k_h;
-  const int my_q = T - R + row;
-  h8_t qreg[8];
-  {
-    const half_t *qr = a.q + b * a.q_b + hq * a.q_h + (int64_t)my_q * a.q_t + 8 * h;
-#pragma unroll
-    for (int s = 0; s < 8; ++s) qreg[s] = *reinterpret_cast<const h8_t *>(qr + 16 * s);
-  }
-  const half_t *mrow = a.mask ? a.mask + b * a.m_b + (int64_t)row * a.m_r : nullptr;
   const int all_tiles = (T + 31) / 32, per_slice = (all_tiles + a.slices - 1) / a.slices;
   const int tile0 = (int)blockIdx.y * per_slice, n_tiles = min(all_tiles, tile0 + per_slice);
+  const half_t *kp = a.k + b * a.k_b + hkv * a.k_h + 8 * piece;
+  half_t *ks = sh_k[w];
+  h8_t k[8];
+  auto fetch = [&](int tile) {   // (rows past the last one repeat it)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) k[j] = *reinterpret_cast<const h8_t *>(kp + (int64_t)min(32 * tile + 4 * j + r4, T - 1) * a.k_t);
+  };
+  fetch(min(tile0 + w, all_tiles - 1));
+  {
+    const half_t *qp = a.q + b * a.q_b + hkv * nrep * a.q_h + 8 * piece;
+    h8_t q[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int c = min(32 * (int)blockIdx.z + 4 * (PA_WAVES * j + w) + r4, nrep * R - 1);   // (columns past the last one repeat it)
+      q[j] = *reinterpret_cast<const h8_t *>(qp + (c / R) * a.q_h + (int64_t)(T - R + c % R) * a.q_t);
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) *reinterpret_cast<h8_t *>(sh_q + ls_piece(4 * (PA_WAVES * j + w) + r4, piece)) = q[j];
+  }
+  const int col = 32 * (int)blockIdx.z + n;                    // (query head of the group, row)
+  const bool live = col < nrep * R;                            // lanes past the last column store nothing
+  const int hq = hkv * nrep + (live ? col : nrep * R - 1) / R, row = (live ? col : nrep * R - 1) % R, my_q = T - R + row;
+  const half_t *mrow = a.mask ? a.mask + b * a.m_b + (int64_t)row * a.m_r : nullptr;
   half_t *prow = a.probs + (((int64_t)b * a.Hq + hq) * R + row) * (int64_t)T;
   float m = -INFINITY, l = 0.f;
-  h8_t k[8];
-  lr_load_keys(kp, a.k_t, T, min(tile0 + w, all_tiles - 1), n, h, k);
+  __syncthreads();
+  h8_t qreg[8];
+#pragma unroll
+  for (int st = 0; st < 8; ++st) qreg[st] = *reinterpret_cast<const h8_t *>(sh_q + ls_piece(n, 2 * st + h));
 #pragma unroll 1
   for (int tile = tile0 + w; tile < n_tiles; tile += PA_WAVES) {
-    f16_t s = (f16_t)(0.f);
-    h8_t nxt[8];
-    lr_load_keys(kp, a.k_t, T, min(tile + PA_WAVES, all_tiles - 1), n, h, nxt);   // (past the last one: read, not used)
 #pragma unroll
-    for (int st = 0; st < 8; ++st) s = __builtin_amdgcn_mfma_f32_32x32x16_f16(k[st], qreg[st], s, 0, 0, 0);
+    for (int j = 0; j < 8; ++j) *reinterpret_cast<h8_t *>(ks + ls_piece(4 * j + r4, piece)) = k[j];
+    fetch(min(tile + PA_WAVES, all_tiles - 1));   // (past the last one: read, not used)
+    lr_wave_fence();   // (a wave's own corner: no other wave waits for it)
+    f16_t s = (f16_t)(0.f);
+#pragma unroll
+    for (int st = 0; st < 8; ++st)
+      s = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const h8_t *>(ks + ls_piece(n, 2 * st + h)), qreg[st], s, 0, 0, 0);
+    lr_wave_fence();
     half_t x[16];
     lr_logits(a, s, mrow, tile, h, my_q, x);
     lr_tile_stats(x, m, l);
@@ -537,8 +563,6 @@ __global__ __launch_bounds__(PA_THREADS, 3) void prompt_last_logits_kernel(LastR
         }
       }
     }
-#pragma unroll
-    for (int st = 0; st < 8; ++st) k[st] = nxt[st];
   }
   lr_merge(m, l, n, h, w, sh_m, sh_l);
   if (threadIdx.x < 32 && live) a.partial[((int64_t)b * a.Hq + hq) * R * a.slices + (int64_t)row * a.slices + blockIdx.y] = make_float2(m, l);
