@@ -627,6 +627,18 @@ def _compress_gather(pkv: tuple, new_K, new_V, res_K, res_V, history: int, compr
     return tuple(t)
 
 
+class _Once:
+    """A callable that forwards its first call."""
+
+    def __init__(self, call):
+        self.call = call
+
+    def __call__(self):
+        call, self.call = self.call, None
+        if call is not None:
+            call()
+
+
 def compress(past_key_value: tuple, compress_length: int, history_length, K_sorted_idx: torch.Tensor,
              K_bit_num: torch.Tensor, V_bit_num: torch.Tensor, token_importance: torch.Tensor,
              quant_strategy: str, *, last_weights=None, block_size: int = 32, group_size: int = 32,
@@ -642,12 +654,8 @@ def compress(past_key_value: tuple, compress_length: int, history_length, K_sort
         raise ValueError('invalid quant_strategy')
     if block_size != BLOCK or group_size != BLOCK:
         raise ValueError("block_size and group_size must be 32")
-    called = []
-
-    def once():
-        if meanwhile is not None and not called:
-            called.append(True)
-            meanwhile()
+    if meanwhile is not None:
+        meanwhile = _Once(meanwhile)
     pkv = past_key_value
     new_K, new_V = pkv[39], pkv[40]
     if new_K is None or new_V is None:
@@ -667,12 +675,13 @@ def compress(past_key_value: tuple, compress_length: int, history_length, K_sort
         ring = last_weights.weights if type(last_weights) is last_attn_weights else None
         done = _lib.host().compress(pkv, history, compress_length, K_sorted_idx.scores, token_importance, bool(times_range),
                                     V_token_range, K_bit_num, V_bit_num, quant_strategy == LOW_NORMAL,
-                                    ring, residual_buffers, _new_array, weakref.ref, None if meanwhile is None else once)
+                                    ring, residual_buffers, _new_array, weakref.ref, meanwhile)
         if done is not None:
             if done[1] is not None and last_weights is not None:
                 last_weights.eviction(done[1])
             return done[0]
-    once()
+    if meanwhile is not None:
+        meanwhile()
     whole = new_K.shape[2] == compress_length and new_V.shape[2] == compress_length   # nothing stays behind
     res_K = None if whole else _none_if_empty(new_K[:, :, compress_length:, :].clone())
     res_V = None if whole else _none_if_empty(new_V[:, :, compress_length:, :].clone())

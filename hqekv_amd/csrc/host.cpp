@@ -1034,15 +1034,7 @@ bool host_orders(const void *const (&scores)[2], int64_t n, const Tensor &order,
   volatile int32_t *p = (volatile int32_t *)order.data_ptr();
   for (int64_t i = 0; i < 2 * n; ++i) p[i] = -1;
   hipError_t err = hipSuccess;
-  const int rc = without_gil([&] { return api.hqekv_rank_blocks(scores, 2, n, (int32_t *)order.data_ptr(), stream_of(dev)); });
-  if (rc) {
-    raise_rc(rc, "rank_blocks");
-    return false;
-  }
-  PyObject *did = meanwhile == Py_None ? nullptr : PyObject_CallNoArgs(meanwhile);
-  const bool raised = meanwhile != Py_None && !did;
-  Py_XDECREF(did);
-  without_gil([&]() -> int {
+  auto wait = [&] {
     const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(2);
     int64_t i = 0;
     while (i < 2 * n) {
@@ -1054,7 +1046,22 @@ bool host_orders(const void *const (&scores)[2], int64_t n, const Tensor &order,
       }
     }
     return HQEKV_OK;
+  };
+  const int rc = without_gil([&]() -> int {
+    const int rc = api.hqekv_rank_blocks(scores, 2, n, (int32_t *)order.data_ptr(), stream_of(dev));
+    return rc || meanwhile != Py_None ? rc : wait();
   });
+  if (rc) {
+    raise_rc(rc, "rank_blocks");
+    return false;
+  }
+  bool raised = false;
+  if (meanwhile != Py_None) {
+    PyObject *did = PyObject_CallNoArgs(meanwhile);
+    raised = !did;
+    Py_XDECREF(did);
+    without_gil(wait);
+  }
   if (raised) return false;
   if (err != hipSuccess) PyErr_Format(PyExc_RuntimeError, "rank_blocks: HIP error %d", (int)err);
   return err == hipSuccess;
