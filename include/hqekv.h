@@ -229,7 +229,8 @@ int hqekv_pv_hybrid(const hqekv_seg *segs, int nseg, const void *p, void *out, i
  *   idx arrays and any mask.
  * flags & HQEKV_FUSE_SOFTMAX: no softmax launch.  The q.K^T launch stores scaled logits and per-tile softmax
  *   statistics, the p.V launch normalises while it gathers; the fixed-order combine stays a third,
- *   small launch.  REQUIRES that the idx arrays of the K segments, and those of the V segments, each cover
+ *   small launch (short steps: at most 20 partial rows per KV head, no form named by the flags, room in the workspace: it
+ *   runs in the p.V launch).  REQUIRES that the idx arrays of the K segments, and those of the V segments, each cover
  *   every position in [0, Tall) exactly once (true for every cache the reference's cache policy builds);
  *   taken only when mask == NULL and both segment lists hold exactly Tall tokens, otherwise the call
  *   silently runs the flags = 0 path.
@@ -297,8 +298,8 @@ int hqekv_decode_attn(const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_segs,
  *                                                          in capacity-sized buffers (see hqekv_seg.slab_tokens)
  *   last_weights.update(attn_weights)                      one row of the importance ring:
  *                                                          attn_weights.sum(0).sum(0), model/public_func.py:243-257
- * -- folded into the call's last launch (extra workgroups of the split-K combine, or a launch of their own when the
- * combine runs inside p.V).  The ring row follows the order in which torch's GPU reduction adds the rows (fp32
+ * -- folded into the call's last launch (extra workgroups of the split-K combine or, in a short step, of p.V; a launch
+ * of their own when HQEKV_FOLD_COMBINE puts the combine inside p.V).  The ring row follows the order in which torch's GPU reduction adds the rows (fp32
  * accumulation, one rounding to fp16 per reduction): ring_order is the number of threads that reduction deals the
  * head rows to for the shape at hand -- 2 when Tall is a multiple of 4, at least 256, and attn_weights is 8-byte
  * aligned; else 1 -- pinned against torch.sum on the device for 32 heads and batch sizes 1..8.
