@@ -51,7 +51,7 @@ constexpr int RING_V = 4;                 // adjacent columns of the ring row a 
 // with a head row per 16 lanes, all heads of a batch row in flight at once and four times as many workgroups: the form for
 // rows that fit one such pass or two (3.3k columns in a step's last launch: 5.4 -> 4.2 us).
 constexpr int RING_SPAN = 64 * RING_V, RING_SPAN_SHORT = 16 * RING_V;
-constexpr int RING_BLOCKS = 512;          // workgroups of a launch of its own: two per CU
+constexpr int RING_BLOCKS = 512;          // workgroups of a launch of its own, at most
 constexpr int RING_LDS_HEADS = 64;        // most heads whose batch sums a pass parks in LDS
 
 // The probabilities as a pointer into global memory: the pointer arrives inside a by-value struct, where the
@@ -75,8 +75,10 @@ struct RingShape {
 template <int NB, int SPAN, bool ALONE, typename Prob>
 __device__ __forceinline__ void ring_heads_to_lds(const RingShape r, ring_src_t col, int shift, int g, int waves,
                                                   half_t *tile_lane, Prob &&prob) {
-  // heads in flight per thread: about eight loads; in short passes the 32 heads are dealt to 64 (16) groups of lanes
-  constexpr int HU = SPAN == RING_SPAN ? 8 / NB : ALONE ? 1 : 2;
+  // heads in flight per thread: in long passes the 32 heads are dealt to 16 groups of lanes, two each (eight loads at most, or
+  // the registers of the pass grow), in short ones to 64 (16) groups.  (A head past the last one is loaded again: with eight
+  // heads in flight for one batch row 20 rows of 4099 probabilities took 9.7 us, now 8.5, of 32768 32.1 / 23.8.)
+  constexpr int HU = SPAN == RING_SPAN ? (NB > 4 ? 1 : 2) : ALONE ? 1 : 2;
   const int64_t hs = r.Tall, bs = (int64_t)r.Hq * r.Tall;
   for (int h0 = g; h0 < r.Hq; h0 += waves * HU) {
     uint64_t raw[HU][NB];   // a quad is loaded, shifted and stored as one 64-bit word
@@ -163,7 +165,12 @@ __device__ __forceinline__ void ring_row_columns(const StepEpilogue &e, int64_t 
         sum = ring_column_alone(r, t);
       }
       // (several rows at once: the columns are (row, token) pairs)
-      line[e.ring_tokens ? t / e.ring_tokens * e.ring_stride + t % e.ring_tokens : t] = (half_t)sum;
+      if (e.ring_tokens) {   // (the store holds fewer than 2^31 elements)
+        const uint32_t n = (uint32_t)e.ring_tokens, row = (uint32_t)t / n;
+        line[row * (uint32_t)e.ring_stride + ((uint32_t)t - row * n)] = (half_t)sum;
+      } else {
+        line[t] = (half_t)sum;
+      }
     }
     if (lds) __syncthreads();
   }
