@@ -122,10 +122,10 @@ struct TilesPlan {
 };
 // head_dim 128, at most 16 query heads per KV head (the rows of A), channel-major fp16 K classes of whole 8-token columns.
 // Every ratio up to there is faster here than in the forms of attn.hip, also where rows are spare.  A step at 1k, 32k and
-// 8 x 64k tokens of the fp16 / 8 / 4 / 2-bit mix, us, here against there: 1 head 10.7 / 14.4, 21.9 / 25.1, 158 / 178; 2 heads
-// 10.8 / 15.5, 22.8 / 26.8, 167 / 187; 4 heads 10.8 / 17.3, 23.3 / 29.3, 178 / 205; 5 heads 11.9 / 20.9, 25.2 / 38.8, 201 /
-// 260; 8 heads 12.0 / 23.3, 26.7 / 51.9, 221 / 322; 9 heads 14.1 / 35.7, 31.8 / 70.4, 242 / 489; 16 heads 15.4 / 45.8, 35.8 /
-// 98.2, 295 / 644.  (One head: p.V alone is a tie, q.K^T is what gains.)
+// 8 x 64k tokens of the fp16 / 8 / 4 / 2-bit mix, us, here against there: 1 head 10.1 / 14.4, 19.4 / 25.1, 153 / 178; 2 heads
+// 10.1 / 15.5, 19.9 / 26.8, 159 / 187; 4 heads 10.2 / 17.3, 20.7 / 29.3, 172 / 205; 5 heads 10.7 / 20.9, 22.6 / 38.8, 180 /
+// 260; 8 heads 10.6 / 23.3, 24.6 / 51.9, 200 / 322; 9 heads 13.3 / 35.7, 28.3 / 70.4, 225 / 489; 16 heads 14.2 / 45.8, 32.4 /
+// 98.2, 275 / 644.  (One head: p.V alone is a tie, q.K^T is what gains.)
 bool tiles_fit(const hqekv_seg *segs, int nseg, bool is_k, int64_t D, int64_t B, int64_t Hq, int64_t Hkv);
 TilesPlan tiles_plan(const hqekv_seg *segs, int nseg, bool is_k, int64_t BHkv, int64_t nrep);
 int64_t tiles_unit_tokens(const TilesPlan &p, const hqekv_seg &s);
