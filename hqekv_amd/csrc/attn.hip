@@ -2004,6 +2004,24 @@ static int64_t seg_total_tokens(const hqekv_seg *segs, int nseg) {
   return n;
 }
 
+static bool has_epilogue(const StepEpilogue &e) { return e.ring_line || e.app_rows > 0 || e.leave_bits; }
+// The epilogue rides in the combine launch as extra workgroups: as many layers of grid.z (B * Hq * D / 32 workgroups each)
+// as make one workgroup per RING_SPAN columns of the ring row at the least.  Without a combine (the partial rows added by p.V)
+// the launch holds the epilogue alone.
+static int launch_combine(const float *partial, void *out, int n_chunks, int64_t n_bhq, int64_t D, int64_t Tall, bool combine, const StepEpilogue *ep,
+                          hipStream_t st) {
+  const dim3 base((unsigned)n_bhq, (unsigned)((D + CB_CH - 1) / CB_CH));
+  unsigned z = combine ? 1u : 0u;
+  if (ep) {
+    const int64_t want = ep->ring_line ? (Tall + RING_SPAN - 1) / RING_SPAN : 1;
+    z += (unsigned)((want + (int64_t)base.x * base.y - 1) / ((int64_t)base.x * base.y));
+  }
+  StepEpilogue none{};
+  hipLaunchKernelGGL(pv_combine_kernel, dim3(base.x, base.y, z), dim3(CB_CH * CB_SLICES), 0, st, partial, (half_t *)out, n_chunks, n_bhq, (int)D,
+                     ep ? *ep : none, combine ? 1 : 0);
+  return check_launch("pv_combine_kernel");
+}
+
 static int launch_pv(const SegTable &tb, int64_t chunk, void *p, void *out, float *partial, int64_t B,
                      int64_t Hq, int64_t Hkv, int64_t D, int64_t Tall, const FuseArgs &fz, hipStream_t st,
                      bool mf, int stages = 3, const StepEpilogue *ep = nullptr) {
@@ -2042,7 +2060,7 @@ static int launch_pv(const SegTable &tb, int64_t chunk, void *p, void *out, floa
     }
   }
   const bool combine = (stages & 2) && !fz.arrive;   // folded: the last p.V workgroups have written the output
-  const bool epilogue = ep && (ep->ring_line || ep->app_rows > 0 || ep->leave_bits) && stages == 3;
+  const bool epilogue = ep && has_epilogue(*ep) && stages == 3;
   if (!combine && !epilogue) return HQEKV_OK;
   if (tb.per_unit && !epilogue) {
     // A workgroup per row, four where rows are few and long (device time of a step, one / four / the 16-wave form, us: 32 rows
@@ -2056,19 +2074,7 @@ static int launch_pv(const SegTable &tb, int64_t chunk, void *p, void *out, floa
 #undef LAUNCH
     return check_launch("pv_rows_sum_kernel");
   }
-  // The epilogue rides in the combine launch as extra workgroups: as many layers of grid.z (B * Hq * D / 32 workgroups each)
-  // as make one workgroup per RING_SPAN columns of the ring row at the least.  Without a combine (folded into p.V) the
-  // launch holds the epilogue alone.
-  const dim3 base((unsigned)n_bhq, (unsigned)((D + CB_CH - 1) / CB_CH));
-  unsigned z = combine ? 1u : 0u;
-  if (epilogue) {
-    const int64_t want = ep->ring_line ? (Tall + RING_SPAN - 1) / RING_SPAN : 1;
-    z += (unsigned)((want + (int64_t)base.x * base.y - 1) / ((int64_t)base.x * base.y));
-  }
-  StepEpilogue none{};
-  hipLaunchKernelGGL(pv_combine_kernel, dim3(base.x, base.y, z), dim3(CB_CH * CB_SLICES), 0, st, partial, (half_t *)out,
-                     (int)tb.total_units, n_bhq, (int)D, epilogue ? *ep : none, combine ? 1 : 0);
-  return check_launch("pv_combine_kernel");
+  return launch_combine(partial, out, (int)tb.total_units, n_bhq, D, Tall, combine, epilogue ? ep : nullptr, st);
 }
 
 }  // namespace hq
@@ -2327,6 +2333,78 @@ extern "C" int hqekv_decode_step(const hqekv_seg *k_segs, int n_k, const hqekv_s
                      workspace, workspace_bytes, flags, stream, extra);
 }
 
+// `n` stretches of `bytes` bytes, `step` apart: the slabs of a tensor, or of a window of one.
+struct Stretches {
+  uintptr_t at;
+  int64_t bytes, n, step;
+};
+static bool meet(const Stretches &a, const Stretches &b) {
+  if (!a.at || !b.at || a.bytes <= 0 || b.bytes <= 0 || a.n <= 0 || b.n <= 0) return false;
+  if (a.at + (a.n - 1) * a.step + a.bytes <= b.at || b.at + (b.n - 1) * b.step + b.bytes <= a.at) return false;
+  if (a.n == 1 && b.n == 1) return true;
+  const int64_t step = a.n > 1 ? a.step : b.step;
+  if (step <= 0 || (b.n > 1 && b.step != step)) return true;   // (one inside the other's range: not looked at any closer)
+  // Stretch j of b lies off + (j - i) step bytes behind stretch i of a.  They share a byte where -b.bytes < off + k step <
+  // a.bytes; k is the first difference past the left end of that.
+  const int64_t off = (int64_t)(b.at - a.at), x = -b.bytes - off;
+  const int64_t k = std::max(x / step - (x % step < 0) + 1, -(a.n - 1));
+  return k < b.n && off + k * step < a.bytes;
+}
+static bool pv_reads(const hqekv_seg *v_segs, int n_v, int64_t slabs, int64_t D, const Stretches &w) {
+  for (int k = 0; k < n_v; ++k) {
+    const hqekv_seg &s = v_segs[k];
+    const int64_t n = s.n_tokens, slab = s.slab_tokens > 0 ? s.slab_tokens : n, row = D * s.bits / 8, params = D / 32 * 2;
+    if (n <= 0) continue;
+    if (meet(w, {(uintptr_t)s.data, n * row, slabs, slab * row}) || meet(w, {(uintptr_t)s.idx, n * 8, 1, 0})) return true;
+    if (s.bits != 16 && (meet(w, {(uintptr_t)s.scale, n * params, slabs, slab * params}) || meet(w, {(uintptr_t)s.zero, n * params, slabs, slab * params})))
+      return true;
+  }
+  return false;
+}
+// Does the epilogue write what p.V reads?  (A sliding window whose oldest row the step's value replaces.)
+static bool epilogue_writes_v(const StepEpilogue &e, const hqekv_seg *v_segs, int n_v, int64_t D) {
+  const int64_t slabs = e.app_bh;
+  auto hit = [&](const Stretches &w) { return pv_reads(v_segs, n_v, slabs, D, w); };
+  if (e.ring_line && hit({(uintptr_t)e.ring_line, e.Tall * 2, 1, 0})) return true;
+  if (e.app_rows > 0)
+    for (int side = 0; side < 2; ++side)
+      if (hit({(uintptr_t)e.app_dst[side], e.app_rows * D * 2, slabs, e.app_dst_slab[side] * 2})) return true;
+  if (!e.leave_bits) return false;
+  const int64_t code = (int64_t)e.leave_groups * e.leave_bits * 4, params = (int64_t)e.leave_groups * 2;
+  return hit({(uintptr_t)e.leave_code, code, slabs, e.leave_rows * code}) || hit({(uintptr_t)e.leave_scale, params, slabs, e.leave_rows * params}) ||
+         hit({(uintptr_t)e.leave_zero, params, slabs, e.leave_rows * params});
+}
+
+// Which launches a call takes.
+struct DecodeRoute {
+  bool k_tiles, v_tiles;   // those of decode_qk.hip and decode_pv.hip
+  bool covers;             // the softmax rides in the two GEMV launches
+  bool in_two;             // a short step: q.K^T leaves its logits in the workspace, p.V does the rest
+  bool rides;              // in_two: the epilogue rides in the p.V launch; else a launch of its own follows (same bits)
+  TilesPlan k_plan, v_plan;
+};
+static DecodeRoute decode_route(const DecodeLayout &L, const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_segs, int n_v, bool mask, const void *attn_out,
+                                int64_t B, int64_t Hq, int64_t Hkv, int64_t D, int64_t Tall, int flags, const StepEpilogue &ep) {
+  DecodeRoute r{};
+  // The launches of decode_qk.hip and decode_pv.hip take the call unless it names a form of the older ones.
+  const bool by_rule = !(flags & (HQEKV_QK_TILING(0xf) | HQEKV_DOT_MFMA | HQEKV_DOT_VALU | HQEKV_TWO_STEP_DEQUANT | HQEKV_FOLD_COMBINE |
+                                 HQEKV_SEPARATE_COMBINE));
+  r.k_tiles = by_rule && n_k > 0 && tiles_fit(k_segs, n_k, true, D, B, Hq, Hkv);
+  r.v_tiles = by_rule && n_v > 0 && tiles_fit(v_segs, n_v, false, D, B, Hq, Hkv);
+  if (r.k_tiles) r.k_plan = tiles_plan(k_segs, n_k, true, B * Hkv, Hq / Hkv);
+  if (r.v_tiles) r.v_plan = tiles_plan(v_segs, n_v, false, B * Hkv, Hq / Hkv);
+  // The softmax can ride inside the two GEMV launches when nothing is added to the logits and every
+  // position is produced by exactly one K token and consumed by exactly one V token.
+  r.covers = (flags & HQEKV_FUSE_SOFTMAX) && !mask && seg_total_tokens(k_segs, n_k) == Tall && seg_total_tokens(v_segs, n_v) == Tall;
+  // In one launch with p.V, its output and the epilogue are written beside its reads: an output over what V's segments read
+  // takes three launches, an epilogue that writes there a launch of its own.
+  r.in_two = L.logits_bytes > 0 && r.covers && r.k_tiles && r.k_plan.per_unit == 1 && r.v_tiles &&
+             !(flags & (HQEKV_ONLY_QK | HQEKV_ONLY_PV | HQEKV_ONLY_COMBINE | HQEKV_ONLY_RAW_QK)) && pv_last_takes(ep, Tall) &&
+             !pv_reads(v_segs, n_v, B * Hkv, D, {(uintptr_t)attn_out, B * Hq * D * 2, 1, 0});
+  r.rides = r.in_two && !epilogue_writes_v(ep, v_segs, n_v, D);
+  return r;
+}
+
 static int decode_impl(const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_segs, int n_v,
                        const void *q, const void *mask, int64_t mask_row_stride, void *attn_weights,
                        void *attn_out, int64_t B, int64_t Hq, int64_t Hkv, int64_t D, int64_t Tall,
@@ -2344,44 +2422,37 @@ static int decode_impl(const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_segs
   int tiling = 0;
   rc = resolve_qk_tiling(qk_tiling_of(flags), k_segs, n_k, B * Hkv, D, "decode_attn", &tiling);
   if (rc) return rc;
-  // The launches of decode_qk.hip and decode_pv.hip take the call unless it names a form of the older ones.
-  const bool by_rule = !(flags & (HQEKV_QK_TILING(0xf) | HQEKV_DOT_MFMA | HQEKV_DOT_VALU | HQEKV_TWO_STEP_DEQUANT | HQEKV_FOLD_COMBINE |
-                                 HQEKV_SEPARATE_COMBINE));
-  const bool k_tiles = by_rule && n_k > 0 && tiles_fit(k_segs, n_k, true, D, B, Hq, Hkv);
-  const bool v_tiles = by_rule && n_v > 0 && tiles_fit(v_segs, n_v, false, D, B, Hq, Hkv);
-  TilesPlan k_plan{}, v_plan{};
-  if (k_tiles) k_plan = tiles_plan(k_segs, n_k, true, B * Hkv, Hq / Hkv);
-  if (v_tiles) v_plan = tiles_plan(v_segs, n_v, false, B * Hkv, Hq / Hkv);
   const int only = flags & (HQEKV_ONLY_QK | HQEKV_ONLY_PV | HQEKV_ONLY_COMBINE);
-  // The softmax can ride inside the two GEMV launches when nothing is added to the logits and every
-  // position is produced by exactly one K token and consumed by exactly one V token.
-  const bool covers = (flags & HQEKV_FUSE_SOFTMAX) && !mask && seg_total_tokens(k_segs, n_k) == Tall && seg_total_tokens(v_segs, n_v) == Tall;
   StepEpilogue ep;
   rc = fill_epilogue(extra, attn_weights, B, Hq, Hkv, D, Tall, &ep);
   if (rc) return rc;
-  // A short step in two launches: q.K^T leaves its logits in the workspace, p.V does the rest.
-  const bool in_two = L.logits_bytes > 0 && covers && k_tiles && k_plan.per_unit == 1 && v_tiles && !only && !(flags & HQEKV_ONLY_RAW_QK) && pv_last_takes(ep, Tall);
+  const DecodeRoute r = decode_route(L, k_segs, n_k, v_segs, n_v, mask != nullptr, attn_out, B, Hq, Hkv, D, Tall, flags, ep);
   SegTable kt{}, vt{};
-  rc = build_table(k_segs, n_k, true, D, qk_tile_of(tiling), Tall, &kt, "decode_attn(K)", k_tiles ? &k_plan : nullptr);
+  rc = build_table(k_segs, n_k, true, D, qk_tile_of(tiling), Tall, &kt, "decode_attn(K)", r.k_tiles ? &r.k_plan : nullptr);
   if (rc) return rc;
-  rc = build_table(v_segs, n_v, false, D, L.chunk, Tall, &vt, "decode_attn(V)", v_tiles ? &v_plan : nullptr);
+  rc = build_table(v_segs, n_v, false, D, L.chunk, Tall, &vt, "decode_attn(V)", r.v_tiles ? &r.v_plan : nullptr);
   if (rc) return rc;
   hipStream_t st = (hipStream_t)stream;
   char *ws = (char *)workspace;
-  const bool fuse = covers && kt.total_units > 0 && vt.total_units > 0;
+  const bool fuse = r.covers && kt.total_units > 0 && vt.total_units > 0;
   FuseArgs fz{};
   if (fuse) {
     fz.stats = (float2 *)(ws + L.stats_off);
     fz.n_stat = (int32_t)kt.total_units;
     fz.inv_sqrt_d = 1.0f / (float)sqrt((double)D);
   }
-  if (in_two) {
+  if (r.in_two) {
     half_t *logits = (half_t *)(ws + L.logits_off);
     fz.arrive = (uint32_t *)(ws + L.arrive_off);
     fz.out = (half_t *)attn_out;
-    ep.weights = logits;   // (the ring row's workgroups make the probabilities themselves)
+    StepEpilogue riding{};
+    if (r.rides) {
+      riding = ep;
+      riding.weights = logits;   // (the ring row's workgroups make the probabilities themselves)
+    }
     rc = launch_qk(kt, q, logits, B, Hq, Hkv, D, Tall, fz, st, tiling, false);
-    return rc ? rc : launch_pv_last(vt, logits, attn_weights, (float *)ws, B, Hq, Hkv, Tall, fz, ep, st);
+    if (!rc) rc = launch_pv_last(vt, logits, attn_weights, (float *)ws, B, Hq, Hkv, Tall, fz, riding, st);
+    return rc || r.rides || !has_epilogue(ep) ? rc : launch_combine(nullptr, nullptr, 0, B * Hq, D, Tall, false, &ep, st);
   }
   // Few chunks per (b, kv head) and a long p.V launch: the last p.V workgroup of each (b, kv head) adds the
   // partials up and the combine launch is dropped.  The write-through stores, the counter and the final loads
@@ -2391,7 +2462,7 @@ static int decode_impl(const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_segs
   const bool fold_pays = seg_total_tokens(v_segs, n_v) * B * Hkv >= CB_FOLD_MIN_TOKEN_ROWS;
   const bool fold_forced = (flags & HQEKV_FOLD_COMBINE) != 0;
   // (more than eight heads per KV head run as several p.V launches against the one counter: they keep the combine launch)
-  if (kt.total_units > 0 && vt.total_units > 0 && !v_tiles && !k_tiles && vt.total_units <= CB_FOLD_MAX && !(flags & HQEKV_SEPARATE_COMBINE) &&
+  if (kt.total_units > 0 && vt.total_units > 0 && !r.v_tiles && !r.k_tiles && vt.total_units <= CB_FOLD_MAX && !(flags & HQEKV_SEPARATE_COMBINE) &&
       (fold_pays || fold_forced) && one_slice(Hq / Hkv)) {
     fz.arrive = (uint32_t *)(ws + L.arrive_off);
     fz.out = (half_t *)attn_out;
@@ -2418,6 +2489,19 @@ static int decode_impl(const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_segs
   if (only_qk) return HQEKV_OK;
   const int stages = only == HQEKV_ONLY_PV ? 1 : (only == HQEKV_ONLY_COMBINE ? 2 : 3);
   return launch_pv(vt, L.chunk, attn_weights, attn_out, (float *)ws, B, Hq, Hkv, D, Tall, fz, st, mf, stages, &ep);
+}
+
+extern "C" int hqekv_selftest_step_form(const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_segs, int n_v, const void *attn_out, int64_t B,
+                                        int64_t Hq, int64_t Hkv, int64_t D, int64_t Tall, int flags, const hqekv_step_extra *extra) {
+  DecodeLayout L;
+  StepEpilogue ep;
+  int rc = check_heads("selftest_step_form", B, Hq, Hkv, D);
+  if (rc) return rc;
+  if (decode_layout(k_segs, n_k, v_segs, n_v, B, Hq, Hkv, D, &L)) return fail(HQEKV_E_ARG, "selftest_step_form: bad segment tables");
+  rc = fill_epilogue(extra, nullptr, B, Hq, Hkv, D, Tall, &ep);
+  if (rc) return rc;
+  const DecodeRoute r = decode_route(L, k_segs, n_k, v_segs, n_v, false, attn_out, B, Hq, Hkv, D, Tall, flags, ep);
+  return !r.in_two ? 0 : r.rides || !has_epilogue(ep) ? 1 : 2;
 }
 
 // ------------------------------------------------------------------ per-class GEMV on the same kernels

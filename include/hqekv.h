@@ -304,7 +304,9 @@ int hqekv_decode_attn(const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_segs,
  * head rows to for the shape at hand -- 2 when Tall is a multiple of 4, at least 256, and attn_weights is 8-byte
  * aligned; else 1 -- pinned against torch.sum on the device for 32 heads and batch sizes 1..8.
  * The appended rows are not read by this call's attention: the caller names this step's key and value as segments of
- * their own.  `extra` may be NULL (then the call is hqekv_decode_attn); single-stage flags are refused.
+ * their own.  They are written after its segments have been read, so that they may replace rows of those (a sliding window's
+ * oldest); where that would not be so in p.V's launch, they get a launch of their own.  So is ring_line.
+ * `extra` may be NULL (then the call is hqekv_decode_attn); single-stage flags are refused.
  */
 typedef struct hqekv_step_extra {
   void *ring_line;             /* (Tall) fp16, any 2-byte alignment; NULL = no ring row                    */
@@ -329,6 +331,11 @@ int hqekv_decode_step(const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_segs,
                       void *attn_weights, void *attn_out, int64_t B, int64_t Hq, int64_t Hkv,
                       int64_t D, int64_t Tall, void *workspace, int64_t workspace_bytes, int flags,
                       void *stream, const hqekv_step_extra *extra);
+/* No counterpart in the reference: which launches that call (extra NULL: hqekv_decode_attn, without a mask) takes, for tests
+ * of the rule.  0: three or more; 1: two, what `extra` asks for in the second; 2: two and one for what `extra` asks for.
+ * Pointers are compared, never followed. */
+int hqekv_selftest_step_form(const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_segs, int n_v, const void *attn_out, int64_t B,
+                             int64_t Hq, int64_t Hkv, int64_t D, int64_t Tall, int flags, const hqekv_step_extra *extra);
 /* The ring row alone: line[t] = rnd16(sum_h rnd16(sum_b attn_weights[b,h,t])) in torch's order (`order` as
  * ring_order above).  Replaces last_attn_weights.update for one decode row (model/public_func.py:250-254). */
 int hqekv_ring_row(const void *attn_weights, int64_t B, int64_t Hq, int64_t Tall, void *line, int order,

@@ -1,0 +1,112 @@
+"""Which launches a decode step takes (``hqekv_selftest_step_form``): what a step writes beside its attention rides in a short
+step's p.V launch unless that launch reads the place it goes to -- then it gets a launch of its own, behind the reads."""
+import ctypes
+import random
+
+import pytest
+import torch
+
+D = 128
+
+
+def _rows(at, n, slab, slabs, row):
+    """Addresses of the 16-byte pieces of n rows in each of `slabs` slabs."""
+    return {at + s * slab * row + i for s in range(slabs) for i in range(0, n * row, 16)}
+
+
+def _form(v, slabs, extra=None, out=1 << 40):
+    """A step over ``v`` = [(address, tokens, slab, bits, idx address)], K covering as many positions elsewhere."""
+    from hqekv_amd import _lib
+    n = sum(e[1] for e in v)
+    vs = (_lib.Seg * len(v))(*(_lib.Seg(bits=b, n_tokens=t, data=at, scale=None if b == 16 else at + (1 << 20), zero=None if b == 16 else at + (1 << 21),
+                                        idx=idx, slab_tokens=slab) for at, t, slab, b, idx in v))
+    ks = (_lib.Seg * 1)(_lib.Seg(bits=16, layout=_lib.LAYOUT_TOKEN_MAJOR, n_tokens=n, data=1 << 42))
+    rc = _lib.load().hqekv_selftest_step_form(ks, 1, vs, len(v), ctypes.c_void_p(out), 1, 4 * slabs, slabs, D, n, _lib.FUSE_SOFTMAX,
+                                              None if extra is None else ctypes.byref(extra))
+    assert rc >= 0, _lib.load().hqekv_last_error()
+    return rc
+
+
+def _append(k_dst, v_dst, slab_k, slab_v, rows=1, **more):
+    from hqekv_amd import _lib
+    return _lib.StepExtra(append_rows=rows, new_k=1 << 43, new_v=1 << 44, k_dst=k_dst, v_dst=v_dst, k_dst_slab_tokens=slab_k, v_dst_slab_tokens=slab_v, **more)
+
+
+def test_appends_over_rows_that_the_step_reads():
+    """Rows at random places in and around a V segment, against sets of addresses."""
+    rng, seen, base = random.Random(1), {1: 0, 2: 0}, 1 << 30
+    for _ in range(4000):
+        slabs, slab, rows = rng.randint(1, 4), rng.randint(1, 9), rng.randint(1, 3)
+        n = rng.randint(1, slab)
+        dst_slab = slab if rng.random() < .7 else max(rows, rng.randint(1, 9))
+        if dst_slab < rows:
+            continue
+        dst = base + 16 * rng.randint(-16 * slab * slabs - 20, 16 * slab * slabs + 20)
+        hit = bool(_rows(base, n, slab, slabs, 256) & _rows(dst, rows, dst_slab, slabs, 256))
+        k_side = rng.random() < .3
+        form = _form([(base, n, slab, 16, None)], slabs, _append(dst if k_side else 1 << 45, 1 << 45 if k_side else dst, dst_slab if k_side else 64,
+                                                                 64 if k_side else dst_slab, rows))
+        seen[form] += 1
+        assert form == 2 if hit else form == 1 or (dst_slab != slab and slabs > 1)
+    assert min(seen.values()) > 500
+
+
+@pytest.mark.parametrize("bits", [8, 4, 2, 1])
+def test_what_a_class_is_read_from(bits):
+    """Codes, scales, zero points and positions of a class, the row that leaves a tail, the ring's row, the output."""
+    from hqekv_amd import _lib
+    base, slabs, slab, n, idx = 1 << 30, 2, 96, 64, 1 << 35
+    v = [(base, n, slab, bits, idx)]
+    row, params = 16 * bits, 8
+    places = [(base, row), (base + (1 << 20), params), (base + (1 << 21), params)]
+    for at, r in places:
+        last = at + slab * r + n * r   # one past the last slab's rows
+        assert _form(v, slabs, _lib.StepExtra(ring_line=last, ring_order=1)) == 1
+        assert _form(v, slabs, _lib.StepExtra(ring_line=last - 2, ring_order=1)) == 2
+    assert _form(v, slabs, _lib.StepExtra(ring_line=idx + 8 * n - 2, ring_order=1)) == 2
+    assert _form(v, slabs, _lib.StepExtra(ring_line=idx + 8 * n, ring_order=1)) == 1
+    for t in (n - 1, n):
+        leave = dict(leave_bits=bits, leave_src=1 << 46, leave_slab_tokens=4, leave_code=base + t * row, leave_scale=base + (1 << 20) + t * params,
+                     leave_zero=base + (1 << 21) + t * params, leave_dst_slab_tokens=slab)
+        assert _form(v, slabs, _lib.StepExtra(**leave)) == (1 if t == n else 2)
+        assert _form(v, slabs, _append(1 << 45, 1 << 47, 64, 64, **leave)) == (1 if t == n else 2)
+    assert _form(v, slabs) == 1 and _form(v, slabs, out=base + slab * row) == 0 and _form(v, slabs, out=base + (slab + n) * row) == 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,Hkv,n", [(1, 8, 64), (2, 2, 63), (3, 8, 1000)])
+def test_sliding_window_replaces_its_oldest_row(dev, B, Hkv, n):
+    """The step's value goes where the window's oldest was, which this step still reads: bit for bit what a step does that
+    puts it elsewhere, and replays of it."""
+    from hqekv_amd import _lib
+    lib, Hq = _lib.load(), 4 * Hkv
+    g = torch.Generator(device=dev).manual_seed(n)
+    q, k, v = (torch.randn(B, h, 1, D, generator=g, device=dev, dtype=torch.float16) for h in (Hq, Hkv, Hkv))
+    kw, vw = (torch.randn(B, Hkv, n, D, generator=g, device=dev, dtype=torch.float16) for _ in range(2))
+
+    def segs(window, new, layout):
+        return (_lib.Seg * 2)(_lib.Seg(bits=16, layout=layout, n_tokens=n, pos_base=0, data=window.data_ptr(), slab_tokens=n),
+                              _lib.Seg(bits=16, layout=layout, n_tokens=1, pos_base=n, data=new.data_ptr(), slab_tokens=1))
+
+    def step(window, dst, slab):
+        ks, vs = segs(kw, k, _lib.LAYOUT_TOKEN_MAJOR), segs(window, v, 0)
+        spare = torch.empty(B, Hkv, 1, D, dtype=torch.float16, device=dev)
+        w, o = torch.empty(B, Hq, 1, n + 1, dtype=torch.float16, device=dev), torch.empty(B, Hq, 1, D, dtype=torch.float16, device=dev)
+        ws = torch.empty(lib.hqekv_decode_workspace_bytes(ks, 2, vs, 2, B, Hq, Hkv, D), dtype=torch.uint8, device=dev)
+        x = _lib.StepExtra(append_rows=1, new_k=k.data_ptr(), new_v=v.data_ptr(), k_dst=spare.data_ptr(), v_dst=dst.data_ptr(), k_dst_slab_tokens=1,
+                           v_dst_slab_tokens=slab)
+        form = lib.hqekv_selftest_step_form(ks, 2, vs, 2, o.data_ptr(), B, Hq, Hkv, D, n + 1, _lib.FUSE_SOFTMAX, ctypes.byref(x))
+        rc = lib.hqekv_decode_step(ks, 2, vs, 2, q.data_ptr(), None, 0, w.data_ptr(), o.data_ptr(), B, Hq, Hkv, D, n + 1, ws.data_ptr(), ws.numel(),
+                                   _lib.FUSE_SOFTMAX, torch.cuda.current_stream().cuda_stream, ctypes.byref(x))
+        assert rc == 0, lib.hqekv_last_error()
+        assert torch.equal(spare, k)
+        return form, w, o
+
+    elsewhere = torch.empty_like(v)
+    form, w0, o0 = step(vw, elsewhere, 1)
+    assert form == 1 and torch.equal(elsewhere, v)
+    for _ in range(4):
+        window = vw.clone()
+        form, w, o = step(window, window, n)
+        assert form == 2 and torch.equal(w, w0) and torch.equal(o, o0)
+        assert torch.equal(window[:, :, :1], v) and torch.equal(window[:, :, 1:], vw[:, :, 1:])
