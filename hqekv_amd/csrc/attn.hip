@@ -2397,11 +2397,12 @@ static DecodeRoute decode_route(const DecodeLayout &L, const hqekv_seg *k_segs, 
   // position is produced by exactly one K token and consumed by exactly one V token.
   r.covers = (flags & HQEKV_FUSE_SOFTMAX) && !mask && seg_total_tokens(k_segs, n_k) == Tall && seg_total_tokens(v_segs, n_v) == Tall;
   // In one launch with p.V, its output and the epilogue are written beside its reads: an output over what V's segments read
-  // takes three launches, an epilogue that writes there a launch of its own.
+  // takes three launches, an epilogue that writes there, or whose ring row p.V's workgroups do not cover, a launch of its own.
+  // (What rides along changes nothing about the attention, so that a step and the separate calls give the same bits.)
   r.in_two = L.logits_bytes > 0 && r.covers && r.k_tiles && r.k_plan.per_unit == 1 && r.v_tiles &&
-             !(flags & (HQEKV_ONLY_QK | HQEKV_ONLY_PV | HQEKV_ONLY_COMBINE | HQEKV_ONLY_RAW_QK)) && pv_last_takes(ep, Tall) &&
+             !(flags & (HQEKV_ONLY_QK | HQEKV_ONLY_PV | HQEKV_ONLY_COMBINE | HQEKV_ONLY_RAW_QK)) &&
              !pv_reads(v_segs, n_v, B * Hkv, D, {(uintptr_t)attn_out, B * Hq * D * 2, 1, 0});
-  r.rides = r.in_two && !epilogue_writes_v(ep, v_segs, n_v, D);
+  r.rides = r.in_two && pv_last_takes(ep, Tall) && !epilogue_writes_v(ep, v_segs, n_v, D);
   return r;
 }
 

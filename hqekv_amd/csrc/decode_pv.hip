@@ -532,7 +532,7 @@ int launch_pv_tiles(const SegTable &tb, void *p, float *partial, int64_t B, int6
 // start at about 20 rows; the host saves 2.5 us at any size.  A step of the fp16 / 8 / 4 / 2-bit mix, B = 1, device time in
 // us, three launches / two: 1k tokens 11.1 / 10.3, 2k 11.0 / 10.4, 4k (18 rows) 12.1 / 11.6, 5k 12.2 / 12.1, 6k (25 rows)
 // 12.6 / 13.0, 8k 13.3 / 14.5; 4 x 2k 13.6 / 12.7, 4 x 4k 15.9 / 15.5, 16 x 2k 21.4 / 20.5, 8 x 4k 20.8 / 20.9; five heads per
-// KV head, 4 x 2k 14.7 / 13.0.  With and without an epilogue alike, so that a step and the separate calls give the same bits.
+// KV head, 4 x 2k 14.7 / 13.0.
 constexpr int64_t PT_LAST_UNITS = 20;
 bool decode_in_two(const hqekv_seg *v_segs, int n_v, int64_t D, int64_t B, int64_t Hq, int64_t Hkv) {
   if (n_v <= 0 || !tiles_fit(v_segs, n_v, false, D, B, Hq, Hkv) || Hq / Hkv > 8) return false;

@@ -110,3 +110,47 @@ def test_sliding_window_replaces_its_oldest_row(dev, B, Hkv, n):
         form, w, o = step(window, window, n)
         assert form == 2 and torch.equal(w, w0) and torch.equal(o, o0)
         assert torch.equal(window[:, :, :1], v) and torch.equal(window[:, :, 1:], vw[:, :, 1:])
+
+
+RING = [(1, 8, 8, 300), (8, 32, 8, 300), (9, 32, 8, 300), (8, 40, 8, 300), (2, 72, 9, 200), (1, 4, 1, 3)]   # the last four past what p.V's workgroups cover
+
+
+def _ring_step(B, Hq, Hkv, n, line, segs):
+    from hqekv_amd import _lib
+    x = _lib.StepExtra(ring_line=line, ring_order=1)
+    return x, _lib.load().hqekv_selftest_step_form(segs[0], 1, segs[1], 1, ctypes.c_void_p(1 << 40), B, Hq, Hkv, D, n, _lib.FUSE_SOFTMAX, ctypes.byref(x))
+
+
+def _dense(n, k, v):
+    from hqekv_amd import _lib
+    return ((_lib.Seg * 1)(_lib.Seg(bits=16, layout=_lib.LAYOUT_TOKEN_MAJOR, n_tokens=n, data=k)), (_lib.Seg * 1)(_lib.Seg(bits=16, n_tokens=n, data=v)))
+
+
+def test_ring_rows_past_what_rides():
+    for i, (B, Hq, Hkv, n) in enumerate(RING):
+        assert _ring_step(B, Hq, Hkv, n, 1 << 36, _dense(n, 1 << 42, 1 << 43))[1] == (1 if i < 2 else 2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,Hq,Hkv,n", RING)
+def test_a_step_and_the_separate_calls(dev, B, Hq, Hkv, n):
+    """Bit for bit: probabilities and output with a ring row beside them and without, the ring row of the one call and of its own."""
+    from hqekv_amd import _lib
+    lib, st = _lib.load(), torch.cuda.current_stream().cuda_stream
+    g = torch.Generator(device=dev).manual_seed(n + B)
+    q, k, v = (torch.randn(B, h, t, D, generator=g, device=dev, dtype=torch.float16) for h, t in ((Hq, 1), (Hkv, n), (Hkv, n)))
+    segs = _dense(n, k.data_ptr(), v.data_ptr())
+    ws = torch.empty(lib.hqekv_decode_workspace_bytes(segs[0], 1, segs[1], 1, B, Hq, Hkv, D), dtype=torch.uint8, device=dev)
+    lines = torch.full((2, n + 2), float("nan"), dtype=torch.float16, device=dev)
+    got = []
+    for step in (True, False):
+        w, o = torch.empty(B, Hq, n, dtype=torch.float16, device=dev), torch.empty(B, Hq, D, dtype=torch.float16, device=dev)
+        x, form = _ring_step(B, Hq, Hkv, n, lines.data_ptr(), segs)
+        assert form > 0
+        rc = lib.hqekv_decode_step(segs[0], 1, segs[1], 1, q.data_ptr(), None, 0, w.data_ptr(), o.data_ptr(), B, Hq, Hkv, D, n, ws.data_ptr(), ws.numel(),
+                                   _lib.FUSE_SOFTMAX, st, ctypes.byref(x) if step else None)
+        assert rc == 0, lib.hqekv_last_error()
+        got.append((w, o))
+    assert lib.hqekv_ring_row(got[1][0].data_ptr(), B, Hq, n, lines[1].data_ptr(), 1, st) == 0
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    assert torch.equal(lines[0, :n], lines[1, :n]) and bool(lines[:, n:].isnan().all()) and bool(lines[:, :n].isfinite().all())
