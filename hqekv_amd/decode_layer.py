@@ -175,10 +175,23 @@ class HqeAttentionLayer:
         the ring keeps).  K and V are read once per KV head, without ``repeat_kv`` copies.  -> (the probabilities, a
         callable that queues the attention): the prompt's compression needs the probabilities alone, so ``forward``
         queues the attention behind the ranking and the host plans while the device is at it (a prompt of 4099 tokens and 24
-        steps: 615 -> 531 us, 8192: 1060 -> 980)."""
+        steps: 615 -> 531 us, 8192: 1060 -> 980).  An attention that fails leaves the ring as it was before the prompt: one
+        that holds rows already, which the prompt's would replace, is written after it."""
+        lw = self.last_weights
         rows = min(q.shape[2], LAST_TOKEN_NUM)
-        attn_weights = last_rows_probabilities(q, k, attention_mask, self.scaling, rows)
-        return attn_weights, lambda: gqa_prompt_attention(q, k, v, attention_mask, self.scaling)
+        if lw.weights is not None:
+            out = gqa_prompt_attention(q, k, v, attention_mask, self.scaling)
+            return last_rows_probabilities(q, k, attention_mask, self.scaling, rows), lambda: out
+        before = lw.kv_seq_len, lw.next_line
+
+        def attention():
+            try:
+                return gqa_prompt_attention(q, k, v, attention_mask, self.scaling)
+            except BaseException:
+                lw.weights, lw.kv_seq_len, lw.next_line = None, *before
+                raise
+
+        return last_rows_probabilities(q, k, attention_mask, self.scaling, rows), attention
 
     # ------------------------------------------------------------------ residual storage
     @staticmethod
