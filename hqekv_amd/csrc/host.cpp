@@ -16,6 +16,7 @@
 
 #include <chrono>
 #include <initializer_list>
+#include <thread>
 #include <vector>
 
 #include <ATen/core/Tensor.h>
@@ -1026,10 +1027,12 @@ bool new_tokens(const Tensor &t, bool is_k, int64_t B, int64_t H, int64_t n, int
 }
 
 // Both block rankings, written by one launch into page-locked memory.  Every entry is stored exactly once, so the ranking
-// is there as soon as no entry holds its initial value: that is watched for a while (a stream synchronisation wakes up
-// some ten microseconds later), then the stream is waited for.  meanwhile: None, or what the caller has to queue that does
-// not need the ranking -- the kernels run it while the host reads the ranking and plans; called once, behind the launch.  (The
-// memory may not be let go before the kernel has written it: what the call raises is raised after the wait.)
+// is there as soon as no entry holds its initial value: that is watched, closely at first (a stream synchronisation wakes up
+// some ten microseconds later), then, where a model's work is queued ahead, every 20 us until the stream has nothing left to do.
+// The stream is not waited for: what is queued behind the ranking would be waited for as well.  meanwhile: None, or what the
+// caller has to queue that does not need the ranking -- the kernels run it while the host reads the ranking and plans; called
+// once, behind the launch.  (The memory may not be let go before the kernel has written it: what the call raises is raised
+// after the wait.)
 bool host_orders(const void *const (&scores)[2], int64_t n, const Tensor &order, const at::Device &dev, PyObject *meanwhile) {
   volatile int32_t *p = (volatile int32_t *)order.data_ptr();
   for (int64_t i = 0; i < 2 * n; ++i) p[i] = -1;
@@ -1041,8 +1044,11 @@ bool host_orders(const void *const (&scores)[2], int64_t n, const Tensor &order,
       if (p[i] >= 0) {
         ++i;
       } else if (std::chrono::steady_clock::now() > until) {
-        err = hipStreamSynchronize((hipStream_t)stream_of(dev));
-        break;
+        err = hipStreamQuery((hipStream_t)stream_of(dev));
+        if (err != hipErrorNotReady) break;
+        err = hipSuccess;
+        (void)hipGetLastError();   // (an answer, not an error for the next launch to find)
+        std::this_thread::sleep_for(std::chrono::microseconds(20));
       }
     }
     return HQEKV_OK;
