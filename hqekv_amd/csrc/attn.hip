@@ -2004,6 +2004,10 @@ static int64_t seg_total_tokens(const hqekv_seg *segs, int nseg) {
   return n;
 }
 
+// A workgroup per row, four where rows are few and long (device time of a step, one / four / the 16-wave form, us: 32 rows
+// of 33 chunks 13.1 / 13.5 / 13.5, of 52 16.4 / 15.7 / 15.9, of 103 21.8 / 20.7 / 20.9; 120 rows of 56 27.0 / - / 28.2).
+int rows_sum_lanes(int64_t n_rows, int64_t n_chunks) { return n_rows >= 96 || n_chunks <= 40 ? 32 : 8; }
+
 static bool has_epilogue(const StepEpilogue &e) { return e.ring_line || e.app_rows > 0 || e.leave_bits; }
 // The epilogue rides in the combine launch as extra workgroups: as many layers of grid.z (B * Hq * D / 32 workgroups each)
 // as make one workgroup per RING_SPAN columns of the ring row at the least.  Without a combine (the partial rows added by p.V)
@@ -2063,13 +2067,10 @@ static int launch_pv(const SegTable &tb, int64_t chunk, void *p, void *out, floa
   const bool epilogue = ep && has_epilogue(*ep) && stages == 3;
   if (!combine && !epilogue) return HQEKV_OK;
   if (tb.per_unit && !epilogue) {
-    // A workgroup per row, four where rows are few and long (device time of a step, one / four / the 16-wave form, us: 32 rows
-    // of 33 chunks 13.1 / 13.5 / 13.5, of 52 16.4 / 15.7 / 15.9, of 103 21.8 / 20.7 / 20.9; 120 rows of 56 27.0 / - / 28.2).
-    const bool one = n_bhq >= 96 || tb.total_units <= 40;
 #define LAUNCH(LANES_)                                                                                                                        \
   hipLaunchKernelGGL((pv_rows_sum_kernel<LANES_>), dim3((unsigned)n_bhq, 32 / LANES_), dim3(RS_THREADS), 0, st, partial, (half_t *)out, \
                      (int)tb.total_units, (uint32_t)n_bhq)
-    if (one) LAUNCH(32);
+    if (rows_sum_lanes(n_bhq, tb.total_units) == 32) LAUNCH(32);
     else LAUNCH(8);
 #undef LAUNCH
     return check_launch("pv_rows_sum_kernel");
@@ -2210,7 +2211,10 @@ static int decode_layout(const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_se
   L->chunks = chunks;
   L->logits_off = L->arrive_off + align_up(B * Hkv * (int64_t)sizeof(uint32_t), 256);
   L->logits_bytes = decode_in_two(v_segs, n_v, D, B, Hq, Hkv) ? align_up(B * Hq * seg_total_tokens(v_segs, n_v) * (int64_t)sizeof(half_t), 256) : 0;
-  if (L->logits_off + L->logits_bytes > (int64_t)HQEKV_STATIC_SCRATCH_BYTES) L->logits_bytes = 0;   // (what fits the static entry's scratch without them still does)
+  // Without them where the fixed scratch of hqekv_decode_attn_static would not hold them, through either entry: what fitted there
+  // still does, and the two entries give the same bits.  (A short step has at most 1536 workgroups, so that only seven and
+  // eight heads per KV head get there: 9 x 4k tokens at eight 27.3 us in three launches, 25.7 in two; 34 x 1184 46.9 either way.)
+  if (L->logits_off + L->logits_bytes > (int64_t)HQEKV_STATIC_SCRATCH_BYTES) L->logits_bytes = 0;
   L->total = L->logits_off + L->logits_bytes;
   return HQEKV_OK;
 }

@@ -25,5 +25,16 @@ int check_launch(const char *what) {
 
 }  // namespace hq
 
+extern "C" int hqekv_selftest_form(int what, int64_t a, int64_t b, int64_t c) {
+  const hq::PromptForm p = hq::prompt_form(a, b);
+  switch (what) {
+    case 0: return 10 * p.key_shares + p.tiles + (p.reversed ? 100 : 0);
+    case 1: return hq::quant_rows_form(a);
+    case 2: return hq::quant_k_staged(a, b, (int)c) ? 1 : 0;
+    case 3: return hq::rows_sum_lanes(a, b);
+    default: return hq::fail(HQEKV_E_ARG, "selftest_form: what=%d", what);
+  }
+}
+
 extern "C" int hqekv_version(void) { return 1; }
 extern "C" const char *hqekv_last_error(void) { return hq::g_err; }

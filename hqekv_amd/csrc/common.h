@@ -17,6 +17,13 @@ namespace hq {
 int fail(int code, const char *fmt, ...);
 int check_launch(const char *what);
 
+// Which variant of a kernel a call of these sizes takes (the rules stand beside the launches; hqekv_selftest_form).
+struct PromptForm { int key_shares, tiles; bool reversed; };   // PaShape's
+PromptForm prompt_form(int64_t T, int64_t BH);
+int quant_rows_form(int64_t n_groups);                             // groups per quad of lanes
+bool quant_k_staged(int64_t n_groups, int64_t n_outer, int bits);   // K through LDS
+int rows_sum_lanes(int64_t n_rows, int64_t n_chunks);               // lanes across a row of the partial sums' 32
+
 __device__ __forceinline__ float h2f(half_t h) { return (float)h; }
 __device__ __forceinline__ half_t f2h(float f) { return (half_t)f; }
 

@@ -622,10 +622,17 @@ static bool rows_16_byte_aligned(const void *p, int64_t s0, int64_t s1, int64_t 
 // 52.6.  Up to 1500 64 keys per step: 512 (2048) 53.2 against 60.5 of <1, 1>, 672 (28 heads over 4, 3000) 84.5 / 93.1, 1056
 // (4099) 165.9 / 171, 1376 (5500) 274 / 288; beyond it is behind: 2048 (8192) 580 / 573, 4128 (16384) 2218 / 2163.
 // Four waves per row group never won (T = 500: 20.0 against 12.6 us).
-static int prompt_form(int64_t T, int64_t BH) {
+// The opposite order of the second 256 workgroups: of the 64-key form always, us without / with it: 416 workgroups (T = 1632)
+// 41.2 / 40.5, 512 53.2 / 52.2, 768 (3000) 94.5 / 92.9, 1056 (4099) 166.7 / 161.9, 1376 (5500) 265.8 / 265.6.  Walks of half the
+// length gain from it past two and a half rounds only: 320 workgroups (T = 478, 40 heads) 13.6 / 14.0, 608 (1200) 27.3 / 27.6, 728
+// (777, B = 2, 28 heads) 26.4 / 25.5, 768 (1500) 36.7 / 36.3.
+namespace hq {
+PromptForm prompt_form(int64_t T, int64_t BH) {
   const int64_t wgs = (T + 127) / 128 * BH;
-  return wgs <= 400 ? 2 : wgs <= 1500 ? 1 : 0;
+  if (wgs <= 400) return PromptForm{2, 1, (T + 63) / 64 * BH > 640};
+  return wgs <= 1500 ? PromptForm{1, 2, true} : PromptForm{1, 1, false};
 }
+}  // namespace hq
 
 extern "C" int hqekv_prompt_attn(const void *q, const int64_t *q_strides, const void *k, const int64_t *k_strides,
                                  const void *v, const int64_t *v_strides, void *out, const int64_t *out_strides, int64_t B,
@@ -650,17 +657,15 @@ extern "C" int hqekv_prompt_attn(const void *q, const int64_t *q_strides, const 
   a.o_b = out_strides[0]; a.o_h = out_strides[1]; a.o_t = out_strides[2];
   a.Hq = (int32_t)Hq; a.Hkv = (int32_t)Hkv; a.T = (int32_t)T; a.scale = scale;
   a.BH = (int32_t)(B * Hq); a.by_xcd = (B * Hkv) % 8 == 0;
-  const int form = prompt_form(T, B * Hq);
-  const int64_t rows = form == 2 ? 64 : 128, wgs = (T + rows - 1) / rows * B * Hq;
+  const PromptForm form = prompt_form(T, B * Hq);
+  const int64_t rows = form.key_shares == 2 ? 64 : 128, wgs = (T + rows - 1) / rows * B * Hq;
   if (wgs > 0x7fffffffLL) return fail(HQEKV_E_UNSUPPORTED, "prompt_attn: T * B * Hq too large");
-  // Walks of half the length gain from the opposite order only when a third round follows: 728 workgroups (T = 777, B = 2, 28
-  // heads) 26.4 -> 25.5 us, 768 (1500) 36.7 -> 36.3; 320 (478, 40 heads) 13.6 / 14.0, 608 (1200) 27.3 / 27.6.
 #define LAUNCH(C_, KS_, NB_, REV_)                                                                                                                \
   hipLaunchKernelGGL((prompt_attn_kernel<C_, PaShape<KS_, NB_, REV_>>), dim3((unsigned)wgs), dim3(PA_THREADS), 0, (hipStream_t)stream, a)
 #define LAUNCH_K(C_)                    \
-  if (form == 2 && wgs > 640) LAUNCH(C_, 2, 1, true); \
-  else if (form == 2) LAUNCH(C_, 2, 1, false);        \
-  else if (form == 1) LAUNCH(C_, 1, 2, true);         \
+  if (form.key_shares == 2 && form.reversed) LAUNCH(C_, 2, 1, true); \
+  else if (form.key_shares == 2) LAUNCH(C_, 2, 1, false);            \
+  else if (form.tiles == 2) LAUNCH(C_, 1, 2, true);                  \
   else LAUNCH(C_, 1, 1, false)
   if (causal) { LAUNCH_K(true); } else { LAUNCH_K(false); }
 #undef LAUNCH_K

@@ -489,6 +489,17 @@ __global__ __launch_bounds__(256) void pack_i32_kernel(const int32_t *__restrict
   code[wid] = w;
 }
 
+// Four groups per quad of lanes where that leaves two workgroups per CU: V of 8 x 16k tokens at 4 bit 11.6 -> 11.2 us, 32 x
+// 64k 136 -> 126; at 8 x 8k 8.0 either way, below it is behind (8 x 2k 4.6 -> 4.9).
+int quant_rows_form(int64_t n_groups) { return n_groups >= 524288 ? 4 : 1; }
+
+// K through LDS or not, us: 8 x 32 tokens 4.8 / 6.5, 8 x 128 5.1 / 5.3, 8 x 256 at 2 bit 5.9 / 5.5, 8 x 4k 7.1 / 6.2, 8 x 8k at 2, 4
+// and 8 bit 8.5 / 8.0, 8.3 / 8.3, 9.1 / 9.3, 8 x 16k 11.6 / 11.4, 11.6 / 11.9, 12.7 / 13.7, 32 x 64k 131 / 158 and 139 / 175 at 2
+// and 4 bit.
+bool quant_k_staged(int64_t n_groups, int64_t n_outer, int bits) {
+  return n_groups <= 4 || (n_groups + QK_GROUPS_PER_BLOCK - 1) / QK_GROUPS_PER_BLOCK * n_outer * (bits < 2 ? 2 : bits) >= 2048;
+}
+
 static inline bool bits_ok(int bits) { return bits == 1 || bits == 2 || bits == 4 || bits == 8; }
 
 }  // namespace hq
@@ -508,9 +519,7 @@ extern "C" int hqekv_quant_pack_rows(const void *x, int64_t xo, int64_t xr, void
   if (((uintptr_t)x & 15) || (xo % 8) || (xr % 8))
     return fail(HQEKV_E_ALIGN, "quant_pack_rows: x rows must be 16-byte aligned");
   const int64_t gpr = L / 32, gps = n_rows * gpr;
-  // Four groups per quad of lanes where that leaves two workgroups per CU: V of 8 x 16k tokens at 4 bit 11.6 -> 11.2 us, 32 x
-  // 64k 136 -> 126; at 8 x 8k 8.0 either way, below it is behind (8 x 2k 4.6 -> 4.9).
-  const int u = n_groups >= 524288 ? 4 : 1;
+  const int u = quant_rows_form(n_groups);
   const int64_t bps = (gps + 64 * u - 1) / (64 * u);
   if (gps > 0x7fffffffLL || bps * n_outer > 0x7fffffffLL)
     return fail(HQEKV_E_ARG, "quant_pack_rows: too many groups");
@@ -550,10 +559,7 @@ extern "C" int hqekv_quant_pack_k_tokenmajor(const void *x, int64_t xo, int64_t 
   hipStream_t st = (hipStream_t)stream;
   const int64_t bps = (n_groups + QK_GROUPS_PER_BLOCK - 1) / QK_GROUPS_PER_BLOCK;
   dim3 grid((unsigned)(bps * n_outer)), block(512);
-  // Which of the two, us here / there: 8 x 32 tokens 6.5 / 4.8, 8 x 128 5.3 / 5.1, 8 x 256 at 2 bit 5.5 / 5.9, 8 x 4k 6.2 / 7.1, 8 x
-  // 8k at 2, 4 and 8 bit 8.0 / 8.5, 8.3 / 8.3, 9.3 / 9.1, 8 x 16k 11.4 / 11.6, 11.9 / 11.6, 13.7 / 12.7, 32 x 64k 158 / 131 and
-  // 175 / 139 at 2 and 4 bit.
-  const bool staged = n_groups <= 4 || bps * n_outer * (bits < 2 ? 2 : bits) >= 2048;
+  const bool staged = quant_k_staged(n_groups, n_outer, bits);
 #define LAUNCH_K(KERNEL_)                                                                                                          \
   hipLaunchKernelGGL(KERNEL_, grid, block, 0, st, (const half_t *)x, xo, xt, (uint32_t *)code, co, cr, (half_t *)scale, (half_t *)zero, \
                      so, sr, (uint32_t)D, (uint32_t)n_groups, (uint32_t)bps)

@@ -127,6 +127,15 @@ int hqekv_selftest_wave_reduce(const void *in, void *out, int64_t n_waves, void 
  */
 int hqekv_selftest_stream_read(const void *src, int64_t bytes, void *sum, int64_t n_workgroups, void *stream);
 
+/* No counterpart in the reference: which variant of a kernel a call of these sizes takes, for tests of the rules.
+ *   what 0   hqekv_prompt_attn: a = T, b = B * Hq -> 10 * shares of a row's keys + 32-key tiles per step, + 100 where every
+ *            second 256 workgroups come in the opposite order
+ *        1   hqekv_quant_pack_rows: a = groups of 32 values -> groups per quad of lanes
+ *        2   hqekv_quant_pack_k_tokenmajor: a = T / 32, b = n_outer, c = bits -> 1: tokens staged in LDS, else 0
+ *        3   the sum of p.V's partial rows: a = B * Hq, b = partial rows of each -> lanes across a row, 32 or 8
+ */
+int hqekv_selftest_form(int what, int64_t a, int64_t b, int64_t c);
+
 /* Replaces pack_along_last_dim (quant/pack_unpack.py:16-70): q is (n_rows, L) int32 codes,
  * code is (n_rows, L/pf) int32, both contiguous. */
 int hqekv_pack_i32(const void *q, void *code, int64_t n_rows, int64_t L, int bits, void *stream);
@@ -229,8 +238,8 @@ int hqekv_pv_hybrid(const hqekv_seg *segs, int nseg, const void *p, void *out, i
  *   idx arrays and any mask.
  * flags & HQEKV_FUSE_SOFTMAX: no softmax launch.  The q.K^T launch stores scaled logits and per-tile softmax
  *   statistics, the p.V launch normalises while it gathers; the fixed-order combine stays a third,
- *   small launch (short steps: at most 20 partial rows per KV head, no form named by the flags, room in the workspace: it
- *   runs in the p.V launch).  REQUIRES that the idx arrays of the K segments, and those of the V segments, each cover
+ *   small launch (short steps: up to eight query heads per KV head, at most 20 partial rows per KV head, no form named by
+ *   the flags, a workspace of at most HQEKV_STATIC_SCRATCH_BYTES: it runs in the p.V launch).  REQUIRES that the idx arrays of the K segments, and those of the V segments, each cover
  *   every position in [0, Tall) exactly once (true for every cache the reference's cache policy builds);
  *   taken only when mask == NULL and both segment lists hold exactly Tall tokens, otherwise the call
  *   silently runs the flags = 0 path.

@@ -14,8 +14,10 @@ def test_against_the_fp16_chain(dev, T, B, Hq, Hkv, R, masked):
     """Tolerance: three roundings of a logit may fall to the other half -- the product's, 2^-5 below 64 and times the scale 2.8e-3,
     the scaled one's and the masked one's, 2^-8 each below 8 -- and move its probability by as much of itself, and the
     probability's own, 2^-11: 1.1e-2."""
+    from hqekv_amd import _lib
     from hqekv_amd.prompt_attention import prompt_last_rows
     R = min(R, T)
+    assert (_lib.load().hqekv_prompt_last_rows_workspace_bytes(B, Hq, T) == 0) == (T <= 512)   # (the form of one launch needs none)
     g = torch.Generator(device=dev).manual_seed(T * 7 + Hq)
     fused = torch.randn(B, T, (Hq + Hkv) * 128, generator=g, device=dev, dtype=torch.float16)
     q = fused[..., :Hq * 128].view(B, T, Hq, 128).transpose(1, 2)

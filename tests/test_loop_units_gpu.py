@@ -14,9 +14,10 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("n_rep", [5, 8])
-@pytest.mark.parametrize("classes", [{4: 64}, {4: 65}, {2: 33, 8: 17}], ids=["resident", "over", "two"])
-def test_line_between_forms(dev, n_rep, classes):
-    from hqekv_amd.attention import decode_attention
+@pytest.mark.parametrize("classes,rows", [({4: 64}, 8), ({4: 65}, 3), ({2: 33, 8: 17}, 4)], ids=["resident", "over", "two"])
+def test_line_between_forms(dev, n_rep, classes, rows):
+    from hqekv_amd import _lib
+    from hqekv_amd.attention import DecodePlan, decode_attention
     B, Hkv, D, n = 24, 8, 128, 32 * sum(classes.values())
     q, K, V = synth.make_qkv(B, n_rep * Hkv, Hkv, n, D, 9)
     tokens, at = {b: torch.arange(0) for b in (16, 8, 4, 2, 1)}, 0
@@ -25,6 +26,8 @@ def test_line_between_forms(dev, n_rep, classes):
         at += 32 * c
     cache = synth.build_cache(K, V, tokens, 0, O.uniform_group_quantize_pack_last_dim)
     w_ref, o_ref = O.qkv_matmul(q, cache, None, D, use_mask=False, round_per_class=False)
+    plan = DecodePlan(q.to(dev), synth.cache_to(cache, dev))
+    assert _lib.load().hqekv_pv_workspace_bytes(plan.v_segs, plan.n_v, B, n_rep * Hkv, Hkv, D) == rows * B * n_rep * Hkv * 512   # blocks: 8, 9, 5 + 5
     w, o = decode_attention(q.to(dev), synth.cache_to(cache, dev), None, n, zero_init=False, flags=1)
     torch.testing.assert_close(w.float().cpu(), w_ref.float(), rtol=1e-3, atol=2e-3)
     moved = (w.float().cpu() - w_ref.float()).abs().sum(-1, keepdim=True) * V.float().abs().max()

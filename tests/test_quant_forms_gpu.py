@@ -22,6 +22,8 @@ def _window(B, H, D, n, bits, dev, at, room):
     (1, 64, 1024, 128), (1, 64, 992, 128), (1, 256, 512, 128), (3, 85, 512, 128), (1, 1024, 224, 64), (1, 1030, 160, 64)])
 def test_both_ways_to_quantise_k(dev, B, H, n, D, bits):
     from hqekv_amd.pack_unpack import quantize_pack_into, uniform_group_quantize_pack_last_dim
+    from hqekv_amd import _lib
+    assert _lib.load().hqekv_selftest_form(2, n // 32, B * H, bits) == (n <= 128 or -(-n // 256) * B * H * max(bits, 2) >= 2048)
     g = torch.Generator(device=dev).manual_seed(n + D + bits)
     k = torch.randn(B, H, n, D, generator=g, device=dev, dtype=torch.float16)
     k[0, 0, :32] = 0.0
@@ -51,6 +53,8 @@ def test_both_ways_to_quantise_k(dev, B, H, n, D, bits):
 def test_rows_in_parts_equal_the_whole(dev, n, bits):
     """Four groups per quad of lanes from 524288 groups on; fewer in halves of the same tensor."""
     from hqekv_amd.pack_unpack import uniform_group_quantize_pack_last_dim
+    from hqekv_amd import _lib
+    assert [_lib.load().hqekv_selftest_form(1, 4 * t, 0, 0) for t in (n, n // 2 + 1)] == [4 if n >= 131072 else 1, 1]
     v = torch.randn(1, 1, n, 128, generator=torch.Generator(device=dev).manual_seed(n), device=dev, dtype=torch.float16)
     whole = uniform_group_quantize_pack_last_dim(v, 32, bits)
     cut = n // 2 + 1

@@ -20,6 +20,10 @@ def test_exact_sums(dev, B, Hq, Hkv, chunks):
     s = _lib.Seg(bits=16, n_tokens=n, data=v.data_ptr(), scale=None, zero=None, idx=None, pos_base=0, layout=0, slab_tokens=0)
     segs = (_lib.Seg * 1)(s)
     ws = torch.empty(lib.hqekv_pv_workspace_bytes(segs, 1, B, Hq, Hkv, D), dtype=torch.uint8, device=dev)
+    # (past what the chip holds at once -- six workgroups per CU, three above eight heads -- a workgroup takes several chunks)
+    rows = ws.numel() // (B * Hq * 512)
+    assert rows == chunks if B * Hkv * chunks <= (1536 if Hq // Hkv <= 8 else 768) else 1 < rows < chunks
+    assert lib.hqekv_selftest_form(3, B * Hq, rows, 0) == (8 if B * Hq < 96 and rows > 40 else 32)
     out = torch.full((B, Hq, D), float("nan"), dtype=torch.float16, device=dev)
     rc = lib.hqekv_pv_hybrid(segs, 1, ctypes.c_void_p(p.data_ptr()), ctypes.c_void_p(out.data_ptr()), B, Hq, Hkv, D, n,
                              ctypes.c_void_p(ws.data_ptr()), ws.numel(), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))

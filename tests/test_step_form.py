@@ -154,3 +154,15 @@ def test_a_step_and_the_separate_calls(dev, B, Hq, Hkv, n):
     assert lib.hqekv_ring_row(got[1][0].data_ptr(), B, Hq, n, lines[1].data_ptr(), 1, st) == 0
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
     assert torch.equal(lines[0, :n], lines[1, :n]) and bool(lines[:, n:].isnan().all()) and bool(lines[:, :n].isfinite().all())
+
+
+def test_lines_of_the_other_rules():
+    """The calls of the kernels' own tests lie on both sides of every line (those tests ask for the form they take)."""
+    from hqekv_amd import _lib
+    form = _lib.load().hqekv_selftest_form
+    assert [form(0, 128 * w, 1, 0) for w in (1, 320, 321, 400, 401, 1500, 1501)] == [21, 21, 121, 121, 112, 112, 11]
+    assert [form(1, n, 0, 0) for n in (1, 524287, 524288)] == [1, 1, 4]
+    for bits in (1, 2, 4, 8):
+        assert [form(2, g, n, bits) for g, n in ((4, 1), (5, 1), (8, 2047 // max(bits, 2)), (8, 2048 // max(bits, 2)))] == [1, 0, 0, 1]
+    assert [form(3, r, u, 0) for r, u in ((95, 40), (95, 41), (96, 41))] == [32, 8, 32]
+    assert form(9, 1, 1, 1) < 0
