@@ -166,3 +166,45 @@ def test_lines_of_the_other_rules():
         assert [form(2, g, n, bits) for g, n in ((4, 1), (5, 1), (8, 2047 // max(bits, 2)), (8, 2048 // max(bits, 2)))] == [1, 0, 0, 1]
     assert [form(3, r, u, 0) for r, u in ((95, 40), (95, 41), (96, 41))] == [32, 8, 32]
     assert form(9, 1, 1, 1) < 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("window", [False, True])
+def test_replays_of_a_launch_of_its_own(dev, window):
+    """Captured into a graph: a ring row past what rides along, a sliding window's row; eager calls between the replays."""
+    from hqekv_amd import _lib
+    lib, B, Hq, Hkv, n = _lib.load(), 9, 32, 8, 300
+    g = torch.Generator(device=dev).manual_seed(8)
+    q, k, v, new = (torch.randn(B, h, t, D, generator=g, device=dev, dtype=torch.float16) for h, t in ((Hq, 1), (Hkv, n), (Hkv, n), (Hkv, 1)))
+    kept, spare = v.clone(), torch.empty_like(new)
+    segs = _dense(n, k.data_ptr(), v.data_ptr())
+    ws = torch.empty(lib.hqekv_decode_workspace_bytes(segs[0], 1, segs[1], 1, B, Hq, Hkv, D), dtype=torch.uint8, device=dev)
+    line, w, o = (torch.empty(s, dtype=torch.float16, device=dev) for s in ((n,), (B, Hq, n), (B, Hq, D)))
+    x = _append(spare.data_ptr(), v.data_ptr(), 1, n) if window else _lib.StepExtra(ring_line=line.data_ptr(), ring_order=1)
+    if window:
+        x.new_k = x.new_v = new.data_ptr()
+    assert lib.hqekv_selftest_step_form(segs[0], 1, segs[1], 1, o.data_ptr(), B, Hq, Hkv, D, n, _lib.FUSE_SOFTMAX, ctypes.byref(x)) == 2
+
+    def step():
+        rc = lib.hqekv_decode_step(segs[0], 1, segs[1], 1, q.data_ptr(), None, 0, w.data_ptr(), o.data_ptr(), B, Hq, Hkv, D, n, ws.data_ptr(), ws.numel(),
+                                   _lib.FUSE_SOFTMAX, torch.cuda.current_stream().cuda_stream, ctypes.byref(x))
+        assert rc == 0, lib.hqekv_last_error()
+
+    def result(run):
+        v.copy_(kept)
+        for t in (line, w, o, spare):
+            t.fill_(7)
+        run()
+        torch.cuda.synchronize()
+        return [t.clone() for t in (line, w, o, v, spare)]
+
+    want = result(step)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        step()
+    for _ in range(3):
+        assert all(torch.equal(a, b) for a, b in zip(result(graph.replay), want))
+        assert all(torch.equal(a, b) for a, b in zip(result(step), want))
+    assert torch.equal(want[3][:, :, :1], new if window else kept[:, :, :1]) and torch.equal(want[3][:, :, 1:], kept[:, :, 1:])
