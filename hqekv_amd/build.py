@@ -25,6 +25,8 @@ HIPCC_FLAGS = [
     "-O3", "-std=c++17", "-fPIC", "--offload-arch=gfx950",
     # packed-FP32 VALU forms are kept out of the generated code on purpose
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # a kernel's first 14 argument words arrive in scalar registers
+    "-mllvm", "-amdgpu-kernarg-preload-count=14",
     "-Wno-unused-command-line-argument", "-Wno-unknown-warning-option",
     f"-I{ROOT / 'include'}", f"-I{CSRC}",
 ]

@@ -93,7 +93,7 @@ struct PtValues {
 };
 
 template <int BITS, int HP, bool EXACT, bool NORMAL, bool LOOP, bool FUSED, bool LAST, bool PAIRED, typename StatsLoad, typename StatsMerge>
-__device__ __forceinline__ void pt_class_job(const SegDev &sg, int blk0, int blk1, int bh, int wave, int lane, const half_t *rows, half_t *prows, int64_t Tall,
+__device__ __forceinline__ void pt_class_job(const TileSeg &sg, int blk0, int blk1, int bh, int wave, int lane, const half_t *rows, half_t *prows, int64_t Tall,
                                              int nrep_arg, PtLds<HP, LOOP> &lds, const float *ml, f4_t (&acc)[8], StatsLoad &&load_stats,
                                              StatsMerge &&merge_stats) {
   using G = PtGeom<BITS>;
@@ -304,16 +304,17 @@ struct PtEpilogue {
 
 // `logits` is `p` unless LAST: then the logits lie in the workspace.
 template <int HP, bool EXACT, bool LOOP, bool FUSED, bool LAST>
-__device__ __forceinline__ void pv_tiles_body(const SegTable &tb, const half_t *logits, half_t *p, float *partial, const TilesArgs &ta, int64_t Tall,
-                                              int64_t n_bhq, const FuseArgs &fz) {
+__device__ __forceinline__ void pv_tiles_body(const TileTable &tb, u32x4 begins, const half_t *logits, half_t *p, const float2 *stats, uint32_t heads,
+                                              uint32_t div_hkv, int64_t Tall, float *partial, uint32_t n_bhq, int n_stat, int per, int total_units,
+                                              uint32_t *arrive, half_t *out) {
   __shared__ __align__(16) PtLds<HP, LOOP> lds;
   __shared__ __align__(16) float red[PT_WAVES][HP][128];
   __shared__ float ml[2 * HP];   // (max, 1 / sum exp) of each head's row
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int bh = blockIdx.x, u = blockIdx.y;
-  const SegDev sg = tb.seg[tiles_segment(tb, u)];
-  const int b = tiles_batch_row(ta, bh), hkv = bh - b * ta.Hkv;
-  const int Hq = ta.hq_slice & 0xffff, head0 = first_head(ta.hq_slice, hkv), nrep = EXACT ? HP : ta.nrep;
+  const TileSeg sg = tb.seg[tiles_segment(begins, u)];
+  const int Hq = heads & 0xffffu, Hkv = heads >> 16, nrep = EXACT ? HP : tiles_nrep(begins);
+  const int b = tiles_batch_row(Hkv, div_hkv, bh), head0 = (bh - b * Hkv) * nrep;
   const half_t *rows = logits + ((int64_t)b * Hq + head0) * Tall;
   half_t *prows = p + ((int64_t)b * Hq + head0) * Tall;
   f4_t acc[8];
@@ -326,23 +327,23 @@ __device__ __forceinline__ void pv_tiles_body(const SegTable &tb, const half_t *
   auto read_stats = [&](const float2 *sp) {
 #pragma unroll
     for (int k = 0; k < 4; ++k)
-      if (k == 0 || fz.n_stat > 64 * k) {
+      if (k == 0 || n_stat > 64 * k) {
         uint32_t w[2];
-        load_words<2, Words4<2>>(sp, 8u * (uint32_t)min(lane + 64 * k, fz.n_stat - 1), w);
+        load_words<2, Words4<2>>(sp, 8u * (uint32_t)min(lane + 64 * k, n_stat - 1), w);
         sv[k] = make_float2(__builtin_bit_cast(float, w[0]), __builtin_bit_cast(float, w[1]));
       }
   };
   const int first = LAST ? (int)threadIdx.x >> 4 : wave;
-  const float2 *srow = fz.stats + ((int64_t)b * Hq + head0 + min(first, nrep - 1)) * fz.n_stat;
+  const float2 *srow = stats + ((int64_t)b * Hq + head0 + min(first, nrep - 1)) * n_stat;
   auto load_stats = [&]() {
-    if constexpr (LAST) row16_read(srow, fz.n_stat, lane & 15, sv);
+    if constexpr (LAST) row16_read(srow, n_stat, lane & 15, sv);
     else if (FUSED) read_stats(srow);
   };
   auto merge_stats = [&]() {
     if (!FUSED) return;
     if constexpr (LAST) {
       if (wave * 4 < nrep) {
-        const float2 v = row16_merge(srow, fz.n_stat, lane & 15, sv);
+        const float2 v = row16_merge(srow, n_stat, lane & 15, sv);
         if ((lane & 15) == 0 && first < nrep) {
           ml[2 * first] = v.x;
           ml[2 * first + 1] = v.y;
@@ -352,19 +353,19 @@ __device__ __forceinline__ void pv_tiles_body(const SegTable &tb, const half_t *
       return;
     }
     for (int h = wave; h < nrep; h += PT_WAVES) {
-      const float2 *sp = srow + (int64_t)(h - wave) * fz.n_stat;
+      const float2 *sp = srow + (int64_t)(h - wave) * n_stat;
       if (h != wave) read_stats(sp);
       float m = sv[0].x;
 #pragma unroll
       for (int k = 1; k < 4; ++k)
-        if (fz.n_stat > 64 * k) m = fmaxf(m, sv[k].x);
-      for (int e = lane + 256; e < fz.n_stat; e += 64) m = fmaxf(m, sp[e].x);
+        if (n_stat > 64 * k) m = fmaxf(m, sv[k].x);
+      for (int e = lane + 256; e < n_stat; e += 64) m = fmaxf(m, sp[e].x);
       m = wave_max(m);
       float l = 0.f;
 #pragma unroll
       for (int k = 0; k < 4; ++k)
-        if (k == 0 || fz.n_stat > 64 * k) l += lane + 64 * k < fz.n_stat ? sv[k].y * __expf(sv[k].x - m) : 0.f;
-      for (int e = lane + 256; e < fz.n_stat; e += 64) {
+        if (k == 0 || n_stat > 64 * k) l += lane + 64 * k < n_stat ? sv[k].y * __expf(sv[k].x - m) : 0.f;
+      for (int e = lane + 256; e < n_stat; e += 64) {
         const float2 w = sp[e];
         l += w.y * __expf(w.x - m);
       }
@@ -376,7 +377,7 @@ __device__ __forceinline__ void pv_tiles_body(const SegTable &tb, const half_t *
     }
     __syncthreads();
   };
-  const int unit = u - sg.unit_begin, per = tb.per_unit, b0 = unit * per;
+  const int unit = u - sg.unit_begin, b0 = unit * per;
   const bool paired = qt_runs(sg) && sg.n_tokens % 2 == 0;
 #define HQ_JOB_P(B_, NORMAL_, PAIRED_)                                                                                                   \
   pt_class_job<B_, HP, EXACT, NORMAL_, LOOP, FUSED, LAST, PAIRED_>(sg, b0, min(b0 + per, (int)((sg.n_tokens + PtGeom<B_>::BLOCK - 1) / PtGeom<B_>::BLOCK)), \
@@ -429,7 +430,7 @@ __device__ __forceinline__ void pv_tiles_body(const SegTable &tb, const half_t *
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     __shared__ int last;
-    if (threadIdx.x == 0) last = __hip_atomic_fetch_add(&fz.arrive[bh], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == (uint32_t)tb.total_units;
+    if (threadIdx.x == 0) last = __hip_atomic_fetch_add(&arrive[bh], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == (uint32_t)total_units;
     __syncthreads();
     if (!last) return;
     // 16 bytes of a row per lane; HP = 4: the even and the odd rows by one half of the workgroup each.
@@ -438,10 +439,10 @@ __device__ __forceinline__ void pv_tiles_body(const SegTable &tb, const half_t *
     const int at = threadIdx.x % LANES, g = threadIdx.x / LANES;
     const bool mine = EXACT || at < nrep * 32;
     const uint32_t row_b = (uint32_t)n_bhq * 512u;   // (the rows of a short launch span a few MB)
-    const rsrc_t rows_of = make_rsrc(partial + ((int64_t)b * Hq + head0) * 128, (uint32_t)(tb.total_units - 1) * row_b + (uint32_t)nrep * 512u);
+    const rsrc_t rows_of = make_rsrc(partial + ((int64_t)b * Hq + head0) * 128, (uint32_t)(total_units - 1) * row_b + (uint32_t)nrep * 512u);
     f4_t v = (f4_t){0.f, 0.f, 0.f, 0.f};
     if (mine) {
-      for (int c0 = 0; c0 < tb.total_units; c0 += GROUPS * PT_LAST_ROWS) {
+      for (int c0 = 0; c0 < total_units; c0 += GROUPS * PT_LAST_ROWS) {
         f4_t t[PT_LAST_ROWS];
         static_for<PT_LAST_ROWS>([&](auto I_) {   // (past the last row: zeros, without a trip to memory)
           constexpr int I = decltype(I_)::value;
@@ -458,23 +459,25 @@ __device__ __forceinline__ void pv_tiles_body(const SegTable &tb, const half_t *
     }
     if (g == 0 && mine) {
       uint2 w = make_uint2(as_u32(pack_h2((half_t)v[0], (half_t)v[1])), as_u32(pack_h2((half_t)v[2], (half_t)v[3])));
-      *reinterpret_cast<uint2 *>(fz.out + ((int64_t)b * Hq + head0) * 128 + 4 * at) = w;
+      *reinterpret_cast<uint2 *>(out + ((int64_t)b * Hq + head0) * 128 + 4 * at) = w;
     }
   }
 }
 
 template <int HP, bool EXACT, bool LOOP, bool FUSED>
-__global__ __launch_bounds__(PT_WAVES * 64, HP <= 8 ? (LOOP ? (HP == 8 ? 3 : 4) : 6) : 2) void pv_tiles_kernel(SegTable tb, half_t *__restrict__ p, float *__restrict__ partial,
-                                                                   TilesArgs ta, int64_t Tall, int64_t n_bhq, FuseArgs fz) {
-  pv_tiles_body<HP, EXACT, LOOP, FUSED, false>(tb, p, p, partial, ta, Tall, n_bhq, fz);
+__global__ __launch_bounds__(PT_WAVES * 64, HP <= 8 ? (LOOP ? (HP == 8 ? 3 : 4) : 6) : 2) void pv_tiles_kernel(
+    u32x4 begins, half_t *__restrict__ p, const float2 *__restrict__ stats, float *__restrict__ partial, uint32_t heads, uint32_t div_hkv, int64_t Tall,
+    uint32_t n_bhq, int32_t n_stat, int32_t per_unit, TileTable tb) {
+  pv_tiles_body<HP, EXACT, LOOP, FUSED, false>(tb, begins, p, p, stats, heads, div_hkv, Tall, partial, n_bhq, n_stat, per_unit, 0, nullptr, nullptr);
 }
 
 template <int HP, bool EXACT>
-__global__ __launch_bounds__(PT_WAVES * 64, 4) void pv_last_kernel(SegTable tb, const half_t *__restrict__ logits, half_t *__restrict__ p,
-                                                                   float *__restrict__ partial, TilesArgs ta, int64_t Tall, int64_t n_bhq, FuseArgs fz,
-                                                                   StepEpilogue ep) {
-  if ((int)blockIdx.y < tb.total_units) {
-    pv_tiles_body<HP, EXACT, false, true, true>(tb, logits, p, partial, ta, Tall, n_bhq, fz);
+__global__ __launch_bounds__(PT_WAVES * 64, 4) void pv_last_kernel(
+    u32x4 begins, const half_t *__restrict__ logits, half_t *__restrict__ p, const float2 *__restrict__ stats, uint32_t heads, uint32_t div_hkv,
+    int64_t Tall, float *__restrict__ partial, uint32_t n_bhq, int32_t n_stat, int32_t total_units, uint32_t *__restrict__ arrive,
+    half_t *__restrict__ out, TileTable tb, StepEpilogue ep) {
+  if ((int)blockIdx.y < total_units) {
+    pv_tiles_body<HP, EXACT, false, true, true>(tb, begins, logits, p, stats, heads, div_hkv, Tall, partial, n_bhq, n_stat, 1, total_units, arrive, out);
     return;
   }
   __shared__ __align__(16) PtEpilogue sh;
@@ -483,17 +486,17 @@ __global__ __launch_bounds__(PT_WAVES * 64, 4) void pv_last_kernel(SegTable tb, 
     for (int row = threadIdx.x >> 4; row < rows; row += 2 * PT_WAVES * 4) {   // two rows at a time
       float2 sv[2][4];
 #pragma unroll
-      for (int k = 0; k < 2; ++k) row16_read(fz.stats + (int64_t)min(row + k * PT_WAVES * 4, rows - 1) * fz.n_stat, fz.n_stat, lane, sv[k]);
+      for (int k = 0; k < 2; ++k) row16_read(stats + (int64_t)min(row + k * PT_WAVES * 4, rows - 1) * n_stat, n_stat, lane, sv[k]);
 #pragma unroll
       for (int k = 0; k < 2; ++k) {
         const int at = min(row + k * PT_WAVES * 4, rows - 1);
-        const float2 v = row16_merge(fz.stats + (int64_t)at * fz.n_stat, fz.n_stat, lane, sv[k]);
+        const float2 v = row16_merge(stats + (int64_t)at * n_stat, n_stat, lane, sv[k]);
         if (lane == 0) sh.ml[at] = v;
       }
     }
     __syncthreads();
   }
-  step_epilogue_block<false>(ep, (int64_t)(blockIdx.y - tb.total_units) * gridDim.x + blockIdx.x, (int64_t)(gridDim.y - tb.total_units) * gridDim.x,
+  step_epilogue_block<false>(ep, (int64_t)(blockIdx.y - total_units) * gridDim.x + blockIdx.x, (int64_t)(gridDim.y - total_units) * gridDim.x,
                              sh.ring, [&](int row, uint64_t quad) {
     const float2 ml = sh.ml[row];
     uint64_t v = 0;
@@ -509,11 +512,12 @@ int64_t pv_block_tokens(int bits) { return bits >= 8 ? PtGeom<8>::BLOCK : PT_BLO
 
 int launch_pv_tiles(const SegTable &tb, void *p, float *partial, int64_t B, int64_t Hq, int64_t Hkv, int64_t Tall, const FuseArgs &fz,
                     hipStream_t st) {
-  const TilesArgs ta = tiles_args(B, Hq, Hkv);
-  const int nrep = ta.nrep;
+  const TilesHost t = tiles_host(tb, Hq, Hkv);
+  const int64_t nrep = Hq / Hkv;
   const dim3 grid((unsigned)(B * Hkv), (unsigned)tb.total_units), block(PT_WAVES * 64);
 #define LAUNCH(HP_, EXACT_, LOOP_, FUSED_) \
-  hipLaunchKernelGGL((pv_tiles_kernel<HP_, EXACT_, LOOP_, FUSED_>), grid, block, 0, st, tb, (half_t *)p, partial, ta, Tall, B * Hq, fz)
+  hipLaunchKernelGGL((pv_tiles_kernel<HP_, EXACT_, LOOP_, FUSED_>), grid, block, 0, st, t.begins, (half_t *)p, fz.stats, partial, t.heads, \
+                     t.div_hkv, Tall, (uint32_t)(B * Hq), fz.n_stat, tb.per_unit, t.table)
   const bool loop = tb.per_unit > 1;
 #define LAUNCH_H(HP_)                                                                 \
   if (!fz.stats) LAUNCH(HP_, false, true, false);                                     \
@@ -545,15 +549,15 @@ bool pv_last_takes(const StepEpilogue &ep, int64_t Tall) {
 
 int launch_pv_last(const SegTable &tb, const void *logits, void *probs, float *partial, int64_t B, int64_t Hq, int64_t Hkv, int64_t Tall,
                    const FuseArgs &fz, const StepEpilogue &ep, hipStream_t st) {
-  const TilesArgs ta = tiles_args(B, Hq, Hkv);
-  const int nrep = ta.nrep;
+  const TilesHost t = tiles_host(tb, Hq, Hkv);
+  const int64_t nrep = Hq / Hkv;
   int64_t more = 0;   // workgroups for the epilogue
   if (ep.ring_line) more = (Tall + RING_SPAN_SHORT - 1) / RING_SPAN_SHORT;
   else if (ep.app_rows > 0 || ep.leave_bits) more = 1;
   const dim3 grid((unsigned)(B * Hkv), (unsigned)(tb.total_units + (more + B * Hkv - 1) / (B * Hkv)));
 #define LAUNCH(HP_, EXACT_)                                                                                                                     \
-  hipLaunchKernelGGL((pv_last_kernel<HP_, EXACT_>), grid, dim3(PT_WAVES * 64), 0, st, tb, (const half_t *)logits, (half_t *)probs, partial, ta, \
-                     Tall, B *Hq, fz, ep)
+  hipLaunchKernelGGL((pv_last_kernel<HP_, EXACT_>), grid, dim3(PT_WAVES * 64), 0, st, t.begins, (const half_t *)logits, (half_t *)probs, fz.stats, \
+                     t.heads, t.div_hkv, Tall, partial, (uint32_t)(B * Hq), fz.n_stat, tb.total_units, fz.arrive, fz.out, t.table, ep)
   if (nrep == 4) LAUNCH(4, true);
   else if (nrep < 4) LAUNCH(4, false);
   else if (nrep == 8) LAUNCH(8, true);

@@ -44,7 +44,7 @@ struct QtLds {
 // test is one addition per score (a step at 32k tokens 19.72 -> 19.80 us, at 3 x 16k with five heads per KV head 25.34 ->
 // 25.50, at 8 x 64k 152.1 -> 151.9); a select per lane after products without bands would cost four times the accumulators.
 template <int BITS, bool NORMAL, bool ROWS>
-__device__ __forceinline__ float qk_alone(const SegDev &sg, int bh, uint32_t token, const half_t *q) {
+__device__ __forceinline__ float qk_alone(const TileSeg &sg, int bh, uint32_t token, const half_t *q) {
   const uint32_t n_tok = (uint32_t)sg.n_tokens;
   float sum = 0.f;
 #pragma unroll 1
@@ -127,7 +127,7 @@ __device__ __forceinline__ void qt_finish_tile(QtLds<HP> &lds, const f4_t (&acc)
 }
 
 template <int BITS, int HP, bool FUSED, bool NORMAL, typename QueryRow>
-__device__ __forceinline__ void qt_class_tile(const SegDev &sg, int tile, int bh, int n_bh, int wave, int lane, u32x4 q, QtLds<HP> &lds,
+__device__ __forceinline__ void qt_class_tile(const TileSeg &sg, int tile, int bh, int n_bh, int wave, int lane, u32x4 q, QtLds<HP> &lds,
                                               half_t *row, bool has_head, float inv_sqrt_d, float &m, float &l, QueryRow &&qrow) {
   using G = QtGeom<BITS>;
   constexpr bool QUANT = BITS != 16;
@@ -230,7 +230,7 @@ __device__ __forceinline__ void qt_class_tile(const SegDev &sg, int tile, int bh
 constexpr int QT_TM_TILE = 64;
 
 template <int HP, bool FUSED, typename QueryRow>
-__device__ __forceinline__ void qt_rows_tile(const SegDev &sg, int tile, int bh, int wave, int lane, u32x4 q, QtLds<HP> &lds, half_t *row,
+__device__ __forceinline__ void qt_rows_tile(const TileSeg &sg, int tile, int bh, int wave, int lane, u32x4 q, QtLds<HP> &lds, half_t *row,
                                              bool has_head, float inv_sqrt_d, float &m, float &l, QueryRow &&qrow) {
   constexpr int BANDS = 16 / HP, TPV = 4 / BANDS;
   const int n = lane & 15, r = lane >> 4;
@@ -263,14 +263,15 @@ __device__ __forceinline__ void qt_rows_tile(const SegDev &sg, int tile, int bh,
 // COUNT: the p.V launch of the same call counts arrivals, from zero (a form of its own: a test for it costs every launch a
 // scalar load in its prologue, 0.3 us of a step at 32k tokens).
 template <int HP, bool FUSED, bool COUNT>
-__global__ __launch_bounds__(QT_WAVES * 64, HP == 16 ? 2 : HP == 4 || FUSED ? 5 : 4) void qk_tiles_kernel(SegTable tb, const half_t *__restrict__ q,
-                                                                    half_t *__restrict__ scores, TilesArgs ta, int64_t Tall, FuseArgs fz) {
+__global__ __launch_bounds__(QT_WAVES * 64, HP == 16 ? 2 : HP == 4 || FUSED ? 5 : 4) void qk_tiles_kernel(
+    u32x4 begins, const half_t *__restrict__ q, half_t *__restrict__ scores, float2 *__restrict__ stats, uint32_t heads, uint32_t div_hkv, int64_t Tall,
+    int32_t n_bh, int32_t n_stat, float inv_sqrt_d, uint32_t *__restrict__ arrive, TileTable tb) {
   __shared__ __align__(16) QtLds<HP> lds;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int bh = blockIdx.x, u = (int)blockIdx.y;
-  const SegDev sg = tb.seg[tiles_segment(tb, u)];
-  const int b = tiles_batch_row(ta, bh), hkv = bh - b * ta.Hkv;
-  const int Hq = ta.hq_slice & 0xffff, head0 = first_head(ta.hq_slice, hkv), nrep = ta.nrep;
+  const TileSeg sg = tb.seg[tiles_segment(begins, u)];
+  const int Hq = heads & 0xffffu, Hkv = heads >> 16, nrep = tiles_nrep(begins);
+  const int b = tiles_batch_row(Hkv, div_hkv, bh), head0 = (bh - b * Hkv) * nrep;
   const int n = lane & 15, r = lane >> 4;
   // row l % 16 of A: head (l % 16) % HP of this launch (rows without a head repeat one, their results are dropped)
   u32x4 qv;
@@ -279,14 +280,14 @@ __global__ __launch_bounds__(QT_WAVES * 64, HP == 16 ? 2 : HP == 4 || FUSED ? 5 
     load_words<4, Words2<4>>(q + ((int64_t)b * Hq + head0) * 128, (uint32_t)min(n % HP, nrep - 1) * 256u + 64u * wave + 16u * r, w);
     qv = (u32x4){w[0], w[1], w[2], w[3]};
   }
-  if (COUNT && u == 0 && threadIdx.x == 0) fz.arrive[bh] = 0u;
+  if (COUNT && u == 0 && threadIdx.x == 0) arrive[bh] = 0u;
   const int tile = u - sg.unit_begin;
   const int head = (4 * r) % HP + wave;   // the head this lane finishes
   const bool has_head = head < nrep;
   half_t *row = scores + ((int64_t)b * Hq + head0 + min(head, nrep - 1)) * Tall;
   auto qrow = [&]() { return q + ((int64_t)b * Hq + head0 + min((4 * (lane >> 4)) % HP + wave, nrep - 1)) * 128; };
   float m = SM_FLOOR, l = 0.f;
-#define HQ_TILE(B_, NORMAL_) qt_class_tile<B_, HP, FUSED, NORMAL_>(sg, tile, bh, ta.n_bh, wave, lane, qv, lds, row, has_head, fz.inv_sqrt_d, m, l, qrow)
+#define HQ_TILE(B_, NORMAL_) qt_class_tile<B_, HP, FUSED, NORMAL_>(sg, tile, bh, n_bh, wave, lane, qv, lds, row, has_head, inv_sqrt_d, m, l, qrow)
   switch (sg.bits) {
     case 1:
       if ((sg.layout & 3) == HQEKV_LAYOUT_NORMAL1) HQ_TILE(1, true);
@@ -296,7 +297,7 @@ __global__ __launch_bounds__(QT_WAVES * 64, HP == 16 ? 2 : HP == 4 || FUSED ? 5 
     case 4: HQ_TILE(4, false); break;
     case 8: HQ_TILE(8, false); break;
     default:
-      if ((sg.layout & 3) == HQEKV_LAYOUT_TOKEN_MAJOR) qt_rows_tile<HP, FUSED>(sg, tile, bh, wave, lane, qv, lds, row, has_head, fz.inv_sqrt_d, m, l, qrow);
+      if ((sg.layout & 3) == HQEKV_LAYOUT_TOKEN_MAJOR) qt_rows_tile<HP, FUSED>(sg, tile, bh, wave, lane, qv, lds, row, has_head, inv_sqrt_d, m, l, qrow);
       else HQ_TILE(16, false);
   }
 #undef HQ_TILE
@@ -316,7 +317,7 @@ __global__ __launch_bounds__(QT_WAVES * 64, HP == 16 ? 2 : HP == 4 || FUSED ? 5 
   l += dpp_f<0x140>(l);
   if (HP <= 4) l += xor_f(l, 16);
   if (HP <= 8) l += xor_f(l, 32);
-  if (n == 0 && 4 * r < HP && has_head) fz.stats[((int64_t)b * Hq + head0 + head) * fz.n_stat + u] = make_float2(mm, l);
+  if (n == 0 && 4 * r < HP && has_head) stats[((int64_t)b * Hq + head0 + head) * n_stat + u] = make_float2(mm, l);
 }
 
 // ---- Long launches: four tiles per workgroup, one per wave, which walks all of head_dim in four steps of 32 channels with
@@ -390,7 +391,7 @@ __device__ __forceinline__ void ql_finish(f4_t (&acc)[TPV], int r, Pos &&pos, in
 }
 
 template <int BITS, int HP, bool FUSED, bool NORMAL>
-__device__ __forceinline__ void ql_class(const SegDev &sg, int unit, int bh, int n_bh, int wave, int lane, const half_t *qrow, uint2 *sz, half_t *rows,
+__device__ __forceinline__ void ql_class(const TileSeg &sg, int unit, int bh, int n_bh, int wave, int lane, const half_t *qrow, uint2 *sz, half_t *rows,
                                          int64_t Tall, int nrep, float inv_sqrt_d, float (&m)[4], float (&l)[4], const half_t *q0) {
   using G = QtGeom<BITS>;
   constexpr bool QUANT = BITS != 16;
@@ -514,7 +515,7 @@ __device__ __forceinline__ void ql_class(const SegDev &sg, int unit, int bh, int
 
 // fp16 K rows stored token by token: a wave takes the 64 tokens of one tile, 32 channels at a time
 template <int HP, bool FUSED>
-__device__ __forceinline__ void ql_rows(const SegDev &sg, int unit, int bh, int wave, int lane, const half_t *qrow, half_t *rows, int64_t Tall, int nrep,
+__device__ __forceinline__ void ql_rows(const TileSeg &sg, int unit, int bh, int wave, int lane, const half_t *qrow, half_t *rows, int64_t Tall, int nrep,
                                         float inv_sqrt_d, float (&m)[4], float (&l)[4], const half_t *q0) {
   constexpr int BANDS = 16 / HP, TPV = 4 / BANDS;
   const int n = lane & 15, r = lane >> 4;
@@ -550,15 +551,16 @@ __device__ __forceinline__ void ql_rows(const SegDev &sg, int unit, int bh, int 
 }
 
 template <int HP, bool FUSED>
-__global__ __launch_bounds__(QT_WAVES * 64, HP == 4 ? 4 : 2) void qk_long_kernel(SegTable tb, const half_t *__restrict__ q, half_t *__restrict__ scores,
-                                                                               TilesArgs ta, int64_t Tall, FuseArgs fz) {
+__global__ __launch_bounds__(QT_WAVES * 64, HP == 4 ? 4 : 2) void qk_long_kernel(
+    u32x4 begins, const half_t *__restrict__ q, half_t *__restrict__ scores, float2 *__restrict__ stats, uint32_t heads, uint32_t div_hkv, int64_t Tall,
+    int32_t n_bh, int32_t n_stat, float inv_sqrt_d, TileTable tb) {
   __shared__ __align__(16) uint2 sz[64 * QL_NGP];
   __shared__ float2 st[QT_WAVES][HP];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int bh = blockIdx.x, u = (int)blockIdx.y;
-  const SegDev sg = tb.seg[tiles_segment(tb, u)];
-  const int b = tiles_batch_row(ta, bh), hkv = bh - b * ta.Hkv;
-  const int Hq = ta.hq_slice & 0xffff, head0 = first_head(ta.hq_slice, hkv), nrep = ta.nrep;
+  const TileSeg sg = tb.seg[tiles_segment(begins, u)];
+  const int Hq = heads & 0xffffu, Hkv = heads >> 16, nrep = tiles_nrep(begins);
+  const int b = tiles_batch_row(Hkv, div_hkv, bh), head0 = (bh - b * Hkv) * nrep;
   const int n = lane & 15, r = lane >> 4, unit = u - sg.unit_begin;
   const half_t *q0 = q + ((int64_t)b * Hq + head0) * 128, *qrow = q0 + min(n % HP, nrep - 1) * 128;
   half_t *rows = scores + ((int64_t)b * Hq + head0) * Tall;
@@ -568,7 +570,7 @@ __global__ __launch_bounds__(QT_WAVES * 64, HP == 4 ? 4 : 2) void qk_long_kernel
     m[h] = SM_FLOOR;
     l[h] = 0.f;
   }
-#define HQ_TILE(B_, NORMAL_) ql_class<B_, HP, FUSED, NORMAL_>(sg, unit, bh, ta.n_bh, wave, lane, qrow, sz, rows, Tall, nrep, fz.inv_sqrt_d, m, l, q0)
+#define HQ_TILE(B_, NORMAL_) ql_class<B_, HP, FUSED, NORMAL_>(sg, unit, bh, n_bh, wave, lane, qrow, sz, rows, Tall, nrep, inv_sqrt_d, m, l, q0)
   switch (sg.bits) {
     case 1:
       if ((sg.layout & 3) == HQEKV_LAYOUT_NORMAL1) HQ_TILE(1, true);
@@ -578,7 +580,7 @@ __global__ __launch_bounds__(QT_WAVES * 64, HP == 4 ? 4 : 2) void qk_long_kernel
     case 4: HQ_TILE(4, false); break;
     case 8: HQ_TILE(8, false); break;
     default:
-      if ((sg.layout & 3) == HQEKV_LAYOUT_TOKEN_MAJOR) ql_rows<HP, FUSED>(sg, unit, bh, wave, lane, qrow, rows, Tall, nrep, fz.inv_sqrt_d, m, l, q0);
+      if ((sg.layout & 3) == HQEKV_LAYOUT_TOKEN_MAJOR) ql_rows<HP, FUSED>(sg, unit, bh, wave, lane, qrow, rows, Tall, nrep, inv_sqrt_d, m, l, q0);
       else HQ_TILE(16, false);
   }
 #undef HQ_TILE
@@ -613,7 +615,7 @@ __global__ __launch_bounds__(QT_WAVES * 64, HP == 4 ? 4 : 2) void qk_long_kernel
     }
 #pragma unroll
     for (int w = 0; w < QT_WAVES; ++w) ll += v[w].x == mm ? v[w].y : v[w].y * __expf(v[w].x - mm);
-    fz.stats[((int64_t)b * Hq + head0 + head) * fz.n_stat + u] = make_float2(mm, ll);
+    stats[((int64_t)b * Hq + head0 + head) * n_stat + u] = make_float2(mm, ll);
   }
 }
 
@@ -664,18 +666,22 @@ int64_t tiles_unit_tokens(const TilesPlan &p, const hqekv_seg &s) { return (p.is
 
 int launch_qk_tiles(const SegTable &tb, const void *q, void *scores, int64_t B, int64_t Hq, int64_t Hkv, int64_t Tall, const FuseArgs &fz,
                     hipStream_t st) {
-  const TilesArgs ta = tiles_args(B, Hq, Hkv);
-  const int nrep = ta.nrep;
+  const TilesHost t = tiles_host(tb, Hq, Hkv);
+  const int64_t nrep = Hq / Hkv;
   const dim3 grid((unsigned)(B * Hkv), (unsigned)tb.total_units);
-#define LAUNCH(...) hipLaunchKernelGGL((__VA_ARGS__), grid, dim3(QT_WAVES * 64), 0, st, tb, (const half_t *)q, (half_t *)scores, ta, Tall, fz)
-#define LAUNCH_H(HP_)                                                             \
-  if (tb.per_unit > 1 && fz.stats) LAUNCH(qk_long_kernel<HP_, true>);             \
-  else if (tb.per_unit > 1) LAUNCH(qk_long_kernel<HP_, false>);                   \
-  else if (fz.stats && fz.arrive) LAUNCH(qk_tiles_kernel<HP_, true, (HP_ <= 8)>); \
-  else if (fz.stats) LAUNCH(qk_tiles_kernel<HP_, true, false>);                   \
-  else LAUNCH(qk_tiles_kernel<HP_, false, false>)
+#define LAUNCH(MORE_, ...)                                                                                                                      \
+  hipLaunchKernelGGL((__VA_ARGS__), grid, dim3(QT_WAVES * 64), 0, st, t.begins, (const half_t *)q, (half_t *)scores, fz.stats, t.heads, t.div_hkv, \
+                     Tall, (int32_t)(B * Hkv), fz.n_stat, fz.inv_sqrt_d MORE_, t.table)
+#define COUNTED , fz.arrive
+#define LAUNCH_H(HP_)                                                                      \
+  if (tb.per_unit > 1 && fz.stats) LAUNCH(, qk_long_kernel<HP_, true>);                    \
+  else if (tb.per_unit > 1) LAUNCH(, qk_long_kernel<HP_, false>);                          \
+  else if (fz.stats && fz.arrive) LAUNCH(COUNTED, qk_tiles_kernel<HP_, true, (HP_ <= 8)>); \
+  else if (fz.stats) LAUNCH(COUNTED, qk_tiles_kernel<HP_, true, false>);                   \
+  else LAUNCH(COUNTED, qk_tiles_kernel<HP_, false, false>)
   if (nrep <= 4) { LAUNCH_H(4); } else if (nrep <= 8) { LAUNCH_H(8); } else { LAUNCH_H(16); }
 #undef LAUNCH_H
+#undef COUNTED
 #undef LAUNCH
   return check_launch("qk_tiles_kernel");
 }

@@ -62,22 +62,36 @@ __device__ __forceinline__ void wave_lds_fence() {
 }
 
 // =============================================================================== what both launches take apart
-// A workgroup's segment, its (b, kv head) taken apart, its first query head: scalar arithmetic only, since everything the
-// workgroup does waits for it (the compiler's own choice went through vector registers for the comparisons and through a
-// float reciprocal for the division).
-struct TilesArgs {
-  int32_t hq_slice, nrep;
-  int32_t Hkv;
-  uint32_t div_hkv;   // ceil(2^32 / Hkv): bh / Hkv is the high word of the product as long as bh Hkv < 2^32
-  int32_t n_bh;
+// What a workgroup needs before it can ask for anything -- the segments' first units, the pointers it starts from, the head
+// counts -- stands first among the arguments, as 14 words that the command processor puts into scalar registers before the
+// wave starts (build.py: -amdgpu-kernarg-preload-count).  Its first load is then the segment's entry, one cache line; with the
+// begins in memory that was the second round, a fifth of a microsecond per launch: a step at 32k tokens 19.37 -> 18.89 us, 3 x
+// 16k with five heads per KV head 24.2 -> 23.5, 8 x 64k 150.3 -> 148.6, a KIVI layer's 24 steps at 4k 450 -> 440.
+struct __attribute__((aligned(64))) TileSeg {
+  const void *data;
+  const half_t *scale;
+  const half_t *zero;
+  const int64_t *idx;
+  int64_t slab_tokens;   // as SegDev's
+  int32_t pos_base, n_tokens;
+  int32_t bits, layout;
+  int32_t unit_begin;
 };
-__device__ __forceinline__ int tiles_segment(const SegTable &tb, int u) {
-  int s = -1;
+static_assert(sizeof(TileSeg) == 64, "one line");
+struct TileTable {
+  TileSeg seg[HQEKV_MAX_SEGS];
+};
+// Seven begins of 16 bits (0xffff: unused; the first segment's is 0) and, in the first half word, the heads per KV head;
+// Hq | Hkv << 16 beside them.
+__device__ __forceinline__ int tiles_nrep(u32x4 begins) { return (int)(begins[0] & 0xffffu); }
+__device__ __forceinline__ int tiles_segment(u32x4 begins, int u) {   // scalar arithmetic only: everything waits for it
+  int s = 0;
 #pragma unroll
-  for (int k = 0; k < HQEKV_MAX_SEGS; ++k) s -= (tb.begin[k] - u - 1) >> 31;   // (an unused entry's begin is INT32_MAX)
+  for (int k = 1; k < HQEKV_MAX_SEGS; ++k) s -= ((int)(k & 1 ? begins[k / 2] >> 16 : begins[k / 2] & 0xffffu) - u - 1) >> 31;
   return s;
 }
-__device__ __forceinline__ int tiles_batch_row(const TilesArgs &a, int bh) { return a.Hkv == 1 ? bh : (int)__umulhi((uint32_t)bh, a.div_hkv); }
+// div_hkv = ceil(2^32 / Hkv): bh / Hkv is the high word of the product as long as bh Hkv < 2^32
+__device__ __forceinline__ int tiles_batch_row(int Hkv, uint32_t div_hkv, int bh) { return Hkv == 1 ? bh : (int)__umulhi((uint32_t)bh, div_hkv); }
 
 // Position of token t, below 2^31 (it indexes a row of Tall scores): the low word of its index is enough, read at the first
 // token of its run of 32 where positions come in runs (HQEKV_LAYOUT_RUNS).  In two parts without a branch between them, so
@@ -85,7 +99,7 @@ __device__ __forceinline__ int tiles_batch_row(const TilesArgs &a, int bh) { ret
 struct Positions {
   const void *src;      // the index, or anything readable
   uint32_t keep, scale, run, base;
-  __device__ __forceinline__ explicit Positions(const SegDev &sg) {
+  __device__ __forceinline__ explicit Positions(const TileSeg &sg) {
     const bool has = sg.idx != nullptr;
     src = has ? (const void *)sg.idx : sg.data;
     keep = __builtin_amdgcn_readfirstlane(has ? ~0u : 0u);   // (or the compiler makes two code paths of it)
@@ -97,7 +111,7 @@ struct Positions {
   __device__ __forceinline__ uint32_t of(uint32_t t, uint32_t fetched) const { return (fetched & keep) + (t & run) + base; }
   __device__ __forceinline__ uint32_t operator()(uint32_t t) const { return of(t, fetch(t)); }
 };
-__device__ __forceinline__ bool qt_runs(const SegDev &sg) { return (sg.layout & HQEKV_LAYOUT_RUNS) || !sg.idx; }
+__device__ __forceinline__ bool qt_runs(const TileSeg &sg) { return (sg.layout & HQEKV_LAYOUT_RUNS) || !sg.idx; }
 
 // =============================================================================== host side
 // p.V workgroups the chip holds at once, of the single-block form, and the workgroups a looping launch is made of: one
@@ -130,9 +144,24 @@ bool tiles_fit(const hqekv_seg *segs, int nseg, bool is_k, int64_t D, int64_t B,
 TilesPlan tiles_plan(const hqekv_seg *segs, int nseg, bool is_k, int64_t BHkv, int64_t nrep);
 int64_t tiles_unit_tokens(const TilesPlan &p, const hqekv_seg &s);
 
-inline TilesArgs tiles_args(int64_t B, int64_t Hq, int64_t Hkv) {
-  const int nrep = (int)(Hq / Hkv);
-  return TilesArgs{hq_with_slice((int)Hq, nrep, 0), nrep, (int32_t)Hkv, (uint32_t)(((1ULL << 32) + Hkv - 1) / Hkv), (int32_t)(B * Hkv)};
+// The arguments of both launches.
+struct TilesHost {
+  u32x4 begins;
+  uint32_t heads, div_hkv;
+  TileTable table;
+};
+inline TilesHost tiles_host(const SegTable &tb, int64_t Hq, int64_t Hkv) {
+  TilesHost h{};
+  for (int k = 0; k < HQEKV_MAX_SEGS; ++k) {
+    const uint32_t v = k == 0 ? (uint32_t)(Hq / Hkv) : k < tb.nseg ? (uint32_t)tb.begin[k] : 0xffffu;   // (65535 units at most)
+    h.begins[k / 2] |= v << (16 * (k & 1));
+    if (k >= tb.nseg) continue;
+    const SegDev &s = tb.seg[k];
+    h.table.seg[k] = TileSeg{s.data, s.scale, s.zero, s.idx, s.slab_tokens, (int32_t)s.pos_base, (int32_t)s.n_tokens, s.bits, s.layout, s.unit_begin};
+  }
+  h.heads = (uint32_t)Hq | (uint32_t)Hkv << 16;
+  h.div_hkv = (uint32_t)(((1ULL << 32) + Hkv - 1) / Hkv);
+  return h;
 }
 
 int64_t pv_block_tokens(int bits);   // tokens of a p.V block
