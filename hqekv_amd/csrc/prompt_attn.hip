@@ -25,6 +25,8 @@ constexpr int PA_D = 128;
 constexpr int PA_WAVES = 4;
 constexpr int PA_THREADS = 64 * PA_WAVES;
 constexpr int PA_BC = 32;              // keys per score tile
+constexpr float PA_SLACK = 8.f;        // powers of two
+constexpr int PA_SHARE = 4;
 // How the four waves of a workgroup share its work, and how many keys a wave takes at a time.
 // <1, 1>: 32 query rows each, 128 per workgroup, every wave walks all key tiles (164 registers, 32 KB of LDS: three
 // workgroups per CU).  For long prompts, which are bound by the chip's power: no order of the same instructions is faster.
@@ -107,8 +109,9 @@ __device__ __forceinline__ f16_t pa_scores(const half_t *ks, const h8_t (&qreg)[
 template <bool CAUSAL, typename S>
 __global__ __launch_bounds__(PA_THREADS, S::WGS) void prompt_attn_kernel(PromptArgs a) {
   constexpr int KS = S::KS, NB = S::NB;
-  __shared__ __align__(16) half_t ks_all[2][S::TILE];
-  __shared__ __align__(16) half_t vs_all[2][S::TILE];
+  __shared__ __align__(16) half_t tiles[2][2][S::TILE];   // K, V: two steps each
+  half_t (&ks_all)[2][S::TILE] = tiles[0];
+  half_t (&vs_all)[2][S::TILE] = tiles[1];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n = lane & 31, h = lane >> 5;
   const int rg = w / KS, sp = w % KS;   // this wave's 32 rows of the workgroup, its share of the key tiles
@@ -173,10 +176,17 @@ __global__ __launch_bounds__(PA_THREADS, S::WGS) void prompt_attn_kernel(PromptA
   }
   // (rows past the end of the prompt are outside the buffer descriptors: whatever such a row holds in LDS -- zeros from
   // this fill or an older tile's finite values -- meets an exponential that is exactly zero)
+  if (n_steps * S::STEP > T) {
 #pragma unroll
-  for (int i = 0; i < 4 * KS * NB; ++i) *reinterpret_cast<uint4 *>(&vs_all[0][0] + (threadIdx.x + PA_THREADS * i) * 8) = make_uint4(0, 0, 0, 0);
-  __syncthreads();
-  pa_tile_dma<S::STEP>(src, 0, ks_all[0], vs_all[0], w);   // (a step past the last one is fetched and never used)
+    for (int i = 0; i < 4 * KS * NB; ++i) *reinterpret_cast<uint4 *>(&vs_all[0][0] + (threadIdx.x + PA_THREADS * i) * 8) = make_uint4(0, 0, 0, 0);
+    __syncthreads();
+  }
+  const int odd = n_steps & 1;
+  pa_tile_dma<S::STEP>(src, 0, ks_all[odd], vs_all[odd], w);   // (a step past the last one is fetched and never used)
+  // The query is waited for here, with the first step.  Left to its first use, the compiler waits for it inside the loop, by a
+  // count that knows nothing of the requests above: every other step then waited for the one it had just asked for.
+#pragma unroll
+  for (int s = 0; s < 8; ++s) asm volatile("" : "+v"(qreg[s]));
   auto step = [&](int j, const half_t *ks, const half_t *vs, half_t *ks_nxt, half_t *vs_nxt) {
     const int k0 = j * S::STEP + sp * PA_BC * NB;
     wait_all_loads();   // this wave's part of step j, requested an iteration ago
@@ -204,32 +214,43 @@ __global__ __launch_bounds__(PA_THREADS, S::WGS) void prompt_attn_kernel(PromptA
     for (int i = 0; i < NB; ++i)
 #pragma unroll
       for (int r = 0; r < 16; ++r) raw = fmaxf(raw, s[i][r]);
-    float mx = fmaxf(m, raw * sl2);   // (sl2 > 0)
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    // (KS = 1: the first tile always holds key 0, which no query masks: mx is finite from then on)
+    // m is what the exponents are taken relative to: the maximum so far, or a little less.  The 64 products of a rescale (and the
+    // exchange between the lane halves) are left out while what passes m does so by less than 2^PA_SLACK and holds less than
+    // 2^-PA_SHARE of the lane's sum: a maximum's own weight is exactly one and has no rounding error, which shows where it
+    // dominates its row.  Relative error (2-norm) against 64 bits of a rescale each time / this / none, T = 1003, two key shares:
+    // N(0, 1) 2.450e-4 / 2.452e-4 / 2.535e-4, four channels of K ten times as large 2.191e-4 / 2.191e-4 / 2.395e-4 (2.461e-4 and
+    // 2.198e-4 with the sum taken before the rounding to fp16).  Time, us: T = 4099 176 / 167 / 163, 32768 8790 / 8650 / 8560 (one
+    // slow box).  (sl2 > 0; KS = 1: the first tile always holds key 0, which no query masks: m is finite from then on.)
     // Per lane on purpose: a divergent branch keeps the accumulators where they are (inactive lanes must keep their
     // values, so the products are in place under the execution mask, skipped when no lane needs them); a wave-uniform
-    // branch made the compiler copy all 64 accumulators per tile, and without a branch the 64 products are a quarter
-    // of the tile's vector instructions.
-    if (mx != m) {   // this query's maximum moved: rescale what it has added up so far
+    // branch made the compiler copy all 64 accumulators per tile.
+    raw *= sl2;
+        const float slack = fminf(fmaxf((float)(__builtin_amdgcn_frexp_expf(lsum) - PA_SHARE), 0.f), PA_SLACK);
+    const uint64_t over = __builtin_amdgcn_ballot_w64(raw > m + slack), both = over | over >> 32 | over << 32;   // a query's two lanes agree
+    if (both >> lane & 1) {
+      const float mx = fmaxf(m, fmaxf(raw, __shfl_xor(raw, 32, 64)));
       const float alpha = __builtin_amdgcn_exp2f(m - mx);   // (the bare instruction: results below 2^-126 may flush to zero)
       lsum *= alpha;
 #pragma unroll
       for (int dt = 0; dt < 4; ++dt) o[dt] *= alpha;
       m = mx;
     }
-    const float base = KS > 1 && mx == -INFINITY ? 0.f : mx;   // nothing but masked keys so far: exponentials of -inf are zero
+    const float base = KS > 1 && m == -INFINITY ? 0.f : m;   // nothing but masked keys so far: exponentials of -inf are zero
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
-      float part = 0.f;
+      // What is added up is what is multiplied: exponentials as fp16 numbers, their sum in fp32.  A weight's rounding then
+      // cancels against its share of the sum (and two are added per instruction).
       h8_t p[2];
+      float part[2];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i][r], sl2, -base));
-        part += e;
-        p[r >> 3][r & 7] = (half_t)e;
+      for (int t = 0; t < 2; ++t) {
+#pragma unroll
+        for (int r = 0; r < 8; ++r) p[t][r] = (half_t)__builtin_amdgcn_exp2f(__builtin_fmaf(s[i][8 * t + r], sl2, -base));
+        part[t] = 0.f;
+#pragma unroll
+        for (int r = 0; r < 8; r += 2) part[t] = __builtin_amdgcn_fdot2((half2_t){p[t][r], p[t][r + 1]}, (half2_t){(half_t)1, (half_t)1}, part[t], false);
       }
-      lsum += part;
+      lsum += part[0] + part[1];
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -246,45 +267,54 @@ __global__ __launch_bounds__(PA_THREADS, S::WGS) void prompt_attn_kernel(PromptA
         }
     }
   };
-  // two steps per round, so that each half works on fixed buffers; an odd count runs one step more, all of it masked
-  for (int j = 0; j < n_steps; j += 2) {
+  // two steps per round, so that each half works on fixed buffers; the odd one first (leaving the loop between the two costs
+  // copies of the accumulators)
+  if (odd) step(0, ks_all[1], vs_all[1], ks_all[0], vs_all[0]);
+  for (int j = odd; j < n_steps; j += 2) {
     step(j, ks_all[0], vs_all[0], ks_all[1], vs_all[1]);
     step(j + 1, ks_all[1], vs_all[1], ks_all[0], vs_all[0]);
   }
   wait_all_loads();   // the last request (a step nobody reads) must have landed before this workgroup's LDS can go to another
   lsum += __shfl_xor(lsum, 32, 64);
+  constexpr int OWN = 4 / KS;   // of the four 32-channel parts of the output, those that a wave brings together and stores
   if constexpr (KS > 1) {
-    // The second wave of a row group leaves (maximum, sum, output) in LDS for the first.  A lane's 64 outputs go to words
-    // 64 apart, lanes adjacent: no bank conflicts.
-    float *pool_o = reinterpret_cast<float *>(&ks_all[0][0]) + rg * 64 * 64;
-    float2 *pool_ml = reinterpret_cast<float2 *>(&vs_all[0][0]) + rg * 64;
-    static_assert(KS == 2 && (4 / KS) * 64 * 64 * 4 <= (int)sizeof(ks_all), "one sender per row group");
+    // The waves of a row group exchange bounds, sums and outputs through LDS, each for its own channels.  A lane's 16 outputs of
+    // a part go to words 64 apart, lanes adjacent: no bank conflicts.
+    static_assert(KS == 2 && PA_WAVES / KS * 4096 * 4 + PA_WAVES * 512 <= (int)sizeof(tiles), "one sender per part");
+    float *pool_o = reinterpret_cast<float *>(&tiles[0][0][0]) + rg * 4096;
+    float2 *pool_ml = reinterpret_cast<float2 *>(reinterpret_cast<float *>(&tiles[0][0][0]) + PA_WAVES / KS * 4096) + rg * KS * 64;
     __syncthreads();   // the tiles are no longer read
-    if (sp == 1) {
-      pool_ml[lane] = make_float2(m, lsum);
+    pool_ml[sp * 64 + lane] = make_float2(m, lsum);
 #pragma unroll
-      for (int i = 0; i < 64; ++i) pool_o[i * 64 + lane] = o[i >> 4][i & 15];
-    }
+    for (int dt = 0; dt < 4; ++dt)
+      if (dt / OWN != sp) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) pool_o[1024 * dt + 64 * i + lane] = o[dt][i];
+      }
     __syncthreads();
-    if (sp == 0) {   // (its tiles start with key 0: m is finite; the other's may all have been masked)
-      const float2 ml = pool_ml[lane];
-      const float mx = fmaxf(m, ml.x), ca = __builtin_amdgcn_exp2f(m - mx), cb = __builtin_amdgcn_exp2f(ml.x - mx);
-      lsum = lsum * ca + ml.y * cb;
+    const float2 ml = pool_ml[(sp ^ 1) * 64 + lane];
+    const float mx = fmaxf(m, ml.x), ca = __builtin_amdgcn_exp2f(m - mx), cb = __builtin_amdgcn_exp2f(ml.x - mx);   // (the first wave's tiles start with key 0: its m is finite)
+    lsum = lsum * ca + ml.y * cb;
 #pragma unroll
-      for (int i = 0; i < 64; ++i) o[i >> 4][i & 15] = o[i >> 4][i & 15] * ca + pool_o[i * 64 + lane] * cb;
-    }
+    for (int dt = 0; dt < 4; ++dt)
+      if (dt / OWN == sp) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[dt][i] = o[dt][i] * ca + pool_o[1024 * dt + 64 * i + lane] * cb;
+      }
   }
-  if (sp == 0 && my_q < T) {
+  if (my_q < T) {
     const float inv = 1.0f / lsum;
     half_t *orow = a.out + b * a.o_b + hq * a.o_h + (int64_t)my_q * a.o_t;
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt)
+      if (KS == 1 || dt / OWN == sp) {
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        h4_t y;
+        for (int g = 0; g < 4; ++g) {
+          h4_t y;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) y[j] = (half_t)(o[dt][4 * g + j] * inv);
-        *reinterpret_cast<h4_t *>(orow + 32 * dt + 8 * g + 4 * h) = y;
+          for (int j = 0; j < 4; ++j) y[j] = (half_t)(o[dt][4 * g + j] * inv);
+          *reinterpret_cast<h4_t *>(orow + 32 * dt + 8 * g + 4 * h) = y;
+        }
       }
   }
 }
