@@ -502,8 +502,8 @@ def decode_attention(q: torch.Tensor, pkv: tuple, mask, Tall: int, zero_init: bo
 
 class DecodePlan:
     """Pre-validated launch plan for one layer's cache: segment tables, outputs and the split-K
-    workspace are built once, so a decode step is a single C call (three kernel launches, two for
-    short caches) with no per-step Python work.  Holds references to every tensor it points into.
+    workspace are built once, so a decode step is a single C call (three kernel launches, one for
+    short caches, or two under stream capture) with no per-step Python work.  Holds references to every tensor it points into.
     """
 
     def __init__(self, q_like: torch.Tensor, pkv: tuple, mask=None, Tall: Optional[int] = None,

@@ -2176,7 +2176,7 @@ extern "C" int hqekv_pv_hybrid(const hqekv_seg *segs, int nseg, const void *p, v
 static int64_t align_up(int64_t v, int64_t a) { return (v + a - 1) / a * a; }
 
 struct DecodeLayout {  // carve-up of the caller's workspace
-  int64_t chunk, partial_bytes, stats_off, stats_bytes, arrive_off, logits_off, logits_bytes, total;
+  int64_t chunk, partial_bytes, stats_off, stats_bytes, arrive_off, logits_off, logits_bytes, records_off, pairs_off, total;
   int64_t n_stat, chunks;
 };
 
@@ -2216,6 +2216,12 @@ static int decode_layout(const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_se
   // eight heads per KV head get there: 9 x 4k tokens at eight 27.3 us in three launches, 25.7 in two; 34 x 1184 46.9 either way.)
   if (L->logits_off + L->logits_bytes > (int64_t)HQEKV_STATIC_SCRATCH_BYTES) L->logits_bytes = 0;
   L->total = L->logits_off + L->logits_bytes;
+  // ... and what one launch needs beside them, by the same rule
+  L->records_off = L->total;
+  L->pairs_off = L->records_off + align_up(B * Hq * tiles * 16, 256);
+  const int64_t one = L->pairs_off + align_up(chunks * B * Hq * D * 8, 256);
+  if (L->logits_bytes && tiles <= STEP_RECORDS && one <= (int64_t)HQEKV_STATIC_SCRATCH_BYTES) L->total = one;
+  else L->records_off = 0;
   return HQEKV_OK;
 }
 
@@ -2354,9 +2360,10 @@ static bool meet(const Stretches &a, const Stretches &b) {
   const int64_t k = std::max(x / step - (x % step < 0) + 1, -(a.n - 1));
   return k < b.n && off + k * step < a.bytes;
 }
-static bool pv_reads(const hqekv_seg *v_segs, int n_v, int64_t slabs, int64_t D, const Stretches &w) {
-  for (int k = 0; k < n_v; ++k) {
-    const hqekv_seg &s = v_segs[k];
+// (Of either side: a channel-major K class is read whole, and its slabs span as many bytes as those of V would.)
+static bool segs_meet(const hqekv_seg *segs, int nseg, int64_t slabs, int64_t D, const Stretches &w) {
+  for (int k = 0; k < nseg; ++k) {
+    const hqekv_seg &s = segs[k];
     const int64_t n = s.n_tokens, slab = s.slab_tokens > 0 ? s.slab_tokens : n, row = D * s.bits / 8, params = D / 32 * 2;
     if (n <= 0) continue;
     if (meet(w, {(uintptr_t)s.data, n * row, slabs, slab * row}) || meet(w, {(uintptr_t)s.idx, n * 8, 1, 0})) return true;
@@ -2365,10 +2372,10 @@ static bool pv_reads(const hqekv_seg *v_segs, int n_v, int64_t slabs, int64_t D,
   }
   return false;
 }
-// Does the epilogue write what p.V reads?  (A sliding window whose oldest row the step's value replaces.)
-static bool epilogue_writes_v(const StepEpilogue &e, const hqekv_seg *v_segs, int n_v, int64_t D) {
+// Does the epilogue write what a side's segments hold?  (A sliding window of V whose oldest row the step's value replaces.)
+static bool epilogue_writes(const StepEpilogue &e, const hqekv_seg *segs, int nseg, int64_t D) {
   const int64_t slabs = e.app_bh;
-  auto hit = [&](const Stretches &w) { return pv_reads(v_segs, n_v, slabs, D, w); };
+  auto hit = [&](const Stretches &w) { return segs_meet(segs, nseg, slabs, D, w); };
   if (e.ring_line && hit({(uintptr_t)e.ring_line, e.Tall * 2, 1, 0})) return true;
   if (e.app_rows > 0)
     for (int side = 0; side < 2; ++side)
@@ -2385,10 +2392,11 @@ struct DecodeRoute {
   bool covers;             // the softmax rides in the two GEMV launches
   bool in_two;             // a short step: q.K^T leaves its logits in the workspace, p.V does the rest
   bool rides;              // in_two: the epilogue rides in the p.V launch; else a launch of its own follows (same bits)
+  bool one;                // in_two: one launch does all of it, unless the stream is captured (same bits)
   TilesPlan k_plan, v_plan;
 };
-static DecodeRoute decode_route(const DecodeLayout &L, const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_segs, int n_v, bool mask, const void *attn_out,
-                                int64_t B, int64_t Hq, int64_t Hkv, int64_t D, int64_t Tall, int flags, const StepEpilogue &ep) {
+static DecodeRoute decode_route(const DecodeLayout &L, const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_segs, int n_v, bool mask, const void *q,
+                                const void *attn_weights, const void *attn_out, int64_t B, int64_t Hq, int64_t Hkv, int64_t D, int64_t Tall, int flags, const StepEpilogue &ep) {
   DecodeRoute r{};
   // The launches of decode_qk.hip and decode_pv.hip take the call unless it names a form of the older ones.
   const bool by_rule = !(flags & (HQEKV_QK_TILING(0xf) | HQEKV_DOT_MFMA | HQEKV_DOT_VALU | HQEKV_TWO_STEP_DEQUANT | HQEKV_FOLD_COMBINE |
@@ -2405,8 +2413,16 @@ static DecodeRoute decode_route(const DecodeLayout &L, const hqekv_seg *k_segs, 
   // (What rides along changes nothing about the attention, so that a step and the separate calls give the same bits.)
   r.in_two = L.logits_bytes > 0 && r.covers && r.k_tiles && r.k_plan.per_unit == 1 && r.v_tiles &&
              !(flags & (HQEKV_ONLY_QK | HQEKV_ONLY_PV | HQEKV_ONLY_COMBINE | HQEKV_ONLY_RAW_QK)) &&
-             !pv_reads(v_segs, n_v, B * Hkv, D, {(uintptr_t)attn_out, B * Hq * D * 2, 1, 0});
-  r.rides = r.in_two && pv_last_takes(ep, Tall) && !epilogue_writes_v(ep, v_segs, n_v, D);
+             !segs_meet(v_segs, n_v, B * Hkv, D, {(uintptr_t)attn_out, B * Hq * D * 2, 1, 0});
+  r.rides = r.in_two && pv_last_takes(ep, Tall) && !epilogue_writes(ep, v_segs, n_v, D);
+  // In one launch q.K^T's reads, too, stand beside p.V's writes and the epilogue's.  (A step's time in two / in one, us: the rule of
+  // decode_in_two, and step_kernel.)
+  auto qk_reads = [&](const void *p, int64_t bytes) {
+    const Stretches w{(uintptr_t)p, bytes, 1, 0};
+    return meet(w, {(uintptr_t)q, B * Hq * D * 2, 1, 0}) || segs_meet(k_segs, n_k, B * Hkv, D, w);
+  };
+  r.one = r.in_two && L.records_off > 0 && !(flags & HQEKV_TWO_LAUNCHES) && !qk_reads(attn_out, B * Hq * D * 2) &&
+          !qk_reads(attn_weights, B * Hq * Tall * 2) && !(r.rides && epilogue_writes(ep, k_segs, n_k, D));
   return r;
 }
 
@@ -2431,13 +2447,17 @@ static int decode_impl(const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_segs
   StepEpilogue ep;
   rc = fill_epilogue(extra, attn_weights, B, Hq, Hkv, D, Tall, &ep);
   if (rc) return rc;
-  const DecodeRoute r = decode_route(L, k_segs, n_k, v_segs, n_v, mask != nullptr, attn_out, B, Hq, Hkv, D, Tall, flags, ep);
+  DecodeRoute r = decode_route(L, k_segs, n_k, v_segs, n_v, mask != nullptr, q, attn_weights, attn_out, B, Hq, Hkv, D, Tall, flags, ep);
   SegTable kt{}, vt{};
   rc = build_table(k_segs, n_k, true, D, qk_tile_of(tiling), Tall, &kt, "decode_attn(K)", r.k_tiles ? &r.k_plan : nullptr);
   if (rc) return rc;
   rc = build_table(v_segs, n_v, false, D, L.chunk, Tall, &vt, "decode_attn(V)", r.v_tiles ? &r.v_plan : nullptr);
   if (rc) return rc;
   hipStream_t st = (hipStream_t)stream;
+  if (r.one) {   // a captured launch would bear the same number in every replay
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusActive;
+    if (hipStreamIsCapturing(st, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) r.one = false;
+  }
   char *ws = (char *)workspace;
   const bool fuse = r.covers && kt.total_units > 0 && vt.total_units > 0;
   FuseArgs fz{};
@@ -2455,8 +2475,11 @@ static int decode_impl(const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_segs
       riding = ep;
       riding.weights = logits;   // (the ring row's workgroups make the probabilities themselves)
     }
-    rc = launch_qk(kt, q, logits, B, Hq, Hkv, D, Tall, fz, st, tiling, false);
-    if (!rc) rc = launch_pv_last(vt, logits, attn_weights, (float *)ws, B, Hq, Hkv, Tall, fz, riding, st);
+    if (r.one)
+      rc = launch_step(kt, vt, q, logits, attn_weights, ws + L.records_off, ws + L.pairs_off, attn_out, B, Hq, Hkv, Tall, fz.inv_sqrt_d, riding,
+                       flags & HQEKV_IMPATIENT ? 0 : STEP_PATIENCE, st);
+    else rc = launch_qk(kt, q, logits, B, Hq, Hkv, D, Tall, fz, st, tiling, false);
+    if (!rc && !r.one) rc = launch_pv_last(vt, logits, attn_weights, (float *)ws, B, Hq, Hkv, Tall, fz, riding, st);
     return rc || r.rides || !has_epilogue(ep) ? rc : launch_combine(nullptr, nullptr, 0, B * Hq, D, Tall, false, &ep, st);
   }
   // Few chunks per (b, kv head) and a long p.V launch: the last p.V workgroup of each (b, kv head) adds the
@@ -2496,17 +2519,32 @@ static int decode_impl(const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_segs
   return launch_pv(vt, L.chunk, attn_weights, attn_out, (float *)ws, B, Hq, Hkv, D, Tall, fz, st, mf, stages, &ep);
 }
 
-extern "C" int hqekv_selftest_step_form(const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_segs, int n_v, const void *attn_out, int64_t B,
-                                        int64_t Hq, int64_t Hkv, int64_t D, int64_t Tall, int flags, const hqekv_step_extra *extra) {
+static int selftest_route(const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_segs, int n_v, const void *q, const void *attn_weights, const void *attn_out,
+                          int64_t B, int64_t Hq, int64_t Hkv, int64_t D, int64_t Tall, int flags, const hqekv_step_extra *extra, DecodeRoute *r, StepEpilogue *ep) {
   DecodeLayout L;
-  StepEpilogue ep;
   int rc = check_heads("selftest_step_form", B, Hq, Hkv, D);
   if (rc) return rc;
   if (decode_layout(k_segs, n_k, v_segs, n_v, B, Hq, Hkv, D, &L)) return fail(HQEKV_E_ARG, "selftest_step_form: bad segment tables");
-  rc = fill_epilogue(extra, nullptr, B, Hq, Hkv, D, Tall, &ep);
+  rc = fill_epilogue(extra, nullptr, B, Hq, Hkv, D, Tall, ep);
   if (rc) return rc;
-  const DecodeRoute r = decode_route(L, k_segs, n_k, v_segs, n_v, false, attn_out, B, Hq, Hkv, D, Tall, flags, ep);
+  *r = decode_route(L, k_segs, n_k, v_segs, n_v, false, q, attn_weights, attn_out, B, Hq, Hkv, D, Tall, flags, *ep);
+  return HQEKV_OK;
+}
+extern "C" int hqekv_selftest_step_form(const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_segs, int n_v, const void *attn_out, int64_t B,
+                                        int64_t Hq, int64_t Hkv, int64_t D, int64_t Tall, int flags, const hqekv_step_extra *extra) {
+  DecodeRoute r;
+  StepEpilogue ep;
+  const int rc = selftest_route(k_segs, n_k, v_segs, n_v, nullptr, nullptr, attn_out, B, Hq, Hkv, D, Tall, flags, extra, &r, &ep);
+  if (rc) return rc;
   return !r.in_two ? 0 : r.rides || !has_epilogue(ep) ? 1 : 2;
+}
+extern "C" int hqekv_selftest_step_one(const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_segs, int n_v, const void *q, const void *attn_weights,
+                                       const void *attn_out, int64_t B, int64_t Hq, int64_t Hkv, int64_t D, int64_t Tall, int flags,
+                                       const hqekv_step_extra *extra) {
+  DecodeRoute r;
+  StepEpilogue ep;
+  const int rc = selftest_route(k_segs, n_k, v_segs, n_v, q, attn_weights, attn_out, B, Hq, Hkv, D, Tall, flags, extra, &r, &ep);
+  return rc ? rc : r.one;
 }
 
 // ------------------------------------------------------------------ per-class GEMV on the same kernels

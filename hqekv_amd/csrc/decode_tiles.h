@@ -22,6 +22,8 @@ namespace hq {
 
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+constexpr int HQ_THROUGH = 16;   // of a buffer access: agent scope (sc1), past the L2 that the XCDs do not share
 
 __device__ __forceinline__ f4_t mfma16(u32x4 a, u32x4 b, f4_t c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, a), __builtin_bit_cast(half8_t, b), c, 0, 0, 0);
@@ -169,9 +171,16 @@ int launch_qk_tiles(const SegTable &tb, const void *q, void *scores, int64_t B, 
                     hipStream_t st);
 int launch_pv_tiles(const SegTable &tb, void *p, float *partial, int64_t B, int64_t Hq, int64_t Hkv, int64_t Tall, const FuseArgs &fz,
                     hipStream_t st);
-// Short steps: p.V, the sum of its partial rows and the step's epilogue in one launch (decode_pv.hip).
+// Short steps in two launches: p.V, the sum of its partial rows and the step's epilogue in one of them (decode_pv.hip).
 bool decode_in_two(const hqekv_seg *v_segs, int n_v, int64_t D, int64_t B, int64_t Hq, int64_t Hkv);
 bool pv_last_takes(const StepEpilogue &ep, int64_t Tall);
+int64_t pv_epilogue_blocks(const StepEpilogue &ep, int64_t Tall);   // workgroups for the epilogue
+// The same steps in one launch (decode_step.hip), with the same bits.
+constexpr int STEP_UNITS = 20;        // most p.V units (and partial rows) of a (b, kv head) of a short step
+constexpr int STEP_RECORDS = 64;      // most tiles, in one launch
+constexpr int STEP_PATIENCE = 2000;   // looks, a microsecond or so each
+int launch_step(const SegTable &kt, const SegTable &vt, const void *q, void *logits, void *probs, void *records, void *pairs, void *out,
+                int64_t B, int64_t Hq, int64_t Hkv, int64_t Tall, float inv_sqrt_d, const StepEpilogue &ep, int patience, hipStream_t st);
 int launch_pv_last(const SegTable &tb, const void *logits, void *probs, float *partial, int64_t B, int64_t Hq, int64_t Hkv, int64_t Tall,
                    const FuseArgs &fz, const StepEpilogue &ep, hipStream_t st);
 

@@ -86,8 +86,14 @@ __device__ __forceinline__ void ring_heads_to_lds(const RingShape r, ring_src_t 
     for (int u = 0; u < HU; ++u) {
       const int h = min(h0 + u * waves, r.Hq - 1);
 #pragma unroll
-      for (int b = 0; b < NB; ++b)   // 8 bytes at the alignment of an element: the target reads unaligned
-        raw[u][b] = reinterpret_cast<ring_quad_src_t>(col + (int64_t)b * bs + (int64_t)h * hs)->v >> (16 * shift);
+      for (int b = 0; b < NB; ++b) {   // 8 bytes at the alignment of an element: the target reads unaligned
+        if constexpr (std::remove_reference_t<Prob>::THROUGH) {   // (written past the L2 in this launch; below 2 GB)
+          const uint32_t at = (uint32_t)(((int64_t)b * r.Hq + h) * hs * 2) + (uint32_t)((uintptr_t)col - (uintptr_t)r.w);
+          raw[u][b] = __builtin_bit_cast(uint64_t, __builtin_amdgcn_raw_buffer_load_b64(make_rsrc((const void *)(uintptr_t)r.w, 0x7fffffffu), (int)at, 0, 16)) >> (16 * shift);
+        } else {
+          raw[u][b] = reinterpret_cast<ring_quad_src_t>(col + (int64_t)b * bs + (int64_t)h * hs)->v >> (16 * shift);
+        }
+      }
     }
 #pragma unroll
     for (int u = 0; u < HU; ++u) {
@@ -177,6 +183,7 @@ __device__ __forceinline__ void ring_row_columns(const StepEpilogue &e, int64_t 
 }
 
 struct RingAsIs {
+  static constexpr bool THROUGH = false;
   __device__ __forceinline__ uint64_t operator()(int, uint64_t quad) const { return quad; }
 };
 

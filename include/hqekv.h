@@ -293,6 +293,10 @@ int hqekv_pv_hybrid(const hqekv_seg *segs, int nseg, const void *p, void *out, i
  * and the form of the dot products the other flags name: what gemv_forward_cuda_qk_group_hq returns
  * (quant/csrc/gemv_cuda.h:78-109), for callers and tests that want the scores of one particular tiling. */
 #define HQEKV_ONLY_RAW_QK 0x2000
+/* A short step is one launch, or two while the stream is captured, with the same bits.  TWO_LAUNCHES: two in any case.
+ * IMPATIENT, for tests: the one launch's workgroups look once for what others leave them and otherwise do it themselves. */
+#define HQEKV_TWO_LAUNCHES 0x4000
+#define HQEKV_IMPATIENT 0x8000
 int64_t hqekv_decode_workspace_bytes(const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_segs, int n_v,
                                      int64_t B, int64_t Hq, int64_t Hkv, int64_t D);
 int hqekv_decode_attn(const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_segs, int n_v,
@@ -341,10 +345,16 @@ int hqekv_decode_step(const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_segs,
                       int64_t D, int64_t Tall, void *workspace, int64_t workspace_bytes, int flags,
                       void *stream, const hqekv_step_extra *extra);
 /* No counterpart in the reference: which launches that call (extra NULL: hqekv_decode_attn, without a mask) takes, for tests
- * of the rule.  0: three or more; 1: two, what `extra` asks for in the second; 2: two and one for what `extra` asks for.
+ * of the rule, while the stream is captured.  0: three or more; 1: two, what `extra` asks for in the second; 2: two and one for
+ * what `extra` asks for.
  * Pointers are compared, never followed. */
 int hqekv_selftest_step_form(const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_segs, int n_v, const void *attn_out, int64_t B,
                              int64_t Hq, int64_t Hkv, int64_t D, int64_t Tall, int flags, const hqekv_step_extra *extra);
+/* The same for one launch: 1 where such a call (`q`, `attn_weights` as it passes them) is one launch outside stream capture, with
+ * what `extra` asks for in it or in a second one as above, else 0. */
+int hqekv_selftest_step_one(const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_segs, int n_v, const void *q, const void *attn_weights,
+                            const void *attn_out, int64_t B, int64_t Hq, int64_t Hkv, int64_t D, int64_t Tall, int flags,
+                            const hqekv_step_extra *extra);
 /* The ring row alone: line[t] = rnd16(sum_h rnd16(sum_b attn_weights[b,h,t])) in torch's order (`order` as
  * ring_order above).  Replaces last_attn_weights.update for one decode row (model/public_func.py:250-254). */
 int hqekv_ring_row(const void *attn_weights, int64_t B, int64_t Hq, int64_t Tall, void *line, int order,
