@@ -44,7 +44,7 @@ LAYOUT_NORMAL1 = 2       # 1-bit segment in normal-quantile coding (scale = std,
 EXPORTS = (
     "hqekv_version", "hqekv_last_error",
     "hqekv_quant_pack_rows", "hqekv_quant_pack_k_tokenmajor", "hqekv_dequant_unpack_rows", "hqekv_pack_i32",
-    "hqekv_selftest_quant_division", "hqekv_selftest_wave_reduce", "hqekv_selftest_stream_read", "hqekv_selftest_form", "hqekv_selftest_step_form", "hqekv_selftest_step_one",
+    "hqekv_selftest_quant_division", "hqekv_selftest_wave_reduce", "hqekv_selftest_stream_read", "hqekv_selftest_form", "hqekv_selftest_step_form", "hqekv_selftest_step_one", "hqekv_selftest_last_rows",
     "hqekv_normal1_quant_pack_rows", "hqekv_normal1_quant_pack_k_tokenmajor", "hqekv_normal1_dequant_unpack_rows",
     "hqekv_gemv_workspace_bytes", "hqekv_gemv_uniform_group", "hqekv_gemv_normal_group",
     "hqekv_qk_hybrid", "hqekv_scale_softmax", "hqekv_pv_workspace_bytes", "hqekv_pv_hybrid",
@@ -148,6 +148,7 @@ _PROTOS = {
     "hqekv_rank_blocks": (C.c_int, [_vp, _int, _i64, _vp, _vp]),
     "hqekv_prompt_attn": (C.c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, C.c_float, _int, _vp]),
     "hqekv_prompt_last_rows": (C.c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, C.c_float, _vp, _i64, _vp]),
+    "hqekv_selftest_last_rows": (C.c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, C.c_float, _vp, _i64, _int, _vp]),
     "hqekv_prompt_last_rows_workspace_bytes": (_i64, [_i64, _i64, _i64]),
     "hqekv_cache_reconstruct": (C.c_int, [_SEGP, _int, _SEGP, _int, _vp, _vp, _i64, _i64, _i64, _vp]),
     "hqekv_cover_once": (C.c_int, [_vp, _vp, _int, _vp, _i64, _vp]),

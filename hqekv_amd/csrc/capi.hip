@@ -1,6 +1,9 @@
 // Error bookkeeping shared by every entry point of libhqekv.
 #include <stdarg.h>
 #include <stdio.h>
+#include <atomic>
+#include <chrono>
+#include <random>
 
 #include "common.h"
 
@@ -21,6 +24,11 @@ int check_launch(const char *what) {
   if (e == hipSuccess) return HQEKV_OK;
   snprintf(g_err, sizeof(g_err), "%s: %s", what, hipGetErrorString(e));
   return (int)e;
+}
+
+uint64_t launch_number() {
+  static std::atomic<uint64_t> next{std::random_device{}() * 0x9e3779b97f4a7c15ull ^ (uint64_t)std::chrono::steady_clock::now().time_since_epoch().count()};
+  return next.fetch_add(1, std::memory_order_relaxed);
 }
 
 }  // namespace hq

@@ -17,6 +17,11 @@ namespace hq {
 int fail(int code, const char *fmt, ...);
 int check_launch(const char *what);
 
+// What a launch tags the records with that its workgroups leave for one another: no other launch of the process has it, and 64
+// bits that begin anywhere are not what lies in memory by chance.
+uint64_t launch_number();
+constexpr int STEP_PATIENCE = 2000;   // looks at a record, a microsecond or so each, before a workgroup does the missing work itself
+
 // Which variant of a kernel a call of these sizes takes (the rules stand beside the launches; hqekv_selftest_form).
 struct PromptForm { int key_shares, tiles; bool reversed; };   // PaShape's
 PromptForm prompt_form(int64_t T, int64_t BH);
@@ -92,6 +97,8 @@ __device__ __forceinline__ uint32_t by_xcd(uint32_t i, uint32_t n) {
 // that never changes, and the row offset in a scalar register -- no vector ALU work per load, and reads
 // past the end of the slab return zero instead of faulting.
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+constexpr int HQ_THROUGH = 16;   // of a buffer access: agent scope (sc1), past the L2 that the XCDs do not share
 __device__ __forceinline__ rsrc_t make_rsrc(const void *base, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int)bytes, 0x00020000);
 }

@@ -1,8 +1,4 @@
 // A whole short decode step in one launch (see decode_tiles.h).
-#include <atomic>
-#include <chrono>
-#include <random>
-
 #include "decode_pv_tile.h"
 #include "decode_qk_tile.h"
 
@@ -351,11 +347,6 @@ __global__ __launch_bounds__(PT_WAVES * 64, HP == 4 ? 5 : 4) void step_kernel(u3
 }
 
 // =============================================================================== host side
-static uint64_t launch_number() {
-  static std::atomic<uint64_t> next{std::random_device{}() * 0x9e3779b97f4a7c15ull ^ (uint64_t)std::chrono::steady_clock::now().time_since_epoch().count()};
-  return next.fetch_add(1, std::memory_order_relaxed);
-}
-
 int launch_step(const SegTable &kt, const SegTable &vt, const void *q, void *logits, void *probs, void *records, void *pairs, void *out,
                 int64_t B, int64_t Hq, int64_t Hkv, int64_t Tall, float inv_sqrt_d, const StepEpilogue &ep, int patience, hipStream_t st) {
   const TilesHost k = tiles_host(kt, Hq, Hkv), v = tiles_host(vt, Hq, Hkv);

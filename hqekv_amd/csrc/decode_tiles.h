@@ -21,9 +21,7 @@
 namespace hq {
 
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-constexpr int HQ_THROUGH = 16;   // of a buffer access: agent scope (sc1), past the L2 that the XCDs do not share
 
 __device__ __forceinline__ f4_t mfma16(u32x4 a, u32x4 b, f4_t c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, a), __builtin_bit_cast(half8_t, b), c, 0, 0, 0);
@@ -178,7 +176,6 @@ int64_t pv_epilogue_blocks(const StepEpilogue &ep, int64_t Tall);   // workgroup
 // The same steps in one launch (decode_step.hip), with the same bits.
 constexpr int STEP_UNITS = 20;        // most p.V units (and partial rows) of a (b, kv head) of a short step
 constexpr int STEP_RECORDS = 64;      // most tiles, in one launch
-constexpr int STEP_PATIENCE = 2000;   // looks, a microsecond or so each
 int launch_step(const SegTable &kt, const SegTable &vt, const void *q, void *logits, void *probs, void *records, void *pairs, void *out,
                 int64_t B, int64_t Hq, int64_t Hkv, int64_t Tall, float inv_sqrt_d, const StepEpilogue &ep, int patience, hipStream_t st);
 int launch_pv_last(const SegTable &tb, const void *logits, void *probs, float *partial, int64_t B, int64_t Hq, int64_t Hkv, int64_t Tall,

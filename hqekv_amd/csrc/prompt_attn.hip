@@ -374,27 +374,28 @@ __device__ __forceinline__ void lr_tile_stats(const half_t (&x)[16], float &m, f
   m = mx;
 }
 // over the two halves of every wave, then the waves: afterwards every thread holds column n's pair
-template <int WAVES>
-__device__ __forceinline__ void lr_merge(float &m, float &l, int n, int h, int w, float (&sh_m)[WAVES][32], float (&sh_l)[WAVES][32]) {
+// (`at(k)`: 32 pairs of LDS for wave k)
+template <int WAVES, typename At>
+__device__ __forceinline__ void lr_merge(float &m, float &l, int n, int h, int w, At at) {
   const float mo = __shfl_xor(m, 32, 64), lo = __shfl_xor(l, 32, 64);
   const float mx = fmaxf(m, mo);
   l = (m == -INFINITY ? 0.f : l * __expf(m - mx)) + (mo == -INFINITY ? 0.f : lo * __expf(mo - mx));
-  if (h == 0) {
-    sh_m[w][n] = mx;
-    sh_l[w][n] = l;
-  }
+  if (h == 0) at(w)[n] = make_float2(mx, l);
   __syncthreads();
+  float2 v[WAVES];
+#pragma unroll
+  for (int k = 0; k < WAVES; ++k) v[k] = at(k)[n];
   m = -INFINITY;
 #pragma unroll
-  for (int k = 0; k < WAVES; ++k) m = fmaxf(m, sh_m[k][n]);
+  for (int k = 0; k < WAVES; ++k) m = fmaxf(m, v[k].x);
   l = 0.f;
 #pragma unroll
-  for (int k = 0; k < WAVES; ++k) l += sh_m[k][n] == -INFINITY ? 0.f : sh_l[k][n] * __expf(sh_m[k][n] - m);
+  for (int k = 0; k < WAVES; ++k) l += v[k].x == -INFINITY ? 0.f : v[k].y * __expf(v[k].x - m);
 }
 
 // Without room for the slices' statistics: one workgroup per (b, query head) walks all keys twice.
 __global__ __launch_bounds__(PA_THREADS, 2) void prompt_last_rows_kernel(LastRowsArgs a) {
-  __shared__ float sh_m[PA_WAVES][32], sh_l[PA_WAVES][32];
+  __shared__ float2 sh_ml[PA_WAVES][32];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n = lane & 31, h = lane >> 5;
   const int b = (int)blockIdx.x / a.Hq, hq = (int)blockIdx.x % a.Hq, hkv = hq / (a.Hq / a.Hkv);
@@ -424,7 +425,7 @@ __global__ __launch_bounds__(PA_THREADS, 2) void prompt_last_rows_kernel(LastRow
     tile_logits(tile, x);
     lr_tile_stats(x, m, l);
   }
-  lr_merge(m, l, n, h, w, sh_m, sh_l);
+  lr_merge<PA_WAVES>(m, l, n, h, w, [&](int k) { return sh_ml[k]; });
   const float inv = 1.0f / l;
   half_t *prow = a.probs + (((int64_t)b * a.Hq + hq) * R + row) * (int64_t)T;
   for (int tile = w; tile < n_tiles; tile += PA_WAVES) {
@@ -457,7 +458,7 @@ template <int WAVES>
 __global__ __launch_bounds__(WAVES * 64, 1) void prompt_last_short_kernel(LastRowsArgs a) {
   __shared__ __align__(16) half_t sh_k[WAVES][32 * PA_D];
   __shared__ __align__(16) half_t sh_q[32 * PA_D];
-  __shared__ float sh_m[WAVES][32], sh_l[WAVES][32];
+  __shared__ float2 sh_ml[WAVES][32];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n = lane & 31, h = lane >> 5, r4 = lane >> 4, piece = lane & 15;   // (a load takes four rows)
   const int b = (int)blockIdx.x / a.Hkv, hkv = (int)blockIdx.x % a.Hkv;
@@ -494,7 +495,7 @@ __global__ __launch_bounds__(WAVES * 64, 1) void prompt_last_short_kernel(LastRo
   float m = -INFINITY, l = 0.f;
   lr_logits(a, s, mrow, w, h, T - R + row, x);   // (a tile past the last one: no key is visible)
   lr_tile_stats(x, m, l);
-  lr_merge(m, l, n, h, w, sh_m, sh_l);
+  lr_merge<WAVES>(m, l, n, h, w, [&](int k) { return sh_ml[k]; });
   if (!live) return;
   const float inv = 1.0f / l;
   half_t *prow = a.probs + (((int64_t)b * a.Hq + hq) * R + row) * (int64_t)T;
@@ -516,7 +517,7 @@ __global__ __launch_bounds__(WAVES * 64, 1) void prompt_last_short_kernel(LastRo
   }
 }
 
-// With room for the slices' statistics, two launches.  Bound: HBM (K once, the rows' probabilities twice through the memory-side cache).
+// With room for the slices' statistics and many keys, two launches.  Bound: HBM (K once, the rows' probabilities twice through the memory-side cache).
 // prompt_last_logits_kernel: the R rows of all query heads of a KV head lie side by side as columns of 32-column tiles
 // (4 heads x 20 rows: three tiles instead of four that are 3/8 empty); a workgroup takes one column tile and one slice of
 // the keys, leaves the logits where the probabilities will be -- four keys of a row per 8-byte store -- and the slice's
@@ -528,7 +529,7 @@ __global__ __launch_bounds__(WAVES * 64, 1) void prompt_last_short_kernel(LastRo
 __global__ __launch_bounds__(PA_THREADS, 3) void prompt_last_logits_kernel(LastRowsArgs a) {
   __shared__ __align__(16) half_t sh_k[PA_WAVES][32 * PA_D];
   __shared__ __align__(16) half_t sh_q[32 * PA_D];
-  __shared__ float sh_m[PA_WAVES][32], sh_l[PA_WAVES][32];
+  __shared__ float2 sh_ml[PA_WAVES][32];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n = lane & 31, h = lane >> 5, r4 = lane >> 4, piece = lane & 15;   // (a load takes four rows)
   const int b = (int)blockIdx.x / a.Hkv, hkv = (int)blockIdx.x % a.Hkv;
@@ -594,8 +595,166 @@ __global__ __launch_bounds__(PA_THREADS, 3) void prompt_last_logits_kernel(LastR
       }
     }
   }
-  lr_merge(m, l, n, h, w, sh_m, sh_l);
+  lr_merge<PA_WAVES>(m, l, n, h, w, [&](int k) { return sh_ml[k]; });
   if (threadIdx.x < 32 && live) a.partial[((int64_t)b * a.Hq + hq) * R * a.slices + (int64_t)row * a.slices + blockIdx.y] = make_float2(m, l);
+}
+
+// The same in one launch where a slice is one tile for each wave: the logits stay in registers, and a workgroup takes the rows'
+// statistics from the records that its slices' workgroups leave beside the launch's number (as in decode_step.hip: nothing has
+// to be cleared, memory without this number is not ready).  A workgroup that has looked `patience` times leaves every record of
+// its column tile itself -- the same instructions on the same operands, hence the same bits -- so that nobody depends on being
+// scheduled beside others; workgroups that wait for one another are neighbours in the grid, within 8 * 48 of each other.  The same
+// bits as in two launches, too: slices, tiles and sums are theirs.
+// Bound: one chain of 6 us at 1003 keys (8.3 in two launches) -- entry, K and query rows, products, statistics across the waves,
+// records written and seen, probabilities -- and for longer prompts what its looks read past the L2.  The records of 32 columns
+// lie side by side: one store per workgroup, one load per thread and eight slices (rows' records apart, a slice per lane: 8.1 us
+// at 1003 keys, 24.5 instead of 12.2 at 4099).  A longer sleep between looks costs 0.3 us and more at 1003 keys and gains nothing.
+struct LastOnceArgs {
+  u32x4 *records;       // (B * Hkv, column tiles, slices, 32): (maximum, number, sum, number)
+  uint32_t lo, hi;      // the launch's number
+  int32_t patience;
+  int32_t near;         // slabs side by side in the grid, then slices
+};
+// A wave's corner of LDS: its keys, then statistics (40 KB in all: four workgroups per CU).
+union LastOnceCorner {
+  half_t __attribute__((aligned(16))) k[32 * PA_D];
+  struct {
+    float2 wave[32], row[8];   // of its tile; of columns 8 w ... + 7, (maximum, 1 / sum)
+    int seen;
+  } after;
+  __device__ LastOnceCorner() {}
+};
+template <int G>   // up to 8 G slices
+__global__ __launch_bounds__(PA_THREADS, 4) void prompt_last_once_kernel(LastRowsArgs a, LastOnceArgs o) {
+  __shared__ LastOnceCorner corner[PA_WAVES];
+  __shared__ __align__(16) half_t sh_q[32 * PA_D];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n = lane & 31, h = lane >> 5, r4 = lane >> 4, piece = lane & 15;   // (a load takes four rows)
+  const int own = (int)blockIdx.x / o.near, bh = (int)blockIdx.y * o.near + (int)blockIdx.x % o.near;
+  const int b = bh / a.Hkv, hkv = bh % a.Hkv;
+  const int T = a.T, R = a.R, nrep = a.Hq / a.Hkv, slices = a.slices;
+  const int all_tiles = (T + 31) / 32, per_slice = (all_tiles + slices - 1) / slices;   // (up to PA_WAVES)
+  const int col0 = 32 * (int)blockIdx.z, columns = nrep * R;
+  const half_t *kp = a.k + b * a.k_b + hkv * a.k_h + 8 * piece;
+  const int64_t row0 = ((int64_t)b * a.Hq + hkv * nrep) * R;   // column c of the KV head is row row0 + c of (B * Hq, R)
+  const rsrc_t records = make_rsrc(o.records + (int64_t)(bh * (int)gridDim.z + (int)blockIdx.z) * slices * 32, (uint32_t)slices * 512u);
+  half_t *ks = corner[w].k;
+  const int col = min(col0 + n, columns - 1);                  // (query head of the group, row); columns past the last one repeat it
+  const bool live = col0 + n < columns;                        // and store nothing
+  const int row = col % R;
+  const half_t *mrow = a.mask ? a.mask + b * a.m_b + (int64_t)row * a.m_r : nullptr;
+  bool q_there = false;
+  half_t x[16];
+  auto slice = [&](int i, half_t (&y)[16]) {   // the logits of this wave's tile of a slice; the slice's record
+    const int tile = w < per_slice ? i * per_slice + w : all_tiles;   // (past the last one: no key is visible)
+    h8_t k[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) k[j] = *reinterpret_cast<const h8_t *>(kp + (int64_t)min(32 * tile + 4 * j + r4, T - 1) * a.k_t);
+    if (!q_there) {
+      const half_t *qp = a.q + b * a.q_b + hkv * nrep * a.q_h + 8 * piece;
+      h8_t q[2];
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int c = min(col0 + 4 * (PA_WAVES * j + w) + r4, columns - 1);
+        q[j] = *reinterpret_cast<const h8_t *>(qp + (c / R) * a.q_h + (int64_t)(T - R + c % R) * a.q_t);
+      }
+#pragma unroll
+      for (int j = 0; j < 2; ++j) *reinterpret_cast<h8_t *>(sh_q + ls_piece(4 * (PA_WAVES * j + w) + r4, piece)) = q[j];
+      q_there = true;
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) *reinterpret_cast<h8_t *>(ks + ls_piece(4 * j + r4, piece)) = k[j];
+    __syncthreads();
+    f16_t s = (f16_t)(0.f);
+#pragma unroll
+    for (int st = 0; st < 8; ++st)
+      s = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const h8_t *>(ks + ls_piece(n, 2 * st + h)),
+                                                 *reinterpret_cast<const h8_t *>(sh_q + ls_piece(n, 2 * st + h)), s, 0, 0, 0);
+    float m = -INFINITY, l = 0.f;
+    lr_logits(a, s, mrow, tile, h, T - R + row, y);
+    lr_tile_stats(y, m, l);
+    lr_merge<PA_WAVES>(m, l, n, h, w, [&](int k) { return corner[k].after.wave; });
+    if (threadIdx.x < 32)
+      __builtin_amdgcn_raw_buffer_store_b128((u32x4){__builtin_bit_cast(uint32_t, m), o.lo, __builtin_bit_cast(uint32_t, l), o.hi}, records, (32 * i + n) * 16, 0,
+                                             HQ_THROUGH);
+  };
+  // Eight lanes merge a column's records, in the order of wave_sum, which prompt_last_probs_kernel takes.
+  auto merge = [&](int patience) {
+    const int c = (int)threadIdx.x >> 3, l8 = lane & 7;
+    u32x4 rec[G];
+    for (int look = 0;; ++look) {
+      bool ready = true;
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+        if (g == 0 || 8 * g < slices)
+          rec[g] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(records, (32 * min(l8 + 8 * g, slices - 1) + c) * 16, 0, HQ_THROUGH));
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+        if (g == 0 || 8 * g < slices) ready = ready && rec[g][1] == o.lo && rec[g][3] == o.hi;
+      if (__builtin_amdgcn_ballot_w64(!ready) == 0) break;
+      if (look >= patience) return false;
+      __builtin_amdgcn_s_sleep(2);
+    }
+    float vm[G], m = -INFINITY, part[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      const uint32_t rm = g == 0 || 8 * g < slices ? rec[g][0] : 0u;   // (bit_cast of a vector's element reads its first)
+      vm[g] = l8 + 8 * g < slices ? __builtin_bit_cast(float, rm) : -INFINITY;
+      m = fmaxf(m, vm[g]);
+    }
+#pragma unroll
+    for (int k = 1; k < 8; k *= 2) m = fmaxf(m, __shfl_xor(m, k, 64));
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      if (g && 8 * g >= slices) break;
+      const uint32_t rl = rec[g][2];
+      part[g] = vm[g] == -INFINITY ? 0.f : __builtin_bit_cast(float, rl) * __expf(vm[g] - m);
+#pragma unroll
+      for (int k = 1; k < 8; k *= 2) part[g] += __shfl_xor(part[g], k, 64);
+    }
+    const float l = ((part[0] + part[1]) + (part[2] + part[3])) + ((part[4] + part[5]) + (part[6] + part[7]));
+    if (l8 == 0) corner[w].after.row[lane >> 3] = make_float2(m, 1.0f / l);
+    return true;
+  };
+  slice(own, x);
+  {
+    const bool there = merge(o.patience);
+    if (lane == 0) corner[w].after.seen = there;
+  }
+  __syncthreads();
+  if (!(corner[0].after.seen && corner[1].after.seen && corner[2].after.seen && corner[3].after.seen)) {
+#pragma unroll 1
+    for (int i = 0; i < slices; ++i) {
+      half_t y[16];
+      __syncthreads();   // (the last slice's tiles and statistics have been read)
+      slice(i, y);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    merge(0);   // (its own records, in memory by now)
+    __syncthreads();
+  }
+  if (!live) return;
+  const float m = corner[n >> 3].after.row[n & 7].x, inv = corner[n >> 3].after.row[n & 7].y;
+  const int key0 = 32 * (own * per_slice + w);
+  if (w >= per_slice) return;
+  half_t *prow = a.probs + (row0 + col) * (int64_t)T;
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    const int key = key0 + 8 * g + 4 * h;
+    half_t p[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) p[j] = (half_t)(__expf((float)x[4 * g + j] - m) * inv);
+    if (key + 3 < T) {
+      lr_quad_t y;
+      __builtin_memcpy(&y, p, 8);
+      *reinterpret_cast<lr_quad_t *>(prow + key) = y;
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (key + j < T) prow[key + j] = p[j];
+    }
+  }
 }
 
 constexpr int LR_SPAN = 2048;   // probabilities of one row per workgroup: 256 lanes x 8
@@ -718,16 +877,24 @@ static int last_rows_slices(int64_t B, int64_t Hq, int64_t T) {
   return T <= LS_KEYS || B * Hq * 32 > 65535 ? 1 : (int)s;
 }
 
+// One launch where a slice is a tile per wave, up to 30 000 (workgroup, slice) pairs: each time all of them look, that is 15 MB of
+// records past the L2, and by then workgroups that wait keep others from beginning.  Two launches / one, us (20 rows, back to back;
+// heads over KV heads, tokens, pairs in thousands): 32/8 600 0.6 7.8 / 5.6, 1003 1.5 8.3 / 5.9, 2048 6 9.6 / 7.4, 3000 14 11.8 / 8.7,
+// 4099 26 15.0 / 12.2, 5460 44 16.7 / 17.3, 6144 55 16.2 / 18.5; 32/32 4099 35 16.3 / 18.2; 40/8 4099 35 17.5 / 17.2; 64/64 3000 37
+// 19.7 / 20.0; 40/8 3800 29 15.4 / 12.3; B = 2 32/8 1003 3 10.2 / 7.1, 3000 28 16.9 / 14.9; B = 4 1003 6 13.4 / 8.7; B = 8 768 7
+// 18.4 / 12.5.
+constexpr int LO_SLICES = 48, LO_PAIRS = 30000;
+static bool last_rows_once(int64_t T, int sl) { return sl > 1 && sl <= LO_SLICES && (T + 31) / 32 <= (int64_t)PA_WAVES * sl; }
+
 extern "C" int64_t hqekv_prompt_last_rows_workspace_bytes(int64_t B, int64_t Hq, int64_t T) {
   if (B <= 0 || Hq <= 0 || T <= 0) return -1;
   const int sl = last_rows_slices(B, Hq, T);
-  return sl > 1 ? B * Hq * sl * 32 * (int64_t)sizeof(float2) : 0;
+  return sl > 1 ? B * Hq * sl * 32 * (int64_t)(last_rows_once(T, sl) ? sizeof(u32x4) : sizeof(float2)) : 0;
 }
 
-extern "C" int hqekv_prompt_last_rows(const void *q, const int64_t *q_strides, const void *k, const int64_t *k_strides,
-                                      const void *mask, const int64_t *mask_strides, void *probs, int64_t B, int64_t Hq,
-                                      int64_t Hkv, int64_t T, int64_t D, int64_t R, float scale, void *workspace,
-                                      int64_t workspace_bytes, void *stream) {
+static int last_rows(const void *q, const int64_t *q_strides, const void *k, const int64_t *k_strides, const void *mask,
+                     const int64_t *mask_strides, void *probs, int64_t B, int64_t Hq, int64_t Hkv, int64_t T, int64_t D, int64_t R, float scale,
+                     void *workspace, int64_t workspace_bytes, int patience, void *stream) {
   if (!q || !k || !probs || !q_strides || !k_strides || (mask && !mask_strides)) return fail(HQEKV_E_ARG, "prompt_last_rows: null pointer");
   if (B <= 0 || Hq <= 0 || Hkv <= 0 || T <= 0 || Hq % Hkv || R <= 0 || R > 32 || R > T)
     return fail(HQEKV_E_ARG, "prompt_last_rows: need B > 0, Hq %% Hkv == 0 and 0 < R <= min(32, T)");
@@ -756,14 +923,33 @@ extern "C" int hqekv_prompt_last_rows(const void *q, const int64_t *q_strides, c
   }
   // the keys in slices when the caller brought room for the slices' statistics; else one workgroup per head
   const int sl = last_rows_slices(B, Hq, T);
-  const int64_t need = hqekv_prompt_last_rows_workspace_bytes(B, Hq, T);
+  const int64_t need = B * Hq * sl * 32 * (int64_t)sizeof(float2);
   if (sl > 1 && workspace && workspace_bytes >= need) {
     if ((uintptr_t)workspace & 7) return fail(HQEKV_E_ALIGN, "prompt_last_rows: workspace not 8-byte aligned");
-    a.partial = (float2 *)workspace;
     a.slices = sl;
-    const int64_t nrep = Hq / Hkv;
-    hipLaunchKernelGGL(prompt_last_logits_kernel, dim3((unsigned)(B * Hkv), (unsigned)sl, (unsigned)((nrep * R + 31) / 32)), dim3(PA_THREADS), 0,
-                       (hipStream_t)stream, a);
+    const dim3 grid((unsigned)(B * Hkv), (unsigned)sl, (unsigned)columns);
+    bool once = last_rows_once(T, sl) && B * Hkv * columns * sl * sl <= LO_PAIRS && patience >= 0 && workspace_bytes >= 2 * need &&
+                ((uintptr_t)workspace & 15) == 0;
+    if (once) {   // (a captured launch would bear the same number in every replay)
+      hipStreamCaptureStatus capture = hipStreamCaptureStatusActive;
+      once = hipStreamIsCapturing((hipStream_t)stream, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone;
+    }
+    if (once) {
+      a.partial = nullptr;
+      const int near = B * Hkv % 8 ? 1 : 8;
+      const dim3 by_slice((unsigned)(sl * near), (unsigned)(B * Hkv / near), (unsigned)columns);
+      const uint64_t number = launch_number();
+      const LastOnceArgs o{(u32x4 *)workspace, (uint32_t)number, (uint32_t)(number >> 32), patience, near};
+#define LAUNCH(G_) hipLaunchKernelGGL(prompt_last_once_kernel<G_>, by_slice, dim3(PA_THREADS), 0, (hipStream_t)stream, a, o)
+      if (sl <= 8) LAUNCH(1);
+      else if (sl <= 16) LAUNCH(2);
+      else if (sl <= 24) LAUNCH(3);
+      else LAUNCH(6);
+#undef LAUNCH
+      return check_launch("prompt_last_rows");
+    }
+    a.partial = (float2 *)workspace;
+    hipLaunchKernelGGL(prompt_last_logits_kernel, grid, dim3(PA_THREADS), 0, (hipStream_t)stream, a);
     hipLaunchKernelGGL(prompt_last_probs_kernel, dim3((unsigned)((T + LR_SPAN - 1) / LR_SPAN), (unsigned)(B * Hq * R)), dim3(PA_THREADS), 0,
                        (hipStream_t)stream, a);
   } else {
@@ -772,4 +958,17 @@ extern "C" int hqekv_prompt_last_rows(const void *q, const int64_t *q_strides, c
     hipLaunchKernelGGL(prompt_last_rows_kernel, dim3((unsigned)(B * Hq)), dim3(PA_THREADS), 0, (hipStream_t)stream, a);
   }
   return check_launch("prompt_last_rows");
+}
+
+extern "C" int hqekv_prompt_last_rows(const void *q, const int64_t *q_strides, const void *k, const int64_t *k_strides,
+                                      const void *mask, const int64_t *mask_strides, void *probs, int64_t B, int64_t Hq,
+                                      int64_t Hkv, int64_t T, int64_t D, int64_t R, float scale, void *workspace,
+                                      int64_t workspace_bytes, void *stream) {
+  return last_rows(q, q_strides, k, k_strides, mask, mask_strides, probs, B, Hq, Hkv, T, D, R, scale, workspace, workspace_bytes, STEP_PATIENCE, stream);
+}
+extern "C" int hqekv_selftest_last_rows(const void *q, const int64_t *q_strides, const void *k, const int64_t *k_strides,
+                                        const void *mask, const int64_t *mask_strides, void *probs, int64_t B, int64_t Hq,
+                                        int64_t Hkv, int64_t T, int64_t D, int64_t R, float scale, void *workspace,
+                                        int64_t workspace_bytes, int patience, void *stream) {
+  return last_rows(q, q_strides, k, k_strides, mask, mask_strides, probs, B, Hq, Hkv, T, D, R, scale, workspace, workspace_bytes, patience, stream);
 }

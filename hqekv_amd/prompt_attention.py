@@ -55,7 +55,7 @@ def prompt_last_rows(q: torch.Tensor, k: torch.Tensor, scaling: float, rows: int
                      attention_mask: Optional[torch.Tensor] = None, sliced: bool = True) -> torch.Tensor:
     """Probabilities of the last ``rows`` query rows over all keys -> (B, Hq, rows, T) fp16, with the reference's
     roundings.  ``attention_mask``: additive (B or 1, 1, >= rows, T), its last ``rows`` rows are used; None: causal.
-    ``sliced``: let the library cut the keys into slices over more workgroups (two launches) when there are few heads."""
+    ``sliced``: let the library cut the keys into slices over more workgroups when there are few heads."""
     if not supported(q, k):
         raise NotImplementedError("prompt_last_rows: fp16 CUDA tensors of head_dim 128 only")
     if attention_mask is None and sliced:

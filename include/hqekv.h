@@ -410,8 +410,10 @@ int hqekv_rank_blocks(const void *const *scores, int rows, int64_t n, int32_t *o
  *                           at -65504, softmax in fp32, to fp16.  mask: additive fp16 (B, 1, R, T) given by its batch
  *                           and row strides (key stride 1), or NULL for the causal rule (row r sees keys <= T - R + r).
  *                           workspace (hqekv_prompt_last_rows_workspace_bytes, may be 0): room for per-slice statistics,
- *                           with which few heads are spread over the chip in two launches; NULL: one workgroup per head.
- *                           Up to 512 keys one launch either way.
+ *                           with which few heads are spread over the chip; NULL: one workgroup per head.  Up to 512 keys one
+ *                           launch either way; with a workspace (16-byte aligned, of the full size) one launch, too, for up to
+ *                           some thousands of keys, else two: also with the stream being captured, or with half the size.
+ *                           The same bits.
  */
 int hqekv_prompt_attn(const void *q, const int64_t *q_strides, const void *k, const int64_t *k_strides, const void *v,
                       const int64_t *v_strides, void *out, const int64_t *out_strides, int64_t B, int64_t Hq, int64_t Hkv,
@@ -421,6 +423,12 @@ int hqekv_prompt_last_rows(const void *q, const int64_t *q_strides, const void *
                            const void *mask, const int64_t *mask_strides, void *probs, int64_t B, int64_t Hq, int64_t Hkv,
                            int64_t T, int64_t D, int64_t R, float scale, void *workspace, int64_t workspace_bytes,
                            void *stream);
+/* The same, for tests, with the number of looks that a workgroup of the one launch takes at what it waits for before it does it
+ * itself (below zero: two launches). */
+int hqekv_selftest_last_rows(const void *q, const int64_t *q_strides, const void *k, const int64_t *k_strides,
+                             const void *mask, const int64_t *mask_strides, void *probs, int64_t B, int64_t Hq, int64_t Hkv,
+                             int64_t T, int64_t D, int64_t R, float scale, void *workspace, int64_t workspace_bytes,
+                             int patience, void *stream);
 
 /* ------------------------------------------------------------------ cache maintenance (one launch per side)
  * Replaces the per-(source, target) gathers, dequantise / re-quantise calls and torch.cat re-copies of one
