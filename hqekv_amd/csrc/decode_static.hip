@@ -52,7 +52,7 @@ extern "C" int hqekv_decode_attn_static(const hqekv_seg *k_segs, int n_k, const 
   void *ws = nullptr;
   const int rc = scratch_address(&ws);
   if (rc) return rc;
-  // every part of the workspace is written before it is read within one call, so nothing has to be cleared
+  // what a call reads of the workspace it has written, or it knows it by the launch's number: nothing has to be cleared
   return hqekv_decode_attn(k_segs, n_k, v_segs, n_v, q, mask, mask_row_stride, attn_weights, attn_out, B, Hq, Hkv, D,
                            Tall, ws, (int64_t)HQEKV_STATIC_SCRATCH_BYTES, flags, stream);
 }

@@ -28,10 +28,10 @@ constexpr int PA_BC = 32;              // keys per score tile
 constexpr float PA_SLACK = 8.f;        // powers of two
 constexpr int PA_SHARE = 4;
 // How the four waves of a workgroup share its work, and how many keys a wave takes at a time.
-// <1, 1>: 32 query rows each, 128 per workgroup, every wave walks all key tiles (164 registers, 32 KB of LDS: three
+// <1, 1>: 32 query rows each, 128 per workgroup, every wave walks all key tiles (154 registers, 32 KB of LDS: three
 // workgroups per CU).  For long prompts, which are bound by the chip's power: no order of the same instructions is faster.
 // <1, 2>: the same with 64 keys per step, two workgroups per CU.  A short prompt waits for its longest walk: a lone wave needs
-// 0.77 us for 32 keys and 1.2 us for 64 (one barrier, one maximum across the lane halves, one test of the rescale; the second
+// 0.63 us for 32 keys and 1.15 us for 64 (one barrier, one maximum across the lane halves, one test of the rescale; the second
 // tile's products run beside the first one's exponentials).
 // <2, 1>: the two waves of 32 query rows deal the key tiles among themselves and merge their maxima, sums and outputs at the
 // end: walks of half the length in twice as many workgroups.  A step stages two tiles, so LDS holds two workgroups per CU.
@@ -806,15 +806,14 @@ static bool rows_16_byte_aligned(const void *p, int64_t s0, int64_t s1, int64_t 
   return ((uintptr_t)p & 15) == 0 && s0 % 8 == 0 && s1 % 8 == 0 && s2 % 8 == 0;
 }
 
-// Which form, by the number of 128-row workgroups.  Up to 400 (B = 1 and 32 heads: T up to 1600) two waves per row group: 256
-// (T = 1003) 22.3 us against 25.3 of <1, 2> and 31.5 of <1, 1>, 384 (1500) 37.2 / 37.7 / 44.1; at 480 (1800) 49.3 / 46.4 /
-// 52.6.  Up to 1500 64 keys per step: 512 (2048) 53.2 against 60.5 of <1, 1>, 672 (28 heads over 4, 3000) 84.5 / 93.1, 1056
-// (4099) 165.9 / 171, 1376 (5500) 274 / 288; beyond it is behind: 2048 (8192) 580 / 573, 4128 (16384) 2218 / 2163.
-// Four waves per row group never won (T = 500: 20.0 against 12.6 us).
-// The opposite order of the second 256 workgroups: of the 64-key form always, us without / with it: 416 workgroups (T = 1632)
-// 41.2 / 40.5, 512 53.2 / 52.2, 768 (3000) 94.5 / 92.9, 1056 (4099) 166.7 / 161.9, 1376 (5500) 265.8 / 265.6.  Walks of half the
-// length gain from it past two and a half rounds only: 320 workgroups (T = 478, 40 heads) 13.6 / 14.0, 608 (1200) 27.3 / 27.6, 728
-// (777, B = 2, 28 heads) 26.4 / 25.5, 768 (1500) 36.7 / 36.3.
+// Which form, by the number of 128-row workgroups, us (the forms compared on one card).  Up to 400 (B = 1 and 32 heads: T up to
+// 1600) two waves per row group: 128 (T = 500) 12.2 against 15.3 of <1, 2> and 17.6 of <1, 1>, 256 (1003) 22.1 / 24.4 / 27.5, 384
+// (1500) 35.9 / 35.7 / 39.2; at 480 (1800) 49.1 / 44.9 / 49.7.  Up to 1500 64 keys per step: 512 (2048) 50.8 against 56.7 of <1, 1>,
+// 672 (28 heads over 4, 3000) 84.8 / 90.9, 1056 (4099) 169.0 / 172.8, 1376 (5500) 279 / 290; beyond it is even or behind: 2048
+// (8192) 586 / 584, 4096 (16384) 2255 / 2203.
+// The opposite order of the second 256 workgroups, us without / with it: of the 64-key form always, 416 workgroups (T = 1632)
+// 39.6 / 38.7, from 512 even; of walks of half the length past two and a half rounds, 608 (1200) 26.2 / 26.0, 728 (777, B = 2, 28
+// heads) 25.1 / 23.5, 768 (1500) 36.0 / 35.6.
 namespace hq {
 PromptForm prompt_form(int64_t T, int64_t BH) {
   const int64_t wgs = (T + 127) / 128 * BH;
