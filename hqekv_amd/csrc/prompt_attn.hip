@@ -467,7 +467,7 @@ __global__ __launch_bounds__(WAVES * 64, 1) void prompt_last_short_kernel(LastRo
   {
     const half_t *kp = a.k + b * a.k_b + hkv * a.k_h + 8 * piece;
     const half_t *qp = a.q + b * a.q_b + hkv * nrep * a.q_h + 8 * piece;
-    h8_t k[8], q[8 / WAVES + 1];
+    h8_t k[8], q[(7 + WAVES) / WAVES];
 #pragma unroll
     for (int j = 0; j < 8; ++j) k[j] = *reinterpret_cast<const h8_t *>(kp + (int64_t)min(32 * w + 4 * j + r4, T - 1) * a.k_t);
 #pragma unroll
@@ -864,6 +864,8 @@ extern "C" int hqekv_prompt_attn(const void *q, const int64_t *q_strides, const 
 // Up to 512 keys one launch, a wave per 32 keys.  One launch against two, us (32 heads over 8, 20 rows, host included): 128 keys
 // 6.2 / 7.1 (one workgroup of four waves per head then), 256 7.1 / 9.3, 512 8.2 / 9.4; B = 4 500 8.0 / 14.2, B = 64 64 / 126;
 // 1003 keys at two tiles per wave 14.6 / 10.1, B = 4 15.3 / 17.6.
+// Waves without a key cost time in the exchange of statistics: up to 384 keys on 12 waves against 16, 257 keys 6.7 / 7.6, 384 6.4 /
+// 7.5, B = 64 300 43.0 / 47.9.
 constexpr int64_t LS_KEYS = 512;
 // Beyond, slices of the keys: about 48 (b, query head) slices per column tile's 32 give the chip four to six workgroups per CU;
 // a slice keeps a tile for each of its four waves.
@@ -916,6 +918,7 @@ static int last_rows(const void *q, const int64_t *q_strides, const void *k, con
     if (T <= 64) LAUNCH(2);
     else if (T <= 128) LAUNCH(4);
     else if (T <= 256) LAUNCH(8);
+    else if (T <= 384) LAUNCH(12);
     else LAUNCH(16);
 #undef LAUNCH
     return check_launch("prompt_last_rows");

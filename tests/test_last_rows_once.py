@@ -1,6 +1,6 @@
 """The probabilities of a prompt's last rows in one launch (slices of at most 128 keys): the same bits as in two, whether the
 slices' statistics come from the other workgroups or a workgroup waits for nobody; each replay of a captured call equals the
-call."""
+call.  And the shorter prompts' launch at its edges of twelve waves."""
 import ctypes as C
 
 import pytest
@@ -86,3 +86,18 @@ def test_captured_call_is_replayed_on_new_inputs():
         q.copy_(torch.randn(q.shape, generator=g, device="cuda"))
         graph.replay()
         assert torch.equal(probs.view(torch.int16), _run(lib, q, k, 20, 2000).view(torch.int16)), i
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,Hq,Hkv,R", [(1, 32, 8, 20), (2, 7, 1, 32)])
+@pytest.mark.parametrize("T", [257, 288, 353, 384, 385])
+def test_twelve_waves(T, B, Hq, Hkv, R):
+    """Tolerance: two roundings of a logit may fall to the other half -- the product's, 2^-5 below 64 and times the scale 2.8e-3, and
+    the scaled one's, 2^-8 below 8 -- and the probability's own, 2^-11: 7.2e-3."""
+    from hqekv_amd.prompt_attention import prompt_last_rows
+    g = torch.Generator("cuda").manual_seed(T)
+    q, k = (torch.randn(B, H, T, 128, generator=g, device="cuda").half() for H in (Hq, Hkv))
+    got = prompt_last_rows(q, k, 128 ** -0.5, R)
+    s = torch.matmul(q[:, :, T - R:].float(), k.float().repeat_interleave(Hq // Hkv, 1).transpose(2, 3).contiguous()).half()
+    s = (s.float() * 128 ** -0.5).half().float().masked_fill(torch.ones(T, T, device="cuda", dtype=torch.bool).triu(1)[T - R:], float("-inf"))
+    torch.testing.assert_close(got.float(), s.softmax(-1), rtol=7.2e-3, atol=1e-6)
