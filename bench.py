@@ -39,13 +39,13 @@ WORKLOADS = {
 
 
 def kernel_source_sha16() -> str:
-    """Hash of the HIP sources the decode-attention kernels are built from (attn.hip, decode_qk.hip, decode_pv.hip and the headers): recorded next
+    """Hash of the HIP sources the decode-attention kernels are built from (attn.hip, decode_qk.hip, decode_pv.hip, decode_step.hip and the headers): recorded next
     to counter-derived figures so that a figure measured on other kernels is recognised as stale."""
     import hashlib
     h = hashlib.sha256()
     csrc = os.path.join(ROOT, "hqekv_amd", "csrc")
     for name in sorted(os.listdir(csrc)):
-        if name in ("attn.hip", "decode_qk.hip", "decode_pv.hip") or name.endswith(".h"):
+        if name in ("attn.hip", "decode_qk.hip", "decode_pv.hip", "decode_step.hip") or name.endswith(".h"):
             h.update(name.encode())
             h.update(open(os.path.join(csrc, name), "rb").read())
     return h.hexdigest()[:16]
