@@ -26,7 +26,11 @@ constexpr int PA_WAVES = 4;
 constexpr int PA_THREADS = 64 * PA_WAVES;
 constexpr int PA_BC = 32;              // keys per score tile
 constexpr float PA_SLACK = 8.f;        // powers of two
-constexpr int PA_SHARE = 4;
+// (powers of two, by the keys that a row block walks; the reason beside its use)
+__device__ __forceinline__ int pa_share(int keys) {
+  const int lg = 32 - __builtin_clz(keys);
+  return keys <= 8192 ? max(5, lg - 7) : lg - 6;
+}
 // How the four waves of a workgroup share its work, and how many keys a wave takes at a time.
 // <1, 1>: 32 query rows each, 128 per workgroup, every wave walks all key tiles (154 registers, 32 KB of LDS: three
 // workgroups per CU).  For long prompts, which are bound by the chip's power: no order of the same instructions is faster.
@@ -146,10 +150,10 @@ __global__ __launch_bounds__(PA_THREADS, S::WGS) void prompt_attn_kernel(PromptA
   f16_t o[4];
 #pragma unroll
   for (int dt = 0; dt < 4; ++dt) o[dt] = (f16_t)(0.f);
-  float m = -INFINITY, lsum = 0.f;
+  float m = -INFINITY, limit = -INFINITY, lsum = 0.f;
   const float sl2 = a.scale * 1.4426950408889634f;
   const int kend = CAUSAL ? min(T, q0 + S::ROWS) : T;
-  const int n_steps = (kend + S::STEP - 1) / S::STEP;
+  const int n_steps = (kend + S::STEP - 1) / S::STEP, share = pa_share(kend);
   PaSource src;
   src.k = make_desc(kp, (uint32_t)((int64_t)T * a.k_t * 2));   // (below 4 GiB: checked by the host)
   src.v = make_desc(vp, (uint32_t)((int64_t)T * a.v_t * 2));
@@ -216,17 +220,20 @@ __global__ __launch_bounds__(PA_THREADS, S::WGS) void prompt_attn_kernel(PromptA
       for (int r = 0; r < 16; ++r) raw = fmaxf(raw, s[i][r]);
     // m is what the exponents are taken relative to: the maximum so far, or a little less.  The 64 products of a rescale (and the
     // exchange between the lane halves) are left out while what passes m does so by less than 2^PA_SLACK and holds less than
-    // 2^-PA_SHARE of the lane's sum: a maximum's own weight is exactly one and has no rounding error, which shows where it
-    // dominates its row.  Relative error (2-norm) against 64 bits of a rescale each time / this / none, T = 1003, two key shares:
-    // N(0, 1) 2.450e-4 / 2.452e-4 / 2.535e-4, four channels of K ten times as large 2.191e-4 / 2.191e-4 / 2.395e-4 (2.461e-4 and
-    // 2.198e-4 with the sum taken before the rounding to fp16).  Time, us: T = 4099 176 / 167 / 163, 32768 8790 / 8650 / 8560 (one
-    // slow box).  (sl2 > 0; KS = 1: the first tile always holds key 0, which no query masks: m is finite from then on.)
+    // 2^-share of the lane's sum: a maximum's own weight is exactly one and has no rounding error, which shows where it
+    // dominates its row -- and in a long walk at a smaller share, since the others are smaller, too (pa_share).  Relative error
+    // (2-norm) against 64 bits, 32 heads over 8, N(0, 1): a rescale each time and the sum taken before the rounding to fp16 / this /
+    // 2^-4 throughout: T = 1003 2.535e-4 / 2.518 / 2.521, 4099 2.589 / 2.582 / 2.595; <1, 1>: 8192 2.520 / 2.518 / 2.535, 16384 2.357 /
+    // 2.353 / 2.370, 32768 2.0737 / 2.0726 / 2.0883; two channels of K ten times as large, 4099 2.357 / 2.347 / 2.352, 32768 2.261 / 2.250 /
+    // 2.269.  Time of the three, us, on one card: T = 2048 50.8 / 49.9 / 48.6, 4099 159.3 / 157.6 / 155.5, 8192 553 / 547 / 532, 32768
+    // 8175 / 8100 / 7960.  (sl2 > 0; KS = 1: the first tile always holds key 0, which no query masks: m is finite from then on.)
     // Per lane on purpose: a divergent branch keeps the accumulators where they are (inactive lanes must keep their
     // values, so the products are in place under the execution mask, skipped when no lane needs them); a wave-uniform
     // branch made the compiler copy all 64 accumulators per tile.
     raw *= sl2;
-        const float slack = fminf(fmaxf((float)(__builtin_amdgcn_frexp_expf(lsum) - PA_SHARE), 0.f), PA_SLACK);
-    const uint64_t over = __builtin_amdgcn_ballot_w64(raw > m + slack), both = over | over >> 32 | over << 32;   // a query's two lanes agree
+    auto bound = [&](int share_of) { return m + fminf(fmaxf((float)(__builtin_amdgcn_frexp_expf(lsum) - share_of), 0.f), PA_SLACK); };
+    if constexpr (KS * NB > 1) limit = bound(share);   // (<1, 1>: by the sum at the last rescale, a smaller one)
+    const uint64_t over = __builtin_amdgcn_ballot_w64(raw > limit), both = over | over >> 32 | over << 32;   // a query's two lanes agree
     if (both >> lane & 1) {
       const float mx = fmaxf(m, fmaxf(raw, __shfl_xor(raw, 32, 64)));
       const float alpha = __builtin_amdgcn_exp2f(m - mx);   // (the bare instruction: results below 2^-126 may flush to zero)
@@ -234,6 +241,7 @@ __global__ __launch_bounds__(PA_THREADS, S::WGS) void prompt_attn_kernel(PromptA
 #pragma unroll
       for (int dt = 0; dt < 4; ++dt) o[dt] *= alpha;
       m = mx;
+      if constexpr (KS * NB == 1) limit = bound(share - 1);
     }
     const float base = KS > 1 && m == -INFINITY ? 0.f : m;   // nothing but masked keys so far: exponentials of -inf are zero
 #pragma unroll
