@@ -2176,7 +2176,7 @@ extern "C" int hqekv_pv_hybrid(const hqekv_seg *segs, int nseg, const void *p, v
 static int64_t align_up(int64_t v, int64_t a) { return (v + a - 1) / a * a; }
 
 struct DecodeLayout {  // carve-up of the caller's workspace
-  int64_t chunk, partial_bytes, stats_off, stats_bytes, arrive_off, logits_off, logits_bytes, records_off, pairs_off, total;
+  int64_t chunk, partial_bytes, stats_off, stats_bytes, arrive_off, logits_off, logits_bytes, records_off, pairs_off, total, least;   // least: without one launch's records
   int64_t n_stat, chunks;
 };
 
@@ -2215,8 +2215,8 @@ static int decode_layout(const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_se
   // still does, and the two entries give the same bits.  (A short step has at most 1536 workgroups, so that only seven and
   // eight heads per KV head get there: 9 x 4k tokens at eight 27.3 us in three launches, 25.7 in two; 34 x 1184 46.9 either way.)
   if (L->logits_off + L->logits_bytes > (int64_t)HQEKV_STATIC_SCRATCH_BYTES) L->logits_bytes = 0;
-  L->total = L->logits_off + L->logits_bytes;
-  // ... and what one launch needs beside them, by the same rule
+  L->total = L->least = L->logits_off + L->logits_bytes;
+  // ... and what one launch needs beside them, by the same rule; a workspace without room for that gets two launches
   L->records_off = L->total;
   L->pairs_off = L->records_off + align_up(B * Hq * tiles * 16, 256);
   const int64_t one = L->pairs_off + align_up(chunks * B * Hq * D * 8, 256);
@@ -2436,9 +2436,10 @@ static int decode_impl(const hqekv_seg *k_segs, int n_k, const hqekv_seg *v_segs
   if (!q || !attn_weights || !attn_out || Tall <= 0) return fail(HQEKV_E_ARG, "decode_attn: null pointer or Tall <= 0");
   DecodeLayout L;
   if (decode_layout(k_segs, n_k, v_segs, n_v, B, Hq, Hkv, D, &L)) return fail(HQEKV_E_ARG, "decode_attn: bad segment tables");
-  if (!workspace || workspace_bytes < L.total)
+  if (!workspace || workspace_bytes < L.least)
     return fail(HQEKV_E_WORKSPACE, "decode_attn: workspace %lld bytes < %lld needed", (long long)workspace_bytes,
-                (long long)L.total);
+                (long long)L.least);
+  if (workspace_bytes < L.total) L.records_off = 0;
   if ((uintptr_t)workspace & 255) return fail(HQEKV_E_ALIGN, "decode_attn: workspace not 256-byte aligned");
   int tiling = 0;
   rc = resolve_qk_tiling(qk_tiling_of(flags), k_segs, n_k, B * Hkv, D, "decode_attn", &tiling);

@@ -293,7 +293,8 @@ int hqekv_pv_hybrid(const hqekv_seg *segs, int nseg, const void *p, void *out, i
  * and the form of the dot products the other flags name: what gemv_forward_cuda_qk_group_hq returns
  * (quant/csrc/gemv_cuda.h:78-109), for callers and tests that want the scores of one particular tiling. */
 #define HQEKV_ONLY_RAW_QK 0x2000
-/* A short step is one launch, or two while the stream is captured, with the same bits.  TWO_LAUNCHES: two in any case.
+/* A short step is one launch, or two while the stream is captured or the workspace has no room for its records, with the
+ * same bits.  TWO_LAUNCHES: two in any case.
  * IMPATIENT, for tests: the one launch's workgroups look once for what others leave them and otherwise do it themselves. */
 #define HQEKV_TWO_LAUNCHES 0x4000
 #define HQEKV_IMPATIENT 0x8000

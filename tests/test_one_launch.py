@@ -143,3 +143,31 @@ def test_two_streams_at_once(dev):
     torch.cuda.synchronize()
     for (plan, _), (w, o) in zip(plans, want):
         assert torch.equal(plan.weights, w) and torch.equal(plan.out, o)
+
+
+@pytest.mark.gpu
+def test_a_workspace_without_room_for_the_records(dev):
+    """What two launches need is enough, with the same bits; less is refused."""
+    from hqekv_amd import _lib
+    from hqekv_amd.attention import DecodePlan
+    lib, pkv = _lib.load(), _cache(dev, 2, 4, (1, 1, 9, 8, 1), 3, False, True, 5)
+    q = torch.randn(2, 16, 1, D, generator=torch.Generator(device=dev).manual_seed(3), device=dev, dtype=torch.float16)
+    plan = DecodePlan(q, pkv)
+    plan.run(q)
+    want = plan.weights.clone(), plan.out.clone()
+    need = lib.hqekv_decode_workspace_bytes(plan.k_segs, len(plan.k_segs), plan.v_segs, len(plan.v_segs), 2, 16, 4, D)
+    ws = torch.empty(need, dtype=torch.uint8, device=dev)
+    low, high = 0, need // 256
+    while high - low > 1:
+        size = 256 * ((low + high) // 2)
+        plan.weights.fill_(7)
+        plan.out.fill_(7)
+        rc = lib.hqekv_decode_attn(plan.k_segs, len(plan.k_segs), plan.v_segs, len(plan.v_segs), q.data_ptr(), None, 0, plan.weights.data_ptr(),
+                                   plan.out.data_ptr(), 2, 16, 4, D, plan.Tall, ws.data_ptr(), size, plan.flags, torch.cuda.current_stream().cuda_stream)
+        if rc == 0:
+            assert torch.equal(plan.weights, want[0]) and torch.equal(plan.out, want[1]), size
+            high = size // 256
+        else:
+            assert rc == -3   # HQEKV_E_WORKSPACE
+            low = size // 256
+    assert 0 < 256 * high < need
